@@ -158,32 +158,6 @@ static int weight_alloc(int dev, int dt, int64_t n, int64_t k, cq_weight **out) 
     return CQ_OK;
 }
 
-// GGML blocks of the caller's type (device memory) into the planes, and back.  A type held in another type's planes
-// goes through that type's blocks in a temporary (set-up paths: they synchronize before freeing it).
-static int64_t weight_blocks(const cq_weight *w) { return w->n * (w->k / cq_block_size(w->dtype)); }
-static hipError_t blocks_to_planes(const cq_weight *w, uint8_t *ggml_aos_dev, hipStream_t s) {
-    if (w->ggml_dtype == w->dtype) return cq_launch_repack(w, ggml_aos_dev, s);
-    void *tmp = nullptr;
-    hipError_t e = hipMalloc(&tmp, (size_t)weight_blocks(w) * (size_t)cq_type_size(w->dtype) + 256);
-    if (e != hipSuccess) return e;
-    e = cq_launch_transcode(w, ggml_aos_dev, (uint8_t *)tmp, weight_blocks(w), false, s);
-    if (e == hipSuccess) e = cq_launch_repack(w, (const uint8_t *)tmp, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(tmp);
-    return e;
-}
-static hipError_t planes_to_blocks(const cq_weight *w, uint8_t *ggml_aos_dev, hipStream_t s) {
-    if (w->ggml_dtype == w->dtype) return cq_launch_unpack(w, ggml_aos_dev, s);
-    void *tmp = nullptr;
-    hipError_t e = hipMalloc(&tmp, (size_t)weight_blocks(w) * (size_t)cq_type_size(w->dtype) + 256);
-    if (e != hipSuccess) return e;
-    e = cq_launch_unpack(w, (uint8_t *)tmp, s);
-    if (e == hipSuccess) e = cq_launch_transcode(w, ggml_aos_dev, (uint8_t *)tmp, weight_blocks(w), true, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(tmp);
-    return e;
-}
-
 extern "C" int cq_weight_zeros(int dev, int dt, int64_t n, int64_t k, cq_weight **out) {
     int rc = weight_alloc(dev, dt, n, k, out);
     if (rc) return rc;
@@ -194,7 +168,7 @@ extern "C" int cq_weight_zeros(int dev, int dt, int64_t n, int64_t k, cq_weight 
         void *tmp = nullptr;
         e = hipMalloc(&tmp, (*out)->ggml_bytes + 256);
         if (e == hipSuccess) e = hipMemset(tmp, 0, (*out)->ggml_bytes);
-        if (e == hipSuccess) e = blocks_to_planes(*out, (uint8_t *)tmp, nullptr);
+        if (e == hipSuccess) e = cq_launch_repack(*out, (const uint8_t *)tmp, nullptr);
         if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
         if (tmp) (void)hipFree(tmp);
     }
@@ -222,7 +196,7 @@ extern "C" int cq_weight_create(int dev, int dt, const void *host_blocks, size_t
     void *tmp = nullptr;
     hipError_t e = hipMalloc(&tmp, nbytes + 256);
     if (e == hipSuccess) e = hipMemcpy(tmp, host_blocks, nbytes, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = blocks_to_planes(w, (uint8_t *)tmp, nullptr);
+    if (e == hipSuccess) e = cq_launch_repack(w, (const uint8_t *)tmp, nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (tmp) (void)hipFree(tmp);
     if (e != hipSuccess) {
@@ -290,7 +264,7 @@ extern "C" int cq_weight_quantize(cq_weight *w, const float *src_dev, void *stre
     CQ_HIP_CHECK(hipMalloc(&tmp, w->ggml_bytes + 256));
     const int64_t nb = w->n * (w->k / cq_block_size(w->dtype));
     hipError_t e = cq_launch_quantize_weight(w->ggml_dtype, src_dev, nb, (uint8_t *)tmp, s);
-    if (e == hipSuccess) e = blocks_to_planes(w, (uint8_t *)tmp, s);
+    if (e == hipSuccess) e = cq_launch_repack(w, (const uint8_t *)tmp, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);  // the temporary is freed below
     (void)hipFree(tmp);
     if (e != hipSuccess) return cq_set_error(CQ_ERR_HIP, "weight quantize failed: %s", hipGetErrorString(e));
@@ -322,7 +296,7 @@ extern "C" int cq_weight_to_ggml(const cq_weight *w, void *host_dst, size_t nbyt
     void *tmp = nullptr;
     CQ_HIP_CHECK(hipMalloc(&tmp, nbytes + 256));
     hipError_t e = hipDeviceSynchronize();
-    if (e == hipSuccess) e = planes_to_blocks(w, (uint8_t *)tmp, nullptr);
+    if (e == hipSuccess) e = cq_launch_unpack(w, (uint8_t *)tmp, nullptr);
     if (e == hipSuccess) e = hipMemcpy(host_dst, tmp, nbytes, hipMemcpyDeviceToHost);
     (void)hipFree(tmp);
     if (e != hipSuccess) return cq_set_error(CQ_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));

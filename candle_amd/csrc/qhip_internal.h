@@ -96,7 +96,7 @@ bool cq_timing_take(hipEvent_t *start, hipEvent_t *stop);
 
 // ---- launchers implemented in the .hip files -------------------------------
 // repack.hip
-hipError_t cq_launch_repack(const cq_weight *w, const uint8_t *aos_dev, hipStream_t s);   // GGML AoS -> planes
+hipError_t cq_launch_repack(const cq_weight *w, const uint8_t *aos_dev, hipStream_t s);   // GGML AoS of w->ggml_dtype -> planes
 hipError_t cq_launch_unpack(const cq_weight *w, uint8_t *aos_dev, hipStream_t s);         // planes -> GGML AoS
 // Types held in another type's planes (same values, same arithmetic): Q5_0 as Q8_0, Q3K as Q6K.
 // Q4_1 and Q5_1 (value d * q + m) are Q8_0 planes with qs = q plus the plane p2 of the blocks' minima m (f16): the
@@ -110,9 +110,6 @@ inline int cq_storage_dtype(int ggml_dtype) {
     if (ggml_dtype == CQ_DTYPE_Q5_0 || cq_has_min32(ggml_dtype)) return CQ_DTYPE_Q8_0;
     return ggml_dtype == CQ_DTYPE_Q3K || ggml_dtype == CQ_DTYPE_Q2K ? CQ_DTYPE_Q6K : ggml_dtype;
 }
-// `w` supplies the planes beside the holding type's blocks: the minima of Q4_1 / Q5_1 (p2), of Q2K (p4, p5)
-hipError_t cq_launch_transcode(const cq_weight *w, uint8_t *ggml_aos_dev, uint8_t *storage_aos_dev, int64_t nblocks, bool inverse,
-                               hipStream_t s);
 // y[r, c] -= sum_b (d8[r, b] * dmin[c, b]) * sum_j bsums[r, b, j] * m[c, b, j] for Q2K weights (k_quants.rs:727-733, :762)
 hipError_t cq_launch_min16_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s);
 // Q8K as a weight type (q8k_weight.hip): planes p0 qs, p1 d (f32), p2 bsums

@@ -112,31 +112,20 @@ __global__ void repack_q5k(const uint8_t *__restrict__ aos, uint8_t *__restrict_
     }
     if (u == 2) return;
     if (u == 1) {
-        uint8_t *src = (uint8_t *)aos + b * 176 + 16;   // GGML qh[32]
-        uint32_t *dst = (uint32_t *)(qh + b * 32);      // {L, H} x 4
-        if (!inverse) {
-            for (int g = 0; g < 4; g++) {
-                uint32_t L = 0, H = 0;
-                for (int i = 0; i < 8; i++)
-                    for (int c = 0; c < 4; c++) {
-                        const uint32_t v = src[4 * i + c];
-                        L |= ((v >> (2 * g)) & 1u) << (8 * c + i);
-                        H |= ((v >> (2 * g + 1)) & 1u) << (8 * c + i);
-                    }
-                dst[2 * g] = L;
-                dst[2 * g + 1] = H;
-            }
-        } else {
-            for (int i = 0; i < 8; i++)
-                for (int c = 0; c < 4; c++) {
-                    uint32_t v = 0;
-                    for (int g = 0; g < 4; g++) {
-                        v |= ((dst[2 * g] >> (8 * c + i)) & 1u) << (2 * g);
-                        v |= ((dst[2 * g + 1] >> (8 * c + i)) & 1u) << (2 * g + 1);
-                    }
-                    src[4 * i + c] = (uint8_t)v;
-                }
+        uint4 *src = (uint4 *)(aos + b * 176 + 16);   // GGML qh[32]
+        uint4 *dst = (uint4 *)(qh + b * 32);          // {L, H} x 4
+        // bit 8c + i of L_g = bit 2g of byte c of word i, bit 8c + i of H_g = bit 2g + 1: a transpose in words, its own form both ways
+        const uint4 x0 = inverse ? dst[0] : src[0], x1 = inverse ? dst[1] : src[1];
+        const uint32_t in[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        uint32_t out[8];
+#pragma unroll
+        for (int o = 0; o < 8; o++) {
+            out[o] = 0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) out[o] |= ((in[i] >> o) & 0x01010101u) << i;
         }
+        (inverse ? src : dst)[0] = make_uint4(out[0], out[1], out[2], out[3]);
+        (inverse ? src : dst)[1] = make_uint4(out[4], out[5], out[6], out[7]);
         return;
     }
     k4_header(a, (uint32_t *)(hd + b * CQ_Q4K_HDR), inverse);
@@ -209,155 +198,208 @@ __global__ void repack_q6k(const uint8_t *__restrict__ aos, uint8_t *__restrict_
 }
 
 // ---- types held in another type's planes --------------------------------------------------------
-// Q5_0 {f16 d; u8 qh[4]; u8 qs[16]} (k_quants.rs:61-67) holds d and 32 five-bit quants q, value d * (q - 16): exactly a
-// Q8_0 block {f16 d; i8 qs[32]} with qs = q - 16, whose dequantization (k_quants.rs:568-584) and dot product with Q8_0
-// activations (:631-649) are the arithmetic of Q5_0's (:428-451, :371-391) operation for operation.
-__global__ void transcode_q5_0_q8_0(uint8_t *__restrict__ q5, uint8_t *__restrict__ q8, int64_t nblocks, bool inverse) {
+// Straight between the GGML blocks and the planes, in words of four quants: the blocks are read and written once and
+// nothing goes through the holding type's blocks in between.  Bound: HBM.  11008 x 4096 elements, per direction, byte loops
+// through a second set of blocks before -> now: Q3K 2581 + 12 -> 12 us, Q2K 2270 + 12 -> 9, Q5_0 / Q4_1 / Q5_1 18-20 + 15 -> 14.
+typedef uint32_t u32_any __attribute__((aligned(2)));                          // GGML blocks lie at even addresses
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ void load16(const uint8_t *p, uint32_t (&v)[4]) {
+    const u32x4_any x = *(const u32x4_any *)p;
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+}
+__device__ __forceinline__ void store16(uint8_t *p, const uint32_t (&v)[4]) {
+    u32x4_any x = {v[0], v[1], v[2], v[3]};
+    *(u32x4_any *)p = x;
+}
+// bits 4i .. 4i+3 of `bits` as bit 0 of the four bytes of a word, and back
+__device__ __forceinline__ uint32_t spread4(uint32_t bits, int i) {
+    const uint32_t n = (bits >> (4 * i)) & 15u;
+    return (n & 1u) | ((n & 2u) << 7) | ((n & 4u) << 14) | ((n & 8u) << 21);
+}
+__device__ __forceinline__ uint32_t gather4(uint32_t w, int i) {
+    return ((w & 1u) | ((w >> 7) & 2u) | ((w >> 14) & 4u) | ((w >> 21) & 8u)) << (4 * i);
+}
+
+// In Q8_0 planes, one thread per block:
+//   Q5_0 {f16 d; u8 qh[4]; u8 qs[16]} (k_quants.rs:61-67) holds d and 32 five-bit quants q, value d * (q - 16): exactly a
+//   Q8_0 block {f16 d; i8 qs[32]} with qs = q - 16, whose dequantization (k_quants.rs:568-584) and dot product with Q8_0
+//   activations (:631-649) are the arithmetic of Q5_0's (:428-451, :371-391) operation for operation.
+//   Q4_1 {f16 d; f16 m; u8 qs[16]} and Q5_1 {f16 d; f16 m; u8 qh[4]; u8 qs[16]} (k_quants.rs:51-57, :69-76), value
+//   d * q + m: the quants (0..15, 0..31) and d as a Q8_0 block, m into its own plane.
+template <int DT>
+__global__ void held_in_q8_0(uint8_t *__restrict__ aos, uint8_t *__restrict__ qs, uint16_t *__restrict__ d,
+                             uint16_t *__restrict__ mins, int64_t nblocks, bool inverse) {
     const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nblocks) return;
-    uint8_t *x = q5 + b * 22, *y = q8 + b * 34;
+    constexpr bool FIVE = DT != CQ_DTYPE_Q4_1, MIN = DT != CQ_DTYPE_Q5_0;
+    constexpr int TS = DT == CQ_DTYPE_Q4_1 ? 20 : DT == CQ_DTYPE_Q5_0 ? 22 : 24, QH = MIN ? 4 : 2, QS = FIVE ? QH + 4 : QH;
+    constexpr uint32_t OFF = DT == CQ_DTYPE_Q5_0 ? 16 : 0;
+    uint8_t *x = aos + b * TS;
+    uint4 *p = (uint4 *)(qs + b * 32);
+    uint32_t lo[4], hi[4];
     if (!inverse) {
-        y[0] = x[0];
-        y[1] = x[1];
-        const uint32_t qh = (uint32_t)x[2] | ((uint32_t)x[3] << 8) | ((uint32_t)x[4] << 16) | ((uint32_t)x[5] << 24);
-        for (int j = 0; j < 16; j++) {
-            const int x0 = (int)((x[6 + j] & 0x0F) | (((qh >> j) & 1u) << 4)) - 16;
-            const int x1 = (int)((x[6 + j] >> 4) | (((qh >> (j + 16)) & 1u) << 4)) - 16;
-            y[2 + j] = (uint8_t)(int8_t)x0;
-            y[2 + j + 16] = (uint8_t)(int8_t)x1;
+        uint32_t q[4];
+        load16(x + QS, q);
+        const uint32_t qh = FIVE ? *(const u32_any *)(x + QH) : 0u;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            lo[i] = q[i] & 0x0F0F0F0Fu;
+            hi[i] = (q[i] >> 4) & 0x0F0F0F0Fu;
+            if (FIVE) {
+                lo[i] |= spread4(qh, i) << 4;
+                hi[i] |= spread4(qh, 4 + i) << 4;
+            }
+            if (OFF) {   // byte - 16 for bytes 0..31: + 0xF0 in each byte without its carry
+                lo[i] = (lo[i] ^ 0x10101010u) | (((~lo[i] >> 4) & 0x01010101u) * 0xE0u);
+                hi[i] = (hi[i] ^ 0x10101010u) | (((~hi[i] >> 4) & 0x01010101u) * 0xE0u);
+            }
         }
+        p[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+        p[1] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        d[b] = *(const uint16_t *)x;
+        if (MIN) mins[b] = *(const uint16_t *)(x + 2);
     } else {
-        x[0] = y[0];
-        x[1] = y[1];
-        uint32_t qh = 0;
-        for (int j = 0; j < 16; j++) {
-            const uint32_t v0 = (uint32_t)((int)(int8_t)y[2 + j] + 16) & 31u, v1 = (uint32_t)((int)(int8_t)y[2 + j + 16] + 16) & 31u;
-            x[6 + j] = (uint8_t)((v0 & 0x0F) | ((v1 & 0x0F) << 4));
-            qh |= (v0 >> 4) << j;
-            qh |= (v1 >> 4) << (j + 16);
+        const uint4 a = p[0], c = p[1];
+        lo[0] = a.x; lo[1] = a.y; lo[2] = a.z; lo[3] = a.w;
+        hi[0] = c.x; hi[1] = c.y; hi[2] = c.z; hi[3] = c.w;
+        uint32_t q[4], qh = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (OFF) {   // the low five bits of q - 16 are those of q with the fifth flipped
+                lo[i] ^= 0x10101010u;
+                hi[i] ^= 0x10101010u;
+            }
+            q[i] = (lo[i] & 0x0F0F0F0Fu) | ((hi[i] & 0x0F0F0F0Fu) << 4);
+            if (FIVE) qh |= gather4(lo[i] >> 4, i) | gather4(hi[i] >> 4, 4 + i);
         }
-        x[2] = (uint8_t)qh; x[3] = (uint8_t)(qh >> 8); x[4] = (uint8_t)(qh >> 16); x[5] = (uint8_t)(qh >> 24);
+        store16(x + QS, q);
+        if (FIVE) *(u32_any *)(x + QH) = qh;
+        *(uint16_t *)x = d[b];
+        if (MIN) *(uint16_t *)(x + 2) = mins[b];
     }
 }
 
-// Q4_1 {f16 d; f16 m; u8 qs[16]} and Q5_1 {f16 d; f16 m; u8 qh[4]; u8 qs[16]} (k_quants.rs:51-57, :69-76): value d * q + m.
-// The quants (0..15, 0..31) and d go into a Q8_0 block, m into its own plane.
-template <bool FIVE>
-__global__ void transcode_q4_1_q8_0(uint8_t *__restrict__ src, uint8_t *__restrict__ q8, uint16_t *__restrict__ mins,
-                                    int64_t nblocks, bool inverse) {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nblocks) return;
-    constexpr int TS = FIVE ? 24 : 20, QS = FIVE ? 8 : 4;
-    uint8_t *x = src + b * TS, *y = q8 + b * 34;
-    if (!inverse) {
-        y[0] = x[0];
-        y[1] = x[1];
-        mins[b] = (uint16_t)(x[2] | (x[3] << 8));
-        const uint32_t qh = FIVE ? ((uint32_t)x[4] | ((uint32_t)x[5] << 8) | ((uint32_t)x[6] << 16) | ((uint32_t)x[7] << 24)) : 0u;
-        for (int j = 0; j < 16; j++) {
-            y[2 + j] = (uint8_t)((x[QS + j] & 0x0F) | (((qh >> j) & 1u) << 4));
-            y[2 + j + 16] = (uint8_t)((x[QS + j] >> 4) | (((qh >> (j + 16)) & 1u) << 4));
-        }
-    } else {
-        x[0] = y[0];
-        x[1] = y[1];
-        x[2] = (uint8_t)(mins[b] & 0xff);
-        x[3] = (uint8_t)(mins[b] >> 8);
-        uint32_t qh = 0;
-        for (int j = 0; j < 16; j++) {
-            const uint32_t v0 = y[2 + j], v1 = y[2 + j + 16];
-            x[QS + j] = (uint8_t)((v0 & 0x0F) | ((v1 & 0x0F) << 4));
-            qh |= ((v0 >> 4) & 1u) << j;
-            qh |= ((v1 >> 4) & 1u) << (j + 16);
-        }
-        if (FIVE) { x[4] = (uint8_t)qh; x[5] = (uint8_t)(qh >> 8); x[6] = (uint8_t)(qh >> 16); x[7] = (uint8_t)(qh >> 24); }
-    }
-}
-
-// Q3K {u8 hmask[32]; u8 qs[64]; u8 scales[12]; f16 d} (k_quants.rs:107-114): sixteen groups of sixteen three-bit quants,
-// value (d * (sc_j - 32)) * (q - 4) with six-bit sc_j: exactly a Q6K block {ql, qh, i8 scales[16], f16 d} with
-// scales[j] = sc_j - 32 and six-bit quants q + 28 (so that q6 - 32 = q - 4), whose dequantization (k_quants.rs:1716-1746)
-// and dot product with Q8K activations (:1585-1641) are those of Q3K (:1094-1146, :890-1009): the same integers, the
-// same products in the same order.
+// In Q6K planes, eight threads per block, thread u = 4h + 2t + i the unit u of the Q6K layout above (ql bytes 16u ..: the
+// elements 128h + 32t + 16i + e in the low and those 64 further on in the high nibbles):
+//   Q3K {u8 hmask[32]; u8 qs[64]; u8 scales[12]; f16 d} (k_quants.rs:107-114): sixteen groups of sixteen three-bit quants,
+//   value (d * (sc_j - 32)) * (q - 4) with six-bit sc_j: exactly a Q6K block {ql, qh, i8 scales[16], f16 d} with
+//   scales[j] = sc_j - 32 and six-bit quants q + 28 (so that q6 - 32 = q - 4), whose dequantization (k_quants.rs:1716-1746)
+//   and dot product with Q8K activations (:1585-1641) are those of Q3K (:1094-1146, :890-1009): the same integers, the
+//   same products in the same order.
+//   Q2K {u8 scales[16]; u8 qs[64]; f16 d; f16 dmin} (k_quants.rs:96-103): value (d * sc_j) * q - dmin * m_j, sc_j and m_j
+//   the nibbles of scales[j].  The first term is a Q6K block with scales sc_j and quants q + 32; m_j and dmin go to planes
+//   of their own.
+// Both hold the two low bits of four elements 32 apart in one byte of qs[32h + 16i ..], at 2 * (element / 32 % 4); Q3K's
+// third bit is bit element / 32 of hmask[16i ..].
 __device__ __forceinline__ int q3k_scale6(const uint8_t *sc, int j) {
     const int low = j < 8 ? (sc[j] & 0xF) : (sc[j - 8] >> 4);
     return low | (((sc[8 + j % 4] >> (2 * (j / 4))) & 3) << 4);
 }
-__global__ void transcode_q3k_q6k(uint8_t *__restrict__ q3, uint8_t *__restrict__ q6, int64_t nblocks, bool inverse) {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nblocks) return;
-    uint8_t *x = q3 + b * 110, *y = q6 + b * 210;
-    uint8_t *hmask = x, *qs = x + 32, *sc3 = x + 96;
-    uint8_t *ql = y, *qh = y + 128, *sc6 = y + 192;
-    if (!inverse) {
-        for (int i = 0; i < 192; i++) y[i] = 0;
-        for (int e = 0; e < 256; e++) {
-            const int half = e / 128, r = e % 128, quad = r / 32, l = r % 32;
-            const int low = (qs[32 * half + l] >> (2 * quad)) & 3;
-            const int v = low + 4 * ((hmask[e % 32] >> (e / 32)) & 1) + 28;   // (q - 4) + 32
-            ql[64 * half + 32 * (quad & 1) + l] |= (uint8_t)((v & 0xF) << (4 * (quad >> 1)));
-            qh[32 * half + l] |= (uint8_t)((v >> 4) << (2 * quad));
-        }
-        for (int j = 0; j < 16; j++) sc6[j] = (uint8_t)(int8_t)(q3k_scale6(sc3, j) - 32);
-        y[208] = x[108];
-        y[209] = x[109];
-    } else {
-        for (int i = 0; i < 108; i++) x[i] = 0;
-        for (int e = 0; e < 256; e++) {
-            const int half = e / 128, r = e % 128, quad = r / 32, l = r % 32;
-            const int v6 = ((ql[64 * half + 32 * (quad & 1) + l] >> (4 * (quad >> 1))) & 0xF) | (((qh[32 * half + l] >> (2 * quad)) & 3) << 4);
-            const int v = v6 - 28;   // 0..7
-            qs[32 * half + l] |= (uint8_t)((v & 3) << (2 * quad));
-            hmask[e % 32] |= (uint8_t)((v >> 2) << (e / 32));
-        }
-        for (int j = 0; j < 16; j++) {
-            const int lv = (int)(int8_t)sc6[j] + 32;
-            if (j < 8) sc3[j] |= (uint8_t)(lv & 0xF);
-            else sc3[j - 8] |= (uint8_t)((lv & 0xF) << 4);
-            sc3[8 + j % 4] |= (uint8_t)((lv >> 4) << (2 * (j / 4)));
-        }
-        x[108] = y[208];
-        x[109] = y[209];
+// the six-bit quants of unit u (16 in the low, 16 in the high nibbles) out of the planes
+__device__ __forceinline__ void q6_unit(const uint8_t *ql, const uint8_t *qh, int64_t b, int u, uint32_t (&lo)[4], uint32_t (&hi)[4]) {
+    const uint4 q = *(const uint4 *)(ql + b * 128 + 16 * u);
+    const uint2 H = *(const uint2 *)(qh + b * 64 + 8 * u);
+    const uint32_t qw[4] = {q.x, q.y, q.z, q.w}, hw[2] = {H.x, H.y};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t f = hw[i >> 1] >> (4 * (i & 1));
+        lo[i] = (qw[i] & 0x0F0F0F0Fu) | ((f & 0x03030303u) << 4);
+        hi[i] = ((qw[i] >> 4) & 0x0F0F0F0Fu) | (((f >> 2) & 0x03030303u) << 4);
     }
 }
-
-// Q2K {u8 scales[16]; u8 qs[64]; f16 d; f16 dmin} (k_quants.rs:96-103): value (d * sc_j) * q - dmin * m_j, sc_j and m_j
-// the nibbles of scales[j].  The first term is a Q6K block with scales sc_j and quants q + 32; m_j and dmin go to
-// planes of their own.
-__global__ void transcode_q2k_q6k(uint8_t *__restrict__ q2, uint8_t *__restrict__ q6, uint8_t *__restrict__ mins,
-                                  uint16_t *__restrict__ dmins, int64_t nblocks, bool inverse) {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+template <int DT>
+__global__ void held_in_q6k(uint8_t *__restrict__ aos, uint8_t *__restrict__ ql, uint8_t *__restrict__ qh, uint8_t *__restrict__ sc,
+                            uint16_t *__restrict__ d, uint8_t *__restrict__ mins, uint16_t *__restrict__ dmins, int64_t nblocks,
+                            bool inverse) {
+    const int64_t t8 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, b = t8 >> 3;
     if (b >= nblocks) return;
-    uint8_t *x = q2 + b * 84, *y = q6 + b * 210;
-    uint8_t *sc2 = x, *qs = x + 16;
-    uint8_t *ql = y, *qh = y + 128, *sc6 = y + 192, *mb = mins + b * 16;
+    constexpr bool Q3 = DT == CQ_DTYPE_Q3K;
+    constexpr int TS = Q3 ? 110 : 84, QS = Q3 ? 32 : 16, D = Q3 ? 108 : 80;
+    constexpr uint32_t OFF = Q3 ? 0x1C1C1C1Cu : 0x20202020u;   // 28 or 32 in each byte
+    const int u = (int)(t8 & 7), h = u >> 2, t = (u >> 1) & 1, i16 = u & 1;
+    uint8_t *x = aos + b * TS;
     if (!inverse) {
-        for (int i = 0; i < 192; i++) y[i] = 0;
-        for (int e = 0; e < 256; e++) {
-            const int half = e / 128, r = e % 128, quad = r / 32, l = r % 32;
-            const int v = ((qs[32 * half + l] >> (2 * quad)) & 3) + 32;
-            ql[64 * half + 32 * (quad & 1) + l] |= (uint8_t)((v & 0xF) << (4 * (quad >> 1)));
-            qh[32 * half + l] |= (uint8_t)((v >> 4) << (2 * quad));
+        uint32_t q[4], m[4] = {0, 0, 0, 0}, out[4], lo[4], hi[4];
+        load16(x + QS + 32 * h + 16 * i16, q);
+        if (Q3) load16(x + 16 * i16, m);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            lo[i] = ((q[i] >> (2 * t)) & 0x03030303u) + OFF;
+            hi[i] = ((q[i] >> (2 * t + 4)) & 0x03030303u) + OFF;
+            if (Q3) {
+                lo[i] += ((m[i] >> (4 * h + t)) & 0x01010101u) << 2;
+                hi[i] += ((m[i] >> (4 * h + t + 2)) & 0x01010101u) << 2;
+            }
+            out[i] = (lo[i] & 0x0F0F0F0Fu) | ((hi[i] & 0x0F0F0F0Fu) << 4);
+            lo[i] = (lo[i] >> 4) & 0x03030303u;
+            hi[i] = (hi[i] >> 4) & 0x03030303u;
         }
-        for (int j = 0; j < 16; j++) {
-            sc6[j] = (uint8_t)(sc2[j] & 0xF);
-            mb[j] = (uint8_t)(sc2[j] >> 4);
+        *(uint4 *)(ql + b * 128 + 16 * u) = make_uint4(out[0], out[1], out[2], out[3]);
+        *(uint2 *)(qh + b * 64 + 8 * u) = make_uint2(lo[0] | (hi[0] << 2) | (lo[1] << 4) | (hi[1] << 6),
+                                                    lo[2] | (hi[2] << 2) | (lo[3] << 4) | (hi[3] << 6));
+        const int js = u + 4 * h;
+        if (Q3) {
+            sc[b * 16 + 2 * u] = (uint8_t)(int8_t)(q3k_scale6(x + 96, js) - 32);
+            sc[b * 16 + 2 * u + 1] = (uint8_t)(int8_t)(q3k_scale6(x + 96, js + 4) - 32);
+        } else {
+            const uint8_t s0 = x[js], s1 = x[js + 4];
+            sc[b * 16 + 2 * u] = s0 & 0xF;
+            sc[b * 16 + 2 * u + 1] = s1 & 0xF;
+            mins[b * 16 + js] = s0 >> 4;
+            mins[b * 16 + js + 4] = s1 >> 4;
         }
-        y[208] = x[80];
-        y[209] = x[81];
-        dmins[b] = (uint16_t)(x[82] | (x[83] << 8));
-    } else {
-        for (int i = 16; i < 80; i++) x[i] = 0;
-        for (int e = 0; e < 256; e++) {
-            const int half = e / 128, r = e % 128, quad = r / 32, l = r % 32;
-            const int v6 = ((ql[64 * half + 32 * (quad & 1) + l] >> (4 * (quad >> 1))) & 0xF) | (((qh[32 * half + l] >> (2 * quad)) & 3) << 4);
-            qs[32 * half + l] |= (uint8_t)(((v6 - 32) & 3) << (2 * quad));
+        if (u == 0) {
+            d[b] = *(const uint16_t *)(x + D);
+            if (!Q3) dmins[b] = *(const uint16_t *)(x + D + 2);
         }
-        for (int j = 0; j < 16; j++) sc2[j] = (uint8_t)((sc6[j] & 0xF) | (mb[j] << 4));
-        x[80] = y[208];
-        x[81] = y[209];
-        x[82] = (uint8_t)(dmins[b] & 0xff);
-        x[83] = (uint8_t)(dmins[b] >> 8);
+        return;
+    }
+    uint32_t lo[4], hi[4];
+    if (t == 0) {
+        // qs[32h + 16i ..]: the units t = 0 (quarters 0 and 2) and t = 1 (1 and 3)
+        uint32_t q[4], lo1[4], hi1[4];
+        q6_unit(ql, qh, b, u, lo, hi);
+        q6_unit(ql, qh, b, u + 2, lo1, hi1);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            q[i] = ((lo[i] - OFF) & 0x03030303u) | (((lo1[i] - OFF) & 0x03030303u) << 2) | (((hi[i] - OFF) & 0x03030303u) << 4) |
+                   (((hi1[i] - OFF) & 0x03030303u) << 6);
+        store16(x + QS + 32 * h + 16 * i16, q);
+    } else if (Q3 && h == 0) {
+        uint32_t m[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int v = 0; v < 4; v++) {   // the units of both halves and quarters with this i: bits 4h + t and 4h + t + 2
+            q6_unit(ql, qh, b, 2 * v + i16, lo, hi);
+            const int bit = 4 * (v >> 1) + (v & 1);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                m[i] |= ((((lo[i] - OFF) >> 2) & 0x01010101u) << bit) | ((((hi[i] - OFF) >> 2) & 0x01010101u) << (bit + 2));
+        }
+        store16(x + 16 * i16, m);
+    } else if (u == 6) {   // h = 1, t = 1, i = 0: the scales (sc' holds group js = u + 4h at 2u and js + 4 at 2u + 1)
+        uint8_t s[16];
+#pragma unroll
+        for (int v = 0; v < 8; v++) {
+            s[v + 4 * (v >> 2)] = sc[b * 16 + 2 * v];
+            s[v + 4 * (v >> 2) + 4] = sc[b * 16 + 2 * v + 1];
+        }
+        if (Q3) {
+            uint8_t o[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const int lv = (int)(int8_t)s[j] + 32;
+                o[j & 7] |= (uint8_t)((lv & 0xF) << (j < 8 ? 0 : 4));
+                o[8 + j % 4] |= (uint8_t)((lv >> 4) << (2 * (j / 4)));
+            }
+#pragma unroll
+            for (int j = 0; j < 12; j++) x[96 + j] = o[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; j++) x[j] = (uint8_t)((s[j] & 0xF) | (mins[b * 16 + j] << 4));
+        }
+    } else if (u == 7) {
+        *(uint16_t *)(x + D) = d[b];
+        if (!Q3) *(uint16_t *)(x + D + 2) = dmins[b];
     }
 }
 
@@ -366,7 +408,18 @@ hipError_t launch(const cq_weight *w, uint8_t *aos, bool inverse, hipStream_t s)
     const int64_t nblocks = w->n * (w->k / bs);
     if (nblocks == 0) return hipSuccess;
     const int threads = 256;
-    switch (w->dtype) {
+    const unsigned per_block = (unsigned)((nblocks + threads - 1) / threads), per_unit = (unsigned)((nblocks * 8 + threads - 1) / threads);
+    uint16_t *p1 = (uint16_t *)w->p1, *p2 = (uint16_t *)w->p2, *p3 = (uint16_t *)w->p3, *p5 = (uint16_t *)w->p5;
+    switch (w->ggml_dtype) {
+    case CQ_DTYPE_Q5_0: held_in_q8_0<CQ_DTYPE_Q5_0><<<per_block, threads, 0, s>>>(aos, w->p0, p1, p2, nblocks, inverse); break;
+    case CQ_DTYPE_Q4_1: held_in_q8_0<CQ_DTYPE_Q4_1><<<per_block, threads, 0, s>>>(aos, w->p0, p1, p2, nblocks, inverse); break;
+    case CQ_DTYPE_Q5_1: held_in_q8_0<CQ_DTYPE_Q5_1><<<per_block, threads, 0, s>>>(aos, w->p0, p1, p2, nblocks, inverse); break;
+    case CQ_DTYPE_Q3K:
+        held_in_q6k<CQ_DTYPE_Q3K><<<per_unit, threads, 0, s>>>(aos, w->p0, w->p1, w->p2, p3, w->p4, p5, nblocks, inverse);
+        break;
+    case CQ_DTYPE_Q2K:
+        held_in_q6k<CQ_DTYPE_Q2K><<<per_unit, threads, 0, s>>>(aos, w->p0, w->p1, w->p2, p3, w->p4, p5, nblocks, inverse);
+        break;
     case CQ_DTYPE_Q4_0: {
         unsigned grid = (unsigned)((nblocks + threads - 1) / threads);
         repack_q4_0<<<grid, threads, 0, s>>>(aos, w->p0, (uint16_t *)w->p1, nblocks, inverse);
@@ -405,23 +458,4 @@ hipError_t cq_launch_repack(const cq_weight *w, const uint8_t *aos_dev, hipStrea
 }
 hipError_t cq_launch_unpack(const cq_weight *w, uint8_t *aos_dev, hipStream_t s) {
     return launch(w, aos_dev, true, s);
-}
-
-// GGML blocks of type `ggml_dtype` <-> GGML blocks of the type whose planes hold them (cq_storage_dtype).
-hipError_t cq_launch_transcode(const cq_weight *w, uint8_t *ggml_aos_dev, uint8_t *storage_aos_dev, int64_t nblocks, bool inverse,
-                               hipStream_t s) {
-    const int ggml_dtype = w->ggml_dtype;
-    uint16_t *min_plane = (uint16_t *)w->p2;
-    if (nblocks == 0) return hipSuccess;
-    const int threads = 128;
-    const unsigned grid = (unsigned)((nblocks + threads - 1) / threads);
-    switch (ggml_dtype) {
-    case CQ_DTYPE_Q5_0: transcode_q5_0_q8_0<<<grid, threads, 0, s>>>(ggml_aos_dev, storage_aos_dev, nblocks, inverse); break;
-    case CQ_DTYPE_Q4_1: transcode_q4_1_q8_0<false><<<grid, threads, 0, s>>>(ggml_aos_dev, storage_aos_dev, min_plane, nblocks, inverse); break;
-    case CQ_DTYPE_Q5_1: transcode_q4_1_q8_0<true><<<grid, threads, 0, s>>>(ggml_aos_dev, storage_aos_dev, min_plane, nblocks, inverse); break;
-    case CQ_DTYPE_Q3K: transcode_q3k_q6k<<<grid, threads, 0, s>>>(ggml_aos_dev, storage_aos_dev, nblocks, inverse); break;
-    case CQ_DTYPE_Q2K: transcode_q2k_q6k<<<grid, threads, 0, s>>>(ggml_aos_dev, storage_aos_dev, w->p4, (uint16_t *)w->p5, nblocks, inverse); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
 }
