@@ -517,8 +517,9 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     // kernel is as fast or faster, it has no per-block scaling of MFMA results to do - where it takes the rows)
     const bool rows_fused = flags == 0 && pre.kind == CQ_PRE_NONE && !in_place && cq_matvec_fused_rows_supported(w, m);
     const int64_t skinny_from = w->dtype == CQ_DTYPE_Q8_0 ? 4 : w->dtype == CQ_DTYPE_Q4_0 ? 5 : 2;
-    const bool has_tile_kernel = cq_gemm_supported(w, m, act);
-    const bool has_tile32 = m > 16 && cq_gemm32_supported(w, act);
+    // (weights of 33 to 127 rows that are no whole number of 32-row tiles stay with the split-K kernel)
+    const bool has_tile_kernel = cq_gemm_supported(w, m, act) || (w->n >= 128 && cq_gemm_takes(w, act));
+    const bool has_tile32 = m > 16 && (cq_gemm32_supported(w, act) || (w->n >= 128 && cq_gemm32_takes(w, act)));
     const bool skinny_rows = m <= 16 || (m <= 24 && w->n < 14336) || (m <= 32 && w->n < 12288) ||
                              (m <= 64 && w->n < 8192 && w->k <= 6144);
     if (flags & CQ_FLAG_FORCE_SKINNY) {
@@ -527,18 +528,18 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
                                 w->dtype, act, (long long)w->n);
         path = kSkinny;
     } else if (!(flags & CQ_FLAG_FORCE_MATVEC) && has_tile32) {
-        // Q8_0 / Q4_0 beyond 16 rows: their own tile kernel (whole 256-element K steps, n a multiple of 32), measured
-        // ahead of the split-K kernel from 17 rows on at every shape
+        // Q8_0 / Q4_0 beyond 16 rows: their own tile kernel, measured ahead of the split-K kernel from 17 rows on at every
+        // shape
         path = kGemm32;
     } else if (!(flags & (CQ_FLAG_FORCE_GEMM | CQ_FLAG_FORCE_MATVEC)) && (m >= skinny_from || (m >= 2 && !rows_fused)) &&
-               cq_skinny_supported(w, act) && (skinny_rows || !has_tile_kernel)) {
+               cq_skinny_takes(w, act) && (skinny_rows || !has_tile_kernel)) {
         // (shapes the tile kernels do not take: the split-K kernel, 32 rows per pass over the weights, stays
         // ahead of the dot-product kernel, 8 rows per pass, at every row count)
         path = kSkinny;
     } else {
         bool use_gemm = false;
         if (flags & CQ_FLAG_FORCE_GEMM) {
-            if (!has_tile_kernel)
+            if (!cq_gemm_supported(w, m, act))
                 return cq_set_error(CQ_ERR_UNSUPPORTED, "no MFMA GEMM for dtype %d with activation dtype %d", w->dtype, act);
             use_gemm = true;
         } else if (!(flags & CQ_FLAG_FORCE_MATVEC)) {
@@ -767,7 +768,7 @@ static int grouped_impl(const cq_weight *const *experts, int n_experts, const fl
         float *ye = y_dev + r0 * w0->n;
         const bool use_gemm = (flags & CQ_FLAG_FORCE_GEMM) ? true
                               : (flags & CQ_FLAG_FORCE_MATVEC) ? false
-                                                               : (te > 8 && cq_gemm_supported(experts[e], te, act));
+                                                               : (te > 8 && cq_gemm_takes(experts[e], act));
         if (use_gemm) CQ_HIP_CHECK(cq_launch_gemm(experts[e], ve, act, te, ye, false, s));
         else CQ_HIP_CHECK(cq_launch_matvec(experts[e], ve, act, te, ye, s));
     }

@@ -594,8 +594,12 @@ __device__ __forceinline__ void block_step(const uint8_t *__restrict__ cur, uint
     if (TRAIL && n_ok) tiles_mac<DT, MT, SPLIT, MT, SHIFT, HALF, DUMP>(cur, g, bl, bh, dw, wmin, lane, out, dl);
 }
 
+// First row of the 32 that a wave whose share begins at row `n_own` takes: where fewer than 32 rows are left it begins
+// earlier, at row n - 32, and stores only its share (every column is contracted by itself, so nothing else changes).
+__device__ __forceinline__ int64_t last_tile(int64_t n_own, int64_t n) { return n_own + 32 <= n ? n_own : n - 32; }
+
 // ------------------------------------------------------------------ kernel ----
-// Requires n % 32 == 0 and an activation workspace with padded rows (cq_act_view::m_stride).
+// Requires n >= 32 and an activation workspace with padded rows (cq_act_view::m_stride).
 // One workgroup: activation rows [m0, m0 + 32*MT) (stored up to row m - 1) x the 256 weight rows of
 // blockIdx.x, K blocks of part blockIdx.z.
 template <int DT, int MT, bool DUMP = false, int WBUF = 1, bool ONCE = false>
@@ -608,8 +612,9 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, col = lane & 31;
     const int64_t kb = w.k >> 8;
-    const int64_t n_tile = ((int64_t)blockIdx.x * kWaves + wave) * 32;
-    const bool n_ok = n_tile < w.n;   // wave-uniform; a wave past the last row only helps with the copies
+    const int64_t n_own = ((int64_t)blockIdx.x * kWaves + wave) * 32;
+    const bool n_ok = n_own < w.n;   // wave-uniform; a wave past the last row only helps with the copies
+    const int64_t n_tile = last_tile(n_own, w.n);
     const int64_t n = n_tile + col;
     const int64_t nc = n_ok ? n : 0;
     // this workgroup's range of K blocks
@@ -689,7 +694,7 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                if (row < m) {
+                if (row < m && n >= n_own) {
                     if (ksplit == 1) y[row * w.n + n] = out[t][i];
                     else unsafeAtomicAdd(&y[row * w.n + n], out[t][i]);
                 }
@@ -761,7 +766,7 @@ __device__ __forceinline__ void block_step_kh(const uint8_t *__restrict__ cur, u
     if (TRAIL && work) tiles_mac<DT, MT, SPLIT, MT, SHIFT, false, false>(cur, g, bl, bh, dw, wmin, lane, out, dl);
 }
 
-// Requires n % 32 == 0.  One workgroup: activation rows [m0, m0 + 32*MT) x the 128 weight rows of blockIdx.x, all K.
+// Requires n >= 32.  One workgroup: activation rows [m0, m0 + 32*MT) x the 128 weight rows of blockIdx.x, all K.
 template <int DT, int MT>
 __global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y) {
     typedef Tile<DT, MT> T;
@@ -773,8 +778,9 @@ __global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_v
     const int colw = wave & 3, half = wave >> 2;
     const int h = lane >> 5, col = lane & 31;
     const int64_t kb = w.k >> 8;
-    const int64_t n_tile = ((int64_t)blockIdx.x * (kWaves / 2) + colw) * 32;
-    const bool n_ok = n_tile < w.n;
+    const int64_t n_own = ((int64_t)blockIdx.x * (kWaves / 2) + colw) * 32;
+    const bool n_ok = n_own < w.n;
+    const int64_t n_tile = last_tile(n_own, w.n);
     const int64_t n = n_tile + col;
     const int64_t nc = n_ok ? n : 0;
     const int64_t nh = (kb + 1) / 2;                        // steps; the first half has nh blocks, the second kb - nh
@@ -832,7 +838,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_v
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                if (row < m) y[row * w.n + n] = out[t][i] + part[(t * 16 + i) * 64 + lane];
+                if (row < m && n >= n_own) y[row * w.n + n] = out[t][i] + part[(t * 16 + i) * 64 + lane];
             }
         }
     }
@@ -1248,7 +1254,7 @@ hipError_t launch_q81_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y,
 }  // namespace
 
 bool cq_gemm_grouped_supported(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
-    if (n_experts > kMaxGroupExperts || !cq_gemm_supported(experts[0], 0, act_dtype)) return false;
+    if (n_experts > kMaxGroupExperts || !cq_gemm_takes(experts[0], act_dtype)) return false;
     int64_t tiles = 0;
     for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + 31) / 32;
     return tiles <= kMaxGroupTiles;
@@ -1279,16 +1285,19 @@ bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, co
 
 bool cq_gemm_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }
 
-bool cq_gemm_supported(const cq_weight *w, int64_t m, int act_dtype) {
-    (void)m;
+bool cq_gemm_takes(const cq_weight *w, int act_dtype) {
     // the copies address rows with 32-bit offsets: 8 rows of activations, 16 rows of a weight plane
     return (w->dtype == CQ_DTYPE_Q4K || w->dtype == CQ_DTYPE_Q5K || w->dtype == CQ_DTYPE_Q6K) && act_dtype == CQ_DTYPE_Q8K && w->k >= 256 &&
-           w->k <= (1 << 24) && w->n % 32 == 0;
+           w->k <= (1 << 24) && w->n >= 32;
+}
+bool cq_gemm_supported(const cq_weight *w, int64_t m, int act_dtype) {
+    (void)m;
+    return cq_gemm_takes(w, act_dtype) && w->n % 32 == 0;
 }
 
 hipError_t cq_launch_gemm(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, bool y_cleared,
                           hipStream_t s) {
-    if (!cq_gemm_supported(w, m, act_dtype)) return hipErrorNotSupported;
+    if (!cq_gemm_takes(w, act_dtype)) return hipErrorNotSupported;
     if (m == 0 || w->n == 0) return hipSuccess;
     if (a.m_stride < (m + 127) / 128 * 128) return hipErrorInvalidValue;   // rows the last tile may read
     if (w->dtype == CQ_DTYPE_Q4K) return launch_dt<CQ_DTYPE_Q4K>(w, a, m, y, y_cleared, s);

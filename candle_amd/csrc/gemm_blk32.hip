@@ -29,6 +29,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef void __attribute__((address_space(3))) *lptr_t;
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));   // (rows of whole 64-element pairs of blocks)
 
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
@@ -121,7 +122,8 @@ __device__ __forceinline__ void stage_weights(uint8_t *wl, const cq_weight &w, c
 
 // DUMP (verification): the block integers are stored through `dump` instead of the result through `y`.
 // ONCE: a launch with a single row tile (up to 32 rows), which reads every weight byte once.
-template <int DT, int MT, bool DUMP, bool ONCE = false>
+// SHORT: K is no multiple of 256, the last step has fewer than eight blocks.
+template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
                                                           int ksplit, cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
@@ -129,10 +131,12 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, col = lane & 31;
-    const int64_t k = w.k, ks = k >> 8;                 // K steps of 256 elements
+    const int64_t k = w.k, ks = (k + 255) >> 8;         // K steps of 256 elements; the last one may be shorter
     const int64_t m0 = (int64_t)blockIdx.y * (MT * 32);
-    const int64_t n_tile = ((int64_t)blockIdx.x * kWaves + wave) * 32;
-    const bool n_ok = n_tile < w.n;                     // wave-uniform; a wave past the last row only helps with the copies
+    const int64_t n_own = ((int64_t)blockIdx.x * kWaves + wave) * 32;
+    const bool n_ok = n_own < w.n;                      // wave-uniform; a wave past the last row only helps with the copies
+    // fewer than 32 rows left: the tile begins earlier, at row n - 32, and only the wave's own share is stored
+    const int64_t n_tile = n_own + 32 <= w.n ? n_own : w.n - 32;
     const int64_t n = n_tile + col;
     const int64_t nc = n_ok ? n : 0;
     const int64_t b0 = ks * blockIdx.z / ksplit, b1 = ks * (blockIdx.z + 1) / ksplit;
@@ -148,7 +152,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
 
     stage_acts<DT, MT>(smem, a, g, k, m0, b0, wave);
     if (n_ok) stage_weights<DT, ONCE>(wl, w, g, n_tile, b0);
-    uint4 dnext = *(const uint4 *)(dplane + nc * (k >> 5) + b0 * 8);
+    u32x4_a4 dnext = *(const u32x4_a4 *)(dplane + nc * (k >> 5) + b0 * 8);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
@@ -175,18 +179,21 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
                     }
                 }
             }
-            const uint4 dcur = dnext;
+            const u32x4_a4 dcur = dnext;
             if (more) {
                 stage_weights<DT, ONCE>(wl, w, g, n_tile, b + 1);
-                dnext = *(const uint4 *)(dplane + nc * (k >> 5) + (b + 1) * 8);
+                dnext = *(const u32x4_a4 *)(dplane + nc * (k >> 5) + (b + 1) * 8);
             }
             // scale operand of block s: dw = b1 + b2 (bf16 pieces, exact: an f16 has 11 significant bits); lanes
             // 0..31 carry b1 in K-slots 0..2, lanes 32..63 carry b2 in K-slots 8..10, the other slots zero
+            // A last step of fewer than eight blocks: what follows the rows in memory (other rows, other planes) was copied
+            // with them, and both scales of the blocks that do not exist are zero.
+            const int nv = (int)((k >> 5) - b * 8);
             const uint32_t dwords[4] = {dcur.x, dcur.y, dcur.z, dcur.w};
             v8bf dw[8];
 #pragma unroll
             for (int s = 0; s < 8; s++) {
-                const float f = cq_h2f((uint16_t)((dwords[s >> 1] >> (16 * (s & 1))) & 0xffffu));
+                const float f = !SHORT || s < nv ? cq_h2f((uint16_t)((dwords[s >> 1] >> (16 * (s & 1))) & 0xffffu)) : 0.0f;
                 const uint32_t fb = __float_as_uint(f);
                 const float b2 = f - __uint_as_float(fb & 0xffff0000u);
                 const uint32_t piece = h == 0 ? fb >> 16 : __float_as_uint(b2) >> 16;
@@ -204,7 +211,8 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
             // waits for the read it has just issued
             auto d8raw = [&](int q) -> float {
                 const int t = q >> 3, s = q & 7;
-                return *(const float *)(cur + T::oD8 + (t * 32 + col) * 32 + s * 4);
+                const float v = *(const float *)(cur + T::oD8 + (t * 32 + col) * 32 + s * 4);
+                return !SHORT || s < nv ? v : 0.0f;
             };
             auto d8frag = [&](float v) -> v8bf {
                 // v = a1 + a2 + a3, each the leading eight bits of what the pieces before it leave (exact);
@@ -238,7 +246,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
                     const int p = (q - 1) & 1, t = (q - 1) >> 3;
 #pragma unroll
                     for (int i = 0; i < 16; i++) {
-                        if (DUMP) {
+                        if (DUMP) {   // (whole K steps only)
                             const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
                             if (row < m) dump.i[(row * w.n + n) * (k >> 5) + b * 8 + ((q - 1) & 7)] = acc[p][i];
                         } else {
@@ -259,7 +267,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                if (row < m) {
+                if (row < m && n >= n_own) {
                     if (ksplit == 1) y[row * w.n + n] = out[t][i];
                     else unsafeAtomicAdd(&y[row * w.n + n], out[t][i]);
                 }
@@ -289,7 +297,7 @@ struct Plan {
     int mt, ksplit;
 };
 Plan pick_plan(const cq_weight *w, int64_t m) {
-    const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks_total = w->k >> 8, cus = num_cus();
+    const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks_total = (w->k + 255) >> 8, cus = num_cus();
     const double atomic_pass = (double)m * (double)w->n * 4.0 / 1.1e6 * 16.0;   // bytes / (1.1e6 bytes per us) in units
     Plan best{1, 1};
     double best_cost = 0.0;
@@ -314,29 +322,36 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
 }
 
 // DUMP: the same launch (tile height, K split) storing the block integers through `d`; y is not touched.
+template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
+hipError_t launch_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, int ksplit, cq_mfma_dump d, hipStream_t s) {
+    const size_t lds = Tile<DT, MT>::kTotal;
+    if (hipError_t e = cq_ensure_lds<gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>>(w->dev, lds); e != hipSuccess) return e;
+    const dim3 grid((unsigned)((w->n + kWaves * 32 - 1) / (kWaves * 32)), (unsigned)((m + MT * 32 - 1) / (MT * 32)), (unsigned)ksplit);
+    CQ_LAUNCH((gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, d);
+    return hipGetLastError();
+}
 template <int DT, int MT, bool DUMP>
 hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int ksplit, bool y_cleared, cq_mfma_dump d,
                      hipStream_t s) {
-    const size_t lds = Tile<DT, MT>::kTotal;
-    if (hipError_t e = cq_ensure_lds<gemm32_kernel<DT, MT, DUMP>>(w->dev, lds); e != hipSuccess) return e;
-    const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), gy = (m + MT * 32 - 1) / (MT * 32);
-    if (!DUMP && ksplit > 1 && !y_cleared) {
-        hipError_t e = cq_launch_fill_zero(y, m * w->n, s);
-        if (e != hipSuccess) return e;
-    }
-    dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)ksplit);
-    if constexpr (MT == 1 && !DUMP) {
-        // a single row tile over 40 MB of weights and more: the copies marked non-temporal (measured at 17 and 32 rows:
-        // 3-7 % faster from there on, 3-5 % slower below)
-        const int64_t plane = DT == CQ_DTYPE_Q8_0 ? w->n * w->k : w->n * w->k / 2;
-        if (gy == 1 && plane >= 40000000) {
-            if (hipError_t e = cq_ensure_lds<gemm32_kernel<DT, 1, false, true>>(w->dev, lds); e != hipSuccess) return e;
-            CQ_LAUNCH((gemm32_kernel<DT, 1, false, true>), grid, kThreads, lds, s, *w, a, m, y, ksplit, d);
-            return hipGetLastError();
+    if constexpr (DUMP) {
+        return launch_inst<DT, MT, true, false, false>(w, a, m, y, ksplit, d, s);   // (whole K steps only)
+    } else {
+        if (ksplit > 1 && !y_cleared) {
+            hipError_t e = cq_launch_fill_zero(y, m * w->n, s);
+            if (e != hipSuccess) return e;
         }
+        const bool whole = w->k % 256 == 0;
+        if constexpr (MT == 1) {
+            // a single row tile over 40 MB of weights and more: the copies marked non-temporal (measured at 17 and 32 rows:
+            // 3-7 % faster from there on, 3-5 % slower below)
+            const int64_t plane = DT == CQ_DTYPE_Q8_0 ? w->n * w->k : w->n * w->k / 2;
+            if (m <= 32 && plane >= 40000000)
+                return whole ? launch_inst<DT, 1, false, true, false>(w, a, m, y, ksplit, d, s)
+                             : launch_inst<DT, 1, false, true, true>(w, a, m, y, ksplit, d, s);
+        }
+        return whole ? launch_inst<DT, MT, false, false, false>(w, a, m, y, ksplit, d, s)
+                     : launch_inst<DT, MT, false, false, true>(w, a, m, y, ksplit, d, s);
     }
-    CQ_LAUNCH((gemm32_kernel<DT, MT, DUMP>), grid, kThreads, lds, s, *w, a, m, y, ksplit, d);
-    return hipGetLastError();
 }
 
 template <int DT, bool DUMP>
@@ -349,17 +364,21 @@ hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, boo
 
 }  // namespace
 
-bool cq_gemm32_supported(const cq_weight *w, int act_dtype) {
-    // whole 256-element K steps; the copies address 8 rows with 32-bit offsets
+bool cq_gemm32_takes(const cq_weight *w, int act_dtype) {
+    // an even number of blocks per row, so that every row's scales begin on four bytes; the copies address 8 rows with 32-bit
+    // offsets and may read up to 255 bytes past a plane's last row (weight planes: CQ_TAIL_PAD, activations: the next plane)
     return (w->dtype == CQ_DTYPE_Q8_0 || w->dtype == CQ_DTYPE_Q4_0) && act_dtype == CQ_DTYPE_Q8_0 && w->k >= 256 &&
-           w->k % 256 == 0 && w->k <= (1 << 24) && w->n % 32 == 0 && w->n > 0;
+           w->k % 64 == 0 && w->k <= (1 << 24) && w->n >= 32;
+}
+bool cq_gemm32_supported(const cq_weight *w, int act_dtype) {
+    return cq_gemm32_takes(w, act_dtype) && w->k % 256 == 0 && w->n % 32 == 0;
 }
 
 bool cq_gemm32_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }
 
 hipError_t cq_launch_gemm32(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, bool y_cleared,
                             hipStream_t s) {
-    if (!cq_gemm32_supported(w, act_dtype)) return hipErrorNotSupported;
+    if (!cq_gemm32_takes(w, act_dtype)) return hipErrorNotSupported;
     if (m == 0) return hipSuccess;
     if (a.m_stride < (m <= 32 ? 32 : (m + 127) / 128 * 128)) return hipErrorInvalidValue;   // rows the last tile may read
     const cq_mfma_dump none{nullptr, nullptr};

@@ -178,7 +178,10 @@ struct cq_mfma_dump {
 hipError_t cq_launch_gemm_dump(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, cq_mfma_dump d, hipStream_t s);
 hipError_t cq_launch_gemm32_dump(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, cq_mfma_dump d, hipStream_t s);
 hipError_t cq_launch_skinny_dump(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, cq_mfma_dump d, hipStream_t s);
+// The matrix-core kernels come with two predicates: *_takes is what the kernel computes, *_supported the shapes of whole
+// tiles (n, and K steps of 256 elements) that CQ_FLAG_FORCE_* and the integer dumps offer.
 // gemm.hip
+bool cq_gemm_takes(const cq_weight *w, int act_dtype);
 bool cq_gemm_supported(const cq_weight *w, int64_t m, int act_dtype);
 // `y_cleared`: y is already zero (a launch that splits K otherwise clears it first); *_splits_k tell
 // beforehand whether the launch will add its results atomically
@@ -190,12 +193,14 @@ bool cq_gemm_grouped_supported(const cq_weight *const *experts, int n_experts, c
 hipError_t cq_launch_gemm_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
                                   float *y, bool y_cleared, hipStream_t s);
 bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets);
-// gemm_blk32.hip: the tile kernel for Q8_0 / Q4_0 weights with Q8_0 activations (K a multiple of 256)
+// gemm_blk32.hip: the tile kernel for Q8_0 / Q4_0 weights with Q8_0 activations (K a multiple of 64)
+bool cq_gemm32_takes(const cq_weight *w, int act_dtype);
 bool cq_gemm32_supported(const cq_weight *w, int act_dtype);
 hipError_t cq_launch_gemm32(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, bool y_cleared,
                             hipStream_t s);
 bool cq_gemm32_splits_k(const cq_weight *w, int64_t m);
 // skinny.hip: a few activation rows (32 per pass) on the int8 MFMA, K split over the waves of a workgroup
+bool cq_skinny_takes(const cq_weight *w, int act_dtype);
 bool cq_skinny_supported(const cq_weight *w, int act_dtype);
 hipError_t cq_launch_skinny(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, hipStream_t s);
 // moe.hip

@@ -21,6 +21,10 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+// the same at four-byte alignment: scales of 32-element blocks in rows of no whole 256 elements
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef int v4i_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float v4f_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 typedef short ss2 __attribute__((ext_vector_type(2)));
 typedef const void __attribute__((address_space(1))) *gptr_t;
@@ -28,6 +32,10 @@ typedef void __attribute__((address_space(3))) *lptr_t;
 
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
+// First weight row of 16-row tile `t`: the last tile of an n that is no multiple of 16 begins at row n - 16, on top of the
+// tile before it (both store the same values there).
+__device__ __forceinline__ int64_t tile_row(int64_t t, int64_t n) { return t * 16 + 16 <= n ? t * 16 : n - 16; }
+
 constexpr int kMaxLds = 160 * 1024;   // LDS of a CU, which a single workgroup may take
 
 // both 16-bit halves of `a` times `b` (a splat: the packed instruction takes one half of its operand twice)
@@ -182,7 +190,7 @@ __device__ __forceinline__ void block_unpack(const uint8_t *wl, int lane, const 
 }
 
 // RT = groups of eight activation rows held (rows m0 .. m0 + 8*RT - 1; the workspace pads rows, so
-// whole groups can be copied); results are stored for rows < m.  Requires n % 16 == 0.
+// whole groups can be copied); results are stored for rows < m.  Requires n >= 16.
 // DUMP (verification): the block integers, and the min term as the f16 MFMA delivers it from a zero accumulator,
 // are stored through `dump` instead of the result through `y`.
 template <int DT, int RT, bool DUMP>
@@ -197,7 +205,7 @@ __global__ void __launch_bounds__(kThreads) skinny_kernel(cq_weight w, cq_act_vi
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
     const int64_t k = w.k, kb = w.k >> 8;
-    const int64_t n_tile = (int64_t)blockIdx.x * 16;
+    const int64_t n_tile = tile_row(blockIdx.x, w.n);
     uint8_t *buf = smem + wave * B::kBytes;
 
     // copy offsets: 8 rows x 128 B per instruction, chunks swizzled by the row
@@ -427,8 +435,8 @@ __device__ __forceinline__ void res_block(const uint8_t *__restrict__ wl, const 
     res_mac<DT, RT, NT, DUMP>(act, lane, o, a_col, out, dump, at, rs, m);
 }
 
-// m <= 8 * RT activation rows (the workspace pads rows, so whole groups are copied); n % 16 == 0; at most
-// kMaxBpw K blocks per wave.  `tiles` = n / 16, dealt to the gridDim.x workgroups in turn.
+// m <= 8 * RT activation rows (the workspace pads rows, so whole groups are copied); n >= 16; at most
+// kMaxBpw K blocks per wave.  `tiles` of 16 rows, dealt to the gridDim.x workgroups in turn.
 constexpr int kMaxBpw = 4;
 template <int DT, int RT, int kWaves, int NBUF, bool DUMP>
 __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight w, cq_act_view a, int64_t m,
@@ -441,7 +449,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
     const int64_t k = w.k, kb = w.k >> 8;
-    const int64_t tiles = w.n / 16;
+    const int64_t tiles = (w.n + 15) / 16;
     uint8_t *wgt_base = smem + kb * R::kActBlk;
 
     const uint32_t r8 = lane >> 3, c8 = lane & 7;
@@ -473,7 +481,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
 #pragma unroll
     for (int j = 0; j < kMaxBpw; j++) {
         const int64_t b = wave + (int64_t)j * kWaves;
-        if (b < kb && tile < tiles) load_head(w, (tile * 16 + r) * kb + b, head[j]);
+        if (b < kb && tile < tiles) load_head(w, (tile_row(tile, w.n) + r) * kb + b, head[j]);
     }
 #pragma unroll
     for (int j = 0; j < kMaxBpw; j++) {
@@ -488,19 +496,19 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
             if (lane < 8 * RT) dma4s(pl.ad, lane * 4u, b * mstr * 4u, act + R::oD8);
             if (MINS && lane < 16 * RT) dma16s(pl.am, lane * 16u, b * mstr * 32u, act + R::oMin);
             if (tile < tiles)
-                res_issue_weights<DT>(wgt_base + (b * NBUF) * R::kWgt, pl, (uint32_t)tile * 16u, b, kb32, wq_off, wh_off, w5_off, lane);
+                res_issue_weights<DT>(wgt_base + (b * NBUF) * R::kWgt, pl, (uint32_t)tile_row(tile, w.n), b, kb32, wq_off, wh_off, w5_off, lane);
         }
     }
     int par = 0;
     for (; tile < tiles; tile += gridDim.x) {
-        const int64_t n_tile = tile * 16, next = tile + gridDim.x;
+        const int64_t n_tile = tile_row(tile, w.n), next = tile + gridDim.x;
         __builtin_amdgcn_s_waitcnt(0);   // this tile's weights (and, the first time, the activations) have landed
         if (NBUF == 2 && next < tiles) {
 #pragma unroll
             for (int j = 0; j < kMaxBpw; j++) {
                 const int64_t b = wave + (int64_t)j * kWaves;
                 if (b < kb)
-                    res_issue_weights<DT>(wgt_base + (b * NBUF + (par ^ 1)) * R::kWgt, pl, (uint32_t)next * 16u, (uint32_t)b, kb32,
+                    res_issue_weights<DT>(wgt_base + (b * NBUF + (par ^ 1)) * R::kWgt, pl, (uint32_t)tile_row(next, w.n), (uint32_t)b, kb32,
                                           wq_off, wh_off, w5_off, lane);
             }
         }
@@ -541,7 +549,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
             for (int j = 0; j < kMaxBpw; j++) {
                 const int64_t b = wave + (int64_t)j * kWaves;
                 if (b < kb)
-                    res_issue_weights<DT>(wgt_base + b * R::kWgt, pl, (uint32_t)next * 16u, (uint32_t)b, kb32, wq_off, wh_off, w5_off, lane);
+                    res_issue_weights<DT>(wgt_base + b * R::kWgt, pl, (uint32_t)tile_row(next, w.n), (uint32_t)b, kb32, wq_off, wh_off, w5_off, lane);
             }
         } else if (NBUF == 2) {
             __syncthreads();   // ... before the tile after the next one is copied over them
@@ -550,7 +558,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
 #pragma unroll
             for (int j = 0; j < kMaxBpw; j++) {
                 const int64_t b = wave + (int64_t)j * kWaves;
-                if (b < kb) load_head(w, (next * 16 + r) * kb + b, head[j]);
+                if (b < kb) load_head(w, (tile_row(next, w.n) + r) * kb + b, head[j]);
             }
         }
         par ^= 1;
@@ -595,7 +603,7 @@ __device__ __forceinline__ void multi_issue(uint8_t *__restrict__ slot, const Re
 // One tile of one wave: operands out of `slot`, then (the slot is free) the copies of the tile two ahead, then the MFMAs.
 template <int DT, int RT, bool DUMP>
 __device__ __forceinline__ void multi_step(uint8_t *__restrict__ slot, const uint8_t *__restrict__ act, int lane, const ResPlanes &pl,
-                                           __amdgpu_buffer_rsrc_t hdr, bool ahead, uint32_t tile_ahead, uint32_t b, uint32_t kb32,
+                                           __amdgpu_buffer_rsrc_t hdr, bool ahead, uint32_t rows_ahead, uint32_t b, uint32_t kb32,
                                            uint32_t wq_off, uint32_t w5_off, uint32_t hd_off, const uint32_t (&a_col)[1][2],
                                            v4f (&out)[1], const cq_mfma_dump &dump, int64_t at, int64_t rs, int64_t m) {
     typedef ResMulti<DT, RT> M;
@@ -608,12 +616,12 @@ __device__ __forceinline__ void multi_step(uint8_t *__restrict__ slot, const uin
     res_unpack<DT, DUMP>(slot, lane, head, dump, o);
     if (ahead) {
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the reads above are done with the slot
-        multi_issue<DT, RT>(slot, pl, hdr, tile_ahead * 16u, b, kb32, wq_off, w5_off, hd_off, lane);
+        multi_issue<DT, RT>(slot, pl, hdr, rows_ahead, b, kb32, wq_off, w5_off, hd_off, lane);
     }
     res_mac<DT, RT, 1, DUMP>(act, lane, o, a_col, out, dump, at, rs, m);
 }
 
-// m <= 8 * RT <= 16 activation rows; n % 16 == 0; k / 256 <= kWaves.
+// m <= 8 * RT <= 16 activation rows; n >= 16; k / 256 <= kWaves.
 template <int DT, int RT, int kWaves, bool DUMP>
 __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_weight w, cq_act_view a, int64_t m,
                                                                             float *__restrict__ y, cq_mfma_dump dump) {
@@ -629,7 +637,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
     const int64_t k = w.k, kb = w.k >> 8;
-    const int64_t tiles = w.n / 16, G = gridDim.x;
+    const int64_t tiles = (w.n + 15) / 16, G = gridDim.x;
     uint8_t *wgt_base = smem + kb * R::kActBlk;
     const bool has = wave < kb;   // this wave owns K block `wave`
     const uint32_t b = (uint32_t)wave;
@@ -673,8 +681,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
         cnt = cnt < kTilesPerRound ? cnt : kTilesPerRound;
         if (has) {
             v4f o0 = {0.0f, 0.0f, 0.0f, 0.0f}, o1 = o0, o2 = o0, o3 = o0;
-            multi_issue<DT, RT>(ring, pl, hdr, (uint32_t)t0 * 16u, b, kb32, wq_off, w5_off, hd_off, lane);
-            if (cnt > 1) multi_issue<DT, RT>(ring + M::kSlot, pl, hdr, (uint32_t)(t0 + G) * 16u, b, kb32, wq_off, w5_off, hd_off, lane);
+            multi_issue<DT, RT>(ring, pl, hdr, (uint32_t)tile_row(t0, w.n), b, kb32, wq_off, w5_off, hd_off, lane);
+            if (cnt > 1) multi_issue<DT, RT>(ring + M::kSlot, pl, hdr, (uint32_t)tile_row(t0 + G, w.n), b, kb32, wq_off, w5_off, hd_off, lane);
 #pragma nounroll
             for (int i = 0; i < cnt; i++) {
                 // everything but the copies of the next tile has landed
@@ -682,8 +690,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
                 else __builtin_amdgcn_s_waitcnt(0x0F70);
                 const int64_t tile = t0 + i * G;
                 v4f acc[1] = {{0.0f, 0.0f, 0.0f, 0.0f}};
-                multi_step<DT, RT, DUMP>(ring + (i & 1) * M::kSlot, act, lane, pl, hdr, i + 2 < cnt, (uint32_t)(tile + 2 * G), b, kb32,
-                                         wq_off, w5_off, hd_off, a_col, acc, dump, (tile * 16 + r) * kb + b, w.n * kb, m);
+                multi_step<DT, RT, DUMP>(ring + (i & 1) * M::kSlot, act, lane, pl, hdr, i + 2 < cnt, (uint32_t)tile_row(tile + 2 * G, w.n), b, kb32,
+                                         wq_off, w5_off, hd_off, a_col, acc, dump, (tile_row(tile, w.n) + r) * kb + b, w.n * kb, m);
                 // (i is wave-uniform: real branches, four moves, instead of sixteen selects - the empty statements keep them)
                 if (i == 0) { o0 = acc[0]; asm volatile(""); }
                 else if (i == 1) { o1 = acc[0]; asm volatile(""); }
@@ -704,7 +712,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
                 const v4f p = *(const v4f *)(wgt_base + (size_t)o * 2 * M::kSlot + wave * 1024 + lane * 16);
                 s += p;
             }
-            const int64_t col = (t0 + wave * G) * 16 + r;
+            const int64_t col = tile_row(t0 + wave * G, w.n) + r;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int64_t row = kq * 4 + i;
@@ -730,6 +738,19 @@ template <int RT> struct BufQ8 {
     static constexpr int kBytes = kRaw;   // >= 2 KiB of partial results
 };
 
+// The eight blocks of a 256-element step, or the `left` that a row ends with (left is wave-uniform; the copies of such a step
+// also bring in what follows the row in memory, which nothing reads).
+template <typename F> __device__ __forceinline__ void each_block(int64_t left, F block) {
+    if (left >= 8) {
+#pragma unroll
+        for (int b = 0; b < 8; b++) block(b);
+    } else {
+#pragma unroll
+        for (int b = 0; b < 7; b++)
+            if (b < left) block(b);
+    }
+}
+
 template <int DT, int RT, bool DUMP>
 __global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m,
                                                                 float *__restrict__ y, cq_mfma_dump dump) {
@@ -740,8 +761,8 @@ __global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
-    const int64_t k = w.k, kg = w.k >> 8, kb = w.k >> 5;
-    const int64_t n_tile = (int64_t)blockIdx.x * 16;
+    const int64_t k = w.k, kg = (w.k + 255) >> 8, kb = w.k >> 5;
+    const int64_t n_tile = tile_row(blockIdx.x, w.n);
     uint8_t *buf = smem + wave * B::kBytes;
 
     // copy offsets: 8 rows x 128 B per instruction, chunks swizzled by the row
@@ -789,18 +810,18 @@ __global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_
             dma16(a.qs + (m0 + rg * 8) * k + g * 256 + kh * 128, row_off, buf + B::oAct + i * 1024);
         }
         // the eight block scales of this lane's weight row, and of the activation rows it scales
-        const uint4 dwv = *(const uint4 *)(w.p1 + ((n_tile + r) * kb + g * 8) * 2);
+        const u32x4_a4 dwv = *(const u32x4_a4 *)(w.p1 + ((n_tile + r) * kb + g * 8) * 2);
         v4f da[NT][4][2];
         v4i bs[Q4 ? NT : 1][4][2];   // Q4_0: the sums of the activation blocks
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const v4f *p = (const v4f *)(a.d + a_row[t][i] * kb + g * 8);
+                const v4f_a4 *p = (const v4f_a4 *)(a.d + a_row[t][i] * kb + g * 8);
                 da[t][i][0] = p[0];
                 da[t][i][1] = p[1];
                 if (Q4) {
-                    const v4i *q = (const v4i *)(a.bsum32 + a_row[t][i] * kb + g * 8);
+                    const v4i_a4 *q = (const v4i_a4 *)(a.bsum32 + a_row[t][i] * kb + g * 8);
                     bs[t][i][0] = q[0];
                     bs[t][i][1] = q[1];
                 }
@@ -808,8 +829,7 @@ __global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_
         __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
 
         const uint32_t dww[4] = {dwv.x, dwv.y, dwv.z, dwv.w};
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
+        auto block = [&](int b) {
             const float dw = cq_h2f((uint16_t)(dww[b >> 1] >> (16 * (b & 1))));
             long wv;
             if (Q4) {
@@ -834,7 +854,8 @@ __global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_
                     }
                 }
             }
-        }
+        };
+        each_block(kb - g * 8, block);
     }
     if (DUMP) return;
 
@@ -876,7 +897,7 @@ template <int DT, int RT> struct ResQ8 {
     static size_t bytes(int64_t kg) { return (size_t)kg * (kActGrp + kWgt); }
 };
 
-// m <= 8 * RT rows; n % 16 == 0, one tile per workgroup (gridDim.x == n / 16); at most kMaxBpw K groups per wave.
+// m <= 8 * RT rows; n >= 16, one 16-row tile per workgroup; at most kMaxBpw K groups per wave.
 template <int DT, int RT, int kWaves, bool DUMP>
 __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_weight w, cq_act_view a, int64_t m,
                                                                             float *__restrict__ y, cq_mfma_dump dump) {
@@ -887,8 +908,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_w
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
-    const int64_t k = w.k, kg = w.k >> 8, kb = w.k >> 5;
-    const int64_t n_tile = (int64_t)blockIdx.x * 16;
+    const int64_t k = w.k, kg = (w.k + 255) >> 8, kb = w.k >> 5;
+    const int64_t n_tile = tile_row(blockIdx.x, w.n);
     uint8_t *wgt_base = smem + kg * R::kActGrp;
 
     const uint32_t r8 = lane >> 3, c8 = lane & 7;
@@ -911,11 +932,11 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_w
     }
 
     // ---- everything this wave will need, requested at once
-    uint4 dwv[kMaxBpw];
+    u32x4_a4 dwv[kMaxBpw];
 #pragma unroll
     for (int j = 0; j < kMaxBpw; j++) {
         const int64_t g = wave + (int64_t)j * kWaves;
-        if (g < kg) dwv[j] = *(const uint4 *)(w.p1 + ((n_tile + r) * kb + g * 8) * 2);
+        if (g < kg) dwv[j] = *(const u32x4_a4 *)(w.p1 + ((n_tile + r) * kb + g * 8) * 2);
     }
 #pragma unroll
     for (int j = 0; j < kMaxBpw; j++) {
@@ -952,8 +973,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_w
         if (g < kg) {
             const uint8_t *act = smem + g * R::kActGrp, *wl = wgt_base + g * R::kWgt;
             const uint32_t dww[4] = {dwv[j].x, dwv[j].y, dwv[j].z, dwv[j].w};
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
+            auto block = [&](int b) {
                 const float dw = cq_h2f((uint16_t)(dww[b >> 1] >> (16 * (b & 1))));
                 long wv;
                 if (Q4) {
@@ -981,7 +1001,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_w
                         }
                     }
                 }
-            }
+            };
+            each_block(kb - g * 8, block);
         }
     }
     if (DUMP) return;
@@ -1045,7 +1066,7 @@ __device__ __forceinline__ void blk32_multi_issue(uint8_t *__restrict__ slot, co
 // One tile of one wave: operands out of `slot` into registers, the copies of a tile ahead into the free slot, MFMAs.
 template <int DT, int RT, bool DUMP>
 __device__ __forceinline__ void blk32_multi_step(uint8_t *__restrict__ slot, const uint8_t *__restrict__ act, int lane, const cq_weight &w,
-                                                 bool ahead, int64_t tile_ahead, int64_t g, uint32_t row_off, uint32_t q4_off,
+                                                 bool ahead, int64_t rows_ahead, int64_t g, uint32_t row_off, uint32_t q4_off,
                                                  uint32_t ws_off, uint32_t w4_col, uint32_t w4_shift, const uint32_t (&w_col)[4],
                                                  const uint32_t (&a_col)[4], v4f &out, const cq_mfma_dump &dump, int64_t at, int64_t rs,
                                                  int64_t m) {
@@ -1067,11 +1088,10 @@ __device__ __forceinline__ void blk32_multi_step(uint8_t *__restrict__ slot, con
     }
     if (ahead) {
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the reads above are done with the slot
-        blk32_multi_issue<DT, RT>(slot, w, tile_ahead * 16, g, row_off, q4_off, ws_off, lane);
+        blk32_multi_issue<DT, RT>(slot, w, rows_ahead, g, row_off, q4_off, ws_off, lane);
     }
     const uint32_t dww[4] = {dwv.x, dwv.y, dwv.z, dwv.w};
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
+    auto block = [&](int b) {
         const float dw = cq_h2f((uint16_t)(dww[b >> 1] >> (16 * (b & 1))));
         const long av = *(const long *)(act + a_col[b & 3] + (b >> 2) * 1024);
         const v4i acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, wv[b], (v4i){0, 0, 0, 0}, 0, 0, 0);
@@ -1088,10 +1108,11 @@ __device__ __forceinline__ void blk32_multi_step(uint8_t *__restrict__ slot, con
                 out[i] = __builtin_fmaf((float)I * dw, da, out[i]);
             }
         }
-    }
+    };
+    each_block((w.k >> 5) - g * 8, block);
 }
 
-// m <= 8 * RT <= 16 rows; n % 16 == 0; k / 256 <= kWaves.
+// m <= 8 * RT <= 16 rows; n >= 16; k / 256 <= kWaves.
 template <int DT, int RT, int kWaves, bool DUMP>
 __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_multi_kernel(cq_weight w, cq_act_view a, int64_t m,
                                                                          float *__restrict__ y, cq_mfma_dump dump) {
@@ -1105,8 +1126,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_multi_kernel(cq_weig
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
-    const int64_t k = w.k, kg = w.k >> 8, kb = w.k >> 5;
-    const int64_t tiles = w.n / 16, G = gridDim.x;
+    const int64_t k = w.k, kg = (w.k + 255) >> 8, kb = w.k >> 5;
+    const int64_t tiles = (w.n + 15) / 16, G = gridDim.x;
     uint8_t *wgt_base = smem + kg * R::kActGrp;
     const bool has = wave < kg;   // this wave owns K group `wave`
     const int64_t g = wave;
@@ -1145,8 +1166,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_multi_kernel(cq_weig
         cnt = cnt < kTilesPerRound ? cnt : kTilesPerRound;
         if (has) {
             v4f o0 = {0.0f, 0.0f, 0.0f, 0.0f}, o1 = o0, o2 = o0, o3 = o0;
-            blk32_multi_issue<DT, RT>(ring, w, t0 * 16, g, row_off, q4_off, ws_off, lane);
-            if (M::kSlots == 2 && cnt > 1) blk32_multi_issue<DT, RT>(ring + M::kSlot, w, (t0 + G) * 16, g, row_off, q4_off, ws_off, lane);
+            blk32_multi_issue<DT, RT>(ring, w, tile_row(t0, w.n), g, row_off, q4_off, ws_off, lane);
+            if (M::kSlots == 2 && cnt > 1) blk32_multi_issue<DT, RT>(ring + M::kSlot, w, tile_row(t0 + G, w.n), g, row_off, q4_off, ws_off, lane);
 #pragma nounroll
             for (int i = 0; i < cnt; i++) {
                 // everything but the copies of a tile in flight ahead has landed
@@ -1155,8 +1176,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_multi_kernel(cq_weig
                 const int64_t tile = t0 + i * G;
                 v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
                 blk32_multi_step<DT, RT, DUMP>(ring + (M::kSlots == 2 ? (i & 1) * M::kSlot : 0), act, lane, w, i + M::kSlots < cnt,
-                                               tile + M::kSlots * G, g, row_off, q4_off, ws_off, w4_col, w4_shift, w_col, a_col, acc, dump,
-                                               (tile * 16 + r) * kb + g * 8, w.n * kb, m);
+                                               tile_row(tile + M::kSlots * G, w.n), g, row_off, q4_off, ws_off, w4_col, w4_shift, w_col, a_col, acc, dump,
+                                               (tile_row(tile, w.n) + r) * kb + g * 8, w.n * kb, m);
                 if (i == 0) { o0 = acc; asm volatile(""); }
                 else if (i == 1) { o1 = acc; asm volatile(""); }
                 else if (i == 2) { o2 = acc; asm volatile(""); }
@@ -1175,7 +1196,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_multi_kernel(cq_weig
                 const v4f p = *(const v4f *)(wgt_base + (size_t)o * M::kSlots * M::kSlot + wave * 1024 + lane * 16);
                 s += p;
             }
-            const int64_t col = (t0 + wave * G) * 16 + r;
+            const int64_t col = tile_row(t0 + wave * G, w.n) + r;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int64_t row = kq * 4 + i;
@@ -1197,13 +1218,13 @@ hipError_t launch_blk32_multi_inst(const cq_weight *w, cq_act_view a, int64_t m,
 template <int DT, int RT, int NW, bool DUMP>
 hipError_t launch_blk32_res_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, size_t lds, cq_mfma_dump d, hipStream_t s) {
     if (hipError_t e = cq_ensure_lds<skinny_blk32_resident_kernel<DT, RT, NW, DUMP>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_blk32_resident_kernel<DT, RT, NW, DUMP>), (unsigned)(w->n / 16), NW * 64, lds, s, *w, a, m, y, d);
+    CQ_LAUNCH((skinny_blk32_resident_kernel<DT, RT, NW, DUMP>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m, y, d);
     return hipGetLastError();
 }
 // Takes the launch (true) where the resident kernel applies: one tile per workgroup, all operands in the LDS.
 template <int DT, int RT, bool DUMP>
 bool launch_blk32_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s, hipError_t *err) {
-    const int64_t kg = w->k >> 8, tiles = w->n / 16;
+    const int64_t kg = (w->k + 255) >> 8, tiles = (w->n + 15) / 16;
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (cus <= 0) cus = 256;
@@ -1239,7 +1260,7 @@ template <int DT, int RT, bool DUMP>
 hipError_t launch_blk32_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = (size_t)BufQ8<RT>::kBytes * kWaves;
     if (hipError_t e = cq_ensure_lds<skinny_blk32_kernel<DT, RT, DUMP>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_blk32_kernel<DT, RT, DUMP>), (unsigned)(w->n / 16), kThreads, lds, s, *w, a, m0, m, y, d);
+    CQ_LAUNCH((skinny_blk32_kernel<DT, RT, DUMP>), (unsigned)((w->n + 15) / 16), kThreads, lds, s, *w, a, m0, m, y, d);
     return hipGetLastError();
 }
 
@@ -1261,7 +1282,7 @@ template <int DT, int RT, bool DUMP>
 hipError_t launch_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = (size_t)Buf<DT, RT>::kBytes * kWaves;
     if (hipError_t e = cq_ensure_lds<skinny_kernel<DT, RT, DUMP>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_kernel<DT, RT, DUMP>), (unsigned)(w->n / 16), kThreads, lds, s, *w, a, m0, m, y, d);
+    CQ_LAUNCH((skinny_kernel<DT, RT, DUMP>), (unsigned)((w->n + 15) / 16), kThreads, lds, s, *w, a, m0, m, y, d);
     return hipGetLastError();
 }
 
@@ -1297,7 +1318,7 @@ hipError_t launch_multi_inst(const cq_weight *w, cq_act_view a, int64_t m, float
 }
 template <int DT, int RT, bool DUMP>
 bool launch_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s, hipError_t *err) {
-    const int64_t kb = w->k >> 8, tiles = w->n / 16;
+    const int64_t kb = w->k >> 8, tiles = (w->n + 15) / 16;
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (cus <= 0) cus = 256;
@@ -1344,7 +1365,7 @@ bool launch_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_
 
 template <bool DUMP>
 hipError_t launch_any(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    if (!cq_skinny_supported(w, act_dtype)) return hipErrorNotSupported;
+    if (!cq_skinny_takes(w, act_dtype)) return hipErrorNotSupported;
     if (m == 0) return hipSuccess;
     if (a.m_stride < (m + 31) / 32 * 32) return hipErrorInvalidValue;   // whole 8-row groups are copied
     hipError_t e = hipSuccess;
@@ -1362,11 +1383,14 @@ hipError_t launch_any(const cq_weight *w, cq_act_view a, int act_dtype, int64_t 
 
 }  // namespace
 
-bool cq_skinny_supported(const cq_weight *w, int act_dtype) {
+bool cq_skinny_takes(const cq_weight *w, int act_dtype) {
     // the copies address 8 rows of activations and 16 rows of a weight plane with 32-bit offsets
     const bool kquant = (w->dtype == CQ_DTYPE_Q4K || w->dtype == CQ_DTYPE_Q5K || w->dtype == CQ_DTYPE_Q6K) && act_dtype == CQ_DTYPE_Q8K;
-    const bool q8 = (w->dtype == CQ_DTYPE_Q8_0 || w->dtype == CQ_DTYPE_Q4_0) && act_dtype == CQ_DTYPE_Q8_0 && w->k % 256 == 0;
-    return (kquant || q8) && w->k >= 256 && w->k <= (1 << 24) && w->n % 16 == 0 && w->n > 0;
+    const bool q8 = (w->dtype == CQ_DTYPE_Q8_0 || w->dtype == CQ_DTYPE_Q4_0) && act_dtype == CQ_DTYPE_Q8_0 && w->k % 64 == 0;
+    return (kquant || q8) && w->k >= 256 && w->k <= (1 << 24) && w->n >= 16;
+}
+bool cq_skinny_supported(const cq_weight *w, int act_dtype) {
+    return cq_skinny_takes(w, act_dtype) && w->k % 256 == 0 && w->n % 16 == 0;
 }
 
 hipError_t cq_launch_skinny(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, hipStream_t s) {
