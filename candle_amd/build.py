@@ -1,4 +1,4 @@
-"""Builds libcandle_qhip.so (HIP kernels + C ABI) for gfx950 with hipcc, in-tree."""
+"""Builds libcandle_qhip.so (HIP kernels + C ABI) for gfx950 and _calls.so (qhip.py's calls in native code) with hipcc, in-tree."""
 from __future__ import annotations
 
 import os
@@ -40,16 +40,35 @@ PROBE_SOURCE = "probe.hip"
 PROBE_LIB_PATH = os.path.join(LIB_DIR, "libcandle_qhip_probe.so")
 
 
+# The native side of qhip.py's calls: a CPython module over torch's C++ tensors, host code only.
+CALLS_SOURCE = "calls.cpp"
+CALLS_PATH = os.path.join(LIB_DIR, "_calls.so")
+
+
+def _build_calls() -> None:
+    import importlib.util
+    import sysconfig
+    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    inc = [f"-I{os.path.join(torch_dir, d)}" for d in ("include", "include/torch/csrc/api/include")]
+    inc.append("-I" + os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"))
+    subprocess.check_call(["hipcc", "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                           *inc, "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, CALLS_SOURCE), "-o", CALLS_PATH,
+                           "-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip"])
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as ex:
+        calls = ex.submit(_build_calls)
         objs = list(ex.map(_compile, SOURCES + [PROBE_SOURCE]))
+        calls.result()
     probe_obj = objs.pop()
     subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs])
     subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", PROBE_LIB_PATH, probe_obj])
     if verbose:
         print("built", LIB_PATH)
         print("built", PROBE_LIB_PATH)
+        print("built", CALLS_PATH)
     return LIB_PATH
 
 

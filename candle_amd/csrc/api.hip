@@ -31,6 +31,16 @@ struct NoSplitScope {
 }  // namespace
 bool cq_no_split_k() { return g_no_split; }
 
+int cq_num_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+            return n;
+        return 256;
+    }();
+    return cus;
+}
+
 bool cq_timing_take(hipEvent_t *start, hipEvent_t *stop) {
     if (!g_timer.armed) return false;
     g_timer.armed = false;

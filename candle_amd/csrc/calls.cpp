@@ -1,0 +1,347 @@
+// The matmul-side calls of qhip.py in native code: argument checks, the result tensor, the workspace and the stream of one
+// call, then the C ABI (include/candle_qhip.h).  A decode launch of the matmul kernel takes about 5 us of device time; the
+// same steps written in Python over ctypes took 10 us of host time per call and bounded it (4096x4096 Q4K, one row, calls
+// back to back: 10.5 us), here they take about 3.
+//
+// Every function returns None where it does not take its arguments (wrong type, shape, device, layout): qhip.py then words
+// the error.  The C functions are handed over by address (`bind`), so that whichever libcandle_qhip.so qhip.py loaded is the
+// one that is called.
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/candle_qhip.h"
+
+namespace {
+
+struct Abi {
+    decltype(&cq_last_error) last_error;
+    decltype(&cq_weight_shape) weight_shape;
+    decltype(&cq_weight_device) weight_device;
+    decltype(&cq_workspace_bytes) workspace_bytes;
+    decltype(&cq_qmatmul) qmatmul;
+    decltype(&cq_qmatmul_fused) qmatmul_fused;
+    decltype(&cq_qmatmul_multi) qmatmul_multi;
+    decltype(&cq_grouped_workspace_bytes) grouped_workspace_bytes;
+    decltype(&cq_qmatmul_grouped) qmatmul_grouped;
+    decltype(&cq_qmatmul_grouped_fused) qmatmul_grouped_fused;
+    decltype(&cq_weight_dequantize) weight_dequantize;
+    decltype(&cq_weight_dequantize_f16) weight_dequantize_f16;
+} g_abi;
+PyObject *g_error = nullptr;                                             // qhip.QHipError
+PyObject *g_s_addr = nullptr, *g_s_buf = nullptr, *g_s_get = nullptr;   // "_addr", "buf", "get"
+
+constexpr int kMaxWeights = 256;   // of one multi or grouped call; more of them take the general path's error
+
+void *stream_now() { return (void *)c10::hip::getCurrentHIPStream().stream(); }
+
+PyObject *fail(int rc) {
+    PyErr_Format(g_error, "[%d] %s", rc, g_abi.last_error());
+    return nullptr;
+}
+
+// The cq_weight behind a qhip.QWeight; null (no Python error) if the object has none.
+const cq_weight *weight_of(PyObject *w) {
+    PyObject *a = PyObject_GetAttr(w, g_s_addr);
+    if (!a) {
+        PyErr_Clear();
+        return nullptr;
+    }
+    void *p = PyLong_AsVoidPtr(a);
+    Py_DECREF(a);
+    if (PyErr_Occurred()) PyErr_Clear();
+    return (const cq_weight *)p;
+}
+
+bool f32_on_device(PyObject *x) {
+    if (!THPVariable_Check(x)) return false;
+    const at::Tensor &t = THPVariable_Unpack(x);
+    return t.is_cuda() && t.scalar_type() == at::kFloat && t.is_contiguous();
+}
+
+// The operand of the fused step `pre`, with the shape rules of qhip._check_pre.
+bool aux_ok(int pre, const at::Tensor &x, PyObject *aux) {
+    if (pre == CQ_PRE_NONE) return true;
+    if (!f32_on_device(aux)) return false;
+    const at::Tensor &a = THPVariable_Unpack(aux);
+    if (pre == CQ_PRE_RMS_NORM) return a.dim() == 1 && a.size(0) == x.size(-1);
+    return pre == CQ_PRE_SILU_MUL && a.sizes() == x.sizes();
+}
+
+const float *floats_of(PyObject *t) { return t == Py_None ? nullptr : (const float *)THPVariable_Unpack(t).data_ptr(); }
+
+// At least `need` bytes on x's device out of a qhip.Workspace (which grows in Python).  A new reference to the tensor
+// in *held; the workspace object keeps it too.
+bool workspace(PyObject *ws, size_t need, const at::Tensor &x, PyObject *px, PyObject **held, void **ptr, size_t *bytes) {
+    PyObject *buf = PyObject_GetAttr(ws, g_s_buf);
+    if (!buf) return false;
+    if (buf == Py_None || (size_t)THPVariable_Unpack(buf).numel() < need || THPVariable_Unpack(buf).device() != x.device()) {
+        Py_DECREF(buf);
+        PyObject *dev = PyObject_GetAttrString(px, "device");
+        PyObject *n = PyLong_FromSize_t(need);
+        buf = dev && n ? PyObject_CallMethodObjArgs(ws, g_s_get, n, dev, nullptr) : nullptr;
+        Py_XDECREF(dev);
+        Py_XDECREF(n);
+        if (!buf) return false;
+    }
+    const at::Tensor &b = THPVariable_Unpack(buf);
+    *held = buf;
+    *ptr = b.data_ptr();
+    *bytes = (size_t)b.numel();
+    return true;
+}
+
+at::Tensor empty_f32(at::IntArrayRef sizes, c10::Device dev) { return at::Tensor(at::detail::empty_cuda(sizes, at::kFloat, dev, std::nullopt)); }
+
+// x's shape with its last dimension replaced by n
+at::Tensor result_like(const at::Tensor &x, int64_t n) {
+    c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
+    sizes.back() = n;
+    return empty_f32(sizes, x.device());
+}
+
+bool as_int(PyObject *o, int *v) {
+    const long l = PyLong_AsLong(o);
+    if (l == -1 && PyErr_Occurred()) return false;
+    *v = (int)l;
+    return true;
+}
+
+// qmatmul(w, x, flags, out, workspace, pre, aux, eps)
+PyObject *py_qmatmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 8) return PyErr_Format(PyExc_TypeError, "qmatmul takes 8 arguments");
+    int flags, pre;
+    if (!as_int(a[2], &flags) || !as_int(a[5], &pre)) return nullptr;
+    const double eps = PyFloat_AsDouble(a[7]);
+    if (eps == -1.0 && PyErr_Occurred()) return nullptr;
+    const cq_weight *w = weight_of(a[0]);
+    PyObject *px = a[1], *out = a[3], *aux = a[6];
+    if (!w || !f32_on_device(px) || (out != Py_None && !THPVariable_Check(out))) Py_RETURN_NONE;
+    const at::Tensor &x = THPVariable_Unpack(px);
+    int64_t n, k;
+    if (g_abi.weight_shape(w, &n, &k) != CQ_OK || x.dim() < 2 || x.size(-1) != k || !aux_ok(pre, x, aux)) Py_RETURN_NONE;
+    const int64_t m = k ? x.numel() / k : 0;
+    PyObject *held = nullptr;
+    void *ws;
+    size_t ws_bytes;
+    if (!workspace(a[4], g_abi.workspace_bytes(w, m, flags), x, px, &held, &ws, &ws_bytes)) return nullptr;
+    const bool mine = out == Py_None;
+    float *y = nullptr;
+    try {
+        if (mine) out = THPVariable_Wrap(result_like(x, n));
+        else Py_INCREF(out);
+        if (out) y = (float *)THPVariable_Unpack(out).data_ptr();
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        out = nullptr;
+    }
+    if (!out) {
+        Py_DECREF(held);
+        return nullptr;
+    }
+    const float *xp = (const float *)x.data_ptr(), *ap = pre == CQ_PRE_NONE ? nullptr : floats_of(aux);
+    void *s = stream_now();
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = pre == CQ_PRE_NONE ? g_abi.qmatmul(w, xp, m, y, flags, ws, ws_bytes, s)
+                            : g_abi.qmatmul_fused(w, pre, xp, ap, (float)eps, m, y, flags, ws, ws_bytes, s);
+    Py_END_ALLOW_THREADS
+    Py_DECREF(held);
+    if (rc != CQ_OK) {
+        Py_DECREF(out);
+        return fail(rc);
+    }
+    return out;
+}
+
+// The weights of a list; their number, or -1 where an element has none or there are too many.
+Py_ssize_t weights_of(PyObject *list, const cq_weight **ws) {
+    if (!PyList_Check(list)) return -1;
+    const Py_ssize_t count = PyList_GET_SIZE(list);
+    if (count < 1 || count > kMaxWeights) return -1;
+    for (Py_ssize_t i = 0; i < count; i++)
+        if (!(ws[i] = weight_of(PyList_GET_ITEM(list, i)))) return -1;
+    return count;
+}
+
+// qmatmul_multi(weights, x, flags, workspace, pre, aux, eps)
+PyObject *py_qmatmul_multi(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 7) return PyErr_Format(PyExc_TypeError, "qmatmul_multi takes 7 arguments");
+    int flags, pre;
+    if (!as_int(a[2], &flags) || !as_int(a[4], &pre)) return nullptr;
+    const double eps = PyFloat_AsDouble(a[6]);
+    if (eps == -1.0 && PyErr_Occurred()) return nullptr;
+    const cq_weight *ws[kMaxWeights];
+    float *ys[kMaxWeights];
+    PyObject *px = a[1], *aux = a[5];
+    const Py_ssize_t count = weights_of(a[0], ws);
+    if (count < 1 || !f32_on_device(px)) Py_RETURN_NONE;
+    const at::Tensor &x = THPVariable_Unpack(px);
+    int64_t n, k;
+    if (g_abi.weight_shape(ws[0], &n, &k) != CQ_OK || x.dim() < 2 || x.size(-1) != k || !aux_ok(pre, x, aux)) Py_RETURN_NONE;
+    const int64_t m = k ? x.numel() / k : 0;
+    size_t need = 0;
+    for (Py_ssize_t i = 0; i < count; i++) need = std::max(need, g_abi.workspace_bytes(ws[i], m, flags));
+    PyObject *held = nullptr;
+    void *wp;
+    size_t ws_bytes;
+    if (!workspace(a[3], need, x, px, &held, &wp, &ws_bytes)) return nullptr;
+    PyObject *outs = PyList_New(count);
+    bool ok = outs != nullptr;
+    try {
+        for (Py_ssize_t i = 0; ok && i < count; i++) {
+            int64_t ni, ki;
+            g_abi.weight_shape(ws[i], &ni, &ki);
+            PyObject *o = THPVariable_Wrap(result_like(x, ni));
+            ok = o != nullptr;
+            if (!ok) break;
+            ys[i] = (float *)THPVariable_Unpack(o).data_ptr();
+            PyList_SET_ITEM(outs, i, o);
+        }
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        ok = false;
+    }
+    int rc = CQ_OK;
+    if (ok) {
+        const float *xp = (const float *)x.data_ptr(), *ap = aux == Py_None ? nullptr : floats_of(aux);
+        void *s = stream_now();
+        Py_BEGIN_ALLOW_THREADS
+        rc = g_abi.qmatmul_multi(ws, (int)count, pre, xp, ap, (float)eps, m, ys, flags, wp, ws_bytes, s);
+        Py_END_ALLOW_THREADS
+    }
+    Py_DECREF(held);
+    if (!ok || rc != CQ_OK) {
+        Py_XDECREF(outs);
+        return ok ? fail(rc) : nullptr;
+    }
+    return outs;
+}
+
+// qmatmul_grouped(experts, x, row_ids, offsets (int32 buffer), flags, workspace, pre, aux, eps)
+PyObject *py_qmatmul_grouped(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 9) return PyErr_Format(PyExc_TypeError, "qmatmul_grouped takes 9 arguments");
+    int flags, pre;
+    if (!as_int(a[4], &flags) || !as_int(a[6], &pre)) return nullptr;
+    const double eps = PyFloat_AsDouble(a[8]);
+    if (eps == -1.0 && PyErr_Occurred()) return nullptr;
+    const cq_weight *ws[kMaxWeights];
+    PyObject *px = a[1], *ids = a[2], *aux = a[7];
+    const Py_ssize_t count = weights_of(a[0], ws);
+    if (count < 1 || !f32_on_device(px) || (ids != Py_None && !THPVariable_Check(ids))) Py_RETURN_NONE;
+    const at::Tensor &x = THPVariable_Unpack(px);
+    int64_t n, k;
+    if (g_abi.weight_shape(ws[0], &n, &k) != CQ_OK || !aux_ok(pre, x, aux)) Py_RETURN_NONE;
+    Py_buffer offs;
+    if (PyObject_GetBuffer(a[3], &offs, PyBUF_C_CONTIGUOUS) != 0) return nullptr;
+    const int32_t *offsets = (const int32_t *)offs.buf;
+    const Py_ssize_t have = offs.len / (Py_ssize_t)sizeof(int32_t);
+    if (offs.itemsize != sizeof(int32_t) || have < count + 1) {
+        PyBuffer_Release(&offs);
+        Py_RETURN_NONE;
+    }
+    const int64_t total = offsets[have - 1];
+    PyObject *held = nullptr, *out = nullptr;
+    void *wp;
+    size_t ws_bytes;
+    int rc = CQ_OK;
+    if (total >= 0 && workspace(a[5], g_abi.grouped_workspace_bytes(ws, (int)count, total, flags), x, px, &held, &wp, &ws_bytes)) {
+        try {
+            out = THPVariable_Wrap(empty_f32({total, n}, x.device()));
+        } catch (const std::exception &e) {
+            PyErr_SetString(PyExc_RuntimeError, e.what());
+        }
+        if (out) {
+            float *y = (float *)THPVariable_Unpack(out).data_ptr();
+            const float *xp = (const float *)x.data_ptr(), *ap = pre == CQ_PRE_NONE ? nullptr : floats_of(aux);
+            const int32_t *rid = ids == Py_None ? nullptr : (const int32_t *)THPVariable_Unpack(ids).data_ptr();
+            void *s = stream_now();
+            Py_BEGIN_ALLOW_THREADS
+            rc = pre == CQ_PRE_NONE ? g_abi.qmatmul_grouped(ws, (int)count, xp, rid, offsets, y, flags, wp, ws_bytes, s)
+                                    : g_abi.qmatmul_grouped_fused(ws, (int)count, pre, xp, ap, (float)eps, rid, offsets, y, flags, wp, ws_bytes, s);
+            Py_END_ALLOW_THREADS
+        }
+        Py_DECREF(held);
+    } else if (total < 0) {
+        PyErr_SetString(g_error, "offsets must be non-negative");
+    }
+    PyBuffer_Release(&offs);
+    if (out && rc != CQ_OK) {
+        Py_DECREF(out);
+        return fail(rc);
+    }
+    return out;
+}
+
+// dequantize(w, f16)
+PyObject *py_dequantize(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 2) return PyErr_Format(PyExc_TypeError, "dequantize takes 2 arguments");
+    const bool f16 = PyObject_IsTrue(a[1]) == 1;
+    const cq_weight *w = weight_of(a[0]);
+    int64_t n, k;
+    if (!w || g_abi.weight_shape(w, &n, &k) != CQ_OK) Py_RETURN_NONE;
+    PyObject *out;
+    void *p;
+    try {
+        const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)g_abi.weight_device(w));
+        out = THPVariable_Wrap(at::Tensor(at::detail::empty_cuda({n, k}, f16 ? at::kHalf : at::kFloat, dev, std::nullopt)));
+        if (!out) return nullptr;
+        p = THPVariable_Unpack(out).data_ptr();
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+    void *s = stream_now();
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = f16 ? g_abi.weight_dequantize_f16(w, (uint16_t *)p, s) : g_abi.weight_dequantize(w, (float *)p, s);
+    Py_END_ALLOW_THREADS
+    if (rc != CQ_OK) {
+        Py_DECREF(out);
+        return fail(rc);
+    }
+    return out;
+}
+
+template <typename F> bool take(PyObject *table, const char *name, F *f) {
+    PyObject *v = PyDict_GetItemString(table, name);
+    if (!v) {
+        PyErr_Format(PyExc_KeyError, "%s", name);
+        return false;
+    }
+    *f = (F)PyLong_AsVoidPtr(v);
+    return !PyErr_Occurred();
+}
+
+// bind({name: address}, error class)
+PyObject *py_bind(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 2 || !PyDict_Check(a[0])) return PyErr_Format(PyExc_TypeError, "bind takes a dict and an exception class");
+#define TAKE(f) take(a[0], "cq_" #f, &g_abi.f)
+    if (!(TAKE(last_error) && TAKE(weight_shape) && TAKE(weight_device) && TAKE(workspace_bytes) && TAKE(qmatmul) && TAKE(qmatmul_fused) &&
+          TAKE(qmatmul_multi) && TAKE(grouped_workspace_bytes) && TAKE(qmatmul_grouped) && TAKE(qmatmul_grouped_fused) &&
+          TAKE(weight_dequantize) && TAKE(weight_dequantize_f16)))
+        return nullptr;
+#undef TAKE
+    Py_INCREF(a[1]);
+    Py_XSETREF(g_error, a[1]);
+    Py_RETURN_NONE;
+}
+
+#define FAST(f) (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr
+PyMethodDef g_methods[] = {{"bind", FAST(py_bind)},
+                           {"qmatmul", FAST(py_qmatmul)},
+                           {"qmatmul_multi", FAST(py_qmatmul_multi)},
+                           {"qmatmul_grouped", FAST(py_qmatmul_grouped)},
+                           {"dequantize", FAST(py_dequantize)},
+                           {nullptr, nullptr, 0, nullptr}};
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__calls(void) {
+    g_s_addr = PyUnicode_InternFromString("_addr");
+    g_s_buf = PyUnicode_InternFromString("buf");
+    g_s_get = PyUnicode_InternFromString("get");
+    return PyModule_Create(&g_module);
+}

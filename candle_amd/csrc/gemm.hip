@@ -1070,19 +1070,6 @@ __global__ void __launch_bounds__(kThreads) gemm_q81_kernel(cq_weight w, cq_act_
     }
 }
 
-int g_cus = 0;
-int num_cus() {
-    if (g_cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            g_cus = n;
-        else
-            g_cus = 256;
-    }
-    return g_cus;
-}
-
 // Too few workgroups for `slots` of them at once: K is split (at least four blocks per part).
 int pick_ksplit(int64_t tiles, int64_t kb, int64_t slots) {
     int ksplit = 1;
@@ -1104,7 +1091,7 @@ struct Plan {
     int kh = 1;   // 2: gemm_kh_kernel (K halved inside the workgroup, 128 weight rows per workgroup)
 };
 Plan pick_plan(const cq_weight *w, int64_t m) {
-    const int64_t gx = n_tiles(w), kb = w->k >> 8, cus = num_cus();
+    const int64_t gx = n_tiles(w), kb = w->k >> 8, cus = cq_num_cus();
     // unpacking one K block of a wave's 32 rows: 152 vector instructions for Q4K, about 370 for Q6K
     const double unpack = w->dtype == CQ_DTYPE_Q4K ? 22.0 : w->dtype == CQ_DTYPE_Q5K ? 32.0 : 50.0;
     const double atomic_pass = (double)m * (double)w->n * 4.0 / 1.1e6 * 16.0;   // bytes / (1.1e6 bytes per us) in units
@@ -1223,7 +1210,7 @@ hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const 
     const size_t lds = grouped_wbuf<DT>() == 2 ? Tile<DT, 1>::kTotal2 : Tile<DT, 1>::kTotal;
     if (hipError_t e = cq_ensure_lds<gemm_grouped_kernel<DT>>(w->dev, lds); e != hipSuccess) return e;
     const int64_t gx = n_tiles(w);
-    const int ksplit = pick_ksplit(gx * ntiles, w->k >> 8, 2 * num_cus());   // two single-tile workgroups per CU
+    const int ksplit = pick_ksplit(gx * ntiles, w->k >> 8, 2 * cq_num_cus());   // two single-tile workgroups per CU
     if (ksplit > 1 && !y_cleared) {
         hipError_t e = cq_launch_fill_zero(y, (int64_t)offsets[n_experts] * w->n, s);
         if (e != hipSuccess) return e;
@@ -1245,7 +1232,7 @@ template <int DT>
 hipError_t launch_q81_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
     // the tallest tile that still gives every CU a workgroup
     int mt = 4;
-    while (mt > 1 && (m <= 16 * mt || n_tiles(w) * ((m + mt * 32 - 1) / (mt * 32)) < num_cus())) mt >>= 1;
+    while (mt > 1 && (m <= 16 * mt || n_tiles(w) * ((m + mt * 32 - 1) / (mt * 32)) < cq_num_cus())) mt >>= 1;
     if (mt == 1) return launch_q81_mt<DT, 1>(w, a, m, y, s);
     if (mt == 2) return launch_q81_mt<DT, 2>(w, a, m, y, s);
     return launch_q81_mt<DT, 4>(w, a, m, y, s);
@@ -1280,7 +1267,7 @@ hipError_t cq_launch_gemm_dump(const cq_weight *w, cq_act_view a, int act_dtype,
 bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets) {
     int64_t tiles = 0;
     for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + 31) / 32;
-    return tiles > 0 && pick_ksplit(n_tiles(experts[0]) * tiles, experts[0]->k >> 8, 2 * num_cus()) > 1;
+    return tiles > 0 && pick_ksplit(n_tiles(experts[0]) * tiles, experts[0]->k >> 8, 2 * cq_num_cus()) > 1;
 }
 
 bool cq_gemm_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }

@@ -276,19 +276,6 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
     }
 }
 
-int g_cus = 0;
-int num_cus() {
-    if (g_cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            g_cus = n;
-        else
-            g_cus = 256;
-    }
-    return g_cus;
-}
-
 // Tile height (MT x 32 activation rows per workgroup) and K split of a launch, from a cost model fitted to
 // measurements (Q8_0, 256 CUs; unit 1/16 us): a workgroup spends 10 units per 256-element K step on its
 // weights and 23 per 32-row tile on it, 24 on starting and finishing; workgroups run one per CU, in rounds;
@@ -297,7 +284,7 @@ struct Plan {
     int mt, ksplit;
 };
 Plan pick_plan(const cq_weight *w, int64_t m) {
-    const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks_total = (w->k + 255) >> 8, cus = num_cus();
+    const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks_total = (w->k + 255) >> 8, cus = cq_num_cus();
     const double atomic_pass = (double)m * (double)w->n * 4.0 / 1.1e6 * 16.0;   // bytes / (1.1e6 bytes per us) in units
     Plan best{1, 1};
     double best_cost = 0.0;

@@ -1276,19 +1276,6 @@ __global__ void __launch_bounds__(kStagedThreads) int_dots_kernel(cq_weight w, c
 }
 
 // ------------------------------------------------------------------------------- launch ----
-int g_num_cus = 0;
-int num_cus() {
-    if (g_num_cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            g_num_cus = n;
-        else
-            g_num_cus = 256;
-    }
-    return g_num_cus;
-}
-
 // Eight waves per workgroup, one workgroup per CU.  Whole workgroups only, and every wave
 // gets at least `depth` rows: wgs * 8 * depth <= n.
 template <int DT, int UPL, int PRE, int NWT = 1, int MB = 1>
@@ -1300,7 +1287,7 @@ hipError_t launch_fused_upl(const cq_weight *w, int64_t n, FusedMore<NWT> more, 
                                               : lds_row_bytes<DT>(w->k) * MB;
     // every workgroup quantizes the whole activation row, so fewer, longer-lived workgroups win: one
     // per CU measured faster than two on every decode shape (11008 x 4096 Q4K: 7.0 us against 7.6 us)
-    const int64_t max_wgs = num_cus();
+    const int64_t max_wgs = cq_num_cus();
     int depth = UPL <= 2 ? 2 : 1;
     if (n < NW * 2) depth = 1;
     if (n < NW) {  // fewer rows than one workgroup's waves: the two-launch path handles it
@@ -1381,7 +1368,7 @@ hipError_t launch_batched_upl(const cq_weight *w, cq_act_view a, int64_t m0, int
     const size_t lds = lds_row_bytes<DT>(w->k) * MB;
     if (hipError_t e = cq_ensure_lds<batched_kernel<DT, UPL, NW, MB>>(w->dev, lds); e != hipSuccess) return e;
     int64_t wgs = w->n / NW;
-    if (wgs > num_cus()) wgs = num_cus();
+    if (wgs > cq_num_cus()) wgs = cq_num_cus();
     const int64_t tw = wgs * NW, rpw = w->n / tw, extra = w->n % tw;
     CQ_LAUNCH((batched_kernel<DT, UPL, NW, MB>), (unsigned)wgs, NW * 64, lds, s, *w, a, m0, m, y, tw, rpw, extra);
     return hipGetLastError();

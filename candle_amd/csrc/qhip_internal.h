@@ -90,6 +90,9 @@ int cq_set_error(int code, const char *fmt, ...);
 // then never split K (no partial sums added atomically in arrival order).
 bool cq_no_split_k();
 
+// Compute units of the device (the first one asked; a process has devices of one kind), looked up once.
+int cq_num_cus();
+
 // Kernel timing hook (api.hip): true when the calling thread armed the timer; the launch then goes
 // through CQ_LAUNCH below with the two events.  Disarms.
 bool cq_timing_take(hipEvent_t *start, hipEvent_t *stop);

@@ -1225,9 +1225,7 @@ hipError_t launch_blk32_res_inst(const cq_weight *w, cq_act_view a, int64_t m, f
 template <int DT, int RT, bool DUMP>
 bool launch_blk32_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s, hipError_t *err) {
     const int64_t kg = (w->k + 255) >> 8, tiles = (w->n + 15) / 16;
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (cus <= 0) cus = 256;
+    const int cus = cq_num_cus();
     const bool sixteen = kg > 8;
     if (tiles > cus) {
         // several tiles per workgroup: rounds of tiles with one meeting each, where a wave has one K group
@@ -1319,9 +1317,7 @@ hipError_t launch_multi_inst(const cq_weight *w, cq_act_view a, int64_t m, float
 template <int DT, int RT, bool DUMP>
 bool launch_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s, hipError_t *err) {
     const int64_t kb = w->k >> 8, tiles = (w->n + 15) / 16;
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (cus <= 0) cus = 256;
+    const int cus = cq_num_cus();
     const unsigned grid = (unsigned)(tiles < cus ? tiles : cus);
     const bool sixteen = kb > 8;
     if (kb > (sixteen ? 16 : 8) * kMaxBpw) return false;

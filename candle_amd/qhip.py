@@ -96,6 +96,27 @@ def load():
     return L
 
 
+CALLS_PATH = os.path.join(_HERE, "lib", "_calls.so")
+_native = None
+
+
+def _calls():
+    """The matmul-side calls in native code (csrc/calls.cpp), bound to the library `load` loaded."""
+    global _native
+    if _native is None:
+        import importlib.util
+        L = load()
+        _torch()   # the module links against it
+        if not os.path.exists(CALLS_PATH):
+            raise QHipError(f"{CALLS_PATH} is not built (run __graft_entry__.build())")
+        spec = importlib.util.spec_from_file_location("_calls", CALLS_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.bind({name: C.cast(getattr(L, name), C.c_void_p).value for name in EXPORTS}, QHipError)
+        _native = mod
+    return _native
+
+
 def check(rc: int):
     if rc != 0:
         raise QHipError(f"[{rc}] {load().cq_last_error().decode()}")
@@ -144,6 +165,7 @@ class QWeight:
 
     def __init__(self, handle, dev: int):
         self._h = C.c_void_p(handle)
+        self._addr = handle or 0   # what the native calls read
         self.dev = dev
 
     # -- constructors
@@ -190,6 +212,7 @@ class QWeight:
             if self._h is not None and self._h.value:
                 load().cq_weight_destroy(self._h)
                 self._h = None
+                self._addr = 0
         except Exception:
             pass
 
@@ -222,18 +245,10 @@ class QWeight:
         return self
 
     def dequantize(self):
-        torch = _torch()
-        n, k = self.shape
-        out = torch.empty((n, k), dtype=torch.float32, device=f"cuda:{self.dev}")
-        check(load().cq_weight_dequantize(self._h, C.c_void_p(out.data_ptr()), _stream_ptr()))
-        return out
+        return (_native or _calls()).dequantize(self, False)
 
     def dequantize_f16(self):
-        torch = _torch()
-        n, k = self.shape
-        out = torch.empty((n, k), dtype=torch.float16, device=f"cuda:{self.dev}")
-        check(load().cq_weight_dequantize_f16(self._h, C.c_void_p(out.data_ptr()), _stream_ptr()))
-        return out
+        return (_native or _calls()).dequantize(self, True)
 
     def to_ggml(self) -> np.ndarray:
         _torch().cuda.synchronize()
@@ -288,29 +303,22 @@ def qmatmul(w: QWeight, x, flags: int = 0, out=None, workspace: Workspace | None
     """QMatMul::forward for a quantized weight: x [..., k] f32 contiguous -> [..., n].  With `pre`
     the model step in front of the matmul (rms_norm with alpha = aux, or silu(x) * aux) is computed
     inside the same launches."""
-    torch = _torch()
-    L = load()
+    y = (_native or _calls()).qmatmul(w, x, flags, out, workspace or _default_ws, pre, aux, eps)
+    if y is None:
+        _refuse(w.shape, x, pre, aux)
+    return y
+
+
+def _refuse(shape, x, pre: int, aux):
+    """Words the error of a call whose arguments the native code did not take."""
     _require_f32_cuda(x)
     _check_pre(pre, x, aux)
-    n, k = w.shape
+    n, k = shape
     if x.dim() < 2:
         raise QHipError(f"input tensor has only one dimension {tuple(x.shape)}")   # mod.rs:480-482
     if x.shape[-1] != k:
         raise QHipError(f"input tensor {tuple(x.shape)} incompatible with {(n, k)}")  # mod.rs:485-487
-    m = x.numel() // k if k else 0
-    out_shape = tuple(x.shape[:-1]) + (n,)
-    if out is None:
-        out = torch.empty(out_shape, dtype=torch.float32, device=x.device)
-    need = L.cq_workspace_bytes(w.handle, m, flags)
-    ws = (workspace or _default_ws).get(need, x.device)
-    if pre == PRE_NONE:
-        check(L.cq_qmatmul(w.handle, C.c_void_p(x.data_ptr()), m, C.c_void_p(out.data_ptr()), flags,
-                           C.c_void_p(ws.data_ptr()), ws.numel(), _stream_ptr()))
-    else:
-        check(L.cq_qmatmul_fused(w.handle, pre, C.c_void_p(x.data_ptr()), C.c_void_p(aux.data_ptr()), eps, m,
-                                 C.c_void_p(out.data_ptr()), flags, C.c_void_p(ws.data_ptr()), ws.numel(),
-                                 _stream_ptr()))
-    return out
+    raise QHipError("invalid argument")
 
 
 def qmatmul_shaped(w: QWeight, shape, x, flags: int = 0, out=None, workspace: Workspace | None = None):
@@ -338,28 +346,13 @@ def qmatmul_multi(ws, x, flags: int = 0, workspace: Workspace | None = None, pre
                   eps: float = 0.0):
     """[x . W^T for W in ws]: several weights (same dtype and row length) on the same activations, one
     launch for one activation row, rows quantized once otherwise (cq_qmatmul_multi)."""
-    torch = _torch()
-    L = load()
-    _require_f32_cuda(x)
-    _check_pre(pre, x, aux)
     ws = list(ws)
     if not ws:
         raise QHipError("no weights")
-    k = ws[0].shape[1]
-    if x.dim() < 2:
-        raise QHipError(f"input tensor has only one dimension {tuple(x.shape)}")
-    if x.shape[-1] != k:
-        raise QHipError(f"input tensor {tuple(x.shape)} incompatible with {ws[0].shape}")
-    m = x.numel() // k if k else 0
-    outs = [torch.empty(tuple(x.shape[:-1]) + (w.shape[0],), dtype=torch.float32, device=x.device) for w in ws]
-    need = max(L.cq_workspace_bytes(w.handle, m, flags) for w in ws)
-    wsp = (workspace or _default_ws).get(need, x.device)
-    vp = C.c_void_p
-    handles = (vp * len(ws))(*[w.handle for w in ws])
-    ys = (vp * len(ws))(*[o.data_ptr() for o in outs])
-    check(L.cq_qmatmul_multi(handles, len(ws), pre, vp(x.data_ptr()), vp(aux.data_ptr()) if aux is not None else None,
-                             eps, m, ys, flags, vp(wsp.data_ptr()), wsp.numel(), _stream_ptr()))
-    return outs
+    ys = (_native or _calls()).qmatmul_multi(ws, x, flags, workspace or _default_ws, pre, aux, eps)
+    if ys is None:
+        _refuse(ws[0].shape, x, pre, aux)
+    return ys
 
 
 def qmatmul_int_dots(w: QWeight, x):
@@ -405,27 +398,12 @@ def qmatmul_grouped(experts, x, row_ids, offsets, flags: int = 0, workspace: Wor
                     pre: int = PRE_NONE, aux=None, eps: float = 0.0):
     """y[p] = x[row_ids[p]] . W_e^T for p in [offsets[e], offsets[e+1]); offsets is a host int32 array.
     With `pre`, the gathered rows go through that step first (aux rows gathered like x rows)."""
-    torch = _torch()
-    L = load()
-    _require_f32_cuda(x)
-    _check_pre(pre, x, aux)
-    n, k = experts[0].shape
     offsets = np.ascontiguousarray(offsets, dtype=np.int32)
-    total = int(offsets[-1])
-    arr = (C.c_void_p * len(experts))(*[e.handle.value for e in experts])
-    y = torch.empty((total, n), dtype=torch.float32, device=x.device)
-    need = L.cq_grouped_workspace_bytes(arr, len(experts), total, flags)
-    ws = (workspace or _default_ws).get(need, x.device)
-    rid = C.c_void_p(row_ids.data_ptr()) if row_ids is not None else None
-    if pre == PRE_NONE:
-        check(L.cq_qmatmul_grouped(arr, len(experts), C.c_void_p(x.data_ptr()), rid,
-                                   offsets.ctypes.data_as(C.POINTER(C.c_int32)), C.c_void_p(y.data_ptr()), flags,
-                                   C.c_void_p(ws.data_ptr()), ws.numel(), _stream_ptr()))
-    else:
-        check(L.cq_qmatmul_grouped_fused(arr, len(experts), pre, C.c_void_p(x.data_ptr()), C.c_void_p(aux.data_ptr()),
-                                         eps, rid, offsets.ctypes.data_as(C.POINTER(C.c_int32)),
-                                         C.c_void_p(y.data_ptr()), flags, C.c_void_p(ws.data_ptr()), ws.numel(),
-                                         _stream_ptr()))
+    y = (_native or _calls()).qmatmul_grouped(list(experts), x, row_ids, offsets, flags, workspace or _default_ws, pre, aux, eps)
+    if y is None:
+        _require_f32_cuda(x)
+        _check_pre(pre, x, aux)
+        raise QHipError("invalid argument")
     return y
 
 
