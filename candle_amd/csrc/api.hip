@@ -377,14 +377,15 @@ extern "C" int cq_quantize_act_fused(int dev, int act_dtype, int pre, const floa
     return quantize_act_impl(dev, act_dtype, x_dev, m, k, cq_pre{pre, aux_dev, eps}, dst, stream);
 }
 
-// Workspace layout for m rows of K elements (see cq_act_view).
-static size_t act_ws_layout(int act_dtype, int64_t m, int64_t k, uint8_t *base, cq_act_view *v) {
+// Workspace layout for m rows of K elements (see cq_act_view).  `grouped`: the rows are sorted by expert, and tiles of up to
+// 128 rows start at any of them.
+static size_t act_ws_layout(int act_dtype, int64_t m, int64_t k, uint8_t *base, cq_act_view *v, bool grouped = false) {
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off = cq_align_up(off + bytes, 256); return o; };
     // Q8K rows are padded (see cq_act_view::m_stride); the others to whole 32-row groups, which the
     // split-K MFMA kernel copies without looking at the row count
     // (beyond 32 rows to whole 128-row tiles, which the 32-element-block tile kernel reads, scales included)
-    const int64_t m_pad = act_dtype == CQ_DTYPE_Q8K ? (m + 63) / 64 * 64 + 256 : m <= 32 ? (m + 31) / 32 * 32 : (m + 127) / 128 * 128;
+    const int64_t m_pad = act_dtype == CQ_DTYPE_Q8K ? (m + 63) / 64 * 64 + 256 : (m <= 32 ? (m + 31) / 32 * 32 : (m + 127) / 128 * 128) + (grouped ? 128 : 0);
     const size_t o_qs = take((size_t)(m_pad * k));
     cq_act_view view{};
     view.m_stride = m_pad;
@@ -708,7 +709,17 @@ extern "C" int cq_qmatmul_int_dots_mfma(const cq_weight *w, const float *x_dev, 
 extern "C" size_t cq_grouped_workspace_bytes(const cq_weight *const *experts, int n_experts, int64_t total_rows,
                                              int flags) {
     if (!experts || n_experts <= 0 || !experts[0] || total_rows <= 0) return 0;
-    return act_ws_layout(act_dtype_for(experts[0], flags), total_rows, experts[0]->k, nullptr, nullptr);
+    return act_ws_layout(act_dtype_for(experts[0], flags), total_rows, experts[0]->k, nullptr, nullptr, true);
+}
+
+// Most rows of one expert up to which the grouped split-K launch is taken.  Measured (8 experts, us of the whole call, split K /
+// tiles; at 1, 2, 8, 11, 20 rows for the fullest one): Q4K 14336 x 4096 19/29, 47/66, 58/70, 72/70, 97/72, 2816 x 1024 10/14 ..
+// 10.6/14.3, 13.4/14.3; Q8_0 14336 x 4096 30/35, 94/95, 107/101, 119/100, 2816 x 1024 10/14 .. 13/14, 23/15; Q4_0 14336 x 4096
+// 39/30, 2816 x 1024 10/13, 17/14.
+static int64_t grouped_skinny_rows(const cq_weight *w) {
+    if (w->dtype == CQ_DTYPE_Q4_0) return w->n * w->k <= (4 << 20) ? 1 : 0;
+    if (w->dtype == CQ_DTYPE_Q8_0) return w->n * w->k <= (4 << 20) ? 16 : 2;
+    return 16;
 }
 
 static int grouped_impl(const cq_weight *const *experts, int n_experts, const float *x_dev, cq_pre pre,
@@ -743,22 +754,32 @@ static int grouped_impl(const cq_weight *const *experts, int n_experts, const fl
     CQ_HIP_CHECK(hipSetDevice(w0->dev));
     hipStream_t s = (hipStream_t)stream;
     cq_act_view v;
-    act_ws_layout(act, total, w0->k, (uint8_t *)ws, &v);
-    // experts with more than eight rows among them: one tile-kernel launch for all experts
+    act_ws_layout(act, total, w0->k, (uint8_t *)ws, &v, true);
     int64_t most = 0;
     for (int e = 0; e < n_experts; e++) most = offsets[e + 1] - offsets[e] > most ? offsets[e + 1] - offsets[e] : most;
-    const bool want_gemm = (flags & CQ_FLAG_FORCE_GEMM) ? true : (flags & CQ_FLAG_FORCE_MATVEC) ? false : most > 8;
-    const bool grouped = want_gemm && cq_gemm_grouped_supported(experts, n_experts, offsets, act);
+    // One launch for all experts: the split-K kernel for few rows per expert, the tile kernels beyond; where neither takes the weights (few weight rows, many experts), a launch per expert.
+    enum { kSkinny, kGemm32, kGemm, kEach } path = kEach;
+    const bool force_gemm = (flags & CQ_FLAG_FORCE_GEMM) != 0, force_skinny = (flags & CQ_FLAG_FORCE_SKINNY) != 0;
+    if (!(flags & CQ_FLAG_FORCE_MATVEC)) {
+        const bool skinny = cq_skinny_grouped_takes(experts, n_experts, offsets, act);
+        if (skinny && !force_gemm && (force_skinny || most <= grouped_skinny_rows(w0))) path = kSkinny;
+        else if (cq_gemm_grouped_supported(experts, n_experts, offsets, act)) path = kGemm;
+        else if (cq_gemm32_grouped_takes(experts, n_experts, offsets, act)) path = kGemm32;
+        else if (skinny && !force_gemm) path = kSkinny;
+    }
     // gather + quantize every routed row once (clearing the output on the way if the grouped launch splits K;
     // with row ids the extent of x is not known here, so nothing is cleared then)
     cq_clear clear = cq_no_clear();
-    if (!reuse && grouped && !row_ids_dev && cq_gemm_grouped_splits_k(experts, n_experts, offsets) &&
-        clear_in_quantizer_ok(y_dev, total * w0->n, x_dev, total * w0->k, pre))
+    const bool splits = path == kGemm ? cq_gemm_grouped_splits_k(experts, n_experts, offsets)
+                                      : path == kGemm32 && cq_gemm32_grouped_splits_k(experts, n_experts, offsets);
+    if (!reuse && !row_ids_dev && splits && clear_in_quantizer_ok(y_dev, total * w0->n, x_dev, total * w0->k, pre))
         clear = cq_clear{y_dev, total * w0->n};
     if (!reuse) CQ_HIP_CHECK(cq_launch_quantize_act_ws(act, x_dev, row_ids_dev, total, w0->k, pre, v, clear, s));
-    if (grouped) {
-        CQ_HIP_CHECK(cq_launch_gemm_grouped(experts, n_experts, offsets, v, y_dev, clear.p != nullptr, s));
-        return CQ_OK;
+    switch (path) {
+    case kSkinny: CQ_HIP_CHECK(cq_launch_skinny_grouped(experts, n_experts, offsets, v, y_dev, s)); return CQ_OK;
+    case kGemm: CQ_HIP_CHECK(cq_launch_gemm_grouped(experts, n_experts, offsets, v, y_dev, clear.p != nullptr, s)); return CQ_OK;
+    case kGemm32: CQ_HIP_CHECK(cq_launch_gemm32_grouped(experts, n_experts, offsets, v, y_dev, clear.p != nullptr, s)); return CQ_OK;
+    case kEach: break;
     }
     // otherwise one matmul per non-empty expert over its slice
     for (int e = 0; e < n_experts; e++) {

@@ -845,7 +845,7 @@ __global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_v
 }
 
 // Grouped (mixture-of-experts) variant: one launch for every expert.  blockIdx.y walks a table of
-// 32-row tiles of the expert-sorted activation rows; each tile names its expert's weights.
+// tiles of 32*MT expert-sorted activation rows; each tile names its expert's weights.
 constexpr int kMaxGroupExperts = 16, kMaxGroupTiles = 96;
 struct GroupArgs {
     cq_weight w[kMaxGroupExperts];
@@ -854,14 +854,16 @@ struct GroupArgs {
     int8_t expert[kMaxGroupTiles];
 };
 
-// Expert weights are read once per launch, cold: the types whose headers can come through the copies take two buffers.
+// One row tile per expert: its weights are read once per launch, cold, and the types whose headers can come through the
+// copies take two buffers.  Taller tiles (experts with more rows) unpack a weight block once for up to 128 rows.
 template <int DT> constexpr int grouped_wbuf() { return DT == CQ_DTYPE_Q4K || DT == CQ_DTYPE_Q5K ? 2 : 1; }
-template <int DT>
+template <int DT, int MT>
 __global__ void __launch_bounds__(kThreads) gemm_grouped_kernel(GroupArgs ga, cq_act_view a, float *__restrict__ y,
                                                                 int ksplit) {
     const int tile = blockIdx.y;
     const cq_weight w = ga.w[ga.expert[tile]];
-    gemm_body<DT, 1, false, grouped_wbuf<DT>(), true>(w, a, ga.row0[tile], ga.row_end[tile], y, ksplit);
+    if constexpr (MT == 1) gemm_body<DT, 1, false, grouped_wbuf<DT>(), true>(w, a, ga.row0[tile], ga.row_end[tile], y, ksplit);
+    else gemm_body<DT, MT>(w, a, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit);
 }
 
 // ------------------------------------------------ K-quant weights x Q8_1 activations (tile kernel) ----
@@ -1190,14 +1192,42 @@ hipError_t launch_dump_dt(const cq_weight *w, cq_act_view a, int64_t m, cq_mfma_
     return launch_dump_mt<DT, 4>(w, a, m, p.ksplit, d, s);
 }
 
-template <int DT>
-hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
-                          float *y, bool y_cleared, hipStream_t s) {
+int64_t grouped_tiles(const int32_t *offsets, int n_experts, int mt) {
+    int64_t tiles = 0;
+    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + 32 * mt - 1) / (32 * mt);
+    return tiles;
+}
+// Tile height and K split of a grouped launch.  A single 32-row tile per expert splits K for two workgroups per CU; taller
+// tiles, by the cost model of pick_plan without a split, where they need fewer rounds of work: 8 experts 14336 x 4096,
+// 512 routed rows (at most 73 each), as 32-row tiles and as planned: Q4K 162 -> 139 us, Q6K 226 -> 174; 4096 x 14336 Q6K
+// 264 -> 185.
+Plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
+    const int64_t gx = n_tiles(w), kb = w->k >> 8, cus = cq_num_cus();
+    const double unpack = w->dtype == CQ_DTYPE_Q4K ? 22.0 : w->dtype == CQ_DTYPE_Q5K ? 32.0 : 50.0;
+    Plan best{1, 1};
+    double best_cost = 0.0;
+    for (int mt = 1; mt <= 4; mt <<= 1) {
+        const int64_t tiles = grouped_tiles(offsets, n_experts, mt);
+        if (mt > 1 && tiles == grouped_tiles(offsets, n_experts, mt / 2)) break;   // half the height holds every expert's rows
+        const int64_t rounds = (gx * tiles + cus - 1) / cus;
+        const double cost = (double)rounds * ((double)kb * (unpack + 13.5 * mt) + 24.0);
+        if (mt == 1 || cost < best_cost) {
+            best = Plan{mt, mt == 1 ? pick_ksplit(gx * tiles, kb, 2 * cus) : 1};
+            best_cost = cost;
+            if (best.ksplit > 1) break;   // (few workgroups: not a case for fewer, taller ones)
+        }
+    }
+    return best;
+}
+
+template <int DT, int MT>
+hipError_t launch_grouped_mt(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
+                             float *y, int ksplit, bool y_cleared, hipStream_t s) {
     GroupArgs ga;
     int ntiles = 0;
     for (int e = 0; e < n_experts; e++) {
         ga.w[e] = *experts[e];
-        for (int32_t r = offsets[e]; r < offsets[e + 1]; r += 32) {
+        for (int32_t r = offsets[e]; r < offsets[e + 1]; r += 32 * MT) {
             if (ntiles == kMaxGroupTiles) return hipErrorInvalidConfiguration;
             ga.row0[ntiles] = r;
             ga.row_end[ntiles] = offsets[e + 1];
@@ -1207,17 +1237,23 @@ hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const 
     }
     if (ntiles == 0) return hipSuccess;
     const cq_weight *w = experts[0];
-    const size_t lds = grouped_wbuf<DT>() == 2 ? Tile<DT, 1>::kTotal2 : Tile<DT, 1>::kTotal;
-    if (hipError_t e = cq_ensure_lds<gemm_grouped_kernel<DT>>(w->dev, lds); e != hipSuccess) return e;
-    const int64_t gx = n_tiles(w);
-    const int ksplit = pick_ksplit(gx * ntiles, w->k >> 8, 2 * cq_num_cus());   // two single-tile workgroups per CU
+    const size_t lds = MT == 1 && grouped_wbuf<DT>() == 2 ? Tile<DT, MT>::kTotal2 : Tile<DT, MT>::kTotal;
+    if (hipError_t e = cq_ensure_lds<gemm_grouped_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
     if (ksplit > 1 && !y_cleared) {
         hipError_t e = cq_launch_fill_zero(y, (int64_t)offsets[n_experts] * w->n, s);
         if (e != hipSuccess) return e;
     }
-    dim3 grid((unsigned)gx, (unsigned)ntiles, (unsigned)ksplit);
-    CQ_LAUNCH((gemm_grouped_kernel<DT>), grid, kThreads, lds, s, ga, a, y, ksplit);
+    dim3 grid((unsigned)n_tiles(w), (unsigned)ntiles, (unsigned)ksplit);
+    CQ_LAUNCH((gemm_grouped_kernel<DT, MT>), grid, kThreads, lds, s, ga, a, y, ksplit);
     return hipGetLastError();
+}
+template <int DT>
+hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
+                          float *y, bool y_cleared, hipStream_t s) {
+    const Plan p = pick_grouped(experts[0], offsets, n_experts);
+    if (p.mt == 1) return launch_grouped_mt<DT, 1>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
+    if (p.mt == 2) return launch_grouped_mt<DT, 2>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
+    return launch_grouped_mt<DT, 4>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
 }
 
 template <int DT, int MT>
@@ -1242,14 +1278,12 @@ hipError_t launch_q81_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y,
 
 bool cq_gemm_grouped_supported(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
     if (n_experts > kMaxGroupExperts || !cq_gemm_takes(experts[0], act_dtype)) return false;
-    int64_t tiles = 0;
-    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + 31) / 32;
-    return tiles <= kMaxGroupTiles;
+    return grouped_tiles(offsets, n_experts, 1) <= kMaxGroupTiles;
 }
 
 hipError_t cq_launch_gemm_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
                                   float *y, bool y_cleared, hipStream_t s) {
-    if (a.m_stride < ((int64_t)offsets[n_experts] + 31) / 32 * 32) return hipErrorInvalidValue;
+    if (a.m_stride < (int64_t)offsets[n_experts] + 127) return hipErrorInvalidValue;   // tiles of up to 128 rows from any row on
     if (experts[0]->dtype == CQ_DTYPE_Q4K) return launch_grouped<CQ_DTYPE_Q4K>(experts, n_experts, offsets, a, y, y_cleared, s);
     if (experts[0]->dtype == CQ_DTYPE_Q5K) return launch_grouped<CQ_DTYPE_Q5K>(experts, n_experts, offsets, a, y, y_cleared, s);
     return launch_grouped<CQ_DTYPE_Q6K>(experts, n_experts, offsets, a, y, y_cleared, s);
@@ -1265,9 +1299,7 @@ hipError_t cq_launch_gemm_dump(const cq_weight *w, cq_act_view a, int act_dtype,
 }
 
 bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets) {
-    int64_t tiles = 0;
-    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + 31) / 32;
-    return tiles > 0 && pick_ksplit(n_tiles(experts[0]) * tiles, experts[0]->k >> 8, 2 * cq_num_cus()) > 1;
+    return grouped_tiles(offsets, n_experts, 1) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
 }
 
 bool cq_gemm_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }

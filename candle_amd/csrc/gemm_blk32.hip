@@ -124,15 +124,14 @@ __device__ __forceinline__ void stage_weights(uint8_t *wl, const cq_weight &w, c
 // ONCE: a launch with a single row tile (up to 32 rows), which reads every weight byte once.
 // SHORT: K is no multiple of 256, the last step has fewer than eight blocks.
 template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
-__global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
-                                                          int ksplit, cq_mfma_dump dump) {
+__device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_view &a, int64_t m0, int64_t m, float *__restrict__ y,
+                                            int ksplit, cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
     extern __shared__ __align__(16) uint8_t smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, col = lane & 31;
     const int64_t k = w.k, ks = (k + 255) >> 8;         // K steps of 256 elements; the last one may be shorter
-    const int64_t m0 = (int64_t)blockIdx.y * (MT * 32);
     const int64_t n_own = ((int64_t)blockIdx.x * kWaves + wave) * 32;
     const bool n_ok = n_own < w.n;                      // wave-uniform; a wave past the last row only helps with the copies
     // fewer than 32 rows left: the tile begins earlier, at row n - 32, and only the wave's own share is stored
@@ -276,6 +275,29 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
     }
 }
 
+template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
+__global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, int ksplit,
+                                                          cq_mfma_dump dump) {
+    gemm32_body<DT, MT, DUMP, ONCE, SHORT>(w, a, (int64_t)blockIdx.y * (MT * 32), m, y, ksplit, dump);
+}
+
+// Mixture-of-experts form: blockIdx.y walks a table of tiles of 32*MT rows of the expert-sorted activation rows; each tile names
+// its expert's weights (as gemm_grouped_kernel of gemm.hip).
+constexpr int kMaxGroupExperts = 16, kMaxGroupTiles = 96;
+struct GroupArgs {
+    cq_weight w[kMaxGroupExperts];
+    int32_t row0[kMaxGroupTiles];      // first activation row of the tile
+    int32_t row_end[kMaxGroupTiles];   // end of its expert's rows
+    int8_t expert[kMaxGroupTiles];
+};
+template <int DT, int MT, bool SHORT>
+__global__ void __launch_bounds__(kThreads) gemm32_grouped_kernel(GroupArgs ga, cq_act_view a, float *__restrict__ y, int ksplit) {
+    const int tile = blockIdx.y;
+    const cq_weight w = ga.w[ga.expert[tile]];
+    gemm32_body<DT, MT, false, MT == 1, SHORT>(w, a, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit,
+                                               cq_mfma_dump{nullptr, nullptr, 0});
+}
+
 // Tile height (MT x 32 activation rows per workgroup) and K split of a launch, from a cost model fitted to
 // measurements (Q8_0, 256 CUs; unit 1/16 us): a workgroup spends 10 units per 256-element K step on its
 // weights and 23 per 32-row tile on it, 24 on starting and finishing; workgroups run one per CU, in rounds;
@@ -349,7 +371,85 @@ hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, boo
     return launch_mt<DT, 4, DUMP>(w, a, m, y, p.ksplit, y_cleared, d, s);
 }
 
+int64_t grouped_tiles(const int32_t *offsets, int n_experts, int mt) {
+    int64_t tiles = 0;
+    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + 32 * mt - 1) / (32 * mt);
+    return tiles;
+}
+// Tile height and K split of a grouped launch.  Too few 32-row tiles for two workgroups per CU: K is split (at least two
+// steps per part).  Otherwise the height with the least work by the cost model of pick_plan.
+Plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
+    const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks = (w->k + 255) >> 8, cus = cq_num_cus();
+    int64_t tiles = grouped_tiles(offsets, n_experts, 1);
+    int split = 1;
+    while (!cq_no_split_k() && gx * tiles * split * 2 <= 2 * cus && ks / (split * 2) >= 2 && split < 16) split *= 2;
+    Plan best{1, split};
+    double best_cost = 0.0;
+    for (int mt = 1; mt <= 4 && split == 1; mt <<= 1) {
+        tiles = grouped_tiles(offsets, n_experts, mt);
+        if (mt > 1 && tiles == grouped_tiles(offsets, n_experts, mt / 2)) break;   // half the height holds every expert's rows
+        const double cost = (double)((gx * tiles + cus - 1) / cus) * ((double)ks * (10.0 + 23.0 * mt) + 24.0);
+        if (mt == 1 || cost < best_cost) {
+            best = Plan{mt, 1};
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+template <int DT, int MT, bool SHORT>
+hipError_t launch_grouped_mt(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
+                             int ksplit, bool y_cleared, hipStream_t s) {
+    GroupArgs ga;
+    int tiles = 0;
+    for (int e = 0; e < n_experts; e++) {
+        ga.w[e] = *experts[e];
+        for (int32_t r = offsets[e]; r < offsets[e + 1]; r += 32 * MT) {
+            if (tiles == kMaxGroupTiles) return hipErrorInvalidConfiguration;
+            ga.row0[tiles] = r;
+            ga.row_end[tiles] = offsets[e + 1];
+            ga.expert[tiles++] = (int8_t)e;
+        }
+    }
+    if (tiles == 0) return hipSuccess;
+    const cq_weight *w = experts[0];
+    const size_t lds = Tile<DT, MT>::kTotal;
+    if (hipError_t e = cq_ensure_lds<gemm32_grouped_kernel<DT, MT, SHORT>>(w->dev, lds); e != hipSuccess) return e;
+    if (ksplit > 1 && !y_cleared) {
+        hipError_t e = cq_launch_fill_zero(y, (int64_t)offsets[n_experts] * w->n, s);
+        if (e != hipSuccess) return e;
+    }
+    const dim3 grid((unsigned)((w->n + kWaves * 32 - 1) / (kWaves * 32)), (unsigned)tiles, (unsigned)ksplit);
+    CQ_LAUNCH((gemm32_grouped_kernel<DT, MT, SHORT>), grid, kThreads, lds, s, ga, a, y, ksplit);
+    return hipGetLastError();
+}
+template <int DT, bool SHORT>
+hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
+                          bool y_cleared, hipStream_t s) {
+    const Plan p = pick_grouped(experts[0], offsets, n_experts);
+    if (p.mt == 1) return launch_grouped_mt<DT, 1, SHORT>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
+    if (p.mt == 2) return launch_grouped_mt<DT, 2, SHORT>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
+    return launch_grouped_mt<DT, 4, SHORT>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
+}
+
 }  // namespace
+
+bool cq_gemm32_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
+    return n_experts <= kMaxGroupExperts && cq_gemm32_takes(experts[0], act_dtype) && grouped_tiles(offsets, n_experts, 1) <= kMaxGroupTiles;
+}
+bool cq_gemm32_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets) {
+    return grouped_tiles(offsets, n_experts, 1) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
+}
+hipError_t cq_launch_gemm32_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
+                                    bool y_cleared, hipStream_t s) {
+    if (a.m_stride < (int64_t)offsets[n_experts] + 127) return hipErrorInvalidValue;   // tiles of up to 128 rows from any row on
+    const bool whole = experts[0]->k % 256 == 0;
+    if (experts[0]->dtype == CQ_DTYPE_Q8_0)
+        return whole ? launch_grouped<CQ_DTYPE_Q8_0, false>(experts, n_experts, offsets, a, y, y_cleared, s)
+                     : launch_grouped<CQ_DTYPE_Q8_0, true>(experts, n_experts, offsets, a, y, y_cleared, s);
+    return whole ? launch_grouped<CQ_DTYPE_Q4_0, false>(experts, n_experts, offsets, a, y, y_cleared, s)
+                 : launch_grouped<CQ_DTYPE_Q4_0, true>(experts, n_experts, offsets, a, y, y_cleared, s);
+}
 
 bool cq_gemm32_takes(const cq_weight *w, int act_dtype) {
     // an even number of blocks per row, so that every row's scales begin on four bytes; the copies address 8 rows with 32-bit

@@ -202,10 +202,18 @@ bool cq_gemm32_supported(const cq_weight *w, int act_dtype);
 hipError_t cq_launch_gemm32(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, bool y_cleared,
                             hipStream_t s);
 bool cq_gemm32_splits_k(const cq_weight *w, int64_t m);
+bool cq_gemm32_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype);
+hipError_t cq_launch_gemm32_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
+                                    bool y_cleared, hipStream_t s);
+bool cq_gemm32_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets);
 // skinny.hip: a few activation rows (32 per pass) on the int8 MFMA, K split over the waves of a workgroup
 bool cq_skinny_takes(const cq_weight *w, int act_dtype);
 bool cq_skinny_supported(const cq_weight *w, int act_dtype);
 hipError_t cq_launch_skinny(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, hipStream_t s);
+// all experts of a mixture-of-experts projection in one launch, for a few rows per expert
+bool cq_skinny_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype);
+hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
+                                    hipStream_t s);
 // moe.hip
 hipError_t cq_launch_silu_mul(const float *a, const float *b, float *h, int64_t count, hipStream_t s);
 hipError_t cq_launch_scatter_add(const float *y, const int32_t *row_ids, const float *weights, int64_t total_rows,

@@ -194,8 +194,8 @@ __device__ __forceinline__ void block_unpack(const uint8_t *wl, int lane, const 
 // DUMP (verification): the block integers, and the min term as the f16 MFMA delivers it from a zero accumulator,
 // are stored through `dump` instead of the result through `y`.
 template <int DT, int RT, bool DUMP>
-__global__ void __launch_bounds__(kThreads) skinny_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m,
-                                                          float *__restrict__ y, cq_mfma_dump dump) {
+__device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_view &a, int64_t m0, int64_t m, float *__restrict__ y,
+                                            cq_mfma_dump dump) {
     typedef Buf<DT, RT> B;
     constexpr bool MINS = is_k4(DT);
     constexpr int NT = (RT + 1) / 2;   // 16-row tiles
@@ -315,6 +315,12 @@ __global__ void __launch_bounds__(kThreads) skinny_kernel(cq_weight w, cq_act_vi
             if (row < m) y[row * w.n + col] = s[i];
         }
     }
+}
+
+template <int DT, int RT, bool DUMP>
+__global__ void __launch_bounds__(kThreads) skinny_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
+                                                          cq_mfma_dump dump) {
+    skinny_body<DT, RT, DUMP>(w, a, m0, m, y, dump);
 }
 
 // ------------------------------------------------------------ resident-activation variant ----
@@ -752,8 +758,8 @@ template <typename F> __device__ __forceinline__ void each_block(int64_t left, F
 }
 
 template <int DT, int RT, bool DUMP>
-__global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m,
-                                                                float *__restrict__ y, cq_mfma_dump dump) {
+__device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_act_view &a, int64_t m0, int64_t m, float *__restrict__ y,
+                                                  cq_mfma_dump dump) {
     typedef BufQ8<RT> B;
     constexpr bool Q4 = DT == CQ_DTYPE_Q4_0;
     constexpr int NT = (RT + 1) / 2;   // 16-row tiles
@@ -877,6 +883,31 @@ __global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_
             if (row < m) y[row * w.n + col] = s[i];
         }
     }
+}
+
+template <int DT, int RT, bool DUMP>
+__global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
+                                                                cq_mfma_dump dump) {
+    skinny_blk32_body<DT, RT, DUMP>(w, a, m0, m, y, dump);
+}
+
+// Mixture-of-experts form of the two: blockIdx.y is a tile of up to 8 * RT routed rows and names its expert's weights, so
+// that a projection of all experts is one launch, as in the grouped tile kernel (gemm.hip).
+constexpr int kMaxGroupExperts = 16, kMaxGroupTiles = 96;
+struct GroupArgs {
+    cq_weight w[kMaxGroupExperts];
+    int32_t row0[kMaxGroupTiles];      // first activation row of the tile
+    int32_t row_end[kMaxGroupTiles];   // end of its expert's rows
+    int8_t expert[kMaxGroupTiles];
+};
+template <int DT, int RT>
+__global__ void __launch_bounds__(kThreads) skinny_grouped_kernel(GroupArgs ga, cq_act_view a, float *__restrict__ y) {
+    const int tile = blockIdx.y;
+    const int64_t m0 = ga.row0[tile], end = ga.row_end[tile], m = m0 + 8 * RT < end ? m0 + 8 * RT : end;
+    const cq_weight w = ga.w[ga.expert[tile]];
+    const cq_mfma_dump none{nullptr, nullptr, 0};
+    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, RT, false>(w, a, m0, m, y, none);
+    else skinny_body<DT, RT, false>(w, a, m0, m, y, none);
 }
 
 // ------------------------------------------- the same with everything of a workgroup in flight at once ----
@@ -1359,6 +1390,41 @@ bool launch_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_
     return false;
 }
 
+template <int DT, int RT>
+hipError_t launch_grouped_rt(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y, hipStream_t s) {
+    GroupArgs ga;
+    int tiles = 0;
+    for (int e = 0; e < n_experts; e++) {
+        ga.w[e] = *experts[e];
+        for (int32_t r = offsets[e]; r < offsets[e + 1]; r += 8 * RT) {
+            if (tiles == kMaxGroupTiles) return hipErrorInvalidConfiguration;
+            ga.row0[tiles] = r;
+            ga.row_end[tiles] = offsets[e + 1];
+            ga.expert[tiles++] = (int8_t)e;
+        }
+    }
+    if (tiles == 0) return hipSuccess;
+    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
+    if (hipError_t e = cq_ensure_lds<skinny_grouped_kernel<DT, RT>>(experts[0]->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_grouped_kernel<DT, RT>), dim3((unsigned)((experts[0]->n + 15) / 16), (unsigned)tiles), kThreads, lds, s, ga, a, y);
+    return hipGetLastError();
+}
+// Rows per tile: what the fullest expert needs, in groups of eight, up to 32 (an expert with more takes several tiles).
+int grouped_rt(int n_experts, const int32_t *offsets) {
+    int64_t most = 0;
+    for (int e = 0; e < n_experts; e++) most = offsets[e + 1] - offsets[e] > most ? offsets[e + 1] - offsets[e] : most;
+    return most <= 8 ? 1 : most <= 16 ? 2 : most <= 24 ? 3 : 4;
+}
+template <int DT>
+hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y, hipStream_t s) {
+    switch (grouped_rt(n_experts, offsets)) {
+    case 1: return launch_grouped_rt<DT, 1>(experts, n_experts, offsets, a, y, s);
+    case 2: return launch_grouped_rt<DT, 2>(experts, n_experts, offsets, a, y, s);
+    case 3: return launch_grouped_rt<DT, 3>(experts, n_experts, offsets, a, y, s);
+    default: return launch_grouped_rt<DT, 4>(experts, n_experts, offsets, a, y, s);
+    }
+}
+
 template <bool DUMP>
 hipError_t launch_any(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     if (!cq_skinny_takes(w, act_dtype)) return hipErrorNotSupported;
@@ -1395,4 +1461,24 @@ hipError_t cq_launch_skinny(const cq_weight *w, cq_act_view a, int act_dtype, in
 
 hipError_t cq_launch_skinny_dump(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, cq_mfma_dump d, hipStream_t s) {
     return launch_any<true>(w, a, act_dtype, m, nullptr, d, s);
+}
+
+bool cq_skinny_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
+    if (n_experts > kMaxGroupExperts || !cq_skinny_takes(experts[0], act_dtype)) return false;
+    const int rows = 8 * grouped_rt(n_experts, offsets);
+    int64_t tiles = 0;
+    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + rows - 1) / rows;
+    return tiles <= kMaxGroupTiles;
+}
+
+hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
+                                    hipStream_t s) {
+    if (a.m_stride < (int64_t)offsets[n_experts] + 31) return hipErrorInvalidValue;   // tiles of up to 32 rows from any row on
+    switch (experts[0]->dtype) {
+    case CQ_DTYPE_Q8_0: return launch_grouped<CQ_DTYPE_Q8_0>(experts, n_experts, offsets, a, y, s);
+    case CQ_DTYPE_Q4_0: return launch_grouped<CQ_DTYPE_Q4_0>(experts, n_experts, offsets, a, y, s);
+    case CQ_DTYPE_Q4K: return launch_grouped<CQ_DTYPE_Q4K>(experts, n_experts, offsets, a, y, s);
+    case CQ_DTYPE_Q5K: return launch_grouped<CQ_DTYPE_Q5K>(experts, n_experts, offsets, a, y, s);
+    default: return launch_grouped<CQ_DTYPE_Q6K>(experts, n_experts, offsets, a, y, s);
+    }
 }
