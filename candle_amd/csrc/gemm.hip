@@ -689,14 +689,21 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
     }
 
     if (n_ok && !DUMP) {
+        // (the lane's column anew: kept from above it would take registers that the 128-row tiles do not have)
+        int wv = wave, ln = lane;
+        asm volatile("" : "+s"(wv), "+v"(ln));
+        const int64_t own = ((int64_t)blockIdx.x * kWaves + wv) * 32, c = last_tile(own, w.n) + (ln & 31);
+        if (c < own) return;
+        float *__restrict__ yc = y + (m0 + (ln >> 5) * 4) * w.n + c;
+        const int64_t left = m - m0 - (ln >> 5) * 4;
 #pragma unroll
         for (int t = 0; t < MT; t++) {
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                if (row < m && n >= n_own) {
-                    if (ksplit == 1) y[row * w.n + n] = out[t][i];
-                    else unsafeAtomicAdd(&y[row * w.n + n], out[t][i]);
+                const int64_t row = t * 32 + (i >> 2) * 8 + (i & 3);
+                if (row < left) {
+                    if (ksplit == 1) yc[row * w.n] = out[t][i];
+                    else unsafeAtomicAdd(&yc[row * w.n], out[t][i]);
                 }
             }
         }
