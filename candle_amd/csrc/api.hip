@@ -652,6 +652,29 @@ extern "C" int cq_qmatmul_multi(const cq_weight *const *ws, int count, int pre, 
     // (two to four rows that the one-launch kernel takes need no quantizer launch to share)
     const bool share = m > 1 && !(flags & CQ_FLAG_REUSE_ACT) &&
                        !(flags == 0 && pre == CQ_PRE_NONE && cq_matvec_fused_rows_supported(ws[0], m));
+    // up to 16 rows: the quantizer launch and one split-K launch over all the weights' rows
+    const int act = cq_vec_dot_type(ws[0]->dtype);
+    if (share && flags == 0 && cq_skinny_shared_takes(ws, count, m, act)) {
+        size_t need = 0;
+        for (int i = 0; i < count; i++) {
+            const size_t b = cq_workspace_bytes(ws[i], m, flags);
+            need = b > need ? b : need;
+        }
+        for (int i = 0; i < count; i++)
+            if (int rc = check_matmul_args(ws[i], x_dev, m, ys_dev[i], workspace, ws_bytes, need)) return rc;
+        if (int rc = check_pre(p)) return rc;
+        CQ_HIP_CHECK(hipSetDevice(ws[0]->dev));
+        hipStream_t s = (hipStream_t)stream;
+        cq_act_view v;
+        act_ws_layout(act, m, ws[0]->k, (uint8_t *)workspace, &v);
+        CQ_HIP_CHECK(cq_launch_quantize_act_ws(act, x_dev, nullptr, m, ws[0]->k, p, v, cq_no_clear(), s));
+        CQ_HIP_CHECK(cq_launch_skinny_shared(ws, count, v, m, ys_dev, s));
+        for (int i = 0; i < count; i++) {
+            if (cq_has_min32(ws[i]->ggml_dtype)) CQ_HIP_CHECK(cq_launch_min32_term(ws[i], v, m, ys_dev[i], s));
+            if (cq_has_min16(ws[i]->ggml_dtype)) CQ_HIP_CHECK(cq_launch_min16_term(ws[i], v, m, ys_dev[i], s));
+        }
+        return CQ_OK;
+    }
     for (int i = 0; i < count; i++) {
         const bool reuse = share && i > 0;
         if (int rc = qmatmul_impl(ws[i], x_dev, reuse ? cq_no_pre() : p, m, ys_dev[i], (reuse ? flags | CQ_FLAG_REUSE_ACT : flags) | det,

@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(256) quantize_q8k_kernel(const float *__restri
     q8k_chunk<AOS>(f, row, b_in_row, k, out);
 }
 
-// rms_norm in front of the quantizer: one workgroup of four waves per row.  The squares are added
+// rms_norm in front of the quantizer: one workgroup per row.  The squares are added
 // in a fixed order that does not depend on the kernel (the decode matvec's prologue follows it
 // too, so a row gives the same bits whatever the batch): groups of 8 consecutive elements as two
 // sequential sums of 4, added; a binary tree over the 32 groups of a 256-element chunk (group j
@@ -196,51 +196,87 @@ __global__ void __launch_bounds__(256) quantize_q8k_kernel(const float *__restri
 // adds all squares one after the other: the two sums agree to rounding, not to the bit.
 // scale = 1 / sqrt(mean + eps) multiplies the elements as in the reference's device kernel
 // (candle-kernels/src/reduce.cu:161-172; its CPU code divides every element by the root).  The
-// second pass reads the row again (from L2):
+// second pass:
 //   Q8_0 / Q8_1: quantizes scale * x * alpha chunk by chunk;
 //   Q8K: quantizes z = x * alpha and multiplies the block scales by `scale`: the quants of
 //        scale * z are those of z, and the decode matvec uses the same form.
 // ACT: 0 = Q8K, 1 = Q8_0, 2 = Q8_1.  Dynamic LDS: one float per chunk.
-template <bool AOS, int ACT>
-__global__ void __launch_bounds__(256) quantize_rms_rows_kernel(const float *__restrict__ x,
-                                                                const int32_t *__restrict__ row_ids, int64_t k,
-                                                                const float *__restrict__ alpha, float eps, Sink out) {
+// A wave keeps its first kRmsHeld chunks (NW * kRmsHeld * 256 elements of the row) in registers between the two passes.
+// Few rows are latency: 16 waves a row, so that a 4096-element row is one load per lane, and wave sums on DPP operands:
+// 4 rows of 4096: 9.3 us with four waves, LDS shuffles and a second read of the row.
+constexpr int kRmsHeld = 2;
+template <bool AOS, int ACT, int NW>
+__global__ void __launch_bounds__(NW * 64) quantize_rms_rows_kernel(const float *__restrict__ x,
+                                                                    const int32_t *__restrict__ row_ids, int64_t k,
+                                                                    const float *__restrict__ alpha, float eps, Sink out) {
     extern __shared__ float chunk_sums[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t row = blockIdx.x;
     const int64_t src_row = row_ids ? (int64_t)row_ids[row] : row;
     const float *xr = x + src_row * k;
-    const int64_t chunks = (k + 255) / 256;
-    clear_floats(out.clear);
-    for (int64_t c = wave; c < chunks; c += 4) {
-        const int64_t e0 = c * 256 + 4 * lane;
-        float t = 0.0f;
-        if (e0 < k) {
-            const float4 f = *(const float4 *)(xr + e0);
-            t = f.x * f.x;
-            t += f.y * f.y;
-            t += f.z * f.z;
-            t += f.w * f.w;
-        }
+    const int chunks = (int)((k + 255) / 256);
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 fx[kRmsHeld], ax[kRmsHeld];
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) t += __shfl_xor(t, off);
-        if (lane == 0) chunk_sums[c] = t;
+    for (int i = 0; i < kRmsHeld; i++) {
+        const int64_t e0 = (int64_t)(wave + i * NW) * 256 + 4 * lane;
+        fx[i] = e0 < k ? *(const float4 *)(xr + e0) : zero;
+        ax[i] = e0 < k ? *(const float4 *)(alpha + e0) : zero;
+    }
+    clear_floats(out.clear);
+    auto chunk_sum = [&](int c, const float4 f) {
+        float t = f.x * f.x;
+        t += f.y * f.y;
+        t += f.z * f.z;
+        t += f.w * f.w;
+        t += dpp_f<kQuadSwap1>(t);
+        t += dpp_f<kQuadSwap2>(t);
+        t += dpp_f<kHalfMirror>(t);
+        t += dpp_f<kRowMirror>(t);
+        const float s = (readlane_f(t, 0) + readlane_f(t, 16)) + (readlane_f(t, 32) + readlane_f(t, 48));
+        if (lane == 0) chunk_sums[c] = s;
+    };
+#pragma unroll
+    for (int i = 0; i < kRmsHeld; i++)
+        if (wave + i * NW < chunks) chunk_sum(wave + i * NW, fx[i]);
+    for (int c = wave + kRmsHeld * NW; c < chunks; c += NW) {
+        const int64_t e0 = (int64_t)c * 256 + 4 * lane;
+        chunk_sum(c, e0 < k ? *(const float4 *)(xr + e0) : zero);
     }
     __syncthreads();
     float sum2 = chunk_sums[0];
-    for (int64_t c = 1; c < chunks; c++) sum2 += chunk_sums[c];
+    int c = 1;
+    for (; c + 4 <= chunks; c += 4) {   // (four reads in flight, the additions in order)
+        const float s0 = chunk_sums[c], s1 = chunk_sums[c + 1], s2 = chunk_sums[c + 2], s3 = chunk_sums[c + 3];
+        sum2 += s0;
+        sum2 += s1;
+        sum2 += s2;
+        sum2 += s3;
+    }
+    for (; c < chunks; c++) sum2 += chunk_sums[c];
     const float scale = 1.0f / sqrtf(sum2 / (float)k + eps);
     // Q8K: a row whose scale is NaN, infinite or zero (NaN or infinities among its elements, squares that overflow) is
     // all NaN or all zero after the reference's normalisation and quantizes to zero blocks; z alone would not
     const float keep = scale > 0.0f && scale < __builtin_inff() ? 1.0f : __builtin_nanf("");
-    for (int64_t c = wave; c < chunks; c += 4) {
-        const int64_t e0 = c * 256 + 4 * lane;
-        const bool active = e0 < k;
-        float4 f = make_float4(0.f, 0.f, 0.f, 0.f), a = f;
-        if (active) { f = *(const float4 *)(xr + e0); a = *(const float4 *)(alpha + e0); }
+    auto quantize = [&](int c, const float4 f, const float4 a) {
+        const int64_t e0 = (int64_t)c * 256 + 4 * lane;
         if (ACT == 0) q8k_chunk<AOS, true>(make_float4(f.x * a.x * keep, f.y * a.y * keep, f.z * a.z * keep, f.w * a.w * keep), row, c, k, out, keep == keep ? scale : 0.0f);
-        else q8_0_chunk<AOS, ACT == 2>(rms_scale4(f, scale, a), active, row, e0, k, out);
+        else q8_0_chunk<AOS, ACT == 2>(rms_scale4(f, scale, a), e0 < k, row, e0, k, out);
+    };
+#pragma unroll
+    for (int i = 0; i < kRmsHeld; i++)
+        if (wave + i * NW < chunks) quantize(wave + i * NW, fx[i], ax[i]);
+    for (int c = wave + kRmsHeld * NW; c < chunks; c += NW) {
+        const int64_t e0 = (int64_t)c * 256 + 4 * lane;
+        const bool active = e0 < k;
+        quantize(c, active ? *(const float4 *)(xr + e0) : zero, active ? *(const float4 *)(alpha + e0) : zero);
     }
+}
+template <bool AOS, int ACT>
+void launch_rms(const float *x, const int32_t *row_ids, int64_t m, int64_t k, cq_pre pre, const Sink &out, hipStream_t s) {
+    const size_t lds = (size_t)((k + 255) / 256) * 4;
+    if (k <= 1024) quantize_rms_rows_kernel<AOS, ACT, 4><<<(unsigned)m, 256, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
+    else quantize_rms_rows_kernel<AOS, ACT, 16><<<(unsigned)m, 1024, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
 }
 
 template <bool AOS>
@@ -250,12 +286,10 @@ hipError_t launch(int act_dtype, const float *x, const int32_t *row_ids, int64_t
     if (act_dtype != CQ_DTYPE_Q8K && act_dtype != CQ_DTYPE_Q8_0 && act_dtype != CQ_DTYPE_Q8_1) return hipErrorInvalidValue;
     const int threads = 256, waves = threads / 64;
     if (pre.kind == CQ_PRE_RMS_NORM) {
-        const unsigned grid = (unsigned)m;
-        const size_t lds = (size_t)((k + 255) / 256) * 4;
-        if (lds > 48 * 1024) return hipErrorInvalidValue;   // rows of more than 3 million elements
-        if (act_dtype == CQ_DTYPE_Q8K) quantize_rms_rows_kernel<AOS, 0><<<grid, threads, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
-        else if (act_dtype == CQ_DTYPE_Q8_0) quantize_rms_rows_kernel<AOS, 1><<<grid, threads, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
-        else quantize_rms_rows_kernel<AOS, 2><<<grid, threads, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
+        if ((size_t)((k + 255) / 256) * 4 > 48 * 1024) return hipErrorInvalidValue;   // rows of more than 3 million elements
+        if (act_dtype == CQ_DTYPE_Q8K) launch_rms<AOS, 0>(x, row_ids, m, k, pre, out, s);
+        else if (act_dtype == CQ_DTYPE_Q8_0) launch_rms<AOS, 1>(x, row_ids, m, k, pre, out, s);
+        else launch_rms<AOS, 2>(x, row_ids, m, k, pre, out, s);
         return hipGetLastError();
     }
     const bool silu = pre.kind == CQ_PRE_SILU_MUL;

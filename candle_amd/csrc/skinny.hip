@@ -194,8 +194,8 @@ __device__ __forceinline__ void block_unpack(const uint8_t *wl, int lane, const 
 // DUMP (verification): the block integers, and the min term as the f16 MFMA delivers it from a zero accumulator,
 // are stored through `dump` instead of the result through `y`.
 template <int DT, int RT, bool DUMP>
-__device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_view &a, int64_t m0, int64_t m, float *__restrict__ y,
-                                            cq_mfma_dump dump) {
+__device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
+                                            float *__restrict__ y, cq_mfma_dump dump) {
     typedef Buf<DT, RT> B;
     constexpr bool MINS = is_k4(DT);
     constexpr int NT = (RT + 1) / 2;   // 16-row tiles
@@ -205,7 +205,7 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
     const int64_t k = w.k, kb = w.k >> 8;
-    const int64_t n_tile = tile_row(blockIdx.x, w.n);
+    const int64_t n_tile = tile_row(tile, w.n);
     uint8_t *buf = smem + wave * B::kBytes;
 
     // copy offsets: 8 rows x 128 B per instruction, chunks swizzled by the row
@@ -320,7 +320,7 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
 template <int DT, int RT, bool DUMP>
 __global__ void __launch_bounds__(kThreads) skinny_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
                                                           cq_mfma_dump dump) {
-    skinny_body<DT, RT, DUMP>(w, a, m0, m, y, dump);
+    skinny_body<DT, RT, DUMP>(w, a, blockIdx.x, m0, m, y, dump);
 }
 
 // ------------------------------------------------------------ resident-activation variant ----
@@ -758,8 +758,8 @@ template <typename F> __device__ __forceinline__ void each_block(int64_t left, F
 }
 
 template <int DT, int RT, bool DUMP>
-__device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_act_view &a, int64_t m0, int64_t m, float *__restrict__ y,
-                                                  cq_mfma_dump dump) {
+__device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
+                                                  float *__restrict__ y, cq_mfma_dump dump) {
     typedef BufQ8<RT> B;
     constexpr bool Q4 = DT == CQ_DTYPE_Q4_0;
     constexpr int NT = (RT + 1) / 2;   // 16-row tiles
@@ -768,7 +768,7 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
     const int64_t k = w.k, kg = (w.k + 255) >> 8, kb = w.k >> 5;
-    const int64_t n_tile = tile_row(blockIdx.x, w.n);
+    const int64_t n_tile = tile_row(tile, w.n);
     uint8_t *buf = smem + wave * B::kBytes;
 
     // copy offsets: 8 rows x 128 B per instruction, chunks swizzled by the row
@@ -888,7 +888,7 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
 template <int DT, int RT, bool DUMP>
 __global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
                                                                 cq_mfma_dump dump) {
-    skinny_blk32_body<DT, RT, DUMP>(w, a, m0, m, y, dump);
+    skinny_blk32_body<DT, RT, DUMP>(w, a, blockIdx.x, m0, m, y, dump);
 }
 
 // Mixture-of-experts form of the two: blockIdx.y is a tile of up to 8 * RT routed rows and names its expert's weights, so
@@ -906,8 +906,26 @@ __global__ void __launch_bounds__(kThreads) skinny_grouped_kernel(GroupArgs ga, 
     const int64_t m0 = ga.row0[tile], end = ga.row_end[tile], m = m0 + 8 * RT < end ? m0 + 8 * RT : end;
     const cq_weight w = ga.w[ga.expert[tile]];
     const cq_mfma_dump none{nullptr, nullptr, 0};
-    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, RT, false>(w, a, m0, m, y, none);
-    else skinny_body<DT, RT, false>(w, a, m0, m, y, none);
+    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, RT, false>(w, a, blockIdx.x, m0, m, y, none);
+    else skinny_body<DT, RT, false>(w, a, blockIdx.x, m0, m, y, none);
+}
+
+// Two or three weights on the same rows (q, k, v; gate and up): their 16-row tiles one after the other.  A weight with few
+// rows (1024: 64 workgroups) does not fill the machine by itself.
+constexpr int kMultiMax = 3;
+struct MultiArgs {
+    cq_weight w[kMultiMax];
+    float *y[kMultiMax];
+    uint32_t first[kMultiMax];   // first tile of the launch that is the weight's
+};
+template <int DT, int RT>
+__global__ void __launch_bounds__(kThreads) skinny_shared_kernel(MultiArgs ma, cq_act_view a, int64_t m) {
+    const uint32_t t = blockIdx.x;
+    const int i = t >= ma.first[2] ? 2 : t >= ma.first[1] ? 1 : 0;
+    const cq_weight w = ma.w[i];
+    const cq_mfma_dump none{nullptr, nullptr, 0};
+    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, RT, false>(w, a, t - ma.first[i], 0, m, ma.y[i], none);
+    else skinny_body<DT, RT, false>(w, a, t - ma.first[i], 0, m, ma.y[i], none);
 }
 
 // ------------------------------------------- the same with everything of a workgroup in flight at once ----
@@ -1391,6 +1409,17 @@ bool launch_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_
 }
 
 template <int DT, int RT>
+hipError_t launch_shared_rt(const MultiArgs &ma, unsigned tiles, cq_act_view a, int64_t m, hipStream_t s) {
+    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
+    if (hipError_t e = cq_ensure_lds<skinny_shared_kernel<DT, RT>>(ma.w[0].dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_shared_kernel<DT, RT>), tiles, kThreads, lds, s, ma, a, m);
+    return hipGetLastError();
+}
+template <int DT> hipError_t launch_shared(const MultiArgs &ma, unsigned tiles, cq_act_view a, int64_t m, hipStream_t s) {
+    return m <= 8 ? launch_shared_rt<DT, 1>(ma, tiles, a, m, s) : launch_shared_rt<DT, 2>(ma, tiles, a, m, s);
+}
+
+template <int DT, int RT>
 hipError_t launch_grouped_rt(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y, hipStream_t s) {
     GroupArgs ga;
     int tiles = 0;
@@ -1480,5 +1509,32 @@ hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_exper
     case CQ_DTYPE_Q4K: return launch_grouped<CQ_DTYPE_Q4K>(experts, n_experts, offsets, a, y, s);
     case CQ_DTYPE_Q5K: return launch_grouped<CQ_DTYPE_Q5K>(experts, n_experts, offsets, a, y, s);
     default: return launch_grouped<CQ_DTYPE_Q6K>(experts, n_experts, offsets, a, y, s);
+    }
+}
+
+bool cq_skinny_shared_takes(const cq_weight *const *ws, int count, int64_t m, int act_dtype) {
+    if (count < 2 || count > kMultiMax || m > 16) return false;
+    for (int i = 0; i < count; i++)
+        if (!cq_skinny_takes(ws[i], act_dtype)) return false;
+    return true;
+}
+
+hipError_t cq_launch_skinny_shared(const cq_weight *const *ws, int count, cq_act_view a, int64_t m, float *const *ys, hipStream_t s) {
+    if (a.m_stride < (m + 31) / 32 * 32) return hipErrorInvalidValue;   // whole 8-row groups are copied
+    MultiArgs ma;
+    int64_t tiles = 0;
+    for (int i = 0; i < kMultiMax; i++) {
+        const int j = i < count ? i : count - 1;   // (an unused place repeats the last weight and begins past the last tile)
+        ma.w[i] = *ws[j];
+        ma.y[i] = ys[j];
+        ma.first[i] = (uint32_t)tiles;
+        if (i < count) tiles += (ws[i]->n + 15) / 16;
+    }
+    switch (ws[0]->dtype) {
+    case CQ_DTYPE_Q8_0: return launch_shared<CQ_DTYPE_Q8_0>(ma, (unsigned)tiles, a, m, s);
+    case CQ_DTYPE_Q4_0: return launch_shared<CQ_DTYPE_Q4_0>(ma, (unsigned)tiles, a, m, s);
+    case CQ_DTYPE_Q4K: return launch_shared<CQ_DTYPE_Q4K>(ma, (unsigned)tiles, a, m, s);
+    case CQ_DTYPE_Q5K: return launch_shared<CQ_DTYPE_Q5K>(ma, (unsigned)tiles, a, m, s);
+    default: return launch_shared<CQ_DTYPE_Q6K>(ma, (unsigned)tiles, a, m, s);
     }
 }
