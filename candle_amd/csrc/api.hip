@@ -401,11 +401,15 @@ static size_t act_ws_layout(int act_dtype, int64_t m, int64_t k, uint8_t *base, 
         }
     } else {
         const size_t o_d = take((size_t)(m_pad * (k / 32)) * 4);
-        const size_t o_s = take((size_t)(m * (k / 32)) * 4);
-        const size_t o_h = take((size_t)(m_pad * (k / 32)) * 2);   // padded: the Q8_1 tile kernel copies whole tiles
+        const size_t o_s = take((size_t)(m * (k / 32)) * 2);
+        // Q8_0: the scales again, block-major; Q8_1: the `s` fields.  Padded: whole tiles are copied (and whole K steps of
+        // eight blocks).
+        const size_t o_t = take(act_dtype == CQ_DTYPE_Q8_1 ? (size_t)(m_pad * (k / 32)) * 2 : (size_t)(m_pad * ((k + 255) / 256)) * 32);
         if (base) {
             view.qs = (int8_t *)(base + o_qs); view.d = (float *)(base + o_d);
-            view.bsum32 = (int32_t *)(base + o_s); view.s16 = (uint16_t *)(base + o_h);
+            view.bsum32 = (int16_t *)(base + o_s);
+            if (act_dtype == CQ_DTYPE_Q8_1) view.s16 = (uint16_t *)(base + o_t);
+            else view.dT = (float *)(base + o_t);
         }
     }
     if (v) *v = view;
@@ -539,9 +543,13 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
                                 w->dtype, act, (long long)w->n);
         path = kSkinny;
     } else if (!(flags & CQ_FLAG_FORCE_MATVEC) && has_tile32) {
-        // Q8_0 / Q4_0 beyond 16 rows: their own tile kernel, measured ahead of the split-K kernel from 17 rows on at every
-        // shape
-        path = kGemm32;
+        // Q8_0 / Q4_0 beyond 16 rows: their own tile kernel, except for up to 32 rows of small weights, where it splits K into
+        // atomic additions and the split-K kernel is ahead (us at 17 / 32 rows, tiles against split K: Q8_0 1024 x 1024 10.4 / 10.5
+        // against 7.7, 4096 x 4096 12.1 / 13.6 against 11.8 / 12.8, 4096 x 14336 20.0 / 23.1 against 24.9 / 27.7; Q4_0 4096 x 4096
+        // 11.7 / 13.3 against 9.7 / 10.3, 8192 x 4096 14.2 / 17.2 against 12.3 / 15.4, 11008 x 4096 17.6 / 19.4 against 16.8 / 22.3)
+        const int64_t small = w->dtype == CQ_DTYPE_Q8_0 ? (1 << 24) : (1 << 25);
+        const bool few = !(flags & CQ_FLAG_FORCE_GEMM) && m <= 32 && w->n <= 8192 && w->n * w->k <= small && cq_skinny_takes(w, act);
+        path = few ? kSkinny : kGemm32;
     } else if (!(flags & (CQ_FLAG_FORCE_GEMM | CQ_FLAG_FORCE_MATVEC)) && (m >= skinny_from || (m >= 2 && !rows_fused)) &&
                cq_skinny_takes(w, act) && (skinny_rows || !has_tile_kernel)) {
         // (shapes the tile kernels do not take: the split-K kernel, 32 rows per pass over the weights, stays
@@ -737,12 +745,10 @@ extern "C" size_t cq_grouped_workspace_bytes(const cq_weight *const *experts, in
 
 // Most rows of one expert up to which the grouped split-K launch is taken.  Measured (8 experts, us of the whole call, split K /
 // tiles; at 1, 2, 8, 11, 20 rows for the fullest one): Q4K 14336 x 4096 19/29, 47/66, 58/70, 72/70, 97/72, 2816 x 1024 10/14 ..
-// 10.6/14.3, 13.4/14.3; Q8_0 14336 x 4096 30/35, 94/95, 107/101, 119/100, 2816 x 1024 10/14 .. 13/14, 23/15; Q4_0 14336 x 4096
-// 39/30, 2816 x 1024 10/13, 17/14.
+// 10.6/14.3, 13.4/14.3; Q4_0 14336 x 4096 19/29, 50/79, 57/81, 69/81, 110/83; Q8_0 14336 x 4096 31/36, 90/101, 102/102, 111/103,
+// 194/105, 2816 x 1024 9/13 .. 12/14, 22/15.
 static int64_t grouped_skinny_rows(const cq_weight *w) {
-    if (w->dtype == CQ_DTYPE_Q4_0) return w->n * w->k <= (4 << 20) ? 1 : 0;
-    if (w->dtype == CQ_DTYPE_Q8_0) return w->n * w->k <= (4 << 20) ? 16 : 2;
-    return 16;
+    return w->dtype == CQ_DTYPE_Q8_0 && w->n * w->k > (4 << 20) ? 4 : 16;
 }
 
 static int grouped_impl(const cq_weight *const *experts, int n_experts, const float *x_dev, cq_pre pre,
@@ -818,6 +824,7 @@ static int grouped_impl(const cq_weight *const *experts, int n_experts, const fl
         } else {
             ve.d += r0 * (w0->k / 32);
             ve.bsum32 += r0 * (w0->k / 32);
+            ve.dT += r0;
         }
         float *ye = y_dev + r0 * w0->n;
         const bool use_gemm = (flags & CQ_FLAG_FORCE_GEMM) ? true

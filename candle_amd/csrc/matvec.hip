@@ -1540,6 +1540,10 @@ hipError_t launch_fused_multi(const cq_weight *const *ws, int count, const float
 // against 10.5.  Every further row costs the dot products of one more row per unpacked unit, so the longer
 // the rows (elements per lane), the fewer rows pay off: K = 8192 Q4K 8.7 / 10.5 / 13.9 against 12.5,
 // K = 14336 Q4K 13.8 / 43 (registers spill) against 17.6.
+// Rows of at most 32 units leave half of a wave's lanes without one, at a fixed cost per weight row and activation row:
+// many of them go to the split-K kernel (Q4K 8192 x 2048 at 4 rows 8.5 against 7.5, 32000 x 2048 at 2 / 4 rows 14.4 / 21.0 against
+// 12.9, 32000 x 1024 13.6 / 20.8 against 9.8; Q4_0 32000 x 1024 at 3 / 4 rows 12.0 / 14.6 against 11.1), and so do four rows of
+// many long ones (32000 x 4096 Q4K 21.8 against 21.0, Q6K 28.9 against 27.1).
 bool cq_matvec_fused_rows_supported(const cq_weight *w, int64_t m) {
     if (m < 2 || m > 4 || !cq_matvec_fused_supported(w)) return false;
     int64_t units = 0, elems = 0;
@@ -1554,6 +1558,9 @@ bool cq_matvec_fused_rows_supported(const cq_weight *w, int64_t m) {
     }
     units = w->k / elems;
     if (units > (m == 2 ? 384 : 256) || row_bytes * (size_t)m > 64 * 1024 - 1024) return false;
+    const bool kquant = w->dtype == CQ_DTYPE_Q4K || w->dtype == CQ_DTYPE_Q5K || w->dtype == CQ_DTYPE_Q6K;
+    if (units <= 32 && ((kquant && w->n * m >= 28000) || (w->dtype == CQ_DTYPE_Q4_0 && w->n * m >= 90000))) return false;
+    if (m == 4 && w->n >= 16384 && kquant && w->dtype != CQ_DTYPE_Q5K) return false;
     const int64_t per_lane = (units + 63) / 64 * elems;   // elements of a row per lane
     return per_lane <= 64 ? true : per_lane <= 128 ? m <= 3 : m <= 2;
 }

@@ -59,18 +59,18 @@ struct cq_weight {
 // that int8 values are 16-byte aligned:
 //   Q8K : qs [m_stride][k] i8 ; d [m][k/256] f32 ; bsums [m][k/256][16] i16
 //   Q8_0: qs [m][k] i8 ; d [m][k/32]  f32 (the f16-rounded scale widened) ;
-//         bsum [m][k/32] i32 (sum of the 32 quants, for the Q4_0 "-8" term)
+//         bsum [m][k/32] i16 (sum of the 32 quants, for the Q4_0 "-8" term)
 // ---------------------------------------------------------------------------
 struct cq_act_view {
     int8_t *qs;
     float *d;
     int16_t *bsums;  // Q8K
-    // Q8K, for the matrix-core kernels (block-major so that a tile of rows is contiguous per block):
-    float *dT;         // [k/256][m_stride] f32, the same values as d
-    uint16_t *bsh;     // [k/256][m_stride][16] f16: the block's sixteen bsums as f16 (exact), the min term's operand
+    // For the matrix-core kernels (block-major so that a tile of rows is contiguous per block):
+    float *dT;         // Q8K [k/256][m_stride], Q8_0 [k/32][m_stride] f32, the same values as d
+    uint16_t *bsh;     // Q8K: [k/256][m_stride][16] f16: the block's sixteen bsums as f16 (exact), the min term's operand
     int64_t m_stride;  // rows allocated: at least 256 more than the rows quantized, so that the GEMM
                        // may read (and ignore) whole 128-row tiles past the last row
-    int32_t *bsum32; // Q8_0 / Q8_1
+    int16_t *bsum32; // Q8_0 / Q8_1: the block's sum of quants (at most 4096 in magnitude)
     uint16_t *s16;   // Q8_1: the block's `s` field (f16 bits)
 };
 

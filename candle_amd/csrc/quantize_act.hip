@@ -87,8 +87,9 @@ __device__ __forceinline__ void q8_0_chunk(const float4 f, bool active, int64_t 
         *(uint32_t *)(out.v.qs + row * k + e0) = packed;
         if (within == 0) {
             out.v.d[blk] = cq_h2f(dh);
-            out.v.bsum32[blk] = sum;
+            out.v.bsum32[blk] = (int16_t)sum;
             if (Q8_1) out.v.s16[blk] = sh;
+            else out.v.dT[(e0 / 32) * out.v.m_stride + row] = cq_h2f(dh);
         }
     }
 }

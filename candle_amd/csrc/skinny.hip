@@ -23,8 +23,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 // the same at four-byte alignment: scales of 32-element blocks in rows of no whole 256 elements
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef int v4i_a4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef float v4f_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 typedef short ss2 __attribute__((ext_vector_type(2)));
 typedef const void __attribute__((address_space(1))) *gptr_t;
@@ -731,18 +729,43 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
 
 // ---------------------------------------------------- Q8_0 / Q4_0 weights x Q8_0 activations ----
 // The same work split for 32-element blocks (k_quants.rs:618-649, :224-254: sumf += sumi * d_w *
-// d_x per block).  Q8_0 weights are int8 already and Q4_0 weights are one mask away from it, so the
+// d_x per block).  Q8_0 weights are int8 already and Q4_0 weights become q - 8 with two instructions a word, so the
 // operands go from LDS (almost) straight into the 16x16x32 MFMA, one per block, and each block's
-// 16 x 16 integers are scaled by the two block scales on the way into the f32 result.  Q4_0 holds
-// q - 8; the MFMA contracts q and 8 * (sum of the block's activations) comes off afterwards.  A wave
+// 16 x 16 integers are scaled by the two block scales on the way into the f32 result.  A wave
 // takes 256 elements (eight blocks) per step.
+// The activation scales come block-major (cq_act_view::dT), one LDS copy per group of eight rows and one 16-byte read per
+// block for a lane's four result rows.  (Row-major they took a 16-byte request per result row and half step from every
+// lane - 8 KiB of requests a step against 4 KiB of Q8_0 weights, twice that for Q4_0 with its block sums.)
 //   wgt : Q8_0 [2 row groups][2 K-halves][8 rows][8 chunks of 16 B], Q4_0 [2 row groups][8 rows][8 chunks
 //         = blocks]; chunk c of row r at c ^ (r%8)
 //   act : [RT row groups][2 K-halves][8 rows][8 chunks], same swizzle
-template <int RT> struct BufQ8 {
-    static constexpr int oAct = 4096, kRaw = oAct + RT * 2048;
-    static constexpr int kBytes = kRaw;   // >= 2 KiB of partial results
+//   d8  : [RT row groups][8 blocks][8 rows] f32
+template <int DT, int RT> struct BufQ8 {
+    static constexpr int oAct = DT == CQ_DTYPE_Q8_0 ? 4096 : 2048, oD8 = oAct + RT * 2048, kRaw = oD8 + RT * 256;
+    static constexpr int kBytes = kRaw;   // >= 1 KiB of partial results per 16 rows
 };
+
+// Activation scales of K step g for the rows m0 .. m0 + 8*RT - 1 into `lds` (row groups of 256 bytes).
+template <int RT> __device__ __forceinline__ void issue_scales(const cq_act_view &a, int64_t m0, int64_t g, uint8_t *lds, int lane) {
+    const uint32_t off = ((uint32_t)(lane >> 3) * (uint32_t)a.m_stride + (lane & 7)) * 4u;
+#pragma unroll
+    for (int rg = 0; rg < RT; rg++) dma4(a.dT + g * 8 * a.m_stride + m0 + rg * 8, off, lds + rg * 256);
+}
+// Where a lane finds the scales of result rows 4kq .. 4kq + 3 of tile t (+ 32 bytes per block); rows past the held groups
+// repeat the last group (they are not stored).
+template <int RT> __device__ __forceinline__ uint32_t scale_col(int t, uint32_t kq) {
+    const uint32_t rg = 2 * t + (kq >> 1) < RT ? 2 * t + (kq >> 1) : RT - 1;
+    return rg * 256u + (kq & 1) * 16u;
+}
+// Eight weight bytes of block b for the 16x16x32 MFMA out of a tile's LDS image.
+template <bool Q4> __device__ __forceinline__ long weight_bytes(const uint8_t *wl, int b, uint32_t r, uint32_t w4_col, uint32_t w4_shift, const uint32_t (&w_col)[4]) {
+    if (!Q4) return *(const long *)(wl + w_col[b & 3] + (b >> 2) * 1024);
+    const uint2 raw = *(const uint2 *)(wl + w4_col + (((uint32_t)b ^ (r & 7)) << 4));
+    // every byte minus 8, no carries between bytes
+    const uint32_t lo = (((raw.x >> w4_shift) & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;
+    const uint32_t hi = (((raw.y >> w4_shift) & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;
+    return (long)(((uint64_t)hi << 32) | lo);
+}
 
 // The eight blocks of a 256-element step, or the `left` that a row ends with (left is wave-uniform; the copies of such a step
 // also bring in what follows the row in memory, which nothing reads).
@@ -760,7 +783,7 @@ template <typename F> __device__ __forceinline__ void each_block(int64_t left, F
 template <int DT, int RT, bool DUMP>
 __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
                                                   float *__restrict__ y, cq_mfma_dump dump) {
-    typedef BufQ8<RT> B;
+    typedef BufQ8<DT, RT> B;
     constexpr bool Q4 = DT == CQ_DTYPE_Q4_0;
     constexpr int NT = (RT + 1) / 2;   // 16-row tiles
     extern __shared__ __align__(16) uint8_t smem[];
@@ -779,7 +802,7 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
     // Q4_0 weights: chunk b, bytes 8(kq%2) .. +8, low nibbles for kq < 2, high nibbles above
     const uint32_t w4_col = (r >> 3) * 1024u + (r & 7) * 128u + (kq & 1) * 8u, w4_shift = 4 * (kq >> 1);
     uint32_t w_col[4], a_col[NT][4];
-    int64_t a_row[NT][4];   // rows whose scales this lane applies (results rows 4kq + i of tile t)
+    uint32_t s_col[NT];
 #pragma unroll
     for (uint32_t c = 0; c < 4; c++) w_col[c] = (r >> 3) * 2048u + (r & 7) * 128u + (((2 * c + (kq >> 1)) ^ (r & 7)) << 4) + (kq & 1) * 8u;
 #pragma unroll
@@ -788,11 +811,7 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
 #pragma unroll
         for (uint32_t c = 0; c < 4; c++)
             a_col[t][c] = B::oAct + (row >> 3) * 2048u + (row & 7) * 128u + (((2 * c + (kq >> 1)) ^ (row & 7)) << 4) + (kq & 1) * 8u;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int64_t row_i = m0 + t * 16 + 4 * kq + i;
-            a_row[t][i] = row_i < m ? row_i : m - 1;
-        }
+        s_col[t] = B::oD8 + scale_col<RT>(t, kq);
     }
 
     v4f out[NT];
@@ -815,48 +834,27 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
             const int rg = i >> 1, kh = i & 1;
             dma16(a.qs + (m0 + rg * 8) * k + g * 256 + kh * 128, row_off, buf + B::oAct + i * 1024);
         }
-        // the eight block scales of this lane's weight row, and of the activation rows it scales
+        issue_scales<RT>(a, m0, g, buf + B::oD8, lane);
+        // the eight block scales of this lane's weight row
         const u32x4_a4 dwv = *(const u32x4_a4 *)(w.p1 + ((n_tile + r) * kb + g * 8) * 2);
-        v4f da[NT][4][2];
-        v4i bs[Q4 ? NT : 1][4][2];   // Q4_0: the sums of the activation blocks
-#pragma unroll
-        for (int t = 0; t < NT; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const v4f_a4 *p = (const v4f_a4 *)(a.d + a_row[t][i] * kb + g * 8);
-                da[t][i][0] = p[0];
-                da[t][i][1] = p[1];
-                if (Q4) {
-                    const v4i_a4 *q = (const v4i_a4 *)(a.bsum32 + a_row[t][i] * kb + g * 8);
-                    bs[t][i][0] = q[0];
-                    bs[t][i][1] = q[1];
-                }
-            }
         __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
 
         const uint32_t dww[4] = {dwv.x, dwv.y, dwv.z, dwv.w};
         auto block = [&](int b) {
             const float dw = cq_h2f((uint16_t)(dww[b >> 1] >> (16 * (b & 1))));
-            long wv;
-            if (Q4) {
-                const uint2 raw = *(const uint2 *)(buf + w4_col + (((uint32_t)b ^ (r & 7)) << 4));
-                const uint32_t lo = (raw.x >> w4_shift) & 0x0F0F0F0Fu, hi = (raw.y >> w4_shift) & 0x0F0F0F0Fu;
-                wv = (long)(((uint64_t)hi << 32) | lo);
-            } else {
-                wv = *(const long *)(buf + w_col[b & 3] + (b >> 2) * 1024);
-            }
+            const long wv = weight_bytes<Q4>(buf, b, r, w4_col, w4_shift, w_col);
 #pragma unroll
             for (int t = 0; t < NT; t++) {
                 const long av = *(const long *)(buf + a_col[t][b & 3] + (b >> 2) * 1024);
+                const v4f da = *(const v4f *)(buf + s_col[t] + b * 32);
                 const v4i acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, wv, (v4i){0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const int I = Q4 ? acc[i] - 8 * bs[Q4 ? t : 0][i][b >> 2][b & 3] : acc[i];
                     if (DUMP) {
                         const int64_t orow = m0 + t * 16 + kq * 4 + i;
-                        if (orow < m) dump.i[(orow * w.n + n_tile + r) * kb + g * 8 + b] = I;
+                        if (orow < m) dump.i[(orow * w.n + n_tile + r) * kb + g * 8 + b] = acc[i];
                     } else {
-                        out[t][i] = __builtin_fmaf((float)I * dw, da[t][i][b >> 2][b & 3], out[t][i]);
+                        out[t][i] = __builtin_fmaf((float)acc[i] * dw, da[i], out[t][i]);
                     }
                 }
             }
@@ -934,15 +932,13 @@ __global__ void __launch_bounds__(kThreads) skinny_shared_kernel(MultiArgs ma, c
 // compute units) and the call's quantized rows fit the LDS beside the weights, every wave requests all it will need -
 // the activation slices, scales and weights of the K groups it owns (wave w: groups w, w + kWaves, ...) - right away,
 // a single memory round trip, and the arithmetic follows as the data lands.
-//   per K group g : act [RT][2 K-halves][8 rows][8 chunks], swizzled as above | d [8*RT rows][8] f32 |
-//                   Q4_0: bs [8*RT rows][8] i32 (sums of the activation blocks)
+//   per K group g : act [RT][2 K-halves][8 rows][8 chunks], swizzled as above | d8 [RT row groups][8 blocks][8 rows] f32
 //   then, per group: the 16 weight rows (Q8_0 4 KiB, Q4_0 2 KiB); a wave's first weight buffer also carries its
 //                   partial results (1 KiB per 16 activation rows)
 template <int DT, int RT> struct ResQ8 {
     static constexpr bool Q4 = DT == CQ_DTYPE_Q4_0;
     static constexpr int kWgt = Q4 ? 2048 : 4096;
-    static constexpr int oD = RT * 2048, oBs = oD + RT * 256;
-    static constexpr int kActGrp = oBs + (Q4 ? RT * 256 : 0);
+    static constexpr int oD = RT * 2048, kActGrp = oD + RT * 256;
     static size_t bytes(int64_t kg) { return (size_t)kg * (kActGrp + kWgt); }
 };
 
@@ -964,10 +960,6 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_w
     const uint32_t r8 = lane >> 3, c8 = lane & 7;
     const uint32_t row_off = r8 * (uint32_t)k + ((c8 ^ r8) << 4);
     const uint32_t q4_off = r8 * (uint32_t)(k >> 1) + ((c8 ^ r8) << 4);
-    // the scales (and block sums) of row l / 2, half l % 2 of its eight blocks; rows past the last one repeat it
-    // (their planes are not padded)
-    const int64_t srow = (int64_t)(lane >> 1) < m ? (lane >> 1) : m - 1;
-    const uint32_t sc_off = (uint32_t)(srow * kb * 4) + (lane & 1) * 16u;
     const uint32_t w4_col = (r >> 3) * 1024u + (r & 7) * 128u + (kq & 1) * 8u, w4_shift = 4 * (kq >> 1);
     uint32_t w_col[4], a_col[NT][4];
 #pragma unroll
@@ -997,8 +989,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_w
                 const int rg = i >> 1, kh = i & 1;
                 dma16(a.qs + (int64_t)(rg * 8) * k + g * 256 + kh * 128, row_off, act + i * 1024);
             }
-            if (lane < 16 * RT) dma16((const uint8_t *)(a.d + g * 8), sc_off, act + R::oD);
-            if (Q4 && lane < 16 * RT) dma16((const uint8_t *)(a.bsum32 + g * 8), sc_off, act + R::oBs);
+            issue_scales<RT>(a, 0, g, act + R::oD, lane);
             if (Q4) {
 #pragma unroll
                 for (int rg = 0; rg < 2; rg++) dma16(w.p0 + (n_tile + rg * 8) * (k >> 1) + g * 128, q4_off, wl + rg * 1024);
@@ -1024,29 +1015,19 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_w
             const uint32_t dww[4] = {dwv[j].x, dwv[j].y, dwv[j].z, dwv[j].w};
             auto block = [&](int b) {
                 const float dw = cq_h2f((uint16_t)(dww[b >> 1] >> (16 * (b & 1))));
-                long wv;
-                if (Q4) {
-                    const uint2 raw = *(const uint2 *)(wl + w4_col + (((uint32_t)b ^ (r & 7)) << 4));
-                    const uint32_t lo = (raw.x >> w4_shift) & 0x0F0F0F0Fu, hi = (raw.y >> w4_shift) & 0x0F0F0F0Fu;
-                    wv = (long)(((uint64_t)hi << 32) | lo);
-                } else {
-                    wv = *(const long *)(wl + w_col[b & 3] + (b >> 2) * 1024);
-                }
+                const long wv = weight_bytes<Q4>(wl, b, r, w4_col, w4_shift, w_col);
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
                     const long av = *(const long *)(act + a_col[t][b & 3] + (b >> 2) * 1024);
+                    const v4f da = *(const v4f *)(act + R::oD + scale_col<RT>(t, kq) + b * 32);
                     const v4i acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, wv, (v4i){0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        // scales of result row 4kq + i of tile t (rows past the held groups: the last one, not stored)
-                        const uint32_t srow_i = t * 16 + 4 * kq + i < 8u * RT ? t * 16 + 4 * kq + i : 8u * RT - 1;
-                        const float da = *(const float *)(act + R::oD + srow_i * 32 + b * 4);
-                        const int I = Q4 ? acc[i] - 8 * *(const int32_t *)(act + R::oBs + srow_i * 32 + b * 4) : acc[i];
                         if (DUMP) {
                             const int64_t orow = t * 16 + kq * 4 + i;
-                            if (orow < m) dump.i[(orow * w.n + n_tile + r) * kb + g * 8 + b] = I;
+                            if (orow < m) dump.i[(orow * w.n + n_tile + r) * kb + g * 8 + b] = acc[i];
                         } else {
-                            out[t][i] = __builtin_fmaf((float)I * dw, da, out[t][i]);
+                            out[t][i] = __builtin_fmaf((float)acc[i] * dw, da[i], out[t][i]);
                         }
                     }
                 }
@@ -1127,13 +1108,7 @@ __device__ __forceinline__ void blk32_multi_step(uint8_t *__restrict__ slot, con
     long wv[8];
 #pragma unroll
     for (int b = 0; b < 8; b++) {
-        if (Q4) {
-            const uint2 raw = *(const uint2 *)(slot + w4_col + (((uint32_t)b ^ (r & 7)) << 4));
-            const uint32_t lo = (raw.x >> w4_shift) & 0x0F0F0F0Fu, hi = (raw.y >> w4_shift) & 0x0F0F0F0Fu;
-            wv[b] = (long)(((uint64_t)hi << 32) | lo);
-        } else {
-            wv[b] = *(const long *)(slot + w_col[b & 3] + (b >> 2) * 1024);
-        }
+        wv[b] = weight_bytes<Q4>(slot, b, r, w4_col, w4_shift, w_col);
     }
     if (ahead) {
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the reads above are done with the slot
@@ -1143,18 +1118,15 @@ __device__ __forceinline__ void blk32_multi_step(uint8_t *__restrict__ slot, con
     auto block = [&](int b) {
         const float dw = cq_h2f((uint16_t)(dww[b >> 1] >> (16 * (b & 1))));
         const long av = *(const long *)(act + a_col[b & 3] + (b >> 2) * 1024);
+        const v4f da = *(const v4f *)(act + R::oD + scale_col<RT>(0, kq) + b * 32);
         const v4i acc = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, wv[b], (v4i){0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            // scales of result row 4kq + i (rows past the held groups: the last one, not stored)
-            const uint32_t srow_i = 4 * kq + i < 8u * RT ? 4 * kq + i : 8u * RT - 1;
-            const float da = *(const float *)(act + R::oD + srow_i * 32 + b * 4);
-            const int I = Q4 ? acc[i] - 8 * *(const int32_t *)(act + R::oBs + srow_i * 32 + b * 4) : acc[i];
             if (DUMP) {
                 const int64_t orow = kq * 4 + i;
-                if (orow < m) dump.i[at + orow * rs + b] = I;
+                if (orow < m) dump.i[at + orow * rs + b] = acc[i];
             } else {
-                out[i] = __builtin_fmaf((float)I * dw, da, out[i]);
+                out[i] = __builtin_fmaf((float)acc[i] * dw, da[i], out[i]);
             }
         }
     };
@@ -1185,8 +1157,6 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_multi_kernel(cq_weig
     const uint32_t row_off = r8 * (uint32_t)k + ((c8 ^ r8) << 4);
     const uint32_t q4_off = r8 * (uint32_t)(k >> 1) + ((c8 ^ r8) << 4);
     const uint32_t ws_off = (uint32_t)lane * (uint32_t)kb * 2u;   // lanes 0..15: the scales of row `lane`
-    const int64_t srow = (int64_t)(lane >> 1) < m ? (lane >> 1) : m - 1;
-    const uint32_t sc_off = (uint32_t)(srow * kb * 4) + (lane & 1) * 16u;
     const uint32_t w4_col = (r >> 3) * 1024u + (r & 7) * 128u + (kq & 1) * 8u, w4_shift = 4 * (kq >> 1);
     uint32_t w_col[4], a_col[4];
     {
@@ -1207,8 +1177,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_multi_kernel(cq_weig
             const int rg = i >> 1, kh = i & 1;
             dma16(a.qs + (int64_t)(rg * 8) * k + g * 256 + kh * 128, row_off, act + i * 1024);
         }
-        if (lane < 16 * RT) dma16((const uint8_t *)(a.d + g * 8), sc_off, act + R::oD);
-        if (Q4 && lane < 16 * RT) dma16((const uint8_t *)(a.bsum32 + g * 8), sc_off, act + R::oBs);
+        issue_scales<RT>(a, 0, g, act + R::oD, lane);
     }
     for (int64_t t0 = blockIdx.x; t0 < tiles; t0 += kTilesPerRound * G) {
         int cnt = (int)((tiles - t0 + G - 1) / G);
@@ -1305,7 +1274,7 @@ bool launch_blk32_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq
 // DUMP (all launchers below): the launch cq_launch_skinny would make, storing the block integers through `d`.
 template <int DT, int RT, bool DUMP>
 hipError_t launch_blk32_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    const size_t lds = (size_t)BufQ8<RT>::kBytes * kWaves;
+    const size_t lds = (size_t)BufQ8<DT, RT>::kBytes * kWaves;
     if (hipError_t e = cq_ensure_lds<skinny_blk32_kernel<DT, RT, DUMP>>(w->dev, lds); e != hipSuccess) return e;
     CQ_LAUNCH((skinny_blk32_kernel<DT, RT, DUMP>), (unsigned)((w->n + 15) / 16), kThreads, lds, s, *w, a, m0, m, y, d);
     return hipGetLastError();
@@ -1410,7 +1379,7 @@ bool launch_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_
 
 template <int DT, int RT>
 hipError_t launch_shared_rt(const MultiArgs &ma, unsigned tiles, cq_act_view a, int64_t m, hipStream_t s) {
-    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
+    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<DT, RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
     if (hipError_t e = cq_ensure_lds<skinny_shared_kernel<DT, RT>>(ma.w[0].dev, lds); e != hipSuccess) return e;
     CQ_LAUNCH((skinny_shared_kernel<DT, RT>), tiles, kThreads, lds, s, ma, a, m);
     return hipGetLastError();
@@ -1433,7 +1402,7 @@ hipError_t launch_grouped_rt(const cq_weight *const *experts, int n_experts, con
         }
     }
     if (tiles == 0) return hipSuccess;
-    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
+    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<DT, RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
     if (hipError_t e = cq_ensure_lds<skinny_grouped_kernel<DT, RT>>(experts[0]->dev, lds); e != hipSuccess) return e;
     CQ_LAUNCH((skinny_grouped_kernel<DT, RT>), dim3((unsigned)((experts[0]->n + 15) / 16), (unsigned)tiles), kThreads, lds, s, ga, a, y);
     return hipGetLastError();
