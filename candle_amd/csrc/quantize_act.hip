@@ -16,6 +16,8 @@
 // has a kernel of its own with one workgroup per row.
 #include "qhip_internal.h"
 
+#include <type_traits>
+
 namespace {
 
 __device__ __forceinline__ float silu_f(float v) { return v / (1.0f + expf(-v)); }
@@ -117,7 +119,8 @@ __global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *__restr
 
 // Q8K: one 256-element block per wave.
 // `f` = the lane's four values of block b_in_row of `row`; called by all 64 lanes.  SCALED: the
-// block's scale is multiplied by `dscale` on the way out (the block then stands for dscale * f).
+// block's scale is multiplied by `dscale` on the way out (the block then stands for dscale * f; a
+// zero block if dscale is 0), which nothing before waits for.
 template <bool AOS, bool SCALED = false>
 __device__ __forceinline__ void q8k_chunk(const float4 f, int64_t row, int64_t b_in_row, int64_t k, const Sink &out,
                                           float dscale = 1.0f) {
@@ -151,7 +154,12 @@ __device__ __forceinline__ void q8k_chunk(const float4 f, int64_t row, int64_t b
                  ((uint32_t)(uint8_t)q3 << 24);
         sum = (int)q0 + (int)q1 + (int)q2 + (int)q3;
         d = 1.0f / iscale;
-        if (SCALED) d *= dscale;
+        if (SCALED) {
+            const bool zero = dscale == 0.0f;
+            packed = zero ? 0 : packed;
+            sum = zero ? 0 : sum;
+            d = zero ? 0.0f : d * dscale;
+        }
     }
     sum += dpp_i<kQuadSwap1>(sum);
     sum += dpp_i<kQuadSwap2>(sum);  // lanes 4j..4j+3 now hold bsums[j]
@@ -203,71 +211,104 @@ __global__ void __launch_bounds__(256) quantize_q8k_kernel(const float *__restri
 //        scale * z are those of z, and the decode matvec uses the same form.
 // ACT: 0 = Q8K, 1 = Q8_0, 2 = Q8_1.  Dynamic LDS: one float per chunk.
 // A wave keeps its first kRmsHeld chunks (NW * kRmsHeld * 256 elements of the row) in registers between the two passes.
-// Few rows are latency: 16 waves a row, so that a 4096-element row is one load per lane, and wave sums on DPP operands:
-// 4 rows of 4096: 9.3 us with four waves, LDS shuffles and a second read of the row.
-constexpr int kRmsHeld = 2;
-template <bool AOS, int ACT, int NW>
+// Few rows are latency, and what a wave computes (about 400 instructions): sixteen waves of one row share the four vector
+// units of a CU.  SPLIT: a row is spread over workgroups of kRmsSplit waves, each of which adds the squares of the whole row
+// (from L2, four chunks side by side) and quantizes one chunk a wave; the same bits.  Kernel alone, us, one workgroup a row of
+// sixteen waves -> split, 4 rows of Q8K: 4096 5.5 -> 4.5, 8192 8.3 -> 5.9, 16384 14.2 -> 8.4.  Up to 2048 elements the sixteen
+// waves are as fast (3.7), and with more workgroups than CUs the second sum of the row costs more than it gives
+// (64 rows of 8192: 8.4 against 8.8).  Eight waves a workgroup: 4096 5.2, 16384 7.6.
+constexpr int kRmsHeld = 2, kRmsSplit = 4;
+template <bool AOS, int ACT, int NW, bool SPLIT>
 __global__ void __launch_bounds__(NW * 64) quantize_rms_rows_kernel(const float *__restrict__ x,
                                                                     const int32_t *__restrict__ row_ids, int64_t k,
                                                                     const float *__restrict__ alpha, float eps, Sink out) {
-    extern __shared__ float chunk_sums[];
+    extern __shared__ __align__(16) float chunk_sums[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t row = blockIdx.x;
+    const int chunks = (int)((k + 255) / 256), parts = SPLIT ? (chunks + NW - 1) / NW : 1;
+    const int64_t row = blockIdx.x / parts;
+    const int part = (int)(blockIdx.x - row * parts);
     const int64_t src_row = row_ids ? (int64_t)row_ids[row] : row;
     const float *xr = x + src_row * k;
-    const int chunks = (int)((k + 255) / 256);
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 fx[kRmsHeld], ax[kRmsHeld];
+    constexpr int kHeld = SPLIT ? 1 : kRmsHeld;
+    float4 fx[kHeld], ax[kHeld];
 #pragma unroll
-    for (int i = 0; i < kRmsHeld; i++) {
-        const int64_t e0 = (int64_t)(wave + i * NW) * 256 + 4 * lane;
+    for (int i = 0; i < kHeld; i++) {
+        const int64_t e0 = (int64_t)(wave + (SPLIT ? part : i) * NW) * 256 + 4 * lane;
         fx[i] = e0 < k ? *(const float4 *)(xr + e0) : zero;
         ax[i] = e0 < k ? *(const float4 *)(alpha + e0) : zero;
     }
     clear_floats(out.clear);
-    auto chunk_sum = [&](int c, const float4 f) {
-        float t = f.x * f.x;
-        t += f.y * f.y;
-        t += f.z * f.z;
-        t += f.w * f.w;
-        t += dpp_f<kQuadSwap1>(t);
-        t += dpp_f<kQuadSwap2>(t);
-        t += dpp_f<kHalfMirror>(t);
-        t += dpp_f<kRowMirror>(t);
-        const float s = (readlane_f(t, 0) + readlane_f(t, 16)) + (readlane_f(t, 32) + readlane_f(t, 48));
-        if (lane == 0) chunk_sums[c] = s;
-    };
+    // the sums of N chunks c, c + NW, ... (side by side: each is a chain of dependent additions)
+    auto chunk_sums_of = [&](auto N, int c, const float4 *f) {
+        float t[N], v = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kRmsHeld; i++)
-        if (wave + i * NW < chunks) chunk_sum(wave + i * NW, fx[i]);
-    for (int c = wave + kRmsHeld * NW; c < chunks; c += NW) {
-        const int64_t e0 = (int64_t)c * 256 + 4 * lane;
-        chunk_sum(c, e0 < k ? *(const float4 *)(xr + e0) : zero);
+        for (int i = 0; i < N; i++) {
+            t[i] = f[i].x * f[i].x;
+            t[i] += f[i].y * f[i].y;
+            t[i] += f[i].z * f[i].z;
+            t[i] += f[i].w * f[i].w;
+        }
+#pragma unroll
+        for (int i = 0; i < N; i++) t[i] += dpp_f<kQuadSwap1>(t[i]);
+#pragma unroll
+        for (int i = 0; i < N; i++) t[i] += dpp_f<kQuadSwap2>(t[i]);
+#pragma unroll
+        for (int i = 0; i < N; i++) t[i] += dpp_f<kHalfMirror>(t[i]);
+#pragma unroll
+        for (int i = 0; i < N; i++) t[i] += dpp_f<kRowMirror>(t[i]);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const float s = (readlane_f(t[i], 0) + readlane_f(t[i], 16)) + (readlane_f(t[i], 32) + readlane_f(t[i], 48));
+            v = lane == i ? s : v;
+        }
+        if (lane < N && c + lane * NW < chunks) chunk_sums[c + lane * NW] = v;
+    };
+    // (zeros up to a multiple of 16 chunks: the sum below reads sixteen at a time)
+    const int padded = (chunks + 15) / 16 * 16;
+    if ((int)threadIdx.x < padded - chunks) chunk_sums[chunks + threadIdx.x] = 0.0f;
+    constexpr std::integral_constant<int, SPLIT ? 4 : kHeld> at_once{};
+    if constexpr (!SPLIT) chunk_sums_of(at_once, wave, fx);
+    for (int c = SPLIT ? wave : wave + kHeld * NW; c < chunks; c += at_once * NW) {
+        float4 f[at_once];
+#pragma unroll
+        for (int i = 0; i < at_once; i++) {
+            const int64_t e0 = (int64_t)(c + i * NW) * 256 + 4 * lane;
+            f[i] = e0 < k ? *(const float4 *)(xr + e0) : zero;
+        }
+        chunk_sums_of(at_once, c, f);
     }
     __syncthreads();
-    float sum2 = chunk_sums[0];
-    int c = 1;
-    for (; c + 4 <= chunks; c += 4) {   // (four reads in flight, the additions in order)
-        const float s0 = chunk_sums[c], s1 = chunk_sums[c + 1], s2 = chunk_sums[c + 2], s3 = chunk_sums[c + 3];
-        sum2 += s0;
-        sum2 += s1;
-        sum2 += s2;
-        sum2 += s3;
+    float sum2 = 0.0f;
+    for (int c = 0; c < padded; c += 16) {   // (sixteen reads in flight, the additions in order)
+        float4 s4[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) s4[i] = *(const float4 *)(chunk_sums + c + 4 * i);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            sum2 += s4[i].x;
+            sum2 += s4[i].y;
+            sum2 += s4[i].z;
+            sum2 += s4[i].w;
+        }
     }
-    for (; c < chunks; c++) sum2 += chunk_sums[c];
     const float scale = 1.0f / sqrtf(sum2 / (float)k + eps);
     // Q8K: a row whose scale is NaN, infinite or zero (NaN or infinities among its elements, squares that overflow) is
     // all NaN or all zero after the reference's normalisation and quantizes to zero blocks; z alone would not
-    const float keep = scale > 0.0f && scale < __builtin_inff() ? 1.0f : __builtin_nanf("");
+    const float q8k_scale = scale > 0.0f && scale < __builtin_inff() ? scale : 0.0f;
     auto quantize = [&](int c, const float4 f, const float4 a) {
         const int64_t e0 = (int64_t)c * 256 + 4 * lane;
-        if (ACT == 0) q8k_chunk<AOS, true>(make_float4(f.x * a.x * keep, f.y * a.y * keep, f.z * a.z * keep, f.w * a.w * keep), row, c, k, out, keep == keep ? scale : 0.0f);
+        if (ACT == 0) q8k_chunk<AOS, true>(make_float4(f.x * a.x, f.y * a.y, f.z * a.z, f.w * a.w), row, c, k, out, q8k_scale);
         else q8_0_chunk<AOS, ACT == 2>(rms_scale4(f, scale, a), e0 < k, row, e0, k, out);
     };
+    if constexpr (SPLIT) {
+        if (part * NW + wave < chunks) quantize(part * NW + wave, fx[0], ax[0]);
+        return;
+    }
 #pragma unroll
-    for (int i = 0; i < kRmsHeld; i++)
+    for (int i = 0; i < kHeld; i++)
         if (wave + i * NW < chunks) quantize(wave + i * NW, fx[i], ax[i]);
-    for (int c = wave + kRmsHeld * NW; c < chunks; c += NW) {
+    for (int c = wave + kHeld * NW; c < chunks; c += NW) {
         const int64_t e0 = (int64_t)c * 256 + 4 * lane;
         const bool active = e0 < k;
         quantize(c, active ? *(const float4 *)(xr + e0) : zero, active ? *(const float4 *)(alpha + e0) : zero);
@@ -275,9 +316,12 @@ __global__ void __launch_bounds__(NW * 64) quantize_rms_rows_kernel(const float 
 }
 template <bool AOS, int ACT>
 void launch_rms(const float *x, const int32_t *row_ids, int64_t m, int64_t k, cq_pre pre, const Sink &out, hipStream_t s) {
-    const size_t lds = (size_t)((k + 255) / 256) * 4;
-    if (k <= 1024) quantize_rms_rows_kernel<AOS, ACT, 4><<<(unsigned)m, 256, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
-    else quantize_rms_rows_kernel<AOS, ACT, 16><<<(unsigned)m, 1024, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
+    const int64_t chunks = (k + 255) / 256, parts = (chunks + kRmsSplit - 1) / kRmsSplit;
+    const size_t lds = (size_t)(chunks + 15) / 16 * 64;
+    if (chunks <= 4) quantize_rms_rows_kernel<AOS, ACT, 4, false><<<(unsigned)m, 256, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
+    else if (chunks > 8 && m * parts <= cq_num_cus())
+        quantize_rms_rows_kernel<AOS, ACT, kRmsSplit, true><<<(unsigned)(m * parts), kRmsSplit * 64, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
+    else quantize_rms_rows_kernel<AOS, ACT, 16, false><<<(unsigned)m, 1024, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
 }
 
 template <bool AOS>
