@@ -48,6 +48,11 @@ __device__ __forceinline__ void clear_floats(const cq_clear &c) {
     }
 }
 
+// a / b of non-negative numbers (a 64-bit division is a hundred vector instructions)
+__device__ __forceinline__ int64_t divide(int64_t a, int64_t b) {
+    return ((uint64_t)a | (uint64_t)b) >> 32 ? a / b : (int64_t)((uint32_t)a / (uint32_t)b);
+}
+
 __device__ __forceinline__ int8_t round_to_i8(float v) { return cq_as_i8(roundf(v)); }
 
 // Q8_0 / Q8_1: eight 32-element blocks per wave, 8 lanes per block.  `f` = the lane's four values
@@ -105,7 +110,7 @@ __global__ void __launch_bounds__(256) quantize_q8_0_kernel(const float *__restr
     const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     clear_floats(out.clear);
     if (wave >= m * chunks_per_row) return;
-    const int64_t row = wave / chunks_per_row;
+    const int64_t row = divide(wave, chunks_per_row);
     const int64_t e0 = (wave - row * chunks_per_row) * 256 + 4 * lane;
     const bool active = e0 < k;  // k % 32 == 0, so a lane is either fully inside or fully outside
     const int64_t src_row = row_ids ? (int64_t)row_ids[row] : row;
@@ -180,6 +185,106 @@ __device__ __forceinline__ void q8k_chunk(const float4 f, int64_t row, int64_t b
     }
 }
 
+// Many rows: a block per sixteen lanes, four blocks a wave.  Lane l of a block's sixteen holds elements 64i + 4l .. + 3 (i = 0..3),
+// reductions end inside the sixteen lanes and every scalar step of a block (index, two divisions, stores) is shared by four.
+// A wave a block (the kernel below) spends about 250 vector instructions on it and is bound by them; here memory is.  Kernel
+// alone, us, with a wave a block -> here: 512 x 4096 6.0 -> 3.3, 1024 x 4096 9.2 -> 5.7, 4096 x 4096 22.3 -> 15.4 (5.5 TB/s), with
+// silu 32.9 -> 26.5, 4096 x 14336 123 -> 105.
+// The signed extremes replace the search for the first largest |x|: only where both signs reach it does the position decide.
+template <bool AOS, bool SILU>
+__global__ void __launch_bounds__(256) quantize_q8k_quad_kernel(const float *__restrict__ x, const int32_t *__restrict__ row_ids,
+                                                                uint32_t blocks, uint32_t kb, const float *__restrict__ x2, Sink out) {
+    clear_floats(out.clear);
+    const uint32_t l = threadIdx.x & 15;
+    const uint32_t blk = blockIdx.x * 16 + (threadIdx.x >> 4);
+    const bool active = blk < blocks;
+    const uint32_t at = active ? blk : blocks - 1;
+    const uint32_t row = at / kb, b_in_row = at - row * kb;
+    const int64_t k = (int64_t)kb * 256, src_row = row_ids ? (int64_t)row_ids[row] : row;
+    const int64_t src = src_row * k + b_in_row * 256 + 4 * l;
+    float4 f[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) f[i] = *(const float4 *)(x + src + 64 * i);
+    if (SILU) {
+        float4 g[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) g[i] = *(const float4 *)(x2 + src + 64 * i);
+#pragma unroll
+        for (int i = 0; i < 4; i++) f[i] = silu_mul4(f[i], g[i]);
+    }
+    float hi = 0.0f, lo = 0.0f;   // (NaN elements fall out of both)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        hi = fmaxf(fmaxf(fmaxf(fmaxf(hi, f[i].x), f[i].y), f[i].z), f[i].w);
+        lo = fminf(fminf(fminf(fminf(lo, f[i].x), f[i].y), f[i].z), f[i].w);
+    }
+    hi = fmaxf(hi, dpp_f<kQuadSwap1>(hi));
+    lo = fminf(lo, dpp_f<kQuadSwap1>(lo));
+    hi = fmaxf(hi, dpp_f<kQuadSwap2>(hi));
+    lo = fminf(lo, dpp_f<kQuadSwap2>(lo));
+    hi = fmaxf(hi, dpp_f<kHalfMirror>(hi));
+    lo = fminf(lo, dpp_f<kHalfMirror>(lo));
+    hi = fmaxf(hi, dpp_f<kRowMirror>(hi));
+    lo = fminf(lo, dpp_f<kRowMirror>(lo));
+    const float amax = fmaxf(hi, -lo);
+    float max = hi > -lo ? hi : lo;
+    if (__any(hi == -lo && amax != 0.0f)) {   // both signs: the sign of the first of them
+        int idx = 0x7fffffff;
+#pragma unroll
+        for (int i = 3; i >= 0; i--) {
+            const float v[4] = {f[i].x, f[i].y, f[i].z, f[i].w};
+#pragma unroll
+            for (int c = 3; c >= 0; c--)
+                if (fabsf(v[c]) == amax) idx = 2 * (64 * i + 4 * (int)l + c) + (v[c] < 0.0f ? 1 : 0);
+        }
+        idx = min(idx, dpp_i<kQuadSwap1>(idx));
+        idx = min(idx, dpp_i<kQuadSwap2>(idx));
+        idx = min(idx, dpp_i<kHalfMirror>(idx));
+        idx = min(idx, dpp_i<kRowMirror>(idx));
+        if (hi == -lo) max = idx & 1 ? lo : hi;
+    }
+    const bool any = amax != 0.0f;
+    const float iscale = -128.0f / max;
+    const float d = any ? 1.0f / iscale : 0.0f;
+    uint32_t packed[4];
+    int sum[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float v[4] = {f[i].x, f[i].y, f[i].z, f[i].w};
+        uint32_t q[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++)   // min(127, round(t)) as i8: clamped first, NaN to 127; |t| is at most 128 and rounding then
+            q[c] = (uint32_t)cq_round_away_i32(fmaxf(fminf(iscale * v[c], 127.0f), -128.0f));
+        const uint32_t p01 = __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u), p23 = __builtin_amdgcn_perm(q[3], q[2], 0x04000c0cu);
+        packed[i] = any ? p01 | p23 : 0u;
+        sum[i] = __builtin_amdgcn_sdot4((int)packed[i], 0x01010101, 0, false);
+        sum[i] += dpp_i<kQuadSwap1>(sum[i]);
+        sum[i] += dpp_i<kQuadSwap2>(sum[i]);   // bsums[4i + l / 4]
+    }
+    if (!active) return;
+    // lane l stores bsums[4 * (l % 4) + l / 4]
+    const uint32_t j = l & 3, sj = 4 * j + (l >> 2);
+    const int mine = j == 0 ? sum[0] : j == 1 ? sum[1] : j == 2 ? sum[2] : sum[3];
+    if (AOS) {
+        uint8_t *b = out.aos + (int64_t)blk * 292;   // 292 = 4 * 73: 4-byte aligned
+        if (l == 0) *(float *)b = d;
+#pragma unroll
+        for (int i = 0; i < 4; i++) *(uint32_t *)(b + 4 + 64 * i + 4 * l) = packed[i];
+        *(int16_t *)(b + 260 + 2 * sj) = (int16_t)mine;
+    } else {
+        int8_t *q = out.v.qs + (int64_t)blk * 256 + 4 * l;
+#pragma unroll
+        for (int i = 0; i < 4; i++) *(uint32_t *)(q + 64 * i) = packed[i];
+        const int64_t tb = (int64_t)b_in_row * out.v.m_stride + row;
+        if (l == 0) {
+            out.v.d[blk] = d;
+            out.v.dT[tb] = d;
+        }
+        out.v.bsums[(int64_t)blk * 16 + sj] = (int16_t)mine;
+        ((_Float16 *)out.v.bsh)[tb * 16 + sj] = (_Float16)(float)mine;
+    }
+}
+
 template <bool AOS, bool SILU>
 __global__ void __launch_bounds__(256) quantize_q8k_kernel(const float *__restrict__ x,
                                                            const int32_t *__restrict__ row_ids, int64_t m, int64_t k,
@@ -189,7 +294,7 @@ __global__ void __launch_bounds__(256) quantize_q8k_kernel(const float *__restri
     const int64_t blk = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     clear_floats(out.clear);
     if (blk >= m * kb) return;
-    const int64_t row = blk / kb;
+    const int64_t row = divide(blk, kb);
     const int64_t b_in_row = blk - row * kb;
     const int64_t src_row = row_ids ? (int64_t)row_ids[row] : row;
     float4 f = *(const float4 *)(x + src_row * k + b_in_row * 256 + 4 * lane);
@@ -324,6 +429,9 @@ void launch_rms(const float *x, const int32_t *row_ids, int64_t m, int64_t k, cq
     else quantize_rms_rows_kernel<AOS, ACT, 16, false><<<(unsigned)m, 1024, lds, s>>>(x, row_ids, k, pre.aux, pre.eps, out);
 }
 
+// Blocks from which four share a wave: below, the chip is not full and the longer chain of a lane decides (256 rows of 1024: 2.8
+// against 3.2 us; with silu, which is most of a lane's work, 64 rows of 1024 3.8 against 3.3).
+constexpr int64_t kQuadBlocks = 1024;
 template <bool AOS>
 hipError_t launch(int act_dtype, const float *x, const int32_t *row_ids, int64_t m, int64_t k, cq_pre pre, Sink out,
                   hipStream_t s) {
@@ -340,7 +448,11 @@ hipError_t launch(int act_dtype, const float *x, const int32_t *row_ids, int64_t
     const bool silu = pre.kind == CQ_PRE_SILU_MUL;
     const int64_t nw = act_dtype == CQ_DTYPE_Q8K ? m * (k / 256) : m * ((k + 255) / 256);
     const unsigned grid = (unsigned)((nw + waves - 1) / waves);
-    if (act_dtype == CQ_DTYPE_Q8K) {
+    if (act_dtype == CQ_DTYPE_Q8K && nw >= kQuadBlocks && nw < (1ll << 31)) {
+        const unsigned quads = (unsigned)((nw + 15) / 16);
+        if (silu) quantize_q8k_quad_kernel<AOS, true><<<quads, threads, 0, s>>>(x, row_ids, (uint32_t)nw, (uint32_t)(k / 256), pre.aux, out);
+        else quantize_q8k_quad_kernel<AOS, false><<<quads, threads, 0, s>>>(x, row_ids, (uint32_t)nw, (uint32_t)(k / 256), nullptr, out);
+    } else if (act_dtype == CQ_DTYPE_Q8K) {
         if (silu) quantize_q8k_kernel<AOS, true><<<grid, threads, 0, s>>>(x, row_ids, m, k, pre.aux, out);
         else quantize_q8k_kernel<AOS, false><<<grid, threads, 0, s>>>(x, row_ids, m, k, nullptr, out);
     } else if (act_dtype == CQ_DTYPE_Q8_0) {
