@@ -603,7 +603,7 @@ __device__ __forceinline__ int64_t last_tile(int64_t n_own, int64_t n) { return 
 // One workgroup: activation rows [m0, m0 + 32*MT) (stored up to row m - 1) x the 256 weight rows of
 // blockIdx.x, K blocks of part blockIdx.z.
 template <int DT, int MT, bool DUMP = false, int WBUF = 1, bool ONCE = false>
-__device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view &a, int64_t m0, int64_t m,
+__device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view &a, int64_t bx, int64_t m0, int64_t m,
                                           float *__restrict__ y, int ksplit, cq_mfma_dump dump = cq_mfma_dump{nullptr, nullptr, 0}) {
     static_assert(WBUF == 1 || DT == CQ_DTYPE_Q4K || DT == CQ_DTYPE_Q5K, "block headers of 20 bytes");
     typedef Tile<DT, MT> T;
@@ -612,7 +612,7 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, col = lane & 31;
     const int64_t kb = w.k >> 8;
-    const int64_t n_own = ((int64_t)blockIdx.x * kWaves + wave) * 32;
+    const int64_t n_own = (bx * kWaves + wave) * 32;
     const bool n_ok = n_own < w.n;   // wave-uniform; a wave past the last row only helps with the copies
     const int64_t n_tile = last_tile(n_own, w.n);
     const int64_t n = n_tile + col;
@@ -692,7 +692,7 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
         // (the lane's column anew: kept from above it would take registers that the 128-row tiles do not have)
         int wv = wave, ln = lane;
         asm volatile("" : "+s"(wv), "+v"(ln));
-        const int64_t own = ((int64_t)blockIdx.x * kWaves + wv) * 32, c = last_tile(own, w.n) + (ln & 31);
+        const int64_t own = (bx * kWaves + wv) * 32, c = last_tile(own, w.n) + (ln & 31);
         if (c < own) return;
         float *__restrict__ yc = y + (m0 + (ln >> 5) * 4) * w.n + c;
         const int64_t left = m - m0 - (ln >> 5) * 4;
@@ -713,7 +713,23 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
 template <int DT, int MT>
 __global__ void __launch_bounds__(kThreads) gemm_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
                                                         int ksplit) {
-    gemm_body<DT, MT>(w, a, (int64_t)blockIdx.y * (MT * 32), m, y, ksplit);
+    gemm_body<DT, MT>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, y, ksplit);
+}
+
+// 128-row tiles in whole rounds of workgroups, and what is left of them in tiles of 32 * TAIL rows: the last round of a launch
+// that does not fill it then lasts as long as a shorter tile.  `whole` of the `gx` x row tiles (column tiles first) are taken
+// whole, the others by 4 / TAIL workgroups each.  Measured at pick_plan.
+template <int DT, int TAIL>
+__global__ void __launch_bounds__(kThreads) gemm_tail_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t gx,
+                                                             uint32_t whole) {
+    const uint32_t id = blockIdx.x;
+    if (id < whole) {
+        gemm_body<DT, 4>(w, a, id % gx, (int64_t)(id / gx) * 128, m, y, 1);
+    } else {
+        const uint32_t t = whole + (id - whole) / (4 / TAIL), part = (id - whole) % (4 / TAIL);
+        const int64_t m0 = (int64_t)(t / gx) * 128 + part * (32 * TAIL);
+        if (m0 < m) gemm_body<DT, TAIL>(w, a, t % gx, m0, m, y, 1);
+    }
 }
 
 // Up to 32 activation rows (one row tile): every weight byte is read once by the launch, cold - the form of the grouped
@@ -722,14 +738,14 @@ template <int DT> constexpr int once_wbuf() { return DT == CQ_DTYPE_Q4K || DT ==
 template <int DT>
 __global__ void __launch_bounds__(kThreads) gemm_once_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
                                                              int ksplit) {
-    gemm_body<DT, 1, false, once_wbuf<DT>(), true>(w, a, 0, m, y, ksplit);
+    gemm_body<DT, 1, false, once_wbuf<DT>(), true>(w, a, blockIdx.x, 0, m, y, ksplit);
 }
 
 // The same launch with the block integers stored instead of the result (verification).
 template <int DT, int MT>
 __global__ void __launch_bounds__(kThreads) gemm_dump_kernel(cq_weight w, cq_act_view a, int64_t m, int ksplit,
                                                              cq_mfma_dump dump) {
-    gemm_body<DT, MT, true>(w, a, (int64_t)blockIdx.y * (MT * 32), m, nullptr, ksplit, dump);
+    gemm_body<DT, MT, true>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, nullptr, ksplit, dump);
 }
 
 // ------------------------------------------------------ few weight rows, long K: K halved inside the workgroup ----
@@ -869,8 +885,8 @@ __global__ void __launch_bounds__(kThreads) gemm_grouped_kernel(GroupArgs ga, cq
                                                                 int ksplit) {
     const int tile = blockIdx.y;
     const cq_weight w = ga.w[ga.expert[tile]];
-    if constexpr (MT == 1) gemm_body<DT, 1, false, grouped_wbuf<DT>(), true>(w, a, ga.row0[tile], ga.row_end[tile], y, ksplit);
-    else gemm_body<DT, MT>(w, a, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit);
+    if constexpr (MT == 1) gemm_body<DT, 1, false, grouped_wbuf<DT>(), true>(w, a, blockIdx.x, ga.row0[tile], ga.row_end[tile], y, ksplit);
+    else gemm_body<DT, MT>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit);
 }
 
 // ------------------------------------------------ K-quant weights x Q8_1 activations (tile kernel) ----
@@ -1098,6 +1114,7 @@ int64_t n_tiles(const cq_weight *w) { return (w->n + kWaves * 32 - 1) / (kWaves 
 struct Plan {
     int mt, ksplit;
     int kh = 1;   // 2: gemm_kh_kernel (K halved inside the workgroup, 128 weight rows per workgroup)
+    int tail = 0; // 1, 2: gemm_tail_kernel, the last round's tiles in heights of 32 * tail rows
 };
 Plan pick_plan(const cq_weight *w, int64_t m) {
     const int64_t gx = n_tiles(w), kb = w->k >> 8, cus = cq_num_cus();
@@ -1114,10 +1131,23 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
             if (ks > 1 && kb / ks < 4) break;
             if (ks > 1 && cq_no_split_k()) break;   // CQ_FLAG_DETERMINISTIC
             const int64_t rounds = (tiles * ks + cus - 1) / cus;
-            const double cost = (double)rounds * ((double)((kb + ks - 1) / ks) * (unpack + 13.5 * mt) + 24.0) +
+            double cost = (double)rounds * ((double)((kb + ks - 1) / ks) * (unpack + 13.5 * mt) + 24.0) +
                                 (ks > 1 ? ks * atomic_pass : 0.0);
+            // A last round that is at most half full (or a quarter), in shorter tiles: nothing else runs beside it, so it lasts
+            // as long as one of its tiles.  Whole calls, us, one height -> two: Q4K 11008 x 4096 at 4096 / 1024 rows 454 -> 424 /
+            // 137 -> 120, 14336 x 4096 at 2048 282 -> 267, 5120 x 5120 at 2000 158 -> 134, 8448 x 2048 at 1024 78 -> 60; Q6K
+            // 11008 x 4096 at 1024 154 -> 139, 4096 x 14336 at 2300 418 -> 399; Q5K 8192 x 4096 at 1100 167 -> 130.
+            int tail = 0;
+            const int64_t left = tiles % cus;
+            for (int t = 2; t >= 1 && mt == 4 && ks == 1 && rounds > 1 && left * (4 / t) > 0 && left * (4 / t) <= cus; t--) {
+                const double c = (double)(rounds - 1) * ((double)kb * (unpack + 13.5 * 4) + 24.0) + ((double)kb * (unpack + 13.5 * t) + 24.0);
+                if (c < cost) {
+                    cost = c;
+                    tail = t;
+                }
+            }
             if (first || cost < best_cost) {
-                best = Plan{mt, ks};
+                best = Plan{mt, ks, 1, tail};
                 best_cost = cost;
                 first = false;
             }
@@ -1173,16 +1203,29 @@ hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, hip
     return hipGetLastError();
 }
 
+template <int DT, int TAIL>
+hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+    const size_t lds = Tile<DT, 4>::kTotal;
+    if (hipError_t e = cq_ensure_lds<gemm_tail_kernel<DT, TAIL>>(w->dev, lds); e != hipSuccess) return e;
+    const int64_t gx = n_tiles(w), tiles = gx * ((m + 127) / 128), whole = tiles / cq_num_cus() * cq_num_cus();
+    CQ_LAUNCH((gemm_tail_kernel<DT, TAIL>), (unsigned)(whole + (tiles - whole) * (4 / TAIL)), kThreads, lds, s, *w, a, m, y, (uint32_t)gx,
+              (uint32_t)whole);
+    return hipGetLastError();
+}
+
 template <int DT>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool y_cleared, hipStream_t s) {
     const Plan p = pick_plan(w, m);
+    if (p.tail == 2) return launch_tail<DT, 2>(w, a, m, y, s);
+    if (p.tail == 1) return launch_tail<DT, 1>(w, a, m, y, s);
     if (p.kh == 2) return p.mt == 1 ? launch_kh<DT, 1>(w, a, m, y, s) : launch_kh<DT, 2>(w, a, m, y, s);
     if (p.mt == 1) return launch_mt<DT, 1>(w, a, m, y, p.ksplit, y_cleared, s);
     if (p.mt == 2) return launch_mt<DT, 2>(w, a, m, y, p.ksplit, y_cleared, s);
     return launch_mt<DT, 4>(w, a, m, y, p.ksplit, y_cleared, s);
 }
 
-// The launch cq_launch_gemm would make (same tile height, same K split), storing the block integers.
+// The launch cq_launch_gemm would make (same tile height, same K split), storing the block integers.  (A launch of two tile
+// heights is dumped in the taller one; the shorter ones' code is that of the launches of one height.)
 template <int DT, int MT>
 hipError_t launch_dump_mt(const cq_weight *w, cq_act_view a, int64_t m, int ksplit, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = Tile<DT, MT>::kTotal;
