@@ -124,7 +124,7 @@ __device__ __forceinline__ void stage_weights(uint8_t *wl, const cq_weight &w, c
 // ONCE: a launch with a single row tile (up to 32 rows), which reads every weight byte once.
 // SHORT: K is no multiple of 256, the last step has fewer than eight blocks.
 template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
-__device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_view &a, int64_t m0, int64_t m, float *__restrict__ y,
+__device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_view &a, int64_t bx, int64_t m0, int64_t m, float *__restrict__ y,
                                             int ksplit, cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -132,7 +132,7 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane >> 5, col = lane & 31;
     const int64_t k = w.k, ks = (k + 255) >> 8;         // K steps of 256 elements; the last one may be shorter
-    const int64_t n_own = ((int64_t)blockIdx.x * kWaves + wave) * 32;
+    const int64_t n_own = (bx * kWaves + wave) * 32;
     const bool n_ok = n_own < w.n;                      // wave-uniform; a wave past the last row only helps with the copies
     // fewer than 32 rows left: the tile begins earlier, at row n - 32, and only the wave's own share is stored
     const int64_t n_tile = n_own + 32 <= w.n ? n_own : w.n - 32;
@@ -278,7 +278,23 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
 template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, int ksplit,
                                                           cq_mfma_dump dump) {
-    gemm32_body<DT, MT, DUMP, ONCE, SHORT>(w, a, (int64_t)blockIdx.y * (MT * 32), m, y, ksplit, dump);
+    gemm32_body<DT, MT, DUMP, ONCE, SHORT>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, y, ksplit, dump);
+}
+
+// 128-row tiles in whole rounds of workgroups, what is left of them in tiles of 32 * TAIL rows (as gemm_tail_kernel of
+// gemm.hip): `whole` of the gx x row tiles, column tiles first, are taken whole, the others by 4 / TAIL workgroups each.
+template <int DT, int TAIL, bool SHORT>
+__global__ void __launch_bounds__(kThreads) gemm32_tail_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t gx,
+                                                               uint32_t whole) {
+    const uint32_t id = blockIdx.x;
+    const cq_mfma_dump none{nullptr, nullptr, 0};
+    if (id < whole) {
+        gemm32_body<DT, 4, false, false, SHORT>(w, a, id % gx, (int64_t)(id / gx) * 128, m, y, 1, none);
+    } else {
+        const uint32_t t = whole + (id - whole) / (4 / TAIL), part = (id - whole) % (4 / TAIL);
+        const int64_t m0 = (int64_t)(t / gx) * 128 + part * (32 * TAIL);
+        if (m0 < m) gemm32_body<DT, TAIL, false, false, SHORT>(w, a, t % gx, m0, m, y, 1, none);
+    }
 }
 
 // Mixture-of-experts form: blockIdx.y walks a table of tiles of 32*MT rows of the expert-sorted activation rows; each tile names
@@ -294,7 +310,7 @@ template <int DT, int MT, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_grouped_kernel(GroupArgs ga, cq_act_view a, float *__restrict__ y, int ksplit) {
     const int tile = blockIdx.y;
     const cq_weight w = ga.w[ga.expert[tile]];
-    gemm32_body<DT, MT, false, MT == 1, SHORT>(w, a, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit,
+    gemm32_body<DT, MT, false, MT == 1, SHORT>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit,
                                                cq_mfma_dump{nullptr, nullptr, 0});
 }
 
@@ -304,6 +320,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_grouped_kernel(GroupArgs ga, 
 // a split launch adds every part to the output atomically, which moves about 1.1 TB/s.
 struct Plan {
     int mt, ksplit;
+    int tail = 0;   // 1, 2: gemm32_tail_kernel, the last round's tiles in heights of 32 * tail rows
 };
 Plan pick_plan(const cq_weight *w, int64_t m) {
     const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks_total = (w->k + 255) >> 8, cus = cq_num_cus();
@@ -318,10 +335,19 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
             if (ks > 1 && ks_total / ks < 2) break;
             if (ks > 1 && cq_no_split_k()) break;   // CQ_FLAG_DETERMINISTIC
             const int64_t rounds = (tiles * ks + cus - 1) / cus;
-            const double cost = (double)rounds * ((double)((ks_total + ks - 1) / ks) * (10.0 + 23.0 * mt) + 24.0) +
+            double cost = (double)rounds * ((double)((ks_total + ks - 1) / ks) * (10.0 + 23.0 * mt) + 24.0) +
                                 (ks > 1 ? ks * atomic_pass : 0.0);
+            // A last round that is at most half full (or a quarter), in shorter tiles.  Whole calls, us, one height -> two: Q8_0
+            // 11008 x 4096 at 4096 / 1024 rows 610 -> 580 / 181 -> 163, 5120 x 5120 at 2000 229 -> 178, 8448 x 2048 at 1024
+            // 99 -> 77; Q4_0 4096 x 14336 at 2300 512 -> 456.
+            int tail = 0;
+            const int64_t left = tiles % cus;
+            for (int t = 2; t >= 1 && mt == 4 && ks == 1 && rounds > 1 && left > 0 && left * (4 / t) <= cus; t--) {
+                cost = (double)(rounds - 1) * ((double)ks_total * (10.0 + 23.0 * 4) + 24.0) + ((double)ks_total * (10.0 + 23.0 * t) + 24.0);
+                tail = t;
+            }
             if (first || cost < best_cost) {
-                best = Plan{mt, ks};
+                best = Plan{mt, ks, tail};
                 best_cost = cost;
                 first = false;
             }
@@ -337,6 +363,15 @@ hipError_t launch_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, i
     if (hipError_t e = cq_ensure_lds<gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>>(w->dev, lds); e != hipSuccess) return e;
     const dim3 grid((unsigned)((w->n + kWaves * 32 - 1) / (kWaves * 32)), (unsigned)((m + MT * 32 - 1) / (MT * 32)), (unsigned)ksplit);
     CQ_LAUNCH((gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, d);
+    return hipGetLastError();
+}
+template <int DT, int TAIL, bool SHORT>
+hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+    const size_t lds = Tile<DT, 4>::kTotal;
+    if (hipError_t e = cq_ensure_lds<gemm32_tail_kernel<DT, TAIL, SHORT>>(w->dev, lds); e != hipSuccess) return e;
+    const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), tiles = gx * ((m + 127) / 128), whole = tiles / cq_num_cus() * cq_num_cus();
+    CQ_LAUNCH((gemm32_tail_kernel<DT, TAIL, SHORT>), (unsigned)(whole + (tiles - whole) * (4 / TAIL)), kThreads, lds, s, *w, a, m, y,
+              (uint32_t)gx, (uint32_t)whole);
     return hipGetLastError();
 }
 template <int DT, int MT, bool DUMP>
@@ -366,6 +401,11 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
 template <int DT, bool DUMP>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool y_cleared, cq_mfma_dump d, hipStream_t s) {
     const Plan p = pick_plan(w, m);
+    if constexpr (!DUMP) {   // (dumped in the taller height: the shorter ones' code is that of the launches of one height)
+        const bool whole = w->k % 256 == 0;
+        if (p.tail == 2) return whole ? launch_tail<DT, 2, false>(w, a, m, y, s) : launch_tail<DT, 2, true>(w, a, m, y, s);
+        if (p.tail == 1) return whole ? launch_tail<DT, 1, false>(w, a, m, y, s) : launch_tail<DT, 1, true>(w, a, m, y, s);
+    }
     if (p.mt == 1) return launch_mt<DT, 1, DUMP>(w, a, m, y, p.ksplit, y_cleared, d, s);
     if (p.mt == 2) return launch_mt<DT, 2, DUMP>(w, a, m, y, p.ksplit, y_cleared, d, s);
     return launch_mt<DT, 4, DUMP>(w, a, m, y, p.ksplit, y_cleared, d, s);

@@ -1,6 +1,6 @@
 """Prompts whose 128-row tiles leave a last round of workgroups at most half full: that round's tiles are 64 or 32 rows high.
 Against the dot-product kernel, which the oracle tests pin: the same block integers, f32 sums over the blocks of a row and the
-f16 min term apart, k / 256 additions of either: 2^-24 each, and as many again for the two products of a block."""
+f16 min term apart, an addition of either per block: 2^-24 each, and as many again for the two products of a block."""
 import pytest
 import torch
 
@@ -10,7 +10,7 @@ from tests.test_gpu_fused_neighbours import qh  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K"])
+@pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K", "Q8_0", "Q4_0"])
 @pytest.mark.parametrize("m,n,k", [(1100, 8192, 512),          # 288 tiles: 32 left, as 32-row tiles, some past the last row
                                    (1025, 8192 - 17, 256),     # ragged weight rows, one live row in the last strip
                                    (1000, 11264, 512),         # 352 tiles: 96 left, as 64-row tiles
@@ -18,6 +18,17 @@ pytestmark = pytest.mark.gpu
                                    (1024, 8448, 256),          # 264: 8 left
                                    (1024, 12544, 256)])        # 392: too many left
 def test_last_round_in_shorter_tiles(qh, dt, m, n, k):  # noqa: F811
+    check(qh, dt, m, n, k)
+
+
+@pytest.mark.parametrize("dt", ["Q8_0", "Q4_0"])
+@pytest.mark.parametrize("m,n,k", [(1100, 8192, 320), (1000, 11264 - 3, 576)])
+def test_rows_of_no_whole_step(qh, dt, m, n, k):  # noqa: F811
+    check(qh, dt, m, n, k)
+
+
+def check(qh, dt, m, n, k):  # noqa: F811
+    block = 32 if dt in ("Q8_0", "Q4_0") else 256
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     w = QTensor.quantize(torch.randn(n, k, generator=g, device="cuda") * 0.02, GgmlDType[dt]).weight
     x = torch.randn(m, k, generator=g, device="cuda")
@@ -25,4 +36,4 @@ def test_last_round_in_shorter_tiles(qh, dt, m, n, k):  # noqa: F811
     want = qh.qmatmul(w, x, qh.FLAG_FORCE_MATVEC)
     # rows apart, so that one wrong tile cannot hide in the rest
     err = (got - want).double().norm(dim=1) / want.double().norm(dim=1)
-    assert err.max().item() <= 4 * (k // 256) * 2.0 ** -24 + 2e-7, err.max().item()
+    assert err.max().item() <= 4 * (k // block) * 2.0 ** -24 + 2e-7, err.max().item()
