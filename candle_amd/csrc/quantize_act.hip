@@ -195,6 +195,10 @@ __device__ __forceinline__ void q8k_chunk(const float4 f, int64_t row, int64_t b
 template <bool AOS, bool SILU>
 __global__ void __launch_bounds__(256) quantize_q8k_quad_kernel(const float *__restrict__ x, const int32_t *__restrict__ row_ids,
                                                                 uint32_t blocks, uint32_t kb, const float *__restrict__ x2, Sink out) {
+    if (blockIdx.x * 16 >= blocks) {   // (a workgroup that only clears)
+        clear_floats(out.clear);
+        return;
+    }
     const uint32_t l = threadIdx.x & 15;
     const uint32_t blk = blockIdx.x * 16 + (threadIdx.x >> 4);
     const bool active = blk < blocks;
@@ -457,7 +461,7 @@ hipError_t launch(int act_dtype, const float *x, const int32_t *row_ids, int64_t
     const int64_t least = clearers < 2 * cq_num_cus() ? clearers : 2 * cq_num_cus(), need = (nw + waves - 1) / waves;
     const unsigned grid = (unsigned)(need > least ? need : least);
     if (act_dtype == CQ_DTYPE_Q8K && nw >= kQuadBlocks && nw < (1ll << 31)) {
-        const unsigned quads = (unsigned)((nw + 15) / 16);
+        const unsigned quads = (unsigned)((nw + 15) / 16 > least ? (nw + 15) / 16 : least);
         if (silu) quantize_q8k_quad_kernel<AOS, true><<<quads, threads, 0, s>>>(x, row_ids, (uint32_t)nw, (uint32_t)(k / 256), pre.aux, out);
         else quantize_q8k_quad_kernel<AOS, false><<<quads, threads, 0, s>>>(x, row_ids, (uint32_t)nw, (uint32_t)(k / 256), nullptr, out);
     } else if (act_dtype == CQ_DTYPE_Q8K) {
