@@ -6,9 +6,13 @@
 // Every function returns None where it does not take its arguments (wrong type, shape, device, layout): qhip.py then words
 // the error.  The C functions are handed over by address (`bind`), so that whichever libcandle_qhip.so qhip.py loaded is the
 // one that is called.
+//
+// torch's C++ side throws (a tensor without memory under vmap, grad or a tracer; no memory left; no device): `entry` turns what
+// reaches it into the Python exception that torch's own calls raise, so references are held by objects that let go of them.
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/candle_qhip.h"
@@ -31,6 +35,21 @@ struct Abi {
 } g_abi;
 PyObject *g_error = nullptr;                                             // qhip.QHipError
 PyObject *g_s_addr = nullptr, *g_s_buf = nullptr, *g_s_get = nullptr;   // "_addr", "buf", "get"
+
+// An owned reference.
+struct Ref {
+    PyObject *p = nullptr;
+    Ref() = default;
+    explicit Ref(PyObject *o) : p(o) {}
+    Ref(const Ref &) = delete;
+    Ref &operator=(const Ref &) = delete;
+    ~Ref() { Py_XDECREF(p); }
+    PyObject *release() {
+        PyObject *o = p;
+        p = nullptr;
+        return o;
+    }
+};
 
 constexpr int kMaxWeights = 256;   // of one multi or grouped call; more of them take the general path's error
 
@@ -73,20 +92,17 @@ const float *floats_of(PyObject *t) { return t == Py_None ? nullptr : (const flo
 
 // At least `need` bytes on x's device out of a qhip.Workspace (which grows in Python).  A new reference to the tensor
 // in *held; the workspace object keeps it too.
-bool workspace(PyObject *ws, size_t need, const at::Tensor &x, PyObject *px, PyObject **held, void **ptr, size_t *bytes) {
-    PyObject *buf = PyObject_GetAttr(ws, g_s_buf);
-    if (!buf) return false;
-    if (buf == Py_None || (size_t)THPVariable_Unpack(buf).numel() < need || THPVariable_Unpack(buf).device() != x.device()) {
-        Py_DECREF(buf);
-        PyObject *dev = PyObject_GetAttrString(px, "device");
-        PyObject *n = PyLong_FromSize_t(need);
-        buf = dev && n ? PyObject_CallMethodObjArgs(ws, g_s_get, n, dev, nullptr) : nullptr;
-        Py_XDECREF(dev);
-        Py_XDECREF(n);
-        if (!buf) return false;
+bool workspace(PyObject *ws, size_t need, const at::Tensor &x, PyObject *px, Ref *held, void **ptr, size_t *bytes) {
+    held->p = PyObject_GetAttr(ws, g_s_buf);
+    if (!held->p) return false;
+    const auto fits = [&](const at::Tensor &b) { return (size_t)b.numel() >= need && b.device() == x.device(); };
+    if (held->p == Py_None || !fits(THPVariable_Unpack(held->p))) {
+        Py_CLEAR(held->p);
+        const Ref dev(PyObject_GetAttrString(px, "device")), n(PyLong_FromSize_t(need));
+        held->p = dev.p && n.p ? PyObject_CallMethodObjArgs(ws, g_s_get, n.p, dev.p, nullptr) : nullptr;
+        if (!held->p) return false;
     }
-    const at::Tensor &b = THPVariable_Unpack(buf);
-    *held = buf;
+    const at::Tensor &b = THPVariable_Unpack(held->p);
     *ptr = b.data_ptr();
     *bytes = (size_t)b.numel();
     return true;
@@ -109,37 +125,30 @@ bool as_int(PyObject *o, int *v) {
 }
 
 // qmatmul(w, x, flags, out, workspace, pre, aux, eps)
-PyObject *py_qmatmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
+PyObject *py_qmatmul(PyObject *const *a, Py_ssize_t na) {
     if (na != 8) return PyErr_Format(PyExc_TypeError, "qmatmul takes 8 arguments");
     int flags, pre;
     if (!as_int(a[2], &flags) || !as_int(a[5], &pre)) return nullptr;
     const double eps = PyFloat_AsDouble(a[7]);
     if (eps == -1.0 && PyErr_Occurred()) return nullptr;
     const cq_weight *w = weight_of(a[0]);
-    PyObject *px = a[1], *out = a[3], *aux = a[6];
-    if (!w || !f32_on_device(px) || (out != Py_None && !THPVariable_Check(out))) Py_RETURN_NONE;
+    PyObject *px = a[1], *aux = a[6];
+    if (!w || !f32_on_device(px) || (a[3] != Py_None && !THPVariable_Check(a[3]))) Py_RETURN_NONE;
     const at::Tensor &x = THPVariable_Unpack(px);
     int64_t n, k;
     if (g_abi.weight_shape(w, &n, &k) != CQ_OK || x.dim() < 2 || x.size(-1) != k || !aux_ok(pre, x, aux)) Py_RETURN_NONE;
     const int64_t m = k ? x.numel() / k : 0;
-    PyObject *held = nullptr;
+    Ref held, out;
     void *ws;
     size_t ws_bytes;
     if (!workspace(a[4], g_abi.workspace_bytes(w, m, flags), x, px, &held, &ws, &ws_bytes)) return nullptr;
-    const bool mine = out == Py_None;
-    float *y = nullptr;
-    try {
-        if (mine) out = THPVariable_Wrap(result_like(x, n));
-        else Py_INCREF(out);
-        if (out) y = (float *)THPVariable_Unpack(out).data_ptr();
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        out = nullptr;
+    if (a[3] == Py_None) {
+        out.p = THPVariable_Wrap(result_like(x, n));
+        if (!out.p) return nullptr;
+    } else {
+        Py_INCREF(out.p = a[3]);
     }
-    if (!out) {
-        Py_DECREF(held);
-        return nullptr;
-    }
+    float *y = (float *)THPVariable_Unpack(out.p).data_ptr();
     const float *xp = (const float *)x.data_ptr(), *ap = pre == CQ_PRE_NONE ? nullptr : floats_of(aux);
     void *s = stream_now();
     int rc;
@@ -147,12 +156,7 @@ PyObject *py_qmatmul(PyObject *, PyObject *const *a, Py_ssize_t na) {
     rc = pre == CQ_PRE_NONE ? g_abi.qmatmul(w, xp, m, y, flags, ws, ws_bytes, s)
                             : g_abi.qmatmul_fused(w, pre, xp, ap, (float)eps, m, y, flags, ws, ws_bytes, s);
     Py_END_ALLOW_THREADS
-    Py_DECREF(held);
-    if (rc != CQ_OK) {
-        Py_DECREF(out);
-        return fail(rc);
-    }
-    return out;
+    return rc == CQ_OK ? out.release() : fail(rc);
 }
 
 // The weights of a list; their number, or -1 where an element has none or there are too many.
@@ -166,7 +170,7 @@ Py_ssize_t weights_of(PyObject *list, const cq_weight **ws) {
 }
 
 // qmatmul_multi(weights, x, flags, workspace, pre, aux, eps)
-PyObject *py_qmatmul_multi(PyObject *, PyObject *const *a, Py_ssize_t na) {
+PyObject *py_qmatmul_multi(PyObject *const *a, Py_ssize_t na) {
     if (na != 7) return PyErr_Format(PyExc_TypeError, "qmatmul_multi takes 7 arguments");
     int flags, pre;
     if (!as_int(a[2], &flags) || !as_int(a[4], &pre)) return nullptr;
@@ -183,44 +187,36 @@ PyObject *py_qmatmul_multi(PyObject *, PyObject *const *a, Py_ssize_t na) {
     const int64_t m = k ? x.numel() / k : 0;
     size_t need = 0;
     for (Py_ssize_t i = 0; i < count; i++) need = std::max(need, g_abi.workspace_bytes(ws[i], m, flags));
-    PyObject *held = nullptr;
+    Ref held;
     void *wp;
     size_t ws_bytes;
     if (!workspace(a[3], need, x, px, &held, &wp, &ws_bytes)) return nullptr;
-    PyObject *outs = PyList_New(count);
-    bool ok = outs != nullptr;
-    try {
-        for (Py_ssize_t i = 0; ok && i < count; i++) {
-            int64_t ni, ki;
-            g_abi.weight_shape(ws[i], &ni, &ki);
-            PyObject *o = THPVariable_Wrap(result_like(x, ni));
-            ok = o != nullptr;
-            if (!ok) break;
-            ys[i] = (float *)THPVariable_Unpack(o).data_ptr();
-            PyList_SET_ITEM(outs, i, o);
-        }
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        ok = false;
+    Ref outs(PyList_New(count));
+    if (!outs.p) return nullptr;
+    for (Py_ssize_t i = 0; i < count; i++) {
+        int64_t ni, ki;
+        g_abi.weight_shape(ws[i], &ni, &ki);
+        PyObject *o = THPVariable_Wrap(result_like(x, ni));
+        if (!o) return nullptr;
+        PyList_SET_ITEM(outs.p, i, o);
+        ys[i] = (float *)THPVariable_Unpack(o).data_ptr();
     }
-    int rc = CQ_OK;
-    if (ok) {
-        const float *xp = (const float *)x.data_ptr(), *ap = aux == Py_None ? nullptr : floats_of(aux);
-        void *s = stream_now();
-        Py_BEGIN_ALLOW_THREADS
-        rc = g_abi.qmatmul_multi(ws, (int)count, pre, xp, ap, (float)eps, m, ys, flags, wp, ws_bytes, s);
-        Py_END_ALLOW_THREADS
-    }
-    Py_DECREF(held);
-    if (!ok || rc != CQ_OK) {
-        Py_XDECREF(outs);
-        return ok ? fail(rc) : nullptr;
-    }
-    return outs;
+    const float *xp = (const float *)x.data_ptr(), *ap = aux == Py_None ? nullptr : floats_of(aux);
+    void *s = stream_now();
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = g_abi.qmatmul_multi(ws, (int)count, pre, xp, ap, (float)eps, m, ys, flags, wp, ws_bytes, s);
+    Py_END_ALLOW_THREADS
+    return rc == CQ_OK ? outs.release() : fail(rc);
 }
 
+struct Buffer {
+    Py_buffer b{};
+    ~Buffer() { PyBuffer_Release(&b); }   // (nothing where no buffer was taken)
+};
+
 // qmatmul_grouped(experts, x, row_ids, offsets (int32 buffer), flags, workspace, pre, aux, eps)
-PyObject *py_qmatmul_grouped(PyObject *, PyObject *const *a, Py_ssize_t na) {
+PyObject *py_qmatmul_grouped(PyObject *const *a, Py_ssize_t na) {
     if (na != 9) return PyErr_Format(PyExc_TypeError, "qmatmul_grouped takes 9 arguments");
     int flags, pre;
     if (!as_int(a[4], &flags) || !as_int(a[6], &pre)) return nullptr;
@@ -233,75 +229,47 @@ PyObject *py_qmatmul_grouped(PyObject *, PyObject *const *a, Py_ssize_t na) {
     const at::Tensor &x = THPVariable_Unpack(px);
     int64_t n, k;
     if (g_abi.weight_shape(ws[0], &n, &k) != CQ_OK || !aux_ok(pre, x, aux)) Py_RETURN_NONE;
-    Py_buffer offs;
-    if (PyObject_GetBuffer(a[3], &offs, PyBUF_C_CONTIGUOUS) != 0) return nullptr;
-    const int32_t *offsets = (const int32_t *)offs.buf;
-    const Py_ssize_t have = offs.len / (Py_ssize_t)sizeof(int32_t);
-    if (offs.itemsize != sizeof(int32_t) || have < count + 1) {
-        PyBuffer_Release(&offs);
-        Py_RETURN_NONE;
-    }
+    Buffer offs;
+    if (PyObject_GetBuffer(a[3], &offs.b, PyBUF_C_CONTIGUOUS) != 0) return nullptr;
+    const int32_t *offsets = (const int32_t *)offs.b.buf;
+    const Py_ssize_t have = offs.b.len / (Py_ssize_t)sizeof(int32_t);
+    if (offs.b.itemsize != sizeof(int32_t) || have < count + 1) Py_RETURN_NONE;
     const int64_t total = offsets[have - 1];
-    PyObject *held = nullptr, *out = nullptr;
+    if (total < 0) return PyErr_Format(g_error, "offsets must be non-negative");
+    Ref held;
     void *wp;
     size_t ws_bytes;
-    int rc = CQ_OK;
-    if (total >= 0 && workspace(a[5], g_abi.grouped_workspace_bytes(ws, (int)count, total, flags), x, px, &held, &wp, &ws_bytes)) {
-        try {
-            out = THPVariable_Wrap(empty_f32({total, n}, x.device()));
-        } catch (const std::exception &e) {
-            PyErr_SetString(PyExc_RuntimeError, e.what());
-        }
-        if (out) {
-            float *y = (float *)THPVariable_Unpack(out).data_ptr();
-            const float *xp = (const float *)x.data_ptr(), *ap = pre == CQ_PRE_NONE ? nullptr : floats_of(aux);
-            const int32_t *rid = ids == Py_None ? nullptr : (const int32_t *)THPVariable_Unpack(ids).data_ptr();
-            void *s = stream_now();
-            Py_BEGIN_ALLOW_THREADS
-            rc = pre == CQ_PRE_NONE ? g_abi.qmatmul_grouped(ws, (int)count, xp, rid, offsets, y, flags, wp, ws_bytes, s)
-                                    : g_abi.qmatmul_grouped_fused(ws, (int)count, pre, xp, ap, (float)eps, rid, offsets, y, flags, wp, ws_bytes, s);
-            Py_END_ALLOW_THREADS
-        }
-        Py_DECREF(held);
-    } else if (total < 0) {
-        PyErr_SetString(g_error, "offsets must be non-negative");
-    }
-    PyBuffer_Release(&offs);
-    if (out && rc != CQ_OK) {
-        Py_DECREF(out);
-        return fail(rc);
-    }
-    return out;
+    if (!workspace(a[5], g_abi.grouped_workspace_bytes(ws, (int)count, total, flags), x, px, &held, &wp, &ws_bytes)) return nullptr;
+    Ref out(THPVariable_Wrap(empty_f32({total, n}, x.device())));
+    if (!out.p) return nullptr;
+    float *y = (float *)THPVariable_Unpack(out.p).data_ptr();
+    const float *xp = (const float *)x.data_ptr(), *ap = pre == CQ_PRE_NONE ? nullptr : floats_of(aux);
+    const int32_t *rid = ids == Py_None ? nullptr : (const int32_t *)THPVariable_Unpack(ids).data_ptr();
+    void *s = stream_now();
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = pre == CQ_PRE_NONE ? g_abi.qmatmul_grouped(ws, (int)count, xp, rid, offsets, y, flags, wp, ws_bytes, s)
+                            : g_abi.qmatmul_grouped_fused(ws, (int)count, pre, xp, ap, (float)eps, rid, offsets, y, flags, wp, ws_bytes, s);
+    Py_END_ALLOW_THREADS
+    return rc == CQ_OK ? out.release() : fail(rc);
 }
 
 // dequantize(w, f16)
-PyObject *py_dequantize(PyObject *, PyObject *const *a, Py_ssize_t na) {
+PyObject *py_dequantize(PyObject *const *a, Py_ssize_t na) {
     if (na != 2) return PyErr_Format(PyExc_TypeError, "dequantize takes 2 arguments");
     const bool f16 = PyObject_IsTrue(a[1]) == 1;
     const cq_weight *w = weight_of(a[0]);
     int64_t n, k;
     if (!w || g_abi.weight_shape(w, &n, &k) != CQ_OK) Py_RETURN_NONE;
-    PyObject *out;
-    void *p;
-    try {
-        const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)g_abi.weight_device(w));
-        out = THPVariable_Wrap(at::Tensor(at::detail::empty_cuda({n, k}, f16 ? at::kHalf : at::kFloat, dev, std::nullopt)));
-        if (!out) return nullptr;
-        p = THPVariable_Unpack(out).data_ptr();
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
-    }
-    void *s = stream_now();
+    const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)g_abi.weight_device(w));
+    Ref out(THPVariable_Wrap(at::Tensor(at::detail::empty_cuda({n, k}, f16 ? at::kHalf : at::kFloat, dev, std::nullopt))));
+    if (!out.p) return nullptr;
+    void *p = THPVariable_Unpack(out.p).data_ptr(), *s = stream_now();
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = f16 ? g_abi.weight_dequantize_f16(w, (uint16_t *)p, s) : g_abi.weight_dequantize(w, (float *)p, s);
     Py_END_ALLOW_THREADS
-    if (rc != CQ_OK) {
-        Py_DECREF(out);
-        return fail(rc);
-    }
-    return out;
+    return rc == CQ_OK ? out.release() : fail(rc);
 }
 
 template <typename F> bool take(PyObject *table, const char *name, F *f) {
@@ -315,7 +283,7 @@ template <typename F> bool take(PyObject *table, const char *name, F *f) {
 }
 
 // bind({name: address}, error class)
-PyObject *py_bind(PyObject *, PyObject *const *a, Py_ssize_t na) {
+PyObject *py_bind(PyObject *const *a, Py_ssize_t na) {
     if (na != 2 || !PyDict_Check(a[0])) return PyErr_Format(PyExc_TypeError, "bind takes a dict and an exception class");
 #define TAKE(f) take(a[0], "cq_" #f, &g_abi.f)
     if (!(TAKE(last_error) && TAKE(weight_shape) && TAKE(weight_device) && TAKE(workspace_bytes) && TAKE(qmatmul) && TAKE(qmatmul_fused) &&
@@ -328,7 +296,16 @@ PyObject *py_bind(PyObject *, PyObject *const *a, Py_ssize_t na) {
     Py_RETURN_NONE;
 }
 
-#define FAST(f) (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr
+template <PyObject *(*F)(PyObject *const *, Py_ssize_t)> PyObject *entry(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    try {
+        return F(a, na);
+    } catch (const std::exception &) {
+        torch::translate_exception_to_python(std::current_exception());
+        return nullptr;
+    }
+}
+
+#define FAST(f) (PyCFunction)(void (*)(void))entry<f>, METH_FASTCALL, nullptr
 PyMethodDef g_methods[] = {{"bind", FAST(py_bind)},
                            {"qmatmul", FAST(py_qmatmul)},
                            {"qmatmul_multi", FAST(py_qmatmul_multi)},

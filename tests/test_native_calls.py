@@ -1,0 +1,91 @@
+"""The native side of qhip's calls (csrc/calls.cpp) on arguments that never reach a kernel, without a GPU: device tensors are
+torch's fake ones, which have no memory, and the C library behind the calls is a handful of Python callbacks.
+
+Each check runs in a process of its own, since what it guards against ends the process."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+N, K = 64, 256
+
+
+def bind():
+    """qhip with its native calls on a stand-in for the C library: every weight is [N, K], every call succeeds."""
+    import ctypes as C
+
+    from candle_amd import qhip
+    native = qhip._calls()
+    vp, i64, ci, sz = C.c_void_p, C.c_int64, C.c_int, C.c_size_t
+
+    def shape(_w, n, k):
+        n[0], k[0] = N, K
+        return 0
+    table = {name: C.CFUNCTYPE(ci)(lambda: 0) for name in qhip.EXPORTS}
+    table["cq_weight_shape"] = C.CFUNCTYPE(ci, vp, C.POINTER(i64), C.POINTER(i64))(shape)
+    table["cq_workspace_bytes"] = C.CFUNCTYPE(sz, vp, i64, ci)(lambda w, m, f: 256)
+    table["cq_grouped_workspace_bytes"] = C.CFUNCTYPE(sz, vp, ci, i64, ci)(lambda w, e, t, f: 256)
+    qhip._kept = table
+    native.bind({name: C.cast(f, vp).value for name, f in table.items()}, qhip.QHipError)
+
+    class Weight:
+        _addr, shape = 1, (N, K)
+    return qhip, Weight()
+
+
+def fake(*shape):
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        return torch.empty(*shape, device="cuda")
+
+
+def raises(kind, call):
+    """The call raises exactly what `kind` names."""
+    try:
+        call()
+    except kind as e:
+        print("ok", type(e).__name__, str(e)[:60], flush=True)
+    else:
+        raise AssertionError("no error")
+
+
+def child_no_memory():
+    """Tensors without memory in each place whose address a call takes (x, the workspace, a given result), plain and behind
+    the wrappers of vmap and grad: a Python exception each."""
+    import numpy as np
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    qhip, w = bind()
+    out, offsets = torch.empty(2, N), np.array([0, 2], np.int32)
+
+    def over(v):   # a workspace whose buffer is the wrapped tensor itself
+        ws = qhip.Workspace()
+        ws.buf = v
+        return ws
+    calls = (lambda v: qhip.qmatmul(w, v, out=out), lambda v: qhip.qmatmul(w, v, out=out, pre=qhip.PRE_SILU_MUL, aux=v),
+             lambda v: qhip.qmatmul(w, v, out=out, workspace=over(v)), lambda v: qhip.qmatmul_multi([w, w], v, workspace=over(v)),
+             lambda v: qhip.qmatmul_grouped([w], v, None, offsets, workspace=over(v)))
+    for call in calls:
+        with FakeTensorMode():
+            x = torch.empty(3, 2, K, device="cuda")
+            raises(RuntimeError, lambda: call(x[0]))
+            raises(RuntimeError, lambda: torch.func.vmap(call)(x))
+            raises(RuntimeError, lambda: torch.func.grad(lambda v: call(v).sum())(x[0]))
+
+
+CHILDREN = {f[len("child_"):]: g for f, g in list(globals().items()) if f.startswith("child_")}
+
+
+@pytest.mark.parametrize("name", CHILDREN)
+def test_native_calls(name):
+    pytest.importorskip("torch")
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), name], cwd=ROOT, capture_output=True, text=True, timeout=300,
+                       env={**os.environ, "PYTHONPATH": ROOT})
+    assert r.returncode == 0, (r.returncode, r.stdout[-1500:], r.stderr[-3000:])
+
+
+if __name__ == "__main__":
+    CHILDREN[sys.argv[1]]()
