@@ -79,7 +79,7 @@ bool f32_on_device(PyObject *x) {
     return t.is_cuda() && t.scalar_type() == at::kFloat && t.is_contiguous();
 }
 
-// The operand of the fused step `pre`, with the shape rules of qhip._check_pre.
+// The operand of the fused step `pre`, with the shape rules of qhip._check_pre.  (Without a step nothing reads it.)
 bool aux_ok(int pre, const at::Tensor &x, PyObject *aux) {
     if (pre == CQ_PRE_NONE) return true;
     if (!f32_on_device(aux)) return false;
@@ -88,7 +88,8 @@ bool aux_ok(int pre, const at::Tensor &x, PyObject *aux) {
     return pre == CQ_PRE_SILU_MUL && a.sizes() == x.sizes();
 }
 
-const float *floats_of(PyObject *t) { return t == Py_None ? nullptr : (const float *)THPVariable_Unpack(t).data_ptr(); }
+// Its address, after aux_ok.
+const float *aux_floats(int pre, PyObject *aux) { return pre == CQ_PRE_NONE ? nullptr : (const float *)THPVariable_Unpack(aux).data_ptr(); }
 
 // At least `need` bytes on x's device out of a qhip.Workspace (which grows in Python).  A new reference to the tensor
 // in *held; the workspace object keeps it too.
@@ -149,7 +150,7 @@ PyObject *py_qmatmul(PyObject *const *a, Py_ssize_t na) {
         Py_INCREF(out.p = a[3]);
     }
     float *y = (float *)THPVariable_Unpack(out.p).data_ptr();
-    const float *xp = (const float *)x.data_ptr(), *ap = pre == CQ_PRE_NONE ? nullptr : floats_of(aux);
+    const float *xp = (const float *)x.data_ptr(), *ap = aux_floats(pre, aux);
     void *s = stream_now();
     int rc;
     Py_BEGIN_ALLOW_THREADS
@@ -180,7 +181,7 @@ PyObject *py_qmatmul_multi(PyObject *const *a, Py_ssize_t na) {
     float *ys[kMaxWeights];
     PyObject *px = a[1], *aux = a[5];
     const Py_ssize_t count = weights_of(a[0], ws);
-    if (count < 1 || !f32_on_device(px)) Py_RETURN_NONE;
+    if (count < 1 || !f32_on_device(px) || (aux != Py_None && !THPVariable_Check(aux))) Py_RETURN_NONE;
     const at::Tensor &x = THPVariable_Unpack(px);
     int64_t n, k;
     if (g_abi.weight_shape(ws[0], &n, &k) != CQ_OK || x.dim() < 2 || x.size(-1) != k || !aux_ok(pre, x, aux)) Py_RETURN_NONE;
@@ -201,7 +202,7 @@ PyObject *py_qmatmul_multi(PyObject *const *a, Py_ssize_t na) {
         PyList_SET_ITEM(outs.p, i, o);
         ys[i] = (float *)THPVariable_Unpack(o).data_ptr();
     }
-    const float *xp = (const float *)x.data_ptr(), *ap = aux == Py_None ? nullptr : floats_of(aux);
+    const float *xp = (const float *)x.data_ptr(), *ap = aux_floats(pre, aux);
     void *s = stream_now();
     int rc;
     Py_BEGIN_ALLOW_THREADS
@@ -243,7 +244,7 @@ PyObject *py_qmatmul_grouped(PyObject *const *a, Py_ssize_t na) {
     Ref out(THPVariable_Wrap(empty_f32({total, n}, x.device())));
     if (!out.p) return nullptr;
     float *y = (float *)THPVariable_Unpack(out.p).data_ptr();
-    const float *xp = (const float *)x.data_ptr(), *ap = pre == CQ_PRE_NONE ? nullptr : floats_of(aux);
+    const float *xp = (const float *)x.data_ptr(), *ap = aux_floats(pre, aux);
     const int32_t *rid = ids == Py_None ? nullptr : (const int32_t *)THPVariable_Unpack(ids).data_ptr();
     void *s = stream_now();
     int rc;

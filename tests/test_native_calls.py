@@ -76,6 +76,21 @@ def child_no_memory():
             raises(RuntimeError, lambda: torch.func.grad(lambda v: call(v).sum())(x[0]))
 
 
+def child_second_operand():
+    """A second operand that is no tensor is refused with every fused step; without one qmatmul_multi looks at it all the same
+    (the other two calls do not read it)."""
+    import numpy as np
+    qhip, w = bind()
+    x, offsets = fake(2, K), np.array([0, 2], np.int32)
+    for aux in (1.5, [1.0], "aux", object(), np.ones((2, K), np.float32)):
+        for pre in (qhip.PRE_NONE, qhip.PRE_RMS_NORM, qhip.PRE_SILU_MUL, 3):
+            bad = (qhip.QHipError, AttributeError)   # (the wording of the refusal asks `aux` whether it is on the device)
+            raises(bad, lambda: qhip.qmatmul_multi([w, w], x, pre=pre, aux=aux))
+            if pre != qhip.PRE_NONE:
+                raises(bad, lambda: qhip.qmatmul(w, x, pre=pre, aux=aux))
+                raises(bad, lambda: qhip.qmatmul_grouped([w], x, None, offsets, pre=pre, aux=aux))
+
+
 CHILDREN = {f[len("child_"):]: g for f, g in list(globals().items()) if f.startswith("child_")}
 
 
