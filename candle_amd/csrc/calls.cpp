@@ -15,6 +15,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <climits>
+
 #include "../../include/candle_qhip.h"
 
 namespace {
@@ -51,7 +53,9 @@ struct Ref {
     }
 };
 
-constexpr int kMaxWeights = 256;   // of one multi or grouped call; more of them take the general path's error
+// The weights of one call, any number of them, and their results.
+using Weights = c10::SmallVector<const cq_weight *, 16>;
+using Results = c10::SmallVector<float *, 16>;
 
 void *stream_now() { return (void *)c10::hip::getCurrentHIPStream().stream(); }
 
@@ -160,14 +164,14 @@ PyObject *py_qmatmul(PyObject *const *a, Py_ssize_t na) {
     return rc == CQ_OK ? out.release() : fail(rc);
 }
 
-// The weights of a list; their number, or -1 where an element has none or there are too many.
-Py_ssize_t weights_of(PyObject *list, const cq_weight **ws) {
-    if (!PyList_Check(list)) return -1;
-    const Py_ssize_t count = PyList_GET_SIZE(list);
-    if (count < 1 || count > kMaxWeights) return -1;
-    for (Py_ssize_t i = 0; i < count; i++)
-        if (!(ws[i] = weight_of(PyList_GET_ITEM(list, i)))) return -1;
-    return count;
+// The weights of a list; false where it is empty or an element has none.
+bool weights_of(PyObject *list, Weights *ws) {
+    if (!PyList_Check(list)) return false;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); i++) {
+        ws->push_back(weight_of(PyList_GET_ITEM(list, i)));
+        if (!ws->back()) return false;
+    }
+    return !ws->empty() && ws->size() <= (size_t)INT_MAX;
 }
 
 // qmatmul_multi(weights, x, flags, workspace, pre, aux, eps)
@@ -177,36 +181,35 @@ PyObject *py_qmatmul_multi(PyObject *const *a, Py_ssize_t na) {
     if (!as_int(a[2], &flags) || !as_int(a[4], &pre)) return nullptr;
     const double eps = PyFloat_AsDouble(a[6]);
     if (eps == -1.0 && PyErr_Occurred()) return nullptr;
-    const cq_weight *ws[kMaxWeights];
-    float *ys[kMaxWeights];
+    Weights ws;
+    Results ys;
     PyObject *px = a[1], *aux = a[5];
-    const Py_ssize_t count = weights_of(a[0], ws);
-    if (count < 1 || !f32_on_device(px) || (aux != Py_None && !THPVariable_Check(aux))) Py_RETURN_NONE;
+    if (!weights_of(a[0], &ws) || !f32_on_device(px) || (aux != Py_None && !THPVariable_Check(aux))) Py_RETURN_NONE;
     const at::Tensor &x = THPVariable_Unpack(px);
     int64_t n, k;
     if (g_abi.weight_shape(ws[0], &n, &k) != CQ_OK || x.dim() < 2 || x.size(-1) != k || !aux_ok(pre, x, aux)) Py_RETURN_NONE;
     const int64_t m = k ? x.numel() / k : 0;
     size_t need = 0;
-    for (Py_ssize_t i = 0; i < count; i++) need = std::max(need, g_abi.workspace_bytes(ws[i], m, flags));
+    for (const cq_weight *w : ws) need = std::max(need, g_abi.workspace_bytes(w, m, flags));
     Ref held;
     void *wp;
     size_t ws_bytes;
     if (!workspace(a[3], need, x, px, &held, &wp, &ws_bytes)) return nullptr;
-    Ref outs(PyList_New(count));
+    Ref outs(PyList_New((Py_ssize_t)ws.size()));
     if (!outs.p) return nullptr;
-    for (Py_ssize_t i = 0; i < count; i++) {
+    for (size_t i = 0; i < ws.size(); i++) {
         int64_t ni, ki;
         g_abi.weight_shape(ws[i], &ni, &ki);
         PyObject *o = THPVariable_Wrap(result_like(x, ni));
         if (!o) return nullptr;
-        PyList_SET_ITEM(outs.p, i, o);
-        ys[i] = (float *)THPVariable_Unpack(o).data_ptr();
+        PyList_SET_ITEM(outs.p, (Py_ssize_t)i, o);
+        ys.push_back((float *)THPVariable_Unpack(o).data_ptr());
     }
     const float *xp = (const float *)x.data_ptr(), *ap = aux_floats(pre, aux);
     void *s = stream_now();
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = g_abi.qmatmul_multi(ws, (int)count, pre, xp, ap, (float)eps, m, ys, flags, wp, ws_bytes, s);
+    rc = g_abi.qmatmul_multi(ws.data(), (int)ws.size(), pre, xp, ap, (float)eps, m, ys.data(), flags, wp, ws_bytes, s);
     Py_END_ALLOW_THREADS
     return rc == CQ_OK ? outs.release() : fail(rc);
 }
@@ -223,10 +226,9 @@ PyObject *py_qmatmul_grouped(PyObject *const *a, Py_ssize_t na) {
     if (!as_int(a[4], &flags) || !as_int(a[6], &pre)) return nullptr;
     const double eps = PyFloat_AsDouble(a[8]);
     if (eps == -1.0 && PyErr_Occurred()) return nullptr;
-    const cq_weight *ws[kMaxWeights];
+    Weights ws;
     PyObject *px = a[1], *ids = a[2], *aux = a[7];
-    const Py_ssize_t count = weights_of(a[0], ws);
-    if (count < 1 || !f32_on_device(px) || (ids != Py_None && !THPVariable_Check(ids))) Py_RETURN_NONE;
+    if (!weights_of(a[0], &ws) || !f32_on_device(px) || (ids != Py_None && !THPVariable_Check(ids))) Py_RETURN_NONE;
     const at::Tensor &x = THPVariable_Unpack(px);
     int64_t n, k;
     if (g_abi.weight_shape(ws[0], &n, &k) != CQ_OK || !aux_ok(pre, x, aux)) Py_RETURN_NONE;
@@ -234,13 +236,13 @@ PyObject *py_qmatmul_grouped(PyObject *const *a, Py_ssize_t na) {
     if (PyObject_GetBuffer(a[3], &offs.b, PyBUF_C_CONTIGUOUS) != 0) return nullptr;
     const int32_t *offsets = (const int32_t *)offs.b.buf;
     const Py_ssize_t have = offs.b.len / (Py_ssize_t)sizeof(int32_t);
-    if (offs.b.itemsize != sizeof(int32_t) || have < count + 1) Py_RETURN_NONE;
+    if (offs.b.itemsize != sizeof(int32_t) || have < (Py_ssize_t)ws.size() + 1) Py_RETURN_NONE;
     const int64_t total = offsets[have - 1];
     if (total < 0) return PyErr_Format(g_error, "offsets must be non-negative");
     Ref held;
     void *wp;
     size_t ws_bytes;
-    if (!workspace(a[5], g_abi.grouped_workspace_bytes(ws, (int)count, total, flags), x, px, &held, &wp, &ws_bytes)) return nullptr;
+    if (!workspace(a[5], g_abi.grouped_workspace_bytes(ws.data(), (int)ws.size(), total, flags), x, px, &held, &wp, &ws_bytes)) return nullptr;
     Ref out(THPVariable_Wrap(empty_f32({total, n}, x.device())));
     if (!out.p) return nullptr;
     float *y = (float *)THPVariable_Unpack(out.p).data_ptr();
@@ -249,8 +251,8 @@ PyObject *py_qmatmul_grouped(PyObject *const *a, Py_ssize_t na) {
     void *s = stream_now();
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = pre == CQ_PRE_NONE ? g_abi.qmatmul_grouped(ws, (int)count, xp, rid, offsets, y, flags, wp, ws_bytes, s)
-                            : g_abi.qmatmul_grouped_fused(ws, (int)count, pre, xp, ap, (float)eps, rid, offsets, y, flags, wp, ws_bytes, s);
+    rc = pre == CQ_PRE_NONE ? g_abi.qmatmul_grouped(ws.data(), (int)ws.size(), xp, rid, offsets, y, flags, wp, ws_bytes, s)
+                            : g_abi.qmatmul_grouped_fused(ws.data(), (int)ws.size(), pre, xp, ap, (float)eps, rid, offsets, y, flags, wp, ws_bytes, s);
     Py_END_ALLOW_THREADS
     return rc == CQ_OK ? out.release() : fail(rc);
 }
