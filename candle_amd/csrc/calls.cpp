@@ -3,7 +3,7 @@
 // same steps written in Python over ctypes took 10 us of host time per call and bounded it (4096x4096 Q4K, one row, calls
 // back to back: 10.5 us), here they take about 3.
 //
-// Every function returns None where it does not take its arguments (wrong type, shape, device, layout): qhip.py then words
+// The matmuls return None where they do not take their arguments (wrong type, shape, device, layout): qhip.py then words
 // the error.  The C functions are handed over by address (`bind`), so that whichever libcandle_qhip.so qhip.py loaded is the
 // one that is called.
 //
@@ -263,7 +263,7 @@ PyObject *py_dequantize(PyObject *const *a, Py_ssize_t na) {
     const bool f16 = PyObject_IsTrue(a[1]) == 1;
     const cq_weight *w = weight_of(a[0]);
     int64_t n, k;
-    if (!w || g_abi.weight_shape(w, &n, &k) != CQ_OK) Py_RETURN_NONE;
+    if (const int rc = g_abi.weight_shape(w, &n, &k); rc != CQ_OK) return fail(rc);   // (no weight is an error there)
     const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)g_abi.weight_device(w));
     Ref out(THPVariable_Wrap(at::Tensor(at::detail::empty_cuda({n, k}, f16 ? at::kHalf : at::kFloat, dev, std::nullopt))));
     if (!out.p) return nullptr;

@@ -108,6 +108,16 @@ def child_many_weights():
                 assert not isinstance(e, qhip.QHipError), (count, e)
 
 
+def child_gone_weight():
+    """A weight that has been given back is refused by every call."""
+    import numpy as np
+    from candle_amd import qhip   # (on the C library itself)
+    w, x = qhip.QWeight(None, 0), fake(2, K)
+    for call in (lambda: w.dequantize(), lambda: w.dequantize_f16(), lambda: qhip.qmatmul(w, x), lambda: qhip.qmatmul_multi([w], x),
+                 lambda: qhip.qmatmul_grouped([w], x, None, np.array([0, 2], np.int32))):
+        raises(qhip.QHipError, call)
+
+
 CHILDREN = {f[len("child_"):]: g for f, g in list(globals().items()) if f.startswith("child_")}
 
 
