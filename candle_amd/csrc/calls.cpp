@@ -35,7 +35,7 @@ struct Abi {
     decltype(&cq_weight_dequantize) weight_dequantize;
     decltype(&cq_weight_dequantize_f16) weight_dequantize_f16;
 } g_abi;
-PyObject *g_error = nullptr;                                             // qhip.QHipError
+PyObject *g_error = nullptr, *g_workspace = nullptr;                     // qhip.QHipError, qhip.Workspace
 PyObject *g_s_addr = nullptr, *g_s_buf = nullptr, *g_s_get = nullptr;   // "_addr", "buf", "get"
 
 // An owned reference.
@@ -95,17 +95,23 @@ bool aux_ok(int pre, const at::Tensor &x, PyObject *aux) {
 // Its address, after aux_ok.
 const float *aux_floats(int pre, PyObject *aux) { return pre == CQ_PRE_NONE ? nullptr : (const float *)THPVariable_Unpack(aux).data_ptr(); }
 
-// At least `need` bytes on x's device out of a qhip.Workspace (which grows in Python).  A new reference to the tensor
-// in *held; the workspace object keeps it too.
+// At least `need` bytes on x's device out of the caller's workspace: anything with a `get(bytes, device)`, which is spared
+// where a qhip.Workspace (and no class derived from it) holds enough already.  *held keeps the buffer alive during the call.
 bool workspace(PyObject *ws, size_t need, const at::Tensor &x, PyObject *px, Ref *held, void **ptr, size_t *bytes) {
-    held->p = PyObject_GetAttr(ws, g_s_buf);
-    if (!held->p) return false;
-    const auto fits = [&](const at::Tensor &b) { return (size_t)b.numel() >= need && b.device() == x.device(); };
-    if (held->p == Py_None || !fits(THPVariable_Unpack(held->p))) {
-        Py_CLEAR(held->p);
+    if ((PyObject *)Py_TYPE(ws) == g_workspace) {
+        held->p = PyObject_GetAttr(ws, g_s_buf);
+        if (!held->p) return false;
+        const auto fits = [&](const at::Tensor &b) { return (size_t)b.numel() >= need && b.device() == x.device(); };
+        if (!THPVariable_Check(held->p) || !fits(THPVariable_Unpack(held->p))) Py_CLEAR(held->p);
+    }
+    if (!held->p) {
         const Ref dev(PyObject_GetAttrString(px, "device")), n(PyLong_FromSize_t(need));
         held->p = dev.p && n.p ? PyObject_CallMethodObjArgs(ws, g_s_get, n.p, dev.p, nullptr) : nullptr;
         if (!held->p) return false;
+        if (!THPVariable_Check(held->p)) {
+            PyErr_Format(PyExc_TypeError, "the workspace gave no tensor");
+            return false;
+        }
     }
     const at::Tensor &b = THPVariable_Unpack(held->p);
     *ptr = b.data_ptr();
@@ -285,9 +291,9 @@ template <typename F> bool take(PyObject *table, const char *name, F *f) {
     return !PyErr_Occurred();
 }
 
-// bind({name: address}, error class)
+// bind({name: address}, error class, workspace class)
 PyObject *py_bind(PyObject *const *a, Py_ssize_t na) {
-    if (na != 2 || !PyDict_Check(a[0])) return PyErr_Format(PyExc_TypeError, "bind takes a dict and an exception class");
+    if (na != 3 || !PyDict_Check(a[0])) return PyErr_Format(PyExc_TypeError, "bind takes a dict and two classes");
 #define TAKE(f) take(a[0], "cq_" #f, &g_abi.f)
     if (!(TAKE(last_error) && TAKE(weight_shape) && TAKE(weight_device) && TAKE(workspace_bytes) && TAKE(qmatmul) && TAKE(qmatmul_fused) &&
           TAKE(qmatmul_multi) && TAKE(grouped_workspace_bytes) && TAKE(qmatmul_grouped) && TAKE(qmatmul_grouped_fused) &&
@@ -296,6 +302,8 @@ PyObject *py_bind(PyObject *const *a, Py_ssize_t na) {
 #undef TAKE
     Py_INCREF(a[1]);
     Py_XSETREF(g_error, a[1]);
+    Py_INCREF(a[2]);
+    Py_XSETREF(g_workspace, a[2]);
     Py_RETURN_NONE;
 }
 

@@ -112,7 +112,7 @@ def _calls():
         spec = importlib.util.spec_from_file_location("_calls", CALLS_PATH)
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
-        mod.bind({name: C.cast(getattr(L, name), C.c_void_p).value for name in EXPORTS}, QHipError)
+        mod.bind({name: C.cast(getattr(L, name), C.c_void_p).value for name in EXPORTS}, QHipError, Workspace)
         _native = mod
     return _native
 

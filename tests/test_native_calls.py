@@ -28,7 +28,7 @@ def bind():
     table["cq_workspace_bytes"] = C.CFUNCTYPE(sz, vp, i64, ci)(lambda w, m, f: 256)
     table["cq_grouped_workspace_bytes"] = C.CFUNCTYPE(sz, vp, ci, i64, ci)(lambda w, e, t, f: 256)
     qhip._kept = table
-    native.bind({name: C.cast(f, vp).value for name, f in table.items()}, qhip.QHipError)
+    native.bind({name: C.cast(f, vp).value for name, f in table.items()}, qhip.QHipError, qhip.Workspace)
 
     class Weight:
         _addr, shape = 1, (N, K)
@@ -116,6 +116,33 @@ def child_gone_weight():
     for call in (lambda: w.dequantize(), lambda: w.dequantize_f16(), lambda: qhip.qmatmul(w, x), lambda: qhip.qmatmul_multi([w], x),
                  lambda: qhip.qmatmul_grouped([w], x, None, np.array([0, 2], np.int32))):
         raises(qhip.QHipError, call)
+
+
+def child_other_workspaces():
+    """A caller's own workspace is anything with a `get`, and a Workspace's own `get` is asked where a class brings one."""
+    import numpy as np
+    qhip, w = bind()
+    x, buf, offsets = fake(2, K), fake(1024), np.array([0, 2], np.int32)
+
+    class Own:
+        asked = 0
+
+        def get(self, nbytes, device):
+            self.asked += 1
+            return buf
+
+    class Pooled(qhip.Workspace):
+        asked = 0
+        get = Own.get
+    pooled = Pooled()
+    pooled.buf = buf
+    for ws in (Own(), pooled):
+        for call in (lambda: qhip.qmatmul(w, x, workspace=ws), lambda: qhip.qmatmul_multi([w, w], x, workspace=ws),
+                     lambda: qhip.qmatmul_grouped([w], x, None, offsets, workspace=ws)):
+            raises(RuntimeError, call)   # (the allocation of the result)
+        assert ws.asked == 3, ws.asked
+    Own.get = lambda self, nbytes, device: 7
+    raises(TypeError, lambda: qhip.qmatmul(w, x, workspace=Own()))
 
 
 CHILDREN = {f[len("child_"):]: g for f, g in list(globals().items()) if f.startswith("child_")}
