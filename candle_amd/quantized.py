@@ -187,7 +187,6 @@ class QMatMul:
         self.arm = arm          # "QTensor" | "Tensor" | "TensorF16"
         self.dense = dense      # the dequantized weight of the two dense arms
         self._ws = qhip.Workspace()
-        self._w = qtensor.weight
 
     @classmethod
     def from_qtensor(cls, qtensor: QTensor) -> "QMatMul":
@@ -208,7 +207,7 @@ class QMatMul:
             return xs.matmul(self.dense.t())
         if self.arm == "TensorF16":     # mod.rs:539-547
             return xs.to(self.dense.dtype).matmul(self.dense.t()).to(xs.dtype)
-        return qhip.qmatmul(self._w, xs, 0, None, self._ws)
+        return qhip.qmatmul(self.qtensor.weight, xs, 0, None, self._ws)
 
     def forward_via_f16(self, xs):
         """mod.rs:452-461."""
@@ -219,12 +218,12 @@ class QMatMul:
         """`self.forward(rms_norm(xs, alpha, eps))` (RmsNorm::forward, candle-transformers/src/
         quantized_nn.rs:121-125, in front of a projection as in quantized_llama.rs:453-466) without
         the normalised tensor going to memory."""
-        return qhip.qmatmul(self._w, xs, workspace=self._ws, pre=qhip.PRE_RMS_NORM, aux=alpha, eps=eps)
+        return qhip.qmatmul(self.qtensor.weight, xs, workspace=self._ws, pre=qhip.PRE_RMS_NORM, aux=alpha, eps=eps)
 
     def forward_silu_mul(self, gate, up):
         """`self.forward(silu(gate) * up)`: the feed-forward's w2 applied to silu(w1 x) * (w3 x)
         (Mlp::forward, quantized_llama.rs:56-63)."""
-        return qhip.qmatmul(self._w, gate, workspace=self._ws, pre=qhip.PRE_SILU_MUL, aux=up)
+        return qhip.qmatmul(self.qtensor.weight, gate, workspace=self._ws, pre=qhip.PRE_SILU_MUL, aux=up)
 
     @staticmethod
     def forward_multi(mats, xs, alpha=None, eps: float = 0.0):
@@ -233,7 +232,7 @@ class QMatMul:
         (:60-61): one launch for one activation row, the rows quantized once otherwise."""
         mats = list(mats)
         pre = qhip.PRE_NONE if alpha is None else qhip.PRE_RMS_NORM
-        return qhip.qmatmul_multi([m._w for m in mats], xs, workspace=mats[0]._ws, pre=pre, aux=alpha, eps=eps)
+        return qhip.qmatmul_multi([m.qtensor.weight for m in mats], xs, workspace=mats[0]._ws, pre=pre, aux=alpha, eps=eps)
 
     def dequantize_f16(self):
         """mod.rs:444-450."""

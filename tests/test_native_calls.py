@@ -156,5 +156,26 @@ def test_native_calls(name):
     assert r.returncode == 0, (r.returncode, r.stdout[-1500:], r.stderr[-3000:])
 
 
+def test_the_weight_is_the_tensor_of_the_call(monkeypatch):
+    """QMatMul reads its tensor when it is called: a tensor put in its place is the one that is used, by every form."""
+    pytest.importorskip("torch")
+    from candle_amd import qhip
+    from candle_amd.quantized import QMatMul
+
+    class Tensor:
+        def __init__(self, weight):
+            self.weight = weight
+
+        def rank(self):
+            return 2
+    monkeypatch.setattr(qhip, "qmatmul", lambda w, *a, **kw: w)
+    monkeypatch.setattr(qhip, "qmatmul_multi", lambda ws, *a, **kw: ws)
+    mat = QMatMul(Tensor("first"))
+    assert mat.forward(None) == "first"
+    mat.qtensor = Tensor("second")
+    assert [mat.forward(None), mat.forward_rms_norm(None, None, 0.0), mat.forward_silu_mul(None, None)] == ["second"] * 3
+    assert QMatMul.forward_multi([mat, mat], None) == ["second"] * 2
+
+
 if __name__ == "__main__":
     CHILDREN[sys.argv[1]]()
