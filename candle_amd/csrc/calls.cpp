@@ -140,7 +140,7 @@ PyObject *py_qmatmul(PyObject *const *a, Py_ssize_t na) {
     if (na != 8) return PyErr_Format(PyExc_TypeError, "qmatmul takes 8 arguments");
     int flags, pre;
     if (!as_int(a[2], &flags) || !as_int(a[5], &pre)) return nullptr;
-    const double eps = PyFloat_AsDouble(a[7]);
+    const double eps = pre == CQ_PRE_NONE ? 0.0 : PyFloat_AsDouble(a[7]);
     if (eps == -1.0 && PyErr_Occurred()) return nullptr;
     const cq_weight *w = weight_of(a[0]);
     PyObject *px = a[1], *aux = a[6];
@@ -230,7 +230,7 @@ PyObject *py_qmatmul_grouped(PyObject *const *a, Py_ssize_t na) {
     if (na != 9) return PyErr_Format(PyExc_TypeError, "qmatmul_grouped takes 9 arguments");
     int flags, pre;
     if (!as_int(a[4], &flags) || !as_int(a[6], &pre)) return nullptr;
-    const double eps = PyFloat_AsDouble(a[8]);
+    const double eps = pre == CQ_PRE_NONE ? 0.0 : PyFloat_AsDouble(a[8]);
     if (eps == -1.0 && PyErr_Occurred()) return nullptr;
     Weights ws;
     PyObject *px = a[1], *ids = a[2], *aux = a[7];

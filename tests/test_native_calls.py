@@ -145,6 +145,18 @@ def child_other_workspaces():
     raises(TypeError, lambda: qhip.qmatmul(w, x, workspace=Own()))
 
 
+def child_eps():
+    """`eps` belongs to the fused step: without one nothing reads it."""
+    import numpy as np
+    qhip, w = bind()
+    x, ws, offsets = fake(2, K), qhip.Workspace(), np.array([0, 2], np.int32)
+    ws.buf = fake(1024)
+    alpha = fake(K)
+    for call in (lambda **a: qhip.qmatmul(w, x, workspace=ws, **a), lambda **a: qhip.qmatmul_grouped([w], x, None, offsets, workspace=ws, **a)):
+        raises(RuntimeError, lambda: call(eps=None))   # (the allocation of the result)
+        raises(TypeError, lambda: call(pre=qhip.PRE_RMS_NORM, aux=alpha, eps=None))
+
+
 CHILDREN = {f[len("child_"):]: g for f, g in list(globals().items()) if f.startswith("child_")}
 
 
