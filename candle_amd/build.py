@@ -45,15 +45,20 @@ CALLS_SOURCE = "calls.cpp"
 CALLS_PATH = os.path.join(LIB_DIR, "_calls.so")
 
 
-def _build_calls() -> None:
+def _build_calls() -> bool:
+    """False without torch: nothing could load the module then."""
     import importlib.util
     import sysconfig
-    torch_dir = importlib.util.find_spec("torch").submodule_search_locations[0]
+    spec = importlib.util.find_spec("torch")
+    if spec is None:
+        return False
+    torch_dir = spec.submodule_search_locations[0]
     inc = [f"-I{os.path.join(torch_dir, d)}" for d in ("include", "include/torch/csrc/api/include")]
     inc.append("-I" + os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"))
     subprocess.check_call(["hipcc", "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
                            *inc, "-I" + sysconfig.get_paths()["include"], os.path.join(CSRC, CALLS_SOURCE), "-o", CALLS_PATH,
                            "-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip"])
+    return True
 
 
 def build(verbose: bool = True) -> str:
@@ -61,14 +66,15 @@ def build(verbose: bool = True) -> str:
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + 1)) as ex:
         calls = ex.submit(_build_calls)
         objs = list(ex.map(_compile, SOURCES + [PROBE_SOURCE]))
-        calls.result()
-    probe_obj = objs.pop()
-    subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs])
-    subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", PROBE_LIB_PATH, probe_obj])
+        probe_obj = objs.pop()
+        # the C libraries first: they need nothing of torch, whatever becomes of the module
+        subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs])
+        subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", PROBE_LIB_PATH, probe_obj])
+        have_calls = calls.result()
     if verbose:
         print("built", LIB_PATH)
         print("built", PROBE_LIB_PATH)
-        print("built", CALLS_PATH)
+        print("built" if have_calls else "not built (no torch):", CALLS_PATH)
     return LIB_PATH
 
 
