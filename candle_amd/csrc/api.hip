@@ -384,8 +384,12 @@ static size_t act_ws_layout(int act_dtype, int64_t m, int64_t k, uint8_t *base, 
     auto take = [&](size_t bytes) { size_t o = off; off = cq_align_up(off + bytes, 256); return o; };
     // Q8K rows are padded (see cq_act_view::m_stride); the others to whole 32-row groups, which the
     // split-K MFMA kernel copies without looking at the row count
-    // (beyond 32 rows to whole 128-row tiles, which the 32-element-block tile kernel reads, scales included)
+    // (beyond 32 rows to whole 128-row tiles, which the 32-element-block tile kernel reads)
     const int64_t m_pad = act_dtype == CQ_DTYPE_Q8K ? (m + 63) / 64 * 64 + 256 : (m <= 32 ? (m + 31) / 32 * 32 : (m + 127) / 128 * 128) + (grouped ? 128 : 0);
+    // Q8_0: the block-major scales come first.  The kernels copy whole K steps of eight blocks: past the last block of a row
+    // they read on into the quants (28 bytes a padded row at most, of 32 and more), past the last row's quants into the scales.
+    const bool q8_0 = act_dtype == CQ_DTYPE_Q8_0;
+    const size_t o_t8 = q8_0 ? take((size_t)(m_pad * (k / 32)) * 4) : 0;
     const size_t o_qs = take((size_t)(m_pad * k));
     cq_act_view view{};
     view.m_stride = m_pad;
@@ -400,16 +404,15 @@ static size_t act_ws_layout(int act_dtype, int64_t m, int64_t k, uint8_t *base, 
             view.bsh = (uint16_t *)(base + o_bh);
         }
     } else {
-        const size_t o_d = take((size_t)(m_pad * (k / 32)) * 4);
+        // Q8_1: scales and `s` fields padded, the tile kernel copies whole tiles of them
+        const size_t o_d = take((size_t)((q8_0 ? m : m_pad) * (k / 32)) * 4);
         const size_t o_s = take((size_t)(m * (k / 32)) * 2);
-        // Q8_0: the scales again, block-major; Q8_1: the `s` fields.  Padded: whole tiles are copied (and whole K steps of
-        // eight blocks).
-        const size_t o_t = take(act_dtype == CQ_DTYPE_Q8_1 ? (size_t)(m_pad * (k / 32)) * 2 : (size_t)(m_pad * ((k + 255) / 256)) * 32);
+        const size_t o_s16 = q8_0 ? 0 : take((size_t)(m_pad * (k / 32)) * 2);
         if (base) {
             view.qs = (int8_t *)(base + o_qs); view.d = (float *)(base + o_d);
             view.bsum32 = (int16_t *)(base + o_s);
-            if (act_dtype == CQ_DTYPE_Q8_1) view.s16 = (uint16_t *)(base + o_t);
-            else view.dT = (float *)(base + o_t);
+            if (q8_0) view.dT = (float *)(base + o_t8);
+            else view.s16 = (uint16_t *)(base + o_s16);
         }
     }
     if (v) *v = view;

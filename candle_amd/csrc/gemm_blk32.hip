@@ -37,9 +37,12 @@ constexpr int kThreads = kWaves * 64;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t wave_rsrc(const void *base) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, -1, 0x00020000);
 }
-// lane l reads 16 bytes at base + off, they land at lds + 16*l (base and lds wave-uniform)
+// lane l reads 16 (4) bytes at base + off, they land at lds + 16*l (4*l; base and lds wave-uniform)
 __device__ __forceinline__ void dma16(const void *base, uint32_t off, uint8_t *lds) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(wave_rsrc(base), (lptr_t)lds, 16, (int)off, 0, 0, 0);
+}
+__device__ __forceinline__ void dma4(const void *base, uint32_t off, uint8_t *lds) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wave_rsrc(base), (lptr_t)lds, 4, (int)off, 0, 0, 0);
 }
 // the same marked non-temporal: bytes that the launch reads once
 __device__ __forceinline__ void dma16_once(const void *base, uint32_t off, uint8_t *lds) {
@@ -48,7 +51,7 @@ __device__ __forceinline__ void dma16_once(const void *base, uint32_t off, uint8
 
 // LDS: two activation stages, then one weight buffer per wave.
 //   act : [MT tiles][2 K-halves][4 row groups][8 rows][8 chunks of 16 B]   chunk c of row r sits at c ^ (r%8)
-//   d8  : [32*MT rows][8 blocks] f32
+//   d8  : [MT tiles][8 blocks][32 rows] f32, out of the block-major plane (a lane per row reads one word of consecutive ones)
 //   wgt : per wave, Q8_0: [2 K-halves][4 row groups][8 rows][8 chunks]; Q4_0: [4 row groups][8 rows][8 chunks]
 template <int DT, int MT> struct Tile {
     static constexpr int kAct = MT * 8 * 1024;
@@ -63,17 +66,18 @@ template <int DT, int MT> struct Tile {
 struct LaneGeo {
     uint32_t row_off;    // copy of 8 rows x 128 B with a row pitch of k bytes: (l/8)*k + ((l%8) ^ (l/8))*16
     uint32_t w4_off;     // the same with the Q4_0 row pitch of k/2 bytes
-    uint32_t d8_off;     // copy of 32 rows x 32 B of block scales: (l/2)*(k/32)*4 + (l%2)*16
+    uint32_t d8_off;     // copy of 8 blocks x 32 rows of scales: block l/8, rows 4*(l%8)..; ANYROW two blocks: block l/32, row l%32
     uint32_t col[4];     // operand read: byte offset of chunk 2j+h of row l%32 inside a [4][8][8] x 16 B image
     uint32_t col4[8];    // Q4_0: chunk s of row l%32 (the 16 bytes of block s)
 };
 
-__device__ __forceinline__ LaneGeo lane_geo(int lane, int64_t k) {
+template <bool ANYROW> __device__ __forceinline__ LaneGeo lane_geo(int lane, int64_t k, int64_t m_stride) {
     LaneGeo g;
     const uint32_t r8 = lane >> 3, c8 = lane & 7;
     g.row_off = r8 * (uint32_t)k + ((c8 ^ r8) << 4);
     g.w4_off = r8 * (uint32_t)(k >> 1) + ((c8 ^ r8) << 4);
-    g.d8_off = (uint32_t)(lane >> 1) * (uint32_t)(k >> 5) * 4u + (uint32_t)(lane & 1) * 16u;
+    g.d8_off = ANYROW ? ((uint32_t)(lane >> 5) * (uint32_t)m_stride + (uint32_t)(lane & 31)) * 4u
+                      : ((uint32_t)(lane >> 3) * (uint32_t)m_stride + (uint32_t)(lane & 7) * 4u) * 4u;
     const uint32_t r = lane & 31, h = lane >> 5;
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) g.col[j] = (r >> 3) * 1024u + (r & 7) * 128u + (((2 * j + h) ^ (r & 7)) << 4);
@@ -82,8 +86,10 @@ __device__ __forceinline__ LaneGeo lane_geo(int lane, int64_t k) {
     return g;
 }
 
-// This wave's share of the activation copies of K step b into stage `buf`.
-template <int DT, int MT>
+// This wave's share of the activation copies of K step b into stage `buf`.  ANYROW: tiles begin at any row (a grouped launch),
+// where the scales of a block lie on four bytes and are copied word by word; otherwise rows and plane pitch are whole
+// 32-row groups, and 16 bytes a lane take a tile's scales in one copy.
+template <int DT, int MT, bool ANYROW>
 __device__ __forceinline__ void stage_acts(uint8_t *buf, const cq_act_view &a, const LaneGeo &g, int64_t k, int64_t m0,
                                            int64_t b, int wave) {
     typedef Tile<DT, MT> T;
@@ -93,10 +99,16 @@ __device__ __forceinline__ void stage_acts(uint8_t *buf, const cq_act_view &a, c
         const int rg = idx & 3, kh = (idx >> 2) & 1, t = idx >> 3;
         dma16(a.qs + (m0 + t * 32 + rg * 8) * k + b * 256 + kh * 128, g.row_off, buf + idx * 1024);
     }
-    // block scales: 32 rows x 8 floats per copy, one copy per tile
 #pragma unroll
     for (int t = 0; t < MT; t++) {
-        if (t + 4 == wave) dma16((const uint8_t *)(a.d + (m0 + t * 32) * (k >> 5) + b * 8), g.d8_off, buf + T::oD8 + t * 1024);
+        if (t + 4 != wave) continue;
+        const float *d8 = a.dT + b * 8 * a.m_stride + m0 + t * 32;
+        if (ANYROW) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) dma4(d8 + 2 * i * a.m_stride, g.d8_off, buf + T::oD8 + t * 1024 + i * 256);
+        } else {
+            dma16(d8, g.d8_off, buf + T::oD8 + t * 1024);
+        }
     }
 }
 
@@ -123,7 +135,7 @@ __device__ __forceinline__ void stage_weights(uint8_t *wl, const cq_weight &w, c
 // DUMP (verification): the block integers are stored through `dump` instead of the result through `y`.
 // ONCE: a launch with a single row tile (up to 32 rows), which reads every weight byte once.
 // SHORT: K is no multiple of 256, the last step has fewer than eight blocks.
-template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
+template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT, bool ANYROW = false>
 __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_view &a, int64_t bx, int64_t m0, int64_t m, float *__restrict__ y,
                                             int ksplit, cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
@@ -139,7 +151,7 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
     const int64_t n = n_tile + col;
     const int64_t nc = n_ok ? n : 0;
     const int64_t b0 = ks * blockIdx.z / ksplit, b1 = ks * (blockIdx.z + 1) / ksplit;
-    const LaneGeo g = lane_geo(lane, k);
+    const LaneGeo g = lane_geo<ANYROW>(lane, k, a.m_stride);
     uint8_t *__restrict__ wl = smem + T::oWgt + wave * T::kWgtWave;
     const uint16_t *dplane = (const uint16_t *)w.p1;    // f16 block scales [n][k/32]
 
@@ -149,7 +161,7 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
 #pragma unroll
         for (int i = 0; i < 16; i++) out[t][i] = 0.0f;
 
-    stage_acts<DT, MT>(smem, a, g, k, m0, b0, wave);
+    stage_acts<DT, MT, ANYROW>(smem, a, g, k, m0, b0, wave);
     if (n_ok) stage_weights<DT, ONCE>(wl, w, g, n_tile, b0);
     u32x4_a4 dnext = *(const u32x4_a4 *)(dplane + nc * (k >> 5) + b0 * 8);
     __builtin_amdgcn_s_waitcnt(0);
@@ -159,7 +171,7 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
         const uint8_t *__restrict__ cur = smem + ((b - b0) & 1) * T::kStage;
         uint8_t *__restrict__ nxt = smem + (((b - b0) & 1) ^ 1) * T::kStage;
         const bool more = b + 1 < b1;
-        if (more) stage_acts<DT, MT>(nxt, a, g, k, m0, b + 1, wave);
+        if (more) stage_acts<DT, MT, ANYROW>(nxt, a, g, k, m0, b + 1, wave);
         if (n_ok) {
             // weight operands of the eight blocks into registers, then the buffer is free for the next step
             v4i bw[8];
@@ -210,7 +222,7 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
             // waits for the read it has just issued
             auto d8raw = [&](int q) -> float {
                 const int t = q >> 3, s = q & 7;
-                const float v = *(const float *)(cur + T::oD8 + (t * 32 + col) * 32 + s * 4);
+                const float v = *(const float *)(cur + T::oD8 + t * 1024 + s * 128 + col * 4);
                 return !SHORT || s < nv ? v : 0.0f;
             };
             auto d8frag = [&](float v) -> v8bf {
@@ -310,7 +322,7 @@ template <int DT, int MT, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_grouped_kernel(GroupArgs ga, cq_act_view a, float *__restrict__ y, int ksplit) {
     const int tile = blockIdx.y;
     const cq_weight w = ga.w[ga.expert[tile]];
-    gemm32_body<DT, MT, false, MT == 1, SHORT>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit,
+    gemm32_body<DT, MT, false, MT == 1, SHORT, true>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit,
                                                cq_mfma_dump{nullptr, nullptr, 0});
 }
 

@@ -58,7 +58,7 @@ struct cq_weight {
 // (workspace layout).  Same numbers as the GGML activation blocks, split so
 // that int8 values are 16-byte aligned:
 //   Q8K : qs [m_stride][k] i8 ; d [m][k/256] f32 ; bsums [m][k/256][16] i16
-//   Q8_0: qs [m][k] i8 ; d [m][k/32]  f32 (the f16-rounded scale widened) ;
+//   Q8_0: dT [k/32][m_stride] f32 ; qs [m_stride][k] i8 ; d [m][k/32]  f32 (the f16-rounded scale widened) ;
 //         bsum [m][k/32] i16 (sum of the 32 quants, for the Q4_0 "-8" term)
 // ---------------------------------------------------------------------------
 struct cq_act_view {
