@@ -1481,11 +1481,26 @@ hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_exper
     }
 }
 
+// One launch over all the weights, or a launch each.  Measured with rms_norm in front, weights from HBM, five types, 2..16 rows,
+// ten pairs and triples from 1024 to 28672 weight rows and K = 1024..8192 (us of the whole call, one launch / a launch each):
+// the one launch is ahead everywhere (Q4K, 8 rows: 4096 + 1024 + 1024 x 4096 12.2 / 18.9, 2 x 14336 x 4096 24.3 / 26.8, 2 x 28672
+// x 8192 77.5 / 82.7; 16 rows: Q6K 2 x 14336 x 4096 32.2 / 37.2, Q8_0 2 x 11008 x 4096 31.2 / 31.8) but for nine rows and more of
+// many Q4K rows of sixteen blocks, where a weight by itself goes by rounds of tiles (launch_res_rt): 2 x 12288 x 4096
+// 26.1 / 24.7, 2 x 14336 28.5 / 28.1, 2 x 16384 30.6 / 28.6, 2 x 28672 47.2 / 44.3, 3 x 28672 67.0 / 63.7; but 2 x 13312 27.1 / 27.4,
+// 2 x 9728 22.0 / 23.2, 3 x 14336 37.5 / 40.2.  Which of them, by the two sums below, which follow these within 1 us (a launch
+// each: 4 us, 2 more for every tile of a workgroup, 1 for every further round of four tiles).  Fewer blocks leave some of
+// the rounds kernel's sixteen waves without one: K = 3840 and below within 3 % of each other, mostly for the one launch.
 bool cq_skinny_shared_takes(const cq_weight *const *ws, int count, int64_t m, int act_dtype) {
     if (count < 2 || count > kMultiMax || m > 16) return false;
-    for (int i = 0; i < count; i++)
+    const int64_t cus = cq_num_cus();
+    double shared = 10.3, each = 4.0;
+    for (int i = 0; i < count; i++) {
         if (!cq_skinny_takes(ws[i], act_dtype)) return false;
-    return true;
+        const int64_t tiles = (ws[i]->n + 15) / 16, turns = (tiles + cus - 1) / cus;
+        shared += 0.64e-3 * 16.0 * (double)tiles;
+        each += 4.0 + 2.0 * (double)turns + (double)((turns - 1) / kTilesPerRound);
+    }
+    return !(m > 8 && ws[0]->dtype == CQ_DTYPE_Q4K && ws[0]->k == 16 * QK_K && each < shared);
 }
 
 hipError_t cq_launch_skinny_shared(const cq_weight *const *ws, int count, cq_act_view a, int64_t m, float *const *ys, hipStream_t s) {

@@ -85,6 +85,41 @@ def test_few_rows_one_launch_equals_separate_calls(qh, dt, m):
         check_f32(y.cpu().numpy(), orc.matmul(dt, x, blocks, w.shape[0]))
 
 
+@pytest.mark.parametrize("dt", WEIGHT_DTYPES)
+@pytest.mark.parametrize("m", [2, 8, 9, 15, 16])
+@pytest.mark.parametrize("ns", [(250, 41, 16), (17, 335)])
+def test_shared_launch_of_ragged_weights(qh, dt, m, ns):
+    """The launch over the tiles of all weights at its edges: one and two groups of eight rows, weight rows that are no
+    multiple of 16, and for the 32-element types a last K step of two blocks.  The separate calls add a row's blocks
+    in another order: as many f32 additions of products as there are blocks (34 or 5), each 2^-24 of the row's size."""
+    k = 1280 if orc.TYPE_SIZE[dt] > 36 else 1088
+    ws = _weights(qh, dt, k, ns, 500 + dt + m)
+    rng = np.random.default_rng(m + dt)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    xd = dev(x)
+    alpha = dev(rng.standard_normal(k).astype(np.float32))
+    for pre, aux in ((qh.PRE_NONE, None), (qh.PRE_RMS_NORM, alpha)):
+        outs = qh.qmatmul_multi([w for w, _ in ws], xd, pre=pre, aux=aux, eps=1e-5)
+        for (w, blocks), y in zip(ws, outs):
+            want = qh.qmatmul(w, xd, pre=pre, aux=aux, eps=1e-5)
+            err = (y - want).double().norm(dim=1) / want.double().norm(dim=1)
+            assert err.max().item() <= 4 * 34 * 2.0 ** -24, err.max().item()
+            if pre == qh.PRE_NONE:
+                check_f32(y.cpu().numpy(), orc.matmul(dt, x, blocks, w.shape[0]))
+
+
+@pytest.mark.parametrize("ns", [(12288, 12288), (16384, 16380), (28672, 28672, 28672)])
+@pytest.mark.parametrize("m", [9, 16])
+def test_many_rows_of_sixteen_blocks_take_a_launch_each(qh, m, ns):
+    """Nine rows and more of these Q4K weights are faster by the kernel that walks rounds of tiles, one weight at a time: the
+    same launches as the separate calls, and so the same bits."""
+    g = torch.Generator(device="cuda").manual_seed(m)
+    ws = [qh.QWeight.zeros(qh.Q4K, n, 4096).quantize_(torch.randn(n, 4096, generator=g, device="cuda") * 0.02) for n in ns]
+    x = torch.randn(m, 4096, generator=g, device="cuda")
+    for w, y in zip(ws, qh.qmatmul_multi(ws, x)):
+        assert torch.equal(y, qh.qmatmul(w, x))
+
+
 def test_single_weight_four_weights_and_errors(qh):
     dt, k = orc.Q4K, 512
     ws = _weights(qh, dt, k, (32, 32, 64, 32), 300)
