@@ -1540,10 +1540,34 @@ hipError_t launch_fused_multi(const cq_weight *const *ws, int count, const float
 // against 10.5.  Every further row costs the dot products of one more row per unpacked unit, so the longer
 // the rows (elements per lane), the fewer rows pay off: K = 8192 Q4K 8.7 / 10.5 / 13.9 against 12.5,
 // K = 14336 Q4K 13.8 / 43 (registers spill) against 17.6.
-// Rows of at most 32 units leave half of a wave's lanes without one, at a fixed cost per weight row and activation row:
-// many of them go to the split-K kernel (Q4K 8192 x 2048 at 4 rows 8.5 against 7.5, 32000 x 2048 at 2 / 4 rows 14.4 / 21.0 against
-// 12.9, 32000 x 1024 13.6 / 20.8 against 9.8; Q4_0 32000 x 1024 at 3 / 4 rows 12.0 / 14.6 against 11.1), and so do four rows of
-// many long ones (32000 x 4096 Q4K 21.8 against 21.0, Q6K 28.9 against 27.1).
+// Whether two to four rows are faster through the quantizer and the split-K kernel than in one launch.  The one launch costs by
+// the weight row and activation row: in one pass of the wave over the row (two above 64 units) always the same whatever the
+// row's length, more where the rows of the quantized image in LDS collide (K-quant rows whose blocks are no multiple of
+// four, and most where they are odd).  The split-K kernel costs by the byte.  The two sums below (us; MB of weights) were fitted
+// to both over five types, 1024..32000 weight rows and every K of whole 256-element blocks up to 4096, weights from HBM:
+// over those 2500 shapes the choice is within 0.2 % of the better one on average and 18 % at worst.  Some of them (us, one
+// launch / split K, at 2, 3, 4 rows): Q4K 24576 x 2048 11.7/12.5, 14.6/12.6, 16.9/12.9; 8192 x 1024 5.7/6.6, 7.1/6.7, 8.4/6.8; 8192 x 1536
+// 7.3/7.2, 8.8/7.2, 12.0/7.3; 8192 x 768 7.2/6.3, 10.4/6.4, 13.9/6.5; Q6K 32000 x 4096 21.3/28.7, 27.2/29.2, 31.0/29.2;
+// Q4_0 16384 x 1024 6.2/8.4, 7.2/8.4, 8.7/8.4; 24576 x 3072 12.8/17.7, 15.8/17.9, 18.8/17.5.  Longer rows, and Q8_0: one launch.
+static bool rows_to_split_k(const cq_weight *w, int64_t m) {
+    if (w->k > 4096 || w->dtype == CQ_DTYPE_Q8_0) return false;
+    const double rows = (double)w->n / 1000.0, mb = (double)w->n * (double)(w->k / 256) * (double)(cq_type_size(w->dtype) * 256 / cq_block_size(w->dtype)) / 1e6;
+    const bool two_passes = w->k > (w->dtype == CQ_DTYPE_Q4K || w->dtype == CQ_DTYPE_Q5K ? 4096 : 2048);
+    if (w->dtype == CQ_DTYPE_Q4_0) {
+        static constexpr double per_row[2][3] = {{0.245, 0.30, 0.36}, {0.405, 0.50, 0.60}};
+        const double split = 4.6 + 0.09 * rows + 0.20 * mb;
+        return 2.1 + per_row[two_passes][m - 2] * rows > (split > 6.3 ? split : 6.3);
+    }
+    static constexpr double per_row[3][3][3] = {{{0.36, 0.45, 0.54}, {0.56, 0.69, 1.06}, {0.56, 0.96, 1.40}},     // Q4K; Q5K 0.05 more
+                                                {{0.35, 0.41, 0.47}, {0.40, 0.46, 0.60}, {0.40, 0.575, 0.76}},    // Q6K
+                                                {{0.54, 0.705, 0.84}, {0.67, 0.85, 1.155}, {0.68, 1.03, 1.45}}};  // Q6K, two passes
+    const bool q6k = w->dtype == CQ_DTYPE_Q6K, q5k = w->dtype == CQ_DTYPE_Q5K;
+    const int collide = w->k % 1024 == 0 ? 0 : w->k % 512 == 0 ? 1 : 2;
+    if (m == 4 && collide >= (q6k && !two_passes ? 2 : 1)) return true;
+    const double one = 1.5 + 0.6 * (double)m + (per_row[q6k ? 1 + two_passes : 0][collide][m - 2] + (q5k ? 0.05 : 0.0)) * rows;
+    const double split = 5.4 + 0.05 * rows + (q5k ? 0.26 : 0.22) * mb;
+    return one > (split > 6.5 ? split : 6.5);
+}
 bool cq_matvec_fused_rows_supported(const cq_weight *w, int64_t m) {
     if (m < 2 || m > 4 || !cq_matvec_fused_supported(w)) return false;
     int64_t units = 0, elems = 0;
@@ -1558,9 +1582,7 @@ bool cq_matvec_fused_rows_supported(const cq_weight *w, int64_t m) {
     }
     units = w->k / elems;
     if (units > (m == 2 ? 384 : 256) || row_bytes * (size_t)m > 64 * 1024 - 1024) return false;
-    const bool kquant = w->dtype == CQ_DTYPE_Q4K || w->dtype == CQ_DTYPE_Q5K || w->dtype == CQ_DTYPE_Q6K;
-    if (units <= 32 && ((kquant && w->n * m >= 28000) || (w->dtype == CQ_DTYPE_Q4_0 && w->n * m >= 90000))) return false;
-    if (m == 4 && w->n >= 16384 && kquant && w->dtype != CQ_DTYPE_Q5K) return false;
+    if (rows_to_split_k(w, m)) return false;
     const int64_t per_lane = (units + 63) / 64 * elems;   // elements of a row per lane
     return per_lane <= 64 ? true : per_lane <= 128 ? m <= 3 : m <= 2;
 }
