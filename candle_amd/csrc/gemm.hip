@@ -719,17 +719,22 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(cq_weight w, cq_act_view
 // 128-row tiles in whole rounds of workgroups, and what is left of them in tiles of 32 * TAIL rows: the last round of a launch
 // that does not fill it then lasts as long as a shorter tile.  `whole` of the `gx` x row tiles (column tiles first) are taken
 // whole, the others by 4 / TAIL workgroups each.  Measured at pick_plan.
-template <int DT, int TAIL>
-__global__ void __launch_bounds__(kThreads) gemm_tail_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t gx,
-                                                             uint32_t whole) {
+template <int DT, int TAIL, bool DUMP>
+__device__ __forceinline__ void tail_body(const cq_weight &w, const cq_act_view &a, int64_t m, float *__restrict__ y, uint32_t gx,
+                                          uint32_t whole, cq_mfma_dump dump) {
     const uint32_t id = blockIdx.x;
     if (id < whole) {
-        gemm_body<DT, 4>(w, a, id % gx, (int64_t)(id / gx) * 128, m, y, 1);
+        gemm_body<DT, 4, DUMP>(w, a, id % gx, (int64_t)(id / gx) * 128, m, y, 1, dump);
     } else {
         const uint32_t t = whole + (id - whole) / (4 / TAIL), part = (id - whole) % (4 / TAIL);
         const int64_t m0 = (int64_t)(t / gx) * 128 + part * (32 * TAIL);
-        if (m0 < m) gemm_body<DT, TAIL>(w, a, t % gx, m0, m, y, 1);
+        if (m0 < m) gemm_body<DT, TAIL, DUMP>(w, a, t % gx, m0, m, y, 1, dump);
     }
+}
+template <int DT, int TAIL>
+__global__ void __launch_bounds__(kThreads) gemm_tail_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t gx,
+                                                             uint32_t whole) {
+    tail_body<DT, TAIL, false>(w, a, m, y, gx, whole, cq_mfma_dump{nullptr, nullptr, 0});
 }
 
 // Up to 32 activation rows (one row tile): every weight byte is read once by the launch, cold - the form of the grouped
@@ -746,6 +751,11 @@ template <int DT, int MT>
 __global__ void __launch_bounds__(kThreads) gemm_dump_kernel(cq_weight w, cq_act_view a, int64_t m, int ksplit,
                                                              cq_mfma_dump dump) {
     gemm_body<DT, MT, true>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, nullptr, ksplit, dump);
+}
+template <int DT, int TAIL>
+__global__ void __launch_bounds__(kThreads) gemm_tail_dump_kernel(cq_weight w, cq_act_view a, int64_t m, uint32_t gx, uint32_t whole,
+                                                                  cq_mfma_dump dump) {
+    tail_body<DT, TAIL, true>(w, a, m, nullptr, gx, whole, dump);
 }
 
 // ------------------------------------------------------ few weight rows, long K: K halved inside the workgroup ----
@@ -1203,29 +1213,34 @@ hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, hip
     return hipGetLastError();
 }
 
-template <int DT, int TAIL>
-hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+// DUMP: the same launch storing the block integers through `d`.
+template <int DT, int TAIL, bool DUMP>
+hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = Tile<DT, 4>::kTotal;
-    if (hipError_t e = cq_ensure_lds<gemm_tail_kernel<DT, TAIL>>(w->dev, lds); e != hipSuccess) return e;
     const int64_t gx = n_tiles(w), tiles = gx * ((m + 127) / 128), whole = tiles / cq_num_cus() * cq_num_cus();
-    CQ_LAUNCH((gemm_tail_kernel<DT, TAIL>), (unsigned)(whole + (tiles - whole) * (4 / TAIL)), kThreads, lds, s, *w, a, m, y, (uint32_t)gx,
-              (uint32_t)whole);
+    const unsigned grid = (unsigned)(whole + (tiles - whole) * (4 / TAIL));
+    if constexpr (DUMP) {
+        if (hipError_t e = cq_ensure_lds<gemm_tail_dump_kernel<DT, TAIL>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm_tail_dump_kernel<DT, TAIL>), grid, kThreads, lds, s, *w, a, m, (uint32_t)gx, (uint32_t)whole, d);
+    } else {
+        if (hipError_t e = cq_ensure_lds<gemm_tail_kernel<DT, TAIL>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm_tail_kernel<DT, TAIL>), grid, kThreads, lds, s, *w, a, m, y, (uint32_t)gx, (uint32_t)whole);
+    }
     return hipGetLastError();
 }
 
 template <int DT>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool y_cleared, hipStream_t s) {
     const Plan p = pick_plan(w, m);
-    if (p.tail == 2) return launch_tail<DT, 2>(w, a, m, y, s);
-    if (p.tail == 1) return launch_tail<DT, 1>(w, a, m, y, s);
+    if (p.tail == 2) return launch_tail<DT, 2, false>(w, a, m, y, cq_mfma_dump{nullptr, nullptr, 0}, s);
+    if (p.tail == 1) return launch_tail<DT, 1, false>(w, a, m, y, cq_mfma_dump{nullptr, nullptr, 0}, s);
     if (p.kh == 2) return p.mt == 1 ? launch_kh<DT, 1>(w, a, m, y, s) : launch_kh<DT, 2>(w, a, m, y, s);
     if (p.mt == 1) return launch_mt<DT, 1>(w, a, m, y, p.ksplit, y_cleared, s);
     if (p.mt == 2) return launch_mt<DT, 2>(w, a, m, y, p.ksplit, y_cleared, s);
     return launch_mt<DT, 4>(w, a, m, y, p.ksplit, y_cleared, s);
 }
 
-// The launch cq_launch_gemm would make (same tile height, same K split), storing the block integers.  (A launch of two tile
-// heights is dumped in the taller one; the shorter ones' code is that of the launches of one height.)
+// The launch cq_launch_gemm would make (same tile heights, same K split), storing the block integers.
 template <int DT, int MT>
 hipError_t launch_dump_mt(const cq_weight *w, cq_act_view a, int64_t m, int ksplit, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = Tile<DT, MT>::kTotal;
@@ -1237,6 +1252,8 @@ hipError_t launch_dump_mt(const cq_weight *w, cq_act_view a, int64_t m, int kspl
 template <int DT>
 hipError_t launch_dump_dt(const cq_weight *w, cq_act_view a, int64_t m, cq_mfma_dump d, hipStream_t s) {
     const Plan p = pick_plan(w, m);
+    if (p.tail == 2) return launch_tail<DT, 2, true>(w, a, m, nullptr, d, s);
+    if (p.tail == 1) return launch_tail<DT, 1, true>(w, a, m, nullptr, d, s);
     if (p.mt == 1) return launch_dump_mt<DT, 1>(w, a, m, p.ksplit, d, s);
     if (p.mt == 2) return launch_dump_mt<DT, 2>(w, a, m, p.ksplit, d, s);
     return launch_dump_mt<DT, 4>(w, a, m, p.ksplit, d, s);

@@ -295,17 +295,16 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
 
 // 128-row tiles in whole rounds of workgroups, what is left of them in tiles of 32 * TAIL rows (as gemm_tail_kernel of
 // gemm.hip): `whole` of the gx x row tiles, column tiles first, are taken whole, the others by 4 / TAIL workgroups each.
-template <int DT, int TAIL, bool SHORT>
+template <int DT, int TAIL, bool DUMP, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_tail_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t gx,
-                                                               uint32_t whole) {
+                                                               uint32_t whole, cq_mfma_dump dump) {
     const uint32_t id = blockIdx.x;
-    const cq_mfma_dump none{nullptr, nullptr, 0};
     if (id < whole) {
-        gemm32_body<DT, 4, false, false, SHORT>(w, a, id % gx, (int64_t)(id / gx) * 128, m, y, 1, none);
+        gemm32_body<DT, 4, DUMP, false, SHORT>(w, a, id % gx, (int64_t)(id / gx) * 128, m, y, 1, dump);
     } else {
         const uint32_t t = whole + (id - whole) / (4 / TAIL), part = (id - whole) % (4 / TAIL);
         const int64_t m0 = (int64_t)(t / gx) * 128 + part * (32 * TAIL);
-        if (m0 < m) gemm32_body<DT, TAIL, false, false, SHORT>(w, a, t % gx, m0, m, y, 1, none);
+        if (m0 < m) gemm32_body<DT, TAIL, DUMP, false, SHORT>(w, a, t % gx, m0, m, y, 1, dump);
     }
 }
 
@@ -377,13 +376,13 @@ hipError_t launch_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, i
     CQ_LAUNCH((gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, d);
     return hipGetLastError();
 }
-template <int DT, int TAIL, bool SHORT>
-hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+template <int DT, int TAIL, bool DUMP, bool SHORT>
+hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = Tile<DT, 4>::kTotal;
-    if (hipError_t e = cq_ensure_lds<gemm32_tail_kernel<DT, TAIL, SHORT>>(w->dev, lds); e != hipSuccess) return e;
+    if (hipError_t e = cq_ensure_lds<gemm32_tail_kernel<DT, TAIL, DUMP, SHORT>>(w->dev, lds); e != hipSuccess) return e;
     const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), tiles = gx * ((m + 127) / 128), whole = tiles / cq_num_cus() * cq_num_cus();
-    CQ_LAUNCH((gemm32_tail_kernel<DT, TAIL, SHORT>), (unsigned)(whole + (tiles - whole) * (4 / TAIL)), kThreads, lds, s, *w, a, m, y,
-              (uint32_t)gx, (uint32_t)whole);
+    CQ_LAUNCH((gemm32_tail_kernel<DT, TAIL, DUMP, SHORT>), (unsigned)(whole + (tiles - whole) * (4 / TAIL)), kThreads, lds, s, *w, a, m, y,
+              (uint32_t)gx, (uint32_t)whole, d);
     return hipGetLastError();
 }
 template <int DT, int MT, bool DUMP>
@@ -413,10 +412,12 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
 template <int DT, bool DUMP>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool y_cleared, cq_mfma_dump d, hipStream_t s) {
     const Plan p = pick_plan(w, m);
-    if constexpr (!DUMP) {   // (dumped in the taller height: the shorter ones' code is that of the launches of one height)
-        const bool whole = w->k % 256 == 0;
-        if (p.tail == 2) return whole ? launch_tail<DT, 2, false>(w, a, m, y, s) : launch_tail<DT, 2, true>(w, a, m, y, s);
-        if (p.tail == 1) return whole ? launch_tail<DT, 1, false>(w, a, m, y, s) : launch_tail<DT, 1, true>(w, a, m, y, s);
+    if (DUMP || w->k % 256 == 0) {   // (whole K steps are all that is dumped)
+        if (p.tail == 2) return launch_tail<DT, 2, DUMP, false>(w, a, m, y, d, s);
+        if (p.tail == 1) return launch_tail<DT, 1, DUMP, false>(w, a, m, y, d, s);
+    } else if constexpr (!DUMP) {
+        if (p.tail == 2) return launch_tail<DT, 2, false, true>(w, a, m, y, d, s);
+        if (p.tail == 1) return launch_tail<DT, 1, false, true>(w, a, m, y, d, s);
     }
     if (p.mt == 1) return launch_mt<DT, 1, DUMP>(w, a, m, y, p.ksplit, y_cleared, d, s);
     if (p.mt == 2) return launch_mt<DT, 2, DUMP>(w, a, m, y, p.ksplit, y_cleared, d, s);

@@ -27,6 +27,19 @@ def test_rows_of_no_whole_step(qh, dt, m, n, k):  # noqa: F811
     check(qh, dt, m, n, k)
 
 
+@pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K", "Q8_0", "Q4_0"])
+@pytest.mark.parametrize("m,n,k", [(1100, 8192, 512), (1025, 8160, 256), (1000, 11264, 512)])
+def test_integers_of_both_heights(qh, dt, m, n, k):  # noqa: F811
+    """The same launches storing their block integers (the min term's as well): every one equals the dot-product kernels'."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w = QTensor.quantize(torch.randn(n, k, generator=g, device="cuda") * 0.02, GgmlDType[dt]).weight
+    x = torch.randn(m, k, generator=g, device="cuda")
+    got, mins = qh.qmatmul_int_dots_mfma(w, x, qh.MFMA_TILE | qh.MFMA_INT_MIN)
+    want, want_mins = qh.qmatmul_int_dots(w, x)
+    assert torch.equal(got, want)
+    assert mins is None or torch.equal(mins.to(torch.int32), want_mins)
+
+
 def check(qh, dt, m, n, k):  # noqa: F811
     block = 32 if dt in ("Q8_0", "Q4_0") else 256
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
