@@ -14,6 +14,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/device_lazy_init.h>
 
 #include <climits>
 
@@ -270,6 +271,7 @@ PyObject *py_dequantize(PyObject *const *a, Py_ssize_t na) {
     const cq_weight *w = weight_of(a[0]);
     int64_t n, k;
     if (const int rc = g_abi.weight_shape(w, &n, &k); rc != CQ_OK) return fail(rc);   // (no weight is an error there)
+    torch::utils::device_lazy_init(c10::kCUDA);   // the one call that may come before torch has touched the device
     const c10::Device dev(c10::kCUDA, (c10::DeviceIndex)g_abi.weight_device(w));
     Ref out(THPVariable_Wrap(at::Tensor(at::detail::empty_cuda({n, k}, f16 ? at::kHalf : at::kFloat, dev, std::nullopt))));
     if (!out.p) return nullptr;

@@ -41,3 +41,16 @@ def test_many_weights_on_the_same_rows(qh):
     want = [qh.qmatmul(w, x) for w in ws]
     for i, y in enumerate(qh.qmatmul_multi([ws[i % 3] for i in range(260)], x)):
         assert torch.equal(y, want[i % 3])
+
+
+def test_dequantize_initialises_torch():
+    """A program whose first device tensor is a dequantized weight: torch knows afterwards that the device is in use (its
+    memory statistics and its check for forked processes ask for that)."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = ("import torch; from candle_amd import qhip; d = qhip.QWeight.zeros(qhip.Q4K, 64, 512).dequantize(); "
+            "assert torch.cuda.is_initialized() and torch.cuda.memory_allocated() >= 64 * 512 * 4; print('ok', flush=True)")
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", (r.returncode, r.stdout, r.stderr[-2000:])
