@@ -879,19 +879,11 @@ __global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_v
 
 // Grouped (mixture-of-experts) variant: one launch for every expert.  blockIdx.y walks a table of
 // tiles of 32*MT expert-sorted activation rows; each tile names its expert's weights.
-constexpr int kMaxGroupExperts = 16, kMaxGroupTiles = 96;
-struct GroupArgs {
-    cq_weight w[kMaxGroupExperts];
-    int32_t row0[kMaxGroupTiles];      // first activation row of the tile
-    int32_t row_end[kMaxGroupTiles];   // end of its expert's rows
-    int8_t expert[kMaxGroupTiles];
-};
-
 // One row tile per expert: its weights are read once per launch, cold, and the types whose headers can come through the
 // copies take two buffers.  Taller tiles (experts with more rows) unpack a weight block once for up to 128 rows.
 template <int DT> constexpr int grouped_wbuf() { return DT == CQ_DTYPE_Q4K || DT == CQ_DTYPE_Q5K ? 2 : 1; }
 template <int DT, int MT>
-__global__ void __launch_bounds__(kThreads) gemm_grouped_kernel(GroupArgs ga, cq_act_view a, float *__restrict__ y,
+__global__ void __launch_bounds__(kThreads) gemm_grouped_kernel(cq_group_args ga, cq_act_view a, float *__restrict__ y,
                                                                 int ksplit) {
     const int tile = blockIdx.y;
     const cq_weight w = ga.w[ga.expert[tile]];
@@ -1259,11 +1251,6 @@ hipError_t launch_dump_dt(const cq_weight *w, cq_act_view a, int64_t m, cq_mfma_
     return launch_dump_mt<DT, 4>(w, a, m, p.ksplit, d, s);
 }
 
-int64_t grouped_tiles(const int32_t *offsets, int n_experts, int mt) {
-    int64_t tiles = 0;
-    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + 32 * mt - 1) / (32 * mt);
-    return tiles;
-}
 // Tile height and K split of a grouped launch.  A single 32-row tile per expert splits K for two workgroups per CU; taller
 // tiles, by the cost model of pick_plan without a split, where they need fewer rounds of work: 8 experts 14336 x 4096,
 // 512 routed rows (at most 73 each), as 32-row tiles and as planned: Q4K 162 -> 139 us, Q6K 226 -> 174; 4096 x 14336 Q6K
@@ -1274,8 +1261,8 @@ Plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
     Plan best{1, 1};
     double best_cost = 0.0;
     for (int mt = 1; mt <= 4; mt <<= 1) {
-        const int64_t tiles = grouped_tiles(offsets, n_experts, mt);
-        if (mt > 1 && tiles == grouped_tiles(offsets, n_experts, mt / 2)) break;   // half the height holds every expert's rows
+        const int64_t tiles = cq_group_tiles(offsets, n_experts, 32 * mt);
+        if (mt > 1 && tiles == cq_group_tiles(offsets, n_experts, 16 * mt)) break;   // half the height holds every expert's rows
         const int64_t rounds = (gx * tiles + cus - 1) / cus;
         const double cost = (double)rounds * ((double)kb * (unpack + 13.5 * mt) + 24.0);
         if (mt == 1 || cost < best_cost) {
@@ -1290,19 +1277,9 @@ Plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
 template <int DT, int MT>
 hipError_t launch_grouped_mt(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
                              float *y, int ksplit, bool y_cleared, hipStream_t s) {
-    GroupArgs ga;
-    int ntiles = 0;
-    for (int e = 0; e < n_experts; e++) {
-        ga.w[e] = *experts[e];
-        for (int32_t r = offsets[e]; r < offsets[e + 1]; r += 32 * MT) {
-            if (ntiles == kMaxGroupTiles) return hipErrorInvalidConfiguration;
-            ga.row0[ntiles] = r;
-            ga.row_end[ntiles] = offsets[e + 1];
-            ga.expert[ntiles] = (int8_t)e;
-            ntiles++;
-        }
-    }
-    if (ntiles == 0) return hipSuccess;
+    cq_group_args ga;
+    const int ntiles = cq_group_table(experts, n_experts, offsets, 32 * MT, &ga);
+    if (ntiles <= 0) return ntiles == 0 ? hipSuccess : hipErrorInvalidConfiguration;
     const cq_weight *w = experts[0];
     const size_t lds = MT == 1 && grouped_wbuf<DT>() == 2 ? Tile<DT, MT>::kTotal2 : Tile<DT, MT>::kTotal;
     if (hipError_t e = cq_ensure_lds<gemm_grouped_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
@@ -1345,7 +1322,7 @@ hipError_t launch_q81_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y,
 
 bool cq_gemm_grouped_supported(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
     if (n_experts > kMaxGroupExperts || !cq_gemm_takes(experts[0], act_dtype)) return false;
-    return grouped_tiles(offsets, n_experts, 1) <= kMaxGroupTiles;
+    return cq_group_tiles(offsets, n_experts, 32) <= kMaxGroupTiles;
 }
 
 hipError_t cq_launch_gemm_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
@@ -1366,7 +1343,7 @@ hipError_t cq_launch_gemm_dump(const cq_weight *w, cq_act_view a, int act_dtype,
 }
 
 bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets) {
-    return grouped_tiles(offsets, n_experts, 1) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
+    return cq_group_tiles(offsets, n_experts, 32) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
 }
 
 bool cq_gemm_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }

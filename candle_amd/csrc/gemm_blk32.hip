@@ -310,15 +310,8 @@ __global__ void __launch_bounds__(kThreads) gemm32_tail_kernel(cq_weight w, cq_a
 
 // Mixture-of-experts form: blockIdx.y walks a table of tiles of 32*MT rows of the expert-sorted activation rows; each tile names
 // its expert's weights (as gemm_grouped_kernel of gemm.hip).
-constexpr int kMaxGroupExperts = 16, kMaxGroupTiles = 96;
-struct GroupArgs {
-    cq_weight w[kMaxGroupExperts];
-    int32_t row0[kMaxGroupTiles];      // first activation row of the tile
-    int32_t row_end[kMaxGroupTiles];   // end of its expert's rows
-    int8_t expert[kMaxGroupTiles];
-};
 template <int DT, int MT, bool SHORT>
-__global__ void __launch_bounds__(kThreads) gemm32_grouped_kernel(GroupArgs ga, cq_act_view a, float *__restrict__ y, int ksplit) {
+__global__ void __launch_bounds__(kThreads) gemm32_grouped_kernel(cq_group_args ga, cq_act_view a, float *__restrict__ y, int ksplit) {
     const int tile = blockIdx.y;
     const cq_weight w = ga.w[ga.expert[tile]];
     gemm32_body<DT, MT, false, MT == 1, SHORT, true>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit,
@@ -424,23 +417,18 @@ hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, boo
     return launch_mt<DT, 4, DUMP>(w, a, m, y, p.ksplit, y_cleared, d, s);
 }
 
-int64_t grouped_tiles(const int32_t *offsets, int n_experts, int mt) {
-    int64_t tiles = 0;
-    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + 32 * mt - 1) / (32 * mt);
-    return tiles;
-}
 // Tile height and K split of a grouped launch.  Too few 32-row tiles for two workgroups per CU: K is split (at least two
 // steps per part).  Otherwise the height with the least work by the cost model of pick_plan.
 Plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
     const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks = (w->k + 255) >> 8, cus = cq_num_cus();
-    int64_t tiles = grouped_tiles(offsets, n_experts, 1);
+    int64_t tiles = cq_group_tiles(offsets, n_experts, 32);
     int split = 1;
     while (!cq_no_split_k() && gx * tiles * split * 2 <= 2 * cus && ks / (split * 2) >= 2 && split < 16) split *= 2;
     Plan best{1, split};
     double best_cost = 0.0;
     for (int mt = 1; mt <= 4 && split == 1; mt <<= 1) {
-        tiles = grouped_tiles(offsets, n_experts, mt);
-        if (mt > 1 && tiles == grouped_tiles(offsets, n_experts, mt / 2)) break;   // half the height holds every expert's rows
+        tiles = cq_group_tiles(offsets, n_experts, 32 * mt);
+        if (mt > 1 && tiles == cq_group_tiles(offsets, n_experts, 16 * mt)) break;   // half the height holds every expert's rows
         const double cost = (double)((gx * tiles + cus - 1) / cus) * ((double)ks * (10.0 + 23.0 * mt) + 24.0);
         if (mt == 1 || cost < best_cost) {
             best = Plan{mt, 1};
@@ -453,18 +441,9 @@ Plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
 template <int DT, int MT, bool SHORT>
 hipError_t launch_grouped_mt(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
                              int ksplit, bool y_cleared, hipStream_t s) {
-    GroupArgs ga;
-    int tiles = 0;
-    for (int e = 0; e < n_experts; e++) {
-        ga.w[e] = *experts[e];
-        for (int32_t r = offsets[e]; r < offsets[e + 1]; r += 32 * MT) {
-            if (tiles == kMaxGroupTiles) return hipErrorInvalidConfiguration;
-            ga.row0[tiles] = r;
-            ga.row_end[tiles] = offsets[e + 1];
-            ga.expert[tiles++] = (int8_t)e;
-        }
-    }
-    if (tiles == 0) return hipSuccess;
+    cq_group_args ga;
+    const int tiles = cq_group_table(experts, n_experts, offsets, 32 * MT, &ga);
+    if (tiles <= 0) return tiles == 0 ? hipSuccess : hipErrorInvalidConfiguration;
     const cq_weight *w = experts[0];
     const size_t lds = Tile<DT, MT>::kTotal;
     if (hipError_t e = cq_ensure_lds<gemm32_grouped_kernel<DT, MT, SHORT>>(w->dev, lds); e != hipSuccess) return e;
@@ -488,10 +467,10 @@ hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const 
 }  // namespace
 
 bool cq_gemm32_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
-    return n_experts <= kMaxGroupExperts && cq_gemm32_takes(experts[0], act_dtype) && grouped_tiles(offsets, n_experts, 1) <= kMaxGroupTiles;
+    return n_experts <= kMaxGroupExperts && cq_gemm32_takes(experts[0], act_dtype) && cq_group_tiles(offsets, n_experts, 32) <= kMaxGroupTiles;
 }
 bool cq_gemm32_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets) {
-    return grouped_tiles(offsets, n_experts, 1) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
+    return cq_group_tiles(offsets, n_experts, 32) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
 }
 hipError_t cq_launch_gemm32_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
                                     bool y_cleared, hipStream_t s) {

@@ -217,6 +217,33 @@ hipError_t cq_launch_skinny_shared(const cq_weight *const *ws, int count, cq_act
 bool cq_skinny_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype);
 hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
                                     hipStream_t s);
+// Table of a grouped launch, passed by value: tiles of up to `rows` expert-sorted activation rows, each of one expert.
+constexpr int kMaxGroupExperts = 16, kMaxGroupTiles = 96;
+struct cq_group_args {
+    cq_weight w[kMaxGroupExperts];
+    int32_t row0[kMaxGroupTiles];      // first activation row of the tile
+    int32_t row_end[kMaxGroupTiles];   // end of its expert's rows
+    int8_t expert[kMaxGroupTiles];
+};
+static inline int64_t cq_group_tiles(const int32_t *offsets, int n_experts, int rows) {
+    int64_t tiles = 0;
+    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + rows - 1) / rows;
+    return tiles;
+}
+// Fills the table; the number of its tiles, or -1 where they do not fit.
+static inline int cq_group_table(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int rows, cq_group_args *ga) {
+    int tiles = 0;
+    for (int e = 0; e < n_experts; e++) {
+        ga->w[e] = *experts[e];
+        for (int32_t r = offsets[e]; r < offsets[e + 1]; r += rows) {
+            if (tiles == kMaxGroupTiles) return -1;
+            ga->row0[tiles] = r;
+            ga->row_end[tiles] = offsets[e + 1];
+            ga->expert[tiles++] = (int8_t)e;
+        }
+    }
+    return tiles;
+}
 // moe.hip
 hipError_t cq_launch_silu_mul(const float *a, const float *b, float *h, int64_t count, hipStream_t s);
 hipError_t cq_launch_scatter_add(const float *y, const int32_t *row_ids, const float *weights, int64_t total_rows,

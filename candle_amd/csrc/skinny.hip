@@ -891,15 +891,8 @@ __global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_
 
 // Mixture-of-experts form of the two: blockIdx.y is a tile of up to 8 * RT routed rows and names its expert's weights, so
 // that a projection of all experts is one launch, as in the grouped tile kernel (gemm.hip).
-constexpr int kMaxGroupExperts = 16, kMaxGroupTiles = 96;
-struct GroupArgs {
-    cq_weight w[kMaxGroupExperts];
-    int32_t row0[kMaxGroupTiles];      // first activation row of the tile
-    int32_t row_end[kMaxGroupTiles];   // end of its expert's rows
-    int8_t expert[kMaxGroupTiles];
-};
 template <int DT, int RT>
-__global__ void __launch_bounds__(kThreads) skinny_grouped_kernel(GroupArgs ga, cq_act_view a, float *__restrict__ y) {
+__global__ void __launch_bounds__(kThreads) skinny_grouped_kernel(cq_group_args ga, cq_act_view a, float *__restrict__ y) {
     const int tile = blockIdx.y;
     const int64_t m0 = ga.row0[tile], end = ga.row_end[tile], m = m0 + 8 * RT < end ? m0 + 8 * RT : end;
     const cq_weight w = ga.w[ga.expert[tile]];
@@ -1390,18 +1383,9 @@ template <int DT> hipError_t launch_shared(const MultiArgs &ma, unsigned tiles, 
 
 template <int DT, int RT>
 hipError_t launch_grouped_rt(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y, hipStream_t s) {
-    GroupArgs ga;
-    int tiles = 0;
-    for (int e = 0; e < n_experts; e++) {
-        ga.w[e] = *experts[e];
-        for (int32_t r = offsets[e]; r < offsets[e + 1]; r += 8 * RT) {
-            if (tiles == kMaxGroupTiles) return hipErrorInvalidConfiguration;
-            ga.row0[tiles] = r;
-            ga.row_end[tiles] = offsets[e + 1];
-            ga.expert[tiles++] = (int8_t)e;
-        }
-    }
-    if (tiles == 0) return hipSuccess;
+    cq_group_args ga;
+    const int tiles = cq_group_table(experts, n_experts, offsets, 8 * RT, &ga);
+    if (tiles <= 0) return tiles == 0 ? hipSuccess : hipErrorInvalidConfiguration;
     const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<DT, RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
     if (hipError_t e = cq_ensure_lds<skinny_grouped_kernel<DT, RT>>(experts[0]->dev, lds); e != hipSuccess) return e;
     CQ_LAUNCH((skinny_grouped_kernel<DT, RT>), dim3((unsigned)((experts[0]->n + 15) / 16), (unsigned)tiles), kThreads, lds, s, ga, a, y);
@@ -1463,10 +1447,7 @@ hipError_t cq_launch_skinny_dump(const cq_weight *w, cq_act_view a, int act_dtyp
 
 bool cq_skinny_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
     if (n_experts > kMaxGroupExperts || !cq_skinny_takes(experts[0], act_dtype)) return false;
-    const int rows = 8 * grouped_rt(n_experts, offsets);
-    int64_t tiles = 0;
-    for (int e = 0; e < n_experts; e++) tiles += (offsets[e + 1] - offsets[e] + rows - 1) / rows;
-    return tiles <= kMaxGroupTiles;
+    return cq_group_tiles(offsets, n_experts, 8 * grouped_rt(n_experts, offsets)) <= kMaxGroupTiles;
 }
 
 hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
