@@ -88,7 +88,7 @@ enum {
     CQ_FLAG_STAGED_ACT = 16,  /* up to four rows: run the stand-alone quantizer into the workspace and a matmul kernel
                                  (two launches, as cuda.rs:249-293 does) instead of the single fused launch           */
     CQ_FLAG_DETERMINISTIC = 64 /* the same bits on every run, like the CPU QMatMul.  Without it one family of launches is
-                                 not: the tile kernels (17 rows and more; grouped experts with more than 8 rows) split K
+                                 not: the tile kernels (17 rows and more; grouped experts with more than 16, of large Q8_0 weights 4) split K
                                  over several workgroups when the weight has few row tiles - n = 4096 at 33 .. 1024
                                  rows, the w2 projection of an expert - and add the partial sums atomically in
                                  arrival order, so the last bits of a result can differ between two runs (far inside
