@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the quantized-matmul hot path on one MI355X.
 
-Workload (BASELINE.json configs[1]): the Llama-2-7B-shaped decode QMatMul stack at batch 1 -
+Workload: the Llama-2-7B-shaped decode QMatMul stack at batch 1 -
 per layer q/k/v/o [4096x4096] Q4_K, gate/up [11008x4096] Q4_K, down [4096x11008] Q6_K, 32 layers,
 plus an lm_head [32000x4096] Q6_K; activations f32 N(0,1) quantized to Q8_K.  A "step" is one
 pass over all 225 QMatMul calls (4 122 255 360 bytes of GGML weights, all distinct, so every call
@@ -150,7 +150,7 @@ def envelope() -> int:
 
 
 def config3_activations(torch, gen, m, k, dev):
-    """f32 N(0,1) with 1 % of the positions at +-8 sigma (the time of an int8 MFMA depends on its
+    """The prefill workload's activations: f32 N(0,1) with 1 % of the positions at +-8 sigma (the time of an int8 MFMA depends on its
     operands' bits, so the prefill figures are timed on the configuration's own inputs)."""
     x = torch.randn((m, k), generator=gen, device=dev, dtype=torch.float32)
     pos = torch.rand((m, k), generator=gen, device=dev) < 0.01
@@ -193,7 +193,7 @@ def mfma_clock_probe(torch):
 
 
 def small_batch_probe(rounds: int, copy_probe: bool = False) -> int:
-    """configs[2] alone, for a profiler run: whole cq_qmatmul calls with 2, 8 and 16 activation rows on Q4_K and
+    """The small batches alone, for a profiler run: whole cq_qmatmul calls with 2, 8 and 16 activation rows on Q4_K and
     Q8_0 weights of both decode shapes, launched eagerly `rounds` times over sixteen distinct weights per shape
     (each call streams its weights from HBM), and the same timed with HIP events.  One JSON line."""
     import ctypes as C
@@ -431,7 +431,7 @@ def main() -> int:
     small_gbs = (sum(b for _, b in small) / sum(d for d, _ in small) / 1e9) if small else None
 
     # ---- the other half of the metric: Q4_K prefill GEMM, M = 512 on the Mistral FFN shape ----
-    # (reported beside the headline, not as `value`)
+    # (the prefill workload; reported beside the headline, not as `value`)
     gm, gk, gn = 512, 4096, 14336
     gen.manual_seed(4242)
     gw = torch.randn((gn, gk), generator=gen, device=dev, dtype=torch.float32) * 0.02
@@ -459,7 +459,7 @@ def main() -> int:
     gemm_tops = 2.0 * gm * gk * gn / (gemm_avg_us * 1e-6) / 1e12
     del gq, gx, gy, gws
 
-    # whole calls (activation quantizer + GEMM) on both shapes of configs[3] and on the attention shape
+    # whole calls (activation quantizer + GEMM) on both prefill shapes and on the attention shape
     whole_calls = {}
     gemm_cases = {}
     if not args.no_extras:
@@ -661,7 +661,7 @@ def main() -> int:
         if not (args.no_extras or args.no_graph):
             print(f"bench.py: merged-projection step not measured ({e})", file=sys.stderr)
 
-    # ---- configs[2]-style small batches on the headline's weights (reported beside the headline) --------
+    # ---- small batches on the headline's weights (reported beside the headline) --------
     # Whole calls (quantizer launch included where there is one), graph replay over the 32 layers' attn_q
     # [4096 x 4096] and ffn_gate [11008 x 4096] weights, so every call streams its weights from HBM.
     small_batch = None
@@ -705,8 +705,8 @@ def main() -> int:
             print(f"bench.py: small batches not measured ({e})", file=sys.stderr)
 
     # ---- the other configurations' shapes, whole calls in a graph replay (reported beside the headline) ------
-    # one Q4_0 [4096 x 4096] matvec (Q8_0 activations); configs[2]'s Q8_0 half: 2-16 rows on
-    # Q8_0 weights of both decode shapes; configs[4]: the Mixtral-shaped expert FFN (8 experts, 64 tokens,
+    # one Q4_0 [4096 x 4096] matvec (Q8_0 activations); the Q8_0 half of the small batches: 2-16 rows on
+    # Q8_0 weights of both decode shapes; the Mixtral-shaped expert FFN (8 experts, 64 tokens,
     # top-2: two grouped launches on the routed rows, silu * mul on the way into the grouped w2 launch,
     # weighted scatter-add).  Sixteen distinct weights per shape take turns so that each call streams from HBM.
     other = None

@@ -1,6 +1,6 @@
 """The per-block integer dot products out of the matrix-core kernels (the small-batch split-K kernels and the prefill
 tile kernels), bit for bit against the oracle's `block_int_dots` (k_quants.rs:1221-1241 for Q4K, :1418-1438 for Q5K,
-:1615-1633 for Q6K, :245-250 / :640-645 for Q4_0 / Q8_0) and, at the BASELINE configs[3] shape, against the
+:1615-1633 for Q6K, :245-250 / :640-645 for Q4_0 / Q8_0) and, at the prefill shape (512 rows), against the
 dot-product kernels' integers over the whole launch.  The Q4K / Q5K min term is not an integer in these kernels: it
 is contracted on the f16 matrix core from operands split in two f16 pieces; its distance to the integer form is
 bounded here."""
@@ -221,7 +221,7 @@ def test_grouped_rows_of_different_magnitudes(qh, dt):
 
 @pytest.mark.parametrize("dt,k,n", [(orc.Q4K, 4096, 14336), (orc.Q6K, 14336, 4096)])
 def test_tile_kernel_integers_config3(qh, dt, k, n):
-    """BASELINE configs[3] at full size (M = 512, 1 % outliers at +-8 sigma): every block integer of the launch equals
+    """The prefill workload at full size (M = 512, 1 % outliers at +-8 sigma): every block integer of the launch equals
     the dot-product kernels' (compared on the device), and sampled rows equal the oracle's."""
     m = 512
     rng = np.random.default_rng(n + int(dt))

@@ -1,6 +1,6 @@
 """Parity of the HIP path (through the C ABI) against the CPU oracle on identical seeded inputs.
 
-Bars (BASELINE north star): quantized activation blocks and per-block integer dot products
+Bars: quantized activation blocks and per-block integer dot products
 bit-exact; f32 outputs within relative L2 1e-4 and max-abs <= 1e-3 * ||row||_2.
 """
 import numpy as np
@@ -42,7 +42,7 @@ def make_inputs(seed, m, k, n, wscale=0.02, outliers=False):
     rng = np.random.default_rng(seed)
     w = (rng.standard_normal((n, k)) * wscale).astype(np.float32)
     x = rng.standard_normal((m, k)).astype(np.float32)
-    if outliers:  # 1% of positions at +-8 sigma
+    if outliers:  # 1% of positions at +-8 sigma (the prefill workload)
         idx = rng.choice(x.size, size=max(1, x.size // 100), replace=False)
         x.ravel()[idx] = np.where(rng.random(idx.size) < 0.5, -8.0, 8.0).astype(np.float32)
     return w, x
@@ -257,7 +257,7 @@ def test_rounding_instruction_selfcheck(qh):
 @pytest.mark.parametrize("m", [2, 4, 8, 16])
 @pytest.mark.parametrize("k,n", [(4096, 4096), (4096, 11008)])
 def test_small_batch_matches_oracle(qh, dt, m, k, n):
-    """M in {2,4,8,16} on the decode shapes."""
+    """Small batches: M in {2,4,8,16} on the decode shapes."""
     w, x = make_inputs(dt + m + n, m, k, n)
     blocks = orc.quantize(dt, w)
     qw = qh.QWeight.from_ggml(dt, blocks, n, k)
@@ -402,7 +402,7 @@ def test_gemm_needs_32_row_multiple(qh, dt):
                                       (orc.Q2K, 512, 14336, 4096), (orc.Q5_0, 16, 4096, 11008), (orc.Q5_0, 512, 4096, 14336),
                                       (orc.Q4_1, 1, 4096, 11008), (orc.Q5_1, 512, 4096, 4096), (orc.Q8K, 3, 4096, 4096)])
 def test_other_weight_types_at_model_shapes(qh, dt, m, k, n):
-    """The types that are held in another type's planes (and Q8K weights) at the shapes of the BASELINE configurations:
+    """The types that are held in another type's planes (and Q8K weights) at the shapes of the measured workloads:
     weights quantized on the device, sampled weight rows (first, last, tile edges, random) over all activation rows
     against the oracle's own code for the type, and the bytes of the sampled rows against the oracle's quantizer."""
     rng = np.random.default_rng(k + n + int(dt))
@@ -431,7 +431,7 @@ def test_other_weight_types_at_model_shapes(qh, dt, m, k, n):
 @pytest.mark.parametrize("dt", [orc.Q4K, orc.Q5K, orc.Q6K])
 @pytest.mark.parametrize("m,k,n", [(512, 4096, 14336), (512, 14336, 4096)])
 def test_prefill_gemm_config3(qh, dt, m, k, n):
-    """BASELINE config 3 at full size: M = 512 tokens on the Mistral FFN shapes, activations N(0,1)
+    """The prefill workload at full size: M = 512 tokens on the Mistral FFN shapes, activations N(0,1)
     with 1% outliers at +-8 sigma.  Weights are quantized on the device (bit-identical to the CPU
     quantizer, checked above).  The oracle evaluates, over all 512 tokens, 96 weight rows: the first and the last
     row of the first, a middle and the last workgroup tile (256 weight rows each), of a wave's 32-row tile inside
@@ -578,7 +578,7 @@ def test_kernel_choice_at_its_row_count_limits(qh, dt, m, k, n):
 def test_moe_ffn_matches_oracle(qh, tokens, starve):
     """Mixtral-shaped expert FFN at reduced width: routed top-2, per-expert gathered QMatMul,
     silu(w1 x) * w3 x, w2, scaled scatter-add (quantized_llama.rs:75-143).  24 tokens keep every
-    expert on the dot-product kernels (at most 8 rows each); 64 tokens (BASELINE config 4's count)
+    expert on the dot-product kernels (at most 8 rows each); 64 tokens (the expert workload's count)
     with one expert that no token picks give experts on the tile kernel and an empty slice."""
     rng = np.random.default_rng(23 + tokens)
     hidden, ffn, n_e, top_k = 512, 1024, 8, 2
@@ -675,7 +675,7 @@ def test_moe_scatter_add_order_and_shapes(qh, tokens, total, hidden):
 
 
 def test_moe_config4_full_size(qh):
-    """BASELINE config 4 at its real shape: 8 experts of w1/w3 [14336 x 4096] Q4K and w2 [4096 x 14336]
+    """The expert workload at its real shape: 8 experts of w1/w3 [14336 x 4096] Q4K and w2 [4096 x 14336]
     Q6K, 64 tokens routed top-2.  The oracle would need minutes for all of it, so: every expert's
     slice of each grouped launch is compared with the plain tile kernel on the same rows (the same
     workgroup body without the tile table), a sample of weight rows of every expert with the

@@ -72,7 +72,7 @@ def test_q8_1_variant_matches_oracle_and_exact_formula(qh, dt, m, k, n):
 @pytest.mark.parametrize("dt", [orc.Q4K, orc.Q6K])
 @pytest.mark.parametrize("k,n", [(4096, 14336), (14336, 4096)])
 def test_q8_1_variant_config3_shapes(qh, dt, k, n):
-    """M = 512 with 1 % outliers at +-8 sigma; sampled weight rows against the oracle (the whole
+    """The prefill workload: M = 512 with 1 % outliers at +-8 sigma; sampled weight rows against the oracle (the whole
     product would take the scalar oracle minutes) and the whole output against the Q8K formulation, from which it may
     differ by the two activation quantizers' noise only."""
     rng = np.random.default_rng(n)
