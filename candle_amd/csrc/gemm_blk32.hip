@@ -7,19 +7,20 @@
 // A 32-element block is exactly one K-slice of v_mfma_i32_32x32x32_i8, so the integer of every
 // (activation row, weight row, block) is one MFMA result element, I (Q4_0 nibbles go in as q - 8, so
 // no correction term is left).  Its scale d8[row, block] * dw[col, block] is an outer product: a
-// second MFMA lays it out in the accumulator layout (v_mfma_f32_32x32x16_bf16 with six non-zero K-slots:
-// d8 goes in as three bf16 pieces and dw, an f16, as two, all exact, so the six products are the exact
-// product whatever the magnitude of the activations - f16 pieces would lose d8 below 2^-14 - and the result is
-// d8 * dw to f32 rounding; the f32 MFMA with one K-slot holds the matrix pipe twice as long), and the VALU
+// second MFMA lays it out in the accumulator layout (v_mfma_f32_32x32x16_bf16 with four non-zero K-slots:
+// both scales are f16 values and go in as two bf16 pieces each, all exact, so the four products are the exact
+// product whatever the magnitude of the activations, and the result is d8 * dw to f32 rounding; the f32 MFMA with
+// one K-slot holds the matrix pipe twice as long), and the VALU
 // work per element is one conversion and one fma.
 //
 // Work split as in the K-quant tile kernel (gemm.hip): a workgroup of eight waves covers 32*MT
 // activation rows x 256 weight rows, a wave owns 32 weight rows; per 256-element step of K the
 // activations (shared) and the wave's weight bytes go from global memory straight into LDS
 // (buffer_load ... lds, 8 rows x 128 B per instruction, 16-byte chunks XOR-swizzled by the row),
-// activations double buffered one step ahead.  With few workgroups K is split over blockIdx.z and
-// the partial results are added atomically into a zeroed output.
+// activations double buffered one step ahead.  Where that gives few workgroups K is split inside them (gemm32_kh_kernel, and
+// for up to 32 rows gemm32_few_kernel) or over blockIdx.z, the partial results then added atomically into a zeroed output.
 #include "qhip_internal.h"
+#include <type_traits>
 
 namespace {
 
@@ -50,7 +51,9 @@ __device__ __forceinline__ void dma16_once(const void *base, uint32_t off, uint8
 }
 
 // LDS: two activation stages, then one weight buffer per wave.
-//   act : [MT tiles][2 K-halves][4 row groups][8 rows][8 chunks of 16 B]   chunk c of row r sits at c ^ (r%8)
+//   act : [MT tiles][2 K-halves][4 row groups][8 rows][8 chunks of 16 B]   chunk c of row r sits at c ^ (r%8) ^ ((r/8)%2)
+//         (a 16-byte read serves sixteen lanes at a time, rows of two groups: with c ^ (r%8) alone they meet in half the banks,
+//         8.3 cycles a read instead of 5.0)
 //   d8  : [MT tiles][8 blocks][32 rows] f32, out of the block-major plane (a lane per row reads one word of consecutive ones)
 //   wgt : per wave, Q8_0: [2 K-halves][4 row groups][8 rows][8 chunks]; Q4_0: [4 row groups][8 rows][8 chunks]
 template <int DT, int MT> struct Tile {
@@ -64,7 +67,7 @@ template <int DT, int MT> struct Tile {
 };
 
 struct LaneGeo {
-    uint32_t row_off;    // copy of 8 rows x 128 B with a row pitch of k bytes: (l/8)*k + ((l%8) ^ (l/8))*16
+    uint32_t row_off;    // copy of 8 rows x 128 B with a row pitch of k bytes: (l/8)*k + ((l%8) ^ (l/8))*16; odd row groups: ^ 16
     uint32_t w4_off;     // the same with the Q4_0 row pitch of k/2 bytes
     uint32_t d8_off;     // copy of 8 blocks x 32 rows of scales: block l/8, rows 4*(l%8)..; ANYROW two blocks: block l/32, row l%32
     uint32_t col[4];     // operand read: byte offset of chunk 2j+h of row l%32 inside a [4][8][8] x 16 B image
@@ -80,9 +83,9 @@ template <bool ANYROW> __device__ __forceinline__ LaneGeo lane_geo(int lane, int
                       : ((uint32_t)(lane >> 3) * (uint32_t)m_stride + (uint32_t)(lane & 7) * 4u) * 4u;
     const uint32_t r = lane & 31, h = lane >> 5;
 #pragma unroll
-    for (uint32_t j = 0; j < 4; j++) g.col[j] = (r >> 3) * 1024u + (r & 7) * 128u + (((2 * j + h) ^ (r & 7)) << 4);
+    for (uint32_t j = 0; j < 4; j++) g.col[j] = (r >> 3) * 1024u + (r & 7) * 128u + (((2 * j + h) ^ (r & 7) ^ ((r >> 3) & 1)) << 4);
 #pragma unroll
-    for (uint32_t s = 0; s < 8; s++) g.col4[s] = (r >> 3) * 1024u + (r & 7) * 128u + ((s ^ (r & 7)) << 4);
+    for (uint32_t s = 0; s < 8; s++) g.col4[s] = (r >> 3) * 1024u + (r & 7) * 128u + ((s ^ (r & 7) ^ ((r >> 3) & 1)) << 4);
     return g;
 }
 
@@ -97,7 +100,7 @@ __device__ __forceinline__ void stage_acts(uint8_t *buf, const cq_act_view &a, c
     for (int j = 0; j < MT * 8 / kWaves; j++) {
         const int idx = wave + kWaves * j;           // = (t*2 + kh)*4 + rg
         const int rg = idx & 3, kh = (idx >> 2) & 1, t = idx >> 3;
-        dma16(a.qs + (m0 + t * 32 + rg * 8) * k + b * 256 + kh * 128, g.row_off, buf + idx * 1024);
+        dma16(a.qs + (m0 + t * 32 + rg * 8) * k + b * 256 + kh * 128, g.row_off ^ (uint32_t)((rg & 1) << 4), buf + idx * 1024);
     }
 #pragma unroll
     for (int t = 0; t < MT; t++) {
@@ -120,15 +123,109 @@ __device__ __forceinline__ void stage_weights(uint8_t *wl, const cq_weight &w, c
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int rg = i & 3, kh = i >> 2;
-            if (ONCE) dma16_once(w.p0 + (n_tile + rg * 8) * k + b * 256 + kh * 128, g.row_off, wl + i * 1024);
-            else dma16(w.p0 + (n_tile + rg * 8) * k + b * 256 + kh * 128, g.row_off, wl + i * 1024);
+            if (ONCE) dma16_once(w.p0 + (n_tile + rg * 8) * k + b * 256 + kh * 128, g.row_off ^ (uint32_t)((rg & 1) << 4), wl + i * 1024);
+            else dma16(w.p0 + (n_tile + rg * 8) * k + b * 256 + kh * 128, g.row_off ^ (uint32_t)((rg & 1) << 4), wl + i * 1024);
         }
     } else {
 #pragma unroll
         for (int rg = 0; rg < 4; rg++) {
-            if (ONCE) dma16_once(w.p0 + (n_tile + rg * 8) * (k >> 1) + b * 128, g.w4_off, wl + rg * 1024);
-            else dma16(w.p0 + (n_tile + rg * 8) * (k >> 1) + b * 128, g.w4_off, wl + rg * 1024);
+            if (ONCE) dma16_once(w.p0 + (n_tile + rg * 8) * (k >> 1) + b * 128, g.w4_off ^ (uint32_t)((rg & 1) << 4), wl + rg * 1024);
+            else dma16(w.p0 + (n_tile + rg * 8) * (k >> 1) + b * 128, g.w4_off ^ (uint32_t)((rg & 1) << 4), wl + rg * 1024);
         }
+    }
+}
+
+// Weight operands of the eight blocks of a K step out of the wave's buffer (which is then free for the next step).
+template <int DT> __device__ __forceinline__ void step_weights(const uint8_t *wl, const LaneGeo &g, int h, v4i (&bw)[8]) {
+    if (DT == CQ_DTYPE_Q8_0) {
+#pragma unroll
+        for (int s = 0; s < 8; s++) bw[s] = *(const v4i *)(wl + (s >> 2) * 4096 + g.col[s & 3]);
+    } else {
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            // block s: 16 bytes, low nibbles = elements 0..15 (h = 0), high nibbles = elements 16..31; as 16 * (q - 8), the
+            // nibble in the upper half of its byte: two instructions a word (the block scale takes the 1/16)
+            const v4i q = *(const v4i *)(wl + g.col4[s]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) bw[s][i] = (int)((((uint32_t)q[i] << (4 - 4 * h)) & 0xF0F0F0F0u) ^ 0x80808080u);
+        }
+    }
+}
+
+// One K step: the eight blocks of `bw` against the MT tiles of the stage `cur`.  `dcur`: the lane's weight row's eight f16 block
+// scales; nv: blocks of the step that exist (SHORT).
+template <int DT, int MT, bool DUMP, bool SHORT>
+__device__ __forceinline__ void step_mac(const uint8_t *cur, const LaneGeo &g, const v4i (&bw)[8], const u32x4_a4 dcur, int nv, int h, int col,
+                                         v16f (&out)[MT], const cq_weight &w, int64_t m0, int64_t m, int64_t n, int64_t b, cq_mfma_dump dump) {
+    typedef Tile<DT, MT> T;
+    // scale operand of block s: dw = b1 + b2 (bf16 pieces, exact: an f16 has 11 significant bits); lanes
+    // 0..31 carry b1 in K-slots 0 and 1, lanes 32..63 carry b2 in K-slots 8 and 9, the other slots zero
+    // A last step of fewer than eight blocks: what follows the rows in memory (other rows, other planes) was copied
+    // with them, and both scales of the blocks that do not exist are zero.
+    const uint32_t dwords[4] = {dcur.x, dcur.y, dcur.z, dcur.w};
+    v8bf dw[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        float f = !SHORT || s < nv ? cq_h2f((uint16_t)((dwords[s >> 1] >> (16 * (s & 1))) & 0xffffu)) : 0.0f;
+        if (DT == CQ_DTYPE_Q4_0) f *= 0.0625f;   // (exact: step_weights)
+        const uint32_t fb = __float_as_uint(f);
+        const float b2 = f - __uint_as_float(fb & 0xffff0000u);
+        const uint32_t piece = h == 0 ? fb >> 16 : __float_as_uint(b2) >> 16;
+        const v4u pk = {piece | (piece << 16), 0u, 0u, 0u};
+        dw[s] = __builtin_bit_cast(v8bf, pk);
+    }
+
+    // steps q = (tile t, block s): the two MFMAs of step q, and in their shadow the scaling of step q-1
+    auto afrag = [&](int q) -> v4i {
+        const int t = q >> 3, s = q & 7;
+        return *(const v4i *)(cur + g.col[s & 3] + (t * 2 + (s >> 2)) * 4096);
+    };
+    // activation scale of (row l%32 of tile t, block s): read two steps ahead, and only turned into
+    // the MFMA operand (two bf16 pieces) in the step that uses it, so that no step
+    // waits for the read it has just issued
+    auto d8raw = [&](int q) -> float {
+        const int t = q >> 3, s = q & 7;
+        const float v = *(const float *)(cur + T::oD8 + t * 1024 + s * 128 + col * 4);
+        return !SHORT || s < nv ? v : 0.0f;
+    };
+    auto d8frag = [&](float v) -> v8bf {
+        // v = a1 + a2, the leading eight bits and the other three of an f16 value (exact); K-slots 0, 1 of both lane halves
+        const uint32_t vb = __float_as_uint(v);
+        const float r1 = v - __uint_as_float(vb & 0xffff0000u);
+        const v4u pk = {__builtin_amdgcn_perm(__float_as_uint(r1), vb, 0x07060302u), 0u, 0u, 0u};
+        return __builtin_bit_cast(v8bf, pk);
+    };
+    v16i acc[2];
+    v16f sc[2];
+    v4i av[3];
+    float dv[3];
+    av[0] = afrag(0); av[1] = afrag(1);
+    dv[0] = d8raw(0); dv[1] = d8raw(1);
+    const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const v16f zerof = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q <= MT * 8; q++) {
+        if (q + 2 < MT * 8) { av[(q + 2) % 3] = afrag(q + 2); dv[(q + 2) % 3] = d8raw(q + 2); }
+        if (q < MT * 8) {
+            acc[q & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[q % 3], bw[q & 7], zero, 0, 0, 0);
+            sc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(d8frag(dv[q % 3]), dw[q & 7], zerof, 0, 0, 0);
+        }
+        // keeps the MFMAs in front of the scaling below: left alone, the scheduler sinks them to the end
+        // of the step, and the next step then starts by waiting for their results
+        __builtin_amdgcn_sched_barrier(0);
+        if (q > 0) {
+            const int p = (q - 1) & 1, t = (q - 1) >> 3;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                if (DUMP) {   // (whole K steps only)
+                    const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+                    if (row < m) dump.i[(row * w.n + n) * (w.k >> 5) + b * 8 + ((q - 1) & 7)] = DT == CQ_DTYPE_Q4_0 ? acc[p][i] >> 4 : acc[p][i];
+                } else {
+                    out[t][i] = __builtin_fmaf((float)acc[p][i], sc[p][i], out[t][i]);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -173,100 +270,14 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
         const bool more = b + 1 < b1;
         if (more) stage_acts<DT, MT, ANYROW>(nxt, a, g, k, m0, b + 1, wave);
         if (n_ok) {
-            // weight operands of the eight blocks into registers, then the buffer is free for the next step
             v4i bw[8];
-            if (DT == CQ_DTYPE_Q8_0) {
-#pragma unroll
-                for (int s = 0; s < 8; s++) bw[s] = *(const v4i *)(wl + (s >> 2) * 4096 + g.col[s & 3]);
-            } else {
-#pragma unroll
-                for (int s = 0; s < 8; s++) {
-                    // block s: 16 bytes, low nibbles = elements 0..15 (h = 0), high nibbles = elements 16..31
-                    const v4i q = *(const v4i *)(wl + g.col4[s]);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const uint32_t x = ((uint32_t)q[i] >> (4 * h)) & 0x0F0F0F0Fu;
-                        bw[s][i] = (int)((x + 0x78787878u) ^ 0x80808080u);   // every byte minus 8, no carries between bytes
-                    }
-                }
-            }
+            step_weights<DT>(wl, g, h, bw);
             const u32x4_a4 dcur = dnext;
             if (more) {
                 stage_weights<DT, ONCE>(wl, w, g, n_tile, b + 1);
                 dnext = *(const u32x4_a4 *)(dplane + nc * (k >> 5) + (b + 1) * 8);
             }
-            // scale operand of block s: dw = b1 + b2 (bf16 pieces, exact: an f16 has 11 significant bits); lanes
-            // 0..31 carry b1 in K-slots 0..2, lanes 32..63 carry b2 in K-slots 8..10, the other slots zero
-            // A last step of fewer than eight blocks: what follows the rows in memory (other rows, other planes) was copied
-            // with them, and both scales of the blocks that do not exist are zero.
-            const int nv = (int)((k >> 5) - b * 8);
-            const uint32_t dwords[4] = {dcur.x, dcur.y, dcur.z, dcur.w};
-            v8bf dw[8];
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const float f = !SHORT || s < nv ? cq_h2f((uint16_t)((dwords[s >> 1] >> (16 * (s & 1))) & 0xffffu)) : 0.0f;
-                const uint32_t fb = __float_as_uint(f);
-                const float b2 = f - __uint_as_float(fb & 0xffff0000u);
-                const uint32_t piece = h == 0 ? fb >> 16 : __float_as_uint(b2) >> 16;
-                const v4u pk = {piece | (piece << 16), piece, 0u, 0u};
-                dw[s] = __builtin_bit_cast(v8bf, pk);
-            }
-
-            // steps q = (tile t, block s): the two MFMAs of step q, and in their shadow the scaling of step q-1
-            auto afrag = [&](int q) -> v4i {
-                const int t = q >> 3, s = q & 7;
-                return *(const v4i *)(cur + g.col[s & 3] + (t * 2 + (s >> 2)) * 4096);
-            };
-            // activation scale of (row l%32 of tile t, block s): read two steps ahead, and only turned into
-            // the MFMA operand (three bf16 pieces) in the step that uses it, so that no step
-            // waits for the read it has just issued
-            auto d8raw = [&](int q) -> float {
-                const int t = q >> 3, s = q & 7;
-                const float v = *(const float *)(cur + T::oD8 + t * 1024 + s * 128 + col * 4);
-                return !SHORT || s < nv ? v : 0.0f;
-            };
-            auto d8frag = [&](float v) -> v8bf {
-                // v = a1 + a2 + a3, each the leading eight bits of what the pieces before it leave (exact);
-                // K-slots 0..2 of both lane halves
-                const uint32_t vb = __float_as_uint(v);
-                const float r1 = v - __uint_as_float(vb & 0xffff0000u);
-                const uint32_t rb = __float_as_uint(r1);
-                const float a3 = r1 - __uint_as_float(rb & 0xffff0000u);
-                const v4u pk = {__builtin_amdgcn_perm(rb, vb, 0x07060302u), __float_as_uint(a3) >> 16, 0u, 0u};
-                return __builtin_bit_cast(v8bf, pk);
-            };
-            v16i acc[2];
-            v16f sc[2];
-            v4i av[3];
-            float dv[3];
-            av[0] = afrag(0); av[1] = afrag(1);
-            dv[0] = d8raw(0); dv[1] = d8raw(1);
-            const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            const v16f zerof = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int q = 0; q <= MT * 8; q++) {
-                if (q + 2 < MT * 8) { av[(q + 2) % 3] = afrag(q + 2); dv[(q + 2) % 3] = d8raw(q + 2); }
-                if (q < MT * 8) {
-                    acc[q & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[q % 3], bw[q & 7], zero, 0, 0, 0);
-                    sc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(d8frag(dv[q % 3]), dw[q & 7], zerof, 0, 0, 0);
-                }
-                // keeps the MFMAs in front of the scaling below: left alone, the scheduler sinks them to the end
-                // of the step, and the next step then starts by waiting for their results
-                __builtin_amdgcn_sched_barrier(0);
-                if (q > 0) {
-                    const int p = (q - 1) & 1, t = (q - 1) >> 3;
-#pragma unroll
-                    for (int i = 0; i < 16; i++) {
-                        if (DUMP) {   // (whole K steps only)
-                            const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                            if (row < m) dump.i[(row * w.n + n) * (k >> 5) + b * 8 + ((q - 1) & 7)] = acc[p][i];
-                        } else {
-                            out[t][i] = __builtin_fmaf((float)acc[p][i], sc[p][i], out[t][i]);
-                        }
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            step_mac<DT, MT, DUMP, SHORT>(cur, g, bw, dcur, (int)((k >> 5) - b * 8), h, col, out, w, m0, m, n, b, dump);
         }
         __builtin_amdgcn_s_waitcnt(0);   // the next stage and the wave's next weights have landed in LDS
         __syncthreads();
@@ -291,6 +302,180 @@ template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, int ksplit,
                                                           cq_mfma_dump dump) {
     gemm32_body<DT, MT, DUMP, ONCE, SHORT>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, y, ksplit, dump);
+}
+
+// Few column tiles: K halved inside the workgroup (as gemm_kh_kernel of gemm.hip).  A workgroup covers 128 weight rows x 32*MT
+// activation rows; waves 0..3 take the first half of the K steps, waves 4..7 the second half for the same weight rows, and
+// the partial tiles meet in LDS, first half + second half: twice the workgroups at the same tile height, no atomic additions.
+// Bound, as above, by vector issue (one conversion and one fma per element and block, two thirds of the instructions).  Whole calls, us, before
+// -> here: Q4_0 32003 x 3200 at 77 rows (251 workgroups of 96 rows for 252 of 64, the upper ones nearly empty) 54.8 -> 42.1,
+// 29731 x 4864 at 90 rows 69.6 -> 51.9, Q8_0 4096 x 4096 at 512 rows 40.7 -> 36.1, 8192 x 2048 at 60 rows 16.1 -> 14.4.
+template <int DT, int MT> struct TileKH {
+    typedef Tile<DT, MT> T;
+    static constexpr int oWgt = 4 * T::kStage;   // two stages of one part per half
+    static constexpr int kTotal = oWgt + kWaves * T::kWgtWave;
+    static_assert(kTotal <= 160 * 1024 && MT * 4096 * (kWaves / 2) <= oWgt, "the stages fit the LDS, the partial tiles the stages");
+};
+// Row tiles that gemm32_kh_kernel's stages leave room for beside the weights (Q8_0: 8 KiB a wave).
+template <int DT> constexpr int kh_tallest() { return DT == CQ_DTYPE_Q4_0 ? 3 : 2; }
+template <int DT, int MT, bool SHORT>
+__global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y) {
+    typedef Tile<DT, MT> T;
+    typedef TileKH<DT, MT> TK;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int colw = wave & 3, half = wave >> 2, h = lane >> 5, col = lane & 31;
+    const int64_t k = w.k, m0 = (int64_t)blockIdx.y * (MT * 32);
+    const int ks = (int)((k + 255) >> 8), nh = (ks + 1) / 2;
+    const int64_t n_own = ((int64_t)blockIdx.x * (kWaves / 2) + colw) * 32;
+    const bool n_ok = n_own < w.n;
+    const int64_t n_tile = n_own + 32 <= w.n ? n_own : w.n - 32, n = n_tile + col;
+    const int first = half ? nh : 0, count = half ? ks - nh : nh;
+    const LaneGeo g = lane_geo<false>(lane, k, a.m_stride);
+    uint8_t *__restrict__ wl = smem + TK::oWgt + wave * T::kWgtWave;
+    const uint16_t *dplane = (const uint16_t *)w.p1 + (n_ok ? n : 0) * (k >> 5);
+
+    v16f out[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) out[t][i] = 0.0f;
+
+    stage_acts<DT, MT, false>(smem, a, g, k, m0, 0, wave);
+    if (ks > nh) stage_acts<DT, MT, false>(smem + T::kStage, a, g, k, m0, nh, wave);
+    u32x4_a4 dnext = {};
+    if (n_ok && count > 0) {
+        stage_weights<DT, false>(wl, w, g, n_tile, first);
+        dnext = *(const u32x4_a4 *)(dplane + first * 8);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    for (int it = 0; it < nh; it++) {
+        const uint8_t *__restrict__ cur = smem + (2 * (it & 1) + half) * T::kStage;
+        uint8_t *__restrict__ nxt = smem + 2 * ((it & 1) ^ 1) * T::kStage;
+        if (it + 1 < nh) stage_acts<DT, MT, false>(nxt, a, g, k, m0, it + 1, wave);
+        if (nh + it + 1 < ks) stage_acts<DT, MT, false>(nxt + T::kStage, a, g, k, m0, nh + it + 1, wave);
+        if (n_ok && it < count) {
+            const int b = first + it;
+            v4i bw[8];
+            step_weights<DT>(wl, g, h, bw);
+            const u32x4_a4 dcur = dnext;
+            if (it + 1 < count) {
+                stage_weights<DT, false>(wl, w, g, n_tile, b + 1);
+                dnext = *(const u32x4_a4 *)(dplane + (b + 1) * 8);
+            }
+            step_mac<DT, MT, false, SHORT>(cur, g, bw, dcur, (int)(k >> 5) - b * 8, h, col, out, w, m0, m, n, b, cq_mfma_dump{nullptr, nullptr, 0});
+        }
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+    }
+    // (the stages are free: every wave is past its last read)
+    float *part = (float *)smem + (size_t)colw * (MT * 16 * 64);
+    if (half == 1) {
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) part[(t * 16 + i) * 64 + lane] = out[t][i];
+    }
+    __syncthreads();
+    if (half == 0 && n_ok) {
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+                if (row < m && n >= n_own) y[row * w.n + n] = out[t][i] + part[(t * 16 + i) * 64 + lane];
+            }
+        }
+    }
+}
+
+// Up to 32 activation rows: every wave by itself.  A workgroup covers 32*CW weight rows, its waves share the K steps: wave p * CW + c
+// takes steps p, p + KS, ... (KS = 8 / CW) of column tile c into a buffer of its own, activations included, so that no wave
+// waits for another before the end, where the KS partial tiles of each column tile are added in order.  No atomic additions, and
+// nothing for the quantizer to clear.  Bound by the weights' way in: a step's weights are requested while the one before is
+// contracted, its activations behind it (there is no LDS for two sets).  Whole calls, us, K split over workgroups -> here: Q4_0 14336 x 4096 at
+// 21 rows 18.2 -> 14.8, Q8_0 20.9 -> 19.5; more partial tiles than that cost more than they give (Q8_0 8192 x 8192 as 256
+// workgroups of one column tile 19.8 -> 24.0).
+template <int DT> struct Few {
+    typedef Tile<DT, 1> T;
+    static constexpr int kWave = T::kStage + T::kWgtWave;
+    static constexpr int kTotal = kWaves * kWave;
+};
+template <int DT, int CW, bool ONCE, bool SHORT>
+__global__ void __launch_bounds__(kThreads) gemm32_few_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y) {
+    typedef Tile<DT, 1> T;
+    constexpr int KS = kWaves / CW;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int colw = wave % CW, part = wave / CW, h = lane >> 5, col = lane & 31;
+    const int64_t k = w.k;
+    const int ks = (int)((k + 255) >> 8), groups = (int)((m + 7) / 8);
+    const int64_t n_own = ((int64_t)blockIdx.x * CW + colw) * 32;
+    const bool n_ok = n_own < w.n;
+    const int64_t n_tile = n_own + 32 <= w.n ? n_own : w.n - 32, n = n_tile + col;
+    const LaneGeo g = lane_geo<false>(lane, k, a.m_stride);
+    uint8_t *__restrict__ act = smem + wave * Few<DT>::kWave;
+    uint8_t *__restrict__ wl = act + T::kStage;
+    const uint16_t *dplane = (const uint16_t *)w.p1 + (n_ok ? n : 0) * (k >> 5);
+
+    v16f out[1];
+#pragma unroll
+    for (int i = 0; i < 16; i++) out[0][i] = 0.0f;
+    auto copy_acts = [&](int b) {
+#pragma unroll
+        for (int idx = 0; idx < 8; idx++) {
+            const int rg = idx & 3, kh = idx >> 2;
+            if (rg < groups) dma16(a.qs + (int64_t)(rg * 8) * k + b * 256 + kh * 128, g.row_off ^ (uint32_t)((rg & 1) << 4), act + idx * 1024);
+        }
+        dma16(a.dT + (int64_t)b * 8 * a.m_stride, g.d8_off, act + T::oD8);
+    };
+    if (n_ok && part < ks) {
+        u32x4_a4 dnext = *(const u32x4_a4 *)(dplane + part * 8);
+        stage_weights<DT, ONCE>(wl, w, g, n_tile, part);
+        copy_acts(part);
+#pragma nounroll
+        for (int b = part; b < ks; b += KS) {
+            __builtin_amdgcn_s_waitcnt(0);   // the step's copies have landed
+            const uint8_t *__restrict__ cur = act;
+            v4i bw[8];
+            step_weights<DT>(wl, g, h, bw);
+            const u32x4_a4 dcur = dnext;
+            if (b + KS < ks) {
+                __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the reads above are done with the buffer
+                dnext = *(const u32x4_a4 *)(dplane + (b + KS) * 8);
+                stage_weights<DT, ONCE>(wl, w, g, n_tile, b + KS);
+            }
+            step_mac<DT, 1, false, SHORT>(cur, g, bw, dcur, (int)(k >> 5) - b * 8, h, col, out, w, 0, m, n, b, cq_mfma_dump{nullptr, nullptr, 0});
+#pragma unroll
+            for (int i = 0; i < 16; i++) asm volatile("" : "+v"(out[0][i]));   // (keeps the arithmetic in front of the branch: it would sink behind it, with all it holds)
+            if (b + KS < ks) {
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                copy_acts(b + KS);
+            }
+        }
+    }
+    if constexpr (KS > 1) {
+        float *mine = (float *)act;
+#pragma unroll
+        for (int i = 0; i < 16; i++) mine[i * 64 + lane] = out[0][i];
+        __syncthreads();
+    }
+    // wave p * CW + c adds and stores registers 16 / KS * p .. of column tile c
+    if (!n_ok || n < n_own) return;
+#pragma unroll
+    for (int j = 0; j < 16 / KS; j++) {
+        const int i = part * (16 / KS) + j;
+        float v = KS > 1 ? 0.0f : out[0][j];
+        if constexpr (KS > 1) {
+#pragma unroll
+            for (int p = 0; p < KS; p++) v += *(const float *)(smem + (p * CW + colw) * Few<DT>::kWave + (i * 64 + lane) * 4);
+        }
+        const int64_t row = (i >> 2) * 8 + h * 4 + (i & 3);
+        if (row < m) y[row * w.n + n] = v;
+    }
 }
 
 // 128-row tiles in whole rounds of workgroups, what is left of them in tiles of 32 * TAIL rows (as gemm_tail_kernel of
@@ -322,9 +507,15 @@ __global__ void __launch_bounds__(kThreads) gemm32_grouped_kernel(cq_group_args 
 // measurements (Q8_0, 256 CUs; unit 1/16 us): a workgroup spends 10 units per 256-element K step on its
 // weights and 23 per 32-row tile on it, 24 on starting and finishing; workgroups run one per CU, in rounds;
 // a split launch adds every part to the output atomically, which moves about 1.1 TB/s.
+// The launches that split K inside the workgroup are priced beside them (half the steps at 11 + 22 units a row tile, 40 for start,
+// end and meeting; up to 32 rows 30 units a step of a wave and 29), taken where one round of workgroups does it and the sum is at least 5 %
+// lower.  Against a sweep of both on 1857 cases (512..32000 weight rows, K 512..14336, 17..2048 rows) the choice is 0.5 % off the
+// better one on average (the tile launches alone 8 %), 5.5 % faster than they are and 7 % slower at worst (Q8_0 512 x 1024 at 512 rows, 0.8 us).
 struct Plan {
     int mt, ksplit;
     int tail = 0;   // 1, 2: gemm32_tail_kernel, the last round's tiles in heights of 32 * tail rows
+    int kh = 0;     // 1: gemm32_kh_kernel
+    int few = 0;    // 1, 2, 4, 8: gemm32_few_kernel with that many column tiles a workgroup
 };
 Plan pick_plan(const cq_weight *w, int64_t m) {
     const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks_total = (w->k + 255) >> 8, cus = cq_num_cus();
@@ -357,6 +548,27 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
             }
         }
     }
+    const double limit = 0.95 * best_cost;
+    best_cost = limit;
+    for (int mt = w->dtype == CQ_DTYPE_Q4_0 ? kh_tallest<CQ_DTYPE_Q4_0>() : kh_tallest<CQ_DTYPE_Q8_0>(); mt >= 1; mt--) {
+        if (mt > 1 && m <= 32 * (mt - 1)) continue;   // a row tile less holds all rows
+        if (mt == 3 && (m + 95) / 96 * 96 > (m + 127) / 128 * 128) continue;   // (the workspace's rows are padded to 128)
+        if ((w->n + 127) / 128 * ((m + mt * 32 - 1) / (mt * 32)) > cus) continue;
+        const double cost = (double)((ks_total + 1) / 2) * (11.0 + 22.0 * mt) + 40.0;
+        if (cost < best_cost) {
+            best = Plan{mt, 1, 0, 1};
+            best_cost = cost;
+        }
+    }
+    for (int cw = 8; cw >= 1 && m <= 32; cw >>= 1) {
+        const int64_t groups = (w->n + 32 * cw - 1) / (32 * cw), parts = kWaves / cw;
+        if (groups > (cw == 1 && w->dtype == CQ_DTYPE_Q8_0 ? cus / 2 : cus)) continue;
+        const double cost = (double)((ks_total + parts - 1) / parts) * 30.0 + 29.0;
+        if (cost < best_cost) {
+            best = Plan{1, 1, 0, 0, cw};
+            best_cost = cost;
+        }
+    }
     return best;
 }
 
@@ -378,6 +590,9 @@ hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, c
               (uint32_t)gx, (uint32_t)whole, d);
     return hipGetLastError();
 }
+// A single row tile over that many bytes of weights and more: the copies marked non-temporal (measured at 17 and 32 rows:
+// 3-7 % faster from there on, 3-5 % slower below).
+constexpr int64_t kOnceBytes = 40000000;
 template <int DT, int MT, bool DUMP>
 hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int ksplit, bool y_cleared, cq_mfma_dump d,
                      hipStream_t s) {
@@ -390,10 +605,8 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
         }
         const bool whole = w->k % 256 == 0;
         if constexpr (MT == 1) {
-            // a single row tile over 40 MB of weights and more: the copies marked non-temporal (measured at 17 and 32 rows:
-            // 3-7 % faster from there on, 3-5 % slower below)
             const int64_t plane = DT == CQ_DTYPE_Q8_0 ? w->n * w->k : w->n * w->k / 2;
-            if (m <= 32 && plane >= 40000000)
+            if (m <= 32 && plane >= kOnceBytes)
                 return whole ? launch_inst<DT, 1, false, true, false>(w, a, m, y, ksplit, d, s)
                              : launch_inst<DT, 1, false, true, true>(w, a, m, y, ksplit, d, s);
         }
@@ -402,9 +615,49 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
     }
 }
 
+template <int DT, int MT> hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+    if (a.m_stride < (m + 32 * MT - 1) / (32 * MT) * (32 * MT)) return hipErrorInvalidValue;   // rows the last tile reads
+    auto go = [&](auto sh) {
+        constexpr bool SHORT = decltype(sh)::value;
+        const size_t lds = TileKH<DT, MT>::kTotal;
+        if (hipError_t e = cq_ensure_lds<gemm32_kh_kernel<DT, MT, SHORT>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm32_kh_kernel<DT, MT, SHORT>), dim3((unsigned)((w->n + 127) / 128), (unsigned)((m + MT * 32 - 1) / (MT * 32))), kThreads, lds, s, *w, a, m, y);
+        return hipGetLastError();
+    };
+    return w->k % 256 == 0 ? go(std::false_type{}) : go(std::true_type{});
+}
+template <int DT, int CW, bool ONCE> hipError_t launch_few(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+    auto go = [&](auto sh) {
+        constexpr bool SHORT = decltype(sh)::value;
+        const size_t lds = Few<DT>::kTotal;
+        if (hipError_t e = cq_ensure_lds<gemm32_few_kernel<DT, CW, ONCE, SHORT>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm32_few_kernel<DT, CW, ONCE, SHORT>), (unsigned)((w->n + 32 * CW - 1) / (32 * CW)), kThreads, lds, s, *w, a, m, y);
+        return hipGetLastError();
+    };
+    return w->k % 256 == 0 ? go(std::false_type{}) : go(std::true_type{});
+}
+
+template <int DT> hipError_t launch_few_cw(const cq_weight *w, cq_act_view a, int64_t m, float *y, int cw, hipStream_t s) {
+    const bool once = (DT == CQ_DTYPE_Q8_0 ? w->n * w->k : w->n * w->k / 2) >= kOnceBytes;
+    switch (cw) {
+    case 1: return once ? launch_few<DT, 1, true>(w, a, m, y, s) : launch_few<DT, 1, false>(w, a, m, y, s);
+    case 2: return once ? launch_few<DT, 2, true>(w, a, m, y, s) : launch_few<DT, 2, false>(w, a, m, y, s);
+    case 4: return once ? launch_few<DT, 4, true>(w, a, m, y, s) : launch_few<DT, 4, false>(w, a, m, y, s);
+    default: return once ? launch_few<DT, 8, true>(w, a, m, y, s) : launch_few<DT, 8, false>(w, a, m, y, s);
+    }
+}
+
 template <int DT, bool DUMP>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool y_cleared, cq_mfma_dump d, hipStream_t s) {
     const Plan p = pick_plan(w, m);
+    if constexpr (!DUMP) {
+        if (p.few) return launch_few_cw<DT>(w, a, m, y, p.few, s);
+        if (p.kh) {
+            if constexpr (kh_tallest<DT>() == 3)
+                if (p.mt == 3) return launch_kh<DT, 3>(w, a, m, y, s);
+            return p.mt == 2 ? launch_kh<DT, 2>(w, a, m, y, s) : launch_kh<DT, 1>(w, a, m, y, s);
+        }
+    }
     if (DUMP || w->k % 256 == 0) {   // (whole K steps are all that is dumped)
         if (p.tail == 2) return launch_tail<DT, 2, DUMP, false>(w, a, m, y, d, s);
         if (p.tail == 1) return launch_tail<DT, 1, DUMP, false>(w, a, m, y, d, s);
