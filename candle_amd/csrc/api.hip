@@ -582,7 +582,9 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     cq_act_view v;
     act_ws_layout(act, m, w->k, (uint8_t *)ws, &v);
     bool y_cleared = false;
-    if (!(flags & CQ_FLAG_REUSE_ACT)) {
+    // a few more rows of a small weight: quantized by the waves of the split-K kernel, which leaves them in the workspace as well
+    const bool direct = flags == 0 && pre.kind == CQ_PRE_NONE && !in_place && path == kSkinny && cq_skinny_direct_takes(w, act, m);
+    if (!(flags & CQ_FLAG_REUSE_ACT) && !direct) {
         cq_clear clear = cq_no_clear();
         const bool splits = path == kGemm32 ? cq_gemm32_splits_k(w, m) : path == kGemm ? cq_gemm_splits_k(w, m) : false;
         if (splits && clear_in_quantizer_ok(y_dev, m * w->n, x_dev, m * w->k, pre)) {
@@ -592,7 +594,7 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
         CQ_HIP_CHECK(cq_launch_quantize_act_ws(act, x_dev, nullptr, m, w->k, pre, v, clear, s));
     }
     switch (path) {
-        case kSkinny: CQ_HIP_CHECK(cq_launch_skinny(w, v, act, m, y_dev, s)); break;
+        case kSkinny: CQ_HIP_CHECK(direct ? cq_launch_skinny_direct(w, v, x_dev, m, y_dev, s) : cq_launch_skinny(w, v, act, m, y_dev, s)); break;
         case kGemm32: CQ_HIP_CHECK(cq_launch_gemm32(w, v, act, m, y_dev, y_cleared, s)); break;
         case kGemm: CQ_HIP_CHECK(cq_launch_gemm(w, v, act, m, y_dev, y_cleared, s)); break;
         case kMatvec: CQ_HIP_CHECK(cq_launch_matvec(w, v, act, m, y_dev, s)); break;

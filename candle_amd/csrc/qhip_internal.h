@@ -210,6 +210,9 @@ bool cq_gemm32_grouped_splits_k(const cq_weight *const *experts, int n_experts, 
 bool cq_skinny_takes(const cq_weight *w, int act_dtype);
 bool cq_skinny_supported(const cq_weight *w, int act_dtype);
 hipError_t cq_launch_skinny(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, hipStream_t s);
+// up to eight rows of a small weight in one launch that quantizes them itself (and leaves them in the workspace)
+bool cq_skinny_direct_takes(const cq_weight *w, int act_dtype, int64_t m);
+hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s);
 // two or three weights (same type and row length) on the same rows in one launch, up to 16 rows, where that is the faster way
 bool cq_skinny_shared_takes(const cq_weight *const *ws, int count, int64_t m, int act_dtype);
 hipError_t cq_launch_skinny_shared(const cq_weight *const *ws, int count, cq_act_view a, int64_t m, float *const *ys, hipStream_t s);

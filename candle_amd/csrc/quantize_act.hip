@@ -14,7 +14,7 @@
 // candle-core/src/op.rs:607-609) is elementwise and goes into the kernels above; rms_norm
 // (candle-nn/src/ops.rs:482-495: x / sqrt(mean(x^2) + eps) * alpha) needs the whole row first and
 // has a kernel of its own with one workgroup per row.
-#include "qhip_internal.h"
+#include "quantize_blocks.h"
 
 #include <type_traits>
 
@@ -53,27 +53,15 @@ __device__ __forceinline__ int64_t divide(int64_t a, int64_t b) {
     return ((uint64_t)a | (uint64_t)b) >> 32 ? a / b : (int64_t)((uint32_t)a / (uint32_t)b);
 }
 
-__device__ __forceinline__ int8_t round_to_i8(float v) { return cq_as_i8(roundf(v)); }
-
 // Q8_0 / Q8_1: eight 32-element blocks per wave, 8 lanes per block.  `f` = the lane's four values
 // at element e0 of `row` (zeros in a lane past the end of the row); called by all 64 lanes.
 template <bool AOS, bool Q8_1>
 __device__ __forceinline__ void q8_0_chunk(const float4 f, bool active, int64_t row, int64_t e0, int64_t k, const Sink &out) {
-    float amax = fmaxf(fmaxf(fmaxf(fmaxf(0.0f, fabsf(f.x)), fabsf(f.y)), fabsf(f.z)), fabsf(f.w));
-    amax = fmaxf(amax, dpp_f<kQuadSwap1>(amax));
-    amax = fmaxf(amax, dpp_f<kQuadSwap2>(amax));
-    amax = fmaxf(amax, dpp_f<kHalfMirror>(amax));  // quads hold one value each: the mirror pairs them
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    const int8_t q0 = round_to_i8(f.x * id), q1 = round_to_i8(f.y * id), q2 = round_to_i8(f.z * id),
-                 q3 = round_to_i8(f.w * id);
-    int sum = (int)q0 + (int)q1 + (int)q2 + (int)q3;
-    sum += dpp_i<kQuadSwap1>(sum);
-    sum += dpp_i<kQuadSwap2>(sum);
-    sum += dpp_i<kHalfMirror>(sum);
+    uint32_t packed;
+    float d;
+    int sum;
+    cq_q8_0_of_eight(f, packed, d, sum);
     if (!active) return;
-    const uint32_t packed = (uint32_t)(uint8_t)q0 | ((uint32_t)(uint8_t)q1 << 8) | ((uint32_t)(uint8_t)q2 << 16) |
-                            ((uint32_t)(uint8_t)q3 << 24);
     const uint16_t dh = cq_f2h(d);
     const int64_t blk = row * (k / 32) + e0 / 32;
     const int within = (int)(e0 & 31);
@@ -191,7 +179,6 @@ __device__ __forceinline__ void q8k_chunk(const float4 f, int64_t row, int64_t b
 // A wave a block (the kernel below) spends about 250 vector instructions on it and is bound by them; here memory is.  Kernel
 // alone, us, with a wave a block -> here: 512 x 4096 6.0 -> 3.3, 1024 x 4096 9.2 -> 5.7, 4096 x 4096 22.3 -> 15.4 (5.5 TB/s), with
 // silu 32.9 -> 26.5, 4096 x 14336 123 -> 105.
-// The signed extremes replace the search for the first largest |x|: only where both signs reach it does the position decide.
 template <bool AOS, bool SILU>
 __global__ void __launch_bounds__(256) quantize_q8k_quad_kernel(const float *__restrict__ x, const int32_t *__restrict__ row_ids,
                                                                 uint32_t blocks, uint32_t kb, const float *__restrict__ x2, Sink out) {
@@ -217,59 +204,13 @@ __global__ void __launch_bounds__(256) quantize_q8k_quad_kernel(const float *__r
 #pragma unroll
         for (int i = 0; i < 4; i++) f[i] = silu_mul4(f[i], g[i]);
     }
-    float hi = 0.0f, lo = 0.0f;   // (NaN elements fall out of both)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        hi = fmaxf(fmaxf(fmaxf(fmaxf(hi, f[i].x), f[i].y), f[i].z), f[i].w);
-        lo = fminf(fminf(fminf(fminf(lo, f[i].x), f[i].y), f[i].z), f[i].w);
-    }
-    hi = fmaxf(hi, dpp_f<kQuadSwap1>(hi));
-    lo = fminf(lo, dpp_f<kQuadSwap1>(lo));
-    hi = fmaxf(hi, dpp_f<kQuadSwap2>(hi));
-    lo = fminf(lo, dpp_f<kQuadSwap2>(lo));
-    hi = fmaxf(hi, dpp_f<kHalfMirror>(hi));
-    lo = fminf(lo, dpp_f<kHalfMirror>(lo));
-    hi = fmaxf(hi, dpp_f<kRowMirror>(hi));
-    lo = fminf(lo, dpp_f<kRowMirror>(lo));
-    const float amax = fmaxf(hi, -lo);
-    float max = hi > -lo ? hi : lo;
-    if (__any(hi == -lo && amax != 0.0f)) {   // both signs: the sign of the first of them
-        int idx = 0x7fffffff;
-#pragma unroll
-        for (int i = 3; i >= 0; i--) {
-            const float v[4] = {f[i].x, f[i].y, f[i].z, f[i].w};
-#pragma unroll
-            for (int c = 3; c >= 0; c--)
-                if (fabsf(v[c]) == amax) idx = 2 * (64 * i + 4 * (int)l + c) + (v[c] < 0.0f ? 1 : 0);
-        }
-        idx = min(idx, dpp_i<kQuadSwap1>(idx));
-        idx = min(idx, dpp_i<kQuadSwap2>(idx));
-        idx = min(idx, dpp_i<kHalfMirror>(idx));
-        idx = min(idx, dpp_i<kRowMirror>(idx));
-        if (hi == -lo) max = idx & 1 ? lo : hi;
-    }
-    const bool any = amax != 0.0f;
-    const float iscale = -128.0f / max;
-    const float d = any ? 1.0f / iscale : 0.0f;
     uint32_t packed[4];
-    int sum[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const float v[4] = {f[i].x, f[i].y, f[i].z, f[i].w};
-        uint32_t q[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++)   // min(127, round(t)) as i8: clamped first, NaN to 127; |t| is at most 128 and rounding then
-            q[c] = (uint32_t)cq_round_away_i32(fmaxf(fminf(iscale * v[c], 127.0f), -128.0f));
-        const uint32_t p01 = __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u), p23 = __builtin_amdgcn_perm(q[3], q[2], 0x04000c0cu);
-        packed[i] = any ? p01 | p23 : 0u;
-        sum[i] = __builtin_amdgcn_sdot4((int)packed[i], 0x01010101, 0, false);
-        sum[i] += dpp_i<kQuadSwap1>(sum[i]);
-        sum[i] += dpp_i<kQuadSwap2>(sum[i]);   // bsums[4i + l / 4]
-    }
+    float d;
+    int mine;
+    cq_q8k_of_sixteen(f, (int)l, packed, d, mine);
     if (!active) return;
     // lane l stores bsums[4 * (l % 4) + l / 4]
     const uint32_t j = l & 3, sj = 4 * j + (l >> 2);
-    const int mine = j == 0 ? sum[0] : j == 1 ? sum[1] : j == 2 ? sum[2] : sum[3];
     if (AOS) {
         uint8_t *b = out.aos + (int64_t)blk * 292;   // 292 = 4 * 73: 4-byte aligned
         if (l == 0) *(float *)b = d;

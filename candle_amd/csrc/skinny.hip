@@ -14,7 +14,7 @@
 // gemm.hip), unpacks, and issues eight MFMAs per 16 activation rows.  The waves' partial 16 x 16
 // results are summed through LDS in wave order (deterministic; no atomics).  Many small workgroups
 // (n / 16) and one block in flight per wave keep enough bytes outstanding per CU.
-#include "qhip_internal.h"
+#include "quantize_blocks.h"
 
 namespace {
 
@@ -187,13 +187,61 @@ __device__ __forceinline__ void block_unpack(const uint8_t *wl, int lane, const 
     wmin = v8h{};
 }
 
+// The wave's rows of K block b, four at a time (lane l: row 4p + l/16, elements 64i + 4(l%16) ..; rows past m repeat the last one).
+template <int RT>
+__device__ __forceinline__ void load_direct(const float *__restrict__ x, int64_t m, int64_t k, int64_t b, int lane, float4 (&xf)[2 * RT][4]) {
+#pragma unroll
+    for (int p = 0; p < 2 * RT; p++) {
+        if (4 * p >= m) continue;
+        const int64_t row = 4 * p + (lane >> 4) < m ? 4 * p + (lane >> 4) : m - 1;
+        const float *src = x + row * k + b * 256 + 4 * (lane & 15);
+#pragma unroll
+        for (int i = 0; i < 4; i++) xf[p][i] = *(const float4 *)(src + 64 * i);
+    }
+}
+// ... quantized into the wave's buffer, in the image the copies of quantized rows make; `keep`: into the workspace as well.
+template <int DT, int RT>
+__device__ __forceinline__ void quantize_direct(const float4 (&xf)[2 * RT][4], const cq_act_view &a, int64_t m, int64_t k, int64_t b, int lane,
+                                                bool keep, uint8_t *buf) {
+    typedef Buf<DT, RT> B;
+    const int l = lane & 15;
+    const uint32_t sj = 4 * (l & 3) + (l >> 2);   // the sum cq_q8k_of_sixteen leaves with this lane
+#pragma unroll
+    for (int p = 0; p < 2 * RT; p++) {
+        if (4 * p >= m) continue;
+        uint32_t packed[4];
+        float d;
+        int bsum;
+        cq_q8k_of_sixteen(xf[p], l, packed, d, bsum);
+        const uint32_t row = 4 * p + (lane >> 4);
+        if (row >= m) continue;
+        uint8_t *at = buf + B::oAct + (row >> 3) * 2048u + (row & 7) * 128u + (l & 3) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; i++) *(uint32_t *)(at + (i >> 1) * 1024 + ((((i & 1) * 4 + (l >> 2)) ^ (row & 7)) << 4)) = packed[i];
+        if (l == 0) *(float *)(buf + B::oD8 + row * 4) = d;
+        if (is_k4(DT)) *(_Float16 *)(buf + B::oMin + row * 32 + sj * 2) = (_Float16)(float)bsum;
+        if (keep) {
+            const int64_t blk = row * (k >> 8) + b, tb = b * a.m_stride + row;
+#pragma unroll
+            for (int i = 0; i < 4; i++) *(uint32_t *)(a.qs + row * k + b * 256 + 64 * i + 4 * l) = packed[i];
+            if (l == 0) {
+                a.d[blk] = d;
+                a.dT[tb] = d;
+            }
+            a.bsums[blk * 16 + sj] = (int16_t)bsum;
+            ((_Float16 *)a.bsh)[tb * 16 + sj] = (_Float16)(float)bsum;
+        }
+    }
+}
+
 // RT = groups of eight activation rows held (rows m0 .. m0 + 8*RT - 1; the workspace pads rows, so
 // whole groups can be copied); results are stored for rows < m.  Requires n >= 16.
 // DUMP (verification): the block integers, and the min term as the f16 MFMA delivers it from a zero accumulator,
 // are stored through `dump` instead of the result through `y`.
-template <int DT, int RT, bool DUMP>
+// DIRECT: the rows come as f32 from `x` and every wave quantizes the blocks it contracts (see skinny_direct_kernel).
+template <int DT, int RT, bool DUMP, bool DIRECT = false>
 __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
-                                            float *__restrict__ y, cq_mfma_dump dump) {
+                                            float *__restrict__ y, cq_mfma_dump dump, const float *__restrict__ x = nullptr) {
     typedef Buf<DT, RT> B;
     constexpr bool MINS = is_k4(DT);
     constexpr int NT = (RT + 1) / 2;   // 16-row tiles
@@ -229,10 +277,16 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
 
     for (int64_t b = wave; b < kb; b += kWaves) {
         // ---- copies of block b: weights of the 16 rows, activation rows, their scales
+        float4 xf[DIRECT ? 2 * RT : 1][4];
+        if constexpr (DIRECT) {
+            load_direct<RT>(x, m, k, b, lane, xf);   // (first: what the quantizer waits for; requests are answered in order)
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int rg = 0; rg < 2; rg++) dma16(w.p0 + ((n_tile + rg * 8) * kb + b) * 128, wq_off, buf + rg * 1024);
         if (DT == CQ_DTYPE_Q6K) dma16(w.p1 + (n_tile * kb + b) * 64, wh_off, buf + 2048);
         if (DT == CQ_DTYPE_Q5K && lane < 32) dma16(w.p2 + (n_tile * kb + b) * 32, w5_off, buf + 2048);
+        if constexpr (!DIRECT) {
 #pragma unroll
         for (int i = 0; i < 2 * RT; i++) {
             const int rg = i >> 1, kh = i & 1;
@@ -240,8 +294,13 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
         }
         if (lane < 8 * RT) dma4(a.dT + b * a.m_stride + m0, lane * 4u, buf + B::oD8);
         if (MINS && lane < 16 * RT) dma16(a.bsh + (b * a.m_stride + m0) * 16, lane * 16u, buf + B::oMin);
+        }
         WHead<DT> head;
         load_head(w, (n_tile + r) * kb + b, head);
+        if constexpr (DIRECT) {
+            __builtin_amdgcn_sched_barrier(0);
+            quantize_direct<DT, RT>(xf, a, m, k, b, lane, tile == 0, buf);
+        }
         __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
 
         // ---- arithmetic of block b
@@ -780,9 +839,43 @@ template <typename F> __device__ __forceinline__ void each_block(int64_t left, F
     }
 }
 
-template <int DT, int RT, bool DUMP>
+// The wave's rows of K step g for the bodies that quantize themselves (lane l: elements 4l .. of the step; zeros past the row's end).
+template <int RT>
+__device__ __forceinline__ void load_direct_q8(const float *__restrict__ x, int64_t m, int64_t k, int64_t g, int lane, float4 (&xf)[8 * RT]) {
+    const int64_t e0 = g * 256 + 4 * lane;
+#pragma unroll
+    for (int row = 0; row < 8 * RT; row++) xf[row] = row < m && e0 < k ? *(const float4 *)(x + row * k + e0) : make_float4(0.f, 0.f, 0.f, 0.f);
+}
+template <int DT, int RT>
+__device__ __forceinline__ void quantize_direct_q8(const float4 (&xf)[8 * RT], const cq_act_view &a, int64_t m, int64_t k, int64_t g, int lane,
+                                                   bool keep, uint8_t *buf) {
+    typedef BufQ8<DT, RT> B;
+    const int64_t e0 = g * 256 + 4 * lane;
+#pragma unroll
+    for (int row = 0; row < 8 * RT; row++) {
+        if (row >= m) continue;
+        uint32_t packed;
+        float d;
+        int sum;
+        cq_q8_0_of_eight(xf[row], packed, d, sum);
+        const float dr = cq_h2f(cq_f2h(d));
+        *(uint32_t *)(buf + B::oAct + (row >> 3) * 2048 + (lane >> 5) * 1024 + (row & 7) * 128 + ((((lane >> 2) & 7) ^ (row & 7)) << 4) + (lane & 3) * 4) = packed;
+        if ((lane & 7) == 0) *(float *)(buf + B::oD8 + (row >> 3) * 256 + (lane >> 3) * 32 + (row & 7) * 4) = dr;
+        if (keep && e0 < k) {
+            *(uint32_t *)(a.qs + row * k + e0) = packed;
+            if ((lane & 7) == 0) {
+                const int64_t blk = row * (k >> 5) + (e0 >> 5);
+                a.d[blk] = dr;
+                a.bsum32[blk] = (int16_t)sum;
+                a.dT[(e0 >> 5) * a.m_stride + row] = dr;
+            }
+        }
+    }
+}
+
+template <int DT, int RT, bool DUMP, bool DIRECT = false>
 __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
-                                                  float *__restrict__ y, cq_mfma_dump dump) {
+                                                  float *__restrict__ y, cq_mfma_dump dump, const float *__restrict__ x = nullptr) {
     typedef BufQ8<DT, RT> B;
     constexpr bool Q4 = DT == CQ_DTYPE_Q4_0;
     constexpr int NT = (RT + 1) / 2;   // 16-row tiles
@@ -819,6 +912,11 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
     for (int t = 0; t < NT; t++) out[t] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
 
     for (int64_t g = wave; g < kg; g += kWaves) {
+        float4 xf[DIRECT ? 8 * RT : 1];
+        if constexpr (DIRECT) {
+            load_direct_q8<RT>(x, m, k, g, lane, xf);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (Q4) {
 #pragma unroll
             for (int rg = 0; rg < 2; rg++) dma16(w.p0 + (n_tile + rg * 8) * (k >> 1) + g * 128, q4_off, buf + rg * 1024);
@@ -829,14 +927,20 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
                 dma16(w.p0 + (n_tile + rg * 8) * k + g * 256 + kh * 128, row_off, buf + i * 1024);
             }
         }
+        if constexpr (!DIRECT) {
 #pragma unroll
         for (int i = 0; i < 2 * RT; i++) {
             const int rg = i >> 1, kh = i & 1;
             dma16(a.qs + (m0 + rg * 8) * k + g * 256 + kh * 128, row_off, buf + B::oAct + i * 1024);
         }
         issue_scales<RT>(a, m0, g, buf + B::oD8, lane);
+        }
         // the eight block scales of this lane's weight row
         const u32x4_a4 dwv = *(const u32x4_a4 *)(w.p1 + ((n_tile + r) * kb + g * 8) * 2);
+        if constexpr (DIRECT) {
+            __builtin_amdgcn_sched_barrier(0);
+            quantize_direct_q8<DT, RT>(xf, a, m, k, g, lane, tile == 0, buf);
+        }
         __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
 
         const uint32_t dww[4] = {dwv.x, dwv.y, dwv.z, dwv.w};
@@ -917,6 +1021,19 @@ __global__ void __launch_bounds__(kThreads) skinny_shared_kernel(MultiArgs ma, c
     const cq_mfma_dump none{nullptr, nullptr, 0};
     if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, RT, false>(w, a, t - ma.first[i], 0, m, ma.y[i], none);
     else skinny_body<DT, RT, false>(w, a, t - ma.first[i], 0, m, ma.y[i], none);
+}
+
+// ------------------------------------------------------------ the rows quantized by the waves that contract them ----
+// One launch for the whole call: no quantizer launch in front, whose start and end are most of a small call (2.5 us of host time and
+// 2-3 us on the device).  A wave quantizes the rows' blocks that it contracts into its own buffer, so that no wave waits for
+// another; every workgroup repeats that, about 130 instructions for four rows of a block of 256, which is why it is for few weight rows
+// and few activation rows (cq_skinny_direct_takes).  Workgroup 0 leaves the quantized rows in the workspace too, where a quantizer
+// launch would have put them.
+template <int DT>
+__global__ void __launch_bounds__(kThreads) skinny_direct_kernel(cq_weight w, cq_act_view a, const float *__restrict__ x, int64_t m, float *__restrict__ y) {
+    const cq_mfma_dump none{nullptr, nullptr, 0};
+    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, 1, false, true>(w, a, blockIdx.x, 0, m, y, none, x);
+    else skinny_body<DT, 1, false, true>(w, a, blockIdx.x, 0, m, y, none, x);
 }
 
 // ------------------------------------------- the same with everything of a workgroup in flight at once ----
@@ -1425,6 +1542,13 @@ hipError_t launch_any(const cq_weight *w, cq_act_view a, int act_dtype, int64_t 
     return launch_dt<CQ_DTYPE_Q6K, DUMP>(w, a, m, y, d, s);
 }
 
+template <int DT> hipError_t launch_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s) {
+    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<DT, 1>::kBytes : (int)Buf<DT, 1>::kBytes) * kWaves;
+    if (hipError_t e = cq_ensure_lds<skinny_direct_kernel<DT>>(w->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_direct_kernel<DT>), (unsigned)((w->n + 15) / 16), kThreads, lds, s, *w, a, x, m, y);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 bool cq_skinny_takes(const cq_weight *w, int act_dtype) {
@@ -1443,6 +1567,27 @@ hipError_t cq_launch_skinny(const cq_weight *w, cq_act_view a, int act_dtype, in
 
 hipError_t cq_launch_skinny_dump(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, cq_mfma_dump d, hipStream_t s) {
     return launch_any<true>(w, a, act_dtype, m, nullptr, d, s);
+}
+
+// The rows quantized by the contracting waves (where the dot-product kernel does not take them in one launch): where the quantizing that
+// every workgroup repeats costs less than the launch it saves.  Measured, us back to back / from a graph, against the two launches:
+//   Q4K 1024 x 1024, 5 rows 4.8 / 4.5 against 7.5 / 5.0; 8 rows 4.8 / 4.5 against 7.4 / 5.1; Q6K 4096 x 1024, 8 rows 5.0 / 4.7 against
+//   7.3 / 5.3; Q8_0 1024 x 1024, 5 rows 4.7 / 4.4 against 7.4 / 5.2, 8 rows 5.5 / 5.3 against 7.4 / 5.3
+// and beyond the limits below behind from a graph or everywhere: two blocks a wave or two workgroups a CU double the quantizing
+// (Q4K 2048 x 2048, 8 rows 6.0 against 6.8 / 5.6; 8192 x 2048 10.6 against 7.3), nine rows take a second group (Q4K 1024 x 1024, 16 rows 6.9
+// against 7.0 / 5.6), Q4_0 with 8 rows 5.9 / 5.7 against 7.4 / 5.5.
+bool cq_skinny_direct_takes(const cq_weight *w, int act_dtype, int64_t m) {
+    return m >= 2 && m <= (w->dtype == CQ_DTYPE_Q4_0 ? 7 : 8) && w->n <= 4096 && w->k <= (m <= 4 ? 2048 : 1024) && cq_skinny_takes(w, act_dtype);
+}
+hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s) {
+    if (m > 8) return hipErrorInvalidValue;
+    switch (w->dtype) {
+    case CQ_DTYPE_Q8_0: return launch_direct<CQ_DTYPE_Q8_0>(w, a, x, m, y, s);
+    case CQ_DTYPE_Q4_0: return launch_direct<CQ_DTYPE_Q4_0>(w, a, x, m, y, s);
+    case CQ_DTYPE_Q4K: return launch_direct<CQ_DTYPE_Q4K>(w, a, x, m, y, s);
+    case CQ_DTYPE_Q5K: return launch_direct<CQ_DTYPE_Q5K>(w, a, x, m, y, s);
+    default: return launch_direct<CQ_DTYPE_Q6K>(w, a, x, m, y, s);
+    }
 }
 
 bool cq_skinny_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
