@@ -114,14 +114,14 @@ inline int cq_storage_dtype(int ggml_dtype) {
     return ggml_dtype == CQ_DTYPE_Q3K || ggml_dtype == CQ_DTYPE_Q2K ? CQ_DTYPE_Q6K : ggml_dtype;
 }
 // y[r, c] -= sum_b (d8[r, b] * dmin[c, b]) * sum_j bsums[r, b, j] * m[c, b, j] for Q2K weights (k_quants.rs:727-733, :762)
-hipError_t cq_launch_min16_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s);
+hipError_t cq_launch_min16_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool apart, hipStream_t s);
 // Q8K as a weight type (q8k_weight.hip): planes p0 qs, p1 d (f32), p2 bsums
 hipError_t cq_launch_repack_q8k(const cq_weight *w, uint8_t *aos, bool inverse, hipStream_t s);
 hipError_t cq_launch_dequantize_q8k(const cq_weight *w, float *d32, uint16_t *d16, hipStream_t s);
 hipError_t cq_launch_q8k_weight_matmul(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s);
 // y[r, c] += sum_b m[c, b] * s8[r, b] for Q4_1 / Q5_1 weights, s8 the `s` field of the activation's Q8_1 block
 // (k_quants.rs:665-691) recomputed from the workspace's block sums and scales.
-hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s);
+hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool apart, hipStream_t s);
 // A step of the caller's model computed on the way into the activation quantizer (CQ_PRE_*):
 // rms_norm: x / sqrt(mean(x^2) + eps) * aux[k]; silu_mul: silu(x) * aux[m][k] (aux indexed like x).
 struct cq_pre {
