@@ -19,7 +19,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # gemm.hip: MFMA results are consumed by VALU code every block; keep the accumulators in ordinary
 # VGPRs rather than AccVGPRs, which VALU instructions cannot read.
 EXTRA_FLAGS = {"gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "gemm_blk32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-               "skinny.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+               "skinny.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "min_term.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _compile(src: str) -> str:
