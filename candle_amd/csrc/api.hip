@@ -173,21 +173,19 @@ static int weight_alloc(int dev, int dt, int64_t n, int64_t k, cq_weight **out) 
 extern "C" int cq_weight_zeros(int dev, int dt, int64_t n, int64_t k, cq_weight **out) {
     int rc = weight_alloc(dev, dt, n, k, out);
     if (rc) return rc;
-    hipError_t e = hipMemset((*out)->base, 0, (*out)->alloc_bytes);
-    if (e == hipSuccess && (*out)->ggml_dtype != (*out)->dtype && (*out)->ggml_bytes) {
-        // all-zero blocks of the caller's type are not all-zero planes of the holding type (a zero quant is stored
-        // with its offset): encode them
-        void *tmp = nullptr;
-        e = hipMalloc(&tmp, (*out)->ggml_bytes + 256);
-        if (e == hipSuccess) e = hipMemset(tmp, 0, (*out)->ggml_bytes);
-        if (e == hipSuccess) e = cq_launch_repack(*out, (const uint8_t *)tmp, nullptr);
+    const cq_weight *w = *out;
+    hipError_t e;
+    if (w->ggml_dtype == w->dtype) {
+        e = hipMemset(w->base, 0, w->alloc_bytes);
+    } else {
+        // a type held in another's planes: a zero quant is stored with its offset there
+        e = cq_launch_zero_planes(w, nullptr);
         if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
-        if (tmp) (void)hipFree(tmp);
     }
     if (e != hipSuccess) {
         cq_weight_destroy(*out);
         *out = nullptr;
-        return cq_set_error(CQ_ERR_HIP, "hipMemset failed: %s", hipGetErrorString(e));
+        return cq_set_error(CQ_ERR_HIP, "clearing a weight failed: %s", hipGetErrorString(e));
     }
     return CQ_OK;
 }
@@ -272,13 +270,20 @@ extern "C" int cq_weight_quantize(cq_weight *w, const float *src_dev, void *stre
     if (w->ggml_bytes == 0) return CQ_OK;
     CQ_HIP_CHECK(hipSetDevice(w->dev));
     hipStream_t s = (hipStream_t)stream;
-    void *tmp = nullptr;
-    CQ_HIP_CHECK(hipMalloc(&tmp, w->ggml_bytes + 256));
-    const int64_t nb = w->n * (w->k / cq_block_size(w->dtype));
-    hipError_t e = cq_launch_quantize_weight(w->ggml_dtype, src_dev, nb, (uint8_t *)tmp, s);
-    if (e == hipSuccess) e = cq_launch_repack(w, (const uint8_t *)tmp, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);  // the temporary is freed below
-    (void)hipFree(tmp);
+    hipError_t e;
+    if (w->dtype == CQ_DTYPE_Q8K) {   // (k_quants.rs:1788-1825) the activation quantizer writing GGML blocks, one 256-element row per block
+        void *tmp = nullptr;
+        CQ_HIP_CHECK(hipMalloc(&tmp, w->ggml_bytes + 256));
+        e = cq_launch_quantize_act_aos(CQ_DTYPE_Q8K, src_dev, w->n * (w->k / 256), 256, cq_no_pre(), (uint8_t *)tmp, s);
+        if (e == hipSuccess) e = cq_launch_repack(w, (const uint8_t *)tmp, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);  // the temporary is freed below
+        (void)hipFree(tmp);
+    } else {
+        // (a new weight is cleared on the null stream, which this stream may not wait for)
+        e = s ? hipStreamSynchronize(nullptr) : hipSuccess;
+        if (e == hipSuccess) e = cq_launch_quantize_weight(w, src_dev, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);  // the weight may be used on any stream from here on
+    }
     if (e != hipSuccess) return cq_set_error(CQ_ERR_HIP, "weight quantize failed: %s", hipGetErrorString(e));
     return CQ_OK;
 }
@@ -299,42 +304,38 @@ extern "C" int cq_weight_dequantize_f16(const cq_weight *w, uint16_t *dst_dev, v
     return CQ_OK;
 }
 
-// ---- device memory into pageable host memory ----
+// ---- a weight's GGML blocks into pageable host memory ----
 // Bound: the link (25 MB: 460 us to pinned memory) and the copy into the caller's pages, 28 GB/s a thread and half of that where the pages are
-// new.  hipMemcpy itself pins and unpins the caller's pages.  Here pieces go to pinned slots and from there to the caller, by up to four
-// threads, each with two slots of its own: one piece on its way over the link, the other being copied.  The threads share nothing but the
-// null stream, on which each launches the copies of its pieces (a kernel: a piece by the copy engine costs 10 us more).  The slots live for
+// new.  hipMemcpy itself pins and unpins the caller's pages.  Here the blocks go in pieces to pinned slots, written there by the kernel that
+// puts them together, and from the slots to the caller, by up to four threads, each with two slots of its own: one piece on its way over
+// the link, the other being copied.  The threads share nothing but the null stream, on which each launches its pieces.  The slots live for
 // the call, 8 MiB of them at most (allocating them takes some 50 us), so that nothing stays pinned after it.
-// us for a whole download, hipMemcpy -> pieces: 8.9 MB 550 -> 400, 26.7 MB 1555 -> 840, 35.7 MB 3500 -> 1310, 71 MB 7150 -> 2700 (one thread
-// 520, 1290, 3050, 6230; two 430, 870, 1910, 3950); 4.4 MB 320 -> 340: below 5 MiB hipMemcpy stays.
+// us for a whole download, hipMemcpy from a device copy -> pieces: below 5 MiB hipMemcpy is as
+// fast, 11008 x 4096 Q4_0 25 MB 1440 -> 740, Q5K 31 MB 1740 -> 1030, Q6K 37 MB 3710 -> 1340, Q8_0 48 MB 4830 -> 1730 (one thread takes twice
+// that; pieces by the copy engine cost 10 us each more).
 namespace {
 constexpr size_t kPiece = 1 << 20;
 constexpr int kCopiers = 4;
 
-__global__ void __launch_bounds__(256) to_slot_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ slot, unsigned count) {
-    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < count; i += gridDim.x * 256) slot[i] = src[i];
-}
-
 // Pieces me, me + of, ... through the two slots of `slots`.
-hipError_t copy_pieces(int dev, const uint8_t *src, uint8_t *dst, size_t bytes, uint8_t *slots, size_t me, size_t of) {
-    const size_t n = (bytes + kPiece - 1) / kPiece;
+hipError_t copy_pieces(const cq_weight *w, uint8_t *dst, uint8_t *slots, int64_t me, int64_t of) {
+    const int64_t ts = cq_type_size(w->ggml_dtype), blocks = w->ggml_bytes / ts, piece = (int64_t)kPiece / ts / 256 * 256;
+    const int64_t n = (blocks + piece - 1) / piece;
     hipEvent_t landed[2] = {nullptr, nullptr};
-    hipError_t e = hipSetDevice(dev);
+    hipError_t e = hipSetDevice(w->dev);
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipEventCreateWithFlags(&landed[i], hipEventDisableTiming);
-    const auto length = [&](size_t c) { return bytes - c * kPiece < kPiece ? bytes - c * kPiece : kPiece; };
-    const auto fetch = [&](size_t c, int slot) {
-        hipLaunchKernelGGL(to_slot_kernel, dim3(64), dim3(256), 0, nullptr, (const uint4 *)(src + c * kPiece), (uint4 *)(slots + slot * kPiece),
-                           (unsigned)((length(c) + 15) / 16));
-        const hipError_t f = hipGetLastError();
+    const auto count = [&](int64_t c) { return blocks - c * piece < piece ? blocks - c * piece : piece; };
+    const auto fetch = [&](int64_t c, int slot) {
+        const hipError_t f = cq_launch_unpack(w, c * piece, count(c), slots + slot * kPiece, nullptr);
         return f == hipSuccess ? hipEventRecord(landed[slot], nullptr) : f;
     };
     for (int i = 0; i < 2 && e == hipSuccess; i++)
         if (me + i * of < n) e = fetch(me + i * of, i);
     int slot = 0;
-    for (size_t c = me; c < n && e == hipSuccess; c += of, slot ^= 1) {
+    for (int64_t c = me; c < n && e == hipSuccess; c += of, slot ^= 1) {
         e = hipEventSynchronize(landed[slot]);
         if (e != hipSuccess) break;
-        memcpy(dst + c * kPiece, slots + slot * kPiece, length(c));
+        memcpy(dst + c * piece * ts, slots + slot * kPiece, (size_t)(count(c) * ts));
         if (c + 2 * of < n) e = fetch(c + 2 * of, slot);
     }
     for (hipEvent_t ev : landed)
@@ -342,19 +343,10 @@ hipError_t copy_pieces(int dev, const uint8_t *src, uint8_t *dst, size_t bytes, 
     return e;
 }
 
-// `src` is padded to whole 16-byte groups.
-hipError_t copy_to_host(int dev, const void *src, void *dst, size_t bytes) {
-    hipPointerAttribute_t attr{};
-    const bool pinned = hipPointerGetAttributes(&attr, dst) == hipSuccess && attr.type == hipMemoryTypeHost;
-    uint8_t *slots = nullptr;
-    if (pinned || bytes < 5 * kPiece || hipHostMalloc((void **)&slots, 2 * kCopiers * kPiece, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
-    }
-    (void)hipGetLastError();   // (a pointer unknown to HIP is an error on some versions)
+hipError_t copy_by_threads(const cq_weight *w, uint8_t *dst, uint8_t *slots) {
     hipError_t err[kCopiers];
     std::thread helpers[kCopiers];
-    const auto work = [&](int t) { err[t] = copy_pieces(dev, (const uint8_t *)src, (uint8_t *)dst, bytes, slots + 2 * t * kPiece, t, kCopiers); };
+    const auto work = [&](int t) { err[t] = copy_pieces(w, dst, slots + 2 * t * kPiece, t, kCopiers); };
     for (int t = 1; t < kCopiers; t++) {
         try {
             helpers[t] = std::thread(work, t);
@@ -365,10 +357,9 @@ hipError_t copy_to_host(int dev, const void *src, void *dst, size_t bytes) {
         if (!helpers[t].joinable()) work(t);
     for (int t = 1; t < kCopiers; t++)
         if (helpers[t].joinable()) helpers[t].join();
-    hipError_t e = hipStreamSynchronize(nullptr);   // (after an error copies into the slots may still be on their way)
+    hipError_t e = hipStreamSynchronize(nullptr);   // (after an error pieces may still be on their way into the slots)
     for (hipError_t each : err)
         if (each != hipSuccess) e = each;
-    (void)hipHostFree(slots);
     return e;
 }
 }  // namespace
@@ -379,12 +370,25 @@ extern "C" int cq_weight_to_ggml(const cq_weight *w, void *host_dst, size_t nbyt
         return cq_set_error(CQ_ERR_INVALID, "expected a %zu-byte destination, got %zu", w->ggml_bytes, nbytes);
     if (nbytes == 0) return CQ_OK;
     CQ_HIP_CHECK(hipSetDevice(w->dev));
-    void *tmp = nullptr;
-    CQ_HIP_CHECK(hipMalloc(&tmp, nbytes + 256));
     hipError_t e = hipDeviceSynchronize();
-    if (e == hipSuccess) e = cq_launch_unpack(w, (uint8_t *)tmp, nullptr);
-    if (e == hipSuccess) e = copy_to_host(w->dev, tmp, host_dst, nbytes);
-    (void)hipFree(tmp);
+    const auto pinned = [&] {
+        hipPointerAttribute_t attr{};
+        return hipPointerGetAttributes(&attr, host_dst) == hipSuccess && attr.type == hipMemoryTypeHost;
+    };
+    void *slots = nullptr;
+    if (e == hipSuccess && nbytes >= 5 * kPiece && w->dtype != CQ_DTYPE_Q8K && !pinned() &&
+        hipHostMalloc(&slots, 2 * kCopiers * kPiece, hipHostMallocDefault) == hipSuccess) {
+        e = copy_by_threads(w, (uint8_t *)host_dst, (uint8_t *)slots);
+        (void)hipHostFree(slots);
+        (void)hipGetLastError();   // (a pointer unknown to HIP is an error on some versions)
+    } else {
+        (void)hipGetLastError();
+        void *tmp = nullptr;
+        if (e == hipSuccess) e = hipMalloc(&tmp, nbytes + 256);
+        if (e == hipSuccess) e = cq_launch_unpack(w, 0, w->n * (w->k / cq_block_size(w->dtype)), (uint8_t *)tmp, nullptr);
+        if (e == hipSuccess) e = hipMemcpy(host_dst, tmp, nbytes, hipMemcpyDeviceToHost);
+        if (tmp) (void)hipFree(tmp);
+    }
     if (e != hipSuccess) return cq_set_error(CQ_ERR_HIP, "weight download failed: %s", hipGetErrorString(e));
     return CQ_OK;
 }

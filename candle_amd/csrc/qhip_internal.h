@@ -99,8 +99,10 @@ bool cq_timing_take(hipEvent_t *start, hipEvent_t *stop);
 
 // ---- launchers implemented in the .hip files -------------------------------
 // repack.hip
+hipError_t cq_launch_zero_planes(const cq_weight *w, hipStream_t s);   // the whole allocation as all-zero GGML blocks leave it
 hipError_t cq_launch_repack(const cq_weight *w, const uint8_t *aos_dev, hipStream_t s);   // GGML AoS of w->ggml_dtype -> planes
-hipError_t cq_launch_unpack(const cq_weight *w, uint8_t *aos_dev, hipStream_t s);         // planes -> GGML AoS
+// planes -> GGML AoS, blocks first .. first + nblocks - 1 (Q8K: all of them); `aos` 16-byte aligned, device or pinned host memory
+hipError_t cq_launch_unpack(const cq_weight *w, int64_t first, int64_t nblocks, uint8_t *aos, hipStream_t s);
 // Types held in another type's planes (same values, same arithmetic): Q5_0 as Q8_0, Q3K as Q6K.
 // Q4_1 and Q5_1 (value d * q + m) are Q8_0 planes with qs = q plus the plane p2 of the blocks' minima m (f16): the
 // holding type's kernels give the sum_i * d * d8 part of their dot product, cq_launch_min32_term adds sum_b m_b * s8_b.
@@ -144,7 +146,8 @@ hipError_t cq_launch_quantize_act_aos(int act_dtype, const float *x, int64_t m, 
 hipError_t cq_launch_quantize_act_ws(int act_dtype, const float *x, const int32_t *row_ids, int64_t m, int64_t k,
                                      cq_pre pre, cq_act_view v, cq_clear clear, hipStream_t s);
 // quantize_weight.hip
-hipError_t cq_launch_quantize_weight(int dtype, const float *src, int64_t nblocks, uint8_t *aos_dev, hipStream_t s);
+// f32 -> the weight's planes (not Q8K)
+hipError_t cq_launch_quantize_weight(const cq_weight *w, const float *src, hipStream_t s);
 // dequantize.hip
 hipError_t cq_launch_dequantize(const cq_weight *w, float *dst32, uint16_t *dst16, hipStream_t s);
 // matvec.hip

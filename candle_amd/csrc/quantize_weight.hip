@@ -15,10 +15,12 @@
 // quants in registers: eight or sixteen times the lanes of one lane per 256-element block, and no array in scratch.
 // A workgroup's elements come in through LDS in whole lines (rows padded by four floats, so that the lanes' 16-byte
 // reads of their own groups spread over the banks); what the groups of a block share (scales, quants that meet in one
-// byte) goes through LDS too, and the finished blocks leave as one run of 16-byte stores.
+// byte) goes through LDS too, where the finished blocks are put together and then stored straight to the weight's planes.
 // 11008 x 4096 elements (180 MB read), a lane per block before -> now: Q4K / Q5K 1730 / 1704 -> 119 / 121 us, Q2K 1105 -> 129,
 // Q3K 1574 -> 183, Q6K 520 -> 201, Q4_0 75 -> 36, Q4_1 97 -> 37, Q5_0 171 -> 40, Q5_1 174 -> 40, Q8_0 163 -> 42 (4.9-5.4 TB/s).
-#include "qhip_internal.h"
+// Without GGML blocks in memory between the quantizer and the planes (no temporary to allocate, 12-15 us less of re-packing), a whole
+// call that creates and quantizes 11008 x 4096: Q4K 215 -> 182 us, Q4_0 127 -> 94, Q6K 530 -> 261, Q8_0 383 -> 97, Q5_1 430 -> 113.
+#include "repack_units.h"
 
 namespace {
 
@@ -46,18 +48,13 @@ template <int G> __device__ __forceinline__ void load_groups(const float *__rest
     __syncthreads();   // the same LDS takes the finished blocks
 }
 
-// The workgroup's blocks from their LDS image to `out` (TS bytes each, PER of them in a full workgroup).
-template <int TS, int PER> __device__ __forceinline__ void store_blocks(const uint8_t *img, int64_t nblocks, uint8_t *__restrict__ out) {
-    static_assert(PER * TS % 16 == 0, "whole 16-byte groups");
+// The workgroup's blocks from their LDS image to the weight's planes, PER of them in a full workgroup.
+template <int DT, int PER> __device__ __forceinline__ void store_blocks(uint8_t *img, int64_t nblocks, const cq_planes &pl) {
+    constexpr int U = Ggml<DT>::kUnits;
     const int64_t b0 = (int64_t)blockIdx.x * PER;
-    uint8_t *dst = out + b0 * TS;
+    const int count = (int)(nblocks - b0 < PER ? nblocks - b0 : PER);
     __syncthreads();
-    if (b0 + PER <= nblocks) {
-        for (int i = threadIdx.x; i < PER * TS / 16; i += kLanes) ((uint4 *)dst)[i] = ((const uint4 *)img)[i];
-    } else {
-        const int n = (int)(nblocks - b0) * TS / 2;
-        for (int i = threadIdx.x; i < n; i += kLanes) ((uint16_t *)dst)[i] = ((const uint16_t *)img)[i];
-    }
+    for (int i = threadIdx.x; i < count * U; i += kLanes) repack_unit<DT, false>(img + i / U * Ggml<DT>::kSize, b0 + i / U, i % U, pl);
 }
 
 __device__ __forceinline__ void put16(uint8_t *p, uint16_t v) { *(uint16_t *)p = v; }   // (blocks lie at even offsets)
@@ -83,16 +80,9 @@ __device__ __forceinline__ int round_signed(float v, int lo, int hi) {
 }
 
 // ---------------------------------------------------------------------- blocks of 32: a lane per block ----
-template <int DT> struct Blk32;
-template <> struct Blk32<CQ_DTYPE_Q4_0> { static constexpr int kSize = 18; };
-template <> struct Blk32<CQ_DTYPE_Q4_1> { static constexpr int kSize = 20; };
-template <> struct Blk32<CQ_DTYPE_Q5_0> { static constexpr int kSize = 22; };
-template <> struct Blk32<CQ_DTYPE_Q5_1> { static constexpr int kSize = 24; };
-template <> struct Blk32<CQ_DTYPE_Q8_0> { static constexpr int kSize = 34; };
-
 template <int DT>
-__global__ void __launch_bounds__(kLanes) quantize_blk32(const float *__restrict__ src, int64_t nblocks, uint8_t *__restrict__ out) {
-    constexpr int TS = Blk32<DT>::kSize;
+__global__ void __launch_bounds__(kLanes) quantize_blk32(const float *__restrict__ src, int64_t nblocks, cq_planes pl) {
+    constexpr int TS = Ggml<DT>::kSize;
     __shared__ __align__(16) float lds[kLanes * 36];
     float x[32];
     load_groups<32>(src, nblocks, lds, x);
@@ -176,7 +166,7 @@ __global__ void __launch_bounds__(kLanes) quantize_blk32(const float *__restrict
         }
         put_bytes(y + (FIVE ? 8 : 4), w);
     }
-    store_blocks<TS, kLanes>(img, nblocks, out);
+    store_blocks<DT, kLanes>(img, nblocks, pl);
 }
 
 // ------------------------------------------------------------------- blocks of 256: a lane per group ----
@@ -235,8 +225,8 @@ __device__ __forceinline__ float max_of_8(float v) {
 // LEVELS = 16: Q4K (144-byte blocks).  LEVELS = 32: Q5K (k_quants.rs:1450-1525), the same scale search
 // with 31 as the top level, the quants' fifth bits in qh[32] between the scales and the nibbles.
 template <int LEVELS>
-__global__ void __launch_bounds__(kLanes) quantize_q4k(const float *__restrict__ src, int64_t nblocks, uint8_t *__restrict__ out) {
-    constexpr int TS = LEVELS == 16 ? 144 : 176, PER = kLanes / 8;
+__global__ void __launch_bounds__(kLanes) quantize_q4k(const float *__restrict__ src, int64_t nblocks, cq_planes pl) {
+    constexpr int DT = LEVELS == 16 ? CQ_DTYPE_Q4K : CQ_DTYPE_Q5K, TS = Ggml<DT>::kSize, PER = kLanes / 8;
     constexpr int kQs = LEVELS == 16 ? 16 : 48;   // offset of the nibbles in the block
     __shared__ __align__(16) float lds[kLanes * 36];
     __shared__ __align__(16) uint8_t codes[kLanes * 2];   // per block: eight scale codes, eight min codes
@@ -297,7 +287,7 @@ __global__ void __launch_bounds__(kLanes) quantize_q4k(const float *__restrict__
         if (j < 2) *(uint4 *)(y + 16 + 16 * j) = make_uint4(w[0], w[1], w[2], w[3]);
     }
     if (j == 0) *(uint4 *)y = make_uint4((uint32_t)dh | ((uint32_t)dminh << 16), u0, u1, u2);
-    store_blocks<TS, PER>(img, nblocks, out);
+    store_blocks<DT, PER>(img, nblocks, pl);
 }
 
 // utils.rs:61-198 specialised to n = 16, nmax = 32, rmse_type = 1 (weights w = x*x; returns after
@@ -398,8 +388,8 @@ __device__ __forceinline__ uint4 pack16(const int (&q)[16]) {
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-__global__ void __launch_bounds__(kLanes) quantize_q6k(const float *__restrict__ src, int64_t nblocks, uint8_t *__restrict__ out) {
-    constexpr int TS = 210, PER = kLanes / 16;
+__global__ void __launch_bounds__(kLanes) quantize_q6k(const float *__restrict__ src, int64_t nblocks, cq_planes pl) {
+    constexpr int DT = CQ_DTYPE_Q6K, TS = Ggml<DT>::kSize, PER = kLanes / 16;
     __shared__ __align__(16) float lds[kLanes * 20];
     __shared__ __align__(16) float scales[kLanes];
     __shared__ __align__(16) uint4 quants[kLanes];
@@ -455,7 +445,7 @@ __global__ void __launch_bounds__(kLanes) quantize_q6k(const float *__restrict__
     } else if (j == 12) {
         put16(y + 208, dh);
     }
-    store_blocks<TS, PER>(img, nblocks, out);
+    store_blocks<DT, PER>(img, nblocks, pl);
 }
 
 // Two-bit quants of a 256-element block, four elements 32 apart in one byte (Q2K, Q3K): chunk c < 4 of 16 bytes.
@@ -474,8 +464,8 @@ __device__ __forceinline__ void put_two_bits(const uint4 *Q, int c, uint8_t *p) 
 }
 
 // Q2K (k_quants.rs:770-839): sixteen groups of sixteen, make_qkx1_quants with three levels, 4-bit scales and minima
-__global__ void __launch_bounds__(kLanes) quantize_q2k(const float *__restrict__ src, int64_t nblocks, uint8_t *__restrict__ out) {
-    constexpr int TS = 84, PER = kLanes / 16;
+__global__ void __launch_bounds__(kLanes) quantize_q2k(const float *__restrict__ src, int64_t nblocks, cq_planes pl) {
+    constexpr int DT = CQ_DTYPE_Q2K, TS = Ggml<DT>::kSize, PER = kLanes / 16;
     const float Q4SCALE = 15.0f;
     __shared__ __align__(16) float lds[kLanes * 20];
     __shared__ __align__(16) uint4 quants[kLanes];
@@ -515,7 +505,7 @@ __global__ void __launch_bounds__(kLanes) quantize_q2k(const float *__restrict__
     if (j < 4) put_two_bits(quants + blk * 16, j, y + 16 + 16 * j);
     else if (j == 4) put16(y + 80, dh);
     else if (j == 5) put16(y + 82, dmh);
-    store_blocks<TS, PER>(img, nblocks, out);
+    store_blocks<DT, PER>(img, nblocks, pl);
 }
 
 // utils.rs:261-326 with nmax = 4, do_rmse = true, n = 16: only the returned scale is used
@@ -564,8 +554,8 @@ __device__ __forceinline__ float make_q3_quants_16(const float (&x)[16]) {
     return sumlx / suml2;
 }
 
-__global__ void __launch_bounds__(kLanes) quantize_q3k(const float *__restrict__ src, int64_t nblocks, uint8_t *__restrict__ out) {
-    constexpr int TS = 110, PER = kLanes / 16;
+__global__ void __launch_bounds__(kLanes) quantize_q3k(const float *__restrict__ src, int64_t nblocks, cq_planes pl) {
+    constexpr int DT = CQ_DTYPE_Q3K, TS = Ggml<DT>::kSize, PER = kLanes / 16;
     __shared__ __align__(16) float lds[kLanes * 20];
     __shared__ __align__(16) float scales[kLanes];
     __shared__ __align__(16) uint4 quants[kLanes];
@@ -623,32 +613,31 @@ __global__ void __launch_bounds__(kLanes) quantize_q3k(const float *__restrict__
     } else if (j == 7) {
         put16(y + 108, dh);
     }
-    store_blocks<TS, PER>(img, nblocks, out);
+    store_blocks<DT, PER>(img, nblocks, pl);
 }
 
-template <typename K> hipError_t launch(K kernel, int64_t nblocks, int lanes_per_block, const float *src, uint8_t *out, hipStream_t s) {
-    const int64_t groups = nblocks * lanes_per_block;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)((groups + kLanes - 1) / kLanes)), dim3(kLanes), 0, s, src, nblocks, out);
+template <typename K> hipError_t launch(K kernel, const cq_weight *w, int lanes_per_block, const float *src, hipStream_t s) {
+    const int64_t nblocks = w->n * (w->k / cq_block_size(w->ggml_dtype)), groups = nblocks * lanes_per_block;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((groups + kLanes - 1) / kLanes)), dim3(kLanes), 0, s, src, nblocks,
+                       cq_planes{w->p0, w->p1, w->p2, w->p3, w->p4, w->p5});
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t cq_launch_quantize_weight(int dtype, const float *src, int64_t nblocks, uint8_t *aos_dev, hipStream_t s) {
-    if (nblocks == 0) return hipSuccess;
-    switch (dtype) {
-    case CQ_DTYPE_Q4_0: return launch(quantize_blk32<CQ_DTYPE_Q4_0>, nblocks, 1, src, aos_dev, s);
-    case CQ_DTYPE_Q4_1: return launch(quantize_blk32<CQ_DTYPE_Q4_1>, nblocks, 1, src, aos_dev, s);
-    case CQ_DTYPE_Q5_0: return launch(quantize_blk32<CQ_DTYPE_Q5_0>, nblocks, 1, src, aos_dev, s);
-    case CQ_DTYPE_Q5_1: return launch(quantize_blk32<CQ_DTYPE_Q5_1>, nblocks, 1, src, aos_dev, s);
-    case CQ_DTYPE_Q8_0: return launch(quantize_blk32<CQ_DTYPE_Q8_0>, nblocks, 1, src, aos_dev, s);
-    case CQ_DTYPE_Q4K: return launch(quantize_q4k<16>, nblocks, 8, src, aos_dev, s);
-    case CQ_DTYPE_Q5K: return launch(quantize_q4k<32>, nblocks, 8, src, aos_dev, s);
-    case CQ_DTYPE_Q2K: return launch(quantize_q2k, nblocks, 16, src, aos_dev, s);
-    case CQ_DTYPE_Q3K: return launch(quantize_q3k, nblocks, 16, src, aos_dev, s);
-    case CQ_DTYPE_Q6K: return launch(quantize_q6k, nblocks, 16, src, aos_dev, s);
-    // Q8K (k_quants.rs:1788-1825): the activation quantizer writing GGML blocks, one 256-element row per block
-    case CQ_DTYPE_Q8K: return cq_launch_quantize_act_aos(CQ_DTYPE_Q8K, src, nblocks, 256, cq_no_pre(), aos_dev, s);
+hipError_t cq_launch_quantize_weight(const cq_weight *w, const float *src, hipStream_t s) {
+    if (w->n == 0 || w->k == 0) return hipSuccess;
+    switch (w->ggml_dtype) {
+    case CQ_DTYPE_Q4_0: return launch(quantize_blk32<CQ_DTYPE_Q4_0>, w, 1, src, s);
+    case CQ_DTYPE_Q4_1: return launch(quantize_blk32<CQ_DTYPE_Q4_1>, w, 1, src, s);
+    case CQ_DTYPE_Q5_0: return launch(quantize_blk32<CQ_DTYPE_Q5_0>, w, 1, src, s);
+    case CQ_DTYPE_Q5_1: return launch(quantize_blk32<CQ_DTYPE_Q5_1>, w, 1, src, s);
+    case CQ_DTYPE_Q8_0: return launch(quantize_blk32<CQ_DTYPE_Q8_0>, w, 1, src, s);
+    case CQ_DTYPE_Q4K: return launch(quantize_q4k<16>, w, 8, src, s);
+    case CQ_DTYPE_Q5K: return launch(quantize_q4k<32>, w, 8, src, s);
+    case CQ_DTYPE_Q2K: return launch(quantize_q2k, w, 16, src, s);
+    case CQ_DTYPE_Q3K: return launch(quantize_q3k, w, 16, src, s);
+    case CQ_DTYPE_Q6K: return launch(quantize_q6k, w, 16, src, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -1,461 +1,112 @@
-// GGML array-of-blocks <-> device planes (and back).  Pure byte permutations:
+// GGML array-of-blocks <-> device planes (and back).  Pure byte permutations (repack_units.h):
 // cq_launch_unpack(cq_launch_repack(x)) == x for every input.
 //
 // Replaces the plain host->device copy of cuda::load_quantized
 // (candle-core/src/quantized/cuda.rs:591-612); the inverse serves QStorage::data
 // (mod.rs:118-130).
-#include "qhip_internal.h"
+#include "repack_units.h"
 
 namespace {
 
-// ---- Q4_0: 18-byte blocks {f16 d; u8 qs[16]} --------------------------------
-__global__ void repack_q4_0(const uint8_t *__restrict__ aos, uint8_t *__restrict__ qs, uint16_t *__restrict__ d,
-                            int64_t nblocks, bool inverse) {
-    int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nblocks) return;
-    uint16_t *a16 = (uint16_t *)(aos + b * 18);   // 18*b is even
-    uint16_t *q16 = (uint16_t *)(qs + b * 16);
-    if (!inverse) {
-        d[b] = a16[0];
-        for (int i = 0; i < 8; i++) q16[i] = a16[1 + i];
-    } else {
-        a16[0] = d[b];
-        for (int i = 0; i < 8; i++) a16[1 + i] = q16[i];
-    }
+template <int DT> __global__ void __launch_bounds__(256) repack_kernel(const uint8_t *__restrict__ aos, cq_planes pl, int64_t nblocks) {
+    constexpr int U = Ggml<DT>::kUnits;
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, b = t / U;
+    if (b < nblocks) repack_unit<DT, false>((uint8_t *)aos + b * Ggml<DT>::kSize, b, (int)(t - b * U), pl);
 }
 
-// ---- Q8_0: 34-byte blocks {f16 d; i8 qs[32]} --------------------------------
-__global__ void repack_q8_0(const uint8_t *__restrict__ aos, uint8_t *__restrict__ qs, uint16_t *__restrict__ d,
-                            int64_t nblocks, bool inverse) {
-    int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nblocks) return;
-    uint16_t *a16 = (uint16_t *)(aos + b * 34);
-    uint16_t *q16 = (uint16_t *)(qs + b * 32);
-    if (!inverse) {
-        d[b] = a16[0];
-        for (int i = 0; i < 16; i++) q16[i] = a16[1 + i];
-    } else {
-        a16[0] = d[b];
-        for (int i = 0; i < 16; i++) a16[1 + i] = q16[i];
-    }
+// Blocks first .. first + nblocks - 1 to `out`, which may be pinned host memory: the blocks are put together in LDS and leave in runs of
+// 16-byte stores, whatever their size.
+template <int DT> struct UnpackGroup { static constexpr int kBlocks = Ggml<DT>::kUnits == 1 ? 256 : 64; };
+template <int DT> __global__ void __launch_bounds__(256) unpack_kernel(cq_planes pl, int64_t first, int64_t nblocks, uint8_t *__restrict__ out) {
+    constexpr int U = Ggml<DT>::kUnits, TS = Ggml<DT>::kSize, PER = UnpackGroup<DT>::kBlocks;
+    static_assert(PER * TS % 16 == 0, "whole 16-byte groups");
+    __shared__ __align__(16) uint8_t img[PER * TS];
+    const int64_t g0 = (int64_t)blockIdx.x * PER;
+    const int count = (int)(nblocks - g0 < PER ? nblocks - g0 : PER);
+    for (int i = threadIdx.x; i < count * U; i += 256) repack_unit<DT, true>(img + i / U * TS, first + g0 + i / U, i % U, pl);
+    __syncthreads();
+    uint8_t *dst = out + g0 * TS;
+    const int whole = count * TS / 16;
+    for (int i = threadIdx.x; i < whole; i += 256) ((uint4 *)dst)[i] = ((const uint4 *)img)[i];
+    for (int i = whole * 8 + threadIdx.x; i < count * TS / 2; i += 256) ((uint16_t *)dst)[i] = ((const uint16_t *)img)[i];
 }
 
-// The 16 header bytes {f16 d; f16 dmin; u8 scales[12]} of a Q4K / Q5K block <-> the 20-byte device
-// record: the twelve bytes of 6-bit fields (utils.rs:49-59 get_scale_min_k4) unpacked to one byte
-// per field and grouped per 32 qs bytes, record g = {sc[2g], sc[2g+1], mn[2g], mn[2g+1]}; the
-// inverse packs them back (every one of the 96 bits is a field bit, so the round trip is exact).
-__device__ void k4_header(uint4 *a, uint32_t *h, bool inverse) {
-    if (!inverse) {
-        const uint4 v = *a;
-        h[0] = v.x;
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            int s0, m0, s1, m1;
-            cq_scale_min_k4(2 * g, v.y, v.z, v.w, s0, m0);
-            cq_scale_min_k4(2 * g + 1, v.y, v.z, v.w, s1, m1);
-            h[1 + g] = (uint32_t)s0 | ((uint32_t)s1 << 8) | ((uint32_t)m0 << 16) | ((uint32_t)m1 << 24);
-        }
-    } else {
-        uint32_t sc[8], mn[8];
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const uint32_t r = h[1 + g];
-            sc[2 * g] = r & 0xff; sc[2 * g + 1] = (r >> 8) & 0xff;
-            mn[2 * g] = (r >> 16) & 0xff; mn[2 * g + 1] = r >> 24;
-        }
-        uint32_t w[3] = {0, 0, 0};   // scales[0..3], scales[4..7], scales[8..11]
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            w[0] |= ((sc[j] & 63) | ((sc[j + 4] >> 4) << 6)) << (8 * j);
-            w[1] |= ((mn[j] & 63) | ((mn[j + 4] >> 4) << 6)) << (8 * j);
-            w[2] |= ((sc[j + 4] & 15) | ((mn[j + 4] & 15) << 4)) << (8 * j);
-        }
-        *a = make_uint4(h[0], w[0], w[1], w[2]);
-    }
+// The allocation as all-zero GGML blocks leave it: planes 0, 1 and 2 (16-byte groups up to their ends) of one byte each, zeros elsewhere.
+__global__ void __launch_bounds__(256) zero_planes_kernel(uint4 *__restrict__ base, int64_t groups, int64_t end0, int64_t from1, int64_t end1,
+                                                          int64_t from2, int64_t end2, uint32_t v0, uint32_t v1, uint32_t v2) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= groups) return;
+    const uint32_t v = i < end0 ? v0 : i >= from1 && i < end1 ? v1 : i >= from2 && i < end2 ? v2 : 0u;
+    base[i] = make_uint4(v, v, v, v);
 }
 
-// ---- Q4K: 144-byte blocks {f16 d; f16 dmin; u8 scales[12]; u8 qs[128]} ------
-// One thread per 16-byte unit: unit 0 is the header, units 1..8 the nibbles.
-__global__ void repack_q4k(const uint8_t *__restrict__ aos, uint8_t *__restrict__ qs, uint8_t *__restrict__ hd,
-                           int64_t nblocks, bool inverse) {
-    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t b = t / 9;
-    int u = (int)(t - b * 9);
-    if (b >= nblocks) return;
-    uint4 *a = (uint4 *)(aos + b * 144) + u;      // 144 = 9 * 16, base is 256-byte aligned
-    if (u != 0) {
-        uint4 *p = (uint4 *)(qs + b * 128) + (u - 1);
-        if (!inverse) *p = *a; else *a = *p;
-        return;
-    }
-    k4_header(a, (uint32_t *)(hd + b * CQ_Q4K_HDR), inverse);
-}
+cq_planes planes_of(const cq_weight *w) { return cq_planes{w->p0, w->p1, w->p2, w->p3, w->p4, w->p5}; }
 
-// ---- Q5K: 176-byte blocks {f16 d; f16 dmin; u8 scales[12]; u8 qh[32]; u8 qs[128]} ------
-// (k_quants.rs:119-127).  Header and nibbles as Q4K.  Bit j of qh[l] is the fifth bit of element
-// l of sub-block j, i.e. of the low (j even) or high (j odd) nibble of qs byte 32*(j/2) + l.  The
-// device plane holds, per 32 qs bytes g, two words L (sub-block 2g) and H (sub-block 2g+1) with
-//   bit 8c + i  =  fifth bit belonging to byte c of qs word i  (l = 4i + c),
-// so that (W >> i) & 0x01010101 lines the four bits up with the four nibbles of word i.
-// One thread per 16-byte unit of the block: 0 header, 1 the whole qh (32 bytes), 2 idle, 3..10 qs.
-__global__ void repack_q5k(const uint8_t *__restrict__ aos, uint8_t *__restrict__ qs, uint8_t *__restrict__ hd,
-                           uint8_t *__restrict__ qh, int64_t nblocks, bool inverse) {
-    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t b = t / 11;
-    int u = (int)(t - b * 11);
-    if (b >= nblocks) return;
-    uint4 *a = (uint4 *)(aos + b * 176) + u;      // 176 = 11 * 16, base is 256-byte aligned
-    if (u >= 3) {
-        uint4 *p = (uint4 *)(qs + b * 128) + (u - 3);
-        if (!inverse) *p = *a; else *a = *p;
-        return;
-    }
-    if (u == 2) return;
-    if (u == 1) {
-        uint4 *src = (uint4 *)(aos + b * 176 + 16);   // GGML qh[32]
-        uint4 *dst = (uint4 *)(qh + b * 32);          // {L, H} x 4
-        // bit 8c + i of L_g = bit 2g of byte c of word i, bit 8c + i of H_g = bit 2g + 1: a transpose in words, its own form both ways
-        const uint4 x0 = inverse ? dst[0] : src[0], x1 = inverse ? dst[1] : src[1];
-        const uint32_t in[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-        uint32_t out[8];
-#pragma unroll
-        for (int o = 0; o < 8; o++) {
-            out[o] = 0;
-#pragma unroll
-            for (int i = 0; i < 8; i++) out[o] |= ((in[i] >> o) & 0x01010101u) << i;
-        }
-        (inverse ? src : dst)[0] = make_uint4(out[0], out[1], out[2], out[3]);
-        (inverse ? src : dst)[1] = make_uint4(out[4], out[5], out[6], out[7]);
-        return;
-    }
-    k4_header(a, (uint32_t *)(hd + b * CQ_Q4K_HDR), inverse);
+template <int DT> hipError_t repack(const cq_weight *w, const uint8_t *aos, int64_t nblocks, hipStream_t s) {
+    hipLaunchKernelGGL(repack_kernel<DT>, dim3((unsigned)((nblocks * Ggml<DT>::kUnits + 255) / 256)), dim3(256), 0, s, aos, planes_of(w), nblocks);
+    return hipGetLastError();
 }
-
-// ---- Q6K: 210-byte blocks {u8 ql[128]; u8 qh[64]; i8 scales[16]; f16 d} -----
-// qh is re-ordered so that the thread that owns ql bytes [16u, 16u+16) of a block
-// finds the high bits of exactly those 32 elements in qh' bytes [8u, 8u+8):
-//   u = 4h + 2t + i  ->  ql byte 64h + 32t + 16i + e  (e < 16)
-//   low  nibble: element 128h + 32t + 16i + e        hi bits = qh[32h + 16i + e] >> 2t
-//   high nibble: element 128h + 64 + 32t + 16i + e   hi bits = qh[32h + 16i + e] >> (2t + 4)
-//   qh'[8u + 4x + c] (x < 2, c < 4) =   lo2(8x + c)       | hi2(8x + c) << 2
-//                                      | lo2(8x + 4 + c) << 4 | hi2(8x + 4 + c) << 6
-//   sc'[2u], sc'[2u + 1] = scales[js], scales[js + 4] with js = u + 4h: the scales of the lane's
-//   low-nibble and high-nibble 16-element groups, one 2-byte load per lane.
-// i.e. for the two ql words 2x and 2x+1 of the lane, (H >> {0,2,4,6}) & 0x03030303 lines the
-// two high bits up with each byte of {word 2x low, word 2x high, word 2x+1 low, word 2x+1 high}.
-__global__ void repack_q6k(const uint8_t *__restrict__ aos, uint8_t *__restrict__ ql, uint8_t *__restrict__ qh,
-                           uint8_t *__restrict__ sc, uint16_t *__restrict__ d, int64_t nblocks, bool inverse) {
-    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t b = t / 8;
-    int u = (int)(t & 7);
-    if (b >= nblocks) return;
-    uint8_t *a = (uint8_t *)aos + b * 210;
-    uint8_t *a_ql = a, *a_qh = a + 128, *a_sc = a + 192, *a_d = a + 208;
-    const int h = u >> 2, tt = (u >> 1) & 1, i0 = (u & 1) * 16;
-    uint8_t *pql = ql + b * 128 + 16 * u;
-    uint8_t *pqh = qh + b * 64 + 8 * u;
-    if (!inverse) {
-        for (int e = 0; e < 16; e++) pql[e] = a_ql[16 * u + e];
-        for (int x = 0; x < 2; x++)
-            for (int c = 0; c < 4; c++) {
-                uint8_t s0 = a_qh[32 * h + i0 + 8 * x + c];
-                uint8_t s1 = a_qh[32 * h + i0 + 8 * x + 4 + c];
-                uint8_t v = (uint8_t)(((s0 >> (2 * tt)) & 3) | (((s0 >> (2 * tt + 4)) & 3) << 2) |
-                                      (((s1 >> (2 * tt)) & 3) << 4) | (((s1 >> (2 * tt + 4)) & 3) << 6));
-                pqh[4 * x + c] = v;
-            }
-        // the lane's two 16-element scale groups (low nibbles: js, high nibbles: js + 4) side by side
-        const int js = u + 4 * h;
-        sc[b * 16 + 2 * u] = a_sc[js];
-        sc[b * 16 + 2 * u + 1] = a_sc[js + 4];
-        if (u == 0) d[b] = (uint16_t)(a_d[0] | (a_d[1] << 8));
-    } else {
-        for (int e = 0; e < 16; e++) a_ql[16 * u + e] = pql[e];
-        const int js = u + 4 * h;
-        a_sc[js] = sc[b * 16 + 2 * u];
-        a_sc[js + 4] = sc[b * 16 + 2 * u + 1];
-        if (u == 0) {
-            a_d[0] = (uint8_t)(d[b] & 0xff);
-            a_d[1] = (uint8_t)(d[b] >> 8);
-        }
-        // Each GGML qh byte 32h + j collects 2-bit fields from the two lanes t = 0, 1 that share
-        // (h, i); lane (h, t = 0, i) rebuilds the 16 bytes 32h + 16i + e from both lanes' qh'.
-        if (tt == 0) {
-            const uint8_t *p0 = qh + b * 64 + 8 * u;        // t = 0
-            const uint8_t *p1 = qh + b * 64 + 8 * (u + 2);  // t = 1
-            for (int x = 0; x < 2; x++)
-                for (int c = 0; c < 4; c++) {
-                    uint8_t v0 = p0[4 * x + c], v1 = p1[4 * x + c];
-                    // element e = 8x + c : fields lo2 (bits 0-1) and hi2 (bits 2-3)
-                    a_qh[32 * h + i0 + 8 * x + c] =
-                        (uint8_t)((v0 & 3) | ((v1 & 3) << 2) | (((v0 >> 2) & 3) << 4) | (((v1 >> 2) & 3) << 6));
-                    // element e = 8x + 4 + c : fields at bits 4-5 and 6-7
-                    a_qh[32 * h + i0 + 8 * x + 4 + c] = (uint8_t)(((v0 >> 4) & 3) | (((v1 >> 4) & 3) << 2) |
-                                                                  (((v0 >> 6) & 3) << 4) | (((v1 >> 6) & 3) << 6));
-                }
-        }
-    }
-}
-
-// ---- types held in another type's planes --------------------------------------------------------
-// Straight between the GGML blocks and the planes, in words of four quants: the blocks are read and written once and
-// nothing goes through the holding type's blocks in between.  Bound: HBM.  11008 x 4096 elements, per direction, byte loops
-// through a second set of blocks before -> now: Q3K 2581 + 12 -> 12 us, Q2K 2270 + 12 -> 9, Q5_0 / Q4_1 / Q5_1 18-20 + 15 -> 14.
-typedef uint32_t u32_any __attribute__((aligned(2)));                          // GGML blocks lie at even addresses
-typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
-__device__ __forceinline__ void load16(const uint8_t *p, uint32_t (&v)[4]) {
-    const u32x4_any x = *(const u32x4_any *)p;
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-}
-__device__ __forceinline__ void store16(uint8_t *p, const uint32_t (&v)[4]) {
-    u32x4_any x = {v[0], v[1], v[2], v[3]};
-    *(u32x4_any *)p = x;
-}
-// bits 4i .. 4i+3 of `bits` as bit 0 of the four bytes of a word, and back
-__device__ __forceinline__ uint32_t spread4(uint32_t bits, int i) {
-    const uint32_t n = (bits >> (4 * i)) & 15u;
-    return (n & 1u) | ((n & 2u) << 7) | ((n & 4u) << 14) | ((n & 8u) << 21);
-}
-__device__ __forceinline__ uint32_t gather4(uint32_t w, int i) {
-    return ((w & 1u) | ((w >> 7) & 2u) | ((w >> 14) & 4u) | ((w >> 21) & 8u)) << (4 * i);
-}
-
-// In Q8_0 planes, one thread per block:
-//   Q5_0 {f16 d; u8 qh[4]; u8 qs[16]} (k_quants.rs:61-67) holds d and 32 five-bit quants q, value d * (q - 16): exactly a
-//   Q8_0 block {f16 d; i8 qs[32]} with qs = q - 16, whose dequantization (k_quants.rs:568-584) and dot product with Q8_0
-//   activations (:631-649) are the arithmetic of Q5_0's (:428-451, :371-391) operation for operation.
-//   Q4_1 {f16 d; f16 m; u8 qs[16]} and Q5_1 {f16 d; f16 m; u8 qh[4]; u8 qs[16]} (k_quants.rs:51-57, :69-76), value
-//   d * q + m: the quants (0..15, 0..31) and d as a Q8_0 block, m into its own plane.
-template <int DT>
-__global__ void held_in_q8_0(uint8_t *__restrict__ aos, uint8_t *__restrict__ qs, uint16_t *__restrict__ d,
-                             uint16_t *__restrict__ mins, int64_t nblocks, bool inverse) {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nblocks) return;
-    constexpr bool FIVE = DT != CQ_DTYPE_Q4_1, MIN = DT != CQ_DTYPE_Q5_0;
-    constexpr int TS = DT == CQ_DTYPE_Q4_1 ? 20 : DT == CQ_DTYPE_Q5_0 ? 22 : 24, QH = MIN ? 4 : 2, QS = FIVE ? QH + 4 : QH;
-    constexpr uint32_t OFF = DT == CQ_DTYPE_Q5_0 ? 16 : 0;
-    uint8_t *x = aos + b * TS;
-    uint4 *p = (uint4 *)(qs + b * 32);
-    uint32_t lo[4], hi[4];
-    if (!inverse) {
-        uint32_t q[4];
-        load16(x + QS, q);
-        const uint32_t qh = FIVE ? *(const u32_any *)(x + QH) : 0u;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            lo[i] = q[i] & 0x0F0F0F0Fu;
-            hi[i] = (q[i] >> 4) & 0x0F0F0F0Fu;
-            if (FIVE) {
-                lo[i] |= spread4(qh, i) << 4;
-                hi[i] |= spread4(qh, 4 + i) << 4;
-            }
-            if (OFF) {   // byte - 16 for bytes 0..31: + 0xF0 in each byte without its carry
-                lo[i] = (lo[i] ^ 0x10101010u) | (((~lo[i] >> 4) & 0x01010101u) * 0xE0u);
-                hi[i] = (hi[i] ^ 0x10101010u) | (((~hi[i] >> 4) & 0x01010101u) * 0xE0u);
-            }
-        }
-        p[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-        p[1] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-        d[b] = *(const uint16_t *)x;
-        if (MIN) mins[b] = *(const uint16_t *)(x + 2);
-    } else {
-        const uint4 a = p[0], c = p[1];
-        lo[0] = a.x; lo[1] = a.y; lo[2] = a.z; lo[3] = a.w;
-        hi[0] = c.x; hi[1] = c.y; hi[2] = c.z; hi[3] = c.w;
-        uint32_t q[4], qh = 0;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            if (OFF) {   // the low five bits of q - 16 are those of q with the fifth flipped
-                lo[i] ^= 0x10101010u;
-                hi[i] ^= 0x10101010u;
-            }
-            q[i] = (lo[i] & 0x0F0F0F0Fu) | ((hi[i] & 0x0F0F0F0Fu) << 4);
-            if (FIVE) qh |= gather4(lo[i] >> 4, i) | gather4(hi[i] >> 4, 4 + i);
-        }
-        store16(x + QS, q);
-        if (FIVE) *(u32_any *)(x + QH) = qh;
-        *(uint16_t *)x = d[b];
-        if (MIN) *(uint16_t *)(x + 2) = mins[b];
-    }
-}
-
-// In Q6K planes, eight threads per block, thread u = 4h + 2t + i the unit u of the Q6K layout above (ql bytes 16u ..: the
-// elements 128h + 32t + 16i + e in the low and those 64 further on in the high nibbles):
-//   Q3K {u8 hmask[32]; u8 qs[64]; u8 scales[12]; f16 d} (k_quants.rs:107-114): sixteen groups of sixteen three-bit quants,
-//   value (d * (sc_j - 32)) * (q - 4) with six-bit sc_j: exactly a Q6K block {ql, qh, i8 scales[16], f16 d} with
-//   scales[j] = sc_j - 32 and six-bit quants q + 28 (so that q6 - 32 = q - 4), whose dequantization (k_quants.rs:1716-1746)
-//   and dot product with Q8K activations (:1585-1641) are those of Q3K (:1094-1146, :890-1009): the same integers, the
-//   same products in the same order.
-//   Q2K {u8 scales[16]; u8 qs[64]; f16 d; f16 dmin} (k_quants.rs:96-103): value (d * sc_j) * q - dmin * m_j, sc_j and m_j
-//   the nibbles of scales[j].  The first term is a Q6K block with scales sc_j and quants q + 32; m_j and dmin go to planes
-//   of their own.
-// Both hold the two low bits of four elements 32 apart in one byte of qs[32h + 16i ..], at 2 * (element / 32 % 4); Q3K's
-// third bit is bit element / 32 of hmask[16i ..].
-__device__ __forceinline__ int q3k_scale6(const uint8_t *sc, int j) {
-    const int low = j < 8 ? (sc[j] & 0xF) : (sc[j - 8] >> 4);
-    return low | (((sc[8 + j % 4] >> (2 * (j / 4))) & 3) << 4);
-}
-// the six-bit quants of unit u (16 in the low, 16 in the high nibbles) out of the planes
-__device__ __forceinline__ void q6_unit(const uint8_t *ql, const uint8_t *qh, int64_t b, int u, uint32_t (&lo)[4], uint32_t (&hi)[4]) {
-    const uint4 q = *(const uint4 *)(ql + b * 128 + 16 * u);
-    const uint2 H = *(const uint2 *)(qh + b * 64 + 8 * u);
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w}, hw[2] = {H.x, H.y};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t f = hw[i >> 1] >> (4 * (i & 1));
-        lo[i] = (qw[i] & 0x0F0F0F0Fu) | ((f & 0x03030303u) << 4);
-        hi[i] = ((qw[i] >> 4) & 0x0F0F0F0Fu) | (((f >> 2) & 0x03030303u) << 4);
-    }
-}
-template <int DT>
-__global__ void held_in_q6k(uint8_t *__restrict__ aos, uint8_t *__restrict__ ql, uint8_t *__restrict__ qh, uint8_t *__restrict__ sc,
-                            uint16_t *__restrict__ d, uint8_t *__restrict__ mins, uint16_t *__restrict__ dmins, int64_t nblocks,
-                            bool inverse) {
-    const int64_t t8 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, b = t8 >> 3;
-    if (b >= nblocks) return;
-    constexpr bool Q3 = DT == CQ_DTYPE_Q3K;
-    constexpr int TS = Q3 ? 110 : 84, QS = Q3 ? 32 : 16, D = Q3 ? 108 : 80;
-    constexpr uint32_t OFF = Q3 ? 0x1C1C1C1Cu : 0x20202020u;   // 28 or 32 in each byte
-    const int u = (int)(t8 & 7), h = u >> 2, t = (u >> 1) & 1, i16 = u & 1;
-    uint8_t *x = aos + b * TS;
-    if (!inverse) {
-        uint32_t q[4], m[4] = {0, 0, 0, 0}, out[4], lo[4], hi[4];
-        load16(x + QS + 32 * h + 16 * i16, q);
-        if (Q3) load16(x + 16 * i16, m);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            lo[i] = ((q[i] >> (2 * t)) & 0x03030303u) + OFF;
-            hi[i] = ((q[i] >> (2 * t + 4)) & 0x03030303u) + OFF;
-            if (Q3) {
-                lo[i] += ((m[i] >> (4 * h + t)) & 0x01010101u) << 2;
-                hi[i] += ((m[i] >> (4 * h + t + 2)) & 0x01010101u) << 2;
-            }
-            out[i] = (lo[i] & 0x0F0F0F0Fu) | ((hi[i] & 0x0F0F0F0Fu) << 4);
-            lo[i] = (lo[i] >> 4) & 0x03030303u;
-            hi[i] = (hi[i] >> 4) & 0x03030303u;
-        }
-        *(uint4 *)(ql + b * 128 + 16 * u) = make_uint4(out[0], out[1], out[2], out[3]);
-        *(uint2 *)(qh + b * 64 + 8 * u) = make_uint2(lo[0] | (hi[0] << 2) | (lo[1] << 4) | (hi[1] << 6),
-                                                    lo[2] | (hi[2] << 2) | (lo[3] << 4) | (hi[3] << 6));
-        const int js = u + 4 * h;
-        if (Q3) {
-            sc[b * 16 + 2 * u] = (uint8_t)(int8_t)(q3k_scale6(x + 96, js) - 32);
-            sc[b * 16 + 2 * u + 1] = (uint8_t)(int8_t)(q3k_scale6(x + 96, js + 4) - 32);
-        } else {
-            const uint8_t s0 = x[js], s1 = x[js + 4];
-            sc[b * 16 + 2 * u] = s0 & 0xF;
-            sc[b * 16 + 2 * u + 1] = s1 & 0xF;
-            mins[b * 16 + js] = s0 >> 4;
-            mins[b * 16 + js + 4] = s1 >> 4;
-        }
-        if (u == 0) {
-            d[b] = *(const uint16_t *)(x + D);
-            if (!Q3) dmins[b] = *(const uint16_t *)(x + D + 2);
-        }
-        return;
-    }
-    uint32_t lo[4], hi[4];
-    if (t == 0) {
-        // qs[32h + 16i ..]: the units t = 0 (quarters 0 and 2) and t = 1 (1 and 3)
-        uint32_t q[4], lo1[4], hi1[4];
-        q6_unit(ql, qh, b, u, lo, hi);
-        q6_unit(ql, qh, b, u + 2, lo1, hi1);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            q[i] = ((lo[i] - OFF) & 0x03030303u) | (((lo1[i] - OFF) & 0x03030303u) << 2) | (((hi[i] - OFF) & 0x03030303u) << 4) |
-                   (((hi1[i] - OFF) & 0x03030303u) << 6);
-        store16(x + QS + 32 * h + 16 * i16, q);
-    } else if (Q3 && h == 0) {
-        uint32_t m[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int v = 0; v < 4; v++) {   // the units of both halves and quarters with this i: bits 4h + t and 4h + t + 2
-            q6_unit(ql, qh, b, 2 * v + i16, lo, hi);
-            const int bit = 4 * (v >> 1) + (v & 1);
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                m[i] |= ((((lo[i] - OFF) >> 2) & 0x01010101u) << bit) | ((((hi[i] - OFF) >> 2) & 0x01010101u) << (bit + 2));
-        }
-        store16(x + 16 * i16, m);
-    } else if (u == 6) {   // h = 1, t = 1, i = 0: the scales (sc' holds group js = u + 4h at 2u and js + 4 at 2u + 1)
-        uint8_t s[16];
-#pragma unroll
-        for (int v = 0; v < 8; v++) {
-            s[v + 4 * (v >> 2)] = sc[b * 16 + 2 * v];
-            s[v + 4 * (v >> 2) + 4] = sc[b * 16 + 2 * v + 1];
-        }
-        if (Q3) {
-            uint8_t o[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const int lv = (int)(int8_t)s[j] + 32;
-                o[j & 7] |= (uint8_t)((lv & 0xF) << (j < 8 ? 0 : 4));
-                o[8 + j % 4] |= (uint8_t)((lv >> 4) << (2 * (j / 4)));
-            }
-#pragma unroll
-            for (int j = 0; j < 12; j++) x[96 + j] = o[j];
-        } else {
-#pragma unroll
-            for (int j = 0; j < 16; j++) x[j] = (uint8_t)((s[j] & 0xF) | (mins[b * 16 + j] << 4));
-        }
-    } else if (u == 7) {
-        *(uint16_t *)(x + D) = d[b];
-        if (!Q3) *(uint16_t *)(x + D + 2) = dmins[b];
-    }
-}
-
-hipError_t launch(const cq_weight *w, uint8_t *aos, bool inverse, hipStream_t s) {
-    const int64_t bs = cq_block_size(w->dtype);
-    const int64_t nblocks = w->n * (w->k / bs);
-    if (nblocks == 0) return hipSuccess;
-    const int threads = 256;
-    const unsigned per_block = (unsigned)((nblocks + threads - 1) / threads), per_unit = (unsigned)((nblocks * 8 + threads - 1) / threads);
-    uint16_t *p1 = (uint16_t *)w->p1, *p2 = (uint16_t *)w->p2, *p3 = (uint16_t *)w->p3, *p5 = (uint16_t *)w->p5;
-    switch (w->ggml_dtype) {
-    case CQ_DTYPE_Q5_0: held_in_q8_0<CQ_DTYPE_Q5_0><<<per_block, threads, 0, s>>>(aos, w->p0, p1, p2, nblocks, inverse); break;
-    case CQ_DTYPE_Q4_1: held_in_q8_0<CQ_DTYPE_Q4_1><<<per_block, threads, 0, s>>>(aos, w->p0, p1, p2, nblocks, inverse); break;
-    case CQ_DTYPE_Q5_1: held_in_q8_0<CQ_DTYPE_Q5_1><<<per_block, threads, 0, s>>>(aos, w->p0, p1, p2, nblocks, inverse); break;
-    case CQ_DTYPE_Q3K:
-        held_in_q6k<CQ_DTYPE_Q3K><<<per_unit, threads, 0, s>>>(aos, w->p0, w->p1, w->p2, p3, w->p4, p5, nblocks, inverse);
-        break;
-    case CQ_DTYPE_Q2K:
-        held_in_q6k<CQ_DTYPE_Q2K><<<per_unit, threads, 0, s>>>(aos, w->p0, w->p1, w->p2, p3, w->p4, p5, nblocks, inverse);
-        break;
-    case CQ_DTYPE_Q4_0: {
-        unsigned grid = (unsigned)((nblocks + threads - 1) / threads);
-        repack_q4_0<<<grid, threads, 0, s>>>(aos, w->p0, (uint16_t *)w->p1, nblocks, inverse);
-        break;
-    }
-    case CQ_DTYPE_Q8_0: {
-        unsigned grid = (unsigned)((nblocks + threads - 1) / threads);
-        repack_q8_0<<<grid, threads, 0, s>>>(aos, w->p0, (uint16_t *)w->p1, nblocks, inverse);
-        break;
-    }
-    case CQ_DTYPE_Q4K: {
-        unsigned grid = (unsigned)((nblocks * 9 + threads - 1) / threads);
-        repack_q4k<<<grid, threads, 0, s>>>(aos, w->p0, w->p1, nblocks, inverse);
-        break;
-    }
-    case CQ_DTYPE_Q5K: {
-        unsigned grid = (unsigned)((nblocks * 11 + threads - 1) / threads);
-        repack_q5k<<<grid, threads, 0, s>>>(aos, w->p0, w->p1, w->p2, nblocks, inverse);
-        break;
-    }
-    case CQ_DTYPE_Q6K: {
-        unsigned grid = (unsigned)((nblocks * 8 + threads - 1) / threads);
-        repack_q6k<<<grid, threads, 0, s>>>(aos, w->p0, w->p1, w->p2, (uint16_t *)w->p3, nblocks, inverse);
-        break;
-    }
-    case CQ_DTYPE_Q8K: return cq_launch_repack_q8k(w, aos, inverse, s);
-    default: return hipErrorInvalidValue;
-    }
+template <int DT> hipError_t unpack(const cq_weight *w, int64_t first, int64_t nblocks, uint8_t *out, hipStream_t s) {
+    constexpr int PER = UnpackGroup<DT>::kBlocks;
+    hipLaunchKernelGGL(unpack_kernel<DT>, dim3((unsigned)((nblocks + PER - 1) / PER)), dim3(256), 0, s, planes_of(w), first, nblocks, out);
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t cq_launch_repack(const cq_weight *w, const uint8_t *aos_dev, hipStream_t s) {
-    return launch(w, (uint8_t *)aos_dev, false, s);
+hipError_t cq_launch_zero_planes(const cq_weight *w, hipStream_t s) {
+    const int64_t groups = (int64_t)(w->alloc_bytes / 16), from1 = (w->p1 - w->p0) / 16, from2 = (w->p2 - w->p0) / 16, elems = w->n * w->k;
+    int64_t g0 = 0, g1 = 0, g2 = 0;   // 16-byte groups of the planes
+    uint32_t v0 = 0, v1 = 0, v2 = 0;
+    switch (w->ggml_dtype) {
+    case CQ_DTYPE_Q5_0: g0 = elems / 16; v0 = 0xf0f0f0f0u; break;                             // q - 16
+    case CQ_DTYPE_Q3K:                                                                        // six-bit quants q + 28, scales -32
+        g0 = elems / 32; v0 = 0xccccccccu;
+        g1 = elems / 64; v1 = 0x55555555u;
+        g2 = elems / 256; v2 = 0xe0e0e0e0u;
+        break;
+    case CQ_DTYPE_Q2K: g1 = elems / 64; v1 = 0xaaaaaaaau; break;                              // six-bit quants q + 32
+    default: break;
+    }
+    if (groups == 0) return hipSuccess;
+    hipLaunchKernelGGL(zero_planes_kernel, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, (uint4 *)w->base, groups, g0, from1, from1 + g1,
+                       from2, from2 + g2, v0, v1, v2);
+    return hipGetLastError();
 }
-hipError_t cq_launch_unpack(const cq_weight *w, uint8_t *aos_dev, hipStream_t s) {
-    return launch(w, aos_dev, true, s);
+
+hipError_t cq_launch_repack(const cq_weight *w, const uint8_t *aos_dev, hipStream_t s) {
+    const int64_t nb = w->n * (w->k / cq_block_size(w->dtype));
+    if (nb == 0) return hipSuccess;
+    switch (w->ggml_dtype) {
+    case CQ_DTYPE_Q4_0: return repack<CQ_DTYPE_Q4_0>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q4_1: return repack<CQ_DTYPE_Q4_1>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q5_0: return repack<CQ_DTYPE_Q5_0>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q5_1: return repack<CQ_DTYPE_Q5_1>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q8_0: return repack<CQ_DTYPE_Q8_0>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q2K: return repack<CQ_DTYPE_Q2K>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q3K: return repack<CQ_DTYPE_Q3K>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q4K: return repack<CQ_DTYPE_Q4K>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q5K: return repack<CQ_DTYPE_Q5K>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q6K: return repack<CQ_DTYPE_Q6K>(w, aos_dev, nb, s);
+    case CQ_DTYPE_Q8K: return cq_launch_repack_q8k(w, (uint8_t *)aos_dev, false, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+hipError_t cq_launch_unpack(const cq_weight *w, int64_t first, int64_t nblocks, uint8_t *aos, hipStream_t s) {
+    if (nblocks == 0) return hipSuccess;
+    switch (w->ggml_dtype) {
+    case CQ_DTYPE_Q4_0: return unpack<CQ_DTYPE_Q4_0>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q4_1: return unpack<CQ_DTYPE_Q4_1>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q5_0: return unpack<CQ_DTYPE_Q5_0>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q5_1: return unpack<CQ_DTYPE_Q5_1>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q8_0: return unpack<CQ_DTYPE_Q8_0>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q2K: return unpack<CQ_DTYPE_Q2K>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q3K: return unpack<CQ_DTYPE_Q3K>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q4K: return unpack<CQ_DTYPE_Q4K>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q5K: return unpack<CQ_DTYPE_Q5K>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q6K: return unpack<CQ_DTYPE_Q6K>(w, first, nblocks, aos, s);
+    case CQ_DTYPE_Q8K: return first == 0 ? cq_launch_repack_q8k(w, aos, true, s) : hipErrorInvalidValue;   // (all blocks)
+    default: return hipErrorInvalidValue;
+    }
 }

@@ -33,6 +33,21 @@ def test_same_bytes(qh, dt, nblocks):  # noqa: F811
     assert np.array_equal(guarded[1:blocks.size + 1], blocks) and guarded[0] == 7 and (guarded[blocks.size + 1:] == 7).all()
 
 
+@pytest.mark.parametrize("dt", [orc.Q4_1, orc.Q5_0, orc.Q5_1, orc.Q2K, orc.Q3K, orc.Q8_0, orc.Q6K])
+@pytest.mark.parametrize("nblocks", [1, 7, 300])
+def test_zeros_and_quantized_into_them(qh, dt, nblocks):  # noqa: F811
+    bs = orc.BLOCK_SIZE[dt]
+    w = qh.QWeight.zeros_flat(dt, nblocks * bs)
+    assert not w.to_ggml().any() and not w.dequantize().cpu().numpy().any()
+    x = np.random.default_rng(nblocks).standard_normal(nblocks * bs).astype(np.float32)
+    side = torch.cuda.Stream()
+    xd = torch.from_numpy(x).cuda()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        w.quantize_(xd)
+    assert np.array_equal(w.to_ggml(), orc.quantize(dt, x.reshape(1, -1)))
+
+
 def test_threads(qh):  # noqa: F811
     made = [weight(qh, orc.Q8_0, (6 + i) * MIB // 34, i) for i in range(3)]
     same = [0] * 3
