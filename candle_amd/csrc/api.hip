@@ -309,24 +309,26 @@ extern "C" int cq_weight_dequantize_f16(const cq_weight *w, uint16_t *dst_dev, v
 // new.  hipMemcpy itself pins and unpins the caller's pages.  Here the blocks go in pieces to pinned slots, written there by the kernel that
 // puts them together, and from the slots to the caller, by up to four threads, each with two slots of its own: one piece on its way over
 // the link, the other being copied.  The threads share nothing but the null stream, on which each launches its pieces.  The slots live for
-// the call, 8 MiB of them at most (allocating them takes some 50 us), so that nothing stays pinned after it.
+// the call, 16 MiB of them at most (allocating them takes some 50 us), so that nothing stays pinned after it.
 // us for a whole download, hipMemcpy from a device copy -> pieces: below 5 MiB hipMemcpy is as
 // fast, 11008 x 4096 Q4_0 25 MB 1440 -> 740, Q5K 31 MB 1740 -> 1030, Q6K 37 MB 3710 -> 1340, Q8_0 48 MB 4830 -> 1730 (one thread takes twice
 // that; pieces by the copy engine cost 10 us each more).
 namespace {
-constexpr size_t kPiece = 1 << 20;
 constexpr int kCopiers = 4;
+// Bytes of a slot: larger pieces are fewer launches and waits, smaller ones fill and drain the line sooner (quantize and download of
+// 11008 x 4096 with pieces of 0.5, 1 and 2 MiB: Q4K 1176, 1074 and 1007 us, Q6K 2330, 2100 and 1690).
+size_t slot_bytes(size_t bytes) { return bytes < (12u << 20) ? 1u << 20 : bytes < (24u << 20) ? bytes / 12 & ~(size_t)4095 : 2u << 20; }
 
 // Pieces me, me + of, ... through the two slots of `slots`.
-hipError_t copy_pieces(const cq_weight *w, uint8_t *dst, uint8_t *slots, int64_t me, int64_t of) {
-    const int64_t ts = cq_type_size(w->ggml_dtype), blocks = w->ggml_bytes / ts, piece = (int64_t)kPiece / ts / 256 * 256;
+hipError_t copy_pieces(const cq_weight *w, uint8_t *dst, uint8_t *slots, size_t slot_size, int64_t me, int64_t of) {
+    const int64_t ts = cq_type_size(w->ggml_dtype), blocks = w->ggml_bytes / ts, piece = (int64_t)slot_size / ts / 256 * 256;
     const int64_t n = (blocks + piece - 1) / piece;
     hipEvent_t landed[2] = {nullptr, nullptr};
     hipError_t e = hipSetDevice(w->dev);
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipEventCreateWithFlags(&landed[i], hipEventDisableTiming);
     const auto count = [&](int64_t c) { return blocks - c * piece < piece ? blocks - c * piece : piece; };
     const auto fetch = [&](int64_t c, int slot) {
-        const hipError_t f = cq_launch_unpack(w, c * piece, count(c), slots + slot * kPiece, nullptr);
+        const hipError_t f = cq_launch_unpack(w, c * piece, count(c), slots + slot * slot_size, nullptr);
         return f == hipSuccess ? hipEventRecord(landed[slot], nullptr) : f;
     };
     for (int i = 0; i < 2 && e == hipSuccess; i++)
@@ -335,7 +337,7 @@ hipError_t copy_pieces(const cq_weight *w, uint8_t *dst, uint8_t *slots, int64_t
     for (int64_t c = me; c < n && e == hipSuccess; c += of, slot ^= 1) {
         e = hipEventSynchronize(landed[slot]);
         if (e != hipSuccess) break;
-        memcpy(dst + c * piece * ts, slots + slot * kPiece, (size_t)(count(c) * ts));
+        memcpy(dst + c * piece * ts, slots + slot * slot_size, (size_t)(count(c) * ts));
         if (c + 2 * of < n) e = fetch(c + 2 * of, slot);
     }
     for (hipEvent_t ev : landed)
@@ -343,10 +345,10 @@ hipError_t copy_pieces(const cq_weight *w, uint8_t *dst, uint8_t *slots, int64_t
     return e;
 }
 
-hipError_t copy_by_threads(const cq_weight *w, uint8_t *dst, uint8_t *slots) {
+hipError_t copy_by_threads(const cq_weight *w, uint8_t *dst, uint8_t *slots, size_t slot_size) {
     hipError_t err[kCopiers];
     std::thread helpers[kCopiers];
-    const auto work = [&](int t) { err[t] = copy_pieces(w, dst, slots + 2 * t * kPiece, t, kCopiers); };
+    const auto work = [&](int t) { err[t] = copy_pieces(w, dst, slots + 2 * t * slot_size, slot_size, t, kCopiers); };
     for (int t = 1; t < kCopiers; t++) {
         try {
             helpers[t] = std::thread(work, t);
@@ -376,9 +378,9 @@ extern "C" int cq_weight_to_ggml(const cq_weight *w, void *host_dst, size_t nbyt
         return hipPointerGetAttributes(&attr, host_dst) == hipSuccess && attr.type == hipMemoryTypeHost;
     };
     void *slots = nullptr;
-    if (e == hipSuccess && nbytes >= 5 * kPiece && w->dtype != CQ_DTYPE_Q8K && !pinned() &&
-        hipHostMalloc(&slots, 2 * kCopiers * kPiece, hipHostMallocDefault) == hipSuccess) {
-        e = copy_by_threads(w, (uint8_t *)host_dst, (uint8_t *)slots);
+    if (e == hipSuccess && nbytes >= (5u << 20) && w->dtype != CQ_DTYPE_Q8K && !pinned() &&
+        hipHostMalloc(&slots, 2 * kCopiers * slot_bytes(nbytes), hipHostMallocDefault) == hipSuccess) {
+        e = copy_by_threads(w, (uint8_t *)host_dst, (uint8_t *)slots, slot_bytes(nbytes));
         (void)hipHostFree(slots);
         (void)hipGetLastError();   // (a pointer unknown to HIP is an error on some versions)
     } else {
