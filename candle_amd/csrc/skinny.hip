@@ -239,7 +239,7 @@ __device__ __forceinline__ void quantize_direct(const float4 (&xf)[2 * RT][4], c
 // DUMP (verification): the block integers, and the min term as the f16 MFMA delivers it from a zero accumulator,
 // are stored through `dump` instead of the result through `y`.
 // DIRECT: the rows come as f32 from `x` and every wave quantizes the blocks it contracts (see skinny_direct_kernel).
-template <int DT, int RT, bool DUMP, bool DIRECT = false>
+template <int DT, int RT, bool DUMP, bool DIRECT = false, int NW = kWaves>
 __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
                                             float *__restrict__ y, cq_mfma_dump dump, const float *__restrict__ x = nullptr) {
     typedef Buf<DT, RT> B;
@@ -275,7 +275,7 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
 #pragma unroll
     for (int t = 0; t < NT; t++) out[t] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
 
-    for (int64_t b = wave; b < kb; b += kWaves) {
+    for (int64_t b = wave; b < kb; b += NW) {
         // ---- copies of block b: weights of the 16 rows, activation rows, their scales
         float4 xf[DIRECT ? 2 * RT : 1][4];
         if constexpr (DIRECT) {
@@ -290,7 +290,8 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
 #pragma unroll
         for (int i = 0; i < 2 * RT; i++) {
             const int rg = i >> 1, kh = i & 1;
-            dma16(a.qs + (m0 + rg * 8) * k + b * 256 + kh * 128, act_off, buf + B::oAct + i * 1024);
+            if (RT > 1 || (int64_t)r8 < m - m0)   // (few rows: the others' copies are most of the activations')
+                dma16(a.qs + (m0 + rg * 8) * k + b * 256 + kh * 128, act_off, buf + B::oAct + i * 1024);
         }
         if (lane < 8 * RT) dma4(a.dT + b * a.m_stride + m0, lane * 4u, buf + B::oD8);
         if (MINS && lane < 16 * RT) dma16(a.bsh + (b * a.m_stride + m0) * 16, lane * 16u, buf + B::oMin);
@@ -361,7 +362,7 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
     if (wave < NT) {
         v4f s = *(const v4f *)(smem + wave * 1024 + lane * 16);
 #pragma unroll
-        for (int o = 1; o < kWaves; o++) {
+        for (int o = 1; o < NW; o++) {
             const v4f p = *(const v4f *)(smem + o * B::kBytes + wave * 1024 + lane * 16);
             s += p;
         }
@@ -374,10 +375,10 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
     }
 }
 
-template <int DT, int RT, bool DUMP>
-__global__ void __launch_bounds__(kThreads) skinny_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
+template <int DT, int RT, bool DUMP, int NW = kWaves>
+__global__ void __launch_bounds__(NW * 64) skinny_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
                                                           cq_mfma_dump dump) {
-    skinny_body<DT, RT, DUMP>(w, a, blockIdx.x, m0, m, y, dump);
+    skinny_body<DT, RT, DUMP, false, NW>(w, a, blockIdx.x, m0, m, y, dump);
 }
 
 // ------------------------------------------------------------ resident-activation variant ----
@@ -648,14 +649,51 @@ template <int DT, int RT> struct ResMulti {
     static size_t bytes(int64_t kb) { return (size_t)kb * Res<DT, RT>::kActBlk + (size_t)kb * 2 * kSlot; }
 };
 
+constexpr int kMultiMax = 3;
+struct MultiArgs {
+    cq_weight w[kMultiMax];
+    float *y[kMultiMax];
+    uint32_t first[kMultiMax];   // first tile of the launch that is the weight's
+};
+// Where a tile of the launch lies: its weight's planes and first row.  One weight, or two or three with the same rows (skinny_shared_kernel).
+struct TileAt {
+    const uint8_t *p0, *p1, *p2;
+    float *y;
+    int64_t n;
+    uint32_t row;
+};
+struct OneWeight {
+    const cq_weight &w;
+    float *y;
+    __device__ int64_t k() const { return w.k; }
+    __device__ int64_t tiles() const { return (w.n + 15) / 16; }
+    __device__ TileAt at(int64_t t) const { return {w.p0, w.p1, w.p2, y, w.n, (uint32_t)tile_row(t, w.n)}; }
+};
+struct SomeWeights {
+    const MultiArgs &ma;
+    uint32_t total;
+    __device__ int64_t k() const { return ma.w[0].k; }
+    __device__ int64_t tiles() const { return total; }
+    __device__ TileAt at(int64_t t) const {
+        const bool b = t >= ma.first[1], c = t >= ma.first[2];
+        const auto pick = [&](auto x, auto y, auto z) { return c ? z : b ? y : x; };
+        const int64_t n = pick(ma.w[0].n, ma.w[1].n, ma.w[2].n);
+        return {pick(ma.w[0].p0, ma.w[1].p0, ma.w[2].p0), pick(ma.w[0].p1, ma.w[1].p1, ma.w[2].p1), pick(ma.w[0].p2, ma.w[1].p2, ma.w[2].p2),
+                pick(ma.y[0], ma.y[1], ma.y[2]), n, (uint32_t)tile_row(t - pick(ma.first[0], ma.first[1], ma.first[2]), n)};
+    }
+};
+
 // The copies of one tile's K block b into `slot`: weights as res_issue_weights, then the 16 rows' headers
 // (bytes 0..15 of row r at oHdr + 16 r, bytes 16..19 at oHdr + 256 + 4 r; lanes 0..15).
 template <int DT, int RT>
-__device__ __forceinline__ void multi_issue(uint8_t *__restrict__ slot, const ResPlanes &pl, __amdgpu_buffer_rsrc_t hdr, uint32_t n_tile,
-                                            uint32_t b, uint32_t kb, uint32_t wq_off, uint32_t w5_off, uint32_t hd_off, int lane) {
+__device__ __forceinline__ void multi_issue(uint8_t *__restrict__ slot, const TileAt &at, uint32_t b, uint32_t kb, uint32_t wq_off, uint32_t w5_off, uint32_t hd_off, int lane) {
     typedef ResMulti<DT, RT> M;
-    res_issue_weights<DT>(slot, pl, n_tile, b, kb, wq_off, 0, w5_off, lane);
-    const uint32_t blk = n_tile * kb + b;
+    ResPlanes pl;
+    pl.wq = wave_rsrc(at.p0);
+    pl.w5 = wave_rsrc(at.p2);
+    const __amdgpu_buffer_rsrc_t hdr = wave_rsrc(at.p1);
+    res_issue_weights<DT>(slot, pl, at.row, b, kb, wq_off, 0, w5_off, lane);
+    const uint32_t blk = at.row * kb + b;
     if (lane < 16) {
         dma16s(hdr, hd_off, blk * (uint32_t)CQ_Q4K_HDR, slot + M::oHdr);
         // (the instruction's immediate offset moves both addresses: bytes 16.. of the header, and 16 bytes on in LDS)
@@ -665,8 +703,8 @@ __device__ __forceinline__ void multi_issue(uint8_t *__restrict__ slot, const Re
 
 // One tile of one wave: operands out of `slot`, then (the slot is free) the copies of the tile two ahead, then the MFMAs.
 template <int DT, int RT, bool DUMP>
-__device__ __forceinline__ void multi_step(uint8_t *__restrict__ slot, const uint8_t *__restrict__ act, int lane, const ResPlanes &pl,
-                                           __amdgpu_buffer_rsrc_t hdr, bool ahead, uint32_t rows_ahead, uint32_t b, uint32_t kb32,
+__device__ __forceinline__ void multi_step(uint8_t *__restrict__ slot, const uint8_t *__restrict__ act, int lane, bool ahead,
+                                           const TileAt &next, uint32_t b, uint32_t kb32,
                                            uint32_t wq_off, uint32_t w5_off, uint32_t hd_off, const uint32_t (&a_col)[1][2],
                                            v4f (&out)[1], const cq_mfma_dump &dump, int64_t at, int64_t rs, int64_t m) {
     typedef ResMulti<DT, RT> M;
@@ -679,15 +717,14 @@ __device__ __forceinline__ void multi_step(uint8_t *__restrict__ slot, const uin
     res_unpack<DT, DUMP>(slot, lane, head, dump, o);
     if (ahead) {
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the reads above are done with the slot
-        multi_issue<DT, RT>(slot, pl, hdr, rows_ahead, b, kb32, wq_off, w5_off, hd_off, lane);
+        multi_issue<DT, RT>(slot, next, b, kb32, wq_off, w5_off, hd_off, lane);
     }
     res_mac<DT, RT, 1, DUMP>(act, lane, o, a_col, out, dump, at, rs, m);
 }
 
 // m <= 8 * RT <= 16 activation rows; n >= 16; k / 256 <= kWaves.
-template <int DT, int RT, int kWaves, bool DUMP>
-__global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_weight w, cq_act_view a, int64_t m,
-                                                                            float *__restrict__ y, cq_mfma_dump dump) {
+template <int DT, int RT, int kWaves, bool DUMP, typename Set>
+__device__ __forceinline__ void resident_rounds(const Set &set, const cq_act_view &a, int64_t m, const cq_mfma_dump &dump) {
     typedef Res<DT, RT> R;
     typedef ResMulti<DT, RT> M;
     static_assert(DT == CQ_DTYPE_Q4K || DT == CQ_DTYPE_Q5K, "block headers of 20 bytes");
@@ -699,8 +736,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
-    const int64_t k = w.k, kb = w.k >> 8;
-    const int64_t tiles = (w.n + 15) / 16, G = gridDim.x;
+    const int64_t k = set.k(), kb = k >> 8;
+    const int64_t tiles = set.tiles(), G = gridDim.x;
     uint8_t *wgt_base = smem + kb * R::kActBlk;
     const bool has = wave < kb;   // this wave owns K block `wave`
     const uint32_t b = (uint32_t)wave;
@@ -717,13 +754,9 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
         for (uint32_t e = 0; e < 2; e++) a_col[0][e] = (row >> 3) * 2048u + (row & 7) * 128u + (((4 * e + kq) ^ (row & 7)) << 4);
     }
     ResPlanes pl;
-    pl.wq = wave_rsrc(w.p0);
-    pl.wh = wave_rsrc(w.p1);
-    pl.w5 = wave_rsrc(w.p2);
     pl.aq = wave_rsrc(a.qs);
     pl.ad = wave_rsrc(a.dT);
     pl.am = wave_rsrc(a.bsh);
-    const __amdgpu_buffer_rsrc_t hdr = wave_rsrc(w.p1);
     const uint32_t kb32 = (uint32_t)kb, k32 = (uint32_t)k, mstr = (uint32_t)a.m_stride;
     uint8_t *act = smem + b * R::kActBlk;
     uint8_t *ring = wgt_base + (size_t)b * 2 * M::kSlot;
@@ -744,8 +777,8 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
         cnt = cnt < kTilesPerRound ? cnt : kTilesPerRound;
         if (has) {
             v4f o0 = {0.0f, 0.0f, 0.0f, 0.0f}, o1 = o0, o2 = o0, o3 = o0;
-            multi_issue<DT, RT>(ring, pl, hdr, (uint32_t)tile_row(t0, w.n), b, kb32, wq_off, w5_off, hd_off, lane);
-            if (cnt > 1) multi_issue<DT, RT>(ring + M::kSlot, pl, hdr, (uint32_t)tile_row(t0 + G, w.n), b, kb32, wq_off, w5_off, hd_off, lane);
+            multi_issue<DT, RT>(ring, set.at(t0), b, kb32, wq_off, w5_off, hd_off, lane);
+            if (cnt > 1) multi_issue<DT, RT>(ring + M::kSlot, set.at(t0 + G), b, kb32, wq_off, w5_off, hd_off, lane);
 #pragma nounroll
             for (int i = 0; i < cnt; i++) {
                 // everything but the copies of the next tile has landed
@@ -753,8 +786,9 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
                 else __builtin_amdgcn_s_waitcnt(0x0F70);
                 const int64_t tile = t0 + i * G;
                 v4f acc[1] = {{0.0f, 0.0f, 0.0f, 0.0f}};
-                multi_step<DT, RT, DUMP>(ring + (i & 1) * M::kSlot, act, lane, pl, hdr, i + 2 < cnt, (uint32_t)tile_row(tile + 2 * G, w.n), b, kb32,
-                                         wq_off, w5_off, hd_off, a_col, acc, dump, (tile_row(tile, w.n) + r) * kb + b, w.n * kb, m);
+                const TileAt here = set.at(tile);   // (for the dump)
+                multi_step<DT, RT, DUMP>(ring + (i & 1) * M::kSlot, act, lane, i + 2 < cnt, set.at(i + 2 < cnt ? tile + 2 * G : tile), b, kb32, wq_off,
+                                         w5_off, hd_off, a_col, acc, dump, ((int64_t)here.row + r) * kb + b, here.n * kb, m);
                 // (i is wave-uniform: real branches, four moves, instead of sixteen selects - the empty statements keep them)
                 if (i == 0) { o0 = acc[0]; asm volatile(""); }
                 else if (i == 1) { o1 = acc[0]; asm volatile(""); }
@@ -775,15 +809,23 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_w
                 const v4f p = *(const v4f *)(wgt_base + (size_t)o * 2 * M::kSlot + wave * 1024 + lane * 16);
                 s += p;
             }
-            const int64_t col = tile_row(t0 + wave * G, w.n) + r;
+            const TileAt at = set.at(t0 + wave * G);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int64_t row = kq * 4 + i;
-                if (row < m) y[row * w.n + col] = s[i];
+                if (row < m) at.y[row * at.n + at.row + r] = s[i];
             }
         }
         if (t0 + kTilesPerRound * G < tiles) __syncthreads();   // the sums have been read: the slots take the next round's copies
     }
+}
+template <int DT, int RT, int kWaves, bool DUMP>
+__global__ void __launch_bounds__(kWaves * 64) skinny_resident_multi_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
+                                                                            cq_mfma_dump dump) {
+    resident_rounds<DT, RT, kWaves, DUMP>(OneWeight{w, y}, a, m, dump);
+}
+__global__ void __launch_bounds__(16 * 64) skinny_shared_rounds_kernel(MultiArgs ma, uint32_t tiles, cq_act_view a, int64_t m) {
+    resident_rounds<CQ_DTYPE_Q4K, 2, 16, false>(SomeWeights{ma, tiles}, a, m, cq_mfma_dump{nullptr, nullptr, 0});
 }
 
 // ---------------------------------------------------- Q8_0 / Q4_0 weights x Q8_0 activations ----
@@ -873,7 +915,7 @@ __device__ __forceinline__ void quantize_direct_q8(const float4 (&xf)[8 * RT], c
     }
 }
 
-template <int DT, int RT, bool DUMP, bool DIRECT = false>
+template <int DT, int RT, bool DUMP, bool DIRECT = false, int NW = kWaves>
 __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
                                                   float *__restrict__ y, cq_mfma_dump dump, const float *__restrict__ x = nullptr) {
     typedef BufQ8<DT, RT> B;
@@ -911,7 +953,7 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
 #pragma unroll
     for (int t = 0; t < NT; t++) out[t] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
 
-    for (int64_t g = wave; g < kg; g += kWaves) {
+    for (int64_t g = wave; g < kg; g += NW) {
         float4 xf[DIRECT ? 8 * RT : 1];
         if constexpr (DIRECT) {
             load_direct_q8<RT>(x, m, k, g, lane, xf);
@@ -931,7 +973,8 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
 #pragma unroll
         for (int i = 0; i < 2 * RT; i++) {
             const int rg = i >> 1, kh = i & 1;
-            dma16(a.qs + (m0 + rg * 8) * k + g * 256 + kh * 128, row_off, buf + B::oAct + i * 1024);
+            if (RT > 1 || (int64_t)r8 < m - m0)   // (few rows: the others' copies are most of the activations')
+                dma16(a.qs + (m0 + rg * 8) * k + g * 256 + kh * 128, row_off, buf + B::oAct + i * 1024);
         }
         issue_scales<RT>(a, m0, g, buf + B::oD8, lane);
         }
@@ -974,7 +1017,7 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
     if (wave < NT) {
         v4f s = *(const v4f *)(smem + wave * 1024 + lane * 16);
 #pragma unroll
-        for (int o = 1; o < kWaves; o++) {
+        for (int o = 1; o < NW; o++) {
             const v4f p = *(const v4f *)(smem + o * B::kBytes + wave * 1024 + lane * 16);
             s += p;
         }
@@ -987,10 +1030,10 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
     }
 }
 
-template <int DT, int RT, bool DUMP>
-__global__ void __launch_bounds__(kThreads) skinny_blk32_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
+template <int DT, int RT, bool DUMP, int NW = kWaves>
+__global__ void __launch_bounds__(NW * 64) skinny_blk32_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
                                                                 cq_mfma_dump dump) {
-    skinny_blk32_body<DT, RT, DUMP>(w, a, blockIdx.x, m0, m, y, dump);
+    skinny_blk32_body<DT, RT, DUMP, false, NW>(w, a, blockIdx.x, m0, m, y, dump);
 }
 
 // Mixture-of-experts form of the two: blockIdx.y is a tile of up to 8 * RT routed rows and names its expert's weights, so
@@ -1007,12 +1050,6 @@ __global__ void __launch_bounds__(kThreads) skinny_grouped_kernel(cq_group_args 
 
 // Two or three weights on the same rows (q, k, v; gate and up): their 16-row tiles one after the other.  A weight with few
 // rows (1024: 64 workgroups) does not fill the machine by itself.
-constexpr int kMultiMax = 3;
-struct MultiArgs {
-    cq_weight w[kMultiMax];
-    float *y[kMultiMax];
-    uint32_t first[kMultiMax];   // first tile of the launch that is the weight's
-};
 template <int DT, int RT>
 __global__ void __launch_bounds__(kThreads) skinny_shared_kernel(MultiArgs ma, cq_act_view a, int64_t m) {
     const uint32_t t = blockIdx.x;
@@ -1382,12 +1419,27 @@ bool launch_blk32_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq
 }
 
 // DUMP (all launchers below): the launch cq_launch_skinny would make, storing the block integers through `d`.
+// Sixteen waves to a workgroup instead of eight, for rows too long for the resident kernels: with a workgroup or less a CU, eight waves with a
+// block each in flight leave the memory idle.  Measured, whole calls in us, eight waves -> sixteen, 4 and 8 rows: 4096 x 14336 Q4K 15.2 -> 13.6
+// and 15.4 -> 14.6, Q4_0 16.0 -> 13.0 and 16.2 -> 13.8, Q6K 17.3 -> 16.2 and 17.5 -> 17.3; 2048 x 11008 Q4K 12.2 -> 10.7, Q4_0 13.2 -> 10.6.  Not
+// for Q8_0, whose blocks are twice as long (4096 x 14336 18.1 -> 18.6), from nine rows on (Q4K 16.2 -> 17.3), or with more workgroups than CUs
+// (8192 x 8192 Q6K 18.9 -> 20.9, Q4_0 14.8 -> 15.8).
+template <int DT, int RT> bool sixteen_waves(const cq_weight *w) {
+    return RT == 1 && DT != CQ_DTYPE_Q8_0 && w->k > 8 * QK_K && (w->n + 15) / 16 <= cq_num_cus();
+}
+
+template <int DT, int RT, bool DUMP, int NW>
+hipError_t launch_blk32_waves(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
+    const size_t lds = (size_t)BufQ8<DT, RT>::kBytes * NW;
+    if (hipError_t e = cq_ensure_lds<skinny_blk32_kernel<DT, RT, DUMP, NW>>(w->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_blk32_kernel<DT, RT, DUMP, NW>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m0, m, y, d);
+    return hipGetLastError();
+}
 template <int DT, int RT, bool DUMP>
 hipError_t launch_blk32_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    const size_t lds = (size_t)BufQ8<DT, RT>::kBytes * kWaves;
-    if (hipError_t e = cq_ensure_lds<skinny_blk32_kernel<DT, RT, DUMP>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_blk32_kernel<DT, RT, DUMP>), (unsigned)((w->n + 15) / 16), kThreads, lds, s, *w, a, m0, m, y, d);
-    return hipGetLastError();
+    if constexpr (RT == 1 && DT != CQ_DTYPE_Q8_0 && !DUMP)
+        if (sixteen_waves<DT, RT>(w)) return launch_blk32_waves<DT, RT, DUMP, 16>(w, a, m0, m, y, d, s);
+    return launch_blk32_waves<DT, RT, DUMP, kWaves>(w, a, m0, m, y, d, s);
 }
 
 template <int DT, bool DUMP>
@@ -1404,12 +1456,18 @@ hipError_t launch_blk32(const cq_weight *w, cq_act_view a, int64_t m, float *y, 
     return hipSuccess;
 }
 
+template <int DT, int RT, bool DUMP, int NW>
+hipError_t launch_waves(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
+    const size_t lds = (size_t)Buf<DT, RT>::kBytes * NW;
+    if (hipError_t e = cq_ensure_lds<skinny_kernel<DT, RT, DUMP, NW>>(w->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_kernel<DT, RT, DUMP, NW>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m0, m, y, d);
+    return hipGetLastError();
+}
 template <int DT, int RT, bool DUMP>
 hipError_t launch_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    const size_t lds = (size_t)Buf<DT, RT>::kBytes * kWaves;
-    if (hipError_t e = cq_ensure_lds<skinny_kernel<DT, RT, DUMP>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_kernel<DT, RT, DUMP>), (unsigned)((w->n + 15) / 16), kThreads, lds, s, *w, a, m0, m, y, d);
-    return hipGetLastError();
+    if constexpr (RT == 1 && DT != CQ_DTYPE_Q8_0 && !DUMP)
+        if (sixteen_waves<DT, RT>(w)) return launch_waves<DT, RT, DUMP, 16>(w, a, m0, m, y, d, s);
+    return launch_waves<DT, RT, DUMP, kWaves>(w, a, m0, m, y, d, s);
 }
 
 template <int DT, bool DUMP>
@@ -1494,7 +1552,26 @@ hipError_t launch_shared_rt(const MultiArgs &ma, unsigned tiles, cq_act_view a, 
     CQ_LAUNCH((skinny_shared_kernel<DT, RT>), tiles, kThreads, lds, s, ma, a, m);
     return hipGetLastError();
 }
+// Nine rows and more of Q4K with nine to sixteen blocks a row: by rounds of tiles over all the weights, as launch_res_rt does for one.  Measured
+// with rms_norm in front, whole calls in us, tile by tile (for many rows a launch for each weight) -> rounds, 16 rows: 3 x 4096 x 4096 17.1 -> 15.1,
+// 4096 + 1024 + 1024 x 4096 13.7 -> 12.2, 2 x 6912 x 2560 14.3 -> 13.9, 2 x 14336 x 4096 28.0 -> 27.9, 2 x 28672 40.0 -> 40.0.  Not with up to eight
+// rows (3 x 4096 x 4096, 4 rows 14.3 -> 14.9, 2 x 14336 22.1 -> 24.2: more workgroups share a CU) and not for Q5K (16 rows, 2 x 14336 32.0 -> 32.0,
+// 2 x 6912 x 2560 17.3 -> 17.5).
+bool shared_by_rounds(const MultiArgs &ma, const cq_act_view &a, int64_t m) {
+    const int64_t kb = ma.w[0].k >> 8;
+    for (const cq_weight &w : ma.w)
+        if ((uint64_t)w.n * (uint64_t)kb * 128u >= (1ull << 32)) return false;   // (32-bit byte offsets)
+    return m > 8 && kb > 8 && kb <= 16 && ResMulti<CQ_DTYPE_Q4K, 2>::bytes(kb) <= (size_t)kMaxLds && (uint64_t)a.m_stride * (uint64_t)ma.w[0].k < (1ull << 32);
+}
+hipError_t launch_shared_rounds(const MultiArgs &ma, unsigned tiles, cq_act_view a, int64_t m, hipStream_t s) {
+    const size_t lds = ResMulti<CQ_DTYPE_Q4K, 2>::bytes(ma.w[0].k >> 8);
+    if (hipError_t e = cq_ensure_lds<skinny_shared_rounds_kernel>(ma.w[0].dev, lds); e != hipSuccess) return e;
+    const unsigned cus = (unsigned)cq_num_cus();
+    CQ_LAUNCH(skinny_shared_rounds_kernel, tiles < cus ? tiles : cus, 16 * 64, lds, s, ma, tiles, a, m);
+    return hipGetLastError();
+}
 template <int DT> hipError_t launch_shared(const MultiArgs &ma, unsigned tiles, cq_act_view a, int64_t m, hipStream_t s) {
+    if (DT == CQ_DTYPE_Q4K && shared_by_rounds(ma, a, m)) return launch_shared_rounds(ma, tiles, a, m, s);
     return m <= 8 ? launch_shared_rt<DT, 1>(ma, tiles, a, m, s) : launch_shared_rt<DT, 2>(ma, tiles, a, m, s);
 }
 
@@ -1607,26 +1684,15 @@ hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_exper
     }
 }
 
-// One launch over all the weights, or a launch each.  Measured with rms_norm in front, weights from HBM, five types, 2..16 rows,
+// One launch over all the weights rather than a launch each.  Measured with rms_norm in front, weights from HBM, five types, 2..16 rows,
 // ten pairs and triples from 1024 to 28672 weight rows and K = 1024..8192 (us of the whole call, one launch / a launch each):
 // the one launch is ahead everywhere (Q4K, 8 rows: 4096 + 1024 + 1024 x 4096 12.2 / 18.9, 2 x 14336 x 4096 24.3 / 26.8, 2 x 28672
-// x 8192 77.5 / 82.7; 16 rows: Q6K 2 x 14336 x 4096 32.2 / 37.2, Q8_0 2 x 11008 x 4096 31.2 / 31.8) but for nine rows and more of
-// many Q4K rows of sixteen blocks, where a weight by itself goes by rounds of tiles (launch_res_rt): 2 x 12288 x 4096
-// 26.1 / 24.7, 2 x 14336 28.5 / 28.1, 2 x 16384 30.6 / 28.6, 2 x 28672 47.2 / 44.3, 3 x 28672 67.0 / 63.7; but 2 x 13312 27.1 / 27.4,
-// 2 x 9728 22.0 / 23.2, 3 x 14336 37.5 / 40.2.  Which of them, by the two sums below, which follow these within 1 us (a launch
-// each: 4 us, 2 more for every tile of a workgroup, 1 for every further round of four tiles).  Fewer blocks leave some of
-// the rounds kernel's sixteen waves without one: K = 3840 and below within 3 % of each other, mostly for the one launch.
+// x 8192 77.5 / 82.7; 16 rows: Q6K 2 x 14336 x 4096 32.2 / 37.2, Q8_0 2 x 11008 x 4096 31.2 / 31.8).
 bool cq_skinny_shared_takes(const cq_weight *const *ws, int count, int64_t m, int act_dtype) {
     if (count < 2 || count > kMultiMax || m > 16) return false;
-    const int64_t cus = cq_num_cus();
-    double shared = 10.3, each = 4.0;
-    for (int i = 0; i < count; i++) {
+    for (int i = 0; i < count; i++)
         if (!cq_skinny_takes(ws[i], act_dtype)) return false;
-        const int64_t tiles = (ws[i]->n + 15) / 16, turns = (tiles + cus - 1) / cus;
-        shared += 0.64e-3 * 16.0 * (double)tiles;
-        each += 4.0 + 2.0 * (double)turns + (double)((turns - 1) / kTilesPerRound);
-    }
-    return !(m > 8 && ws[0]->dtype == CQ_DTYPE_Q4K && ws[0]->k == 16 * QK_K && each < shared);
+    return true;
 }
 
 hipError_t cq_launch_skinny_shared(const cq_weight *const *ws, int count, cq_act_view a, int64_t m, float *const *ys, hipStream_t s) {
