@@ -1423,9 +1423,10 @@ bool launch_blk32_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq
 // block each in flight leave the memory idle.  Measured, whole calls in us, eight waves -> sixteen, 4 and 8 rows: 4096 x 14336 Q4K 15.2 -> 13.6
 // and 15.4 -> 14.6, Q4_0 16.0 -> 13.0 and 16.2 -> 13.8, Q6K 17.3 -> 16.2 and 17.5 -> 17.3; 2048 x 11008 Q4K 12.2 -> 10.7, Q4_0 13.2 -> 10.6.  Not
 // for Q8_0, whose blocks are twice as long (4096 x 14336 18.1 -> 18.6), from nine rows on (Q4K 16.2 -> 17.3), or with more workgroups than CUs
-// (8192 x 8192 Q6K 18.9 -> 20.9, Q4_0 14.8 -> 15.8).
+// (8192 x 8192 Q6K 18.9 -> 20.9, Q5K 18.6 -> 20.6, Q4_0 14.8 -> 15.8), but for Q4K, of whose blocks two workgroups of sixteen waves fit a CU (8192 x
+// 8192 16.0 -> 15.2, 5120 x 13824 18.4 -> 18.0; 14336 + 14336 x 4096 22.4 -> 25.2).
 template <int DT, int RT> bool sixteen_waves(const cq_weight *w) {
-    return RT == 1 && DT != CQ_DTYPE_Q8_0 && w->k > 8 * QK_K && (w->n + 15) / 16 <= cq_num_cus();
+    return RT == 1 && DT != CQ_DTYPE_Q8_0 && w->k > 16 * QK_K && (w->n + 15) / 16 <= (DT == CQ_DTYPE_Q4K ? 2 : 1) * cq_num_cus();
 }
 
 template <int DT, int RT, bool DUMP, int NW>
