@@ -681,8 +681,9 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
         case kGemm: CQ_HIP_CHECK(cq_launch_gemm(w, v, act, m, y_dev, y_cleared, s)); break;
         case kMatvec: CQ_HIP_CHECK(cq_launch_matvec(w, v, act, m, y_dev, s)); break;
     }
-    if (cq_has_min32(w->ggml_dtype)) CQ_HIP_CHECK(cq_launch_min32_term(w, v, m, y_dev, path == kMatvec, s));
-    if (cq_has_min16(w->ggml_dtype)) CQ_HIP_CHECK(cq_launch_min16_term(w, v, m, y_dev, path == kMatvec, s));
+    // (the split-K kernel adds the offset term itself)
+    if (path != kSkinny && cq_has_min32(w->ggml_dtype)) CQ_HIP_CHECK(cq_launch_min32_term(w, v, m, y_dev, path == kMatvec, s));
+    if (path != kSkinny && cq_has_min16(w->ggml_dtype)) CQ_HIP_CHECK(cq_launch_min16_term(w, v, m, y_dev, path == kMatvec, s));
     return CQ_OK;
 }
 
@@ -764,10 +765,6 @@ extern "C" int cq_qmatmul_multi(const cq_weight *const *ws, int count, int pre, 
         act_ws_layout(act, m, ws[0]->k, (uint8_t *)workspace, &v);
         CQ_HIP_CHECK(cq_launch_quantize_act_ws(act, x_dev, nullptr, m, ws[0]->k, p, v, cq_no_clear(), s));
         CQ_HIP_CHECK(cq_launch_skinny_shared(ws, count, v, m, ys_dev, s));
-        for (int i = 0; i < count; i++) {
-            if (cq_has_min32(ws[i]->ggml_dtype)) CQ_HIP_CHECK(cq_launch_min32_term(ws[i], v, m, ys_dev[i], false, s));
-            if (cq_has_min16(ws[i]->ggml_dtype)) CQ_HIP_CHECK(cq_launch_min16_term(ws[i], v, m, ys_dev[i], false, s));
-        }
         return CQ_OK;
     }
     for (int i = 0; i < count; i++) {

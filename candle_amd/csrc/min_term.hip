@@ -26,7 +26,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 // No LDS and no barrier: the operands are a few hundred bytes a row, read straight into registers (cache hits after the first tile); what
 // is left is the pass over y and, with few tiles, a chain of loads.  Against the sums on the vector units through LDS, us a whole call before
 // and after: Q5_1 2225 x 3328 with 3343 rows 187 -> 127, Q4_1 14336 x 4096 with 512 rows 184 -> 134, 4096 x 4096 with 64 rows 36.0 -> 21.2,
-// with 8 rows 23.2 -> 12.6, Q2K 4096 x 4096 with 1024 rows 147 -> 88, with 128 rows 59.9 -> 28.7.  Error of the m * s term against 64 bits
+// Q2K 4096 x 4096 with 1024 rows 147 -> 88, with 128 rows 59.9 -> 28.7 (few rows: the split-K kernels add the terms themselves, skinny.hip).  Error of the m * s term against 64 bits
 // (4096 x 4096, 64 rows, relative rms): 8.9e-8 -> 6.0e-8.
 //   SHARE = false: every wave a 64 x 64 tile of its own (workgroup: 64 rows x 256 weight rows)
 //   SHARE = true:  up to 32 rows x 32 weight rows a workgroup, the steps dealt round-robin to its four waves: few rows leave too few tiles to
@@ -277,8 +277,7 @@ __global__ void __launch_bounds__(256) min16_small_kernel(const uint8_t *__restr
 
 // `apart`: a row's bits may not depend on how many rows there are.  For that, one kernel takes all of them (Q2K: its unshared tiles add
 // the blocks in the small kernel's order, with the same roundings).
-// Whether a tile of 64 x 64 for every wave would be fewer than one wave for each SIMD.  (Up to four rows: the small kernels, whose sixteen lanes
-// a weight row leave no MFMA row idle.)
+// Whether a tile of 64 x 64 for every wave would be fewer than one wave for each SIMD.
 static bool share_tile(const cq_weight *w, int64_t m) { return m <= 32 || ((w->n + 63) / 64) * ((m + 63) / 64) < 4 * cq_num_cus(); }
 
 hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool apart, hipStream_t s) {
@@ -286,7 +285,7 @@ hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, fl
     if (m == 0 || w->n == 0 || w->k == 0) return hipSuccess;
     const int64_t nb = w->k / 32;
     const uint16_t *mins = (const uint16_t *)w->p2;
-    if (apart || m <= kSmallRows)
+    if (apart)
         CQ_LAUNCH(min32_small_kernel, dim3((unsigned)((w->n + 15) / 16), (unsigned)((m + kSmallRows - 1) / kSmallRows)), 256, 0, s, mins, a,
                   w->n, nb, m, y);
     else if (share_tile(w, m))

@@ -21,6 +21,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 // the same at four-byte alignment: scales of 32-element blocks in rows of no whole 256 elements
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
@@ -187,6 +188,66 @@ __device__ __forceinline__ void block_unpack(const uint8_t *wl, int lane, const 
     wmin = v8h{};
 }
 
+// ---- the offset terms (min_term.hip), added to the result tiles of the waves ----
+// A launch of its own for them is 4 of the 10 us of a call of a few rows (whole calls, launch on the vector units -> here: Q4_1 4096 x 4096 with
+// 8 rows 23.2 -> 8.6, 11008 x 4096 30.2 -> 17.9, 1792 x 1792 with 5 rows 14.4 -> 7.1, Q2K 4096 x 4096 with 8 rows 13.9 -> 9.0).  out[t] += a step of 32 blocks' m * s products for the types held in
+// Q8_0 planes, -= a block's dmin term for Q2K: the same products, exact in f32, on the same operands as there.  `first` and `stride` deal the
+// steps to the waves.  Instances of their own (OFF), so that the kernels of the plain Q8_0 and
+// Q6K weights keep their registers.
+template <int NT>
+__device__ __forceinline__ void add_min32(const cq_weight &w, const cq_act_view &a, int64_t n_tile, int64_t m0, int64_t m, int64_t first,
+                                          int64_t stride, int lane, v4f (&out)[NT]) {
+    const uint32_t r = lane & 15, kq = lane >> 4;
+    const int64_t nb = w.k >> 5;
+#pragma nounroll
+    for (int64_t b0 = first * 32; b0 < nb; b0 += stride * 32) {
+        const int64_t b = b0 + 8 * kq;   // (rows have an even number of blocks: pairs of 16-bit values start on a word)
+        uint32_t mw[4];
+        const uint32_t *mp = (const uint32_t *)w.p2 + (((n_tile + r) * nb + b) >> 1);
+#pragma unroll
+        for (int i = 0; i < 4; i++) mw[i] = b + 2 * i < nb ? mp[i] : 0u;
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const int64_t row = m0 + t * 16 + r < m ? m0 + t * 16 + r : m - 1;
+            const uint32_t *sp = (const uint32_t *)a.bsum32 + ((row * nb + b) >> 1);
+            const float *dp = a.d + row * nb + b;
+            v8h sv;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const bool in = b + 2 * i < nb;
+                const uint32_t s = in ? sp[i] : 0u;
+                const float d0 = in ? dp[2 * i] : 0.0f, d1 = in ? dp[2 * i + 1] : 0.0f;
+                sv[2 * i] = (_Float16)((float)(_Float16)(float)(int16_t)s * d0);
+                sv[2 * i + 1] = (_Float16)((float)(_Float16)(float)(int16_t)(s >> 16) * d1);
+            }
+            out[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sv, __builtin_bit_cast(v8h, mw), out[t], 0, 0, 0);
+        }
+    }
+}
+template <int NT>
+__device__ __forceinline__ void add_min16(const cq_weight &w, const cq_act_view &a, int64_t n_tile, int64_t m0, int64_t first, int64_t stride,
+                                          int lane, v4f (&out)[NT]) {
+    const uint32_t r = lane & 15, kq = lane >> 4;
+    const int64_t kb = w.k >> 8;
+#pragma nounroll
+    for (int64_t b = first; b < kb; b += stride) {
+        const int64_t blk = (n_tile + r) * kb + b;
+        const uint32_t mq = *(const uint32_t *)(w.p4 + blk * 16 + 4 * kq);   // minima 4kq .. of the lane's weight row
+        const float dm = cq_h2f(((const uint16_t *)w.p5)[blk]);
+        v4h mv;
+#pragma unroll
+        for (int i = 0; i < 4; i++) mv[i] = (_Float16)(float)((mq >> (8 * i)) & 0xff);
+#pragma unroll
+        for (int t = 0; t < NT; t++) {   // (rows past the last one are the workspace's padding)
+            const v4h sv = *(const v4h *)(a.bsh + (b * a.m_stride + m0 + t * 16 + r) * 16 + 4 * kq);
+            const v4f d8 = *(const v4f *)(a.dT + b * a.m_stride + m0 + t * 16 + 4 * kq);
+            const v4f sum = __builtin_amdgcn_mfma_f32_16x16x16f16(sv, mv, (v4f){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) out[t][i] -= (d8[i] * dm) * sum[i];
+        }
+    }
+}
+
 // The wave's rows of K block b, four at a time (lane l: row 4p + l/16, elements 64i + 4(l%16) ..; rows past m repeat the last one).
 template <int RT>
 __device__ __forceinline__ void load_direct(const float *__restrict__ x, int64_t m, int64_t k, int64_t b, int lane, float4 (&xf)[2 * RT][4]) {
@@ -239,7 +300,7 @@ __device__ __forceinline__ void quantize_direct(const float4 (&xf)[2 * RT][4], c
 // DUMP (verification): the block integers, and the min term as the f16 MFMA delivers it from a zero accumulator,
 // are stored through `dump` instead of the result through `y`.
 // DIRECT: the rows come as f32 from `x` and every wave quantizes the blocks it contracts (see skinny_direct_kernel).
-template <int DT, int RT, bool DUMP, bool DIRECT = false, int NW = kWaves>
+template <int DT, int RT, bool DUMP, bool DIRECT = false, int NW = kWaves, bool OFF = false>
 __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
                                             float *__restrict__ y, cq_mfma_dump dump, const float *__restrict__ x = nullptr) {
     typedef Buf<DT, RT> B;
@@ -354,8 +415,9 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
         }
     }
     if (DUMP) return;
+    if constexpr (OFF) add_min16<NT>(w, a, n_tile, m0, wave, NW, lane, out);
 
-    // ---- sum the eight waves' partial tiles in wave order
+    // ---- sum the waves' partial tiles in wave order
 #pragma unroll
     for (int t = 0; t < NT; t++) *(v4f *)(buf + t * 1024 + lane * 16) = out[t];
     __syncthreads();
@@ -375,10 +437,10 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
     }
 }
 
-template <int DT, int RT, bool DUMP, int NW = kWaves>
+template <int DT, int RT, bool DUMP, int NW = kWaves, bool OFF = false>
 __global__ void __launch_bounds__(NW * 64) skinny_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
                                                           cq_mfma_dump dump) {
-    skinny_body<DT, RT, DUMP, false, NW>(w, a, blockIdx.x, m0, m, y, dump);
+    skinny_body<DT, RT, DUMP, false, NW, OFF>(w, a, blockIdx.x, m0, m, y, dump);
 }
 
 // ------------------------------------------------------------ resident-activation variant ----
@@ -502,7 +564,7 @@ __device__ __forceinline__ void res_block(const uint8_t *__restrict__ wl, const 
 // m <= 8 * RT activation rows (the workspace pads rows, so whole groups are copied); n >= 16; at most
 // kMaxBpw K blocks per wave.  `tiles` of 16 rows, dealt to the gridDim.x workgroups in turn.
 constexpr int kMaxBpw = 4;
-template <int DT, int RT, int kWaves, int NBUF, bool DUMP>
+template <int DT, int RT, int kWaves, int NBUF, bool DUMP, bool OFF = false>
 __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight w, cq_act_view a, int64_t m,
                                                                       float *__restrict__ y, cq_mfma_dump dump) {
     typedef Res<DT, RT> R;
@@ -585,6 +647,9 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
             if (b < kb)
                 res_block<DT, RT, NT, DUMP>(wgt_base + (b * NBUF + (NBUF == 2 ? par : 0)) * R::kWgt, smem + b * R::kActBlk, lane,
                                             head[j], a_col, out, dump, (n_tile + r) * kb + b, w.n * kb, m);
+        }
+        if constexpr (OFF) {
+            if (wave < kb) add_min16<NT>(w, a, n_tile, 0, wave, kb < kWaves ? kb : kWaves, lane, out);
         }
         // ---- sum the waves' partial tiles in wave order (through the wave's first weight buffer of this tile)
         uint8_t *part = wgt_base + ((int64_t)wave * NBUF + (NBUF == 2 ? par : 0)) * R::kWgt;
@@ -915,7 +980,7 @@ __device__ __forceinline__ void quantize_direct_q8(const float4 (&xf)[8 * RT], c
     }
 }
 
-template <int DT, int RT, bool DUMP, bool DIRECT = false, int NW = kWaves>
+template <int DT, int RT, bool DUMP, bool DIRECT = false, int NW = kWaves, bool OFF = false>
 __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_act_view &a, int64_t tile, int64_t m0, int64_t m,
                                                   float *__restrict__ y, cq_mfma_dump dump, const float *__restrict__ x = nullptr) {
     typedef BufQ8<DT, RT> B;
@@ -1009,8 +1074,9 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
         each_block(kb - g * 8, block);
     }
     if (DUMP) return;
+    if constexpr (OFF) add_min32<NT>(w, a, n_tile, m0, m, wave, NW, lane, out);
 
-    // ---- sum the eight waves' partial tiles in wave order
+    // ---- sum the waves' partial tiles in wave order
 #pragma unroll
     for (int t = 0; t < NT; t++) *(v4f *)(buf + t * 1024 + lane * 16) = out[t];
     __syncthreads();
@@ -1030,10 +1096,10 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
     }
 }
 
-template <int DT, int RT, bool DUMP, int NW = kWaves>
+template <int DT, int RT, bool DUMP, int NW = kWaves, bool OFF = false>
 __global__ void __launch_bounds__(NW * 64) skinny_blk32_kernel(cq_weight w, cq_act_view a, int64_t m0, int64_t m, float *__restrict__ y,
                                                                 cq_mfma_dump dump) {
-    skinny_blk32_body<DT, RT, DUMP, false, NW>(w, a, blockIdx.x, m0, m, y, dump);
+    skinny_blk32_body<DT, RT, DUMP, false, NW, OFF>(w, a, blockIdx.x, m0, m, y, dump);
 }
 
 // Mixture-of-experts form of the two: blockIdx.y is a tile of up to 8 * RT routed rows and names its expert's weights, so
@@ -1050,14 +1116,14 @@ __global__ void __launch_bounds__(kThreads) skinny_grouped_kernel(cq_group_args 
 
 // Two or three weights on the same rows (q, k, v; gate and up): their 16-row tiles one after the other.  A weight with few
 // rows (1024: 64 workgroups) does not fill the machine by itself.
-template <int DT, int RT>
+template <int DT, int RT, bool OFF>
 __global__ void __launch_bounds__(kThreads) skinny_shared_kernel(MultiArgs ma, cq_act_view a, int64_t m) {
     const uint32_t t = blockIdx.x;
     const int i = t >= ma.first[2] ? 2 : t >= ma.first[1] ? 1 : 0;
     const cq_weight w = ma.w[i];
     const cq_mfma_dump none{nullptr, nullptr, 0};
-    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, RT, false>(w, a, t - ma.first[i], 0, m, ma.y[i], none);
-    else skinny_body<DT, RT, false>(w, a, t - ma.first[i], 0, m, ma.y[i], none);
+    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, RT, false, false, kWaves, OFF>(w, a, t - ma.first[i], 0, m, ma.y[i], none);
+    else skinny_body<DT, RT, false, false, kWaves, OFF>(w, a, t - ma.first[i], 0, m, ma.y[i], none);
 }
 
 // ------------------------------------------------------------ the rows quantized by the waves that contract them ----
@@ -1090,7 +1156,7 @@ template <int DT, int RT> struct ResQ8 {
 };
 
 // m <= 8 * RT rows; n >= 16, one 16-row tile per workgroup; at most kMaxBpw K groups per wave.
-template <int DT, int RT, int kWaves, bool DUMP>
+template <int DT, int RT, int kWaves, bool DUMP, bool OFF = false>
 __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_weight w, cq_act_view a, int64_t m,
                                                                             float *__restrict__ y, cq_mfma_dump dump) {
     typedef ResQ8<DT, RT> R;
@@ -1184,6 +1250,9 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_resident_kernel(cq_w
     }
     if (DUMP) return;
 
+    if constexpr (OFF) {
+        if (wave < kg) add_min32<NT>(w, a, n_tile, 0, m, wave, kg < kWaves ? kg : kWaves, lane, out);
+    }
     // ---- sum the waves' partial tiles in wave order (through each wave's first weight buffer)
     if (wave < kg) {
 #pragma unroll
@@ -1372,6 +1441,10 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_blk32_multi_kernel(cq_weig
     }
 }
 
+// Weight types held in DT's planes that have an offset term.
+template <int DT, bool DUMP> constexpr bool kCanOffset = !DUMP && (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q6K);
+bool has_offset(const cq_weight &w) { return cq_has_min32(w.ggml_dtype) || cq_has_min16(w.ggml_dtype); }
+
 template <int DT, int RT, int NW, bool DUMP>
 hipError_t launch_blk32_multi_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, size_t lds, unsigned grid, cq_mfma_dump d,
                                    hipStream_t s) {
@@ -1380,10 +1453,10 @@ hipError_t launch_blk32_multi_inst(const cq_weight *w, cq_act_view a, int64_t m,
     return hipGetLastError();
 }
 
-template <int DT, int RT, int NW, bool DUMP>
+template <int DT, int RT, int NW, bool DUMP, bool OFF = false>
 hipError_t launch_blk32_res_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, size_t lds, cq_mfma_dump d, hipStream_t s) {
-    if (hipError_t e = cq_ensure_lds<skinny_blk32_resident_kernel<DT, RT, NW, DUMP>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_blk32_resident_kernel<DT, RT, NW, DUMP>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m, y, d);
+    if (hipError_t e = cq_ensure_lds<skinny_blk32_resident_kernel<DT, RT, NW, DUMP, OFF>>(w->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_blk32_resident_kernel<DT, RT, NW, DUMP, OFF>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m, y, d);
     return hipGetLastError();
 }
 // Takes the launch (true) where the resident kernel applies: one tile per workgroup, all operands in the LDS.
@@ -1394,9 +1467,10 @@ bool launch_blk32_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y,
     const bool sixteen = kg > 8;
     if (tiles > cus) {
         // several tiles per workgroup: rounds of tiles with one meeting each, where a wave has one K group
+        // (the types with an offset term: tile by tile, where it is added)
         if constexpr (RT <= 2) {
             const size_t lm = ResQ8Multi<DT, RT>::bytes(kg);
-            if (sixteen && kg <= 16 && lm <= (size_t)kMaxLds && (uint64_t)w->n * (uint64_t)w->k < (1ull << 32)) {
+            if (!cq_has_min32(w->ggml_dtype) && sixteen && kg <= 16 && lm <= (size_t)kMaxLds && (uint64_t)w->n * (uint64_t)w->k < (1ull << 32)) {
                 *err = launch_blk32_multi_inst<DT, RT, 16, DUMP>(w, a, m, y, lm, (unsigned)cus, d, s);
                 return true;
             }
@@ -1406,6 +1480,12 @@ bool launch_blk32_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y,
     if (kg > (sixteen ? 16 : 8) * kMaxBpw) return false;
     const size_t lds = ResQ8<DT, RT>::bytes(kg);
     if (lds > (size_t)kMaxLds) return false;
+    if constexpr (kCanOffset<DT, DUMP>) {
+        if (has_offset(*w)) {
+            *err = sixteen ? launch_blk32_res_inst<DT, RT, 16, DUMP, true>(w, a, m, y, lds, d, s) : launch_blk32_res_inst<DT, RT, 8, DUMP, true>(w, a, m, y, lds, d, s);
+            return true;
+        }
+    }
     *err = sixteen ? launch_blk32_res_inst<DT, RT, 16, DUMP>(w, a, m, y, lds, d, s) : launch_blk32_res_inst<DT, RT, 8, DUMP>(w, a, m, y, lds, d, s);
     return true;
 }
@@ -1429,18 +1509,20 @@ template <int DT, int RT> bool sixteen_waves(const cq_weight *w) {
     return RT == 1 && DT != CQ_DTYPE_Q8_0 && w->k > 16 * QK_K && (w->n + 15) / 16 <= (DT == CQ_DTYPE_Q4K ? 2 : 1) * cq_num_cus();
 }
 
-template <int DT, int RT, bool DUMP, int NW>
+template <int DT, int RT, bool DUMP, int NW, bool OFF>
 hipError_t launch_blk32_waves(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = (size_t)BufQ8<DT, RT>::kBytes * NW;
-    if (hipError_t e = cq_ensure_lds<skinny_blk32_kernel<DT, RT, DUMP, NW>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_blk32_kernel<DT, RT, DUMP, NW>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m0, m, y, d);
+    if (hipError_t e = cq_ensure_lds<skinny_blk32_kernel<DT, RT, DUMP, NW, OFF>>(w->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_blk32_kernel<DT, RT, DUMP, NW, OFF>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m0, m, y, d);
     return hipGetLastError();
 }
 template <int DT, int RT, bool DUMP>
 hipError_t launch_blk32_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    if constexpr (RT == 1 && DT != CQ_DTYPE_Q8_0 && !DUMP)
-        if (sixteen_waves<DT, RT>(w)) return launch_blk32_waves<DT, RT, DUMP, 16>(w, a, m0, m, y, d, s);
-    return launch_blk32_waves<DT, RT, DUMP, kWaves>(w, a, m0, m, y, d, s);
+    const bool sixteen = sixteen_waves<DT, RT>(w);
+    constexpr int kMany = RT == 1 && DT != CQ_DTYPE_Q8_0 && !DUMP ? 16 : kWaves;
+    if constexpr (kCanOffset<DT, DUMP>)
+        if (has_offset(*w)) return sixteen ? launch_blk32_waves<DT, RT, DUMP, kMany, true>(w, a, m0, m, y, d, s) : launch_blk32_waves<DT, RT, DUMP, kWaves, true>(w, a, m0, m, y, d, s);
+    return sixteen ? launch_blk32_waves<DT, RT, DUMP, kMany, false>(w, a, m0, m, y, d, s) : launch_blk32_waves<DT, RT, DUMP, kWaves, false>(w, a, m0, m, y, d, s);
 }
 
 template <int DT, bool DUMP>
@@ -1457,18 +1539,20 @@ hipError_t launch_blk32(const cq_weight *w, cq_act_view a, int64_t m, float *y, 
     return hipSuccess;
 }
 
-template <int DT, int RT, bool DUMP, int NW>
+template <int DT, int RT, bool DUMP, int NW, bool OFF>
 hipError_t launch_waves(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = (size_t)Buf<DT, RT>::kBytes * NW;
-    if (hipError_t e = cq_ensure_lds<skinny_kernel<DT, RT, DUMP, NW>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_kernel<DT, RT, DUMP, NW>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m0, m, y, d);
+    if (hipError_t e = cq_ensure_lds<skinny_kernel<DT, RT, DUMP, NW, OFF>>(w->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_kernel<DT, RT, DUMP, NW, OFF>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m0, m, y, d);
     return hipGetLastError();
 }
 template <int DT, int RT, bool DUMP>
 hipError_t launch_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    if constexpr (RT == 1 && DT != CQ_DTYPE_Q8_0 && !DUMP)
-        if (sixteen_waves<DT, RT>(w)) return launch_waves<DT, RT, DUMP, 16>(w, a, m0, m, y, d, s);
-    return launch_waves<DT, RT, DUMP, kWaves>(w, a, m0, m, y, d, s);
+    const bool sixteen = sixteen_waves<DT, RT>(w);
+    constexpr int kMany = RT == 1 && DT != CQ_DTYPE_Q8_0 && !DUMP ? 16 : kWaves;
+    if constexpr (kCanOffset<DT, DUMP>)
+        if (has_offset(*w)) return sixteen ? launch_waves<DT, RT, DUMP, kMany, true>(w, a, m0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, true>(w, a, m0, m, y, d, s);
+    return sixteen ? launch_waves<DT, RT, DUMP, kMany, false>(w, a, m0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, false>(w, a, m0, m, y, d, s);
 }
 
 template <int DT, bool DUMP>
@@ -1487,11 +1571,11 @@ hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_
 
 
 // The resident-activation kernel where the call's activations and the weight buffers fit the LDS (see above).
-template <int DT, int RT, int NW, int NBUF, bool DUMP>
+template <int DT, int RT, int NW, int NBUF, bool DUMP, bool OFF = false>
 hipError_t launch_res_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, size_t lds, unsigned grid, cq_mfma_dump d,
                            hipStream_t s) {
-    if (hipError_t e = cq_ensure_lds<skinny_resident_kernel<DT, RT, NW, NBUF, DUMP>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_resident_kernel<DT, RT, NW, NBUF, DUMP>), grid, NW * 64, lds, s, *w, a, m, y, d);
+    if (hipError_t e = cq_ensure_lds<skinny_resident_kernel<DT, RT, NW, NBUF, DUMP, OFF>>(w->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_resident_kernel<DT, RT, NW, NBUF, DUMP, OFF>), grid, NW * 64, lds, s, *w, a, m, y, d);
     return hipGetLastError();
 }
 template <int DT, int RT, int NW, bool DUMP>
@@ -1531,6 +1615,13 @@ bool launch_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mf
     }
     const size_t one = Res<DT, RT>::bytes(kb, 1);
     if (one <= (size_t)kMaxLds) {
+        if constexpr (kCanOffset<DT, DUMP>) {
+            if (has_offset(*w)) {
+                *err = sixteen ? launch_res_inst<DT, RT, 16, 1, DUMP, true>(w, a, m, y, one, grid, d, s)
+                               : launch_res_inst<DT, RT, 8, 1, DUMP, true>(w, a, m, y, one, grid, d, s);
+                return true;
+            }
+        }
         *err = sixteen ? launch_res_inst<DT, RT, 16, 1, DUMP>(w, a, m, y, one, grid, d, s)
                        : launch_res_inst<DT, RT, 8, 1, DUMP>(w, a, m, y, one, grid, d, s);
         return true;
@@ -1546,12 +1637,18 @@ bool launch_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_
     return false;
 }
 
+template <int DT, int RT, bool OFF>
+hipError_t launch_shared_inst(const MultiArgs &ma, unsigned tiles, cq_act_view a, int64_t m, hipStream_t s) {
+    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<DT, RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
+    if (hipError_t e = cq_ensure_lds<skinny_shared_kernel<DT, RT, OFF>>(ma.w[0].dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_shared_kernel<DT, RT, OFF>), tiles, kThreads, lds, s, ma, a, m);
+    return hipGetLastError();
+}
 template <int DT, int RT>
 hipError_t launch_shared_rt(const MultiArgs &ma, unsigned tiles, cq_act_view a, int64_t m, hipStream_t s) {
-    const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<DT, RT>::kBytes : (int)Buf<DT, RT>::kBytes) * kWaves;
-    if (hipError_t e = cq_ensure_lds<skinny_shared_kernel<DT, RT>>(ma.w[0].dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_shared_kernel<DT, RT>), tiles, kThreads, lds, s, ma, a, m);
-    return hipGetLastError();
+    if constexpr (kCanOffset<DT, false>)
+        if (has_offset(ma.w[0])) return launch_shared_inst<DT, RT, true>(ma, tiles, a, m, s);   // (all of one type)
+    return launch_shared_inst<DT, RT, false>(ma, tiles, a, m, s);
 }
 // Nine rows and more of Q4K with nine to sixteen blocks a row: by rounds of tiles over all the weights, as launch_res_rt does for one.  Measured
 // with rms_norm in front, whole calls in us, tile by tile (for many rows a launch for each weight) -> rounds, 16 rows: 3 x 4096 x 4096 17.1 -> 15.1,
@@ -1655,7 +1752,8 @@ hipError_t cq_launch_skinny_dump(const cq_weight *w, cq_act_view a, int act_dtyp
 // (Q4K 2048 x 2048, 8 rows 6.0 against 6.8 / 5.6; 8192 x 2048 10.6 against 7.3), nine rows take a second group (Q4K 1024 x 1024, 16 rows 6.9
 // against 7.0 / 5.6), Q4_0 with 8 rows 5.9 / 5.7 against 7.4 / 5.5.
 bool cq_skinny_direct_takes(const cq_weight *w, int act_dtype, int64_t m) {
-    return m >= 2 && m <= (w->dtype == CQ_DTYPE_Q4_0 ? 7 : 8) && w->n <= 4096 && w->k <= (m <= 4 ? 2048 : 1024) && cq_skinny_takes(w, act_dtype);
+    return m >= 2 && m <= (w->dtype == CQ_DTYPE_Q4_0 ? 7 : 8) && w->n <= 4096 && w->k <= (m <= 4 ? 2048 : 1024) &&
+           !cq_has_min32(w->ggml_dtype) && !cq_has_min16(w->ggml_dtype) && cq_skinny_takes(w, act_dtype);
 }
 hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s) {
     if (m > 8) return hipErrorInvalidValue;

@@ -11,7 +11,7 @@ from tests.test_gpu_fused_neighbours import qh  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 40, 64), (4, 100, 4160), (5, 100, 64), (5, 33, 4160), (31, 1000, 576), (33, 70, 1088), (64, 4096, 2112), (65, 16390, 128), (700, 8200, 1088)]
+SHAPES = [(1, 40, 64), (6, 100, 11008), (16, 4112, 4096), (4, 100, 4160), (5, 100, 64), (5, 33, 4160), (31, 1000, 576), (33, 70, 1088), (64, 4096, 2112), (65, 16390, 128), (700, 8200, 1088)]
 
 
 def f16(x):
