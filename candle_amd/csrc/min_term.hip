@@ -23,14 +23,14 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 // Both factors of the m * s term are f16 values and their product is exact in f32; so are Q2K's integer sums, at most 16 * 2048 * 15.
 // MFMA 32x32x16 (f16): lane l holds row l % 32 of either operand, k = 8 * (l / 32) .. + 7, and of the result column l % 32, rows
 // 8 * (i / 4) + 4 * (l / 32) + i % 4.  Activation rows are the rows, weight rows the columns, so that a wave's stores are runs of 128 bytes.
-// No LDS and no barrier: the operands are a few hundred bytes a row, read straight into registers (cache hits after the first tile); what
-// is left is the pass over y and, with few tiles, a chain of loads.  Against the sums on the vector units through LDS, us a whole call before
-// and after: Q5_1 2225 x 3328 with 3343 rows 187 -> 127, Q4_1 14336 x 4096 with 512 rows 184 -> 134, 4096 x 4096 with 64 rows 36.0 -> 21.2,
-// Q2K 4096 x 4096 with 1024 rows 147 -> 88, with 128 rows 59.9 -> 28.7 (few rows: the split-K kernels add the terms themselves, skinny.hip).  Error of the m * s term against 64 bits
-// (4096 x 4096, 64 rows, relative rms): 8.9e-8 -> 6.0e-8.
-//   SHARE = false: every wave a 64 x 64 tile of its own (workgroup: 64 rows x 256 weight rows)
-//   SHARE = true:  up to 32 rows x 32 weight rows a workgroup, the steps dealt round-robin to its four waves: few rows leave too few tiles to
-//                  fill the machine, and one wave would walk the whole row by itself
+// Many tiles: every wave one of 32 rows x 64 weight rows.  Few tiles: 32 x 32, their steps dealt to the four waves of a workgroup, since few rows
+// leave too few tiles to fill the machine and one wave would walk the whole row by itself.
+// Bound: the pass over y and the gather of the operands, 16 bytes of a row at a time.  Against the sums on the vector units through LDS, us a
+// whole call before and after: Q5_1 2225 x 3328 with 3343 rows 187 -> 119, Q4_1 14336 x 4096 with 512 rows 184 -> 119, 4096 x 4096 with 64 rows
+// 36.0 -> 21.0, Q2K 4096 x 4096 with 1024 rows 147 -> 81, with 128 rows 59.9 -> 28.7, 10400 x 768 with 561 rows 59 -> 36 (without the term:
+// 94, 95, -, 58, -, 25).  A wave's part of y is requested before its sums are done: 10400 x 768 45.5 -> 36.2
+// (few rows: the split-K kernels add the terms themselves, skinny.hip).  Error of the m * s term against 64 bits (4096 x 4096, 64 rows, relative
+// rms): 8.9e-8 -> 6.0e-8.
 struct HalfRow { uint32_t w[4]; };   // eight 16-bit values; rows have an even number of blocks and so start on a word
 __device__ __forceinline__ HalfRow load_eight(const void *plane, int64_t row, int64_t b, int64_t nb) {
     const uint32_t *p = (const uint32_t *)plane + ((row * nb + b) >> 1);
@@ -45,94 +45,138 @@ __device__ __forceinline__ HalfRow load_eight(const void *plane, int64_t row, in
     return r;
 }
 
-// Adds (or, SUB, subtracts) the tile to y; SHARE: the four waves' parts first, in order.
-template <bool SHARE, bool SUB, int RT, int CT>
-__device__ __forceinline__ void add_tiles(v16f (&acc)[RT][CT], int64_t r0, int64_t c0, int64_t m, int64_t n, float *__restrict__ y) {
-    const int lane = threadIdx.x & 63, col = lane & 31, h = lane >> 5;
-    if constexpr (SHARE) {
-        __shared__ float part[4][16][64];
-        const int wave = threadIdx.x >> 6;
+// One column tile of y, requested ahead of the sums that are added to it (element i: row 8 * (i / 4) + 4 * (lane / 32) + i % 4).
+__device__ __forceinline__ void load_tile(const float *y, int64_t r0, int64_t c, int64_t m, int64_t n, int h, v16f &old) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) part[wave][i][lane] = acc[0][0][i];
-        __syncthreads();
-        if (c0 + col >= n) return;
+    for (int i = 0; i < 16; i++) {
+        const int64_t r = r0 + 8 * (i >> 2) + 4 * h + (i & 3);
+        old[i] = r < m && c < n ? y[r * n + c] : 0.0f;
+    }
+}
+// Adds (SUB: subtracts) the tiles.
+template <bool SUB, int CT>
+__device__ __forceinline__ void add_tiles(const v16f (&acc)[CT], const v16f (&old)[CT], int64_t r0, int64_t c0, int64_t m, int64_t n, float *y) {
+    const int lane = threadIdx.x & 63, h = lane >> 5;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {   // wave w finishes result registers 4w .. 4w + 3
-            const int i = 4 * wave + j;
-            const int64_t r = r0 + 8 * wave + 4 * h + j;
-            const float t = ((part[0][i][lane] + part[1][i][lane]) + part[2][i][lane]) + part[3][i][lane];
-            if (r < m) y[r * n + c0 + col] += SUB ? -t : t;
+    for (int ct = 0; ct < CT; ct++) {
+        const int64_t c = c0 + 32 * ct + (lane & 31);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int64_t r = r0 + 8 * (i >> 2) + 4 * h + (i & 3);
+            if (r < m && c < n) y[r * n + c] = old[ct][i] + (SUB ? -acc[ct][i] : acc[ct][i]);
         }
-    } else {
+    }
+}
+// The same for a tile whose four waves hold parts of the sums: added in order first.
+template <bool SUB>
+__device__ __forceinline__ void add_shared_tile(const v16f &acc, int64_t r0, int64_t c0, int64_t m, int64_t n, float *__restrict__ y) {
+    __shared__ float part[4][16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5;
+    const int64_t c = c0 + (lane & 31), r = r0 + 8 * wave + 4 * h;   // wave w finishes result registers 4w .. 4w + 3
+    float old[4];
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++)
+    for (int j = 0; j < 4; j++) old[j] = r + j < m && c < n ? y[(r + j) * n + c] : 0.0f;
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++) {
-                const int64_t c = c0 + 32 * ct + col;
-                float old[16];
+    for (int i = 0; i < 16; i++) part[wave][i][lane] = acc[i];
+    __syncthreads();
 #pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int64_t r = r0 + 32 * rt + 8 * (i >> 2) + 4 * h + (i & 3);
-                    if (r < m && c < n) old[i] = y[r * n + c];
-                }
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int64_t r = r0 + 32 * rt + 8 * (i >> 2) + 4 * h + (i & 3);
-                    if (r < m && c < n) y[r * n + c] = old[i] + (SUB ? -acc[rt][ct][i] : acc[rt][ct][i]);
-                }
-            }
+    for (int j = 0; j < 4; j++) {
+        const int i = 4 * wave + j;
+        const float t = ((part[0][i][lane] + part[1][i][lane]) + part[2][i][lane]) + part[3][i][lane];
+        if (r + j < m && c < n) y[(r + j) * n + c] = old[j] + (SUB ? -t : t);
     }
 }
 
-template <bool SHARE>
-__global__ void __launch_bounds__(256) min32_mfma_kernel(const uint16_t *__restrict__ mins, cq_act_view a, int64_t n, int64_t nb, int64_t m,
-                                                         float *__restrict__ y) {
-    constexpr int RT = SHARE ? 1 : 2, CT = SHARE ? 1 : 2;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5;
-    const int64_t r0 = (int64_t)blockIdx.y * 32 * RT, c0 = ((int64_t)blockIdx.x * (SHARE ? 1 : 4) + (SHARE ? 0 : wave)) * 32 * CT;
-    v16f acc[RT][CT];
+__device__ __forceinline__ void load_scales(const float *row, int64_t b, int64_t nb, float (&d)[8]) {
+    if (b + 8 <= nb) {
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++)
+        for (int i = 0; i < 8; i++) d[i] = row[b + i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++) d[i] = b + i < nb ? row[b + i] : 0.0f;
+    }
+}
+// The s fields of eight blocks.
+__device__ __forceinline__ v8h scaled_sums(const HalfRow &sums, const float (&d)[8]) {
+    v8h s;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float hs = (float)(_Float16)(float)(int16_t)(sums.w[i >> 1] >> (16 * (i & 1)));
+        s[i] = (_Float16)(hs * d[i]);
+    }
+    return s;
+}
+struct Raw32 {
+    HalfRow mins, sums;
+    float d[8];
+};
+__device__ __forceinline__ void load_raw32(const uint16_t *mins, const cq_act_view &a, int64_t col, int64_t row, int64_t b, int64_t nb, Raw32 &o) {
+    o.mins = load_eight(mins, col, b, nb);
+    o.sums = load_eight(a.bsum32, row, b, nb);
+    load_scales(a.d + row * nb, b, nb, o.d);
+}
+
+// The steps of a 32 x 32 tile dealt to the waves.
+__global__ void __launch_bounds__(256) min32_shared_kernel(const uint16_t *__restrict__ mins, cq_act_view a, int64_t n, int64_t nb, int64_t m, float *y) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5;
+    const int64_t r0 = (int64_t)blockIdx.y * 32, c0 = (int64_t)blockIdx.x * 32;
+    // (rows and weight rows past the end repeat the last one; their results are not stored)
+    const int64_t row = r0 + (lane & 31) < m ? r0 + (lane & 31) : m - 1, col = c0 + (lane & 31) < n ? c0 + (lane & 31) : n - 1;
+    v16f acc;
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = 0.0f;
+    Raw32 cur, nxt;
+    int64_t b0 = 16 * wave;
+    if (b0 < nb) load_raw32(mins, a, col, row, b0 + 8 * h, nb, cur);
+    for (; b0 < nb; b0 += 64) {
+        if (b0 + 64 < nb) load_raw32(mins, a, col, row, b0 + 64 + 8 * h, nb, nxt);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(scaled_sums(cur.sums, cur.d), __builtin_bit_cast(v8h, cur.mins), acc, 0, 0, 0);
+        cur = nxt;
+    }
+    add_shared_tile<false>(acc, r0, c0, m, n, y);
+}
+// Every wave a 32 x 64 tile, the workgroup's four side by side.  The rows' s values are formed once a workgroup, 64 blocks at a time, in LDS; the
+// minima of a weight row are read four steps at once, a whole line.  (Step by step a wave takes 32 bytes of every line it touches and the
+// line is gone before the next step: four times the traffic from L2, 38 us of the 134 at 14336 x 4096 with 512 rows.)
+__global__ void __launch_bounds__(256) min32_tiles_kernel(const uint16_t *__restrict__ mins, cq_act_view a, int64_t n, int64_t nb, int64_t m, float *y) {
+    constexpr int CT = 2, kAhead = 64, kRow = kAhead + 8;   // (rows of 144 bytes: 16-byte reads of 32 rows meet every bank equally often)
+    __shared__ __align__(16) _Float16 sv[32 * kRow];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5;
+    const int64_t r0 = (int64_t)blockIdx.y * 32, c0 = ((int64_t)blockIdx.x * 4 + wave) * 32 * CT;
+    const int srow = threadIdx.x >> 3, sblk = (threadIdx.x & 7) * 8;   // the s values this thread forms
+    const int64_t row = r0 + srow < m ? r0 + srow : m - 1;
+    v16f acc[CT], old[CT];
+    int64_t cols[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        cols[ct] = c0 + 32 * ct + (lane & 31) < n ? c0 + 32 * ct + (lane & 31) : n - 1;
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[ct][i] = 0.0f;
+    }
+    for (int64_t b0 = 0; b0 < nb; b0 += kAhead) {
+        HalfRow mw[4][CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ct++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) acc[rt][ct][i] = 0.0f;
-    int64_t rows[RT], cols[CT];   // (rows and weight rows past the end repeat the last one; their results are not stored)
+            for (int s = 0; s < 4; s++) mw[s][ct] = load_eight(mins, cols[ct], b0 + 16 * s + 8 * h, nb);
+        float d[8];
+        const HalfRow sums = load_eight(a.bsum32, row, b0 + sblk, nb);
+        load_scales(a.d + row * nb, b0 + sblk, nb, d);
+        if (b0 + kAhead >= nb) {   // (behind the last operands)
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) rows[rt] = r0 + 32 * rt + (lane & 31) < m ? r0 + 32 * rt + (lane & 31) : m - 1;
+            for (int ct = 0; ct < CT; ct++) load_tile(y, r0, c0 + 32 * ct + (lane & 31), m, n, h, old[ct]);
+        }
+        if (b0) __syncthreads();   // the values of the blocks before have been read
+        *(v8h *)(sv + srow * kRow + sblk) = scaled_sums(sums, d);
+        __syncthreads();
 #pragma unroll
-    for (int ct = 0; ct < CT; ct++) cols[ct] = c0 + 32 * ct + (lane & 31) < n ? c0 + 32 * ct + (lane & 31) : n - 1;
-    if (SHARE || c0 < n) {
-        for (int64_t b0 = SHARE ? 16 * wave : 0; b0 < nb; b0 += SHARE ? 64 : 16) {
-            const int64_t b = b0 + 8 * h;
-            v8h mv[CT], sv[RT];
+        for (int s = 0; s < 4; s++) {   // (blocks past the end: both factors zero)
+            const v8h op = *(const v8h *)(sv + (lane & 31) * kRow + 16 * s + 8 * h);
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++) mv[ct] = __builtin_bit_cast(v8h, load_eight(mins, cols[ct], b, nb));
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                const HalfRow sums = load_eight(a.bsum32, rows[rt], b, nb);
-                const float *d = a.d + rows[rt] * nb + b;
-                float dv[8];
-                if (b + 8 <= nb) {
-#pragma unroll
-                    for (int i = 0; i < 8; i++) dv[i] = d[i];
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; i++) dv[i] = b + i < nb ? d[i] : 0.0f;
-                }
-#pragma unroll
-                for (int i = 0; i < 8; i++) {   // (blocks past the end: both factors zero)
-                    const float hs = (float)(_Float16)(float)(int16_t)(sums.w[i >> 1] >> (16 * (i & 1)));
-                    sv[rt][i] = (_Float16)(hs * dv[i]);
-                }
-            }
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-                for (int ct = 0; ct < CT; ct++) acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv[rt], mv[ct], acc[rt][ct], 0, 0, 0);
+            for (int ct = 0; ct < CT; ct++) acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(op, __builtin_bit_cast(v8h, mw[s][ct]), acc[ct], 0, 0, 0);
         }
     }
-    add_tiles<SHARE, false, RT, CT>(acc, r0, c0, m, n, y);
+    add_tiles<false, CT>(acc, old, r0, c0, m, n, y);
 }
 
 // Few rows (decode, small batches): sixteen lanes per weight row, each a chunk of eight blocks out of 128 at a time; lane
@@ -178,58 +222,73 @@ __global__ void __launch_bounds__(256) min32_small_kernel(const uint16_t *__rest
 // ---- Q2K: the dmin term of its dot product with Q8K activations (k_quants.rs:727-733, :762) ----
 //   y[r, c] -= sum_b (d8[r, b] * h2f(dmin[c, b])) * float(sum_j bsums[r, b, j] * m[c, b, j])
 // Many rows: a block's sixteen products are one MFMA step, its result the exact integer; scaled and added block by block.
+template <int CT> struct Raw16 {
+    uint2 mins[CT];
+    uint16_t dmin[CT];
+    v8h sums;
+    float4 d[4];
+};
+template <int CT>
+__device__ __forceinline__ void load_raw16(const uint8_t *mins, const uint16_t *dmins, const cq_act_view &a, const int64_t (&cols)[CT], int64_t r0,
+                                           int64_t b, int64_t kb, int lane, Raw16<CT> &o) {
+    const int h = lane >> 5;
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        o.mins[ct] = *(const uint2 *)(mins + (cols[ct] * kb + b) * 16 + 8 * h);
+        o.dmin[ct] = dmins[cols[ct] * kb + b];
+    }
+    o.sums = *(const v8h *)(a.bsh + ((b * a.m_stride + r0 + (lane & 31)) * 16 + 8 * h));
+#pragma unroll
+    for (int g = 0; g < 4; g++) o.d[g] = *(const float4 *)(a.dT + b * a.m_stride + r0 + 8 * g + 4 * h);
+}
 template <bool SHARE>
 __global__ void __launch_bounds__(256) min16_mfma_kernel(const uint8_t *__restrict__ mins, const uint16_t *__restrict__ dmins, cq_act_view a,
-                                                         int64_t n, int64_t kb, int64_t m, float *__restrict__ y) {
-    constexpr int RT = SHARE ? 1 : 2, CT = SHARE ? 1 : 2;
+                                                         int64_t n, int64_t kb, int64_t m, float *y) {
+    constexpr int CT = SHARE ? 1 : 2;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = lane >> 5;
-    const int64_t r0 = (int64_t)blockIdx.y * 32 * RT, c0 = ((int64_t)blockIdx.x * (SHARE ? 1 : 4) + (SHARE ? 0 : wave)) * 32 * CT;
-    v16f acc[RT][CT];
-    v16f zero;
+    const int64_t r0 = (int64_t)blockIdx.y * 32, c0 = ((int64_t)blockIdx.x * (SHARE ? 1 : 4) + (SHARE ? 0 : wave)) * 32 * CT;
+    v16f acc[CT], old[CT], zero;
+    int64_t cols[CT];   // (weight rows past the end repeat the last one; rows past the end are the workspace's padding; neither is stored)
 #pragma unroll
     for (int i = 0; i < 16; i++) zero[i] = 0.0f;
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++) acc[rt][ct] = zero;
-    int64_t cols[CT];   // (weight rows past the end repeat the last one; rows past the end are the workspace's padding; neither is stored)
-#pragma unroll
-    for (int ct = 0; ct < CT; ct++) cols[ct] = c0 + 32 * ct + (lane & 31) < n ? c0 + 32 * ct + (lane & 31) : n - 1;
+    for (int ct = 0; ct < CT; ct++) {
+        cols[ct] = c0 + 32 * ct + (lane & 31) < n ? c0 + 32 * ct + (lane & 31) : n - 1;
+        acc[ct] = zero;
+    }
     if (SHARE || c0 < n) {
-        for (int64_t b = SHARE ? wave : 0; b < kb; b += SHARE ? 4 : 1) {
-            v8h mv[CT], sv[RT];
-            float dm[CT];
-            const _Float16 k1024 = (_Float16)1024.0f;
+        const int64_t step = SHARE ? 4 : 1;
+        Raw16<CT> cur, nxt;
+        int64_t b = SHARE ? wave : 0;
+        if (b < kb) load_raw16<CT>(mins, dmins, a, cols, r0, b, kb, lane, cur);
+        if constexpr (!SHARE) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++) load_tile(y, r0, c0 + 32 * ct + (lane & 31), m, n, h, old[ct]);
+        }
+        for (; b < kb; b += step) {
+            if (b + step < kb) load_raw16<CT>(mins, dmins, a, cols, r0, b + step, kb, lane, nxt);
 #pragma unroll
             for (int ct = 0; ct < CT; ct++) {
-                const uint2 w = *(const uint2 *)(mins + (cols[ct] * kb + b) * 16 + 8 * h);
-                dm[ct] = cq_h2f(dmins[cols[ct] * kb + b]);
+                const uint2 w = cur.mins[ct];
                 const uint32_t u[4] = {__builtin_amdgcn_perm(w.x, w.x, 0x0c010c00u) | 0x64006400u, __builtin_amdgcn_perm(w.x, w.x, 0x0c030c02u) | 0x64006400u,
                                        __builtin_amdgcn_perm(w.y, w.y, 0x0c010c00u) | 0x64006400u, __builtin_amdgcn_perm(w.y, w.y, 0x0c030c02u) | 0x64006400u};
-                mv[ct] = __builtin_bit_cast(v8h, u);   // 0x6400 | v is the f16 1024 + v
+                v8h mv = __builtin_bit_cast(v8h, u);   // 0x6400 | v is the f16 1024 + v
 #pragma unroll
-                for (int i = 0; i < 8; i++) mv[ct][i] -= k1024;
-            }
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) sv[rt] = *(const v8h *)(a.bsh + ((b * a.m_stride + r0 + 32 * rt + (lane & 31)) * 16 + 8 * h));
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                float dr[16];
+                for (int i = 0; i < 8; i++) mv[i] -= (_Float16)1024.0f;
+                const float dm = cq_h2f(cur.dmin[ct]);
+                const v16f s = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.sums, mv, zero, 0, 0, 0);
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
-                    const float4 f = *(const float4 *)(a.dT + b * a.m_stride + r0 + 32 * rt + 8 * g + 4 * h);
-                    dr[4 * g] = f.x, dr[4 * g + 1] = f.y, dr[4 * g + 2] = f.z, dr[4 * g + 3] = f.w;
-                }
+                    const float dr[4] = {cur.d[g].x, cur.d[g].y, cur.d[g].z, cur.d[g].w};
 #pragma unroll
-                for (int ct = 0; ct < CT; ct++) {
-                    const v16f s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv[rt], mv[ct], zero, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 16; i++) acc[rt][ct][i] += (dr[i] * dm[ct]) * s[i];
+                    for (int i = 0; i < 4; i++) acc[ct][4 * g + i] += (dr[i] * dm) * s[4 * g + i];
                 }
             }
+            cur = nxt;
         }
     }
-    add_tiles<SHARE, true, RT, CT>(acc, r0, c0, m, n, y);
+    if constexpr (SHARE) add_shared_tile<true>(acc[0], r0, c0, m, n, y);
+    else if (c0 < n) add_tiles<true, CT>(acc, old, r0, c0, m, n, y);
 }
 
 // Few rows (decode, small batches): sixteen lanes per weight row, each one block out of sixteen at a time; lane 0 of the
@@ -277,8 +336,8 @@ __global__ void __launch_bounds__(256) min16_small_kernel(const uint8_t *__restr
 
 // `apart`: a row's bits may not depend on how many rows there are.  For that, one kernel takes all of them (Q2K: its unshared tiles add
 // the blocks in the small kernel's order, with the same roundings).
-// Whether a tile of 64 x 64 for every wave would be fewer than one wave for each SIMD.
-static bool share_tile(const cq_weight *w, int64_t m) { return m <= 32 || ((w->n + 63) / 64) * ((m + 63) / 64) < 4 * cq_num_cus(); }
+// Whether a tile for every wave would be fewer than one wave for each SIMD.
+static bool share_tile(const cq_weight *w, int64_t m) { return ((w->n + 63) / 64) * ((m + 31) / 32) < 4 * cq_num_cus(); }
 
 hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool apart, hipStream_t s) {
     if (!cq_has_min32(w->ggml_dtype)) return hipErrorInvalidValue;
@@ -289,8 +348,8 @@ hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, fl
         CQ_LAUNCH(min32_small_kernel, dim3((unsigned)((w->n + 15) / 16), (unsigned)((m + kSmallRows - 1) / kSmallRows)), 256, 0, s, mins, a,
                   w->n, nb, m, y);
     else if (share_tile(w, m))
-        CQ_LAUNCH(min32_mfma_kernel<true>, dim3((unsigned)((w->n + 31) / 32), (unsigned)((m + 31) / 32)), 256, 0, s, mins, a, w->n, nb, m, y);
-    else CQ_LAUNCH(min32_mfma_kernel<false>, dim3((unsigned)((w->n + 255) / 256), (unsigned)((m + 63) / 64)), 256, 0, s, mins, a, w->n, nb, m, y);
+        CQ_LAUNCH(min32_shared_kernel, dim3((unsigned)((w->n + 31) / 32), (unsigned)((m + 31) / 32)), 256, 0, s, mins, a, w->n, nb, m, y);
+    else CQ_LAUNCH(min32_tiles_kernel, dim3((unsigned)((w->n + 255) / 256), (unsigned)((m + 31) / 32)), 256, 0, s, mins, a, w->n, nb, m, y);
     return hipGetLastError();
 }
 
@@ -304,6 +363,6 @@ hipError_t cq_launch_min16_term(const cq_weight *w, cq_act_view a, int64_t m, fl
                   dmins, a, w->n, kb, m, y);
     else if (!apart && share_tile(w, m))
         CQ_LAUNCH(min16_mfma_kernel<true>, dim3((unsigned)((w->n + 31) / 32), (unsigned)((m + 31) / 32)), 256, 0, s, w->p4, dmins, a, w->n, kb, m, y);
-    else CQ_LAUNCH(min16_mfma_kernel<false>, dim3((unsigned)((w->n + 255) / 256), (unsigned)((m + 63) / 64)), 256, 0, s, w->p4, dmins, a, w->n, kb, m, y);
+    else CQ_LAUNCH(min16_mfma_kernel<false>, dim3((unsigned)((w->n + 255) / 256), (unsigned)((m + 31) / 32)), 256, 0, s, w->p4, dmins, a, w->n, kb, m, y);
     return hipGetLastError();
 }
