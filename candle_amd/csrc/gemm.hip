@@ -1117,6 +1117,7 @@ struct Plan {
     int mt, ksplit;
     int kh = 1;   // 2: gemm_kh_kernel (K halved inside the workgroup, 128 weight rows per workgroup)
     int tail = 0; // 1, 2: gemm_tail_kernel, the last round's tiles in heights of 32 * tail rows
+    double work = 0.0, merge = 0.0;   // the cost: workgroups, adding up the parts
 };
 Plan pick_plan(const cq_weight *w, int64_t m) {
     const int64_t gx = n_tiles(w), kb = w->k >> 8, cus = cq_num_cus();
@@ -1133,8 +1134,8 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
             if (ks > 1 && kb / ks < 4) break;
             if (ks > 1 && cq_no_split_k()) break;   // CQ_FLAG_DETERMINISTIC
             const int64_t rounds = (tiles * ks + cus - 1) / cus;
-            double cost = (double)rounds * ((double)((kb + ks - 1) / ks) * (unpack + 13.5 * mt) + 24.0) +
-                                (ks > 1 ? ks * atomic_pass : 0.0);
+            const double merge = ks > 1 ? ks * atomic_pass : 0.0;
+            double cost = (double)rounds * ((double)((kb + ks - 1) / ks) * (unpack + 13.5 * mt) + 24.0) + merge;
             // A last round that is at most half full (or a quarter), in shorter tiles: nothing else runs beside it, so it lasts
             // as long as one of its tiles.  Whole calls, us, one height -> two: Q4K 11008 x 4096 at 4096 / 1024 rows 454 -> 424 /
             // 137 -> 120, 14336 x 4096 at 2048 282 -> 267, 5120 x 5120 at 2000 158 -> 134, 8448 x 2048 at 1024 78 -> 60; Q6K
@@ -1149,7 +1150,7 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
                 }
             }
             if (first || cost < best_cost) {
-                best = Plan{mt, ks, 1, tail};
+                best = Plan{mt, ks, 1, tail, cost - merge, merge};
                 best_cost = cost;
                 first = false;
             }
@@ -1167,7 +1168,7 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
         const int64_t rounds = 1;
         const double cost = (double)rounds * ((double)((kb + 1) / 2) * (unpack + 13.5 * mt) + 24.0 + 8.0);
         if (cost < best_cost) {
-            best = Plan{mt, 1, 2};
+            best = Plan{mt, 1, 2, 0, cost, 0.0};
             best_cost = cost;
         }
     }
@@ -1346,6 +1347,13 @@ bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, co
     return cq_group_tiles(offsets, n_experts, 32) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
 }
 
+// us of the tile launch beside the quantizer and the stores, from the plan's cost (fitted to the calls of groups_us in skinny.hip: 5 % rms).
+double cq_gemm_us(const cq_weight *w, int64_t m) {
+    const Plan p = pick_plan(w, m);
+    const int t = w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2;
+    static constexpr double start[3] = {5.3, 5.3, 5.8}, work[3] = {0.67, 0.79, 0.52}, merge[3] = {1.02, 1.02, 1.12};
+    return start[t] + (work[t] * p.work + merge[t] * p.merge) / 16.0;
+}
 bool cq_gemm_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }
 
 bool cq_gemm_takes(const cq_weight *w, int act_dtype) {
