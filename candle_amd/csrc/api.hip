@@ -620,11 +620,12 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     // (weights of 33 to 127 rows that are no whole number of 32-row tiles stay with the split-K kernel)
     const bool has_tile_kernel = cq_gemm_supported(w, m, act) || (w->n >= 128 && cq_gemm_takes(w, act));
     const bool has_tile32 = m > 16 && (cq_gemm32_supported(w, act) || (w->n >= 128 && cq_gemm32_takes(w, act)));
-    //   (K-quants) where its groups of rows are well ahead by the two estimates: small weights, whose tiles leave most of the machine idle.
+    //   where its groups of rows are well ahead by the two estimates: small weights, whose tiles leave most of the machine idle.
     //   The factor keeps the calls whose estimates are too close to tell: over 3500 shapes the choice is slower than the tile kernel by more than
     //   3 % in 0.3 %, and 22 % faster on average.
+    const auto groups_ahead = [&] { return cq_skinny_in_groups(w, m) && 1.2 * cq_skinny_groups_us(w, m) < (has_tile32 ? cq_gemm32_us(w, m) : cq_gemm_us(w, m)); };
     const bool skinny_rows = m <= 16 || (m <= 24 && w->n < 14336) || (m <= 32 && w->n < 12288) || (m <= 64 && w->n < 8192 && w->k <= 6144) ||
-                             (cq_skinny_in_groups(w, m) && 1.2 * cq_skinny_groups_us(w, m) < cq_gemm_us(w, m));
+                             (!has_tile32 && groups_ahead());
     if (flags & CQ_FLAG_FORCE_SKINNY) {
         if (!cq_skinny_supported(w, act))
             return cq_set_error(CQ_ERR_UNSUPPORTED, "no split-K MFMA kernel for dtype %d with activation dtype %d and n = %lld",
@@ -636,7 +637,7 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
         // against 7.7, 4096 x 4096 12.1 / 13.6 against 11.8 / 12.8, 4096 x 14336 20.0 / 23.1 against 24.9 / 27.7; Q4_0 4096 x 4096
         // 11.7 / 13.3 against 9.7 / 10.3, 8192 x 4096 14.2 / 17.2 against 12.3 / 15.4, 11008 x 4096 17.6 / 19.4 against 16.8 / 22.3)
         const int64_t small = w->dtype == CQ_DTYPE_Q8_0 ? (1 << 24) : (1 << 25);
-        const bool few = !(flags & CQ_FLAG_FORCE_GEMM) && m <= 32 && w->n <= 8192 && w->n * w->k <= small && cq_skinny_takes(w, act);
+        const bool few = !(flags & CQ_FLAG_FORCE_GEMM) && cq_skinny_takes(w, act) && ((m <= 32 && w->n <= 8192 && w->n * w->k <= small) || groups_ahead());
         path = few ? kSkinny : kGemm32;
     } else if (!(flags & (CQ_FLAG_FORCE_GEMM | CQ_FLAG_FORCE_MATVEC)) && (m >= skinny_from || (m >= 2 && !rows_fused)) &&
                cq_skinny_takes(w, act) && (skinny_rows || !has_tile_kernel)) {

@@ -516,6 +516,7 @@ struct Plan {
     int tail = 0;   // 1, 2: gemm32_tail_kernel, the last round's tiles in heights of 32 * tail rows
     int kh = 0;     // 1: gemm32_kh_kernel
     int few = 0;    // 1, 2, 4, 8: gemm32_few_kernel with that many column tiles a workgroup
+    double work = 0.0, merge = 0.0;   // the cost: workgroups, adding up the parts
 };
 Plan pick_plan(const cq_weight *w, int64_t m) {
     const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks_total = (w->k + 255) >> 8, cus = cq_num_cus();
@@ -530,8 +531,8 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
             if (ks > 1 && ks_total / ks < 2) break;
             if (ks > 1 && cq_no_split_k()) break;   // CQ_FLAG_DETERMINISTIC
             const int64_t rounds = (tiles * ks + cus - 1) / cus;
-            double cost = (double)rounds * ((double)((ks_total + ks - 1) / ks) * (10.0 + 23.0 * mt) + 24.0) +
-                                (ks > 1 ? ks * atomic_pass : 0.0);
+            const double merge = ks > 1 ? ks * atomic_pass : 0.0;
+            double cost = (double)rounds * ((double)((ks_total + ks - 1) / ks) * (10.0 + 23.0 * mt) + 24.0) + merge;
             // A last round that is at most half full (or a quarter), in shorter tiles.  Whole calls, us, one height -> two: Q8_0
             // 11008 x 4096 at 4096 / 1024 rows 610 -> 580 / 181 -> 163, 5120 x 5120 at 2000 229 -> 178, 8448 x 2048 at 1024
             // 99 -> 77; Q4_0 4096 x 14336 at 2300 512 -> 456.
@@ -542,7 +543,7 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
                 tail = t;
             }
             if (first || cost < best_cost) {
-                best = Plan{mt, ks, tail};
+                best = Plan{mt, ks, tail, 0, 0, cost - merge, merge};
                 best_cost = cost;
                 first = false;
             }
@@ -556,7 +557,7 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
         if ((w->n + 127) / 128 * ((m + mt * 32 - 1) / (mt * 32)) > cus) continue;
         const double cost = (double)((ks_total + 1) / 2) * (11.0 + 22.0 * mt) + 40.0;
         if (cost < best_cost) {
-            best = Plan{mt, 1, 0, 1};
+            best = Plan{mt, 1, 0, 1, 0, cost, 0.0};
             best_cost = cost;
         }
     }
@@ -565,7 +566,7 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
         if (groups > (cw == 1 && w->dtype == CQ_DTYPE_Q8_0 ? cus / 2 : cus)) continue;
         const double cost = (double)((ks_total + parts - 1) / parts) * 30.0 + 29.0;
         if (cost < best_cost) {
-            best = Plan{1, 1, 0, 0, cw};
+            best = Plan{1, 1, 0, 0, cw, cost, 0.0};
             best_cost = cost;
         }
     }
@@ -746,6 +747,13 @@ bool cq_gemm32_supported(const cq_weight *w, int act_dtype) {
     return cq_gemm32_takes(w, act_dtype) && w->k % 256 == 0 && w->n % 32 == 0;
 }
 
+// us of the tile launch beside the quantizer and the stores, from the plan's cost (fitted to the calls of groups_us in skinny.hip: 6 % rms).
+double cq_gemm32_us(const cq_weight *w, int64_t m) {
+    const Plan p = pick_plan(w, m);
+    const int t = w->dtype == CQ_DTYPE_Q8_0 ? 0 : 1, form = p.few ? 2 : p.kh ? 1 : 0;
+    static constexpr double start[2][3] = {{4.6, 3.25, 2.9}, {4.9, 3.7, 3.65}}, work[2][3] = {{0.97, 1.07, 1.30}, {0.92, 1.0, 1.16}};
+    return start[t][form] + (work[t][form] * p.work + (t ? 1.13 : 1.33) * p.merge) / 16.0;
+}
 bool cq_gemm32_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }
 
 hipError_t cq_launch_gemm32(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, bool y_cleared,

@@ -213,11 +213,12 @@ bool cq_gemm32_grouped_splits_k(const cq_weight *const *experts, int n_experts, 
 bool cq_skinny_takes(const cq_weight *w, int act_dtype);
 bool cq_skinny_supported(const cq_weight *w, int act_dtype);
 hipError_t cq_launch_skinny(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, hipStream_t s);
-// more than 16 rows of a K-quant in groups of rows beside each other in one launch, and what that takes (us, beside the quantizer and
-// the stores; the tile kernel the same way)
+// more than 16 rows in groups of rows beside each other in one launch, and what that takes (us, beside the quantizer and
+// the stores; the tile kernels the same way)
 bool cq_skinny_in_groups(const cq_weight *w, int64_t m);
 double cq_skinny_groups_us(const cq_weight *w, int64_t m);
 double cq_gemm_us(const cq_weight *w, int64_t m);
+double cq_gemm32_us(const cq_weight *w, int64_t m);
 // up to eight rows of a small weight in one launch that quantizes them itself (and leaves them in the workspace)
 bool cq_skinny_direct_takes(const cq_weight *w, int act_dtype, int64_t m);
 hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s);

@@ -1555,43 +1555,8 @@ hipError_t launch_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, f
     return sixteen ? launch_waves<DT, RT, DUMP, kMany, false>(w, a, m0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, false>(w, a, m0, m, y, d, s);
 }
 
-// All the rows in one launch, 8 * RT of them to a workgroup.
-template <int DT, int RT>
-hipError_t launch_groups(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
-    const cq_mfma_dump none{nullptr, nullptr, 0};
-    const int64_t most = (int64_t)8 * RT * 65535;
-    for (int64_t m0 = 0; m0 < m; m0 += most) {
-        const unsigned groups = (unsigned)(((m - m0 < most ? m - m0 : most) + 8 * RT - 1) / (8 * RT));
-        hipError_t e = hipErrorInvalidValue;
-        if (!has_offset(*w)) e = launch_waves<DT, RT, false, kWaves, false>(w, a, m0, m, y, none, s, groups);
-        else if constexpr (kCanOffset<DT, false>) e = launch_waves<DT, RT, false, kWaves, true>(w, a, m0, m, y, none, s, groups);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
-}
-// More than 16 rows, us beside the quantizer and the stores: groups of 16 and of 32 rows.  A workgroup goes through a row in steps of eight blocks,
-// one a wave; three or two of them share a CU with 16 rows, one with 32 (LDS).  Fitted to 35000 measured calls of Q4K, Q5K and Q6K (24 to
-// 9400 weight rows, k 256 to 15104, 17 to 1024 rows), 8 and 7 % rms.
-struct GroupsUs {
-    double sixteen, thirty_two;
-};
-GroupsUs groups_us(const cq_weight *w, int64_t m) {
-    const int t = w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2;
-    const double tiles = (double)((w->n + 15) / 16), cus = (double)cq_num_cus(), steps = (double)((w->k + 2047) / 2048);
-    const double f16 = tiles * (double)((m + 15) / 16) / cus, f32 = tiles * (double)((m + 31) / 32) / cus, rounds = f32 <= 1.0 ? 1.0 : ceil(f32);
-    static constexpr double a16[3] = {0.94, 1.19, 1.05}, b16[3] = {0.62, 0.94, 0.88};
-    static constexpr double a32[3] = {1.25, 1.65, 1.46}, b32[3] = {0.16, 0.22, 0.23}, c32[3] = {0.49, 0.32, 0.41};
-    return {5.35 + steps * (a16[t] + b16[t] * f16), 5.15 + steps * (a32[t] * rounds + b32[t] * f32) + c32[t] * rounds};
-}
-
 template <int DT, bool DUMP>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    if constexpr (!DUMP) {
-        if (cq_skinny_in_groups(w, m)) {
-            const GroupsUs us = groups_us(w, m);
-            return us.sixteen <= us.thirty_two || m <= 32 ? launch_groups<DT, 2>(w, a, m, y, s) : launch_groups<DT, 4>(w, a, m, y, s);
-        }
-    }
     for (int64_t m0 = 0; m0 < m; m0 += 32) {
         const int64_t left = m - m0;
         hipError_t e;
@@ -1734,20 +1699,75 @@ hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const 
     }
 }
 
+// All the rows in one launch, 8 * RT of them to a workgroup.
+template <int DT, int RT, bool OFF>
+hipError_t launch_groups_inst(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, hipStream_t s, unsigned groups) {
+    const cq_mfma_dump none{nullptr, nullptr, 0};
+    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) return launch_blk32_waves<DT, RT, false, kWaves, OFF>(w, a, m0, m, y, none, s, groups);
+    else return launch_waves<DT, RT, false, kWaves, OFF>(w, a, m0, m, y, none, s, groups);
+}
+template <int DT, int RT>
+hipError_t launch_groups(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+    const int64_t most = (int64_t)8 * RT * 65535;
+    for (int64_t m0 = 0; m0 < m; m0 += most) {
+        const unsigned groups = (unsigned)(((m - m0 < most ? m - m0 : most) + 8 * RT - 1) / (8 * RT));
+        hipError_t e = hipErrorInvalidValue;
+        if (!has_offset(*w)) e = launch_groups_inst<DT, RT, false>(w, a, m0, m, y, s, groups);
+        else if constexpr (kCanOffset<DT, false>) e = launch_groups_inst<DT, RT, true>(w, a, m0, m, y, s, groups);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+// More than 16 rows, us beside the quantizer and the stores: groups of 16 and (K-quants) of 32 rows.  A workgroup goes through a row in steps of
+// 2048 elements, 256 a wave; three or two of them share a CU with 16 rows, one with 32 (LDS; groups of 32 are never ahead for Q8_0 and Q4_0).
+// Fitted to 35000 measured calls of Q4K, Q5K and Q6K and 21000 of Q8_0 and Q4_0 (24 to 9400 weight rows, k 256 to 15104, 17 to 1024 rows), 7 to 9 %
+// rms.
+struct GroupsUs {
+    double sixteen, thirty_two;
+};
+GroupsUs groups_us(const cq_weight *w, int64_t m) {
+    const double tiles = (double)((w->n + 15) / 16), cus = (double)cq_num_cus(), steps = (double)((w->k + 2047) / 2048);
+    const double f16 = tiles * (double)((m + 15) / 16) / cus, f32 = tiles * (double)((m + 31) / 32) / cus, rounds = f32 <= 1.0 ? 1.0 : ceil(f32);
+    if (w->dtype == CQ_DTYPE_Q8_0) return {5.0 + steps * (1.19 + 0.96 * f16), 1e30};
+    if (w->dtype == CQ_DTYPE_Q4_0) return {5.15 + steps * (1.25 + 0.66 * f16), 1e30};
+    const int t = w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2;
+    static constexpr double a16[3] = {0.94, 1.19, 1.05}, b16[3] = {0.62, 0.94, 0.88};
+    static constexpr double a32[3] = {1.25, 1.65, 1.46}, b32[3] = {0.16, 0.22, 0.23}, c32[3] = {0.49, 0.32, 0.41};
+    return {5.35 + steps * (a16[t] + b16[t] * f16), 5.15 + steps * (a32[t] * rounds + b32[t] * f32) + c32[t] * rounds};
+}
+
+template <int DT>
+hipError_t launch_in_groups(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+    const GroupsUs us = groups_us(w, m);
+    if (us.sixteen <= us.thirty_two || m <= 32) return launch_groups<DT, 2>(w, a, m, y, s);
+    if constexpr (DT != CQ_DTYPE_Q8_0 && DT != CQ_DTYPE_Q4_0) return launch_groups<DT, 4>(w, a, m, y, s);
+    return hipErrorInvalidValue;
+}
+
 template <bool DUMP>
 hipError_t launch_any(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     if (!cq_skinny_takes(w, act_dtype)) return hipErrorNotSupported;
     if (m == 0) return hipSuccess;
     if (a.m_stride < (m + 31) / 32 * 32) return hipErrorInvalidValue;   // whole 8-row groups are copied
     hipError_t e = hipSuccess;
+    if constexpr (!DUMP) {
+        if (cq_skinny_in_groups(w, m)) {
+            switch (w->dtype) {
+            case CQ_DTYPE_Q8_0: return launch_in_groups<CQ_DTYPE_Q8_0>(w, a, m, y, s);
+            case CQ_DTYPE_Q4_0: return launch_in_groups<CQ_DTYPE_Q4_0>(w, a, m, y, s);
+            case CQ_DTYPE_Q4K: return launch_in_groups<CQ_DTYPE_Q4K>(w, a, m, y, s);
+            case CQ_DTYPE_Q5K: return launch_in_groups<CQ_DTYPE_Q5K>(w, a, m, y, s);
+            default: return launch_in_groups<CQ_DTYPE_Q6K>(w, a, m, y, s);
+            }
+        }
+    }
     if (w->dtype == CQ_DTYPE_Q8_0 && launch_blk32_res<CQ_DTYPE_Q8_0, DUMP>(w, a, m, y, d, s, &e)) return e;
     if (w->dtype == CQ_DTYPE_Q4_0 && launch_blk32_res<CQ_DTYPE_Q4_0, DUMP>(w, a, m, y, d, s, &e)) return e;
     if (w->dtype == CQ_DTYPE_Q8_0) return launch_blk32<CQ_DTYPE_Q8_0, DUMP>(w, a, m, y, d, s);
     if (w->dtype == CQ_DTYPE_Q4_0) return launch_blk32<CQ_DTYPE_Q4_0, DUMP>(w, a, m, y, d, s);
-    const bool in_groups = !DUMP && cq_skinny_in_groups(w, m);
-    if (w->dtype == CQ_DTYPE_Q4K && !in_groups && launch_res<CQ_DTYPE_Q4K, DUMP>(w, a, m, y, d, s, &e)) return e;
-    if (w->dtype == CQ_DTYPE_Q5K && !in_groups && launch_res<CQ_DTYPE_Q5K, DUMP>(w, a, m, y, d, s, &e)) return e;
-    if (w->dtype == CQ_DTYPE_Q6K && !in_groups && launch_res<CQ_DTYPE_Q6K, DUMP>(w, a, m, y, d, s, &e)) return e;
+    if (w->dtype == CQ_DTYPE_Q4K && launch_res<CQ_DTYPE_Q4K, DUMP>(w, a, m, y, d, s, &e)) return e;
+    if (w->dtype == CQ_DTYPE_Q5K && launch_res<CQ_DTYPE_Q5K, DUMP>(w, a, m, y, d, s, &e)) return e;
+    if (w->dtype == CQ_DTYPE_Q6K && launch_res<CQ_DTYPE_Q6K, DUMP>(w, a, m, y, d, s, &e)) return e;
     if (w->dtype == CQ_DTYPE_Q4K) return launch_dt<CQ_DTYPE_Q4K, DUMP>(w, a, m, y, d, s);
     if (w->dtype == CQ_DTYPE_Q5K) return launch_dt<CQ_DTYPE_Q5K, DUMP>(w, a, m, y, d, s);
     return launch_dt<CQ_DTYPE_Q6K, DUMP>(w, a, m, y, d, s);
@@ -1768,13 +1788,15 @@ bool cq_skinny_takes(const cq_weight *w, int act_dtype) {
     const bool q8 = (w->dtype == CQ_DTYPE_Q8_0 || w->dtype == CQ_DTYPE_Q4_0) && act_dtype == CQ_DTYPE_Q8_0 && w->k % 64 == 0;
     return (kquant || q8) && w->k >= 256 && w->k <= (1 << 24) && w->n >= 16;
 }
-// More than 16 rows of a K-quant in groups of 16 or 32, one launch: beyond 32 rows always (against a launch for every 32 rows), up to 32 where a
-// group of 16 for every CU does it and a wave has more than one block (the resident kernel is as fast below).  Whole calls, us, before -> groups:
-// Q4K 1024 x 4096 with 24 / 64 / 128 rows 9.4 -> 7.7 / 13.9 -> 8.3 / 14.0 -> 9.4, 411 x 3584 with 128 17.6 -> 8.6, Q6K 512 x 4096 with 33 13.4 ->
-// 8.1, 2048 x 2048 with 64 11.7 -> 7.7, Q3K 256 x 13312 with 52 22.0 -> 13.9; 48 x 3072 with 256 rows (no tile kernel) 39 -> 8.2.
+// More than 16 rows in groups of 16 or 32, one launch: beyond 32 rows always (against a launch for every 32 rows), up to 32 where a group of 16 for
+// every CU does it (K-quants: and a wave has more than one block; the resident kernel is as fast below.  Q8_0 / Q4_0 with one step: two
+// groups for every CU).  Whole calls, us, before -> groups: Q4K 1024 x 4096 with 24 / 64 / 128 rows 9.4 -> 7.7 / 13.9 -> 8.3 / 14.0 -> 9.4, 411 x
+// 3584 with 128 17.6 -> 8.6, Q6K 512 x 4096 with 33 13.4 -> 8.1, 2048 x 2048 with 64 11.7 -> 7.7, Q3K 256 x 13312 with 52 22.0 -> 13.9, Q8_0 1528 x 960
+// with 48 11.3 -> 7.2; without a tile kernel Q4K 48 x 3072 with 256 rows 39 -> 8.2, Q8_0 28 x 1920 with 48 11.1 -> 6.8.
 bool cq_skinny_in_groups(const cq_weight *w, int64_t m) {
-    const bool kquant = w->dtype == CQ_DTYPE_Q4K || w->dtype == CQ_DTYPE_Q5K || w->dtype == CQ_DTYPE_Q6K;
-    return kquant && (m > 32 || (m > 16 && w->k > 8 * QK_K && (w->n + 15) / 16 * 2 <= cq_num_cus()));
+    const bool blk32 = w->dtype == CQ_DTYPE_Q8_0 || w->dtype == CQ_DTYPE_Q4_0, one_step = w->k <= 8 * QK_K;
+    const int64_t pairs = (w->n + 15) / 16 * 2, cus = cq_num_cus();   // groups of 16 with up to 32 rows
+    return m > 32 || (m > 16 && (blk32 ? pairs <= (one_step ? 2 : 1) * cus : !one_step && pairs <= cus));
 }
 double cq_skinny_groups_us(const cq_weight *w, int64_t m) {
     const GroupsUs us = groups_us(w, m);

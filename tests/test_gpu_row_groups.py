@@ -11,18 +11,29 @@ from tests.test_gpu_few_rows_long import close
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K", "Q3K", "Q2K"])
+@pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K", "Q3K", "Q2K", "Q8_0", "Q4_0", "Q4_1", "Q5_1"])
 @pytest.mark.parametrize("m,n,k", [(17, 16, 2304), (31, 2048, 2560), (33, 33, 256), (40, 1000, 2304), (48, 130, 13312), (64, 384, 512), (100, 411, 3584),
                                    (257, 40, 256), (500, 256, 1024), (96, 2047, 1792), (128, 1024, 4096), (1025, 24, 768)])
 def test_groups(qh, dt, m, n, k):  # noqa: F811
+    run(qh, dt, m, n, k)
+
+
+def run(qh, dt, m, n, k):  # noqa: F811
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     w = QTensor.quantize(torch.randn(n, k, generator=g, device="cuda") * 0.02, GgmlDType[dt]).weight
     x = torch.randn(m, k, generator=g, device="cuda")
     out = torch.full((m + 1, n), 7.0, device="cuda")
     qh.qmatmul(w, x, out=out[:m])
     assert bool((out[m] == 7.0).all())
-    close(out[:m], qh.qmatmul(w, x, qh.FLAG_FORCE_MATVEC | qh.FLAG_STAGED_ACT), k // 256)
+    close(out[:m], qh.qmatmul(w, x, qh.FLAG_FORCE_MATVEC | qh.FLAG_STAGED_ACT), k // (256 if dt.endswith("K") else 32))
     bad = x.clone()
     bad[m // 2, 3], bad[m // 2, k - 1] = float("inf"), float("nan")
     keep = [r for r in range(m) if r != m // 2]
-    assert torch.equal(qh.qmatmul(w, bad)[keep], out[keep])
+    # (shapes whose choice is the tile kernel: without parts added up atomically)
+    assert torch.equal(qh.qmatmul(w, bad, qh.FLAG_DETERMINISTIC)[keep], qh.qmatmul(w, x, qh.FLAG_DETERMINISTIC)[keep])
+
+
+@pytest.mark.parametrize("dt", ["Q8_0", "Q4_0", "Q5_0", "Q4_1"])
+@pytest.mark.parametrize("m,n,k", [(17, 16, 320), (20, 2050, 2112), (33, 100, 4160), (129, 31, 576), (40, 1500, 960)])
+def test_steps_of_no_whole_length(qh, dt, m, n, k):  # noqa: F811
+    run(qh, dt, m, n, k)
