@@ -668,7 +668,7 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     cq_act_view v;
     act_ws_layout(act, m, w->k, (uint8_t *)ws, &v);
     bool y_cleared = false;
-    // a few more rows of a small weight: quantized by the waves of the split-K kernel, which leaves them in the workspace as well
+    // a small weight: the rows quantized by the waves of the split-K kernel, which leaves them in the workspace as well
     const bool direct = flags == 0 && pre.kind == CQ_PRE_NONE && !in_place && path == kSkinny && cq_skinny_direct_takes(w, act, m);
     if (!(flags & CQ_FLAG_REUSE_ACT) && !direct) {
         cq_clear clear = cq_no_clear();

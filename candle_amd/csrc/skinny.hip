@@ -262,7 +262,7 @@ __device__ __forceinline__ void load_direct(const float *__restrict__ x, int64_t
 }
 // ... quantized into the wave's buffer, in the image the copies of quantized rows make; `keep`: into the workspace as well.
 template <int DT, int RT>
-__device__ __forceinline__ void quantize_direct(const float4 (&xf)[2 * RT][4], const cq_act_view &a, int64_t m, int64_t k, int64_t b, int lane,
+__device__ __forceinline__ void quantize_direct(const float4 (&xf)[2 * RT][4], const cq_act_view &a, int64_t m0, int64_t m, int64_t k, int64_t b, int lane,
                                                 bool keep, uint8_t *buf) {
     typedef Buf<DT, RT> B;
     const int l = lane & 15;
@@ -282,9 +282,9 @@ __device__ __forceinline__ void quantize_direct(const float4 (&xf)[2 * RT][4], c
         if (l == 0) *(float *)(buf + B::oD8 + row * 4) = d;
         if (is_k4(DT)) *(_Float16 *)(buf + B::oMin + row * 32 + sj * 2) = (_Float16)(float)bsum;
         if (keep) {
-            const int64_t blk = row * (k >> 8) + b, tb = b * a.m_stride + row;
+            const int64_t to = m0 + row, blk = to * (k >> 8) + b, tb = b * a.m_stride + to;
 #pragma unroll
-            for (int i = 0; i < 4; i++) *(uint32_t *)(a.qs + row * k + b * 256 + 64 * i + 4 * l) = packed[i];
+            for (int i = 0; i < 4; i++) *(uint32_t *)(a.qs + to * k + b * 256 + 64 * i + 4 * l) = packed[i];
             if (l == 0) {
                 a.d[blk] = d;
                 a.dT[tb] = d;
@@ -340,7 +340,7 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
         // ---- copies of block b: weights of the 16 rows, activation rows, their scales
         float4 xf[DIRECT ? 2 * RT : 1][4];
         if constexpr (DIRECT) {
-            load_direct<RT>(x, m, k, b, lane, xf);   // (first: what the quantizer waits for; requests are answered in order)
+            load_direct<RT>(x + m0 * k, m - m0, k, b, lane, xf);   // (first: what the quantizer waits for; requests are answered in order)
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
@@ -361,7 +361,7 @@ __device__ __forceinline__ void skinny_body(const cq_weight &w, const cq_act_vie
         load_head(w, (n_tile + r) * kb + b, head);
         if constexpr (DIRECT) {
             __builtin_amdgcn_sched_barrier(0);
-            quantize_direct<DT, RT>(xf, a, m, k, b, lane, tile == 0, buf);
+            quantize_direct<DT, RT>(xf, a, m0, m - m0, k, b, lane, tile == 0, buf);
         }
         __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
 
@@ -954,7 +954,7 @@ __device__ __forceinline__ void load_direct_q8(const float *__restrict__ x, int6
     for (int row = 0; row < 8 * RT; row++) xf[row] = row < m && e0 < k ? *(const float4 *)(x + row * k + e0) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 template <int DT, int RT>
-__device__ __forceinline__ void quantize_direct_q8(const float4 (&xf)[8 * RT], const cq_act_view &a, int64_t m, int64_t k, int64_t g, int lane,
+__device__ __forceinline__ void quantize_direct_q8(const float4 (&xf)[8 * RT], const cq_act_view &a, int64_t m0, int64_t m, int64_t k, int64_t g, int lane,
                                                    bool keep, uint8_t *buf) {
     typedef BufQ8<DT, RT> B;
     const int64_t e0 = g * 256 + 4 * lane;
@@ -969,12 +969,13 @@ __device__ __forceinline__ void quantize_direct_q8(const float4 (&xf)[8 * RT], c
         *(uint32_t *)(buf + B::oAct + (row >> 3) * 2048 + (lane >> 5) * 1024 + (row & 7) * 128 + ((((lane >> 2) & 7) ^ (row & 7)) << 4) + (lane & 3) * 4) = packed;
         if ((lane & 7) == 0) *(float *)(buf + B::oD8 + (row >> 3) * 256 + (lane >> 3) * 32 + (row & 7) * 4) = dr;
         if (keep && e0 < k) {
-            *(uint32_t *)(a.qs + row * k + e0) = packed;
+            const int64_t to = m0 + row;
+            *(uint32_t *)(a.qs + to * k + e0) = packed;
             if ((lane & 7) == 0) {
-                const int64_t blk = row * (k >> 5) + (e0 >> 5);
+                const int64_t blk = to * (k >> 5) + (e0 >> 5);
                 a.d[blk] = dr;
                 a.bsum32[blk] = (int16_t)sum;
-                a.dT[(e0 >> 5) * a.m_stride + row] = dr;
+                a.dT[(e0 >> 5) * a.m_stride + to] = dr;
             }
         }
     }
@@ -1021,7 +1022,7 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
     for (int64_t g = wave; g < kg; g += NW) {
         float4 xf[DIRECT ? 8 * RT : 1];
         if constexpr (DIRECT) {
-            load_direct_q8<RT>(x, m, k, g, lane, xf);
+            load_direct_q8<RT>(x + m0 * k, m - m0, k, g, lane, xf);
             __builtin_amdgcn_sched_barrier(0);
         }
         if (Q4) {
@@ -1047,7 +1048,7 @@ __device__ __forceinline__ void skinny_blk32_body(const cq_weight &w, const cq_a
         const u32x4_a4 dwv = *(const u32x4_a4 *)(w.p1 + ((n_tile + r) * kb + g * 8) * 2);
         if constexpr (DIRECT) {
             __builtin_amdgcn_sched_barrier(0);
-            quantize_direct_q8<DT, RT>(xf, a, m, k, g, lane, tile == 0, buf);
+            quantize_direct_q8<DT, RT>(xf, a, m0, m - m0, k, g, lane, tile == 0, buf);
         }
         __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
 
@@ -1130,13 +1131,14 @@ __global__ void __launch_bounds__(kThreads) skinny_shared_kernel(MultiArgs ma, c
 // One launch for the whole call: no quantizer launch in front, whose start and end are most of a small call (2.5 us of host time and
 // 2-3 us on the device).  A wave quantizes the rows' blocks that it contracts into its own buffer, so that no wave waits for
 // another; every workgroup repeats that, about 130 instructions for four rows of a block of 256, which is why it is for few weight rows
-// and few activation rows (cq_skinny_direct_takes).  Workgroup 0 leaves the quantized rows in the workspace too, where a quantizer
+// and few activation rows (cq_skinny_direct_takes).  The workgroups of tile 0 leave the quantized rows in the workspace too, where a quantizer
 // launch would have put them.
 template <int DT>
 __global__ void __launch_bounds__(kThreads) skinny_direct_kernel(cq_weight w, cq_act_view a, const float *__restrict__ x, int64_t m, float *__restrict__ y) {
     const cq_mfma_dump none{nullptr, nullptr, 0};
-    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, 1, false, true>(w, a, blockIdx.x, 0, m, y, none, x);
-    else skinny_body<DT, 1, false, true>(w, a, blockIdx.x, 0, m, y, none, x);
+    const int64_t m0 = blockIdx.y * 8, end = m0 + 8 < m ? m0 + 8 : m;   // (the result tile has sixteen rows)
+    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) skinny_blk32_body<DT, 1, false, true>(w, a, blockIdx.x, m0, end, y, none, x);
+    else skinny_body<DT, 1, false, true>(w, a, blockIdx.x, m0, end, y, none, x);
 }
 
 // ------------------------------------------- the same with everything of a workgroup in flight at once ----
@@ -1776,7 +1778,7 @@ hipError_t launch_any(const cq_weight *w, cq_act_view a, int act_dtype, int64_t 
 template <int DT> hipError_t launch_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s) {
     const size_t lds = (size_t)(DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0 ? (int)BufQ8<DT, 1>::kBytes : (int)Buf<DT, 1>::kBytes) * kWaves;
     if (hipError_t e = cq_ensure_lds<skinny_direct_kernel<DT>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_direct_kernel<DT>), (unsigned)((w->n + 15) / 16), kThreads, lds, s, *w, a, x, m, y);
+    CQ_LAUNCH((skinny_direct_kernel<DT>), dim3((unsigned)((w->n + 15) / 16), (unsigned)((m + 7) / 8)), kThreads, lds, s, *w, a, x, m, y);
     return hipGetLastError();
 }
 
@@ -1815,18 +1817,22 @@ hipError_t cq_launch_skinny_dump(const cq_weight *w, cq_act_view a, int act_dtyp
 }
 
 // The rows quantized by the contracting waves (where the dot-product kernel does not take them in one launch): where the quantizing that
-// every workgroup repeats costs less than the launch it saves.  Measured, us back to back / from a graph, against the two launches:
-//   Q4K 1024 x 1024, 5 rows 4.8 / 4.5 against 7.5 / 5.0; 8 rows 4.8 / 4.5 against 7.4 / 5.1; Q6K 4096 x 1024, 8 rows 5.0 / 4.7 against
-//   7.3 / 5.3; Q8_0 1024 x 1024, 5 rows 4.7 / 4.4 against 7.4 / 5.2, 8 rows 5.5 / 5.3 against 7.4 / 5.3
+// every workgroup repeats for its eight rows costs less than the launch it saves.  Measured, us back to back / from a graph, against the two
+// launches:
+//   Q4K 1024 x 1024, 5 rows 4.8 / 4.5 against 7.5 / 5.0; 8 rows 4.8 / 4.5 against 7.4 / 5.1; 326 x 768, 12 rows 4.7 / 4.7 against 8.6 / 5.7; Q6K
+//   4096 x 1024, 8 rows 5.0 / 4.7 against 7.3 / 5.3; Q8_0 1024 x 1024, 5 rows 4.7 / 4.4 against 7.4 / 5.2, 8 rows 5.5 / 5.3 against 7.4 / 5.3
 // and beyond the limits below behind from a graph or everywhere: two blocks a wave or two workgroups a CU double the quantizing
-// (Q4K 2048 x 2048, 8 rows 6.0 against 6.8 / 5.6; 8192 x 2048 10.6 against 7.3), nine rows take a second group (Q4K 1024 x 1024, 16 rows 6.9
-// against 7.0 / 5.6), Q4_0 with 8 rows 5.9 / 5.7 against 7.4 / 5.5.
+// (Q4K 2048 x 2048, 8 rows 6.0 against 6.8 / 5.6; 8192 x 2048 10.6 against 7.3), Q4_0 with 8 rows 5.9 / 5.7 against 7.4 / 5.5.
+// More than eight rows (K-quants): up to a workgroup a CU and a block a wave, on random shapes 1.25 to 1.7 times as fast back to back (1024 x 1024
+// with 32 rows 8.1 -> 5.2, Q6K 512 x 2048 with 64 11.9 -> 6.8, Q5K 256 x 1024 with 128 11.3 -> 5.6) and at least 1.03 times from a graph; Q8_0 and
+// Q4_0, whose rows a wave quantizes one by one, 1.05 to 1.4 but from a graph 0.8 to 0.95 (Q4_0 20 x 1536 with 28 rows 8.5 / 6.2 -> 7.2 / 7.5).
 bool cq_skinny_direct_takes(const cq_weight *w, int act_dtype, int64_t m) {
-    return m >= 2 && m <= (w->dtype == CQ_DTYPE_Q4_0 ? 7 : 8) && w->n <= 4096 && w->k <= (m <= 4 ? 2048 : 1024) &&
-           !cq_has_min32(w->ggml_dtype) && !cq_has_min16(w->ggml_dtype) && cq_skinny_takes(w, act_dtype);
+    if (m < 2 || cq_has_min32(w->ggml_dtype) || cq_has_min16(w->ggml_dtype) || !cq_skinny_takes(w, act_dtype)) return false;
+    const int64_t groups = (w->n + 15) / 16 * ((m + 7) / 8);
+    if (m > 8) return act_dtype == CQ_DTYPE_Q8K && groups <= cq_num_cus() && w->k <= 8 * QK_K;
+    return m <= (w->dtype == CQ_DTYPE_Q4_0 ? 7 : 8) && w->n <= 4096 && w->k <= (m <= 4 ? 2048 : 1024);
 }
 hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s) {
-    if (m > 8) return hipErrorInvalidValue;
     switch (w->dtype) {
     case CQ_DTYPE_Q8_0: return launch_direct<CQ_DTYPE_Q8_0>(w, a, x, m, y, s);
     case CQ_DTYPE_Q4_0: return launch_direct<CQ_DTYPE_Q4_0>(w, a, x, m, y, s);

@@ -1,4 +1,4 @@
-"""A few rows of a small weight: the launch whose waves quantize the rows they contract.  The same bits as the quantizer launch and the split-K
+"""Rows of a small weight: the launch whose waves quantize the rows they contract.  The same bits as the quantizer launch and the split-K
 launch after it, in y and in the workspace (read back through a call that reuses it), also for rows of zeros, infinities and NaN and for a block
 whose largest magnitude comes with both signs."""
 import pytest
@@ -15,7 +15,8 @@ def same_bits(a, b):
 
 
 @pytest.mark.parametrize("dt,n,k,m", [("Q4K", 16, 256, 5), ("Q4K", 4096, 1024, 8), ("Q4K", 1000, 768, 4), ("Q5K", 1031, 768, 7), ("Q6K", 33, 512, 5),
-                                      ("Q6K", 4090, 256, 4), ("Q3K", 512, 1024, 6), ("Q2K", 300, 512, 5), ("Q8_0", 16, 256, 5), ("Q8_0", 4096, 1024, 8),
+                                      ("Q6K", 4090, 256, 4), ("Q3K", 512, 1024, 6), ("Q2K", 300, 512, 5), ("Q4K", 2048, 2048, 16), ("Q5K", 300, 1792, 37), ("Q6K", 16, 1024, 255), ("Q3K", 65, 256, 9),
+                                      ("Q8_0", 16, 256, 5), ("Q8_0", 4096, 1024, 8),
                                       ("Q4_0", 1000, 320, 7), ("Q4_0", 4095, 960, 6), ("Q4_1", 500, 704, 5), ("Q5_1", 129, 1024, 7)])
 def test_same_bits_as_two_launches(qh, dt, n, k, m):  # noqa: F811
     g = torch.Generator(device="cuda").manual_seed(n + k + m)
