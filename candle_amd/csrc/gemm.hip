@@ -1347,6 +1347,19 @@ bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, co
     return cq_group_tiles(offsets, n_experts, 32) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
 }
 
+// us of a grouped tile launch with its quantizer: rounds of workgroups, workgroups per CU, bytes added up atomically (fitted to the calls of
+// plan_grouped in skinny.hip: 5 % rms).
+double cq_gemm_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets) {
+    const int t = w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2;
+    static constexpr double start[3] = {8.47, 8.74, 6.87}, unpack[3] = {0.69, 1.81, 1.62}, tile[3] = {0.64, 0.47, 0.52}, fill[3] = {0.72, 0.80, 0.97};
+    static constexpr double add[3] = {0.76, 0.86, 0.71};
+    const Plan p = pick_grouped(w, offsets, n_experts);
+    const double wgs = (double)((w->n + kWaves * 32 - 1) / (kWaves * 32)) * (double)cq_group_tiles(offsets, n_experts, 32 * p.mt) * p.ksplit;
+    const double per_cu = wgs / (double)cq_num_cus(), blocks = ceil((double)((w->k + 255) / 256) / p.ksplit);
+    const double added = p.ksplit > 1 ? (double)w->n * (double)offsets[n_experts] * 4e-6 * p.ksplit : 0.0;
+    return start[t] + blocks * (ceil(per_cu) * (unpack[t] + tile[t] * p.mt) + fill[t] * per_cu) + add[t] * added;
+}
+
 // us of the tile launch beside the quantizer and the stores, from the plan's cost (fitted to the calls of groups_us in skinny.hip: 5 % rms).
 double cq_gemm_us(const cq_weight *w, int64_t m) {
     const Plan p = pick_plan(w, m);

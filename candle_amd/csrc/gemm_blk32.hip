@@ -720,6 +720,16 @@ hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const 
 
 }  // namespace
 
+// us of a grouped tile launch, as cq_gemm_grouped_us in gemm.hip (5 % rms over the same calls).
+double cq_gemm32_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets) {
+    const int t = w->dtype == CQ_DTYPE_Q8_0 ? 0 : 1;
+    static constexpr double start[2] = {5.47, 5.55}, load[2] = {1.08, 0.82}, tile[2] = {1.15, 1.32}, fill[2] = {0.97, 0.25}, add[2] = {0.74, 0.78};
+    const Plan p = pick_grouped(w, offsets, n_experts);
+    const double wgs = (double)((w->n + kWaves * 32 - 1) / (kWaves * 32)) * (double)cq_group_tiles(offsets, n_experts, 32 * p.mt) * p.ksplit;
+    const double per_cu = wgs / (double)cq_num_cus(), blocks = ceil((double)((w->k + 255) / 256) / p.ksplit);
+    const double added = p.ksplit > 1 ? (double)w->n * (double)offsets[n_experts] * 4e-6 * p.ksplit : 0.0;
+    return start[t] + blocks * (ceil(per_cu) * (load[t] + tile[t] * p.mt) + fill[t] * per_cu) + add[t] * added;
+}
 bool cq_gemm32_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
     return n_experts <= kMaxGroupExperts && cq_gemm32_takes(experts[0], act_dtype) && cq_group_tiles(offsets, n_experts, 32) <= kMaxGroupTiles;
 }

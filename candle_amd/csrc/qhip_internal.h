@@ -199,6 +199,7 @@ bool cq_gemm_grouped_supported(const cq_weight *const *experts, int n_experts, c
 hipError_t cq_launch_gemm_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
                                   float *y, bool y_cleared, hipStream_t s);
 bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets);
+double cq_gemm_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets);
 // gemm_blk32.hip: the tile kernel for Q8_0 / Q4_0 weights with Q8_0 activations (K a multiple of 64)
 bool cq_gemm32_takes(const cq_weight *w, int act_dtype);
 bool cq_gemm32_supported(const cq_weight *w, int act_dtype);
@@ -209,6 +210,7 @@ bool cq_gemm32_grouped_takes(const cq_weight *const *experts, int n_experts, con
 hipError_t cq_launch_gemm32_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
                                     bool y_cleared, hipStream_t s);
 bool cq_gemm32_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets);
+double cq_gemm32_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets);
 // skinny.hip: a few activation rows (32 per pass) on the int8 MFMA, K split over the waves of a workgroup
 bool cq_skinny_takes(const cq_weight *w, int act_dtype);
 bool cq_skinny_supported(const cq_weight *w, int act_dtype);
@@ -227,6 +229,7 @@ bool cq_skinny_shared_takes(const cq_weight *const *ws, int count, int64_t m, in
 hipError_t cq_launch_skinny_shared(const cq_weight *const *ws, int count, cq_act_view a, int64_t m, float *const *ys, hipStream_t s);
 // all experts of a mixture-of-experts projection in one launch, for a few rows per expert
 bool cq_skinny_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype);
+double cq_skinny_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets);   // the estimates of the grouped launches
 hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
                                     hipStream_t s);
 // Table of a grouped launch, passed by value: tiles of up to `rows` expert-sorted activation rows, each of one expert.

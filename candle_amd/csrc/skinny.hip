@@ -1685,18 +1685,46 @@ hipError_t launch_grouped_rt(const cq_weight *const *experts, int n_experts, con
     CQ_LAUNCH((skinny_grouped_kernel<DT, RT>), dim3((unsigned)((experts[0]->n + 15) / 16), (unsigned)tiles), kThreads, lds, s, ga, a, y);
     return hipGetLastError();
 }
-// Rows per tile: what the fullest expert needs, in groups of eight, up to 32 (an expert with more takes several tiles).
-int grouped_rt(int n_experts, const int32_t *offsets) {
-    int64_t most = 0;
-    for (int e = 0; e < n_experts; e++) most = offsets[e + 1] - offsets[e] > most ? offsets[e + 1] - offsets[e] : most;
-    return most <= 8 ? 1 : most <= 16 ? 2 : most <= 24 ? 3 : 4;
+// Groups of eight rows a tile, and the us of the launch with its quantizer: weight bytes of the experts that have rows, blocks of all tiles per CU
+// and bytes stored.  Up to 16 rows for the fullest expert what holds them (Q8_0 beyond eight: by the estimate), beyond by the estimate among 16 and
+// 24 (Q8_0 8 and 16, Q4_0 16); 32 only where more tiles than a launch names would be needed.  Fitted to 8600 grouped calls (8 experts, 1024
+// to 4096 elements by 1.5 to 3.5 times as many, either way round, 2 to 512 routed rows), 5 to 8 % rms.
+struct GroupedPlan {
+    int rt;
+    double us;
+};
+GroupedPlan plan_grouped(const cq_weight *w, int n_experts, const int32_t *offsets) {
+    const int t = w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : w->dtype == CQ_DTYPE_Q8_0 ? 3 : w->dtype == CQ_DTYPE_Q4_0 ? 4 : 2;
+    static constexpr double bits[5] = {4.625, 5.625, 6.5625, 8.5, 4.5};
+    static constexpr double bytes_us[3][5] = {{0.044, 0.056, 0.049, 0.068, 0.061}, {0.054, 0.074, 0.062, 0.068, 0.055}, {0.070, 0.066, 0.059, 0, 0}};
+    static constexpr double block_us[3][5] = {{0.070, 0.108, 0.100, 0.085, 0.071}, {0.084, 0.101, 0.101, 0.108, 0.088}, {0.099, 0.129, 0.127, 0, 0}};
+    static constexpr double out_us[3][5] = {{2.5, 3.8, 3.0, 2.5, 3.5}, {1.6, 3.5, 2.8, 2.3, 1.8}, {2.4, 2.8, 2.1, 0, 0}};
+    int64_t most = 0, active = 0;
+    for (int e = 0; e < n_experts; e++) {
+        const int64_t rows = offsets[e + 1] - offsets[e];
+        most = rows > most ? rows : most;
+        active += rows > 0;
+    }
+    const int first = most <= 8 || t == 3 ? 1 : 2, last = most <= 8 ? 1 : most <= 16 || t >= 3 ? 2 : 3;
+    const double mb = (double)active * (double)w->n * (double)w->k * bits[t] / 8e6, out = (double)w->n * (double)offsets[n_experts] * 4e-6;
+    GroupedPlan best{4, 1e30};
+    for (int rt = first; rt <= last; rt++) {
+        const int64_t tiles = cq_group_tiles(offsets, n_experts, 8 * rt);
+        if (tiles > kMaxGroupTiles) continue;
+        const double blocks = (double)w->k / 256.0 * (double)((w->n + 15) / 16) * (double)tiles / (double)cq_num_cus();
+        const double us = 7.0 + bytes_us[rt - 1][t] * mb + block_us[rt - 1][t] * blocks + out_us[rt - 1][t] * out;
+        if (us < best.us) best = GroupedPlan{rt, us};
+    }
+    return best;
 }
 template <int DT>
 hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y, hipStream_t s) {
-    switch (grouped_rt(n_experts, offsets)) {
+    switch (plan_grouped(experts[0], n_experts, offsets).rt) {
     case 1: return launch_grouped_rt<DT, 1>(experts, n_experts, offsets, a, y, s);
     case 2: return launch_grouped_rt<DT, 2>(experts, n_experts, offsets, a, y, s);
-    case 3: return launch_grouped_rt<DT, 3>(experts, n_experts, offsets, a, y, s);
+    case 3:
+        if constexpr (DT != CQ_DTYPE_Q8_0 && DT != CQ_DTYPE_Q4_0) return launch_grouped_rt<DT, 3>(experts, n_experts, offsets, a, y, s);
+        return hipErrorInvalidValue;   // (never planned)
     default: return launch_grouped_rt<DT, 4>(experts, n_experts, offsets, a, y, s);
     }
 }
@@ -1844,8 +1872,9 @@ hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const floa
 
 bool cq_skinny_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
     if (n_experts > kMaxGroupExperts || !cq_skinny_takes(experts[0], act_dtype)) return false;
-    return cq_group_tiles(offsets, n_experts, 8 * grouped_rt(n_experts, offsets)) <= kMaxGroupTiles;
+    return cq_group_tiles(offsets, n_experts, 8 * plan_grouped(experts[0], n_experts, offsets).rt) <= kMaxGroupTiles;
 }
+double cq_skinny_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets) { return plan_grouped(w, n_experts, offsets).us; }
 
 hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
                                     hipStream_t s) {
