@@ -1097,14 +1097,6 @@ __global__ void __launch_bounds__(kThreads) gemm_q81_kernel(cq_weight w, cq_act_
     }
 }
 
-// Too few workgroups for `slots` of them at once: K is split (at least four blocks per part).
-int pick_ksplit(int64_t tiles, int64_t kb, int64_t slots) {
-    int ksplit = 1;
-    if (cq_no_split_k()) return 1;   // CQ_FLAG_DETERMINISTIC
-    while (tiles * ksplit * 2 <= slots && kb / (ksplit * 2) >= 4 && ksplit < 16) ksplit *= 2;
-    return ksplit;
-}
-
 int64_t n_tiles(const cq_weight *w) { return (w->n + kWaves * 32 - 1) / (kWaves * 32); }
 
 // Tile height (MT x 32 activation rows per workgroup) and K split of a launch, from a cost model fitted to
@@ -1252,27 +1244,9 @@ hipError_t launch_dump_dt(const cq_weight *w, cq_act_view a, int64_t m, cq_mfma_
     return launch_dump_mt<DT, 4>(w, a, m, p.ksplit, d, s);
 }
 
-// Tile height and K split of a grouped launch.  A single 32-row tile per expert splits K for two workgroups per CU; taller
-// tiles, by the cost model of pick_plan without a split, where they need fewer rounds of work: 8 experts 14336 x 4096,
-// 512 routed rows (at most 73 each), as 32-row tiles and as planned: Q4K 162 -> 139 us, Q6K 226 -> 174; 4096 x 14336 Q6K
-// 264 -> 185.
-Plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
-    const int64_t gx = n_tiles(w), kb = w->k >> 8, cus = cq_num_cus();
-    const double unpack = w->dtype == CQ_DTYPE_Q4K ? 22.0 : w->dtype == CQ_DTYPE_Q5K ? 32.0 : 50.0;
-    Plan best{1, 1};
-    double best_cost = 0.0;
-    for (int mt = 1; mt <= 4; mt <<= 1) {
-        const int64_t tiles = cq_group_tiles(offsets, n_experts, 32 * mt);
-        if (mt > 1 && tiles == cq_group_tiles(offsets, n_experts, 16 * mt)) break;   // half the height holds every expert's rows
-        const int64_t rounds = (gx * tiles + cus - 1) / cus;
-        const double cost = (double)rounds * ((double)kb * (unpack + 13.5 * mt) + 24.0);
-        if (mt == 1 || cost < best_cost) {
-            best = Plan{mt, mt == 1 ? pick_ksplit(gx * tiles, kb, 2 * cus) : 1};
-            best_cost = cost;
-            if (best.ksplit > 1) break;   // (few workgroups: not a case for fewer, taller ones)
-        }
-    }
-    return best;
+cq_grouped_plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
+    static constexpr cq_grouped_cost q4{5.5, 2.2, 0.65, 0.65, 0.68, 0.64}, q5{5.3, 3.4, 1.41, 0.67, 0.85, 0.56}, q6{5.7, 0.8, 1.54, 0.52, 1.02, 0.69};
+    return cq_plan_grouped_tiles(w, offsets, n_experts, w->dtype == CQ_DTYPE_Q4K ? q4 : w->dtype == CQ_DTYPE_Q5K ? q5 : q6);
 }
 
 template <int DT, int MT>
@@ -1295,7 +1269,7 @@ hipError_t launch_grouped_mt(const cq_weight *const *experts, int n_experts, con
 template <int DT>
 hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
                           float *y, bool y_cleared, hipStream_t s) {
-    const Plan p = pick_grouped(experts[0], offsets, n_experts);
+    const cq_grouped_plan p = pick_grouped(experts[0], offsets, n_experts);
     if (p.mt == 1) return launch_grouped_mt<DT, 1>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
     if (p.mt == 2) return launch_grouped_mt<DT, 2>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
     return launch_grouped_mt<DT, 4>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
@@ -1347,18 +1321,7 @@ bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, co
     return cq_group_tiles(offsets, n_experts, 32) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
 }
 
-// us of a grouped tile launch with its quantizer: rounds of workgroups, workgroups per CU, bytes added up atomically (fitted to the calls of
-// plan_grouped in skinny.hip: 5 % rms).
-double cq_gemm_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets) {
-    const int t = w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2;
-    static constexpr double start[3] = {8.47, 8.74, 6.87}, unpack[3] = {0.69, 1.81, 1.62}, tile[3] = {0.64, 0.47, 0.52}, fill[3] = {0.72, 0.80, 0.97};
-    static constexpr double add[3] = {0.76, 0.86, 0.71};
-    const Plan p = pick_grouped(w, offsets, n_experts);
-    const double wgs = (double)((w->n + kWaves * 32 - 1) / (kWaves * 32)) * (double)cq_group_tiles(offsets, n_experts, 32 * p.mt) * p.ksplit;
-    const double per_cu = wgs / (double)cq_num_cus(), blocks = ceil((double)((w->k + 255) / 256) / p.ksplit);
-    const double added = p.ksplit > 1 ? (double)w->n * (double)offsets[n_experts] * 4e-6 * p.ksplit : 0.0;
-    return start[t] + blocks * (ceil(per_cu) * (unpack[t] + tile[t] * p.mt) + fill[t] * per_cu) + add[t] * added;
-}
+double cq_gemm_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets) { return pick_grouped(w, offsets, n_experts).us; }
 
 // us of the tile launch beside the quantizer and the stores, from the plan's cost (fitted to the calls of groups_us in skinny.hip: 5 % rms).
 double cq_gemm_us(const cq_weight *w, int64_t m) {

@@ -671,25 +671,9 @@ hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, boo
     return launch_mt<DT, 4, DUMP>(w, a, m, y, p.ksplit, y_cleared, d, s);
 }
 
-// Tile height and K split of a grouped launch.  Too few 32-row tiles for two workgroups per CU: K is split (at least two
-// steps per part).  Otherwise the height with the least work by the cost model of pick_plan.
-Plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
-    const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), ks = (w->k + 255) >> 8, cus = cq_num_cus();
-    int64_t tiles = cq_group_tiles(offsets, n_experts, 32);
-    int split = 1;
-    while (!cq_no_split_k() && gx * tiles * split * 2 <= 2 * cus && ks / (split * 2) >= 2 && split < 16) split *= 2;
-    Plan best{1, split};
-    double best_cost = 0.0;
-    for (int mt = 1; mt <= 4 && split == 1; mt <<= 1) {
-        tiles = cq_group_tiles(offsets, n_experts, 32 * mt);
-        if (mt > 1 && tiles == cq_group_tiles(offsets, n_experts, 16 * mt)) break;   // half the height holds every expert's rows
-        const double cost = (double)((gx * tiles + cus - 1) / cus) * ((double)ks * (10.0 + 23.0 * mt) + 24.0);
-        if (mt == 1 || cost < best_cost) {
-            best = Plan{mt, 1};
-            best_cost = cost;
-        }
-    }
-    return best;
+cq_grouped_plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_experts) {
+    static constexpr cq_grouped_cost q8{5.8, 0.4, 1.15, 1.01, 0.97, 0.67}, q4{5.9, 0.85, 0.71, 1.16, 0.43, 0.69};
+    return cq_plan_grouped_tiles(w, offsets, n_experts, w->dtype == CQ_DTYPE_Q8_0 ? q8 : q4);
 }
 
 template <int DT, int MT, bool SHORT>
@@ -712,7 +696,7 @@ hipError_t launch_grouped_mt(const cq_weight *const *experts, int n_experts, con
 template <int DT, bool SHORT>
 hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a, float *y,
                           bool y_cleared, hipStream_t s) {
-    const Plan p = pick_grouped(experts[0], offsets, n_experts);
+    const cq_grouped_plan p = pick_grouped(experts[0], offsets, n_experts);
     if (p.mt == 1) return launch_grouped_mt<DT, 1, SHORT>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
     if (p.mt == 2) return launch_grouped_mt<DT, 2, SHORT>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
     return launch_grouped_mt<DT, 4, SHORT>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
@@ -720,16 +704,7 @@ hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const 
 
 }  // namespace
 
-// us of a grouped tile launch, as cq_gemm_grouped_us in gemm.hip (5 % rms over the same calls).
-double cq_gemm32_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets) {
-    const int t = w->dtype == CQ_DTYPE_Q8_0 ? 0 : 1;
-    static constexpr double start[2] = {5.47, 5.55}, load[2] = {1.08, 0.82}, tile[2] = {1.15, 1.32}, fill[2] = {0.97, 0.25}, add[2] = {0.74, 0.78};
-    const Plan p = pick_grouped(w, offsets, n_experts);
-    const double wgs = (double)((w->n + kWaves * 32 - 1) / (kWaves * 32)) * (double)cq_group_tiles(offsets, n_experts, 32 * p.mt) * p.ksplit;
-    const double per_cu = wgs / (double)cq_num_cus(), blocks = ceil((double)((w->k + 255) / 256) / p.ksplit);
-    const double added = p.ksplit > 1 ? (double)w->n * (double)offsets[n_experts] * 4e-6 * p.ksplit : 0.0;
-    return start[t] + blocks * (ceil(per_cu) * (load[t] + tile[t] * p.mt) + fill[t] * per_cu) + add[t] * added;
-}
+double cq_gemm32_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets) { return pick_grouped(w, offsets, n_experts).us; }
 bool cq_gemm32_grouped_takes(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype) {
     return n_experts <= kMaxGroupExperts && cq_gemm32_takes(experts[0], act_dtype) && cq_group_tiles(offsets, n_experts, 32) <= kMaxGroupTiles;
 }

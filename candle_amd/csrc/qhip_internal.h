@@ -259,6 +259,36 @@ static inline int cq_group_table(const cq_weight *const *experts, int n_experts,
     }
     return tiles;
 }
+// Tile height (32 * mt routed rows) and K split of a grouped tile launch of 256 weight rows a workgroup, and its us with the quantizer.  A round of
+// workgroups, one a CU, costs a fixed part and, for each 256 elements of its part of K, the weights and the row tiles; workgroups of a
+// last round that is not full get on faster (fill); parts of K are added up atomically (us per MB).  Constants of the types fitted to
+// 46000 forced plans (8 experts, 1024 to 14336 by 1024 to 14336, 16 to 800 routed rows), 5 to 7 % rms; the plan it picks takes 1.003 to 1.012
+// times as long as the best one on average.  (Two workgroups a CU by powers of two, as it was: 1.12 to 1.20.  us of whole calls from a graph:
+// 4096 x 14336 with 64 tokens Q4K 72 -> 67, Q5K 103 -> 94, Q6K 103 -> 98; Q8_0 5120 x 2048 with 117 tokens 39.6 -> 32.6.)
+struct cq_grouped_cost {
+    double start, round, load, tile, fill, add;
+};
+struct cq_grouped_plan {
+    int mt, ksplit;
+    double us;
+};
+static inline cq_grouped_plan cq_plan_grouped_tiles(const cq_weight *w, const int32_t *offsets, int n_experts, const cq_grouped_cost &c) {
+    const int64_t gx = (w->n + 255) / 256, kb = (w->k + 255) / 256, cus = cq_num_cus();
+    const double out = (double)w->n * (double)offsets[n_experts] * 4e-6;
+    cq_grouped_plan best{1, 1, 1e30};
+    for (int mt = 1; mt <= 4; mt <<= 1) {
+        const int64_t tiles = cq_group_tiles(offsets, n_experts, 32 * mt);
+        if (mt > 1 && tiles == cq_group_tiles(offsets, n_experts, 16 * mt)) break;   // half the height holds every expert's rows
+        const int most = cq_no_split_k() ? 1 : 16;
+        for (int ks = 1; ks <= most && (ks == 1 || (gx * tiles * ks <= 2 * cus && kb / ks >= 2)); ks++) {
+            const double rounds = (double)((gx * tiles * ks + cus - 1) / cus), blocks = (double)((kb + ks - 1) / ks);
+            const double us = c.start + rounds * c.round + blocks * (rounds * (c.load + c.tile * mt) + c.fill * (double)(gx * tiles * ks) / (double)cus) +
+                              (ks > 1 ? c.add * out * ks : 0.0);
+            if (us < best.us) best = cq_grouped_plan{mt, ks, us};
+        }
+    }
+    return best;
+}
 // moe.hip
 hipError_t cq_launch_silu_mul(const float *a, const float *b, float *h, int64_t count, hipStream_t s);
 hipError_t cq_launch_scatter_add(const float *y, const int32_t *row_ids, const float *weights, int64_t total_rows,

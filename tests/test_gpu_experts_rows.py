@@ -28,3 +28,18 @@ def test_rows_beyond_a_tile(qh, dt, n, k, rows):  # noqa: F811
     bad[off[-1] - 1, 3], bad[0, k - 1] = float("inf"), float("nan")
     same = [qh.qmatmul_grouped(ws, v, None, off, flags=qh.FLAG_DETERMINISTIC)[1:-1] for v in (bad, x)]
     assert torch.equal(*same)
+
+
+@pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K", "Q8_0", "Q4_0"])
+@pytest.mark.parametrize("n,k,rows", [(256, 2304, (33, 70, 65)), (300, 1536, (20, 31, 5)), (512, 8448, (1, 40)), (64, 512, (130, 0, 129)),
+                                      (2048, 1792, (40, 60, 90, 33))])
+def test_parts_of_k_and_tile_heights(qh, dt, n, k, rows):  # noqa: F811
+    """The tile kernels with parts of two blocks and more, equal or not, added up by one, two and four row tiles a workgroup."""
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    ws = [QTensor.quantize(torch.randn(n, k, generator=g, device="cuda") * 0.02, GgmlDType[dt]).weight for _ in rows]
+    off = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    x = torch.randn(int(off[-1]), k, generator=g, device="cuda")
+    want = torch.cat([qh.qmatmul(w, x[a:b].contiguous(), qh.FLAG_FORCE_MATVEC | qh.FLAG_STAGED_ACT) for w, a, b in zip(ws, off, off[1:]) if b > a])
+    blocks = k // (256 if dt.endswith("K") else 32)
+    close(qh.qmatmul_grouped(ws, x, None, off, flags=qh.FLAG_FORCE_GEMM), want, blocks)
+    close(qh.qmatmul_grouped(ws, x, None, off, flags=qh.FLAG_FORCE_GEMM | qh.FLAG_DETERMINISTIC), want, blocks)
