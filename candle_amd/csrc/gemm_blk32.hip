@@ -154,7 +154,8 @@ template <int DT> __device__ __forceinline__ void step_weights(const uint8_t *wl
 
 // One K step: the eight blocks of `bw` against the MT tiles of the stage `cur`.  `dcur`: the lane's weight row's eight f16 block
 // scales; nv: blocks of the step that exist (SHORT).
-template <int DT, int MT, bool DUMP, bool SHORT>
+// LOWER: at most sixteen rows of the last tile are live, and its upper sixteen (results 8..15) are not scaled.
+template <int DT, int MT, bool DUMP, bool SHORT, bool LOWER = false>
 __device__ __forceinline__ void step_mac(const uint8_t *cur, const LaneGeo &g, const v4i (&bw)[8], const u32x4_a4 dcur, int nv, int h, int col,
                                          v16f (&out)[MT], const cq_weight &w, int64_t m0, int64_t m, int64_t n, int64_t b, cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
@@ -216,7 +217,7 @@ __device__ __forceinline__ void step_mac(const uint8_t *cur, const LaneGeo &g, c
         if (q > 0) {
             const int p = (q - 1) & 1, t = (q - 1) >> 3;
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
+            for (int i = 0; i < (LOWER && t == MT - 1 ? 8 : 16); i++) {
                 if (DUMP) {   // (whole K steps only)
                     const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
                     if (row < m) dump.i[(row * w.n + n) * (w.k >> 5) + b * 8 + ((q - 1) & 7)] = DT == CQ_DTYPE_Q4_0 ? acc[p][i] >> 4 : acc[p][i];
@@ -309,7 +310,8 @@ __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_vi
 // the partial tiles meet in LDS, first half + second half: twice the workgroups at the same tile height, no atomic additions.
 // Bound, as above, by vector issue (one conversion and one fma per element and block, two thirds of the instructions).  Whole calls, us, before
 // -> here: Q4_0 32003 x 3200 at 77 rows (251 workgroups of 96 rows for 252 of 64, the upper ones nearly empty) 54.8 -> 42.1,
-// 29731 x 4864 at 90 rows 69.6 -> 51.9, Q8_0 4096 x 4096 at 512 rows 40.7 -> 36.1, 8192 x 2048 at 60 rows 16.1 -> 14.4.
+// 29731 x 4864 at 90 rows 69.6 -> 51.9; with the scaling of sixteen rows of padding left out (LOWER) 42.2 -> 40.5 at 77 rows, 29731 x 4864
+// 50.7 -> 48.7; Q8_0 4096 x 4096 at 512 rows 40.7 -> 36.1, 8192 x 2048 at 60 rows 16.1 -> 14.4.
 template <int DT, int MT> struct TileKH {
     typedef Tile<DT, MT> T;
     static constexpr int oWgt = 4 * T::kStage;   // two stages of one part per half
@@ -318,7 +320,7 @@ template <int DT, int MT> struct TileKH {
 };
 // Row tiles that gemm32_kh_kernel's stages leave room for beside the weights (Q8_0: 8 KiB a wave).
 template <int DT> constexpr int kh_tallest() { return DT == CQ_DTYPE_Q4_0 ? 3 : 2; }
-template <int DT, int MT, bool SHORT>
+template <int DT, int MT, bool SHORT, bool LOWER>
 __global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y) {
     typedef Tile<DT, MT> T;
     typedef TileKH<DT, MT> TK;
@@ -365,7 +367,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act
                 stage_weights<DT, false>(wl, w, g, n_tile, b + 1);
                 dnext = *(const u32x4_a4 *)(dplane + (b + 1) * 8);
             }
-            step_mac<DT, MT, false, SHORT>(cur, g, bw, dcur, (int)(k >> 5) - b * 8, h, col, out, w, m0, m, n, b, cq_mfma_dump{nullptr, nullptr, 0});
+            step_mac<DT, MT, false, SHORT, LOWER>(cur, g, bw, dcur, (int)(k >> 5) - b * 8, h, col, out, w, m0, m, n, b, cq_mfma_dump{nullptr, nullptr, 0});
         }
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
@@ -618,14 +620,18 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
 
 template <int DT, int MT> hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
     if (a.m_stride < (m + 32 * MT - 1) / (32 * MT) * (32 * MT)) return hipErrorInvalidValue;   // rows the last tile reads
-    auto go = [&](auto sh) {
-        constexpr bool SHORT = decltype(sh)::value;
+    auto go = [&](auto sh, auto low) {
+        constexpr bool SHORT = decltype(sh)::value, LOWER = decltype(low)::value;
         const size_t lds = TileKH<DT, MT>::kTotal;
-        if (hipError_t e = cq_ensure_lds<gemm32_kh_kernel<DT, MT, SHORT>>(w->dev, lds); e != hipSuccess) return e;
-        CQ_LAUNCH((gemm32_kh_kernel<DT, MT, SHORT>), dim3((unsigned)((w->n + 127) / 128), (unsigned)((m + MT * 32 - 1) / (MT * 32))), kThreads, lds, s, *w, a, m, y);
+        if (hipError_t e = cq_ensure_lds<gemm32_kh_kernel<DT, MT, SHORT, LOWER>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm32_kh_kernel<DT, MT, SHORT, LOWER>), dim3((unsigned)((w->n + 127) / 128), (unsigned)((m + MT * 32 - 1) / (MT * 32))), kThreads, lds, s, *w, a, m, y);
         return hipGetLastError();
     };
-    return w->k % 256 == 0 ? go(std::false_type{}) : go(std::true_type{});
+    // One row of workgroups whose upper sixteen rows are padding (with 64-row tiles no faster).  An instance of its own: as a branch in the step, or
+    // around two steps, the loop lost its unrolling or its registers (Q4_0 32003 x 3200 at 77 rows 42 -> 56 to 711 us).
+    if constexpr (MT == 3)
+        if (m <= 32 * MT - 16) return w->k % 256 == 0 ? go(std::false_type{}, std::true_type{}) : go(std::true_type{}, std::true_type{});
+    return w->k % 256 == 0 ? go(std::false_type{}, std::false_type{}) : go(std::true_type{}, std::false_type{});
 }
 template <int DT, int CW, bool ONCE> hipError_t launch_few(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
     auto go = [&](auto sh) {
