@@ -831,7 +831,7 @@ extern "C" size_t cq_grouped_workspace_bytes(const cq_weight *const *experts, in
     return act_ws_layout(act_dtype_for(experts[0], flags), total_rows, experts[0]->k, nullptr, nullptr, true);
 }
 
-// Most rows of one expert up to which the grouped split-K launch is taken.  Measured (8 experts, us of the whole call, split K /
+// Most rows of one expert up to which the grouped split-K launch is taken without a look at the estimates.  Measured (8 experts, us of the whole call, split K /
 // tiles; at 1, 2, 8, 11, 20 rows for the fullest one): Q4K 14336 x 4096 19/29, 47/66, 58/70, 72/70, 97/72, 2816 x 1024 10/14 ..
 // 10.6/14.3, 13.4/14.3; Q4_0 14336 x 4096 19/29, 50/79, 57/81, 69/81, 110/83; Q8_0 14336 x 4096 31/36, 90/101, 102/102, 111/103,
 // 194/105, 2816 x 1024 9/13 .. 12/14, 22/15.
@@ -874,7 +874,8 @@ static int grouped_impl(const cq_weight *const *experts, int n_experts, const fl
     act_ws_layout(act, total, w0->k, (uint8_t *)ws, &v, true);
     int64_t most = 0;
     for (int e = 0; e < n_experts; e++) most = offsets[e + 1] - offsets[e] > most ? offsets[e + 1] - offsets[e] : most;
-    // One launch for all experts: the split-K kernel for few rows per expert, the tile kernels beyond; where neither takes the weights (few weight rows, many experts), a launch per expert.
+    // One launch for all experts: the split-K kernel for few rows per expert and where it is ahead, the tile kernels otherwise; where neither takes
+    // the weights (few weight rows, many experts), a launch per expert.
     enum { kSkinny, kGemm32, kGemm, kEach } path = kEach;
     const bool force_gemm = (flags & CQ_FLAG_FORCE_GEMM) != 0, force_skinny = (flags & CQ_FLAG_FORCE_SKINNY) != 0;
     if (!(flags & CQ_FLAG_FORCE_MATVEC)) {
