@@ -339,9 +339,11 @@ __global__ void __launch_bounds__(256) min16_small_kernel(const uint8_t *__restr
 // Whether a tile for every wave would be fewer than one wave for each SIMD.
 static bool share_tile(const cq_weight *w, int64_t m) { return ((w->n + 63) / 64) * ((m + 31) / 32) < 4 * cq_num_cus(); }
 
-hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool apart, hipStream_t s) {
-    if (!cq_has_min32(w->ggml_dtype)) return hipErrorInvalidValue;
-    if (m == 0 || w->n == 0 || w->k == 0) return hipSuccess;
+// A workgroup names its rows by blockIdx.y, a grid has 65535 of those at most: more rows than the smallest groups make of them go in
+// several launches (a whole number of four rows each: the scales of the tiles are read four rows at a time).
+constexpr int64_t kMostRows = (int64_t)65535 * kSmallRows;
+
+static void launch_min32(const cq_weight *w, const cq_act_view &a, int64_t m, float *y, bool apart, hipStream_t s) {
     const int64_t nb = w->k / 32;
     const uint16_t *mins = (const uint16_t *)w->p2;
     if (apart)
@@ -350,12 +352,21 @@ hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, fl
     else if (share_tile(w, m))
         CQ_LAUNCH(min32_shared_kernel, dim3((unsigned)((w->n + 31) / 32), (unsigned)((m + 31) / 32)), 256, 0, s, mins, a, w->n, nb, m, y);
     else CQ_LAUNCH(min32_tiles_kernel, dim3((unsigned)((w->n + 255) / 256), (unsigned)((m + 31) / 32)), 256, 0, s, mins, a, w->n, nb, m, y);
-    return hipGetLastError();
+}
+hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool apart, hipStream_t s) {
+    if (!cq_has_min32(w->ggml_dtype)) return hipErrorInvalidValue;
+    if (m == 0 || w->n == 0 || w->k == 0) return hipSuccess;
+    for (int64_t r = 0; r < m; r += kMostRows) {
+        cq_act_view v = a;
+        v.d += r * (w->k / 32);
+        v.bsum32 += r * (w->k / 32);
+        launch_min32(w, v, m - r < kMostRows ? m - r : kMostRows, y + r * w->n, apart, s);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
-hipError_t cq_launch_min16_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool apart, hipStream_t s) {
-    if (!cq_has_min16(w->ggml_dtype)) return hipErrorInvalidValue;
-    if (m == 0 || w->n == 0 || w->k == 0) return hipSuccess;
+static void launch_min16(const cq_weight *w, const cq_act_view &a, int64_t m, float *y, bool apart, hipStream_t s) {
     const uint16_t *dmins = (const uint16_t *)w->p5;
     const int64_t kb = w->k / 256;
     if (m <= kSmallRows)
@@ -364,5 +375,18 @@ hipError_t cq_launch_min16_term(const cq_weight *w, cq_act_view a, int64_t m, fl
     else if (!apart && share_tile(w, m))
         CQ_LAUNCH(min16_mfma_kernel<true>, dim3((unsigned)((w->n + 31) / 32), (unsigned)((m + 31) / 32)), 256, 0, s, w->p4, dmins, a, w->n, kb, m, y);
     else CQ_LAUNCH(min16_mfma_kernel<false>, dim3((unsigned)((w->n + 255) / 256), (unsigned)((m + 31) / 32)), 256, 0, s, w->p4, dmins, a, w->n, kb, m, y);
-    return hipGetLastError();
+}
+hipError_t cq_launch_min16_term(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool apart, hipStream_t s) {
+    if (!cq_has_min16(w->ggml_dtype)) return hipErrorInvalidValue;
+    if (m == 0 || w->n == 0 || w->k == 0) return hipSuccess;
+    for (int64_t r = 0; r < m; r += kMostRows) {
+        cq_act_view v = a;   // (row-major planes by row, block-major ones by place)
+        v.d += r * (w->k / 256);
+        v.bsums += r * (w->k / 256) * 16;
+        v.dT += r;
+        v.bsh += r * 16;
+        launch_min16(w, v, m - r < kMostRows ? m - r : kMostRows, y + r * w->n, apart, s);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
