@@ -179,9 +179,59 @@ __global__ void __launch_bounds__(256) min32_tiles_kernel(const uint16_t *__rest
     add_tiles<false, CT>(acc, old, r0, c0, m, n, y);
 }
 
-// Few rows (decode, small batches): sixteen lanes per weight row, each a chunk of eight blocks out of 128 at a time; lane
-// 0 of the sixteen adds the chunk sums in order.  Sixteen weight rows and four activation rows per workgroup.
+// ---- rows that keep their bits whatever the row count ----
+// Two kernels with one order of the f32 additions: the blocks of a weight row in chunks of eight, a chunk's products added one after the
+// other from zero, the chunk sums added one after the other.  (apart32_small says which takes a call.)
 constexpr int kChunk = 8;
+
+// A workgroup forms a 32 x 32 tile of outputs, thread (i, j) the 2 x 2 outputs (i, i+16) x (j, j+16); the minima and the s values of 32
+// blocks at a time go through LDS.
+constexpr int kT = 32, kB = 32;
+__global__ void __launch_bounds__(256) min32_tile_kernel(const uint16_t *__restrict__ mins, cq_act_view a, int64_t n, int64_t nb,
+                                                         int64_t m, float *__restrict__ y) {
+    __shared__ float sm[kT][kB + 1], ss[kT][kB + 1];
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int64_t c0 = (int64_t)blockIdx.x * kT, r0 = (int64_t)blockIdx.y * kT;
+    float acc[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+    for (int64_t b0 = 0; b0 < nb; b0 += kB) {
+        for (int e = threadIdx.x; e < kT * kB; e += 256) {
+            const int row = e / kB, bb = e % kB;
+            const int64_t b = b0 + bb;
+            const bool ok = b < nb;
+            sm[row][bb] = ok && c0 + row < n ? cq_h2f(mins[(c0 + row) * nb + b]) : 0.0f;
+            ss[row][bb] = ok && r0 + row < m ? block_s(a, (r0 + row) * nb + b) : 0.0f;
+        }
+        __syncthreads();
+        for (int g = 0; g < kB && b0 + g < nb; g += kChunk) {
+            float t[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+#pragma unroll
+            for (int i = 0; i < kChunk; i++) {
+                if (b0 + g + i < nb) {   // blocks past the end of the row are left out, not added as zeros
+                    const float s0 = ss[ty][g + i], s1 = ss[ty + 16][g + i], m0 = sm[tx][g + i], m1 = sm[tx + 16][g + i];
+                    t[0][0] += m0 * s0;
+                    t[0][1] += m1 * s0;
+                    t[1][0] += m0 * s1;
+                    t[1][1] += m1 * s1;
+                }
+            }
+            acc[0][0] += t[0][0];
+            acc[0][1] += t[0][1];
+            acc[1][0] += t[1][0];
+            acc[1][1] += t[1][1];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int64_t r = r0 + ty + 16 * i, c = c0 + tx + 16 * j;
+            if (r < m && c < n) y[r * n + c] += acc[i][j];
+        }
+}
+
+// Few outputs: sixteen lanes per weight row, each a chunk of eight blocks out of 128 at a time; lane
+// 0 of the sixteen adds the chunk sums in order.  Sixteen weight rows and four activation rows per workgroup.
 constexpr int kSmallRows = 4;
 __global__ void __launch_bounds__(256) min32_small_kernel(const uint16_t *__restrict__ mins, cq_act_view a, int64_t n, int64_t nb,
                                                           int64_t m, float *__restrict__ y) {
@@ -334,8 +384,6 @@ __global__ void __launch_bounds__(256) min16_small_kernel(const uint8_t *__restr
 
 }  // namespace
 
-// `apart`: a row's bits may not depend on how many rows there are.  For that, one kernel takes all of them (Q2K: its unshared tiles add
-// the blocks in the small kernel's order, with the same roundings).
 // Whether a tile for every wave would be fewer than one wave for each SIMD.
 static bool share_tile(const cq_weight *w, int64_t m) { return ((w->n + 63) / 64) * ((m + 31) / 32) < 4 * cq_num_cus(); }
 
@@ -343,12 +391,23 @@ static bool share_tile(const cq_weight *w, int64_t m) { return ((w->n + 63) / 64
 // several launches (a whole number of four rows each: the scales of the tiles are read four rows at a time).
 constexpr int64_t kMostRows = (int64_t)65535 * kSmallRows;
 
+// `apart`: a row's bits may not depend on how many rows there are: the kernels with one order of the sums.  The one of sixteen lanes a weight
+// row up to four rows, and for rows of 80 blocks and more (fewer leave most of a chunk's lanes idle) up to 24000 outputs.  Whole calls, us,
+// 32 x 32 tiles / sixteen lanes: Q4_1 with 8 rows 4096 x 128 13.8 / 16.4, 4096 x 4096 28.5 / 30.0, 300 x 4096 26.7 / 23.0, with 16 rows 1000 x
+// 2560 32.0 / 30.3, 300 x 2048 28.2 / 28.4, with 64 rows 4096 x 4096 112 / 191, 300 x 4096 97.8 / 97.1, 8 x 4096 94.3 / 87.7.
+static bool apart32_small(const cq_weight *w, int64_t m) { return m <= kSmallRows || (w->k >= 80 * 32 && w->n * m <= 24000); }
+// Q2K: the tiles without sharing add the blocks in the small kernel's order, with the same roundings.  Up to 64 rows the small kernel, but for many
+// outputs of short rows.  Whole calls, us, tiles / small: 8 rows 8 x 4096 26.0 / 19.1, 5 rows 4096 x 1280 21.6 / 19.3, 64 rows 4096 x 4096
+// 129 / 127, 4096 x 1280 114.6 / 117.4, 4096 x 256 99.8 / 104.9.
+static bool apart16_small(const cq_weight *w, int64_t m) { return m <= 64 && (w->k > 8 * QK_K || w->n * m <= (1 << 17)); }
+
 static void launch_min32(const cq_weight *w, const cq_act_view &a, int64_t m, float *y, bool apart, hipStream_t s) {
     const int64_t nb = w->k / 32;
     const uint16_t *mins = (const uint16_t *)w->p2;
-    if (apart)
+    if (apart && apart32_small(w, m))
         CQ_LAUNCH(min32_small_kernel, dim3((unsigned)((w->n + 15) / 16), (unsigned)((m + kSmallRows - 1) / kSmallRows)), 256, 0, s, mins, a,
                   w->n, nb, m, y);
+    else if (apart) CQ_LAUNCH(min32_tile_kernel, dim3((unsigned)((w->n + kT - 1) / kT), (unsigned)((m + kT - 1) / kT)), 256, 0, s, mins, a, w->n, nb, m, y);
     else if (share_tile(w, m))
         CQ_LAUNCH(min32_shared_kernel, dim3((unsigned)((w->n + 31) / 32), (unsigned)((m + 31) / 32)), 256, 0, s, mins, a, w->n, nb, m, y);
     else CQ_LAUNCH(min32_tiles_kernel, dim3((unsigned)((w->n + 255) / 256), (unsigned)((m + 31) / 32)), 256, 0, s, mins, a, w->n, nb, m, y);
@@ -369,7 +428,7 @@ hipError_t cq_launch_min32_term(const cq_weight *w, cq_act_view a, int64_t m, fl
 static void launch_min16(const cq_weight *w, const cq_act_view &a, int64_t m, float *y, bool apart, hipStream_t s) {
     const uint16_t *dmins = (const uint16_t *)w->p5;
     const int64_t kb = w->k / 256;
-    if (m <= kSmallRows)
+    if (m <= kSmallRows || (apart && apart16_small(w, m)))
         CQ_LAUNCH(min16_small_kernel, dim3((unsigned)((w->n + 15) / 16), (unsigned)((m + kSmallRows - 1) / kSmallRows)), 256, 0, s, w->p4,
                   dmins, a, w->n, kb, m, y);
     else if (!apart && share_tile(w, m))
