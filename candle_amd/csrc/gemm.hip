@@ -266,6 +266,16 @@ struct DumpLane {
 struct MinW {
     v8h p1, p2;
 };
+// DUMP with int_min: the minima themselves as the operand, so that the MFMAs deliver the integer Mn_b.
+template <int DT> __device__ __forceinline__ void dump_operands(const WHead<DT> &head, int lane, const DumpLane &dl, MinW &wmin) {
+    if constexpr (is_k4(DT)) {
+        if (dl.int_min) {
+            const uint32_t rec[4] = {head.rec.x, head.rec.y, head.rec.z, head.rec.w};
+            wmin.p1 = __builtin_bit_cast(v8h, cq_min_term_groups_int(rec, (lane >> 5) != 0, false));
+            wmin.p2 = __builtin_bit_cast(v8h, cq_min_term_groups_int(rec, (lane >> 5) != 0, true));
+        }
+    }
+}
 // One block for this wave's 32 weight rows against the MT activation tiles in `cur`, as a
 // hand-laid software pipeline of 8*(MT+1) steps.  Step (t, s) issues the two int8 MFMAs of tile t,
 // K-slice s, and, in their shadow, the scaling of integers of tile t-1 (VALU); LDS reads run ahead.
@@ -562,13 +572,7 @@ __device__ __forceinline__ void block_step(const uint8_t *__restrict__ cur, uint
         WHead<DT> hcur = hreg;
         if (WBUF == 2) head_from_lds(wl + Tile<DT, MT>::oHdr, lane, hcur);
         block_unpack(wl, g, hcur, lane, bl, bh, dw, wmin);
-        if constexpr (DUMP && is_k4(DT)) {
-            if (dl.int_min) {   // verification: the minima themselves as the operand, so the MFMAs deliver the integer Mn_b
-                const uint32_t rec[4] = {hcur.rec.x, hcur.rec.y, hcur.rec.z, hcur.rec.w};
-                wmin.p1 = __builtin_bit_cast(v8h, cq_min_term_groups_int(rec, (lane >> 5) != 0, false));
-                wmin.p2 = __builtin_bit_cast(v8h, cq_min_term_groups_int(rec, (lane >> 5) != 0, true));
-            }
-        }
+        if constexpr (DUMP) dump_operands(hcur, lane, dl, wmin);
         if (WBUF == 2) {
             if (more) {
                 __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the reads above are done with the buffer
@@ -752,6 +756,10 @@ __global__ void __launch_bounds__(kThreads) gemm_dump_kernel(cq_weight w, cq_act
                                                              cq_mfma_dump dump) {
     gemm_body<DT, MT, true>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, nullptr, ksplit, dump);
 }
+template <int DT>
+__global__ void __launch_bounds__(kThreads) gemm_once_dump_kernel(cq_weight w, cq_act_view a, int64_t m, int ksplit, cq_mfma_dump dump) {
+    gemm_body<DT, 1, true, once_wbuf<DT>(), true>(w, a, blockIdx.x, 0, m, nullptr, ksplit, dump);
+}
 template <int DT, int TAIL>
 __global__ void __launch_bounds__(kThreads) gemm_tail_dump_kernel(cq_weight w, cq_act_view a, int64_t m, uint32_t gx, uint32_t whole,
                                                                   cq_mfma_dump dump) {
@@ -775,15 +783,14 @@ template <int DT, int MT> struct TileKH {
     static_assert(MT * 16 * 256 * (kWaves / 2) <= oWgt, "the partial tiles of the second half fit the stages");
 };
 
-template <int DT, int MT, bool TRAIL>
+template <int DT, int MT, bool TRAIL, bool DUMP>
 __device__ __forceinline__ void block_step_kh(const uint8_t *__restrict__ cur, uint8_t *__restrict__ nxt, uint8_t *__restrict__ wl,
                                               const cq_weight &w, const cq_act_view &a, const LaneGeo &g, int64_t m0, int64_t n_tile,
                                               bool work, int64_t next0, int64_t next1, int64_t mine_next, int wave, int lane,
-                                              const WHead<DT> &hcur, v16f (&out)[MT]) {
+                                              const WHead<DT> &hcur, v16f (&out)[MT], const DumpLane &dl) {
     typedef Tile<DT, MT> T;
     constexpr int SHIFT = DT == CQ_DTYPE_Q4K ? 3 : 8;
     constexpr int SPLIT = TRAIL ? MT / 2 : MT;   // tiles [SPLIT, MT) follow the barrier
-    const DumpLane dl{nullptr, nullptr, 0, 0, false};
     v4i bl[8], bh[8];
     float dw = 0.0f;
     MinW wmin = {};
@@ -791,17 +798,20 @@ __device__ __forceinline__ void block_step_kh(const uint8_t *__restrict__ cur, u
     if (next1 >= 0) stage_issue<DT, MT>(nxt + T::kBytes, w, a, g, m0, next1, wave, lane);
     if (work) {
         block_unpack(wl, g, hcur, lane, bl, bh, dw, wmin);
+        if constexpr (DUMP) dump_operands(hcur, lane, dl, wmin);
         if (mine_next >= 0) stage_weights<DT>(wl, w, g, n_tile, mine_next);
-        tiles_mac<DT, MT, 0, SPLIT, SHIFT, false, false>(cur, g, bl, bh, dw, wmin, lane, out, dl);
+        tiles_mac<DT, MT, 0, SPLIT, SHIFT, false, DUMP>(cur, g, bl, bh, dw, wmin, lane, out, dl);
     }
     __builtin_amdgcn_s_waitcnt(0);   // the next stage and the wave's next weights have landed in LDS
     __syncthreads();
-    if (TRAIL && work) tiles_mac<DT, MT, SPLIT, MT, SHIFT, false, false>(cur, g, bl, bh, dw, wmin, lane, out, dl);
+    if (TRAIL && work) tiles_mac<DT, MT, SPLIT, MT, SHIFT, false, DUMP>(cur, g, bl, bh, dw, wmin, lane, out, dl);
 }
 
 // Requires n >= 32.  One workgroup: activation rows [m0, m0 + 32*MT) x the 128 weight rows of blockIdx.x, all K.
-template <int DT, int MT>
-__global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y) {
+// (D: nothing, or cq_mfma_dump for the launch that stores the block integers: the production kernel keeps its arguments and registers)
+template <int DT, int MT, typename... D>
+__global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, D... dump) {
+    constexpr bool DUMP = sizeof...(D) > 0;
     typedef Tile<DT, MT> T;
     typedef TileKH<DT, MT> TK;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -846,14 +856,22 @@ __global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_v
         if (n_ok && mine_next >= 0) load_head(w, nc * kb + mine_next, hnxt);
         const uint8_t *cur = smem + ic * TK::kStage + half * T::kBytes;
         uint8_t *nxt = smem + in * TK::kStage;
-        if (half == 0) block_step_kh<DT, MT, false>(cur, nxt, wl, w, a, g, m0, n_tile, work, next0, next1, mine_next, wave, lane, hcur, out);
-        else block_step_kh<DT, MT, true>(cur, nxt, wl, w, a, g, m0, n_tile, work, next0, next1, mine_next, wave, lane, hcur, out);
+        DumpLane dl{nullptr, nullptr, 0, 0, false};
+        if constexpr (DUMP) {
+            const cq_mfma_dump d{dump...};
+            const int64_t at = (m0 * w.n + nc) * kb + first + it;
+            dl = DumpLane{d.i + at, d.mn ? d.mn + at : nullptr, w.n * kb, m - m0, d.int_min != 0};
+        }
+        if (half == 0) block_step_kh<DT, MT, false, DUMP>(cur, nxt, wl, w, a, g, m0, n_tile, work, next0, next1, mine_next, wave, lane, hcur, out, dl);
+        else block_step_kh<DT, MT, true, DUMP>(cur, nxt, wl, w, a, g, m0, n_tile, work, next0, next1, mine_next, wave, lane, hcur, out, dl);
         hcur = hnxt;
         const int t = ic;
         ic = in;
         in = ifree;
         ifree = t;
     }
+
+    if (DUMP) return;
 
     // ---- first half + second half through LDS (the stages are free: every wave is past its last read)
     __syncthreads();
@@ -1167,6 +1185,7 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
     return best;
 }
 
+template <int DT> constexpr size_t once_lds() { return once_wbuf<DT>() == 2 ? Tile<DT, 1>::kTotal2 : Tile<DT, 1>::kTotal; }
 template <int DT, int MT>
 hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int ksplit, bool y_cleared, hipStream_t s) {
     const size_t lds = Tile<DT, MT>::kTotal;
@@ -1179,7 +1198,7 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
     dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)ksplit);
     if constexpr (MT == 1) {
         if (gy == 1) {
-            const size_t lds1 = once_wbuf<DT>() == 2 ? Tile<DT, 1>::kTotal2 : Tile<DT, 1>::kTotal;
+            const size_t lds1 = once_lds<DT>();
             if (hipError_t e = cq_ensure_lds<gemm_once_kernel<DT>>(w->dev, lds1); e != hipSuccess) return e;
             CQ_LAUNCH((gemm_once_kernel<DT>), grid, kThreads, lds1, s, *w, a, m, y, ksplit);
             return hipGetLastError();
@@ -1189,16 +1208,21 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
     return hipGetLastError();
 }
 
-template <int DT, int MT>
-hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+// DUMP (here and below): the same launch storing the block integers through `d`.
+template <int DT, int MT, bool DUMP>
+hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = TileKH<DT, MT>::kTotal;
-    if (hipError_t e = cq_ensure_lds<gemm_kh_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
     dim3 grid((unsigned)((w->n + 127) / 128), (unsigned)((m + MT * 32 - 1) / (MT * 32)), 1);
-    CQ_LAUNCH((gemm_kh_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y);
+    if constexpr (DUMP) {
+        if (hipError_t e = cq_ensure_lds<gemm_kh_kernel<DT, MT, cq_mfma_dump>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm_kh_kernel<DT, MT, cq_mfma_dump>), grid, kThreads, lds, s, *w, a, m, y, d);
+    } else {
+        if (hipError_t e = cq_ensure_lds<gemm_kh_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm_kh_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y);
+    }
     return hipGetLastError();
 }
 
-// DUMP: the same launch storing the block integers through `d`.
 template <int DT, int TAIL, bool DUMP>
 hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = Tile<DT, 4>::kTotal;
@@ -1217,20 +1241,29 @@ hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, c
 template <int DT>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool y_cleared, hipStream_t s) {
     const Plan p = pick_plan(w, m);
-    if (p.tail == 2) return launch_tail<DT, 2, false>(w, a, m, y, cq_mfma_dump{nullptr, nullptr, 0}, s);
-    if (p.tail == 1) return launch_tail<DT, 1, false>(w, a, m, y, cq_mfma_dump{nullptr, nullptr, 0}, s);
-    if (p.kh == 2) return p.mt == 1 ? launch_kh<DT, 1>(w, a, m, y, s) : launch_kh<DT, 2>(w, a, m, y, s);
+    const cq_mfma_dump none{nullptr, nullptr, 0};
+    if (p.tail == 2) return launch_tail<DT, 2, false>(w, a, m, y, none, s);
+    if (p.tail == 1) return launch_tail<DT, 1, false>(w, a, m, y, none, s);
+    if (p.kh == 2) return p.mt == 1 ? launch_kh<DT, 1, false>(w, a, m, y, none, s) : launch_kh<DT, 2, false>(w, a, m, y, none, s);
     if (p.mt == 1) return launch_mt<DT, 1>(w, a, m, y, p.ksplit, y_cleared, s);
     if (p.mt == 2) return launch_mt<DT, 2>(w, a, m, y, p.ksplit, y_cleared, s);
     return launch_mt<DT, 4>(w, a, m, y, p.ksplit, y_cleared, s);
 }
 
-// The launch cq_launch_gemm would make (same tile heights, same K split), storing the block integers.
+// The launch cq_launch_gemm would make, storing the block integers.
 template <int DT, int MT>
 hipError_t launch_dump_mt(const cq_weight *w, cq_act_view a, int64_t m, int ksplit, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = Tile<DT, MT>::kTotal;
-    if (hipError_t e = cq_ensure_lds<gemm_dump_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
     dim3 grid((unsigned)n_tiles(w), (unsigned)((m + MT * 32 - 1) / (MT * 32)), (unsigned)ksplit);
+    if constexpr (MT == 1) {
+        if (grid.y == 1) {
+            const size_t lds1 = once_lds<DT>();
+            if (hipError_t e = cq_ensure_lds<gemm_once_dump_kernel<DT>>(w->dev, lds1); e != hipSuccess) return e;
+            CQ_LAUNCH((gemm_once_dump_kernel<DT>), grid, kThreads, lds1, s, *w, a, m, ksplit, d);
+            return hipGetLastError();
+        }
+    }
+    if (hipError_t e = cq_ensure_lds<gemm_dump_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
     CQ_LAUNCH((gemm_dump_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, ksplit, d);
     return hipGetLastError();
 }
@@ -1239,6 +1272,7 @@ hipError_t launch_dump_dt(const cq_weight *w, cq_act_view a, int64_t m, cq_mfma_
     const Plan p = pick_plan(w, m);
     if (p.tail == 2) return launch_tail<DT, 2, true>(w, a, m, nullptr, d, s);
     if (p.tail == 1) return launch_tail<DT, 1, true>(w, a, m, nullptr, d, s);
+    if (p.kh == 2) return p.mt == 1 ? launch_kh<DT, 1, true>(w, a, m, nullptr, d, s) : launch_kh<DT, 2, true>(w, a, m, nullptr, d, s);
     if (p.mt == 1) return launch_dump_mt<DT, 1>(w, a, m, p.ksplit, d, s);
     if (p.mt == 2) return launch_dump_mt<DT, 2>(w, a, m, p.ksplit, d, s);
     return launch_dump_mt<DT, 4>(w, a, m, p.ksplit, d, s);

@@ -320,8 +320,8 @@ template <int DT, int MT> struct TileKH {
 };
 // Row tiles that gemm32_kh_kernel's stages leave room for beside the weights (Q8_0: 8 KiB a wave).
 template <int DT> constexpr int kh_tallest() { return DT == CQ_DTYPE_Q4_0 ? 3 : 2; }
-template <int DT, int MT, bool SHORT, bool LOWER>
-__global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y) {
+template <int DT, int MT, bool DUMP, bool SHORT, bool LOWER>
+__global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
     typedef TileKH<DT, MT> TK;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -367,11 +367,12 @@ __global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act
                 stage_weights<DT, false>(wl, w, g, n_tile, b + 1);
                 dnext = *(const u32x4_a4 *)(dplane + (b + 1) * 8);
             }
-            step_mac<DT, MT, false, SHORT, LOWER>(cur, g, bw, dcur, (int)(k >> 5) - b * 8, h, col, out, w, m0, m, n, b, cq_mfma_dump{nullptr, nullptr, 0});
+            step_mac<DT, MT, DUMP, SHORT, LOWER>(cur, g, bw, dcur, (int)(k >> 5) - b * 8, h, col, out, w, m0, m, n, b, dump);
         }
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
     }
+    if (DUMP) return;
     // (the stages are free: every wave is past its last read)
     float *part = (float *)smem + (size_t)colw * (MT * 16 * 64);
     if (half == 1) {
@@ -405,8 +406,8 @@ template <int DT> struct Few {
     static constexpr int kWave = T::kStage + T::kWgtWave;
     static constexpr int kTotal = kWaves * kWave;
 };
-template <int DT, int CW, bool ONCE, bool SHORT>
-__global__ void __launch_bounds__(kThreads) gemm32_few_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y) {
+template <int DT, int CW, bool DUMP, bool ONCE, bool SHORT>
+__global__ void __launch_bounds__(kThreads) gemm32_few_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, cq_mfma_dump dump) {
     typedef Tile<DT, 1> T;
     constexpr int KS = kWaves / CW;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -450,7 +451,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_few_kernel(cq_weight w, cq_ac
                 dnext = *(const u32x4_a4 *)(dplane + (b + KS) * 8);
                 stage_weights<DT, ONCE>(wl, w, g, n_tile, b + KS);
             }
-            step_mac<DT, 1, false, SHORT>(cur, g, bw, dcur, (int)(k >> 5) - b * 8, h, col, out, w, 0, m, n, b, cq_mfma_dump{nullptr, nullptr, 0});
+            step_mac<DT, 1, DUMP, SHORT>(cur, g, bw, dcur, (int)(k >> 5) - b * 8, h, col, out, w, 0, m, n, b, dump);
 #pragma unroll
             for (int i = 0; i < 16; i++) asm volatile("" : "+v"(out[0][i]));   // (keeps the arithmetic in front of the branch: it would sink behind it, with all it holds)
             if (b + KS < ks) {
@@ -459,6 +460,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_few_kernel(cq_weight w, cq_ac
             }
         }
     }
+    if (DUMP) return;
     if constexpr (KS > 1) {
         float *mine = (float *)act;
 #pragma unroll
@@ -575,7 +577,8 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
     return best;
 }
 
-// DUMP: the same launch (tile height, K split) storing the block integers through `d`; y is not touched.
+// DUMP (here and below): the same launch (kernel, tile height, K split; copies never marked non-temporal) storing the block integers through
+// `d`; y is not touched.
 template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
 hipError_t launch_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, int ksplit, cq_mfma_dump d, hipStream_t s) {
     const size_t lds = Tile<DT, MT>::kTotal;
@@ -618,52 +621,60 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
     }
 }
 
-template <int DT, int MT> hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+template <int DT, int MT, bool DUMP> hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     if (a.m_stride < (m + 32 * MT - 1) / (32 * MT) * (32 * MT)) return hipErrorInvalidValue;   // rows the last tile reads
     auto go = [&](auto sh, auto low) {
         constexpr bool SHORT = decltype(sh)::value, LOWER = decltype(low)::value;
         const size_t lds = TileKH<DT, MT>::kTotal;
-        if (hipError_t e = cq_ensure_lds<gemm32_kh_kernel<DT, MT, SHORT, LOWER>>(w->dev, lds); e != hipSuccess) return e;
-        CQ_LAUNCH((gemm32_kh_kernel<DT, MT, SHORT, LOWER>), dim3((unsigned)((w->n + 127) / 128), (unsigned)((m + MT * 32 - 1) / (MT * 32))), kThreads, lds, s, *w, a, m, y);
+        if (hipError_t e = cq_ensure_lds<gemm32_kh_kernel<DT, MT, DUMP, SHORT, LOWER>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm32_kh_kernel<DT, MT, DUMP, SHORT, LOWER>), dim3((unsigned)((w->n + 127) / 128), (unsigned)((m + MT * 32 - 1) / (MT * 32))), kThreads, lds, s, *w,
+                  a, m, y, d);
         return hipGetLastError();
+    };
+    auto whole_or_short = [&](auto low) {
+        if constexpr (!DUMP)   // (whole K steps are all that is dumped)
+            if (w->k % 256 != 0) return go(std::true_type{}, low);
+        return go(std::false_type{}, low);
     };
     // One row of workgroups whose upper sixteen rows are padding (with 64-row tiles no faster).  An instance of its own: as a branch in the step, or
     // around two steps, the loop lost its unrolling or its registers (Q4_0 32003 x 3200 at 77 rows 42 -> 56 to 711 us).
     if constexpr (MT == 3)
-        if (m <= 32 * MT - 16) return w->k % 256 == 0 ? go(std::false_type{}, std::true_type{}) : go(std::true_type{}, std::true_type{});
-    return w->k % 256 == 0 ? go(std::false_type{}, std::false_type{}) : go(std::true_type{}, std::false_type{});
+        if (m <= 32 * MT - 16) return whole_or_short(std::true_type{});
+    return whole_or_short(std::false_type{});
 }
-template <int DT, int CW, bool ONCE> hipError_t launch_few(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
-    auto go = [&](auto sh) {
-        constexpr bool SHORT = decltype(sh)::value;
+template <int DT, int CW, bool DUMP> hipError_t launch_few(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
+    auto go = [&](auto on, auto sh) {
+        constexpr bool ONCE = decltype(on)::value, SHORT = decltype(sh)::value;
         const size_t lds = Few<DT>::kTotal;
-        if (hipError_t e = cq_ensure_lds<gemm32_few_kernel<DT, CW, ONCE, SHORT>>(w->dev, lds); e != hipSuccess) return e;
-        CQ_LAUNCH((gemm32_few_kernel<DT, CW, ONCE, SHORT>), (unsigned)((w->n + 32 * CW - 1) / (32 * CW)), kThreads, lds, s, *w, a, m, y);
+        if (hipError_t e = cq_ensure_lds<gemm32_few_kernel<DT, CW, DUMP, ONCE, SHORT>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm32_few_kernel<DT, CW, DUMP, ONCE, SHORT>), (unsigned)((w->n + 32 * CW - 1) / (32 * CW)), kThreads, lds, s, *w, a, m, y, d);
         return hipGetLastError();
     };
-    return w->k % 256 == 0 ? go(std::false_type{}) : go(std::true_type{});
+    if constexpr (!DUMP) {
+        const bool once = (DT == CQ_DTYPE_Q8_0 ? w->n * w->k : w->n * w->k / 2) >= kOnceBytes;
+        if (w->k % 256 != 0) return once ? go(std::true_type{}, std::true_type{}) : go(std::false_type{}, std::true_type{});
+        if (once) return go(std::true_type{}, std::false_type{});
+    }
+    return go(std::false_type{}, std::false_type{});
 }
 
-template <int DT> hipError_t launch_few_cw(const cq_weight *w, cq_act_view a, int64_t m, float *y, int cw, hipStream_t s) {
-    const bool once = (DT == CQ_DTYPE_Q8_0 ? w->n * w->k : w->n * w->k / 2) >= kOnceBytes;
+template <int DT, bool DUMP> hipError_t launch_few_cw(const cq_weight *w, cq_act_view a, int64_t m, float *y, int cw, cq_mfma_dump d, hipStream_t s) {
     switch (cw) {
-    case 1: return once ? launch_few<DT, 1, true>(w, a, m, y, s) : launch_few<DT, 1, false>(w, a, m, y, s);
-    case 2: return once ? launch_few<DT, 2, true>(w, a, m, y, s) : launch_few<DT, 2, false>(w, a, m, y, s);
-    case 4: return once ? launch_few<DT, 4, true>(w, a, m, y, s) : launch_few<DT, 4, false>(w, a, m, y, s);
-    default: return once ? launch_few<DT, 8, true>(w, a, m, y, s) : launch_few<DT, 8, false>(w, a, m, y, s);
+    case 1: return launch_few<DT, 1, DUMP>(w, a, m, y, d, s);
+    case 2: return launch_few<DT, 2, DUMP>(w, a, m, y, d, s);
+    case 4: return launch_few<DT, 4, DUMP>(w, a, m, y, d, s);
+    default: return launch_few<DT, 8, DUMP>(w, a, m, y, d, s);
     }
 }
 
 template <int DT, bool DUMP>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool y_cleared, cq_mfma_dump d, hipStream_t s) {
     const Plan p = pick_plan(w, m);
-    if constexpr (!DUMP) {
-        if (p.few) return launch_few_cw<DT>(w, a, m, y, p.few, s);
-        if (p.kh) {
-            if constexpr (kh_tallest<DT>() == 3)
-                if (p.mt == 3) return launch_kh<DT, 3>(w, a, m, y, s);
-            return p.mt == 2 ? launch_kh<DT, 2>(w, a, m, y, s) : launch_kh<DT, 1>(w, a, m, y, s);
-        }
+    if (p.few) return launch_few_cw<DT, DUMP>(w, a, m, y, p.few, d, s);
+    if (p.kh) {
+        if constexpr (kh_tallest<DT>() == 3)
+            if (p.mt == 3) return launch_kh<DT, 3, DUMP>(w, a, m, y, d, s);
+        return p.mt == 2 ? launch_kh<DT, 2, DUMP>(w, a, m, y, d, s) : launch_kh<DT, 1, DUMP>(w, a, m, y, d, s);
     }
     if (DUMP || w->k % 256 == 0) {   // (whole K steps are all that is dumped)
         if (p.tail == 2) return launch_tail<DT, 2, DUMP, false>(w, a, m, y, d, s);

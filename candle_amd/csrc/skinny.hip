@@ -1501,6 +1501,7 @@ bool launch_blk32_res(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq
 }
 
 // DUMP (all launchers below): the launch cq_launch_skinny would make, storing the block integers through `d`.
+
 // Sixteen waves to a workgroup instead of eight, for rows too long for the resident kernels: with a workgroup or less a CU, eight waves with a
 // block each in flight leave the memory idle.  Measured, whole calls in us, eight waves -> sixteen, 4 and 8 rows: 4096 x 14336 Q4K 15.2 -> 13.6
 // and 15.4 -> 14.6, Q4_0 16.0 -> 13.0 and 16.2 -> 13.8, Q6K 17.3 -> 16.2 and 17.5 -> 17.3; 2048 x 11008 Q4K 12.2 -> 10.7, Q4_0 13.2 -> 10.6.  Not
@@ -1521,7 +1522,7 @@ hipError_t launch_blk32_waves(const cq_weight *w, cq_act_view a, int64_t m0, int
 template <int DT, int RT, bool DUMP>
 hipError_t launch_blk32_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const bool sixteen = sixteen_waves<DT, RT>(w);
-    constexpr int kMany = RT == 1 && DT != CQ_DTYPE_Q8_0 && !DUMP ? 16 : kWaves;
+    constexpr int kMany = RT == 1 && DT != CQ_DTYPE_Q8_0 ? 16 : kWaves;
     if constexpr (kCanOffset<DT, DUMP>)
         if (has_offset(*w)) return sixteen ? launch_blk32_waves<DT, RT, DUMP, kMany, true>(w, a, m0, m, y, d, s) : launch_blk32_waves<DT, RT, DUMP, kWaves, true>(w, a, m0, m, y, d, s);
     return sixteen ? launch_blk32_waves<DT, RT, DUMP, kMany, false>(w, a, m0, m, y, d, s) : launch_blk32_waves<DT, RT, DUMP, kWaves, false>(w, a, m0, m, y, d, s);
@@ -1551,7 +1552,7 @@ hipError_t launch_waves(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m
 template <int DT, int RT, bool DUMP>
 hipError_t launch_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const bool sixteen = sixteen_waves<DT, RT>(w);
-    constexpr int kMany = RT == 1 && DT != CQ_DTYPE_Q8_0 && !DUMP ? 16 : kWaves;
+    constexpr int kMany = RT == 1 && DT != CQ_DTYPE_Q8_0 ? 16 : kWaves;
     if constexpr (kCanOffset<DT, DUMP>)
         if (has_offset(*w)) return sixteen ? launch_waves<DT, RT, DUMP, kMany, true>(w, a, m0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, true>(w, a, m0, m, y, d, s);
     return sixteen ? launch_waves<DT, RT, DUMP, kMany, false>(w, a, m0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, false>(w, a, m0, m, y, d, s);
@@ -1730,20 +1731,20 @@ hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const 
 }
 
 // All the rows in one launch, 8 * RT of them to a workgroup.
-template <int DT, int RT, bool OFF>
-hipError_t launch_groups_inst(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, hipStream_t s, unsigned groups) {
-    const cq_mfma_dump none{nullptr, nullptr, 0};
-    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) return launch_blk32_waves<DT, RT, false, kWaves, OFF>(w, a, m0, m, y, none, s, groups);
-    else return launch_waves<DT, RT, false, kWaves, OFF>(w, a, m0, m, y, none, s, groups);
+template <int DT, int RT, bool DUMP, bool OFF>
+hipError_t launch_groups_inst(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s, unsigned groups) {
+    if constexpr (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q4_0) return launch_blk32_waves<DT, RT, DUMP, kWaves, OFF>(w, a, m0, m, y, d, s, groups);
+    else return launch_waves<DT, RT, DUMP, kWaves, OFF>(w, a, m0, m, y, d, s, groups);
 }
-template <int DT, int RT>
-hipError_t launch_groups(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+template <int DT, int RT, bool DUMP>
+hipError_t launch_groups(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const int64_t most = (int64_t)8 * RT * 65535;
     for (int64_t m0 = 0; m0 < m; m0 += most) {
         const unsigned groups = (unsigned)(((m - m0 < most ? m - m0 : most) + 8 * RT - 1) / (8 * RT));
         hipError_t e = hipErrorInvalidValue;
-        if (!has_offset(*w)) e = launch_groups_inst<DT, RT, false>(w, a, m0, m, y, s, groups);
-        else if constexpr (kCanOffset<DT, false>) e = launch_groups_inst<DT, RT, true>(w, a, m0, m, y, s, groups);
+        if constexpr (kCanOffset<DT, DUMP>) e = has_offset(*w) ? launch_groups_inst<DT, RT, DUMP, true>(w, a, m0, m, y, d, s, groups)
+                                                               : launch_groups_inst<DT, RT, DUMP, false>(w, a, m0, m, y, d, s, groups);
+        else e = launch_groups_inst<DT, RT, DUMP, false>(w, a, m0, m, y, d, s, groups);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -1766,11 +1767,11 @@ GroupsUs groups_us(const cq_weight *w, int64_t m) {
     return {5.35 + steps * (a16[t] + b16[t] * f16), 5.15 + steps * (a32[t] * rounds + b32[t] * f32) + c32[t] * rounds};
 }
 
-template <int DT>
-hipError_t launch_in_groups(const cq_weight *w, cq_act_view a, int64_t m, float *y, hipStream_t s) {
+template <int DT, bool DUMP>
+hipError_t launch_in_groups(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const GroupsUs us = groups_us(w, m);
-    if (us.sixteen <= us.thirty_two || m <= 32) return launch_groups<DT, 2>(w, a, m, y, s);
-    if constexpr (DT != CQ_DTYPE_Q8_0 && DT != CQ_DTYPE_Q4_0) return launch_groups<DT, 4>(w, a, m, y, s);
+    if (us.sixteen <= us.thirty_two || m <= 32) return launch_groups<DT, 2, DUMP>(w, a, m, y, d, s);
+    if constexpr (DT != CQ_DTYPE_Q8_0 && DT != CQ_DTYPE_Q4_0) return launch_groups<DT, 4, DUMP>(w, a, m, y, d, s);
     return hipErrorInvalidValue;
 }
 
@@ -1780,15 +1781,13 @@ hipError_t launch_any(const cq_weight *w, cq_act_view a, int act_dtype, int64_t 
     if (m == 0) return hipSuccess;
     if (a.m_stride < (m + 31) / 32 * 32) return hipErrorInvalidValue;   // whole 8-row groups are copied
     hipError_t e = hipSuccess;
-    if constexpr (!DUMP) {
-        if (cq_skinny_in_groups(w, m)) {
-            switch (w->dtype) {
-            case CQ_DTYPE_Q8_0: return launch_in_groups<CQ_DTYPE_Q8_0>(w, a, m, y, s);
-            case CQ_DTYPE_Q4_0: return launch_in_groups<CQ_DTYPE_Q4_0>(w, a, m, y, s);
-            case CQ_DTYPE_Q4K: return launch_in_groups<CQ_DTYPE_Q4K>(w, a, m, y, s);
-            case CQ_DTYPE_Q5K: return launch_in_groups<CQ_DTYPE_Q5K>(w, a, m, y, s);
-            default: return launch_in_groups<CQ_DTYPE_Q6K>(w, a, m, y, s);
-            }
+    if (cq_skinny_in_groups(w, m)) {
+        switch (w->dtype) {
+        case CQ_DTYPE_Q8_0: return launch_in_groups<CQ_DTYPE_Q8_0, DUMP>(w, a, m, y, d, s);
+        case CQ_DTYPE_Q4_0: return launch_in_groups<CQ_DTYPE_Q4_0, DUMP>(w, a, m, y, d, s);
+        case CQ_DTYPE_Q4K: return launch_in_groups<CQ_DTYPE_Q4K, DUMP>(w, a, m, y, d, s);
+        case CQ_DTYPE_Q5K: return launch_in_groups<CQ_DTYPE_Q5K, DUMP>(w, a, m, y, d, s);
+        default: return launch_in_groups<CQ_DTYPE_Q6K, DUMP>(w, a, m, y, d, s);
         }
     }
     if (w->dtype == CQ_DTYPE_Q8_0 && launch_blk32_res<CQ_DTYPE_Q8_0, DUMP>(w, a, m, y, d, s, &e)) return e;

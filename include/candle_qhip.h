@@ -207,9 +207,12 @@ int cq_qmatmul_int_dots(const cq_weight *w, const float *x_dev, int64_t m, int32
                         void *stream);
 
 /* The same integers out of the matrix-core kernels (the verification above runs the dot-product kernels): `kernel`
- * picks the small-batch kernel (CQ_MFMA_SKINNY: the launch cq_qmatmul makes for few rows, whatever m is here) or
- * the tile kernel of the prefill path (CQ_MFMA_TILE, with the tile height and K split cq_qmatmul picks for m;
- * Q8_0 and Q4_0 weights: more than 16 rows, as in cq_qmatmul).
+ * picks the small-batch kernels (CQ_MFMA_SKINNY: the launch cq_qmatmul makes behind its quantizer launch where the
+ * split-K kernels take m rows, with its row groups, waves and resident activations, whatever m is here) or the tile
+ * kernels of the prefill path (CQ_MFMA_TILE: the kernel, tile height and K split cq_qmatmul picks for m; Q8_0 and Q4_0
+ * weights: more than 16 rows, as in cq_qmatmul; their weight copies are never marked non-temporal here).  The launch
+ * that quantizes a small weight's rows itself and the launches over several weights or experts have no dump: they run
+ * the same bodies.
  * out_i as above.  out_mn (Q4K, Q5K; else NULL) is a float: those kernels contract the min term on the f16 matrix
  * core and never hold the integer sum: -dmin * sum_j min_{j/2}*bsums_j over the sixteen sums of a block (exact in
  * f16) with -dmin*min in two f16 pieces, stored as that contraction delivers it for one block (small-batch kernels) or

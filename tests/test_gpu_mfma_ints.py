@@ -131,6 +131,50 @@ def test_tile_kernel_integers(qh, dt, m, k, n):
     check_dump(qh, dt, qh.MFMA_TILE, m, k, n, 13 * dt + m + k + n)
 
 
+@pytest.mark.parametrize("dt", KQ + B32)
+@pytest.mark.parametrize("m,k,n", [(64, 1024, 96), (300, 2304, 48), (128, 4096, 1024), (33, 256, 2064)])
+def test_skinny_kernel_integers_groups_of_rows(qh, dt, m, k, n):
+    """More than 32 rows: groups of 16 and (K-quants, the third) 32 rows side by side, the last one short."""
+    check_dump(qh, dt, qh.MFMA_SKINNY, m, k, n, 3 * dt + m + k + n)
+
+
+@pytest.mark.parametrize("dt", KQ + B32)
+@pytest.mark.parametrize("m,k,n", [(24, 2304, 2064), (32, 2304, 2064), (20, 512, 4112), (31, 512, 4112), (25, 1024, 3008),
+                                   (7, 2304, 96), (16, 2304, 96), (8, 512, 4112)])
+def test_skinny_kernel_integers_groups_of_eight(qh, dt, m, k, n):
+    """One to four groups of eight rows in a workgroup (17 rows and more: too many weight rows for groups beside each other), resident and not."""
+    check_dump(qh, dt, qh.MFMA_SKINNY, m, k, n, 5 * dt + m + k + n)
+
+
+@pytest.mark.parametrize("dt", KQ + [orc.Q4_0])
+@pytest.mark.parametrize("m,k,n", [(3, 8448, 48), (8, 14336, 528)])
+def test_skinny_kernel_integers_sixteen_waves(qh, dt, m, k, n):
+    """Rows too long for the resident kernels: sixteen waves, some with one block more than others."""
+    check_dump(qh, dt, qh.MFMA_SKINNY, m, k, n, 7 * dt + m + k + n)
+
+
+def test_skinny_kernel_integers_rounds_of_tiles_q5k(qh):
+    """Two groups of eight rows: 15 blocks a row are the most that leave the LDS room for the slots."""
+    check_dump(qh, orc.Q5K, qh.MFMA_SKINNY, 16, 3840, 16 * 300, 3)
+
+
+@pytest.mark.parametrize("dt", KQ)
+@pytest.mark.parametrize("m,k,n", [(64, 256, 33792), (65, 256, 43680), (128, 2048, 4096), (20, 512, 4096)])
+def test_tile_kernel_integers_other_plans(qh, dt, m, k, n):
+    """64-row and 128-row tiles over all of K, K halved inside the workgroup, one row tile."""
+    check_dump(qh, dt, qh.MFMA_TILE, m, k, n, 19 * dt + m + k + n)
+
+
+@pytest.mark.parametrize("dt", B32)
+@pytest.mark.parametrize("m,k,n", [(17, 4096, 4064), (32, 1024, 11968), (24, 512, 16416), (21, 1536, 32800),   # 1, 2, 4, 8 column tiles
+                                   (33, 512, 2080), (64, 1024, 4096), (129, 768, 160), (48, 1536, 16896),
+                                   (190, 512, 16256), (77, 512, 32000),   # (Q4_0: 96-row tiles, of the last one sixteen rows left out)
+                                   (33, 256, 33792), (65, 256, 43680)])   # (all of K in one wave: 64 and 128 rows)
+def test_tile_kernel_integers_split_inside(qh, dt, m, k, n):
+    """Q8_0 / Q4_0 launches that split K inside the workgroup: up to 32 rows a wave by itself, beyond that K halved between the waves."""
+    check_dump(qh, dt, qh.MFMA_TILE, m, k, n, 17 * dt + m + k + n)
+
+
 @pytest.mark.parametrize("x_scale", [1e-30, 1e-8, 1e-2, 1.0, 500.0, 1e6, 1e30])
 @pytest.mark.parametrize("kernel", ["skinny", "tile64", "tile"])
 def test_min_term_error_bound_across_magnitudes(qh, kernel, x_scale):

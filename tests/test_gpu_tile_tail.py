@@ -28,7 +28,7 @@ def test_rows_of_no_whole_step(qh, dt, m, n, k):  # noqa: F811
 
 
 @pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K", "Q8_0", "Q4_0"])
-@pytest.mark.parametrize("m,n,k", [(1100, 8192, 512), (1025, 8160, 256), (1000, 11264, 512)])
+@pytest.mark.parametrize("m,n,k", [(1100, 8192, 512), (1025, 8160, 256), (1000, 11264, 512), (512, 4096, 1024)])   # (the last: 64 rows, K halved)
 def test_integers_of_both_heights(qh, dt, m, n, k):  # noqa: F811
     """The same launches storing their block integers (the min term's as well): every one equals the dot-product kernels'."""
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
