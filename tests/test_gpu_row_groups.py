@@ -37,3 +37,12 @@ def run(qh, dt, m, n, k):  # noqa: F811
 @pytest.mark.parametrize("m,n,k", [(17, 16, 320), (20, 2050, 2112), (33, 100, 4160), (129, 31, 576), (40, 1500, 960)])
 def test_steps_of_no_whole_length(qh, dt, m, n, k):  # noqa: F811
     run(qh, dt, m, n, k)
+
+
+@pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K", "Q3K", "Q2K", "Q8_0", "Q4_0", "Q4_1", "Q5_1"])
+@pytest.mark.parametrize("m,n,k", [(17, 4090, 2304), (24, 2065, 2560), (25, 4096, 2304), (32, 3000, 2816), (20, 3001, 512), (32, 4000, 1024), (24, 4100, 2304),
+                                   (31, 4130, 768), (12, 1000, 2304), (16, 4100, 3840)])
+def test_all_rows_in_one_workgroup(qh, dt, m, n, k):  # noqa: F811
+    """Nine to 32 rows, from 17 on of too many weight rows for groups: two to four groups of eight, resident (up to 4096 weight rows), by rounds
+    of tiles and not."""
+    run(qh, dt, m, n, k)

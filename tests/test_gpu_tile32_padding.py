@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("m", [65, 77, 80, 81])
-@pytest.mark.parametrize("n,k", [(32000, 512), (31999, 576), (28001, 1280)])
+@pytest.mark.parametrize("n,k", [(32000, 512), (31999, 576), (28001, 1280), (24003, 1088)])   # (the last: steps of no whole length)
 def test_padding_rows(qh, m, n, k):  # noqa: F811
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     w = QTensor.quantize(torch.randn(n, k, generator=g, device="cuda") * 0.02, GgmlDType.Q4_0).weight
