@@ -641,7 +641,7 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
         path = few ? kSkinny : kGemm32;
     } else if (!(flags & (CQ_FLAG_FORCE_GEMM | CQ_FLAG_FORCE_MATVEC)) && (m >= skinny_from || (m >= 2 && !rows_fused)) &&
                cq_skinny_takes(w, act) && (skinny_rows || !has_tile_kernel)) {
-        // (shapes the tile kernels do not take: the split-K kernel, 32 rows per pass over the weights, stays
+        // (shapes the tile kernels do not take: the split-K kernel, groups of 16 or 32 rows beside each other, stays
         // ahead of the dot-product kernel, 8 rows per pass, at every row count)
         path = kSkinny;
     } else {

@@ -1,4 +1,4 @@
-// Skinny matmul on int8 MFMA for a few activation rows (32 per pass over the weights; cq_qmatmul sends it 2..16 rows,
+// Skinny matmul on int8 MFMA for a few activation rows (up to 32 to a workgroup; cq_qmatmul sends it 2..16 rows,
 // more where the weight has few rows): y[m, n] = x[m, k] . W[n, k]^T with K-quant
 // weights and Q8K activations (Q8_0 weights with Q8_0 activations: second kernel below) (k_quants.rs:1842-1883 with vec_dot :1171-1250 for Q4K, :1585-1641
 // for Q6K) - the small-batch decode and the per-expert shapes of a mixture-of-experts layer, where
@@ -1480,15 +1480,17 @@ bool launch_blk32_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y,
         return false;
     }
     if (kg > (sixteen ? 16 : 8) * kMaxBpw) return false;
+    if (RT > 2 && !sixteen) return false;   // (these go in groups of rows: cq_skinny_in_groups)
+    constexpr int kFew = RT > 2 ? 16 : 8;
     const size_t lds = ResQ8<DT, RT>::bytes(kg);
     if (lds > (size_t)kMaxLds) return false;
     if constexpr (kCanOffset<DT, DUMP>) {
         if (has_offset(*w)) {
-            *err = sixteen ? launch_blk32_res_inst<DT, RT, 16, DUMP, true>(w, a, m, y, lds, d, s) : launch_blk32_res_inst<DT, RT, 8, DUMP, true>(w, a, m, y, lds, d, s);
+            *err = sixteen ? launch_blk32_res_inst<DT, RT, 16, DUMP, true>(w, a, m, y, lds, d, s) : launch_blk32_res_inst<DT, RT, kFew, DUMP, true>(w, a, m, y, lds, d, s);
             return true;
         }
     }
-    *err = sixteen ? launch_blk32_res_inst<DT, RT, 16, DUMP>(w, a, m, y, lds, d, s) : launch_blk32_res_inst<DT, RT, 8, DUMP>(w, a, m, y, lds, d, s);
+    *err = sixteen ? launch_blk32_res_inst<DT, RT, 16, DUMP>(w, a, m, y, lds, d, s) : launch_blk32_res_inst<DT, RT, kFew, DUMP>(w, a, m, y, lds, d, s);
     return true;
 }
 template <int DT, bool DUMP>
@@ -1520,26 +1522,21 @@ hipError_t launch_blk32_waves(const cq_weight *w, cq_act_view a, int64_t m0, int
     return hipGetLastError();
 }
 template <int DT, int RT, bool DUMP>
-hipError_t launch_blk32_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
+hipError_t launch_blk32_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const bool sixteen = sixteen_waves<DT, RT>(w);
     constexpr int kMany = RT == 1 && DT != CQ_DTYPE_Q8_0 ? 16 : kWaves;
     if constexpr (kCanOffset<DT, DUMP>)
-        if (has_offset(*w)) return sixteen ? launch_blk32_waves<DT, RT, DUMP, kMany, true>(w, a, m0, m, y, d, s) : launch_blk32_waves<DT, RT, DUMP, kWaves, true>(w, a, m0, m, y, d, s);
-    return sixteen ? launch_blk32_waves<DT, RT, DUMP, kMany, false>(w, a, m0, m, y, d, s) : launch_blk32_waves<DT, RT, DUMP, kWaves, false>(w, a, m0, m, y, d, s);
+        if (has_offset(*w)) return sixteen ? launch_blk32_waves<DT, RT, DUMP, kMany, true>(w, a, 0, m, y, d, s) : launch_blk32_waves<DT, RT, DUMP, kWaves, true>(w, a, 0, m, y, d, s);
+    return sixteen ? launch_blk32_waves<DT, RT, DUMP, kMany, false>(w, a, 0, m, y, d, s) : launch_blk32_waves<DT, RT, DUMP, kWaves, false>(w, a, 0, m, y, d, s);
 }
 
+// (up to 32 rows: more go in groups)
 template <int DT, bool DUMP>
 hipError_t launch_blk32(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    for (int64_t m0 = 0; m0 < m; m0 += 32) {
-        const int64_t left = m - m0;
-        hipError_t e;
-        if (left <= 8) e = launch_blk32_rt<DT, 1, DUMP>(w, a, m0, m, y, d, s);
-        else if (left <= 16) e = launch_blk32_rt<DT, 2, DUMP>(w, a, m0, m, y, d, s);
-        else if (left <= 24) e = launch_blk32_rt<DT, 3, DUMP>(w, a, m0, m, y, d, s);
-        else e = launch_blk32_rt<DT, 4, DUMP>(w, a, m0, m, y, d, s);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    if (m <= 8) return launch_blk32_rt<DT, 1, DUMP>(w, a, m, y, d, s);
+    if (m <= 16) return launch_blk32_rt<DT, 2, DUMP>(w, a, m, y, d, s);
+    if (m <= 24) return launch_blk32_rt<DT, 3, DUMP>(w, a, m, y, d, s);
+    return launch_blk32_rt<DT, 4, DUMP>(w, a, m, y, d, s);
 }
 
 template <int DT, int RT, bool DUMP, int NW, bool OFF>
@@ -1550,26 +1547,21 @@ hipError_t launch_waves(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m
     return hipGetLastError();
 }
 template <int DT, int RT, bool DUMP>
-hipError_t launch_rt(const cq_weight *w, cq_act_view a, int64_t m0, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
+hipError_t launch_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
     const bool sixteen = sixteen_waves<DT, RT>(w);
     constexpr int kMany = RT == 1 && DT != CQ_DTYPE_Q8_0 ? 16 : kWaves;
     if constexpr (kCanOffset<DT, DUMP>)
-        if (has_offset(*w)) return sixteen ? launch_waves<DT, RT, DUMP, kMany, true>(w, a, m0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, true>(w, a, m0, m, y, d, s);
-    return sixteen ? launch_waves<DT, RT, DUMP, kMany, false>(w, a, m0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, false>(w, a, m0, m, y, d, s);
+        if (has_offset(*w)) return sixteen ? launch_waves<DT, RT, DUMP, kMany, true>(w, a, 0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, true>(w, a, 0, m, y, d, s);
+    return sixteen ? launch_waves<DT, RT, DUMP, kMany, false>(w, a, 0, m, y, d, s) : launch_waves<DT, RT, DUMP, kWaves, false>(w, a, 0, m, y, d, s);
 }
 
+// (up to 32 rows: more go in groups)
 template <int DT, bool DUMP>
 hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mfma_dump d, hipStream_t s) {
-    for (int64_t m0 = 0; m0 < m; m0 += 32) {
-        const int64_t left = m - m0;
-        hipError_t e;
-        if (left <= 8) e = launch_rt<DT, 1, DUMP>(w, a, m0, m, y, d, s);
-        else if (left <= 16) e = launch_rt<DT, 2, DUMP>(w, a, m0, m, y, d, s);
-        else if (left <= 24) e = launch_rt<DT, 3, DUMP>(w, a, m0, m, y, d, s);
-        else e = launch_rt<DT, 4, DUMP>(w, a, m0, m, y, d, s);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    if (m <= 8) return launch_rt<DT, 1, DUMP>(w, a, m, y, d, s);
+    if (m <= 16) return launch_rt<DT, 2, DUMP>(w, a, m, y, d, s);
+    if (m <= 24) return launch_rt<DT, 3, DUMP>(w, a, m, y, d, s);
+    return launch_rt<DT, 4, DUMP>(w, a, m, y, d, s);
 }
 
 
