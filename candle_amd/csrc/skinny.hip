@@ -448,18 +448,18 @@ __global__ void __launch_bounds__(NW * 64) skinny_kernel(cq_weight w, cq_act_vie
 // bytes (from L2) than the weights themselves (16 K against 9 K per workgroup for Q4K), and the launch is bound
 // by it.  When the quantized activations of the call fit the LDS beside the weight buffers (4096 columns x 16
 // rows: 75 KiB) a launch of at most one workgroup per CU copies them once, each wave the K blocks it owns (sixteen
-// waves: one block each for 4096 columns, a single memory round trip), and then walks its share of the 16-row
-// weight tiles (tile t of workgroup g: g + t * G) streaming weights only.  The launcher takes it where every
-// workgroup has one tile (n <= 16 x the number of CUs); with more tiles per workgroup it measured no faster than
-// the kernel above, also with the next tile's weights copied ahead into a second buffer (NBUF == 2).
+// waves: one block each for 4096 columns, a single memory round trip).  The launcher takes it where every
+// workgroup has one 16-row weight tile (n <= 16 x the number of CUs); walking several tiles measured no faster than
+// the kernel above, also with the next tile's weights copied ahead into a second buffer.  The loop over tiles cost registers that sixteen
+// waves do not have, and spills with 17 rows and more (whole calls, us, with it -> without, 4096 x 4096: 24 rows Q4K 9.3 -> 7.8, Q5K 11.9 ->
+// 8.6, Q2K 10.7 -> 8.9; 8 rows Q4K 7.0 -> 6.8, Q2K 8.7 -> 8.1; Q6K level).
 //   per K block b  : act [RT][2 K-halves][8 rows][8 chunks] | d8 [8*RT] f32 | bsh [8*RT][16] f16 (k4 types)
-//   per wave, block: weights of one tile (kWgt bytes), twice when NBUF == 2; a wave's first buffer of a tile also
-//                    carries its partial results of that tile (1 KiB per 16 activation rows)
+//   per K block    : weights (kWgt bytes); a wave's first buffer also carries its partial results (1 KiB per 16 activation rows)
 template <int DT, int RT> struct Res {
     static constexpr int kWgt = Buf<DT, RT>::kWgt;
     static constexpr int kActBlk = RT * 2048 + RT * 32 + (is_k4(DT) ? RT * 256 : 0);
     static constexpr int oD8 = RT * 2048, oMin = oD8 + RT * 32;
-    static size_t bytes(int64_t kb, int nbuf) { return (size_t)kb * kActBlk + (size_t)kb * nbuf * kWgt; }
+    static size_t bytes(int64_t kb) { return (size_t)kb * (kActBlk + kWgt); }
 };
 
 // Copies with one descriptor per plane, built once, and the position inside the plane as a 32-bit scalar offset
@@ -561,10 +561,10 @@ __device__ __forceinline__ void res_block(const uint8_t *__restrict__ wl, const 
     res_mac<DT, RT, NT, DUMP>(act, lane, o, a_col, out, dump, at, rs, m);
 }
 
-// m <= 8 * RT activation rows (the workspace pads rows, so whole groups are copied); n >= 16; at most
-// kMaxBpw K blocks per wave.  `tiles` of 16 rows, dealt to the gridDim.x workgroups in turn.
+// m <= 8 * RT activation rows (the workspace pads rows, so whole groups are copied); n >= 16, one 16-row tile per workgroup; at most
+// kMaxBpw K blocks per wave.
 constexpr int kMaxBpw = 4;
-template <int DT, int RT, int kWaves, int NBUF, bool DUMP, bool OFF = false>
+template <int DT, int RT, int kWaves, bool DUMP, bool OFF = false>
 __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight w, cq_act_view a, int64_t m,
                                                                       float *__restrict__ y, cq_mfma_dump dump) {
     typedef Res<DT, RT> R;
@@ -575,7 +575,7 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t r = lane & 15, kq = lane >> 4;
     const int64_t k = w.k, kb = w.k >> 8;
-    const int64_t tiles = (w.n + 15) / 16;
+    const int64_t n_tile = tile_row(blockIdx.x, w.n);
     uint8_t *wgt_base = smem + kb * R::kActBlk;
 
     const uint32_t r8 = lane >> 3, c8 = lane & 7;
@@ -600,14 +600,13 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
     pl.ad = wave_rsrc(a.dT);
     pl.am = wave_rsrc(a.bsh);
     const uint32_t kb32 = (uint32_t)kb, k32 = (uint32_t)k, mstr = (uint32_t)a.m_stride;
-    // ---- the wave's K blocks: the small fields of the first tile's weights (registers; requested first, they are
-    // what the unpacking starts with), activation slices once, weights of the first tile
-    int64_t tile = blockIdx.x;
+    // ---- the wave's K blocks: the small fields of the weights (registers; requested first, they are what the unpacking
+    // starts with), activation slices, weights
     WHead<DT> head[kMaxBpw];
 #pragma unroll
     for (int j = 0; j < kMaxBpw; j++) {
         const int64_t b = wave + (int64_t)j * kWaves;
-        if (b < kb && tile < tiles) load_head(w, (tile_row(tile, w.n) + r) * kb + b, head[j]);
+        if (b < kb) load_head(w, (n_tile + r) * kb + b, head[j]);
     }
 #pragma unroll
     for (int j = 0; j < kMaxBpw; j++) {
@@ -621,76 +620,48 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
             }
             if (lane < 8 * RT) dma4s(pl.ad, lane * 4u, b * mstr * 4u, act + R::oD8);
             if (MINS && lane < 16 * RT) dma16s(pl.am, lane * 16u, b * mstr * 32u, act + R::oMin);
-            if (tile < tiles)
-                res_issue_weights<DT>(wgt_base + (b * NBUF) * R::kWgt, pl, (uint32_t)tile_row(tile, w.n), b, kb32, wq_off, wh_off, w5_off, lane);
+            res_issue_weights<DT>(wgt_base + b * R::kWgt, pl, (uint32_t)n_tile, b, kb32, wq_off, wh_off, w5_off, lane);
         }
     }
-    int par = 0;
-    for (; tile < tiles; tile += gridDim.x) {
-        const int64_t n_tile = tile_row(tile, w.n), next = tile + gridDim.x;
-        __builtin_amdgcn_s_waitcnt(0);   // this tile's weights (and, the first time, the activations) have landed
-        if (NBUF == 2 && next < tiles) {
+    __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
+    if constexpr (DT == CQ_DTYPE_Q6K) {
+        // (the block scale is converted from here on: the conversion moved up to its load, which then was waited for before any copy went out)
 #pragma unroll
-            for (int j = 0; j < kMaxBpw; j++) {
-                const int64_t b = wave + (int64_t)j * kWaves;
-                if (b < kb)
-                    res_issue_weights<DT>(wgt_base + (b * NBUF + (par ^ 1)) * R::kWgt, pl, (uint32_t)tile_row(next, w.n), (uint32_t)b, kb32,
-                                          wq_off, wh_off, w5_off, lane);
-            }
-        }
-        v4f out[NT];
+        for (int j = 0; j < kMaxBpw; j++) asm volatile("" : "+v"(head[j].d));
+    }
+    v4f out[NT];
 #pragma unroll
-        for (int t = 0; t < NT; t++) out[t] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    for (int t = 0; t < NT; t++) out[t] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 0; j < kMaxBpw; j++) {
-            const int64_t b = wave + (int64_t)j * kWaves;
-            if (b < kb)
-                res_block<DT, RT, NT, DUMP>(wgt_base + (b * NBUF + (NBUF == 2 ? par : 0)) * R::kWgt, smem + b * R::kActBlk, lane,
-                                            head[j], a_col, out, dump, (n_tile + r) * kb + b, w.n * kb, m);
-        }
-        if constexpr (OFF) {
-            if (wave < kb) add_min16<NT>(w, a, n_tile, 0, wave, kb < kWaves ? kb : kWaves, lane, out);
-        }
-        // ---- sum the waves' partial tiles in wave order (through the wave's first weight buffer of this tile)
-        uint8_t *part = wgt_base + ((int64_t)wave * NBUF + (NBUF == 2 ? par : 0)) * R::kWgt;
-        if (wave < kb) {   // (a wave without a K block has no buffer and nothing to add)
+    for (int j = 0; j < kMaxBpw; j++) {
+        const int64_t b = wave + (int64_t)j * kWaves;
+        if (b < kb)
+            res_block<DT, RT, NT, DUMP>(wgt_base + b * R::kWgt, smem + b * R::kActBlk, lane, head[j], a_col, out, dump, (n_tile + r) * kb + b, w.n * kb, m);
+    }
+    if (DUMP) return;
+    if constexpr (OFF) {
+        if (wave < kb) add_min16<NT>(w, a, n_tile, 0, wave, kb < kWaves ? kb : kWaves, lane, out);
+    }
+    // ---- sum the waves' partial tiles in wave order (through each wave's first weight buffer)
+    if (wave < kb) {   // (a wave without a K block has no buffer and nothing to add)
+        uint8_t *part = wgt_base + (int64_t)wave * R::kWgt;
 #pragma unroll
-            for (int t = 0; t < NT; t++) *(v4f *)(part + t * 1024 + lane * 16) = out[t];
+        for (int t = 0; t < NT; t++) *(v4f *)(part + t * 1024 + lane * 16) = out[t];
+    }
+    __syncthreads();
+    if (wave < NT) {
+        v4f s = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+        const int64_t nw = kb < kWaves ? kb : kWaves;   // waves that own a block
+        for (int64_t o = 0; o < nw; o++) {
+            const v4f p = *(const v4f *)(wgt_base + o * R::kWgt + wave * 1024 + lane * 16);
+            s += p;
         }
-        __syncthreads();
-        if (wave < NT && !DUMP) {
-            v4f s = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-            const int64_t nw = kb < kWaves ? kb : kWaves;   // waves that own a block
-            for (int64_t o = 0; o < nw; o++) {
-                const v4f p = *(const v4f *)(wgt_base + (o * NBUF + (NBUF == 2 ? par : 0)) * R::kWgt + wave * 1024 + lane * 16);
-                s += p;
-            }
-            const int64_t col = n_tile + r;
+        const int64_t col = n_tile + r;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int64_t row = wave * 16 + kq * 4 + i;
-                if (row < m) y[row * w.n + col] = s[i];
-            }
+        for (int i = 0; i < 4; i++) {
+            const int64_t row = wave * 16 + kq * 4 + i;
+            if (row < m) y[row * w.n + col] = s[i];
         }
-        if (NBUF == 1 && next < tiles) {
-            __syncthreads();   // the partial results have been read: the buffers take the next tile's weights
-#pragma unroll
-            for (int j = 0; j < kMaxBpw; j++) {
-                const int64_t b = wave + (int64_t)j * kWaves;
-                if (b < kb)
-                    res_issue_weights<DT>(wgt_base + b * R::kWgt, pl, (uint32_t)tile_row(next, w.n), (uint32_t)b, kb32, wq_off, wh_off, w5_off, lane);
-            }
-        } else if (NBUF == 2) {
-            __syncthreads();   // ... before the tile after the next one is copied over them
-        }
-        if (next < tiles) {
-#pragma unroll
-            for (int j = 0; j < kMaxBpw; j++) {
-                const int64_t b = wave + (int64_t)j * kWaves;
-                if (b < kb) load_head(w, (tile_row(next, w.n) + r) * kb + b, head[j]);
-            }
-        }
-        par ^= 1;
     }
 }
 
@@ -1566,11 +1537,10 @@ hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_
 
 
 // The resident-activation kernel where the call's activations and the weight buffers fit the LDS (see above).
-template <int DT, int RT, int NW, int NBUF, bool DUMP, bool OFF = false>
-hipError_t launch_res_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, size_t lds, unsigned grid, cq_mfma_dump d,
-                           hipStream_t s) {
-    if (hipError_t e = cq_ensure_lds<skinny_resident_kernel<DT, RT, NW, NBUF, DUMP, OFF>>(w->dev, lds); e != hipSuccess) return e;
-    CQ_LAUNCH((skinny_resident_kernel<DT, RT, NW, NBUF, DUMP, OFF>), grid, NW * 64, lds, s, *w, a, m, y, d);
+template <int DT, int RT, int NW, bool DUMP, bool OFF = false>
+hipError_t launch_res_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, size_t lds, cq_mfma_dump d, hipStream_t s) {
+    if (hipError_t e = cq_ensure_lds<skinny_resident_kernel<DT, RT, NW, DUMP, OFF>>(w->dev, lds); e != hipSuccess) return e;
+    CQ_LAUNCH((skinny_resident_kernel<DT, RT, NW, DUMP, OFF>), (unsigned)((w->n + 15) / 16), NW * 64, lds, s, *w, a, m, y, d);
     return hipGetLastError();
 }
 template <int DT, int RT, int NW, bool DUMP>
@@ -1608,17 +1578,17 @@ bool launch_res_rt(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_mf
         }
         return false;
     }
-    const size_t one = Res<DT, RT>::bytes(kb, 1);
+    const size_t one = Res<DT, RT>::bytes(kb);
     if (one <= (size_t)kMaxLds) {
         if constexpr (kCanOffset<DT, DUMP>) {
             if (has_offset(*w)) {
-                *err = sixteen ? launch_res_inst<DT, RT, 16, 1, DUMP, true>(w, a, m, y, one, grid, d, s)
-                               : launch_res_inst<DT, RT, 8, 1, DUMP, true>(w, a, m, y, one, grid, d, s);
+                *err = sixteen ? launch_res_inst<DT, RT, 16, DUMP, true>(w, a, m, y, one, d, s)
+                               : launch_res_inst<DT, RT, 8, DUMP, true>(w, a, m, y, one, d, s);
                 return true;
             }
         }
-        *err = sixteen ? launch_res_inst<DT, RT, 16, 1, DUMP>(w, a, m, y, one, grid, d, s)
-                       : launch_res_inst<DT, RT, 8, 1, DUMP>(w, a, m, y, one, grid, d, s);
+        *err = sixteen ? launch_res_inst<DT, RT, 16, DUMP>(w, a, m, y, one, d, s)
+                       : launch_res_inst<DT, RT, 8, DUMP>(w, a, m, y, one, d, s);
         return true;
     }
     return false;
