@@ -98,6 +98,21 @@ __device__ __forceinline__ void load_head(const cq_weight &w, int64_t blk, WHead
     r.d = ((const uint16_t *)w.p3)[blk];
 }
 
+// An empty statement that may change the fields (in the registers their loads came to, four at once).
+__device__ __forceinline__ void hold_head(WHead<CQ_DTYPE_Q4K> &r) {
+    v4i v = {(int)r.dd, (int)r.rec.x, (int)r.rec.y, (int)r.rec.z};
+    asm volatile("" : "+v"(v), "+v"(r.rec.w));
+    r.dd = (uint32_t)v.x;
+    r.rec.x = (uint32_t)v.y;
+    r.rec.y = (uint32_t)v.z;
+    r.rec.z = (uint32_t)v.w;
+}
+__device__ __forceinline__ void hold_head(WHead<CQ_DTYPE_Q6K> &r) {
+    v4i v = __builtin_bit_cast(v4i, r.sc);
+    asm volatile("" : "+v"(v), "+v"(r.d));
+    r.sc = __builtin_bit_cast(uint4, v);
+}
+
 // Weight operands of one block for lane (row r = l%16, k quarter kq = l/16): the two digit operands
 // of the four 64-wide K-slices, the block scale and the Q4K min-term operand.
 __device__ __forceinline__ void block_unpack(const uint8_t *wl, int lane, const WHead<CQ_DTYPE_Q4K> &wb, v4i (&bl)[4],
@@ -451,8 +466,8 @@ __global__ void __launch_bounds__(NW * 64) skinny_kernel(cq_weight w, cq_act_vie
 // waves: one block each for 4096 columns, a single memory round trip).  The launcher takes it where every
 // workgroup has one 16-row weight tile (n <= 16 x the number of CUs); walking several tiles measured no faster than
 // the kernel above, also with the next tile's weights copied ahead into a second buffer.  The loop over tiles cost registers that sixteen
-// waves do not have, and spills with 17 rows and more (whole calls, us, with it -> without, 4096 x 4096: 24 rows Q4K 9.3 -> 7.8, Q5K 11.9 ->
-// 8.6, Q2K 10.7 -> 8.9; 8 rows Q4K 7.0 -> 6.8, Q2K 8.7 -> 8.1; Q6K level).
+// waves do not have, and spills with 17 rows and more (whole calls from a graph, weights from HBM, us, with it -> without, 4096 x 4096: 24 rows
+// Q4K 10.7 -> 9.4, Q5K 14.2 -> 9.9, Q2K 12.6 -> 11.2; 8 rows Q2K 10.0 -> 9.7; Q4K, Q5K and Q6K with 8 and 16 rows level).
 //   per K block b  : act [RT][2 K-halves][8 rows][8 chunks] | d8 [8*RT] f32 | bsh [8*RT][16] f16 (k4 types)
 //   per K block    : weights (kWgt bytes); a wave's first buffer also carries its partial results (1 KiB per 16 activation rows)
 template <int DT, int RT> struct Res {
@@ -623,20 +638,25 @@ __global__ void __launch_bounds__(kWaves * 64) skinny_resident_kernel(cq_weight 
             res_issue_weights<DT>(wgt_base + b * R::kWgt, pl, (uint32_t)n_tile, b, kb32, wq_off, wh_off, w5_off, lane);
         }
     }
-    __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
-    if constexpr (DT == CQ_DTYPE_Q6K) {
-        // (the block scale is converted from here on: the conversion moved up to its load, which then was waited for before any copy went out)
-#pragma unroll
-        for (int j = 0; j < kMaxBpw; j++) asm volatile("" : "+v"(head[j].d));
-    }
     v4f out[NT];
 #pragma unroll
     for (int t = 0; t < NT; t++) out[t] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    // One pass of a loop whose count the compiler does not know: what does not depend on the data (addresses in the images, the lane's masks) is
+    // then formed in front of it, while the copies are on their way, and not behind the wait in each block that uses it.  The block fields
+    // change in the loop as far as the compiler can see, so that nothing made of them moves in front and waits for them there.  (Without the
+    // loop, weights from HBM: Q6K 4096 x 4096 with 8 rows 9.0 -> 9.3 us, with 24 10.1 -> 10.2, Q4K 4096 x 2048 6.7 -> 6.9.)
+    int passes = 1;
+    asm volatile("" : "+s"(passes));
+    for (int pass = 0; pass < passes; pass++) {
+        __builtin_amdgcn_s_waitcnt(0);   // everything above has landed
 #pragma unroll
-    for (int j = 0; j < kMaxBpw; j++) {
-        const int64_t b = wave + (int64_t)j * kWaves;
-        if (b < kb)
-            res_block<DT, RT, NT, DUMP>(wgt_base + b * R::kWgt, smem + b * R::kActBlk, lane, head[j], a_col, out, dump, (n_tile + r) * kb + b, w.n * kb, m);
+        for (int j = 0; j < kMaxBpw; j++) {
+            const int64_t b = wave + (int64_t)j * kWaves;
+            if (b < kb) {
+                hold_head(head[j]);
+                res_block<DT, RT, NT, DUMP>(wgt_base + b * R::kWgt, smem + b * R::kActBlk, lane, head[j], a_col, out, dump, (n_tile + r) * kb + b, w.n * kb, m);
+            }
+        }
     }
     if (DUMP) return;
     if constexpr (OFF) {
