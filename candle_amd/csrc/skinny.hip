@@ -1809,9 +1809,14 @@ bool cq_skinny_in_groups(const cq_weight *w, int64_t m) {
     const int64_t pairs = (w->n + 15) / 16 * 2, cus = cq_num_cus();   // groups of 16 with up to 32 rows
     return m > 32 || (m > 16 && (blk32 ? pairs <= (one_step ? 2 : 1) * cus : !one_step && pairs <= cus));
 }
+// (33 to 128 weight rows: 0.4 us more for every MiB of quantized rows.  With so few weight tiles the launch waits for the rows, and the tile kernel,
+// half of whose waves are idle there, is ahead of its estimate.  Without that the choice lost up to a fifth, us, tiles -> groups: Q4K 128 x 8192
+// with 2048 rows 32.6 -> 41.0, 96 x 8192 with 512 14.1 -> 16.8, Q8_0 96 x 4096 with 1024 15.5 -> 18.5.  Of 375 cases (64, 96 and 128 weight rows,
+// 128 to 2048 rows) 76 change to the tiles: 53 are more than 3 % faster, 7 slower, by 7 % at most.)
 double cq_skinny_groups_us(const cq_weight *w, int64_t m) {
     const GroupsUs us = groups_us(w, m);
-    return us.sixteen < us.thirty_two ? us.sixteen : us.thirty_two;
+    const double rows = w->n > 32 && w->n <= 128 ? 0.4 * (double)m * (double)w->k / (double)(1 << 20) : 0.0;
+    return (us.sixteen < us.thirty_two ? us.sixteen : us.thirty_two) + rows;
 }
 bool cq_skinny_supported(const cq_weight *w, int act_dtype) {
     return cq_skinny_takes(w, act_dtype) && w->k % 256 == 0 && w->n % 16 == 0;
