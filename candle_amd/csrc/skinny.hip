@@ -1834,8 +1834,9 @@ hipError_t cq_launch_skinny_dump(const cq_weight *w, cq_act_view a, int act_dtyp
 // every workgroup repeats for its eight rows costs less than the launch it saves.  Measured, us back to back / from a graph, against the two
 // launches:
 //   Q4K 1024 x 1024, 5 rows 4.8 / 4.5 against 7.5 / 5.0; 8 rows 4.8 / 4.5 against 7.4 / 5.1; 326 x 768, 12 rows 4.7 / 4.7 against 8.6 / 5.7; Q6K
-//   4096 x 1024, 8 rows 5.0 / 4.7 against 7.3 / 5.3; Q8_0 1024 x 1024, 5 rows 4.7 / 4.4 against 7.4 / 5.2, 8 rows 5.5 / 5.3 against 7.4 / 5.3
-// and beyond the limits below behind from a graph or everywhere: two blocks a wave or two workgroups a CU double the quantizing
+//   4096 x 1024, 8 rows 5.0 / 4.7 against 7.3 / 5.3; Q8_0 1024 x 1024, 5 rows 5.0 / 4.8 against 8.0 / 5.2
+// level or a little behind from a graph at the most rows of the 32-element types (Q8_0 1024 x 1024, 8 rows 5.9 / 5.6 against 7.9 / 5.3, Q4_0, 7
+// rows 5.9 / 5.7 against 8.0 / 5.5), and beyond the limits below behind from a graph or everywhere: two blocks a wave or two workgroups a CU double the quantizing
 // (Q4K 2048 x 2048, 8 rows 6.0 against 6.8 / 5.6; 8192 x 2048 10.6 against 7.3), Q4_0 with 8 rows 5.9 / 5.7 against 7.4 / 5.5.
 // More than eight rows (K-quants): up to a workgroup a CU and a block a wave, on random shapes 1.25 to 1.7 times as fast back to back (1024 x 1024
 // with 32 rows 8.1 -> 5.2, Q6K 512 x 2048 with 64 11.9 -> 6.8, Q5K 256 x 1024 with 128 11.3 -> 5.6) and at least 1.03 times from a graph; Q8_0 and
