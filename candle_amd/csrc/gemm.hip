@@ -716,23 +716,26 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
 
 template <int DT, int MT>
 __global__ void __launch_bounds__(kThreads) gemm_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
-                                                        int ksplit) {
-    gemm_body<DT, MT>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, y, ksplit);
+                                                        int ksplit, int strips) {
+    const cq_tile t = cq_tile_at(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, strips);
+    gemm_body<DT, MT>(w, a, t.x, (int64_t)t.y * (MT * 32), m, y, ksplit);
 }
 
 // 128-row tiles in whole rounds of workgroups, and what is left of them in tiles of 32 * TAIL rows: the last round of a launch
-// that does not fill it then lasts as long as a shorter tile.  `whole` of the `gx` x row tiles (column tiles first) are taken
+// that does not fill it then lasts as long as a shorter tile.  `whole` of the `gx` x row tiles (in strips) are taken
 // whole, the others by 4 / TAIL workgroups each.  Measured at pick_plan.
 template <int DT, int TAIL, bool DUMP>
 __device__ __forceinline__ void tail_body(const cq_weight &w, const cq_act_view &a, int64_t m, float *__restrict__ y, uint32_t gx,
                                           uint32_t whole, cq_mfma_dump dump) {
-    const uint32_t id = blockIdx.x;
+    const uint32_t id = blockIdx.x, gy = (uint32_t)((m + 127) / 128);
     if (id < whole) {
-        gemm_body<DT, 4, DUMP>(w, a, id % gx, (int64_t)(id / gx) * 128, m, y, 1, dump);
+        const cq_tile t = cq_tile_in_strips(cq_tile_of_xcd(id, whole), gx, gy);
+        gemm_body<DT, 4, DUMP>(w, a, t.x, (int64_t)t.y * 128, m, y, 1, dump);
     } else {
-        const uint32_t t = whole + (id - whole) / (4 / TAIL), part = (id - whole) % (4 / TAIL);
-        const int64_t m0 = (int64_t)(t / gx) * 128 + part * (32 * TAIL);
-        if (m0 < m) gemm_body<DT, TAIL, DUMP>(w, a, t % gx, m0, m, y, 1, dump);
+        const uint32_t at = cq_tile_of_xcd(id - whole, gridDim.x - whole);
+        const cq_tile t = cq_tile_in_strips(whole + at / (4 / TAIL), gx, gy);
+        const int64_t m0 = (int64_t)t.y * 128 + at % (4 / TAIL) * (32 * TAIL);
+        if (m0 < m) gemm_body<DT, TAIL, DUMP>(w, a, t.x, m0, m, y, 1, dump);
     }
 }
 template <int DT, int TAIL>
@@ -1204,7 +1207,7 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
             return hipGetLastError();
         }
     }
-    CQ_LAUNCH((gemm_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y, ksplit);
+    CQ_LAUNCH((gemm_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, cq_tiles_in_strips(gx * gy, ksplit));
     return hipGetLastError();
 }
 

@@ -301,8 +301,9 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
 
 template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, int ksplit,
-                                                          cq_mfma_dump dump) {
-    gemm32_body<DT, MT, DUMP, ONCE, SHORT>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, y, ksplit, dump);
+                                                          int strips, cq_mfma_dump dump) {
+    const cq_tile t = cq_tile_at(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, strips);
+    gemm32_body<DT, MT, DUMP, ONCE, SHORT>(w, a, t.x, (int64_t)t.y * (MT * 32), m, y, ksplit, dump);
 }
 
 // Few column tiles: K halved inside the workgroup (as gemm_kh_kernel of gemm.hip).  A workgroup covers 128 weight rows x 32*MT
@@ -483,17 +484,19 @@ __global__ void __launch_bounds__(kThreads) gemm32_few_kernel(cq_weight w, cq_ac
 }
 
 // 128-row tiles in whole rounds of workgroups, what is left of them in tiles of 32 * TAIL rows (as gemm_tail_kernel of
-// gemm.hip): `whole` of the gx x row tiles, column tiles first, are taken whole, the others by 4 / TAIL workgroups each.
+// gemm.hip): `whole` of the gx x row tiles, in strips, are taken whole, the others by 4 / TAIL workgroups each.
 template <int DT, int TAIL, bool DUMP, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_tail_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t gx,
                                                                uint32_t whole, cq_mfma_dump dump) {
-    const uint32_t id = blockIdx.x;
+    const uint32_t id = blockIdx.x, gy = (uint32_t)((m + 127) / 128);
     if (id < whole) {
-        gemm32_body<DT, 4, DUMP, false, SHORT>(w, a, id % gx, (int64_t)(id / gx) * 128, m, y, 1, dump);
+        const cq_tile t = cq_tile_in_strips(cq_tile_of_xcd(id, whole), gx, gy);
+        gemm32_body<DT, 4, DUMP, false, SHORT>(w, a, t.x, (int64_t)t.y * 128, m, y, 1, dump);
     } else {
-        const uint32_t t = whole + (id - whole) / (4 / TAIL), part = (id - whole) % (4 / TAIL);
-        const int64_t m0 = (int64_t)(t / gx) * 128 + part * (32 * TAIL);
-        if (m0 < m) gemm32_body<DT, TAIL, DUMP, false, SHORT>(w, a, t % gx, m0, m, y, 1, dump);
+        const uint32_t at = cq_tile_of_xcd(id - whole, gridDim.x - whole);
+        const cq_tile t = cq_tile_in_strips(whole + at / (4 / TAIL), gx, gy);
+        const int64_t m0 = (int64_t)t.y * 128 + at % (4 / TAIL) * (32 * TAIL);
+        if (m0 < m) gemm32_body<DT, TAIL, DUMP, false, SHORT>(w, a, t.x, m0, m, y, 1, dump);
     }
 }
 
@@ -584,7 +587,7 @@ hipError_t launch_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, i
     const size_t lds = Tile<DT, MT>::kTotal;
     if (hipError_t e = cq_ensure_lds<gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>>(w->dev, lds); e != hipSuccess) return e;
     const dim3 grid((unsigned)((w->n + kWaves * 32 - 1) / (kWaves * 32)), (unsigned)((m + MT * 32 - 1) / (MT * 32)), (unsigned)ksplit);
-    CQ_LAUNCH((gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, d);
+    CQ_LAUNCH((gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, cq_tiles_in_strips((int64_t)grid.x * grid.y, ksplit), d);
     return hipGetLastError();
 }
 template <int DT, int TAIL, bool DUMP, bool SHORT>

@@ -21,6 +21,14 @@ def test_last_round_in_shorter_tiles(qh, dt, m, n, k):  # noqa: F811
     check(qh, dt, m, n, k)
 
 
+@pytest.mark.parametrize("dt", ["Q4K", "Q6K", "Q8_0"])
+@pytest.mark.parametrize("m,n,k", [(2100, 6400, 256),          # 17 x 25 tiles in strips of eight columns: the last strip has one
+                                   (17000, 700, 256),          # three columns only
+                                   (4400, 1800, 512)])         # one whole strip
+def test_several_rounds_in_strips(qh, dt, m, n, k):  # noqa: F811
+    check(qh, dt, m, n, k)
+
+
 @pytest.mark.parametrize("dt", ["Q8_0", "Q4_0"])
 @pytest.mark.parametrize("m,n,k", [(1100, 8192, 320), (1000, 11264 - 3, 576)])
 def test_rows_of_no_whole_step(qh, dt, m, n, k):  # noqa: F811
