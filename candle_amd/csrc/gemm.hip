@@ -608,7 +608,7 @@ __device__ __forceinline__ int64_t last_tile(int64_t n_own, int64_t n) { return 
 // blockIdx.x, K blocks of part blockIdx.z.
 template <int DT, int MT, bool DUMP = false, int WBUF = 1, bool ONCE = false>
 __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view &a, int64_t bx, int64_t m0, int64_t m,
-                                          float *__restrict__ y, int ksplit, cq_mfma_dump dump = cq_mfma_dump{nullptr, nullptr, 0}) {
+                                          float *__restrict__ y, int ksplit, bool stream, cq_mfma_dump dump = cq_mfma_dump{nullptr, nullptr, 0}) {
     static_assert(WBUF == 1 || DT == CQ_DTYPE_Q4K || DT == CQ_DTYPE_Q5K, "block headers of 20 bytes");
     typedef Tile<DT, MT> T;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -700,25 +700,24 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
         if (c < own) return;
         float *__restrict__ yc = y + (m0 + (ln >> 5) * 4) * w.n + c;
         const int64_t left = m - m0 - (ln >> 5) * 4;
+        cq_put_results(ksplit, stream, [&](auto how) {
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
+            for (int t = 0; t < MT; t++) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int64_t row = t * 32 + (i >> 2) * 8 + (i & 3);
-                if (row < left) {
-                    if (ksplit == 1) yc[row * w.n] = out[t][i];
-                    else unsafeAtomicAdd(&yc[row * w.n], out[t][i]);
+                for (int i = 0; i < 16; i++) {
+                    const int64_t row = t * 32 + (i >> 2) * 8 + (i & 3);
+                    if (row < left) cq_put_result<decltype(how)::value>(&yc[row * w.n], out[t][i]);
                 }
             }
-        }
+        });
     }
 }
 
 template <int DT, int MT>
 __global__ void __launch_bounds__(kThreads) gemm_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
-                                                        int ksplit, int strips) {
+                                                        int ksplit, int strips, int stream) {
     const cq_tile t = cq_tile_at(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, strips);
-    gemm_body<DT, MT>(w, a, t.x, (int64_t)t.y * (MT * 32), m, y, ksplit);
+    gemm_body<DT, MT>(w, a, t.x, (int64_t)t.y * (MT * 32), m, y, ksplit, stream != 0);
 }
 
 // 128-row tiles in whole rounds of workgroups, and what is left of them in tiles of 32 * TAIL rows: the last round of a launch
@@ -726,22 +725,22 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(cq_weight w, cq_act_view
 // whole, the others by 4 / TAIL workgroups each.  Measured at pick_plan.
 template <int DT, int TAIL, bool DUMP>
 __device__ __forceinline__ void tail_body(const cq_weight &w, const cq_act_view &a, int64_t m, float *__restrict__ y, uint32_t gx,
-                                          uint32_t whole, cq_mfma_dump dump) {
+                                          uint32_t whole, bool stream, cq_mfma_dump dump) {
     const uint32_t id = blockIdx.x, gy = (uint32_t)((m + 127) / 128);
     if (id < whole) {
         const cq_tile t = cq_tile_in_strips(cq_tile_of_xcd(id, whole), gx, gy);
-        gemm_body<DT, 4, DUMP>(w, a, t.x, (int64_t)t.y * 128, m, y, 1, dump);
+        gemm_body<DT, 4, DUMP>(w, a, t.x, (int64_t)t.y * 128, m, y, 1, stream, dump);
     } else {
         const uint32_t at = cq_tile_of_xcd(id - whole, gridDim.x - whole);
         const cq_tile t = cq_tile_in_strips(whole + at / (4 / TAIL), gx, gy);
         const int64_t m0 = (int64_t)t.y * 128 + at % (4 / TAIL) * (32 * TAIL);
-        if (m0 < m) gemm_body<DT, TAIL, DUMP>(w, a, t.x, m0, m, y, 1, dump);
+        if (m0 < m) gemm_body<DT, TAIL, DUMP>(w, a, t.x, m0, m, y, 1, stream, dump);
     }
 }
 template <int DT, int TAIL>
 __global__ void __launch_bounds__(kThreads) gemm_tail_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t gx,
-                                                             uint32_t whole) {
-    tail_body<DT, TAIL, false>(w, a, m, y, gx, whole, cq_mfma_dump{nullptr, nullptr, 0});
+                                                             uint32_t whole, int stream) {
+    tail_body<DT, TAIL, false>(w, a, m, y, gx, whole, stream != 0, cq_mfma_dump{nullptr, nullptr, 0});
 }
 
 // Up to 32 activation rows (one row tile): every weight byte is read once by the launch, cold - the form of the grouped
@@ -750,23 +749,23 @@ template <int DT> constexpr int once_wbuf() { return DT == CQ_DTYPE_Q4K || DT ==
 template <int DT>
 __global__ void __launch_bounds__(kThreads) gemm_once_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
                                                              int ksplit) {
-    gemm_body<DT, 1, false, once_wbuf<DT>(), true>(w, a, blockIdx.x, 0, m, y, ksplit);
+    gemm_body<DT, 1, false, once_wbuf<DT>(), true>(w, a, blockIdx.x, 0, m, y, ksplit, false);
 }
 
 // The same launch with the block integers stored instead of the result (verification).
 template <int DT, int MT>
 __global__ void __launch_bounds__(kThreads) gemm_dump_kernel(cq_weight w, cq_act_view a, int64_t m, int ksplit,
                                                              cq_mfma_dump dump) {
-    gemm_body<DT, MT, true>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, nullptr, ksplit, dump);
+    gemm_body<DT, MT, true>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, nullptr, ksplit, false, dump);
 }
 template <int DT>
 __global__ void __launch_bounds__(kThreads) gemm_once_dump_kernel(cq_weight w, cq_act_view a, int64_t m, int ksplit, cq_mfma_dump dump) {
-    gemm_body<DT, 1, true, once_wbuf<DT>(), true>(w, a, blockIdx.x, 0, m, nullptr, ksplit, dump);
+    gemm_body<DT, 1, true, once_wbuf<DT>(), true>(w, a, blockIdx.x, 0, m, nullptr, ksplit, false, dump);
 }
 template <int DT, int TAIL>
 __global__ void __launch_bounds__(kThreads) gemm_tail_dump_kernel(cq_weight w, cq_act_view a, int64_t m, uint32_t gx, uint32_t whole,
                                                                   cq_mfma_dump dump) {
-    tail_body<DT, TAIL, true>(w, a, m, nullptr, gx, whole, dump);
+    tail_body<DT, TAIL, true>(w, a, m, nullptr, gx, whole, false, dump);
 }
 
 // ------------------------------------------------------ few weight rows, long K: K halved inside the workgroup ----
@@ -813,7 +812,7 @@ __device__ __forceinline__ void block_step_kh(const uint8_t *__restrict__ cur, u
 // Requires n >= 32.  One workgroup: activation rows [m0, m0 + 32*MT) x the 128 weight rows of blockIdx.x, all K.
 // (D: nothing, or cq_mfma_dump for the launch that stores the block integers: the production kernel keeps its arguments and registers)
 template <int DT, int MT, typename... D>
-__global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, D... dump) {
+__global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, int stream, D... dump) {
     constexpr bool DUMP = sizeof...(D) > 0;
     typedef Tile<DT, MT> T;
     typedef TileKH<DT, MT> TK;
@@ -887,14 +886,16 @@ __global__ void __launch_bounds__(kThreads) gemm_kh_kernel(cq_weight w, cq_act_v
     }
     __syncthreads();
     if (half == 0 && n_ok) {
+        cq_put_results(1, stream != 0, [&](auto how) {
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
+            for (int t = 0; t < MT; t++) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                if (row < m && n >= n_own) y[row * w.n + n] = out[t][i] + part[(t * 16 + i) * 64 + lane];
+                for (int i = 0; i < 16; i++) {
+                    const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+                    if (row < m && n >= n_own) cq_put_result<decltype(how)::value>(&y[row * w.n + n], out[t][i] + part[(t * 16 + i) * 64 + lane]);
+                }
             }
-        }
+        });
     }
 }
 
@@ -908,8 +909,8 @@ __global__ void __launch_bounds__(kThreads) gemm_grouped_kernel(cq_group_args ga
                                                                 int ksplit) {
     const int tile = blockIdx.y;
     const cq_weight w = ga.w[ga.expert[tile]];
-    if constexpr (MT == 1) gemm_body<DT, 1, false, grouped_wbuf<DT>(), true>(w, a, blockIdx.x, ga.row0[tile], ga.row_end[tile], y, ksplit);
-    else gemm_body<DT, MT>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit);
+    if constexpr (MT == 1) gemm_body<DT, 1, false, grouped_wbuf<DT>(), true>(w, a, blockIdx.x, ga.row0[tile], ga.row_end[tile], y, ksplit, false);
+    else gemm_body<DT, MT>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit, false);
 }
 
 // ------------------------------------------------ K-quant weights x Q8_1 activations (tile kernel) ----
@@ -1207,7 +1208,7 @@ hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int
             return hipGetLastError();
         }
     }
-    CQ_LAUNCH((gemm_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, cq_tiles_in_strips(gx * gy, ksplit));
+    CQ_LAUNCH((gemm_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, cq_tiles_in_strips(gx * gy, ksplit), (int)cq_streams_result(w, m));
     return hipGetLastError();
 }
 
@@ -1218,10 +1219,10 @@ hipError_t launch_kh(const cq_weight *w, cq_act_view a, int64_t m, float *y, cq_
     dim3 grid((unsigned)((w->n + 127) / 128), (unsigned)((m + MT * 32 - 1) / (MT * 32)), 1);
     if constexpr (DUMP) {
         if (hipError_t e = cq_ensure_lds<gemm_kh_kernel<DT, MT, cq_mfma_dump>>(w->dev, lds); e != hipSuccess) return e;
-        CQ_LAUNCH((gemm_kh_kernel<DT, MT, cq_mfma_dump>), grid, kThreads, lds, s, *w, a, m, y, d);
+        CQ_LAUNCH((gemm_kh_kernel<DT, MT, cq_mfma_dump>), grid, kThreads, lds, s, *w, a, m, y, 0, d);
     } else {
         if (hipError_t e = cq_ensure_lds<gemm_kh_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
-        CQ_LAUNCH((gemm_kh_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y);
+        CQ_LAUNCH((gemm_kh_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y, (int)cq_streams_result(w, m));
     }
     return hipGetLastError();
 }
@@ -1236,7 +1237,7 @@ hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, c
         CQ_LAUNCH((gemm_tail_dump_kernel<DT, TAIL>), grid, kThreads, lds, s, *w, a, m, (uint32_t)gx, (uint32_t)whole, d);
     } else {
         if (hipError_t e = cq_ensure_lds<gemm_tail_kernel<DT, TAIL>>(w->dev, lds); e != hipSuccess) return e;
-        CQ_LAUNCH((gemm_tail_kernel<DT, TAIL>), grid, kThreads, lds, s, *w, a, m, y, (uint32_t)gx, (uint32_t)whole);
+        CQ_LAUNCH((gemm_tail_kernel<DT, TAIL>), grid, kThreads, lds, s, *w, a, m, y, (uint32_t)gx, (uint32_t)whole, (int)cq_streams_result(w, m));
     }
     return hipGetLastError();
 }

@@ -235,7 +235,7 @@ __device__ __forceinline__ void step_mac(const uint8_t *cur, const LaneGeo &g, c
 // SHORT: K is no multiple of 256, the last step has fewer than eight blocks.
 template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT, bool ANYROW = false>
 __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_view &a, int64_t bx, int64_t m0, int64_t m, float *__restrict__ y,
-                                            int ksplit, cq_mfma_dump dump) {
+                                            int ksplit, bool stream, cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
     extern __shared__ __align__(16) uint8_t smem[];
     const int lane = threadIdx.x & 63;
@@ -285,25 +285,24 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
     }
 
     if (n_ok && !DUMP) {
+        cq_put_results(ksplit, stream, [&](auto how) {
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
+            for (int t = 0; t < MT; t++) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                if (row < m && n >= n_own) {
-                    if (ksplit == 1) y[row * w.n + n] = out[t][i];
-                    else unsafeAtomicAdd(&y[row * w.n + n], out[t][i]);
+                for (int i = 0; i < 16; i++) {
+                    const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+                    if (row < m && n >= n_own) cq_put_result<decltype(how)::value>(&y[row * w.n + n], out[t][i]);
                 }
             }
-        }
+        });
     }
 }
 
 template <int DT, int MT, bool DUMP, bool ONCE, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, int ksplit,
-                                                          int strips, cq_mfma_dump dump) {
+                                                          int strips, int stream, cq_mfma_dump dump) {
     const cq_tile t = cq_tile_at(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, strips);
-    gemm32_body<DT, MT, DUMP, ONCE, SHORT>(w, a, t.x, (int64_t)t.y * (MT * 32), m, y, ksplit, dump);
+    gemm32_body<DT, MT, DUMP, ONCE, SHORT>(w, a, t.x, (int64_t)t.y * (MT * 32), m, y, ksplit, stream != 0, dump);
 }
 
 // Few column tiles: K halved inside the workgroup (as gemm_kh_kernel of gemm.hip).  A workgroup covers 128 weight rows x 32*MT
@@ -322,7 +321,8 @@ template <int DT, int MT> struct TileKH {
 // Row tiles that gemm32_kh_kernel's stages leave room for beside the weights (Q8_0: 8 KiB a wave).
 template <int DT> constexpr int kh_tallest() { return DT == CQ_DTYPE_Q4_0 ? 3 : 2; }
 template <int DT, int MT, bool DUMP, bool SHORT, bool LOWER>
-__global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, cq_mfma_dump dump) {
+__global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, int stream,
+                                                             cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
     typedef TileKH<DT, MT> TK;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -384,14 +384,16 @@ __global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act
     }
     __syncthreads();
     if (half == 0 && n_ok) {
+        cq_put_results(1, stream != 0, [&](auto how) {
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
+            for (int t = 0; t < MT; t++) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                if (row < m && n >= n_own) y[row * w.n + n] = out[t][i] + part[(t * 16 + i) * 64 + lane];
+                for (int i = 0; i < 16; i++) {
+                    const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
+                    if (row < m && n >= n_own) cq_put_result<decltype(how)::value>(&y[row * w.n + n], out[t][i] + part[(t * 16 + i) * 64 + lane]);
+                }
             }
-        }
+        });
     }
 }
 
@@ -487,16 +489,16 @@ __global__ void __launch_bounds__(kThreads) gemm32_few_kernel(cq_weight w, cq_ac
 // gemm.hip): `whole` of the gx x row tiles, in strips, are taken whole, the others by 4 / TAIL workgroups each.
 template <int DT, int TAIL, bool DUMP, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_tail_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t gx,
-                                                               uint32_t whole, cq_mfma_dump dump) {
+                                                               uint32_t whole, int stream, cq_mfma_dump dump) {
     const uint32_t id = blockIdx.x, gy = (uint32_t)((m + 127) / 128);
     if (id < whole) {
         const cq_tile t = cq_tile_in_strips(cq_tile_of_xcd(id, whole), gx, gy);
-        gemm32_body<DT, 4, DUMP, false, SHORT>(w, a, t.x, (int64_t)t.y * 128, m, y, 1, dump);
+        gemm32_body<DT, 4, DUMP, false, SHORT>(w, a, t.x, (int64_t)t.y * 128, m, y, 1, stream != 0, dump);
     } else {
         const uint32_t at = cq_tile_of_xcd(id - whole, gridDim.x - whole);
         const cq_tile t = cq_tile_in_strips(whole + at / (4 / TAIL), gx, gy);
         const int64_t m0 = (int64_t)t.y * 128 + at % (4 / TAIL) * (32 * TAIL);
-        if (m0 < m) gemm32_body<DT, TAIL, DUMP, false, SHORT>(w, a, t.x, m0, m, y, 1, dump);
+        if (m0 < m) gemm32_body<DT, TAIL, DUMP, false, SHORT>(w, a, t.x, m0, m, y, 1, stream != 0, dump);
     }
 }
 
@@ -506,7 +508,7 @@ template <int DT, int MT, bool SHORT>
 __global__ void __launch_bounds__(kThreads) gemm32_grouped_kernel(cq_group_args ga, cq_act_view a, float *__restrict__ y, int ksplit) {
     const int tile = blockIdx.y;
     const cq_weight w = ga.w[ga.expert[tile]];
-    gemm32_body<DT, MT, false, MT == 1, SHORT, true>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit,
+    gemm32_body<DT, MT, false, MT == 1, SHORT, true>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit, false,
                                                cq_mfma_dump{nullptr, nullptr, 0});
 }
 
@@ -587,7 +589,8 @@ hipError_t launch_inst(const cq_weight *w, cq_act_view a, int64_t m, float *y, i
     const size_t lds = Tile<DT, MT>::kTotal;
     if (hipError_t e = cq_ensure_lds<gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>>(w->dev, lds); e != hipSuccess) return e;
     const dim3 grid((unsigned)((w->n + kWaves * 32 - 1) / (kWaves * 32)), (unsigned)((m + MT * 32 - 1) / (MT * 32)), (unsigned)ksplit);
-    CQ_LAUNCH((gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, cq_tiles_in_strips((int64_t)grid.x * grid.y, ksplit), d);
+    CQ_LAUNCH((gemm32_kernel<DT, MT, DUMP, ONCE, SHORT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, cq_tiles_in_strips((int64_t)grid.x * grid.y, ksplit),
+              (int)cq_streams_result(w, m), d);
     return hipGetLastError();
 }
 template <int DT, int TAIL, bool DUMP, bool SHORT>
@@ -596,7 +599,7 @@ hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, c
     if (hipError_t e = cq_ensure_lds<gemm32_tail_kernel<DT, TAIL, DUMP, SHORT>>(w->dev, lds); e != hipSuccess) return e;
     const int64_t gx = (w->n + kWaves * 32 - 1) / (kWaves * 32), tiles = gx * ((m + 127) / 128), whole = tiles / cq_num_cus() * cq_num_cus();
     CQ_LAUNCH((gemm32_tail_kernel<DT, TAIL, DUMP, SHORT>), (unsigned)(whole + (tiles - whole) * (4 / TAIL)), kThreads, lds, s, *w, a, m, y,
-              (uint32_t)gx, (uint32_t)whole, d);
+              (uint32_t)gx, (uint32_t)whole, (int)cq_streams_result(w, m), d);
     return hipGetLastError();
 }
 // A single row tile over that many bytes of weights and more: the copies marked non-temporal (measured at 17 and 32 rows:
@@ -631,7 +634,7 @@ template <int DT, int MT, bool DUMP> hipError_t launch_kh(const cq_weight *w, cq
         const size_t lds = TileKH<DT, MT>::kTotal;
         if (hipError_t e = cq_ensure_lds<gemm32_kh_kernel<DT, MT, DUMP, SHORT, LOWER>>(w->dev, lds); e != hipSuccess) return e;
         CQ_LAUNCH((gemm32_kh_kernel<DT, MT, DUMP, SHORT, LOWER>), dim3((unsigned)((w->n + 127) / 128), (unsigned)((m + MT * 32 - 1) / (MT * 32))), kThreads, lds, s, *w,
-                  a, m, y, d);
+                  a, m, y, (int)cq_streams_result(w, m), d);
         return hipGetLastError();
     };
     auto whole_or_short = [&](auto low) {

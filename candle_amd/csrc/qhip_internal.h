@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <type_traits>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -90,6 +91,14 @@ int cq_set_error(int code, const char *fmt, ...);
 // then never split K (no partial sums added atomically in arrival order).
 bool cq_no_split_k();
 
+// Whether a plain tile launch marks its results non-temporal: outputs that would push the operands which the workgroups share out of the L2s (which hand
+// the lines on at the end of the launch anyway) and that no launch behind it reads back (the offset term of Q2K, Q4_1 and Q5_1 does).  Whole calls,
+// us, plain -> non-temporal: Q4K 11008 x 4096 at 4096 rows 425 -> 416, 14336 x 4096 at 512 74.8 -> 71.5, 3840 x 1536 at 1466 34.7 -> 31.9, 6636 x 768
+// at 659 22.1 -> 20.9, Q3K 16800 x 4096 at 226 70.5 -> 67.3, Q4_0 14080 x 1280 at 190 21.4 -> 20.5, Q8_0 11008 x 4096 at 4096 554 -> 550.  Read back: Q2K
+// 7447 x 3840 at 220 48.4 -> 49.2, Q4_1 1536 x 768 at 113 13.0 -> 13.5; gate and up of 8 small experts, which w2 reads, 33.8 -> 36.6; the few
+// single floats of the one-row kernels: Q4K 4096 x 4096 4.07 -> 4.41.  Up to 4 MB of results level.
+inline bool cq_streams_result(const cq_weight *w, int64_t m);
+
 // Compute units of the device (the first one asked; a process has devices of one kind), looked up once.
 int cq_num_cus();
 // Whether the tiles of a launch go to the workgroups in strips (cq_tile_at): more tiles than run at a time, K not split.  With one round the
@@ -114,6 +123,9 @@ __host__ __device__ inline bool cq_has_min32(int ggml_dtype) { return ggml_dtype
 // q + 32, plus the planes p4 / p5 of the groups' minima and dmin: the Q6K kernels give sum_b d * d8 * I_b of its dot
 // product with Q8K activations, cq_launch_min16_term subtracts sum_b dmin * d8 * sum_j bsums_j * m_j.
 __host__ __device__ inline bool cq_has_min16(int ggml_dtype) { return ggml_dtype == CQ_DTYPE_Q2K; }
+inline bool cq_streams_result(const cq_weight *w, int64_t m) {
+    return !cq_has_min32(w->ggml_dtype) && !cq_has_min16(w->ggml_dtype) && m * w->n >= (1 << 20);
+}
 inline int cq_storage_dtype(int ggml_dtype) {
     if (ggml_dtype == CQ_DTYPE_Q5_0 || cq_has_min32(ggml_dtype)) return CQ_DTYPE_Q8_0;
     return ggml_dtype == CQ_DTYPE_Q3K || ggml_dtype == CQ_DTYPE_Q2K ? CQ_DTYPE_Q6K : ggml_dtype;
@@ -484,6 +496,21 @@ __device__ __forceinline__ cq_u32x4 cq_min_term_groups_int(const uint32_t (&rec)
         out[2 * g + 1] = __builtin_amdgcn_perm(u, u, 0x03020302u);
     }
     return out;
+}
+
+// How a tile kernel's results leave a workgroup: plain stores, stores marked non-temporal (cq_streams_result says when), atomic additions (K split).
+enum cq_put { kPutPlain, kPutStream, kPutAdd };
+template <int HOW> __device__ __forceinline__ void cq_put_result(float *p, float v) {
+    if constexpr (HOW == kPutAdd) unsafeAtomicAdd(p, v);
+    // (a builtin store would be merged with the plain one of the other path and lose the mark)
+    else if constexpr (HOW == kPutStream) asm volatile("global_store_dword %0, %1, off nt" : : "v"(p), "v"(v) : "memory");
+    else *p = v;
+}
+// f(how) for the way that is wanted, a loop over the results each.
+template <class F> __device__ __forceinline__ void cq_put_results(int ksplit, bool stream, F f) {
+    if (ksplit > 1) f(std::integral_constant<int, kPutAdd>{});
+    else if (stream) f(std::integral_constant<int, kPutStream>{});
+    else f(std::integral_constant<int, kPutPlain>{});
 }
 
 // Which tile of `gx` column tiles x `gy` row tiles a workgroup of a tile kernel takes where the launch has several rounds of workgroups.
