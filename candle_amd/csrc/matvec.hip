@@ -424,7 +424,7 @@ template <int DT> struct UnitRaw {
 struct RowPtr {
     const uint8_t *p0, *p1, *p2, *p3;
 };
-template <int DT> __device__ __forceinline__ RowPtr row_ptr(const cq_weight &w, int64_t row, uint32_t units) {
+template <int DT, typename Planes> __device__ __forceinline__ RowPtr row_ptr(const Planes &w, int64_t row, uint32_t units) {
     constexpr int kB = Geo<DT>::kUnitsPerBlock;
     const int64_t g0 = row * units;   // units per row is a multiple of the units per block
     RowPtr rp;
@@ -631,8 +631,8 @@ __device__ __forceinline__ float offset_term(const uint8_t *smem, const LdsRow r
 // Loads of one weight row for this lane: units lane, lane + 64, ...  Lanes past the end of the row
 // re-read its last unit (same cache line as a neighbour, no extra traffic) and are masked when
 // accumulating, so the loads are unconditional and nothing waits on them early.
-template <int DT, int UPL, bool ORDERED = false>
-__device__ __forceinline__ void load_row(const cq_weight &w, int64_t row, uint32_t units, UnitRaw<DT> (&buf)[UPL]) {
+template <int DT, int UPL, bool ORDERED = false, typename Planes>
+__device__ __forceinline__ void load_row(const Planes &w, int64_t row, uint32_t units, UnitRaw<DT> (&buf)[UPL]) {
     const uint32_t lane = threadIdx.x & 63;
     constexpr uint32_t kB = Geo<DT>::kUnitsPerBlock;
     const RowPtr rp = row_ptr<DT>(w, row, units);
@@ -730,20 +730,25 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
     const uint32_t units = (uint32_t)(w.k / Geo<DT>::kElems);
     const int64_t row0 = (int64_t)blockIdx.x * NW + wave;
     const int64_t T = total_waves;
-    // weight, output and local row of a row of the launch (wave-uniform: scalar selects)
-    auto pick = [&](int64_t row, cq_weight &ws, float *&ys) -> int64_t {
-        ws = w;
+    // planes, output and local row of a row of the launch (wave-uniform: scalar selects; one value at a time, since a whole cq_weight
+    // that is overwritten in part is kept in scratch, for Q5K and Q6K: 80-104 bytes a lane, stored and read back for every row.  Whole calls,
+    // weights from HBM, one row, us: rms_norm + 3 x 4096 x 4096 Q6K 16.1 -> 10.6, Q5K 14.6 -> 9.8, 2 x 14336 x 4096 Q6K 30.3 -> 19.9)
+    auto pick = [&](int64_t row, RowPtr &p, float *&ys, int64_t &n) -> int64_t {
+        p = RowPtr{w.p0, w.p1, w.p2, w.p3};
         ys = y;
+        n = w.n;
         int64_t first = 0;
         if constexpr (NWT > 1) {
 #pragma unroll
             for (int t = 0; t < NWT - 1; t++) {
-                if (row >= more.first[t]) {
-                    ws.p0 = more.p[t][0]; ws.p1 = more.p[t][1]; ws.p2 = more.p[t][2]; ws.p3 = more.p[t][3];
-                    ws.n = more.n[t];
-                    ys = more.y[t];
-                    first = more.first[t];
-                }
+                const bool at = row >= more.first[t];
+                p.p0 = at ? more.p[t][0] : p.p0;
+                p.p1 = at ? more.p[t][1] : p.p1;
+                p.p2 = at ? more.p[t][2] : p.p2;
+                p.p3 = at ? more.p[t][3] : p.p3;
+                ys = at ? more.y[t] : ys;
+                n = at ? more.n[t] : n;
+                first = at ? more.first[t] : first;
             }
         }
         return row - first;
@@ -754,15 +759,16 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
     static_assert(!OFFSETS || (PRE == CQ_PRE_NONE && NWT == 1 && (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q6K)), "offset terms: Q8_0 / Q6K planes, one weight, no fused step");
     constexpr bool kOffsets = OFFSETS;
     auto load_launch_row = [&](int64_t row, UnitRaw<DT> (&buf)[UPL], OffsetRow<DT> &o) {
-        cq_weight ws;
+        RowPtr p;
         float *ys;
-        const int64_t lr = pick(row, ws, ys);
+        int64_t n;
+        const int64_t lr = pick(row, p, ys, n);
         // one activation row, longer weight rows of the types with one main plane: requests in unit order (measured:
         // Q8_0 4096 x 4096 5.9 -> 5.7 us, Q4K K = 14336 10.5 -> 10.3; Q6K, with three planes a unit, gains nothing at
         // one row and loses 11 % at two)
         constexpr bool kOrdered = MB == 1 && UPL >= 3 && DT != CQ_DTYPE_Q6K;
-        load_row<DT, UPL, kOrdered>(ws, lr, units, buf);
-        if constexpr (kOffsets) offset_load<DT>(ws, lr, o);
+        load_row<DT, UPL, kOrdered>(p, lr, units, buf);
+        if constexpr (kOffsets) offset_load<DT>(w, lr, o);
     };
     // rows of this wave (>= DEPTH): n / T, plus one for the first n % T waves (both from the host)
     const int64_t cnt = rows_per_wave + (row0 < rows_extra ? 1 : 0);
@@ -892,17 +898,18 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
         yscale_ok = yscale > 0.0f && yscale < __builtin_inff();
     }
     auto put = [&](int64_t row, Sums<MB> v, const OffsetRow<DT> &o) {
-        cq_weight ws;
+        RowPtr p;
         float *ys;
-        const int64_t lr = pick(row, ws, ys);
+        int64_t n;
+        const int64_t lr = pick(row, p, ys, n);
 #pragma unroll
         for (int m = 0; m < MB; m++) {
             float t = v.v[m];
             if constexpr (kRms && kPairs) t = yscale_ok ? t * yscale : 0.0f;
             if constexpr (kOffsets) {
-                t += offset_term<DT>(smem, rm[m], ws, o);   // the f32 addition the workspace path's second launch makes
+                t += offset_term<DT>(smem, rm[m], w, o);   // the f32 addition the workspace path's second launch makes
             }
-            if (lane == 0) ys[m * ws.n + lr] = t;
+            if (lane == 0) ys[m * n + lr] = t;
         }
     };
 
