@@ -546,8 +546,9 @@ static bool clear_in_quantizer_ok(const float *y, int64_t ny, const float *x, in
     return true;
 }
 
+// leave_rows: the quantized rows stay in the workspace for a call with CQ_FLAG_REUSE_ACT
 static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int64_t m, float *y_dev, int flags,
-                        void *ws, size_t ws_bytes, void *stream) {
+                        void *ws, size_t ws_bytes, void *stream, bool leave_rows = false) {
     const NoSplitScope no_split(flags);
     flags &= ~CQ_FLAG_DETERMINISTIC;   // (only the tile kernels' launch plans look at it; every other kernel is deterministic as it is)
     const size_t need = cq_workspace_bytes(w, m, flags);
@@ -615,7 +616,8 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     //   up to 64 rows where n is small and k short, so that the tile kernel cannot fill the machine.
     // (the 32-element-block types from 4 rows (Q8_0) or 5 rows (Q4_0) on: below that the one-launch dot-product
     // kernel is as fast or faster, it has no per-block scaling of MFMA results to do - where it takes the rows)
-    const bool rows_fused = flags == 0 && pre.kind == CQ_PRE_NONE && !in_place && cq_matvec_fused_rows_supported(w, m);
+    const bool rows_fused = flags == 0 && !in_place && ((pre.kind == CQ_PRE_NONE && cq_matvec_fused_rows_supported(w, m)) ||
+                                                        (pre.kind == CQ_PRE_RMS_NORM && !leave_rows && cq_matvec_fused_rms_rows_supported(&w, 1, m)));
     const int64_t skinny_from = w->dtype == CQ_DTYPE_Q8_0 ? 4 : w->dtype == CQ_DTYPE_Q4_0 ? 5 : 2;
     // (weights of 33 to 127 rows that are no whole number of 32-row tiles stay with the split-K kernel)
     const bool has_tile_kernel = cq_gemm_supported(w, m, act) || (w->n >= 128 && cq_gemm_takes(w, act));
@@ -662,7 +664,8 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     // two to four rows of short enough weight rows: the one-launch kernel again, every unpacked weight unit
     // contracted with each activation row
     if (rows_fused) {
-        CQ_HIP_CHECK(cq_launch_matvec_fused_rows(w, x_dev, m, y_dev, s));
+        if (pre.kind == CQ_PRE_RMS_NORM) CQ_HIP_CHECK(cq_launch_matvec_fused_multi(&w, 1, x_dev, pre, m, &y_dev, s));
+        else CQ_HIP_CHECK(cq_launch_matvec_fused_rows(w, x_dev, m, y_dev, s));
         return CQ_OK;
     }
     cq_act_view v;
@@ -774,7 +777,7 @@ extern "C" int cq_qmatmul_multi(const cq_weight *const *ws, int count, int pre, 
     for (int i = 0; i < count; i++) {
         const bool reuse = share && i > 0;
         if (int rc = qmatmul_impl(ws[i], x_dev, reuse ? cq_no_pre() : p, m, ys_dev[i], (reuse ? flags | CQ_FLAG_REUSE_ACT : flags) | det,
-                                  workspace, ws_bytes, stream))
+                                  workspace, ws_bytes, stream, share && count > 1))
             return rc;
     }
     return CQ_OK;

@@ -206,8 +206,8 @@ __device__ __forceinline__ float sum_sq4(float4 f) {
     t += f.w * f.w;
     return t;
 }
-// LDS offset of the per-chunk sums of squares: behind the activation image
-template <int DT> __host__ __device__ constexpr size_t fused_red_offset(int64_t k) { return (lds_row_bytes<DT>(k) + 15) / 16 * 16; }
+// LDS offset of the per-chunk sums of squares: behind the activation images
+template <int DT> __host__ __device__ constexpr size_t fused_red_offset(int64_t k, int rows = 1) { return (lds_row_bytes<DT>(k) * rows + 15) / 16 * 16; }
 
 // ---- Q8K activations, two chunks per wave ------------------------------------------------------
 // Lane l takes the eight consecutive elements 8*(l%32) + [0,8) of chunk 2*pair + l/32, so a wave
@@ -718,7 +718,7 @@ template <> struct FusedMore<1> {};
 // NWT > 1: up to NWT weights of the same type and row length take the same activations in one launch
 // (q, k, v of an attention block).  The launch's rows are the weights' rows one after the other;
 // `more` names the planes, outputs and row ranges of the weights behind the first.
-// MB > 1 (with PRE none and one weight): MB activation rows x[MB][k], outputs y[MB][n]; every weight row is
+// MB > 1 (with PRE none or rms_norm): MB activation rows x[MB][k], outputs y[MB][n]; every weight row is
 // unpacked once and contracted with each of them.
 template <int DT, int UPL, int NW, int DEPTH, int PRE, int NWT = 1, int MB = 1, bool OFFSETS = false>
 __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float *x, cq_pre pre,
@@ -757,6 +757,7 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
     // weights carry nothing for them): the minima of a row travel with the row's units, requested when they are and
     // summed when the row's result is stored.
     static_assert(!OFFSETS || (PRE == CQ_PRE_NONE && NWT == 1 && (DT == CQ_DTYPE_Q8_0 || DT == CQ_DTYPE_Q6K)), "offset terms: Q8_0 / Q6K planes, one weight, no fused step");
+    static_assert(MB == 1 || PRE == CQ_PRE_NONE || (PRE == CQ_PRE_RMS_NORM && Geo<DT>::kActK), "more rows: plain, or rms_norm of Q8K activations");
     constexpr bool kOffsets = OFFSETS;
     auto load_launch_row = [&](int64_t row, UnitRaw<DT> (&buf)[UPL], OffsetRow<DT> &o) {
         RowPtr p;
@@ -822,12 +823,12 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
     // there the elements are scaled before they are quantized, behind a barrier of its own.
     constexpr bool kRms = PRE == CQ_PRE_RMS_NORM;
     constexpr int kSlots = (kPairs ? 2 : 1) * XCH * NW;   // chunk slots of the workgroup (a multiple of 8)
-    const uint32_t red = (uint32_t)fused_red_offset<DT>(w.k);
-    auto row_scale = [&]() {
+    const uint32_t red = (uint32_t)fused_red_offset<DT>(w.k, MB);   // kSlots floats per activation row
+    auto row_scale = [&](int m) {
         // all slots are read at once and added in order; the zeros behind the last chunk change nothing
         float4 ps[kSlots / 4];
 #pragma unroll
-        for (int c = 0; c < kSlots / 4; c++) ps[c] = lds_get<float4>(smem, red + 16 * c);
+        for (int c = 0; c < kSlots / 4; c++) ps[c] = lds_get<float4>(smem, red + 4 * kSlots * m + 16 * c);
         float sum2 = ps[0].x;
         sum2 += ps[0].y; sum2 += ps[0].z; sum2 += ps[0].w;
 #pragma unroll
@@ -837,32 +838,35 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
     if constexpr (kRms) {
         const int chunks = (int)((w.k + 255) / 256);
 #pragma unroll
-        for (int i = 0; i < XCH; i++) {
-            if constexpr (kPairs) {
-                float t = sum_sq4(fx8[i].a) + sum_sq4(fx8[i].b);   // lane = group; 32 lanes = chunk
-                t += dpp_f<kQuadSwap1>(t);
-                t += dpp_f<kQuadSwap2>(t);
-                t += dpp_f<kHalfMirror>(t);
-                t += dpp_f<kRowMirror>(t);
-                const float p_lo = readlane_f(t, 0) + readlane_f(t, 16), p_hi = readlane_f(t, 32) + readlane_f(t, 48);
-                const int c = 2 * (wave + i * NW) + lane;   // every slot below kSlots is written: zero past the row
-                if (lane < 2) lds_put<float>(smem, red + 4 * c, c < chunks ? (lane ? p_hi : p_lo) : 0.0f);
-                fx8[i].a = mul4(fx8[i].a, gx8[i].a);
-                fx8[i].b = mul4(fx8[i].b, gx8[i].b);
-            } else {
-                const int c = wave + i * NW;
-                float t = c * 256 + 4 * lane < w.k ? sum_sq4(fx[i]) : 0.0f;   // two lanes = group
-                t += dpp_f<kQuadSwap1>(t);
-                t += dpp_f<kQuadSwap2>(t);
-                t += dpp_f<kHalfMirror>(t);
-                t += dpp_f<kRowMirror>(t);
-                const float p = (readlane_f(t, 0) + readlane_f(t, 16)) + (readlane_f(t, 32) + readlane_f(t, 48));
-                if (lane == 0) lds_put<float>(smem, red + 4 * c, c < chunks ? p : 0.0f);
+        for (int m = 0; m < MB; m++) {
+#pragma unroll
+            for (int i = 0; i < XCH; i++) {
+                if constexpr (kPairs) {
+                    float t = sum_sq4(fx8a[m][i].a) + sum_sq4(fx8a[m][i].b);   // lane = group; 32 lanes = chunk
+                    t += dpp_f<kQuadSwap1>(t);
+                    t += dpp_f<kQuadSwap2>(t);
+                    t += dpp_f<kHalfMirror>(t);
+                    t += dpp_f<kRowMirror>(t);
+                    const float p_lo = readlane_f(t, 0) + readlane_f(t, 16), p_hi = readlane_f(t, 32) + readlane_f(t, 48);
+                    const int c = 2 * (wave + i * NW) + lane;   // every slot below kSlots is written: zero past the row
+                    if (lane < 2) lds_put<float>(smem, red + 4 * (kSlots * m + c), c < chunks ? (lane ? p_hi : p_lo) : 0.0f);
+                    fx8a[m][i].a = mul4(fx8a[m][i].a, gx8[i].a);
+                    fx8a[m][i].b = mul4(fx8a[m][i].b, gx8[i].b);
+                } else {
+                    const int c = wave + i * NW;
+                    float t = c * 256 + 4 * lane < w.k ? sum_sq4(fx[i]) : 0.0f;   // two lanes = group
+                    t += dpp_f<kQuadSwap1>(t);
+                    t += dpp_f<kQuadSwap2>(t);
+                    t += dpp_f<kHalfMirror>(t);
+                    t += dpp_f<kRowMirror>(t);
+                    const float p = (readlane_f(t, 0) + readlane_f(t, 16)) + (readlane_f(t, 32) + readlane_f(t, 48));
+                    if (lane == 0) lds_put<float>(smem, red + 4 * (kSlots * m + c), c < chunks ? p : 0.0f);
+                }
             }
         }
         if constexpr (!kPairs) {
             __syncthreads();
-            const float scale = row_scale();
+            const float scale = row_scale(0);
 #pragma unroll
             for (int i = 0; i < XCH; i++) fx[i] = rms_scale4(fx[i], scale, gx[i]);
         }
@@ -891,11 +895,15 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
         }
         __syncthreads();
     }
-    float yscale = 1.0f;
-    bool yscale_ok = true;   // (a NaN, infinite or zero scale: the reference's normalised row quantizes to zero blocks)
+    float yscale[MB];
+    bool yscale_ok[MB];   // (a NaN, infinite or zero scale: the reference's normalised row quantizes to zero blocks)
     if constexpr (kRms && kPairs) {
-        yscale = row_scale();
-        yscale_ok = yscale > 0.0f && yscale < __builtin_inff();
+        const float mine = row_scale(MB == 1 ? 0 : lane % MB);   // (each lane one row's: a chain of additions, a root and two divisions)
+#pragma unroll
+        for (int m = 0; m < MB; m++) {
+            yscale[m] = MB == 1 ? mine : readlane_f(mine, m);
+            yscale_ok[m] = yscale[m] > 0.0f && yscale[m] < __builtin_inff();
+        }
     }
     auto put = [&](int64_t row, Sums<MB> v, const OffsetRow<DT> &o) {
         RowPtr p;
@@ -905,7 +913,7 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
 #pragma unroll
         for (int m = 0; m < MB; m++) {
             float t = v.v[m];
-            if constexpr (kRms && kPairs) t = yscale_ok ? t * yscale : 0.0f;
+            if constexpr (kRms && kPairs) t = yscale_ok[m] ? t * yscale[m] : 0.0f;
             if constexpr (kOffsets) {
                 t += offset_term<DT>(smem, rm[m], w, o);   // the f32 addition the workspace path's second launch makes
             }
@@ -1290,7 +1298,7 @@ hipError_t launch_fused_upl(const cq_weight *w, int64_t n, FusedMore<NWT> more, 
                             hipStream_t s) {
     constexpr int NW = 8;
     constexpr int kXch = (UPL * Geo<DT>::kElems / (Geo<DT>::kActK ? 8 : 4) + NW - 1) / NW;   // as in the kernel
-    const size_t lds = PRE == CQ_PRE_RMS_NORM ? fused_red_offset<DT>(w->k) + 4 * (size_t)((Geo<DT>::kActK ? 2 : 1) * kXch * NW)
+    const size_t lds = PRE == CQ_PRE_RMS_NORM ? fused_red_offset<DT>(w->k, MB) + 4 * (size_t)((Geo<DT>::kActK ? 2 : 1) * kXch * NW) * MB
                                               : lds_row_bytes<DT>(w->k) * MB;
     // every workgroup quantizes the whole activation row, so fewer, longer-lived workgroups win: one
     // per CU measured faster than two on every decode shape (11008 x 4096 Q4K: 7.0 us against 7.6 us)
@@ -1503,8 +1511,11 @@ hipError_t launch_fused_rows(const cq_weight *w, const float *x, int64_t m, floa
     return launch_fused_rows_mb<DT, 4>(w, x, y, s);
 }
 
+// Elements of a row per lane up to which the one-launch kernel takes m activation rows.
+constexpr int rows_lane_limit(int m) { return m >= 4 ? 64 : m == 3 ? 128 : 256; }
+
 // Two or three weights on the same activations (same type, row length and device; rows of at most 256
-// units): one launch over all their rows.
+// units): one launch over all their rows.  (One weight with rms_norm in front of several rows takes the same instances.)
 constexpr int kMultiMax = 3;
 template <int DT, int PRE, int MB = 1>
 hipError_t launch_fused_multi_pre(const cq_weight *const *ws, int count, const float *x, cq_pre pre, float *const *ys,
@@ -1522,14 +1533,32 @@ hipError_t launch_fused_multi_pre(const cq_weight *const *ws, int count, const f
     // (a slot that repeats the last weight starts at the end of the launch: no row reaches it)
     const cq_weight *w = ws[0];
     const int upl = (int)((w->k / Geo<DT>::kElems + 63) / 64);
-    if (upl <= 1) return launch_fused_upl<DT, 1, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
-    if (upl <= 2) return launch_fused_upl<DT, 2, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
-    if (upl <= 3) return launch_fused_upl<DT, 3, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
-    return launch_fused_upl<DT, 4, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
+    if constexpr (PRE == CQ_PRE_RMS_NORM && MB > 1) {   // (no instances of what rows_lane_limit refuses)
+        constexpr int most = rows_lane_limit(MB) / Geo<DT>::kElems < 4 ? rows_lane_limit(MB) / Geo<DT>::kElems : 4;
+        if (upl > most) return hipErrorInvalidConfiguration;
+        if (upl <= 1) return launch_fused_upl<DT, 1, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
+        if constexpr (most >= 2) { if (upl <= 2) return launch_fused_upl<DT, 2, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s); }
+        if constexpr (most >= 3) { if (upl <= 3) return launch_fused_upl<DT, 3, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s); }
+        if constexpr (most >= 4) return launch_fused_upl<DT, 4, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
+        return hipErrorInvalidConfiguration;
+    } else {
+        if (upl <= 1) return launch_fused_upl<DT, 1, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
+        if (upl <= 2) return launch_fused_upl<DT, 2, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
+        if (upl <= 3) return launch_fused_upl<DT, 3, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
+        return launch_fused_upl<DT, 4, PRE, kMultiMax, MB>(w, n, more, x, pre, ys[0], s);
+    }
 }
 template <int DT>
 hipError_t launch_fused_multi(const cq_weight *const *ws, int count, const float *x, cq_pre pre, int64_t m,
                               float *const *ys, hipStream_t s) {
+    if constexpr (Geo<DT>::kActK) {
+        if (pre.kind == CQ_PRE_RMS_NORM && m > 1) {
+            if (m == 2) return launch_fused_multi_pre<DT, CQ_PRE_RMS_NORM, 2>(ws, count, x, pre, ys, s);
+            if (m == 3) return launch_fused_multi_pre<DT, CQ_PRE_RMS_NORM, 3>(ws, count, x, pre, ys, s);
+            return launch_fused_multi_pre<DT, CQ_PRE_RMS_NORM, 4>(ws, count, x, pre, ys, s);
+        }
+    }
+    if (m > 1 && pre.kind != CQ_PRE_NONE) return hipErrorInvalidValue;
     if (m == 2) return launch_fused_multi_pre<DT, CQ_PRE_NONE, 2>(ws, count, x, pre, ys, s);
     if (m == 3) return launch_fused_multi_pre<DT, CQ_PRE_NONE, 3>(ws, count, x, pre, ys, s);
     if (m == 4) return launch_fused_multi_pre<DT, CQ_PRE_NONE, 4>(ws, count, x, pre, ys, s);
@@ -1556,42 +1585,83 @@ hipError_t launch_fused_multi(const cq_weight *const *ws, int count, const float
 // launch / split K, at 2, 3, 4 rows): Q4K 24576 x 2048 11.7/12.5, 14.6/12.6, 16.9/12.9; 8192 x 1024 5.7/6.6, 7.1/6.7, 8.4/6.8; 8192 x 1536
 // 7.3/7.2, 8.8/7.2, 12.0/7.3; 8192 x 768 7.2/6.3, 10.4/6.4, 13.9/6.5; Q6K 32000 x 4096 21.3/28.7, 27.2/29.2, 31.0/29.2;
 // Q4_0 16384 x 1024 6.2/8.4, 7.2/8.4, 8.7/8.4; 24576 x 3072 12.8/17.7, 15.8/17.9, 18.8/17.5.  Longer rows, and Q8_0: one launch.
-static bool rows_to_split_k(const cq_weight *w, int64_t m) {
-    if (w->k > 4096 || w->dtype == CQ_DTYPE_Q8_0) return false;
-    const double rows = (double)w->n / 1000.0, mb = (double)w->n * (double)(w->k / 256) * (double)(cq_type_size(w->dtype) * 256 / cq_block_size(w->dtype)) / 1e6;
-    const bool two_passes = w->k > (w->dtype == CQ_DTYPE_Q4K || w->dtype == CQ_DTYPE_Q5K ? 4096 : 2048);
-    if (w->dtype == CQ_DTYPE_Q4_0) {
-        static constexpr double per_row[2][3] = {{0.245, 0.30, 0.36}, {0.405, 0.50, 0.60}};
-        const double split = 4.6 + 0.09 * rows + 0.20 * mb;
-        return 2.1 + per_row[two_passes][m - 2] * rows > (split > 6.3 ? split : 6.3);
-    }
+static double weight_mb(const cq_weight *w) { return (double)w->n * (double)(w->k / 256) * (double)(cq_type_size(w->dtype) * 256 / cq_block_size(w->dtype)) / 1e6; }
+// The one launch's estimate for K-quant rows of up to 4096 elements (infinity where the rows collide too much in LDS).
+static double one_launch_us(const cq_weight *w, int64_t m) {
     static constexpr double per_row[3][3][3] = {{{0.36, 0.45, 0.54}, {0.56, 0.69, 1.06}, {0.56, 0.96, 1.40}},     // Q4K; Q5K 0.05 more
                                                 {{0.35, 0.41, 0.47}, {0.40, 0.46, 0.60}, {0.40, 0.575, 0.76}},    // Q6K
                                                 {{0.54, 0.705, 0.84}, {0.67, 0.85, 1.155}, {0.68, 1.03, 1.45}}};  // Q6K, two passes
-    const bool q6k = w->dtype == CQ_DTYPE_Q6K, q5k = w->dtype == CQ_DTYPE_Q5K;
+    const bool q6k = w->dtype == CQ_DTYPE_Q6K, two_passes = w->k > (q6k ? 2048 : 4096);
     const int collide = w->k % 1024 == 0 ? 0 : w->k % 512 == 0 ? 1 : 2;
-    if (m == 4 && collide >= (q6k && !two_passes ? 2 : 1)) return true;
-    const double one = 1.5 + 0.6 * (double)m + (per_row[q6k ? 1 + two_passes : 0][collide][m - 2] + (q5k ? 0.05 : 0.0)) * rows;
-    const double split = 5.4 + 0.05 * rows + (q5k ? 0.26 : 0.22) * mb;
-    return one > (split > 6.5 ? split : 6.5);
+    if (m == 4 && collide >= (q6k && !two_passes ? 2 : 1)) return __builtin_inf();
+    return 1.5 + 0.6 * (double)m + (per_row[q6k ? 1 + two_passes : 0][collide][m - 2] + (w->dtype == CQ_DTYPE_Q5K ? 0.05 : 0.0)) * ((double)w->n / 1000.0);
 }
-bool cq_matvec_fused_rows_supported(const cq_weight *w, int64_t m) {
-    if (m < 2 || m > 4 || !cq_matvec_fused_supported(w)) return false;
-    int64_t units = 0, elems = 0;
-    size_t row_bytes = 0;
-    switch (w->dtype) {
-    case CQ_DTYPE_Q4_0: elems = Geo<CQ_DTYPE_Q4_0>::kElems; row_bytes = lds_row_bytes<CQ_DTYPE_Q4_0>(w->k); break;
-    case CQ_DTYPE_Q8_0: elems = Geo<CQ_DTYPE_Q8_0>::kElems; row_bytes = lds_row_bytes<CQ_DTYPE_Q8_0>(w->k); break;
-    case CQ_DTYPE_Q4K: elems = Geo<CQ_DTYPE_Q4K>::kElems; row_bytes = lds_row_bytes<CQ_DTYPE_Q4K>(w->k); break;
-    case CQ_DTYPE_Q5K: elems = Geo<CQ_DTYPE_Q5K>::kElems; row_bytes = lds_row_bytes<CQ_DTYPE_Q5K>(w->k); break;
-    case CQ_DTYPE_Q6K: elems = Geo<CQ_DTYPE_Q6K>::kElems; row_bytes = lds_row_bytes<CQ_DTYPE_Q6K>(w->k); break;
-    default: return false;
+static bool rows_to_split_k(const cq_weight *w, int64_t m) {
+    if (w->k > 4096 || w->dtype == CQ_DTYPE_Q8_0) return false;
+    const double rows = (double)w->n / 1000.0, mb = weight_mb(w);
+    if (w->dtype == CQ_DTYPE_Q4_0) {
+        static constexpr double per_row[2][3] = {{0.245, 0.30, 0.36}, {0.405, 0.50, 0.60}};
+        const bool two_passes = w->k > 2048;
+        const double split = 4.6 + 0.09 * rows + 0.20 * mb;
+        return 2.1 + per_row[two_passes][m - 2] * rows > (split > 6.3 ? split : 6.3);
     }
-    units = w->k / elems;
+    const double split = 5.4 + 0.05 * rows + (w->dtype == CQ_DTYPE_Q5K ? 0.26 : 0.22) * mb;
+    return one_launch_us(w, m) > (split > 6.5 ? split : 6.5);
+}
+static int64_t unit_elems(int dtype) {   // (of the types the one-launch kernels take)
+    switch (dtype) {
+    case CQ_DTYPE_Q8_0: return Geo<CQ_DTYPE_Q8_0>::kElems;
+    case CQ_DTYPE_Q4_0: return Geo<CQ_DTYPE_Q4_0>::kElems;
+    case CQ_DTYPE_Q6K: return Geo<CQ_DTYPE_Q6K>::kElems;
+    default: return Geo<CQ_DTYPE_Q4K>::kElems;
+    }
+}
+static size_t fused_row_bytes(const cq_weight *w) {
+    switch (w->dtype) {
+    case CQ_DTYPE_Q4_0: return lds_row_bytes<CQ_DTYPE_Q4_0>(w->k);
+    case CQ_DTYPE_Q8_0: return lds_row_bytes<CQ_DTYPE_Q8_0>(w->k);
+    case CQ_DTYPE_Q4K: return lds_row_bytes<CQ_DTYPE_Q4K>(w->k);
+    case CQ_DTYPE_Q5K: return lds_row_bytes<CQ_DTYPE_Q5K>(w->k);
+    default: return lds_row_bytes<CQ_DTYPE_Q6K>(w->k);
+    }
+}
+// The shapes that the one-launch kernel takes with m activation rows, whichever is faster.
+static bool rows_fit_one_launch(const cq_weight *w, int64_t m) {
+    if (m < 2 || m > 4 || !cq_matvec_fused_supported(w)) return false;
+    const int64_t elems = unit_elems(w->dtype), units = w->k / elems;
+    const size_t row_bytes = fused_row_bytes(w);
     if (units > (m == 2 ? 384 : 256) || row_bytes * (size_t)m > 64 * 1024 - 1024) return false;
-    if (rows_to_split_k(w, m)) return false;
     const int64_t per_lane = (units + 63) / 64 * elems;   // elements of a row per lane
-    return per_lane <= 64 ? true : per_lane <= 128 ? m <= 3 : m <= 2;
+    return per_lane <= rows_lane_limit((int)m);
+}
+bool cq_matvec_fused_rows_supported(const cq_weight *w, int64_t m) { return rows_fit_one_launch(w, m) && !rows_to_split_k(w, m); }
+
+// rms_norm in front of two to four rows of `count` weights (one to three): the prologue of the one launch does it, a launch of
+// the quantizer saved.  (K-quants only: with the 32-element types a row's bits are the ones of the quantizer and the kernel behind it.)
+// It costs the one launch a few hundred instructions (four rows of 4096 elements about 1.5 us) and the quantizer, one dependent chain over the
+// row, 0.2 us for every block of it: the sums above with these terms, fitted to 450 shapes (three types, 1024..32000 weight rows, K 512..8192,
+// weights from HBM).  With the 3 % in favour of the two launches the choice is 0.6 % behind the better one on average, 9 % at worst, and
+// 8 % ahead of two launches throughout.  Some (us, two launches / one): Q4K 4096 x 4096 at two rows 9.1/6.0, three 9.2/7.3, four 9.3/8.7; 32000 x
+// 4096 26.8/22.6, 26.4/24.9, 26.3/28.0; 8192 x 512 6.8/8.5; Q6K 32000 x 2048 19.8/18.4, 20.6/22.4; Q5K 4096 x 4096 10.4/6.5, 10.5/7.8, 10.5/9.6.
+bool cq_matvec_fused_rms_rows_supported(const cq_weight *const *ws, int count, int64_t m) {
+    if (count < 1 || count > kMultiMax || cq_has_min16(ws[0]->ggml_dtype) || ws[0]->dtype == CQ_DTYPE_Q8_0 || ws[0]->dtype == CQ_DTYPE_Q4_0) return false;
+    cq_weight all = *ws[0];
+    for (int i = 0; i < count; i++) {
+        if (ws[i]->n == 0 || !cq_matvec_fused_supported(ws[i]) || ws[i]->k / unit_elems(ws[i]->dtype) > 256) return false;
+        if (i) all.n += ws[i]->n;
+    }
+    if (!rows_fit_one_launch(&all, m)) return false;
+    const double rows = (double)all.n / 1000.0, more = (double)(m - 2);
+    double one;
+    if (all.k <= 4096) {
+        one = one_launch_us(&all, m) + 0.4 + 0.48 * (double)m + 0.09 * rows;
+    } else {   // (by the elements of a row per lane: whole passes of the wave)
+        const int64_t pass = 64 * unit_elems(all.dtype);
+        const double lane = (double)((all.k + pass - 1) / pass * unit_elems(all.dtype));
+        const double per_row = all.dtype == CQ_DTYPE_Q6K ? 0.0088 : all.dtype == CQ_DTYPE_Q5K ? 0.0079 : 0.0065;
+        one = 0.9 + 0.048 * lane + 0.85 * lane / 64.0 * more + (per_row * lane + 0.15 * more) * rows;
+    }
+    return 1.03 * one + 0.15 < 4.7 + 0.14 * rows + 0.196 * weight_mb(&all) + 0.2 * (double)(all.k / 256);
 }
 
 hipError_t cq_launch_matvec_fused_rows(const cq_weight *w, const float *x, int64_t m, float *y, hipStream_t s) {
@@ -1608,21 +1678,12 @@ hipError_t cq_launch_matvec_fused_rows(const cq_weight *w, const float *x, int64
 
 bool cq_matvec_fused_multi_supported(const cq_weight *const *ws, int count, int pre_kind, int64_t m) {
     if (count < 2 || count > kMultiMax || (pre_kind != CQ_PRE_NONE && pre_kind != CQ_PRE_RMS_NORM)) return false;
-    if (m != 1 && (pre_kind != CQ_PRE_NONE || !cq_matvec_fused_rows_supported(ws[0], m))) return false;
+    if (m != 1 && !(pre_kind == CQ_PRE_NONE ? cq_matvec_fused_rows_supported(ws[0], m) : cq_matvec_fused_rms_rows_supported(ws, count, m))) return false;
     for (int i = 0; i < count; i++) {
         if (ws[i]->dtype != ws[0]->dtype || ws[i]->k != ws[0]->k || ws[i]->dev != ws[0]->dev || ws[i]->n == 0) return false;
         if (!cq_matvec_fused_supported(ws[i])) return false;
     }
-    int64_t units = 0;
-    switch (ws[0]->dtype) {
-    case CQ_DTYPE_Q4_0: units = ws[0]->k / Geo<CQ_DTYPE_Q4_0>::kElems; break;
-    case CQ_DTYPE_Q8_0: units = ws[0]->k / Geo<CQ_DTYPE_Q8_0>::kElems; break;
-    case CQ_DTYPE_Q4K: units = ws[0]->k / Geo<CQ_DTYPE_Q4K>::kElems; break;
-    case CQ_DTYPE_Q5K: units = ws[0]->k / Geo<CQ_DTYPE_Q5K>::kElems; break;
-    case CQ_DTYPE_Q6K: units = ws[0]->k / Geo<CQ_DTYPE_Q6K>::kElems; break;
-    default: return false;
-    }
-    return units <= 256;
+    return ws[0]->k / unit_elems(ws[0]->dtype) <= 256;
 }
 
 hipError_t cq_launch_matvec_fused_multi(const cq_weight *const *ws, int count, const float *x, cq_pre pre, int64_t m,

@@ -1,0 +1,50 @@
+"""rms_norm in front of two to four rows in the one-launch decode kernel: a row's bits are those of its own one-row call (the same
+sums in the same order), for one weight and for several, at one to four passes of a wave over the row, full and partly filled."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+from oracle import cpu_oracle as orc  # noqa: E402  (checker only)
+from test_gpu_parity import check_f32, dev, make_inputs  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def qh():
+    from candle_amd import qhip
+    qhip.load()
+    assert qhip.load().cq_device_count() >= 1, "no HIP device visible"
+    return qhip
+
+
+@pytest.mark.parametrize("dt,m,k", [
+    (orc.Q4K, 2, 256), (orc.Q4K, 3, 3840), (orc.Q4K, 4, 4096), (orc.Q4K, 2, 4352), (orc.Q4K, 3, 8192), (orc.Q4K, 2, 16384),
+    (orc.Q5K, 4, 4096), (orc.Q5K, 2, 12032), (orc.Q6K, 2, 512), (orc.Q6K, 4, 3072), (orc.Q6K, 4, 4096), (orc.Q6K, 3, 5888),
+    (orc.Q6K, 3, 8192), (orc.Q3K, 2, 1024), (orc.Q3K, 4, 4096)])
+@pytest.mark.parametrize("ns", [(8,), (77,), (9, 40, 131), (300, 16)])
+def test_rows_equal_their_one_row_calls(qh, dt, m, k, ns):
+    rng = np.random.default_rng(k + m + len(ns))
+    x = rng.standard_normal((m, k)).astype(np.float32) * np.float32([[1e-3], [7.0], [1.0], [300.0]])[:m]
+    alpha = rng.standard_normal(k).astype(np.float32)
+    blocks = [orc.quantize(dt, make_inputs(k + i, 1, k, n)[0]) for i, n in enumerate(ns)]
+    ws = [qh.QWeight.from_ggml(dt, b, n, k) for b, n in zip(blocks, ns)]
+    xd, ad = dev(x), dev(alpha)
+    kw = dict(pre=qh.PRE_RMS_NORM, aux=ad, eps=1e-5)
+    outs = qh.qmatmul_multi(ws, xd, **kw) if len(ws) > 1 else [qh.qmatmul(ws[0], xd, **kw)]
+    for w, b, y in zip(ws, blocks, outs):
+        for r in range(m):
+            assert torch.equal(y[r:r + 1], qh.qmatmul(w, xd[r:r + 1].contiguous(), **kw))
+        check_f32(y.cpu().numpy(), orc.matmul(dt, orc.rms_norm(x, alpha, 1e-5), b, w.shape[0]))
+
+
+def test_a_reused_workspace_follows_more_than_three_weights(qh):
+    """Four weights: no launch over all of them, so the first call leaves its rows in the workspace for the others."""
+    k, m = 1024, 2
+    rng = np.random.default_rng(3)
+    x, alpha = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal(k).astype(np.float32)
+    blocks = [orc.quantize(orc.Q4K, make_inputs(i, 1, k, 48)[0]) for i in range(4)]
+    ws = [qh.QWeight.from_ggml(orc.Q4K, b, 48, k) for b in blocks]
+    for b, y in zip(blocks, qh.qmatmul_multi(ws, dev(x), pre=qh.PRE_RMS_NORM, aux=dev(alpha), eps=1e-5)):
+        check_f32(y.cpu().numpy(), orc.matmul(orc.Q4K, orc.rms_norm(x, alpha, 1e-5), b, 48))
