@@ -578,7 +578,7 @@ __device__ __forceinline__ float unit_value(const uint8_t *smem, const UnitW<DT>
 // subtracts sum_b (d8_b * dmin_b) * sum_j bsums_j * m_j: the sums of the kernels in min_term.hip, formed from the
 // quantized row in LDS with the same operations in the same order (chunk and block sums per lane, added lane after
 // lane), so that the one-launch decode gives the bits of the launches that go through the workspace.  Called by whole
-// waves; `lr` = the weight row.  Returns the value to add to the row's result.
+// waves; `lr` = the weight row.
 // The rows of the one-launch kernels have at most 16 384 elements: one lane per group of eight 32-element blocks
 // (Q4_1 / Q5_1, whole groups only) or per 256-element block (Q2K) covers a row, so the weight side of a row's term
 // is one unconditional request per lane, made together with the row's units (a request behind a branch or in a loop
@@ -598,33 +598,51 @@ template <int DT> __device__ __forceinline__ void offset_load(const cq_weight &w
         o.dmin = ((const uint16_t *)ws.p5)[lr * kb + b];
     }
 }
+// The lane's part of an activation row's term: eight blocks (Q4_1 / Q5_1) or one (Q2K); zero in the lanes past the row.
+template <int DT> __device__ __forceinline__ uint32_t offset_lanes(int64_t k) { return (uint32_t)(k / 256); }
 template <int DT>
-__device__ __forceinline__ float offset_term(const uint8_t *smem, const LdsRow r, const cq_weight &ws, const OffsetRow<DT> &o) {
-    const uint32_t lane = threadIdx.x & 63;
+__device__ __forceinline__ float offset_part(const uint8_t *smem, const LdsRow r, const cq_weight &ws, const OffsetRow<DT> &o) {
+    const uint32_t lane = threadIdx.x & 63, lanes = offset_lanes<DT>(ws.k), at = lane < lanes ? lane : lanes - 1;
     const uint32_t mw[4] = {o.mw.x, o.mw.y, o.mw.z, o.mw.w};
-    float acc = 0.0f;
     if constexpr (DT == CQ_DTYPE_Q8_0) {
-        const uint32_t nb = (uint32_t)(ws.k / 32), b = lane * 8, bc = b < nb ? b : nb - 8;
         // the blocks' scaled sums, left in place of the integer sums by the kernel's prologue
-        const float4 s0 = lds_get<float4>(smem, r.bs + 4 * bc), s1 = lds_get<float4>(smem, r.bs + 4 * bc + 16);
+        const float4 s0 = lds_get<float4>(smem, r.bs + 32 * at), s1 = lds_get<float4>(smem, r.bs + 32 * at + 16);
         const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
         float t = 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; i++) t += cq_h2f((uint16_t)(mw[i >> 1] >> (16 * (i & 1)))) * sv[i];
-        t = b < nb ? t : 0.0f;
-        for (uint32_t jj = 0; jj * 8 < nb; jj++) acc += readlane_f(t, jj);
-        return acc;
+        return lane < lanes ? t : 0.0f;
     } else {
-        const uint32_t kb = (uint32_t)(ws.k / 256), b = lane < kb ? lane : kb - 1;
+        typedef short v2s __attribute__((ext_vector_type(2)));
         int summs = 0;
 #pragma unroll
-        for (int g = 0; g < 16; g++)
-            summs += (int)lds_get<int16_t>(smem, r.bs + 32 * b + 2 * g) * (int)((mw[g >> 2] >> (8 * (g & 3))) & 0xff);
-        float term = (lds_get<float>(smem, r.d + 4 * b) * cq_h2f(o.dmin)) * (float)summs;
-        term = lane < kb ? term : 0.0f;
-        for (uint32_t jj = 0; jj < kb; jj++) acc += readlane_f(term, jj);
-        return -acc;
+        for (int g = 0; g < 8; g++) {   // two groups: their sums are neighbours, their minima bytes of one word
+            const uint32_t two = __builtin_amdgcn_perm(mw[g >> 1], mw[g >> 1], g & 1 ? 0x0c030c02u : 0x0c010c00u);
+            summs = __builtin_amdgcn_sdot2(__builtin_bit_cast(v2s, lds_get<uint32_t>(smem, r.bs + 32 * at + 4 * g)), __builtin_bit_cast(v2s, two), summs, false);
+        }
+        const float term = (lds_get<float>(smem, r.d + 4 * at) * cq_h2f(o.dmin)) * (float)summs;
+        return lane < lanes ? -term : 0.0f;
     }
+}
+// v[0] + v[1] + ... of the first `lanes` lanes, added one lane after the other, for MB values a lane.  A step adds every lane's own value to what
+// its left neighbour has: after j steps the lanes up to j hold the sum up to themselves and keep it, so that steps beyond the last
+// lane change nothing.  Bound by the instructions; before, a read of every lane into a scalar register and an addition behind it, four to six
+// instructions a lane and activation row.  With Q2K's group sums two at a time, whole calls, weights from HBM, us: Q4_1 32000 x 4096 at 2 / 3 /
+// 4 rows 36.9 / 47.1 / 54.1 -> 31.2 / 34.3 / 39.0, 4096 x 4096 8.3 / 10.1 / 12.0 -> 7.6 / 8.4 / 9.7, one row 6.6 -> 6.1; Q2K 32000 x 4096
+// 42.1 / 52.8 / 65.5 -> 31.3 / 36.2 / 42.3, 4096 x 4096 8.7 / 10.7 / 12.8 -> 7.4 / 8.7 / 10.1, one row 7.1 -> 6.1.
+constexpr int kWaveShr1 = 0x138;
+template <int MB> __device__ __forceinline__ void sums_in_lane_order(float (&v)[MB], uint32_t lanes) {
+    float a[MB];
+#pragma unroll
+    for (int m = 0; m < MB; m++) a[m] = v[m];
+    for (uint32_t j = 1; j < lanes; j += 8) {
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int m = 0; m < MB; m++) a[m] = dpp_f<kWaveShr1>(a[m]) + v[m];
+    }
+#pragma unroll
+    for (int m = 0; m < MB; m++) v[m] = readlane_f(a[m], lanes - 1);
 }
 
 // --------------------------------------------------------------------- fused kernel (m = 1) ----
@@ -910,13 +928,17 @@ __global__ void __launch_bounds__(NW * 64) fused_kernel(cq_weight w, const float
         float *ys;
         int64_t n;
         const int64_t lr = pick(row, p, ys, n);
+        float off[MB];   // the f32 additions the workspace path's second launch makes
+        if constexpr (kOffsets) {
+#pragma unroll
+            for (int m = 0; m < MB; m++) off[m] = offset_part<DT>(smem, rm[m], w, o);
+            sums_in_lane_order<MB>(off, offset_lanes<DT>(w.k));
+        }
 #pragma unroll
         for (int m = 0; m < MB; m++) {
             float t = v.v[m];
             if constexpr (kRms && kPairs) t = yscale_ok[m] ? t * yscale[m] : 0.0f;
-            if constexpr (kOffsets) {
-                t += offset_term<DT>(smem, rm[m], w, o);   // the f32 addition the workspace path's second launch makes
-            }
+            if constexpr (kOffsets) t += off[m];
             if (lane == 0) ys[m * n + lr] = t;
         }
     };
