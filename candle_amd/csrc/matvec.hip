@@ -1618,7 +1618,39 @@ static double one_launch_us(const cq_weight *w, int64_t m) {
     if (m == 4 && collide >= (q6k && !two_passes ? 2 : 1)) return __builtin_inf();
     return 1.5 + 0.6 * (double)m + (per_row[q6k ? 1 + two_passes : 0][collide][m - 2] + (w->dtype == CQ_DTYPE_Q5K ? 0.05 : 0.0)) * ((double)w->n / 1000.0);
 }
+static int64_t unit_elems(int dtype) {   // (of the types the one-launch kernels take)
+    switch (dtype) {
+    case CQ_DTYPE_Q8_0: return Geo<CQ_DTYPE_Q8_0>::kElems;
+    case CQ_DTYPE_Q4_0: return Geo<CQ_DTYPE_Q4_0>::kElems;
+    case CQ_DTYPE_Q6K: return Geo<CQ_DTYPE_Q6K>::kElems;
+    default: return Geo<CQ_DTYPE_Q4K>::kElems;
+    }
+}
+static int64_t elems_per_lane(const cq_weight *w) {   // (in whole passes of a wave over the row)
+    const int64_t elems = unit_elems(w->dtype);
+    return (w->k / elems + 63) / 64 * elems;
+}
+// The same choice for Q4_1 / Q5_1 and Q2K, whose offset term costs the one launch about as much as the row itself: by the elements of a row per
+// lane, nearly level up to 4096 weight rows (two a wave, in flight together).  Fitted to 371 shapes (256..32000 weight rows, K 512..8192,
+// weights from HBM); 12 % in favour of the one launch, whose rows have the bits of their own one-row calls, the choice is 1 % behind
+// the better one on average, the one launch throughout 10 %.  Some (us, one launch / split K, at 2, 3, 4 rows): Q2K 32000 x 2048
+// 19.9/21.2, 24.1/20.9, 28.7/21.1, 8192 x 1024 6.9/7.3, 8.5/7.4, 10.1/7.5, two rows of 4096 x 11008 24.3/15.7 (its registers spill);
+// Q4_1 32000 x 1024 14.7/16.0, 16.3/16.3, 20.1/16.5, 32000 x 4096 31.2/37.4, 34.3/37.7, 39.0/38.4.
+static bool offset_rows_to_split_k(const cq_weight *w, int64_t m) {
+    const double lane = (double)elems_per_lane(w), rows = (double)w->n / 1000.0, few = rows < 4.1 ? rows : 4.1, many = rows - few, md = (double)m;
+    const double mb = (double)w->n * (double)w->k * 1e-6, blocks = (double)(w->k / 256);
+    if (cq_has_min16(w->ggml_dtype)) {
+        if (lane > 128) return w->n > 1024;   // (few weight rows keep the bits)
+        const int collide = w->k % 1024 == 0 ? 0 : w->k % 512 == 0 ? 1 : 2;
+        const double one = 2.5 + 1.13 * md + (lane > 32 ? 0.4 + 0.0138 * (lane - 32) * md : 0.0) + (0.1 + 0.0085 * (lane - 32)) * few +
+                           (0.2 + 0.0092 * lane + (0.12 + 0.065 * collide) * (md - 2)) * many;
+        return one > 1.12 * (5.0 + 0.125 * rows + 0.171 * mb + 0.131 * blocks);
+    }
+    const double one = 2.0 + 0.9 * md + 0.0095 * (lane - 16) * md + (0.06 + 0.0115 * (lane - 16)) * few + (0.2 + 0.0102 * lane + 0.06 * (md - 2)) * many;
+    return one > 1.12 * (5.1 + 0.118 * rows + 0.2 * mb + 0.122 * blocks);
+}
 static bool rows_to_split_k(const cq_weight *w, int64_t m) {
+    if (cq_has_min32(w->ggml_dtype) || cq_has_min16(w->ggml_dtype)) return offset_rows_to_split_k(w, m);
     if (w->k > 4096 || w->dtype == CQ_DTYPE_Q8_0) return false;
     const double rows = (double)w->n / 1000.0, mb = weight_mb(w);
     if (w->dtype == CQ_DTYPE_Q4_0) {
@@ -1629,14 +1661,6 @@ static bool rows_to_split_k(const cq_weight *w, int64_t m) {
     }
     const double split = 5.4 + 0.05 * rows + (w->dtype == CQ_DTYPE_Q5K ? 0.26 : 0.22) * mb;
     return one_launch_us(w, m) > (split > 6.5 ? split : 6.5);
-}
-static int64_t unit_elems(int dtype) {   // (of the types the one-launch kernels take)
-    switch (dtype) {
-    case CQ_DTYPE_Q8_0: return Geo<CQ_DTYPE_Q8_0>::kElems;
-    case CQ_DTYPE_Q4_0: return Geo<CQ_DTYPE_Q4_0>::kElems;
-    case CQ_DTYPE_Q6K: return Geo<CQ_DTYPE_Q6K>::kElems;
-    default: return Geo<CQ_DTYPE_Q4K>::kElems;
-    }
 }
 static size_t fused_row_bytes(const cq_weight *w) {
     switch (w->dtype) {
@@ -1650,11 +1674,10 @@ static size_t fused_row_bytes(const cq_weight *w) {
 // The shapes that the one-launch kernel takes with m activation rows, whichever is faster.
 static bool rows_fit_one_launch(const cq_weight *w, int64_t m) {
     if (m < 2 || m > 4 || !cq_matvec_fused_supported(w)) return false;
-    const int64_t elems = unit_elems(w->dtype), units = w->k / elems;
+    const int64_t units = w->k / unit_elems(w->dtype);
     const size_t row_bytes = fused_row_bytes(w);
     if (units > (m == 2 ? 384 : 256) || row_bytes * (size_t)m > 64 * 1024 - 1024) return false;
-    const int64_t per_lane = (units + 63) / 64 * elems;   // elements of a row per lane
-    return per_lane <= rows_lane_limit((int)m);
+    return elems_per_lane(w) <= rows_lane_limit((int)m);
 }
 bool cq_matvec_fused_rows_supported(const cq_weight *w, int64_t m) { return rows_fit_one_launch(w, m) && !rows_to_split_k(w, m); }
 
@@ -1678,8 +1701,7 @@ bool cq_matvec_fused_rms_rows_supported(const cq_weight *const *ws, int count, i
     if (all.k <= 4096) {
         one = one_launch_us(&all, m) + 0.4 + 0.48 * (double)m + 0.09 * rows;
     } else {   // (by the elements of a row per lane: whole passes of the wave)
-        const int64_t pass = 64 * unit_elems(all.dtype);
-        const double lane = (double)((all.k + pass - 1) / pass * unit_elems(all.dtype));
+        const double lane = (double)elems_per_lane(&all);
         const double per_row = all.dtype == CQ_DTYPE_Q6K ? 0.0088 : all.dtype == CQ_DTYPE_Q5K ? 0.0079 : 0.0065;
         one = 0.9 + 0.048 * lane + 0.85 * lane / 64.0 * more + (per_row * lane + 0.15 * more) * rows;
     }
