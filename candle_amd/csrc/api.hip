@@ -612,7 +612,7 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     enum { kSkinny, kGemm32, kGemm, kMatvec } path;
     // Few rows: split K over the waves instead of tiling rows.  Measured (weights from HBM, 4096..32000 weight rows,
     // k 4096..14336) faster than the dot-product kernels from 2 rows on and than the tile kernels
-    //   up to 16 rows everywhere; up to 24 rows below 14336 weight rows; up to 32 rows below 12288 weight rows;
+    //   up to 16 rows everywhere; up to 32 rows where two fitted sums say so (cq_skinny_few_ahead);
     //   up to 64 rows where n is small and k short, so that the tile kernel cannot fill the machine.
     // (the 32-element-block types from 4 rows (Q8_0) or 5 rows (Q4_0) on: below that the one-launch dot-product
     // kernel is as fast or faster, it has no per-block scaling of MFMA results to do - where it takes the rows)
@@ -626,7 +626,9 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     //   The factor keeps the calls whose estimates are too close to tell: over 3500 shapes the choice is slower than the tile kernel by more than
     //   3 % in 0.3 %, and 22 % faster on average.
     const auto groups_ahead = [&] { return cq_skinny_in_groups(w, m) && 1.2 * cq_skinny_groups_us(w, m) < (has_tile32 ? cq_gemm32_us(w, m) : cq_gemm_us(w, m)); };
-    const bool skinny_rows = m <= 16 || (m <= 24 && w->n < 14336) || (m <= 32 && w->n < 12288) || (m <= 64 && w->n < 8192 && w->k <= 6144) ||
+    const bool k_quant = act == CQ_DTYPE_Q8K && !min32;   // (Q2K: the tile kernels add its offset term in a launch of its own)
+    const bool few_ahead = k_quant && m > 16 && m <= 32 ? cq_skinny_few_ahead(w, m) : (m <= 24 && w->n < 14336) || (m <= 32 && w->n < 12288);
+    const bool skinny_rows = m <= 16 || few_ahead || (m <= 64 && w->n < 8192 && w->k <= 6144) ||
                              (!has_tile32 && groups_ahead());
     if (flags & CQ_FLAG_FORCE_SKINNY) {
         if (!cq_skinny_supported(w, act))
