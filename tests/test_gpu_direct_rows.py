@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-from oracle import cpu_oracle as orc  # noqa: E402  (checker only)
+from oracle import cpu_oracle as orc  # noqa: E402
 from test_gpu_fused_neighbours import qh  # noqa: E402,F401
 from test_gpu_parity import check_f32, dev, make_inputs  # noqa: E402
 
