@@ -617,8 +617,7 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     //   up to 64 rows where n is small and k short, so that the tile kernel cannot fill the machine.
     // (the 32-element-block types from 4 rows (Q8_0) or 5 rows (Q4_0) on: below that the one-launch dot-product
     // kernel is as fast or faster, it has no per-block scaling of MFMA results to do - where it takes the rows)
-    const bool rows_direct = flags == 0 && !in_place && pre.kind == CQ_PRE_NONE && cq_skinny_direct_rows_ahead(w, act, m);
-    const bool rows_fused = flags == 0 && !in_place && ((pre.kind == CQ_PRE_NONE && !rows_direct && cq_matvec_fused_rows_supported(w, m)) ||
+    const bool rows_fused = flags == 0 && !in_place && ((pre.kind == CQ_PRE_NONE && cq_matvec_fused_rows_supported(w, m)) ||
                                                         (pre.kind == CQ_PRE_RMS_NORM && !leave_rows && cq_matvec_fused_rms_rows_supported(&w, 1, m)));
     const int64_t skinny_from = w->dtype == CQ_DTYPE_Q8_0 ? 4 : w->dtype == CQ_DTYPE_Q4_0 ? 5 : 2;
     // (weights of 33 to 127 rows that are no whole number of 32-row tiles stay with the split-K kernel)

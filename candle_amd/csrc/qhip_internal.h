@@ -238,7 +238,6 @@ double cq_skinny_groups_us(const cq_weight *w, int64_t m);
 double cq_gemm_us(const cq_weight *w, int64_t m);
 double cq_gemm32_us(const cq_weight *w, int64_t m);
 // the rows of a small weight in one launch that quantizes them itself (and leaves them in the workspace)
-bool cq_skinny_direct_rows_ahead(const cq_weight *w, int act_dtype, int64_t m);
 bool cq_skinny_few_ahead(const cq_weight *w, int64_t m);
 bool cq_skinny_direct_takes(const cq_weight *w, int act_dtype, int64_t m);
 hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s);

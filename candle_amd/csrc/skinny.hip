@@ -1847,14 +1847,6 @@ bool cq_skinny_direct_takes(const cq_weight *w, int act_dtype, int64_t m) {
     if (m > 8) return act_dtype == CQ_DTYPE_Q8K && groups <= cq_num_cus() && w->k <= 8 * QK_K;
     return m <= (w->dtype == CQ_DTYPE_Q4_0 ? 7 : 8) && w->n <= 4096 && w->k <= (m <= 4 ? 2048 : 1024);
 }
-// Two to four rows of a small K-quant weight that the dot-product kernel would take in one launch as well.  Its rows collide in LDS where their
-// blocks are no multiple of four, most at three and four rows; the kernel above does not.  us from a graph, weights from HBM, dot products /
-// this: Q4K 2048 x 768 at 2 / 3 rows 5.1/3.5, 6.7/3.5, 4096 x 1536 5.4/4.6, 6.6/4.7; Q5K 1024 x 512 4.9/3.7, 6.3/3.8; Q6K 1024 x 768 4.2/3.6, 5.8/3.6, but
-// two rows of 1280 and more 4.3/4.7 (Q5K 5.1/5.1).  Rows of a multiple of 1024 elements stay with the dot products, whose rows have the bits
-// of their own one-row calls (2048 x 1024, Q4K: 4.5/3.6, 5.4/3.7).
-bool cq_skinny_direct_rows_ahead(const cq_weight *w, int act_dtype, int64_t m) {
-    return m <= 4 && act_dtype == CQ_DTYPE_Q8K && w->k % 1024 != 0 && (m > 2 || w->dtype == CQ_DTYPE_Q4K || w->k < 1024) && cq_skinny_direct_takes(w, act_dtype, m);
-}
 hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s) {
     switch (w->dtype) {
     case CQ_DTYPE_Q8_0: return launch_direct<CQ_DTYPE_Q8_0>(w, a, x, m, y, s);
