@@ -756,10 +756,12 @@ extern "C" int cq_qmatmul_multi(const cq_weight *const *ws, int count, int pre, 
         CQ_HIP_CHECK(cq_launch_matvec_fused_multi(ws, count, x_dev, p, m, ys_dev, (hipStream_t)stream));
         return CQ_OK;
     }
-    // otherwise one matmul per weight; with more than one row the rows are quantized once, by the first
+    // otherwise one matmul per weight; with more than one row the rows are quantized once, by the first weight that has rows
     // (two to four rows that the one-launch kernel takes need no quantizer launch to share)
+    int first = 0;
+    while (first < count - 1 && ws[first]->n == 0) first++;
     const bool share = m > 1 && !(flags & CQ_FLAG_REUSE_ACT) &&
-                       !(flags == 0 && pre == CQ_PRE_NONE && cq_matvec_fused_rows_supported(ws[0], m));
+                       !(flags == 0 && pre == CQ_PRE_NONE && cq_matvec_fused_rows_supported(ws[first], m));
     // up to 16 rows: the quantizer launch and one split-K launch over all the weights' rows
     const int act = cq_vec_dot_type(ws[0]->dtype);
     if (share && flags == 0 && cq_skinny_shared_takes(ws, count, m, act)) {
@@ -780,7 +782,7 @@ extern "C" int cq_qmatmul_multi(const cq_weight *const *ws, int count, int pre, 
         return CQ_OK;
     }
     for (int i = 0; i < count; i++) {
-        const bool reuse = share && i > 0;
+        const bool reuse = share && i > first;
         if (int rc = qmatmul_impl(ws[i], x_dev, reuse ? cq_no_pre() : p, m, ys_dev[i], (reuse ? flags | CQ_FLAG_REUSE_ACT : flags) | det,
                                   workspace, ws_bytes, stream, share && count > 1))
             return rc;
