@@ -751,6 +751,9 @@ extern "C" int cq_qmatmul_multi(const cq_weight *const *ws, int count, int pre, 
         if ((uintptr_t)x_dev & 15) return cq_set_error(CQ_ERR_INVALID, "x must be 16-byte aligned");
         for (int i = 0; i < count; i++)
             if (!ys_dev[i]) return cq_set_error(CQ_ERR_INVALID, "null argument");
+        // (several rows behind rms_norm went through the workspace before they fitted this launch: it is asked for as then)
+        for (int i = 0; i < count && m > 1 && pre == CQ_PRE_RMS_NORM; i++)
+            if (int rc = check_matmul_args(ws[i], x_dev, m, ys_dev[i], workspace, ws_bytes, cq_workspace_bytes(ws[i], m, flags))) return rc;
         if (int rc = check_pre(p)) return rc;
         CQ_HIP_CHECK(hipSetDevice(ws[0]->dev));
         CQ_HIP_CHECK(cq_launch_matvec_fused_multi(ws, count, x_dev, p, m, ys_dev, (hipStream_t)stream));

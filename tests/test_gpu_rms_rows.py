@@ -1,5 +1,7 @@
 """rms_norm in front of two to four rows in the one-launch decode kernel: a row's bits are those of its own one-row call (the same
 sums in the same order), for one weight and for several, at one to four passes of a wave over the row, full and partly filled."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -48,3 +50,19 @@ def test_a_reused_workspace_follows_more_than_three_weights(qh):
     ws = [qh.QWeight.from_ggml(orc.Q4K, b, 48, k) for b in blocks]
     for b, y in zip(blocks, qh.qmatmul_multi(ws, dev(x), pre=qh.PRE_RMS_NORM, aux=dev(alpha), eps=1e-5)):
         check_f32(y.cpu().numpy(), orc.matmul(orc.Q4K, orc.rms_norm(x, alpha, 1e-5), b, 48))
+
+
+@pytest.mark.parametrize("m", [2, 3, 4])
+def test_the_workspace_is_asked_for(qh, m):
+    """Several weights behind rms_norm in one launch: a missing or short workspace is refused, as where the rows go through it."""
+    k = 1024
+    w = qh.QWeight.from_ggml(orc.Q4K, orc.quantize(orc.Q4K, make_inputs(m, 1, k, 48)[0]), 48, k)
+    L, x, alpha = qh.load(), dev(np.ones((m, k), np.float32)), dev(np.ones(k, np.float32))
+    ys = [torch.full((m, 48), 7.0, device="cuda") for _ in range(2)]
+    need = L.cq_workspace_bytes(w.handle, m, 0)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    handles, outs = (C.c_void_p * 2)(w.handle.value, w.handle.value), (C.c_void_p * 2)(*(y.data_ptr() for y in ys))
+    for room, size in ((None, need), (ws.data_ptr(), need - 1)):
+        assert L.cq_qmatmul_multi(handles, 2, qh.PRE_RMS_NORM, C.c_void_p(x.data_ptr()), C.c_void_p(alpha.data_ptr()), 1e-5, m, outs, 0, room, size, None) == -4
+    torch.cuda.synchronize()
+    assert all(bool((y == 7.0).all()) for y in ys)
