@@ -52,6 +52,31 @@ def test_a_reused_workspace_follows_more_than_three_weights(qh):
         check_f32(y.cpu().numpy(), orc.matmul(orc.Q4K, orc.rms_norm(x, alpha, 1e-5), b, 48))
 
 
+@pytest.mark.parametrize("dt,m,k,ns", [(orc.Q4K, 2, 768, (40,)), (orc.Q4K, 3, 4096, (64, 16)), (orc.Q4K, 4, 4096, (64,)), (orc.Q5K, 3, 2048, (33, 20)),
+                                       (orc.Q6K, 4, 3072, (48, 16, 8)), (orc.Q6K, 3, 5888, (40,))])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e30, 0.0])
+def test_a_bad_row_stays_alone(qh, dt, m, k, ns, bad):
+    """A row with a NaN, an infinity, squares beyond f32, or of zeros only, first, in the middle and last: its own one-row call's bits, and the
+    finite rows beside it theirs."""
+    rng = np.random.default_rng(k + m)
+    alpha = dev(rng.standard_normal(k).astype(np.float32))
+    ws = [qh.QWeight.from_ggml(dt, orc.quantize(dt, make_inputs(k + i, 1, k, n)[0]), n, k) for i, n in enumerate(ns)]
+    kw = dict(pre=qh.PRE_RMS_NORM, aux=alpha, eps=1e-5)
+    for at in range(m):
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        if bad == 0.0:
+            x[at] = 0.0
+        else:
+            x[at, k // 2 + 3] = bad
+        xd = dev(x)
+        outs = qh.qmatmul_multi(ws, xd, **kw) if len(ws) > 1 else [qh.qmatmul(ws[0], xd, **kw)]
+        for w, y in zip(ws, outs):
+            for r in range(m):
+                one = qh.qmatmul(w, xd[r:r + 1].contiguous(), **kw)
+                assert torch.equal(y[r:r + 1].view(torch.int32), one.view(torch.int32)), (at, r)
+                assert r == at or (bool(torch.isfinite(one).all()) and bool((one != 0).any()))
+
+
 @pytest.mark.parametrize("m", [2, 3, 4])
 def test_the_workspace_is_asked_for(qh, m):
     """Several weights behind rms_norm in one launch: a missing or short workspace is refused, as where the rows go through it."""
