@@ -42,7 +42,10 @@ template <bool F16, int ELEMS> struct Run {
     }
     // the run's elements first .. (as far as `total` goes) to the output
     __device__ __forceinline__ void store(float *d32, uint16_t *d16, int64_t first, int64_t total) const {
-        __builtin_amdgcn_wave_barrier();   // (a wave's LDS operations are carried out in order)
+        // the other lanes' writes: the hardware carries out a wave's LDS operations in order, the fences keep the compiler to it
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         typedef uint32_t u4 __attribute__((ext_vector_type(4)));
         u4 *dst = (u4 *)(F16 ? (void *)(d16 + first) : (void *)(d32 + first));
         const int lane = threadIdx.x & 63;
