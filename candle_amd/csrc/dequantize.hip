@@ -13,11 +13,10 @@ constexpr int kThreads = 256;
 
 // The results of a wave's 64 threads (ELEMS each) are one run of the output, of which a thread holds sixteen consecutive elements here and
 // there: they go through LDS, so that every store of the wave is a whole KiB in lane order.  Bound: HBM.  Straight from the threads a store
-// instruction touches every line of the run and fills a quarter of it (f16: half).  The lines are written once and not read here: non-temporal
-// (marking the reads so as well costs 5-20 %).  Whole calls, us, from the threads -> through LDS -> non-temporal: f16 Q6K 32000 x 4096
-// 70.7 -> 63.3 -> 53.2 (6.9 TB/s), Q4K 11008 x 4096 20.9 -> 18.1 -> 15.9, Q4_0 8192 x 4096 24.8 -> 14.0 -> 11.7; f32 Q6K 163 -> 105 -> 88.8,
-// Q4K 56.2 -> 30.9 -> 31.9, Q4_0 43.1 -> 23.5 -> 23.4, Q8_0 43.7 -> 25.7 -> 24.8.
-template <bool F16, int ELEMS> struct Run {
+// instruction touches every line of the run and fills a quarter of it (f16: half).  Kernel times, us, from the threads -> through LDS: f16 Q6K
+// 32000 x 4096 70.7 -> 63.3, Q4K 11008 x 4096 20.9 -> 18.1, Q4_0 8192 x 4096 24.8 -> 14.0; f32 Q6K 163 -> 105, Q4K 56.2 -> 30.9, Q4_0 43.1 -> 23.5,
+// Q8_0 43.7 -> 25.7.  STREAM: stores marked non-temporal (kStreamBytes says when); marking the reads so costs 5-20 %.
+template <bool F16, bool STREAM, int ELEMS> struct Run {
     static constexpr int kSize = F16 ? 2 : 4, kBytes = 64 * ELEMS * kSize, kPer16 = 16 / kSize;
     uint8_t *lds;   // this wave's kBytes
     __device__ __forceinline__ static uint8_t *of_wave() {
@@ -53,15 +52,18 @@ template <bool F16, int ELEMS> struct Run {
         for (int j = 0; j < kBytes / 1024; j++) {
             const uint32_t c = j * 64 + lane;
             const u4 v = *(const u4 *)(lds + at(c));
-            if (first + (int64_t)c * kPer16 < total) __builtin_nontemporal_store(v, dst + c);
+            if (first + (int64_t)c * kPer16 < total) {
+                if constexpr (STREAM) __builtin_nontemporal_store(v, dst + c);
+                else dst[c] = v;
+            }
         }
     }
 };
 
-template <bool F16>
+template <bool F16, bool STREAM>
 __global__ void dequant_q4_0(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ dpl, int64_t nblocks,
                              float *d32, uint16_t *d16) {
-    const Run<F16, 32> run{Run<F16, 32>::of_wave()};
+    const Run<F16, STREAM, 32> run{Run<F16, STREAM, 32>::of_wave()};
     const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x, b = t < nblocks ? t : nblocks - 1;
     const uint4 q = *(const uint4 *)(qs + b * 16);
     const float d = cq_h2f(dpl[b]);
@@ -81,10 +83,10 @@ __global__ void dequant_q4_0(const uint8_t *__restrict__ qs, const uint16_t *__r
 }
 
 // MIN: Q4_1 / Q5_1 held as Q8_0 planes plus the plane of block minima: q * d + m (k_quants.rs:329-349, :533-558)
-template <bool F16, bool MIN>
+template <bool F16, bool STREAM, bool MIN>
 __global__ void dequant_q8_0(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ dpl,
                              const uint16_t *__restrict__ mpl, int64_t nunits, float *d32, uint16_t *d16) {
-    const Run<F16, 16> run{Run<F16, 16>::of_wave()};
+    const Run<F16, STREAM, 16> run{Run<F16, STREAM, 16>::of_wave()};
     const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x, u = t < nunits ? t : nunits - 1;  // 16 elements each
     const uint4 q = *(const uint4 *)(qs + u * 16);
     const float d = cq_h2f(dpl[u >> 1]);
@@ -104,10 +106,10 @@ __global__ void dequant_q8_0(const uint8_t *__restrict__ qs, const uint16_t *__r
 
 // Q5 (Q5K, to_float k_quants.rs:1527-1564): the fifth bits come from the re-ordered qh plane, words
 // {L, H} per 32 qs bytes, bit 8c + i for byte c of qs word i.
-template <bool F16, bool Q5>
+template <bool F16, bool STREAM, bool Q5>
 __global__ void dequant_q4k(const uint8_t *__restrict__ qs, const uint8_t *__restrict__ hd,
                             const uint8_t *__restrict__ qh, int64_t nunits, float *d32, uint16_t *d16) {
-    const Run<F16, 32> run{Run<F16, 32>::of_wave()};
+    const Run<F16, STREAM, 32> run{Run<F16, STREAM, 32>::of_wave()};
     const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x, u = t < nunits ? t : nunits - 1;  // 16 bytes of qs = 32 elements
     const int64_t b = u >> 3;
     const int p = (int)(u & 7), g = p >> 1, half = p & 1;
@@ -137,12 +139,12 @@ __global__ void dequant_q4k(const uint8_t *__restrict__ qs, const uint8_t *__res
 }
 
 // MIN: Q2K held as Q6K planes plus the groups' minima and dmin: (d * sc) * q - dmin * m (k_quants.rs:841-872)
-template <bool F16, bool MIN>
+template <bool F16, bool STREAM, bool MIN>
 __global__ void dequant_q6k(const uint8_t *__restrict__ ql, const uint8_t *__restrict__ qh,
                             const int8_t *__restrict__ sc, const uint16_t *__restrict__ dpl,
                             const uint8_t *__restrict__ mins, const uint16_t *__restrict__ dmins, int64_t nunits,
                             float *d32, uint16_t *d16) {
-    const Run<F16, 32> run{Run<F16, 32>::of_wave()};
+    const Run<F16, STREAM, 32> run{Run<F16, STREAM, 32>::of_wave()};
     const int64_t thread = (int64_t)blockIdx.x * kThreads + threadIdx.x, u = thread < nunits ? thread : nunits - 1;  // 16 bytes of ql = 32 elements
     const int64_t b = u >> 3;
     const int p = (int)(u & 7), h = p >> 2, t = (p >> 1) & 1, i0 = (p & 1) * 16;
@@ -182,7 +184,7 @@ __global__ void dequant_q6k(const uint8_t *__restrict__ ql, const uint8_t *__res
     run.store(d32, d16, (thread - lane) * 32, nunits * 32);
 }
 
-template <bool F16>
+template <bool F16, bool STREAM>
 hipError_t launch(const cq_weight *w, float *d32, uint16_t *d16, hipStream_t s) {
     const int threads = kThreads;
     const int64_t total = w->n * w->k;
@@ -190,28 +192,28 @@ hipError_t launch(const cq_weight *w, float *d32, uint16_t *d16, hipStream_t s) 
     auto grid = [&](int64_t n) { return (unsigned)((n + threads - 1) / threads); };
     switch (w->dtype) {
     case CQ_DTYPE_Q4_0:
-        dequant_q4_0<F16><<<grid(total / 32), threads, 0, s>>>(w->p0, (const uint16_t *)w->p1, total / 32, d32, d16);
+        dequant_q4_0<F16, STREAM><<<grid(total / 32), threads, 0, s>>>(w->p0, (const uint16_t *)w->p1, total / 32, d32, d16);
         break;
     case CQ_DTYPE_Q8_0:
         if (cq_has_min32(w->ggml_dtype))
-            dequant_q8_0<F16, true><<<grid(total / 16), threads, 0, s>>>(w->p0, (const uint16_t *)w->p1, (const uint16_t *)w->p2,
-                                                                         total / 16, d32, d16);
+            dequant_q8_0<F16, STREAM, true><<<grid(total / 16), threads, 0, s>>>(w->p0, (const uint16_t *)w->p1, (const uint16_t *)w->p2,
+                                                                                 total / 16, d32, d16);
         else
-            dequant_q8_0<F16, false><<<grid(total / 16), threads, 0, s>>>(w->p0, (const uint16_t *)w->p1, nullptr, total / 16, d32, d16);
+            dequant_q8_0<F16, STREAM, false><<<grid(total / 16), threads, 0, s>>>(w->p0, (const uint16_t *)w->p1, nullptr, total / 16, d32, d16);
         break;
     case CQ_DTYPE_Q4K:
-        dequant_q4k<F16, false><<<grid(total / 32), threads, 0, s>>>(w->p0, w->p1, nullptr, total / 32, d32, d16);
+        dequant_q4k<F16, STREAM, false><<<grid(total / 32), threads, 0, s>>>(w->p0, w->p1, nullptr, total / 32, d32, d16);
         break;
     case CQ_DTYPE_Q5K:
-        dequant_q4k<F16, true><<<grid(total / 32), threads, 0, s>>>(w->p0, w->p1, w->p2, total / 32, d32, d16);
+        dequant_q4k<F16, STREAM, true><<<grid(total / 32), threads, 0, s>>>(w->p0, w->p1, w->p2, total / 32, d32, d16);
         break;
     case CQ_DTYPE_Q6K:
         if (cq_has_min16(w->ggml_dtype))
-            dequant_q6k<F16, true><<<grid(total / 32), threads, 0, s>>>(w->p0, w->p1, (const int8_t *)w->p2, (const uint16_t *)w->p3,
-                                                                        w->p4, (const uint16_t *)w->p5, total / 32, d32, d16);
+            dequant_q6k<F16, STREAM, true><<<grid(total / 32), threads, 0, s>>>(w->p0, w->p1, (const int8_t *)w->p2, (const uint16_t *)w->p3,
+                                                                                w->p4, (const uint16_t *)w->p5, total / 32, d32, d16);
         else
-            dequant_q6k<F16, false><<<grid(total / 32), threads, 0, s>>>(w->p0, w->p1, (const int8_t *)w->p2, (const uint16_t *)w->p3,
-                                                                         nullptr, nullptr, total / 32, d32, d16);
+            dequant_q6k<F16, STREAM, false><<<grid(total / 32), threads, 0, s>>>(w->p0, w->p1, (const int8_t *)w->p2, (const uint16_t *)w->p3,
+                                                                                 nullptr, nullptr, total / 32, d32, d16);
         break;
     case CQ_DTYPE_Q8K: return cq_launch_dequantize_q8k(w, d32, d16, s);
     default: return hipErrorInvalidValue;
@@ -219,8 +221,18 @@ hipError_t launch(const cq_weight *w, float *d32, uint16_t *d16, hipStream_t s) 
     return hipGetLastError();
 }
 
+// Outputs of more bytes are stored non-temporal.  What reads a dequantized tensor next finds it in the 256 MB of cache in front of the HBM, as long
+// as it did not push itself out.  Dequantize and a product of sixteen rows with the result (torch), us, plain / non-temporal: f16 Q4K 512 x 1024
+// 8.0/9.7, 4096 x 4096 28.1/30.7, 20480 x 4096 (168 MB) 74.5/94.2, 24576 (201 MB) 77.8/90.8, 28672 (235 MB) 120.4/117.3, 32000 (262 MB) 119.8/116.4,
+// 64000 x 2048 108.0/116.3, 40960 x 4096 (336 MB) 164.5/146.3; f32 Q6K 8192 x 8192 (268 MB) 100.5/110.2, 20480 x 4096 (336 MB) 153.1/138.6.  235 to 268
+// MB are level over six shapes and three types.  Without a reader plain is behind by up to 30 % at 8 to 33 MB, level from there to 201 MB (f16 Q6K
+// 20480 x 4096 40.4/41.8) and 5 % behind beyond (32000 x 4096 68.5/63.9).
+constexpr int64_t kStreamBytes = 240000000;
+
 }  // namespace
 
 hipError_t cq_launch_dequantize(const cq_weight *w, float *dst32, uint16_t *dst16, hipStream_t s) {
-    return dst16 ? launch<true>(w, nullptr, dst16, s) : launch<false>(w, dst32, nullptr, s);
+    const bool stream = w->n * w->k * (dst16 ? 2 : 4) > kStreamBytes;
+    if (dst16) return stream ? launch<true, true>(w, nullptr, dst16, s) : launch<true, false>(w, nullptr, dst16, s);
+    return stream ? launch<false, true>(w, dst32, nullptr, s) : launch<false, false>(w, dst32, nullptr, s);
 }

@@ -30,3 +30,20 @@ def test_runs_and_their_ends(qh, dt, elements):  # noqa: F811
             got = out.cpu().numpy()
             assert np.array_equal(got[:n].view(np.uint8), wanted.view(np.uint8)), (n, call)
             assert (got[n:] == 7.0).all(), (n, call)
+
+
+@pytest.mark.parametrize("dt,half", [(orc.Q4_0, True), (orc.Q8_0, True), (orc.Q4_1, False), (orc.Q4K, True), (orc.Q5K, False), (orc.Q6K, False), (orc.Q2K, True)])
+def test_results_around_the_size_of_streamed_ones(qh, dt, half):  # noqa: F811
+    """240 MB of results and more are stored non-temporal: the bits of the same blocks dequantized in smaller parts, on both sides of the line."""
+    k = 4096
+    line = 240_000_000 // (k * (2 if half else 4))
+    for n in (line, line + 1):
+        g = torch.Generator(device="cuda").manual_seed(n)
+        w = qh.QWeight.zeros(dt, n, k).quantize_(torch.randn(n, k, generator=g, device="cuda"))
+        got = w.dequantize_f16() if half else w.dequantize()
+        blocks = w.to_ggml().reshape(n, -1)
+        for lo in range(0, n, 8192):
+            part = blocks[lo:lo + 8192]
+            v = qh.QWeight.from_ggml(dt, part.ravel(), len(part), k)
+            assert torch.equal(got[lo:lo + 8192], v.dequantize_f16() if half else v.dequantize()), lo
+        del w, got
