@@ -91,12 +91,14 @@ int cq_set_error(int code, const char *fmt, ...);
 // then never split K (no partial sums added atomically in arrival order).
 bool cq_no_split_k();
 
-// Whether a plain tile launch marks its results non-temporal: outputs that would push the operands which the workgroups share out of the L2s (which hand
-// the lines on at the end of the launch anyway) and that no launch behind it reads back (the offset term of Q2K, Q4_1 and Q5_1 does).  Whole calls,
-// us, plain -> non-temporal: Q4K 11008 x 4096 at 4096 rows 425 -> 416, 14336 x 4096 at 512 74.8 -> 71.5, 3840 x 1536 at 1466 34.7 -> 31.9, 6636 x 768
-// at 659 22.1 -> 20.9, Q3K 16800 x 4096 at 226 70.5 -> 67.3, Q4_0 14080 x 1280 at 190 21.4 -> 20.5, Q8_0 11008 x 4096 at 4096 554 -> 550.  Read back: Q2K
-// 7447 x 3840 at 220 48.4 -> 49.2, Q4_1 1536 x 768 at 113 13.0 -> 13.5; gate and up of 8 small experts, which w2 reads, 33.8 -> 36.6; the few
-// single floats of the one-row kernels: Q4K 4096 x 4096 4.07 -> 4.41.  Up to 4 MB of results level.
+// Whether a plain tile launch marks its results non-temporal: outputs that would push the operands which the workgroups share out of the L2s.  What
+// reads them next may pay for it, so the line is where a block of launches is ahead: gate and up behind rms_norm and the down-projection that reads both
+// with silu * mul, weights from HBM, six types, four model sizes, 96 to 4096 rows, plain / non-temporal: results of 4 to 8 MB 1.000, 8 to 32 MB 1.018
+// (0.994 to 1.058), 32 to 64 MB 1.003, more 1.007.  Some, us: Q4K 14336 x 4096 at 384 rows 229/224, 1024 473/472, 4096 1704/1692, 2816 x 1024 at 1536 83/79,
+// 5632 x 2048 at 512 94/92, Q8_0 11008 x 4096 at 4096 1677/1667.  A single projection and an elementwise pass over its result: 8 to 32 MB 1.017, beyond
+// level.  The launch alone: Q4K 11008 x 4096 at 4096 rows 432/415, 14336 x 4096 at 2048 287/280, Q3K 16800 x 4096 at 226 70.5/67.3.  Plain stay results
+// that a launch of the call itself reads back (the offset term of Q2K, Q4_1 and Q5_1: Q2K 7447 x 3840 at 220 48.4/49.2), those of experts (w2 reads them:
+// 33.8/36.6) and the few single floats of the one-row kernels (Q4K 4096 x 4096 4.07/4.41).
 inline bool cq_streams_result(const cq_weight *w, int64_t m);
 
 // Compute units of the device (the first one asked; a process has devices of one kind), looked up once.
@@ -124,7 +126,7 @@ __host__ __device__ inline bool cq_has_min32(int ggml_dtype) { return ggml_dtype
 // product with Q8K activations, cq_launch_min16_term subtracts sum_b dmin * d8 * sum_j bsums_j * m_j.
 __host__ __device__ inline bool cq_has_min16(int ggml_dtype) { return ggml_dtype == CQ_DTYPE_Q2K; }
 inline bool cq_streams_result(const cq_weight *w, int64_t m) {
-    return !cq_has_min32(w->ggml_dtype) && !cq_has_min16(w->ggml_dtype) && m * w->n >= (1 << 20);
+    return !cq_has_min32(w->ggml_dtype) && !cq_has_min16(w->ggml_dtype) && m * w->n >= (1 << 21);
 }
 inline int cq_storage_dtype(int ggml_dtype) {
     if (ggml_dtype == CQ_DTYPE_Q5_0 || cq_has_min32(ggml_dtype)) return CQ_DTYPE_Q8_0;
