@@ -550,7 +550,6 @@ static bool clear_in_quantizer_ok(const float *y, int64_t ny, const float *x, in
 static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int64_t m, float *y_dev, int flags,
                         void *ws, size_t ws_bytes, void *stream, bool leave_rows = false) {
     const NoSplitScope no_split(flags);
-    const bool deterministic = (flags & CQ_FLAG_DETERMINISTIC) != 0;
     flags &= ~CQ_FLAG_DETERMINISTIC;   // (only the tile kernels' launch plans look at it; every other kernel is deterministic as it is)
     const size_t need = cq_workspace_bytes(w, m, flags);
     int rc = check_matmul_args(w, x_dev, m, y_dev, ws, ws_bytes, need);
@@ -613,7 +612,7 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     enum { kSkinny, kGemm32, kGemm, kMatvec } path;
     // Few rows: split K over the waves instead of tiling rows.  Measured (weights from HBM, 4096..32000 weight rows,
     // k 4096..14336) faster than the dot-product kernels from 2 rows on and than the tile kernels
-    //   up to 16 rows everywhere; up to 32 rows where two fitted sums say so (cq_skinny_few_ahead);
+    //   up to 16 rows everywhere; up to 32 rows where two fitted sums say so (K-quants: cq_skinny_few_ahead) or below 14336 weight rows (24 rows), 12288 (32);
     //   up to 64 rows where n is small and k short, so that the tile kernel cannot fill the machine.
     // (the 32-element-block types from 4 rows (Q8_0) or 5 rows (Q4_0) on: below that the one-launch dot-product
     // kernel is as fast or faster, it has no per-block scaling of MFMA results to do - where it takes the rows)
@@ -628,9 +627,7 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     //   3 % in 0.3 %, and 22 % faster on average.
     const auto groups_ahead = [&] { return cq_skinny_in_groups(w, m) && 1.2 * cq_skinny_groups_us(w, m) < (has_tile32 ? cq_gemm32_us(w, m) : cq_gemm_us(w, m)); };
     const bool k_quant = act == CQ_DTYPE_Q8K && !min32;   // (Q2K: the tile kernels add its offset term in a launch of its own)
-    // (the sums know the tiles with K split; a deterministic call, which never splits it, stays with the split-K kernel below the lines)
-    const bool few_line = (m <= 24 && w->n < 14336) || (m <= 32 && w->n < 12288);
-    const bool few_ahead = k_quant && m > 16 && m <= 32 ? cq_skinny_few_ahead(w, m) || (deterministic && few_line) : few_line;
+    const bool few_ahead = k_quant && m > 16 && m <= 32 ? cq_skinny_few_ahead(w, m) : (m <= 24 && w->n < 14336) || (m <= 32 && w->n < 12288);
     const bool skinny_rows = m <= 16 || few_ahead || (m <= 64 && w->n < 8192 && w->k <= 6144) ||
                              (!has_tile32 && groups_ahead());
     if (flags & CQ_FLAG_FORCE_SKINNY) {

@@ -1368,6 +1368,14 @@ double cq_gemm_us(const cq_weight *w, int64_t m) {
     static constexpr double start[3] = {5.3, 5.3, 5.8}, work[3] = {0.67, 0.79, 0.52}, merge[3] = {1.02, 1.02, 1.12};
     return start[t] + (work[t] * p.work + merge[t] * p.merge) / 16.0;
 }
+// us of the whole call with 17 to 32 rows and weights from HBM, beside the split-K kernel's at cq_skinny_few_ahead.  (The sum above is of weights that
+// a benchmark loop finds in the caches; with large ones from HBM it is up to 40 % short.)
+double cq_gemm_few_us(const cq_weight *w, int64_t m) {
+    const Plan p = pick_plan(w, m);
+    static constexpr double sum[3][4] = {{5.14, 0.656, 0.480, 0.130}, {5.31, 0.791, 0.820, 0.108}, {5.91, 0.497, 0.434, 0.116}};   // start, work, merge, a MB
+    const double(&c)[4] = sum[w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2];
+    return c[0] + (c[1] * p.work + c[2] * p.merge) / 16.0 + c[3] * (double)w->n * (double)(w->k / 256) * (double)cq_type_size(w->dtype) / 1e6;
+}
 bool cq_gemm_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }
 
 bool cq_gemm_takes(const cq_weight *w, int act_dtype) {

@@ -238,9 +238,11 @@ hipError_t cq_launch_skinny(const cq_weight *w, cq_act_view a, int act_dtype, in
 bool cq_skinny_in_groups(const cq_weight *w, int64_t m);
 double cq_skinny_groups_us(const cq_weight *w, int64_t m);
 double cq_gemm_us(const cq_weight *w, int64_t m);
+double cq_gemm_few_us(const cq_weight *w, int64_t m);
 double cq_gemm32_us(const cq_weight *w, int64_t m);
-// the rows of a small weight in one launch that quantizes them itself (and leaves them in the workspace)
+// 17 to 32 rows of a K-quant: ahead of the tiles
 bool cq_skinny_few_ahead(const cq_weight *w, int64_t m);
+// the rows of a small weight in one launch that quantizes them itself (and leaves them in the workspace)
 bool cq_skinny_direct_takes(const cq_weight *w, int act_dtype, int64_t m);
 hipError_t cq_launch_skinny_direct(const cq_weight *w, cq_act_view a, const float *x, int64_t m, float *y, hipStream_t s);
 // two or three weights (same type and row length) on the same rows in one launch, up to 16 rows, where that is the faster way

@@ -1875,29 +1875,29 @@ hipError_t cq_launch_skinny_grouped(const cq_weight *const *experts, int n_exper
     }
 }
 
+// 17 to 32 rows of a K-quant: whether the split-K kernel is ahead of the tiles (us of both whole calls, the quantizer in front of each; thousands of
+// weight rows, K / 1024).  It walks K once for every round of sixteen weight rows a compute unit, which the bytes hide behind at first, and beyond 24
+// rows one workgroup less fits a compute unit; the tiles cost by their plan, K split or not (cq_gemm_few_us).  Both fitted to 165 shapes of each
+// type at 17, 24 and 32 rows, weights from HBM (8192 to 128256 weight rows with K 512 to 16384, 3072 to 7168 with K 6400 to 28672), mostly to those
+// where the kernels are close: the choice is 0.3 % behind the better one on average, 10 % at worst and more than 3 % in 4 % of the calls; lines at
+// 14336 weight rows (24 rows) and 12288 (32) are 4.6 % behind on average, 61 % at worst.  Some (us, split K / tiles): 24 rows Q4K 8192 x 14336
+// 31.8/26.6, 4128 x 12288 25.6/19.8, 4096 x 14336 18.9/21.0, Q5K 16384 x 3072 19.7/23.8, 6144 x 16384 38.3/33.7; 32 rows Q4K 11008 x 8192 32.5/25.5,
+// 10240 x 1024 11.6/9.9, 4096 x 14336 20.8/22.0, Q6K 8192 x 14336 41.1/34.7, 12288 x 3072 20.3/23.4.  Small weights, whose rows go in groups
+// (cq_skinny_in_groups), stay: level, the tiles up to 18 % ahead only with K beyond 20000 (Q4K 1024 x 28672 23.5/20.2).
+bool cq_skinny_few_ahead(const cq_weight *w, int64_t m) {
+    if (cq_skinny_in_groups(w, m)) return true;
+    static constexpr double split[2][3][4] = {{{6.14, 0.083, 0.030, 0.733}, {6.34, 0.131, 0.026, 0.884}, {6.32, 0.112, 0.044, 0.810}},
+                                              {{5.22, 0.329, 0.014, 0.953}, {5.55, 0.408, 0.009, 1.085}, {5.55, 0.383, 0.033, 0.978}}};
+    const double(&c)[4] = split[m > 24][w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2];
+    const int64_t cus = cq_num_cus(), rounds = ((w->n + 15) / 16 + cus - 1) / cus;
+    const double rows = (double)w->n / 1000.0, k = (double)w->k / 1024.0;
+    return c[0] + c[1] * rows + c[2] * rows * k + c[3] * k * (double)rounds < cq_gemm_few_us(w, m);
+}
+
 // One launch over all the weights rather than a launch each.  Measured with rms_norm in front, weights from HBM, five types, 2..16 rows,
 // ten pairs and triples from 1024 to 28672 weight rows and K = 1024..8192 (us of the whole call, one launch / a launch each):
 // the one launch is ahead everywhere (Q4K, 8 rows: 4096 + 1024 + 1024 x 4096 12.2 / 18.9, 2 x 14336 x 4096 24.3 / 26.8, 2 x 28672
 // x 8192 77.5 / 82.7; 16 rows: Q6K 2 x 14336 x 4096 32.2 / 37.2, Q8_0 2 x 11008 x 4096 31.2 / 31.8).
-// 17 to 32 rows of a K-quant: whether the split-K kernel (groups of 24 or 32 rows) is ahead of the tiles.  It costs by the byte of weight and
-// beyond 24 rows one workgroup less fits a compute unit; the tiles leave compute units idle below some 16000 weight rows and then cost by the row
-// length.  Both sums (us; thousands of weight rows, K / 1024, their product) fitted to 50 shapes of each type, 4096..32000 weight
-// rows, K 1024..14336, weights from HBM: 4 and 6 % off on average.  They decide where they are 8 % apart, and the lines at 14336 weight rows (24
-// rows) or 12288 (32), right for K = 4096, between: the lines alone were 2.3 % behind the better kernel, this 1.3 %, and no shape is slower for
-// it.  Some (us, split K / tiles): 20 rows Q5K 16384 x 3072 20.3/24.5, 14336 x 2048 14.6/17.6, 24576 x 2048 22.0/19.6, Q4K 8192 x 14336 32.2/25.7;
-// 32 rows Q4K 11008 x 8192 33.5/26.1, Q6K 8192 x 14336 42.6/36.0, 12288 x 3072 20.2/23.3.
-bool cq_skinny_few_ahead(const cq_weight *w, int64_t m) {
-    static constexpr double split[2][3][4] = {{{5.243, 0.124, 0.065, 0.208}, {5.275, 0.161, 0.183, 0.240}, {5.196, 0.146, 0.181, 0.240}},
-                                              {{4.528, 0.348, -0.094, 0.262}, {4.674, 0.392, -0.118, 0.312}, {4.487, 0.392, -0.047, 0.301}}};
-    static constexpr double tiles[2][3][4] = {{{11.171, -0.154, 0.077, 0.173}, {13.674, -0.244, 0.321, 0.230}, {13.020, -0.203, 0.156, 0.227}},
-                                              {{11.284, -0.165, 0.124, 0.183}, {13.877, -0.251, 0.334, 0.236}, {13.265, -0.215, 0.137, 0.238}}};
-    const int t = w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2, g = m > 24;
-    const double rows = (double)w->n / 1000.0, k = (double)w->k / 1024.0;
-    const auto us = [&](const double (&c)[4]) { return c[0] + c[1] * rows + c[2] * k + c[3] * rows * k; };
-    const bool line = g ? w->n < 12288 : w->n < 14336;
-    return line ? us(split[g][t]) < 1.08 * us(tiles[g][t]) : 1.08 * us(split[g][t]) < us(tiles[g][t]);
-}
-
 bool cq_skinny_shared_takes(const cq_weight *const *ws, int count, int64_t m, int act_dtype) {
     if (count < 2 || count > kMultiMax || m > 16) return false;
     for (int i = 0; i < count; i++)
