@@ -183,9 +183,10 @@ hipError_t cq_launch_matvec_fused(const cq_weight *w, const float *x, cq_pre pre
 // 2 <= m <= 4 rows in the one-launch kernel (short rows only)
 bool cq_matvec_fused_rows_supported(const cq_weight *w, int64_t m);
 hipError_t cq_launch_matvec_fused_rows(const cq_weight *w, const float *x, int64_t m, float *y, hipStream_t s);
-// several weights on the same activations in one launch (same dtype, k, device; 2 or 3 of them): one row, or
-// as many rows as cq_matvec_fused_rows_supported allows (then without a fused step)
+// the same with rms_norm in front, over the rows of one to three K-quant weights
 bool cq_matvec_fused_rms_rows_supported(const cq_weight *const *ws, int count, int64_t m);
+// several weights on the same activations in one launch (same dtype, k, device; 2 or 3 of them): one row, or as many rows as the two above
+// allow, without a fused step or with rms_norm
 bool cq_matvec_fused_multi_supported(const cq_weight *const *ws, int count, int pre_kind, int64_t m);
 hipError_t cq_launch_matvec_fused_multi(const cq_weight *const *ws, int count, const float *x, cq_pre pre, int64_t m,
                                         float *const *ys, hipStream_t s);

@@ -177,7 +177,11 @@ size_t cq_workspace_bytes(const cq_weight *w, int64_t m, int flags);
  * x contiguous f32; m = product of the leading dims of the input tensor.
  * Q4_1, Q5_0 and Q5_1 weights with an odd number of 32-element blocks per row are refused with
  * CQ_ERR_INVALID, as their vec_dot refuses them (k_quants.rs:273, 363, 469); so do the other matmul
- * entry points. */
+ * entry points.
+ * Bits: a row's last bits depend on the number of rows (not on what the others hold).  Two to four rows take the kernel
+ * of one row, with the bits of their one-row calls, or, where that is faster by the weight's type, n and k, kernels
+ * that add a row's blocks in another order, as every call with more rows does.  Who needs the bits of one-row calls
+ * makes one-row calls. */
 int cq_qmatmul(const cq_weight *w, const float *x_dev, int64_t m, float *y_dev, int flags,
                void *workspace_dev, size_t workspace_bytes, void *stream);
 /* The same with the weight's shape given at the call, exactly as QCudaStorage::fwd(&self, self_shape, ..)
@@ -268,9 +272,12 @@ int cq_qmatmul_fused(const cq_weight *w, int pre, const float *x_dev, const floa
  * `pre` in front as in cq_qmatmul_fused (CQ_PRE_NONE for none).  The weights share dtype, row length k and
  * device; their row counts may differ.  One activation row and two or three weights with rows of at most
  * 256 lane units (k <= 16384 for Q4K/Q5K, 8192 for Q6K/Q4_0, 4096 for Q8_0), flags == 0: a single launch
- * for all of them, each output bit-identical to its own cq_qmatmul_fused call; the same for two to four
- * rows when the weight rows are short enough and few enough for the one-launch kernel, without a step in front
- * or, K-quants, with rms-norm: every row has the bits of its one-row call then.  More rows: the rows are quantized once and every weight takes its matmul from the shared
+ * for all of them, each output bit-identical to its own cq_qmatmul_fused call.  Two to four rows take that
+ * launch too, without a step in front or, K-quants, with rms-norm, where it is the faster way by the weights'
+ * type, k and row counts (the first weight's without a step in front, all of them together with one); every row
+ * then has the bits of its one-row call.  A weight's own call decides by its own row count: where the two decide
+ * apart, and with more rows, an output and that call's agree to the order of their f32 sums, not in bits.
+ * More rows: the rows are quantized once and every weight takes its matmul from the shared
  * workspace (size: the largest cq_workspace_bytes among the weights).  Anything else: one call per weight.  The reference has no
  * counterpart, it calls QMatMul::forward once per weight; a `Hip` arm can offer it to the model code beside
  * forward(). */

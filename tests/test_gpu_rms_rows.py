@@ -52,6 +52,23 @@ def test_a_reused_workspace_follows_more_than_three_weights(qh):
         check_f32(y.cpu().numpy(), orc.matmul(orc.Q4K, orc.rms_norm(x, alpha, 1e-5), b, 48))
 
 
+def test_weights_that_decide_apart(qh):
+    """One weight of many rows and two of few: two launches together, the one launch for the small ones alone.  The outputs agree to the order of
+    the sums."""
+    k, m, ns = 512, 2, (8192, 1024, 1024)
+    rng = np.random.default_rng(5)
+    x, alpha = dev(rng.standard_normal((m, k)).astype(np.float32)), dev(rng.standard_normal(k).astype(np.float32))
+    ws = [qh.QWeight.from_ggml(orc.Q4K, orc.quantize(orc.Q4K, make_inputs(i, 1, k, n)[0]), n, k) for i, n in enumerate(ns)]
+    f = qh.load()._Z34cq_matvec_fused_rms_rows_supportedPKPK9cq_weightil
+    f.restype, f.argtypes = C.c_bool, [C.c_void_p, C.c_int, C.c_int64]
+    assert not f((C.c_void_p * 3)(*(w.handle.value for w in ws)), 3, m) and f((C.c_void_p * 1)(ws[1].handle.value), 1, m)
+    kw = dict(pre=qh.PRE_RMS_NORM, aux=alpha, eps=1e-5)
+    for w, y in zip(ws, qh.qmatmul_multi(ws, x, **kw)):
+        own = qh.qmatmul(w, x, **kw)
+        # (the one launch scales the results, the quantizer its input: a quant beside the middle of two may go the other way)
+        assert ((y - own).norm() / own.norm()).item() <= 2e-3
+
+
 @pytest.mark.parametrize("dt,m,k,ns", [(orc.Q4K, 2, 768, (40,)), (orc.Q4K, 3, 4096, (64, 16)), (orc.Q4K, 4, 4096, (64,)), (orc.Q5K, 3, 2048, (33, 20)),
                                        (orc.Q6K, 4, 3072, (48, 16, 8)), (orc.Q6K, 3, 5888, (40,))])
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e30, 0.0])
