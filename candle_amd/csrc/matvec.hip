@@ -1640,7 +1640,10 @@ static bool offset_rows_to_split_k(const cq_weight *w, int64_t m) {
     const double lane = (double)elems_per_lane(w), rows = (double)w->n / 1000.0, few = rows < 4.1 ? rows : 4.1, many = rows - few, md = (double)m;
     const double mb = (double)w->n * (double)w->k * 1e-6, blocks = (double)(w->k / 256);
     if (cq_has_min16(w->ggml_dtype)) {
-        if (lane > 128) return w->n > 1024;   // (few weight rows keep the bits)
+        // (beyond 8192 elements, two rows, the instance spills.  One launch / split K at K = 8448, 9216, 10240, 11264, 12288: 64 weight rows 13.3/10.4,
+        // 11.5/10.9, 11.5/11.6, 11.7/11.6, 11.9/13.3; 1024 14.9/11.2, 13.1/11.6, 13.2/12.8, 13.5/12.6, 13.7/14.2, 11 % behind on average; 2048 16.2/12.1,
+        // 14.5/12.4, 14.9/13.8, 15.2/13.9, 15.6/15.5; 4096, two weight rows a wave, 22.5/13.4, 21.3/14.0, 21.8/15.3, 22.7/15.5, 22.8/17.3)
+        if (lane > 128) return w->n > 1024;
         const int collide = w->k % 1024 == 0 ? 0 : w->k % 512 == 0 ? 1 : 2;
         const double one = 2.5 + 1.13 * md + (lane > 32 ? 0.4 + 0.0138 * (lane - 32) * md : 0.0) + (0.1 + 0.0085 * (lane - 32)) * few +
                            (0.2 + 0.0092 * lane + (0.12 + 0.065 * collide) * (md - 2)) * many;
