@@ -92,13 +92,14 @@ int cq_set_error(int code, const char *fmt, ...);
 bool cq_no_split_k();
 
 // Whether a plain tile launch marks its results non-temporal: outputs that would push the operands which the workgroups share out of the L2s.  What
-// reads them next may pay for it, so the line is where a block of launches is ahead: gate and up behind rms_norm and the down-projection that reads both
-// with silu * mul, weights from HBM, six types, four model sizes, 96 to 4096 rows, plain / non-temporal: results of 4 to 8 MB 1.000, 8 to 32 MB 1.018
-// (0.994 to 1.058), 32 to 64 MB 1.003, more 1.007.  Some, us: Q4K 14336 x 4096 at 384 rows 229/224, 1024 473/472, 4096 1704/1692, 2816 x 1024 at 1536 83/79,
-// 5632 x 2048 at 512 94/92, Q8_0 11008 x 4096 at 4096 1677/1667.  A single projection and an elementwise pass over its result: 8 to 32 MB 1.017, beyond
-// level.  The launch alone: Q4K 11008 x 4096 at 4096 rows 432/415, 14336 x 4096 at 2048 287/280, Q3K 16800 x 4096 at 226 70.5/67.3.  Plain stay results
-// that a launch of the call itself reads back (the offset term of Q2K, Q4_1 and Q5_1: Q2K 7447 x 3840 at 220 48.4/49.2), those of experts (w2 reads them:
-// 33.8/36.6) and the few single floats of the one-row kernels (Q4K 4096 x 4096 4.07/4.41).
+// reads them next may pay for it, so the line is where launch and reader together are ahead.  Results of 4 to 8 MB, five types, eight shapes of 1344 to
+// 24000 weight rows, weights from HBM, plain / non-temporal: the launch alone 1.018 (0.997 to 1.067), with an elementwise pass over the result 1.016,
+// with the projection behind it 1.006, gate and up behind rms_norm and the down-projection that reads both with silu * mul 1.007 (0.986 to 1.025);
+// that block with 8 to 32 MB 1.018 (0.994 to 1.058), 32 to 64 MB 1.003, more 1.007.  Some blocks, us: Q4K 5632 x 2048 at 350 rows 68.7/67.5, 14336 x 4096
+// at 384 229/224, 4096 1704/1692, 2816 x 1024 at 1536 83/79, Q8_0 11008 x 4096 at 4096 1677/1667.  The launch alone: Q4K 1344 x 512 at 1280 10.6/10.2,
+// 11008 x 4096 at 4096 432/415, Q3K 16800 x 4096 at 226 70.5/67.3.  Below 4 MB level.  Plain stay results that a launch of the call itself reads back (the
+// offset term of Q2K, Q4_1 and Q5_1: Q2K 7447 x 3840 at 220 48.4/49.2), those of experts (w2 reads them: 33.8/36.6) and the few single floats of
+// the one-row kernels (Q4K 4096 x 4096 4.07/4.41).
 inline bool cq_streams_result(const cq_weight *w, int64_t m);
 
 // Compute units of the device (the first one asked; a process has devices of one kind), looked up once.
@@ -126,7 +127,7 @@ __host__ __device__ inline bool cq_has_min32(int ggml_dtype) { return ggml_dtype
 // product with Q8K activations, cq_launch_min16_term subtracts sum_b dmin * d8 * sum_j bsums_j * m_j.
 __host__ __device__ inline bool cq_has_min16(int ggml_dtype) { return ggml_dtype == CQ_DTYPE_Q2K; }
 inline bool cq_streams_result(const cq_weight *w, int64_t m) {
-    return !cq_has_min32(w->ggml_dtype) && !cq_has_min16(w->ggml_dtype) && m * w->n >= (1 << 21);
+    return !cq_has_min32(w->ggml_dtype) && !cq_has_min16(w->ggml_dtype) && m * w->n >= (1 << 20);
 }
 inline int cq_storage_dtype(int ggml_dtype) {
     if (ggml_dtype == CQ_DTYPE_Q5_0 || cq_has_min32(ggml_dtype)) return CQ_DTYPE_Q8_0;

@@ -30,10 +30,9 @@ def test_several_rounds_in_strips(qh, dt, m, n, k):  # noqa: F811
 
 
 @pytest.mark.parametrize("dt", ["Q4K", "Q5K", "Q6K", "Q8_0", "Q4_0"])
-@pytest.mark.parametrize("m,n,k", [(511, 2048, 512), (512, 2048, 512), (2000, 524, 512), (2001, 525, 512), (2200, 480, 4096),
-                                   (1023, 2048, 512), (1024, 2048, 512), (4000, 524, 512), (3996, 525, 512), (4400, 480, 4096)])
+@pytest.mark.parametrize("m,n,k", [(511, 2048, 512), (512, 2048, 512), (2000, 524, 512), (2001, 525, 512), (2200, 480, 4096)])
 def test_results_around_the_size_of_streamed_ones(qh, dt, m, n, k):  # noqa: F811
-    """2^21 results and more are stored non-temporal: whole and halved K, ragged columns, on both sides of the line."""
+    """2^20 results and more are stored non-temporal: whole and halved K, ragged columns, on both sides of the line."""
     check(qh, dt, m, n, k)
 
 
