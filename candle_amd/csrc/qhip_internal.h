@@ -510,7 +510,8 @@ __device__ __forceinline__ cq_u32x4 cq_min_term_groups_int(const uint32_t (&rec)
 enum cq_put { kPutPlain, kPutStream, kPutAdd };
 template <int HOW> __device__ __forceinline__ void cq_put_result(float *p, float v) {
     if constexpr (HOW == kPutAdd) unsafeAtomicAdd(p, v);
-    // (a builtin store would be merged with the plain one of the other path and lose the mark)
+    // (a builtin store would be merged with the plain one of the other path and lose the mark; the compiler puts no wait states in front of this
+    // one, so a value must not come straight out of an MFMA: the callers have a barrier and the addresses, or an addition, between)
     else if constexpr (HOW == kPutStream) asm volatile("global_store_dword %0, %1, off nt" : : "v"(p), "v"(v) : "memory");
     else *p = v;
 }
