@@ -121,42 +121,16 @@ __device__ __forceinline__ void q8k_chunk(const float4 f, int64_t row, int64_t b
     const int lane = threadIdx.x & 63;
     const int64_t blk = row * (k / 256) + b_in_row;
 
-    // The first element whose |x| equals the block maximum decides the sign of the scale (strict
-    // `<` in the reference keeps the earliest).  Reductions run on DPP operands, not through LDS.
-    const float a0 = fabsf(f.x), a1 = fabsf(f.y), a2 = fabsf(f.z), a3 = fabsf(f.w);
-    const float amax = wave_max(fmaxf(fmaxf(fmaxf(fmaxf(0.0f, a0), a1), a2), a3));
-    int idx = 0x7fffffff;
-    if (a3 == amax) idx = 4 * lane + 3;
-    if (a2 == amax) idx = 4 * lane + 2;
-    if (a1 == amax) idx = 4 * lane + 1;
-    if (a0 == amax) idx = 4 * lane;
-    idx = wave_min_i(idx);
-    const int sel = idx & 3;
-    const float cand = sel == 0 ? f.x : (sel == 1 ? f.y : (sel == 2 ? f.z : f.w));
-    const float max = readlane_f(cand, __builtin_amdgcn_readfirstlane(idx >> 2));
-
-    uint32_t packed = 0;
-    int sum = 0;
-    float d = 0.0f;
-    if (amax != 0.0f) {
-        const float iscale = -128.0f / max;
-        const int8_t q0 = cq_as_i8(fminf(roundf(iscale * f.x), 127.0f));
-        const int8_t q1 = cq_as_i8(fminf(roundf(iscale * f.y), 127.0f));
-        const int8_t q2 = cq_as_i8(fminf(roundf(iscale * f.z), 127.0f));
-        const int8_t q3 = cq_as_i8(fminf(roundf(iscale * f.w), 127.0f));
-        packed = (uint32_t)(uint8_t)q0 | ((uint32_t)(uint8_t)q1 << 8) | ((uint32_t)(uint8_t)q2 << 16) |
-                 ((uint32_t)(uint8_t)q3 << 24);
-        sum = (int)q0 + (int)q1 + (int)q2 + (int)q3;
-        d = 1.0f / iscale;
-        if (SCALED) {
-            const bool zero = dscale == 0.0f;
-            packed = zero ? 0 : packed;
-            sum = zero ? 0 : sum;
-            d = zero ? 0.0f : d * dscale;
-        }
+    uint32_t packed;
+    int sum;   // lanes 4j .. 4j + 3 hold bsums[j]
+    float d;
+    cq_q8k_of_wave(f, lane, packed, d, sum);
+    if (SCALED) {
+        const bool zero = dscale == 0.0f;
+        packed = zero ? 0u : packed;
+        sum = zero ? 0 : sum;
+        d = zero ? 0.0f : d * dscale;
     }
-    sum += dpp_i<kQuadSwap1>(sum);
-    sum += dpp_i<kQuadSwap2>(sum);  // lanes 4j..4j+3 now hold bsums[j]
     if (AOS) {
         uint8_t *b = out.aos + blk * 292;  // 292 = 4 * 73: 4-byte aligned
         if (lane == 0) *(float *)b = d;
@@ -175,8 +149,8 @@ __device__ __forceinline__ void q8k_chunk(const float4 f, int64_t row, int64_t b
 }
 
 // Many rows: a block per sixteen lanes, four blocks a wave.  Lane l of a block's sixteen holds elements 64i + 4l .. + 3 (i = 0..3),
-// reductions end inside the sixteen lanes and every scalar step of a block (index, two divisions, stores) is shared by four.
-// A wave a block (the kernel below) spends about 250 vector instructions on it and is bound by them; here memory is.  Kernel
+// reductions end inside the sixteen lanes and every scalar step of a block (two divisions, stores) is shared by four.
+// A wave a block (the kernel below) is bound by its vector instructions; here memory is.  Kernel
 // alone, us, with a wave a block -> here: 512 x 4096 6.0 -> 3.3, 1024 x 4096 9.2 -> 5.7, 4096 x 4096 22.3 -> 15.4 (5.5 TB/s), with
 // silu 32.9 -> 26.5, 4096 x 14336 123 -> 105.
 template <bool AOS, bool SILU>

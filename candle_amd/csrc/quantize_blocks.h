@@ -61,6 +61,46 @@ __device__ __forceinline__ void cq_q8k_of_sixteen(const float4 (&f)[4], int l, u
     bsum = j == 0 ? sum[0] : j == 1 ? sum[1] : j == 2 ? sum[2] : sum[3];
 }
 
+// The same for a block per wave: lane l holds elements 4l .. 4l + 3; all arguments but `f` and `packed` are the wave's.  `sum`: of the lane's four
+// lanes (bsums[l / 4]).  For few blocks: the launch waits for one chain of dependent instructions, which the search for the first largest element,
+// the rounding by itself and the clamp by another made twice as long (24 such launches behind rms_norm and silu, among them the step's other
+// launches: 481.9 -> 479.2 us; eight rows of 4096 with their matmul 10.21 -> 10.18).
+__device__ __forceinline__ void cq_q8k_of_wave(const float4 f, int lane, uint32_t &packed, float &d, int &sum) {
+    float hi = fmaxf(fmaxf(fmaxf(fmaxf(0.0f, f.x), f.y), f.z), f.w), lo = fminf(fminf(fminf(fminf(0.0f, f.x), f.y), f.z), f.w);
+    hi = fmaxf(hi, dpp_f<kQuadSwap1>(hi));
+    lo = fminf(lo, dpp_f<kQuadSwap1>(lo));
+    hi = fmaxf(hi, dpp_f<kQuadSwap2>(hi));
+    lo = fminf(lo, dpp_f<kQuadSwap2>(lo));
+    hi = fmaxf(hi, dpp_f<kHalfMirror>(hi));
+    lo = fminf(lo, dpp_f<kHalfMirror>(lo));
+    hi = fmaxf(hi, dpp_f<kRowMirror>(hi));
+    lo = fminf(lo, dpp_f<kRowMirror>(lo));
+    hi = fmaxf(fmaxf(readlane_f(hi, 0), readlane_f(hi, 16)), fmaxf(readlane_f(hi, 32), readlane_f(hi, 48)));
+    lo = fminf(fminf(readlane_f(lo, 0), readlane_f(lo, 16)), fminf(readlane_f(lo, 32), readlane_f(lo, 48)));
+    const float amax = fmaxf(hi, -lo);
+    float max = hi > -lo ? hi : lo;
+    if (__any(hi == -lo && amax != 0.0f)) {   // both signs: the sign of the first of them
+        int idx = 0x7fffffff;
+        const float v[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+        for (int c = 3; c >= 0; c--)
+            if (fabsf(v[c]) == amax) idx = 2 * (4 * lane + c) + (v[c] < 0.0f ? 1 : 0);
+        max = wave_min_i(idx) & 1 ? lo : hi;
+    }
+    const bool any = amax != 0.0f;
+    const float iscale = -128.0f / max;
+    d = any ? 1.0f / iscale : 0.0f;
+    const float v[4] = {f.x, f.y, f.z, f.w};
+    uint32_t q[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) q[c] = (uint32_t)cq_round_away_i32(fmaxf(fminf(iscale * v[c], 127.0f), -128.0f));   // (as above)
+    const uint32_t p01 = __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u), p23 = __builtin_amdgcn_perm(q[3], q[2], 0x04000c0cu);
+    packed = any ? p01 | p23 : 0u;
+    sum = __builtin_amdgcn_sdot4((int)packed, 0x01010101, 0, false);
+    sum += dpp_i<kQuadSwap1>(sum);
+    sum += dpp_i<kQuadSwap2>(sum);
+}
+
 // Q8_0 / Q8_1 (k_quants.rs:586-615): a block per eight lanes, each with four consecutive elements `f` (zeros past the end of a row; called by
 // all 64 lanes).  The four quants in a word, the unrounded scale, the block's sum.
 __device__ __forceinline__ void cq_q8_0_of_eight(const float4 f, uint32_t &packed, float &d, int &sum) {
