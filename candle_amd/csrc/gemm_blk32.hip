@@ -7,11 +7,14 @@
 // A 32-element block is exactly one K-slice of v_mfma_i32_32x32x32_i8, so the integer of every
 // (activation row, weight row, block) is one MFMA result element, I (Q4_0 nibbles go in as q - 8, so
 // no correction term is left).  Its scale d8[row, block] * dw[col, block] is an outer product: a
-// second MFMA lays it out in the accumulator layout (v_mfma_f32_32x32x16_bf16 with four non-zero K-slots:
-// both scales are f16 values and go in as two bf16 pieces each, all exact, so the four products are the exact
-// product whatever the magnitude of the activations, and the result is d8 * dw to f32 rounding; the f32 MFMA with
-// one K-slot holds the matrix pipe twice as long), and the VALU
+// second MFMA lays it out in the accumulator layout (v_mfma_f32_32x32x8_f16 with one non-zero K-slot: both scales are f16
+// values, and their product, subnormal factors included, is exact in f32), and the VALU
 // work per element is one conversion and one fma.
+// Bound by vector issue.  ns a step of the two waves of a SIMD (a tile and block of each) in a loop of nothing but steps, the scales as two bf16
+// pieces each (v_mfma_f32_32x32x16_bf16: three instructions for the operand, three for the zeros beside it) -> as f16: Q8_0 70.9 -> 62.8, Q4_0
+// 68.5 -> 61.0; without the second MFMA 55.6.  Whole calls, weights from HBM, us: Q8_0 11008 x 4096 at 4096 / 512 / 64 rows 511 -> 474, 93.6 -> 87.4,
+// 23.9 -> 23.3, Q4_0 4096 x 4096 at 512 / 1024 rows 35.6 -> 33.4, 59.0 -> 55.0, 11008 x 4096 at 4096 498 -> 459, Q5_0 4096 x 11008 at 700
+// 150.9 -> 141.2.  (The next step's weight operands read under this step's last tile instead of behind the barrier: level to 2 % slower.)
 //
 // Work split as in the K-quant tile kernel (gemm.hip): a workgroup of eight waves covers 32*MT
 // activation rows x 256 weight rows, a wave owns 32 weight rows; per 256-element step of K the
@@ -27,8 +30,8 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef void __attribute__((address_space(3))) *lptr_t;
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));   // (rows of whole 64-element pairs of blocks)
 
@@ -65,6 +68,9 @@ template <int DT, int MT> struct Tile {
     static constexpr int oWgt = 2 * kStage;
     static constexpr int kTotal = oWgt + kWaves * kWgtWave;
 };
+
+// What the sums are multiplied by on their way out: a power of two, exact (the scales are f16 values: no sum comes near the range of f32).
+template <int DT> constexpr float kUnit = DT == CQ_DTYPE_Q4_0 ? 0.0625f : 1.0f;
 
 struct LaneGeo {
     uint32_t row_off;    // copy of 8 rows x 128 B with a row pitch of k bytes: (l/8)*k + ((l%8) ^ (l/8))*16; odd row groups: ^ 16
@@ -144,7 +150,7 @@ template <int DT> __device__ __forceinline__ void step_weights(const uint8_t *wl
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             // block s: 16 bytes, low nibbles = elements 0..15 (h = 0), high nibbles = elements 16..31; as 16 * (q - 8), the
-            // nibble in the upper half of its byte: two instructions a word (the block scale takes the 1/16)
+            // nibble in the upper half of its byte: two instructions a word (kUnit takes the 1/16 out of the results)
             const v4i q = *(const v4i *)(wl + g.col4[s]);
 #pragma unroll
             for (int i = 0; i < 4; i++) bw[s][i] = (int)((((uint32_t)q[i] << (4 - 4 * h)) & 0xF0F0F0F0u) ^ 0x80808080u);
@@ -159,21 +165,16 @@ template <int DT, int MT, bool DUMP, bool SHORT, bool LOWER = false>
 __device__ __forceinline__ void step_mac(const uint8_t *cur, const LaneGeo &g, const v4i (&bw)[8], const u32x4_a4 dcur, int nv, int h, int col,
                                          v16f (&out)[MT], const cq_weight &w, int64_t m0, int64_t m, int64_t n, int64_t b, cq_mfma_dump dump) {
     typedef Tile<DT, MT> T;
-    // scale operand of block s: dw = b1 + b2 (bf16 pieces, exact: an f16 has 11 significant bits); lanes
-    // 0..31 carry b1 in K-slots 0 and 1, lanes 32..63 carry b2 in K-slots 8 and 9, the other slots zero
+    // scale operand of block s: the f16 scale in the one K-slot that is not zero (lanes 0..31)
     // A last step of fewer than eight blocks: what follows the rows in memory (other rows, other planes) was copied
     // with them, and both scales of the blocks that do not exist are zero.
     const uint32_t dwords[4] = {dcur.x, dcur.y, dcur.z, dcur.w};
-    v8bf dw[8];
+    v4h dw[8];
 #pragma unroll
     for (int s = 0; s < 8; s++) {
-        float f = !SHORT || s < nv ? cq_h2f((uint16_t)((dwords[s >> 1] >> (16 * (s & 1))) & 0xffffu)) : 0.0f;
-        if (DT == CQ_DTYPE_Q4_0) f *= 0.0625f;   // (exact: step_weights)
-        const uint32_t fb = __float_as_uint(f);
-        const float b2 = f - __uint_as_float(fb & 0xffff0000u);
-        const uint32_t piece = h == 0 ? fb >> 16 : __float_as_uint(b2) >> 16;
-        const v4u pk = {piece | (piece << 16), 0u, 0u, 0u};
-        dw[s] = __builtin_bit_cast(v8bf, pk);
+        const uint32_t bits = s & 1 ? dwords[s >> 1] >> 16 : dwords[s >> 1] & 0xffffu;
+        const v2u pk = {h == 0 && (!SHORT || s < nv) ? bits : 0u, 0u};
+        dw[s] = __builtin_bit_cast(v4h, pk);
     }
 
     // steps q = (tile t, block s): the two MFMAs of step q, and in their shadow the scaling of step q-1
@@ -182,19 +183,19 @@ __device__ __forceinline__ void step_mac(const uint8_t *cur, const LaneGeo &g, c
         return *(const v4i *)(cur + g.col[s & 3] + (t * 2 + (s >> 2)) * 4096);
     };
     // activation scale of (row l%32 of tile t, block s): read two steps ahead, and only turned into
-    // the MFMA operand (two bf16 pieces) in the step that uses it, so that no step
+    // the MFMA operand in the step that uses it, so that no step
     // waits for the read it has just issued
     auto d8raw = [&](int q) -> float {
         const int t = q >> 3, s = q & 7;
         const float v = *(const float *)(cur + T::oD8 + t * 1024 + s * 128 + col * 4);
         return !SHORT || s < nv ? v : 0.0f;
     };
-    auto d8frag = [&](float v) -> v8bf {
-        // v = a1 + a2, the leading eight bits and the other three of an f16 value (exact); K-slots 0, 1 of both lane halves
-        const uint32_t vb = __float_as_uint(v);
-        const float r1 = v - __uint_as_float(vb & 0xffff0000u);
-        const v4u pk = {__builtin_amdgcn_perm(__float_as_uint(r1), vb, 0x07060302u), 0u, 0u, 0u};
-        return __builtin_bit_cast(v8bf, pk);
+    auto d8frag = [&](float v) -> v4h {
+        // an f16 value, in the K-slot that the weight's scale is in; in slots where that has zeros stays what the register holds (finite where the
+        // scale is)
+        const _Float16 d = (_Float16)v;
+        const v2u pk = {(uint32_t)__builtin_bit_cast(uint16_t, d), __float_as_uint(v)};
+        return __builtin_bit_cast(v4h, pk);
     };
     v16i acc[2];
     v16f sc[2];
@@ -209,7 +210,7 @@ __device__ __forceinline__ void step_mac(const uint8_t *cur, const LaneGeo &g, c
         if (q + 2 < MT * 8) { av[(q + 2) % 3] = afrag(q + 2); dv[(q + 2) % 3] = d8raw(q + 2); }
         if (q < MT * 8) {
             acc[q & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[q % 3], bw[q & 7], zero, 0, 0, 0);
-            sc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(d8frag(dv[q % 3]), dw[q & 7], zerof, 0, 0, 0);
+            sc[q & 1] = __builtin_amdgcn_mfma_f32_32x32x8f16(d8frag(dv[q % 3]), dw[q & 7], zerof, 0, 0, 0);
         }
         // keeps the MFMAs in front of the scaling below: left alone, the scheduler sinks them to the end
         // of the step, and the next step then starts by waiting for their results
@@ -291,7 +292,7 @@ __device__ __forceinline__ void gemm32_body(const cq_weight &w, const cq_act_vie
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                    if (row < m && n >= n_own) cq_put_result<decltype(how)::value>(&y[row * w.n + n], out[t][i]);
+                    if (row < m && n >= n_own) cq_put_result<decltype(how)::value>(&y[row * w.n + n], out[t][i] * kUnit<DT>);
                 }
             }
         });
@@ -390,7 +391,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_kh_kernel(cq_weight w, cq_act
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int64_t row = m0 + t * 32 + (i >> 2) * 8 + h * 4 + (i & 3);
-                    if (row < m && n >= n_own) cq_put_result<decltype(how)::value>(&y[row * w.n + n], out[t][i] + part[(t * 16 + i) * 64 + lane]);
+                    if (row < m && n >= n_own) cq_put_result<decltype(how)::value>(&y[row * w.n + n], (out[t][i] + part[(t * 16 + i) * 64 + lane]) * kUnit<DT>);
                 }
             }
         });
@@ -481,7 +482,7 @@ __global__ void __launch_bounds__(kThreads) gemm32_few_kernel(cq_weight w, cq_ac
             for (int p = 0; p < KS; p++) v += *(const float *)(smem + (p * CW + colw) * Few<DT>::kWave + (i * 64 + lane) * 4);
         }
         const int64_t row = (i >> 2) * 8 + h * 4 + (i & 3);
-        if (row < m) y[row * w.n + n] = v;
+        if (row < m) y[row * w.n + n] = v * kUnit<DT>;
     }
 }
 
