@@ -964,14 +964,24 @@ extern "C" int cq_silu_mul(int dev, const float *a, const float *b, float *h, in
     return CQ_OK;
 }
 
-extern "C" int cq_moe_scatter_add(int dev, const float *y, const int32_t *row_ids, const float *weights,
-                                  int64_t total_rows, int64_t hidden, float *ys, int64_t tokens, void *stream) {
+static int moe_scatter(int dev, const float *y, const int32_t *row_ids, const float *weights, int64_t total_rows, int64_t hidden, float *ys,
+                       int64_t tokens, bool add, void *stream) {
     if (total_rows < 0 || hidden < 0 || tokens < 0) return cq_set_error(CQ_ERR_INVALID, "negative size");
     if (tokens == 0 || hidden == 0) return CQ_OK;
     if (!ys || (total_rows && (!y || !row_ids || !weights))) return cq_set_error(CQ_ERR_INVALID, "null argument");
     CQ_HIP_CHECK(hipSetDevice(dev));
-    CQ_HIP_CHECK(cq_launch_scatter_add(y, row_ids, weights, total_rows, hidden, ys, tokens, (hipStream_t)stream));
+    CQ_HIP_CHECK(cq_launch_scatter_add(y, row_ids, weights, total_rows, hidden, ys, tokens, add, (hipStream_t)stream));
     return CQ_OK;
+}
+
+extern "C" int cq_moe_scatter_add(int dev, const float *y, const int32_t *row_ids, const float *weights,
+                                  int64_t total_rows, int64_t hidden, float *ys, int64_t tokens, void *stream) {
+    return moe_scatter(dev, y, row_ids, weights, total_rows, hidden, ys, tokens, true, stream);
+}
+
+extern "C" int cq_moe_scatter(int dev, const float *y, const int32_t *row_ids, const float *weights, int64_t total_rows,
+                              int64_t hidden, float *ys, int64_t tokens, void *stream) {
+    return moe_scatter(dev, y, row_ids, weights, total_rows, hidden, ys, tokens, false, stream);
 }
 
 extern "C" int cq_timing_arm(void) {

@@ -16,13 +16,16 @@ __global__ void silu_mul_kernel(const float *__restrict__ a, const float *__rest
 // ys[row_ids[p], j] += weights[p] * y[p, j], positions p visited in increasing order for every
 // destination element (the reference's sequential index_add, cpu_backend/mod.rs:619-653, applied
 // expert by expert).  One thread per destination element; no atomics, so the sum order is fixed.
+// ADD: to what ys holds; else to zero, and ys is only written.  That saves the caller the launch that clears it: qhip.moe_scatter_add, calls back to
+// back, 1 to 256 tokens, 13.3 -> 9.5 us, the expert block of 64 tokens at 4096 x 14336 253.3 -> 250.5.
+template <bool ADD>
 __global__ void scatter_add_kernel(const float *__restrict__ y, const int32_t *__restrict__ row_ids,
                                    const float *__restrict__ weights, int64_t total_rows, int64_t hidden,
                                    float *__restrict__ ys, int64_t tokens) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= tokens * hidden) return;
     const int64_t t = i / hidden, j = i - t * hidden;
-    float acc = ys[i];
+    float acc = ADD ? ys[i] : 0.0f;
     for (int64_t p = 0; p < total_rows; p++) {
         if (row_ids[p] == (int32_t)t) acc += y[p * hidden + j] * weights[p];
     }
@@ -32,6 +35,7 @@ __global__ void scatter_add_kernel(const float *__restrict__ y, const int32_t *_
 // The same sum for hidden % 4 == 0: a workgroup owns 1024 consecutive elements of one token, so the
 // search for the token's rows is wave-uniform (scalar loads and branches) and only the matching
 // rows cost vector work.
+template <bool ADD>
 __global__ void scatter_add4_kernel(const float *__restrict__ y, const int32_t *__restrict__ row_ids,
                                     const float *__restrict__ weights, int total_rows, int64_t hidden,
                                     float *__restrict__ ys) {
@@ -39,7 +43,7 @@ __global__ void scatter_add4_kernel(const float *__restrict__ y, const int32_t *
     const int64_t j = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     const int lane = threadIdx.x & 63;
     const bool live = j < hidden;
-    float4 acc = live ? *(const float4 *)(ys + (int64_t)t * hidden + j) : make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 acc = ADD && live ? *(const float4 *)(ys + (int64_t)t * hidden + j) : make_float4(0.f, 0.f, 0.f, 0.f);
     // 64 row ids per step, one per lane; the matches come out of the lane mask in increasing order
     for (int base = 0; base < total_rows; base += 64) {
         const int q = base + lane;
@@ -74,16 +78,18 @@ hipError_t cq_launch_silu_mul(const float *a, const float *b, float *h, int64_t 
 }
 
 hipError_t cq_launch_scatter_add(const float *y, const int32_t *row_ids, const float *weights, int64_t total_rows,
-                                 int64_t hidden, float *ys, int64_t tokens, hipStream_t s) {
+                                 int64_t hidden, float *ys, int64_t tokens, bool add, hipStream_t s) {
     if (hidden % 4 == 0 && tokens <= 65535 && total_rows <= INT32_MAX && (((uintptr_t)y | (uintptr_t)ys) & 15) == 0) {
         if (tokens == 0 || hidden == 0) return hipSuccess;
-        dim3 grid((unsigned)((hidden / 4 + 255) / 256), (unsigned)tokens);
-        scatter_add4_kernel<<<grid, 256, 0, s>>>(y, row_ids, weights, (int)total_rows, hidden, ys);
+        const dim3 grid((unsigned)((hidden / 4 + 255) / 256), (unsigned)tokens);
+        if (add) scatter_add4_kernel<true><<<grid, 256, 0, s>>>(y, row_ids, weights, (int)total_rows, hidden, ys);
+        else scatter_add4_kernel<false><<<grid, 256, 0, s>>>(y, row_ids, weights, (int)total_rows, hidden, ys);
         return hipGetLastError();
     }
     const int64_t count = tokens * hidden;
-    scatter_add_kernel<<<(unsigned)((count + 255) / 256), 256, 0, s>>>(y, row_ids, weights, total_rows, hidden, ys,
-                                                                        tokens);
+    const unsigned grid = (unsigned)((count + 255) / 256);
+    if (add) scatter_add_kernel<true><<<grid, 256, 0, s>>>(y, row_ids, weights, total_rows, hidden, ys, tokens);
+    else scatter_add_kernel<false><<<grid, 256, 0, s>>>(y, row_ids, weights, total_rows, hidden, ys, tokens);
     return hipGetLastError();
 }
 

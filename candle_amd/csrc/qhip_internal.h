@@ -315,7 +315,7 @@ static inline cq_grouped_plan cq_plan_grouped_tiles(const cq_weight *w, const in
 // moe.hip
 hipError_t cq_launch_silu_mul(const float *a, const float *b, float *h, int64_t count, hipStream_t s);
 hipError_t cq_launch_scatter_add(const float *y, const int32_t *row_ids, const float *weights, int64_t total_rows,
-                                 int64_t hidden, float *ys, int64_t tokens, hipStream_t s);
+                                 int64_t hidden, float *ys, int64_t tokens, bool add, hipStream_t s);
 
 hipError_t cq_launch_fill_zero(float *p, int64_t count, hipStream_t s);
 

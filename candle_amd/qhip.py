@@ -26,7 +26,7 @@ EXPORTS = [
     "cq_weight_dequantize_f16", "cq_weight_to_ggml", "cq_weight_size_in_bytes", "cq_weight_dtype",
     "cq_weight_device", "cq_weight_shape", "cq_weight_destroy", "cq_act_bytes", "cq_quantize_act",
     "cq_workspace_bytes", "cq_qmatmul", "cq_qmatmul_int_dots", "cq_qmatmul_int_dots_mfma", "cq_grouped_workspace_bytes",
-    "cq_qmatmul_grouped", "cq_silu_mul", "cq_moe_scatter_add", "cq_timing_arm", "cq_timing_elapsed_us",
+    "cq_qmatmul_grouped", "cq_silu_mul", "cq_moe_scatter_add", "cq_moe_scatter", "cq_timing_arm", "cq_timing_elapsed_us",
     "cq_selfcheck_round", "cq_quantize_act_fused", "cq_qmatmul_fused", "cq_qmatmul_grouped_fused", "cq_qmatmul_multi",
     "cq_weight_zeros_flat", "cq_weight_create_flat", "cq_weight_elem_count", "cq_weight_set_shape",
     "cq_workspace_bytes_shaped", "cq_qmatmul_shaped", "cq_qmatmul_static",
@@ -77,6 +77,7 @@ def load():
     L.cq_qmatmul_grouped.argtypes = [C.POINTER(vp), ci, vp, vp, C.POINTER(C.c_int32), vp, ci, vp, sz, vp]
     L.cq_silu_mul.argtypes = [ci, vp, vp, vp, i64, vp]
     L.cq_moe_scatter_add.argtypes = [ci, vp, vp, vp, i64, i64, vp, i64, vp]
+    L.cq_moe_scatter.argtypes = [ci, vp, vp, vp, i64, i64, vp, i64, vp]
     L.cq_timing_arm.argtypes = []
     L.cq_timing_elapsed_us.argtypes = [C.POINTER(C.c_double)]
     L.cq_selfcheck_round.argtypes = [ci, C.POINTER(C.c_uint64)]
@@ -418,10 +419,10 @@ def silu_mul(a, b):
 def moe_scatter_add(y, row_ids, weights, tokens: int):
     torch = _torch()
     total, hidden = y.shape
-    ys = torch.zeros((tokens, hidden), dtype=torch.float32, device=y.device)
-    check(load().cq_moe_scatter_add(y.device.index or 0, C.c_void_p(y.data_ptr()), C.c_void_p(row_ids.data_ptr()),
-                                    C.c_void_p(weights.data_ptr()), total, hidden, C.c_void_p(ys.data_ptr()),
-                                    tokens, _stream_ptr()))
+    ys = torch.empty((tokens, hidden), dtype=torch.float32, device=y.device)
+    check(load().cq_moe_scatter(y.device.index or 0, C.c_void_p(y.data_ptr()), C.c_void_p(row_ids.data_ptr()),
+                                C.c_void_p(weights.data_ptr()), total, hidden, C.c_void_p(ys.data_ptr()), tokens,
+                                _stream_ptr()))
     return ys
 
 

@@ -248,6 +248,9 @@ int cq_silu_mul(int dev, const float *a_dev, const float *b_dev, float *h_dev, i
  * increasing p, which is increasing expert index, like the reference's sequential loop. */
 int cq_moe_scatter_add(int dev, const float *y_dev, const int32_t *row_ids_dev, const float *weights_dev,
                        int64_t total_rows, int64_t hidden, float *ys_dev, int64_t tokens, void *stream);
+/* The same sums from zero: ys is written, whatever it holds (tokens without a row: zeros). */
+int cq_moe_scatter(int dev, const float *y_dev, const int32_t *row_ids_dev, const float *weights_dev,
+                   int64_t total_rows, int64_t hidden, float *ys_dev, int64_t tokens, void *stream);
 
 /* ---- the matmul with the preceding model step fused in --------------------------------------
  * What the quantized models run directly in front of a QMatMul, computed on the way into the
