@@ -672,22 +672,21 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     }
     cq_act_view v;
     act_ws_layout(act, m, w->k, (uint8_t *)ws, &v);
-    bool y_cleared = false;
+    uint32_t *const turns = path == kGemm ? cq_act_turns(v, w->k) : nullptr;
+    bool cleared = false;
     // a small weight: the rows quantized by the waves of the split-K kernel, which leaves them in the workspace as well
     const bool direct = flags == 0 && pre.kind == CQ_PRE_NONE && !in_place && path == kSkinny && cq_skinny_direct_takes(w, act, m);
     if (!(flags & CQ_FLAG_REUSE_ACT) && !direct) {
-        cq_clear clear = cq_no_clear();
-        const bool splits = path == kGemm32 ? cq_gemm32_splits_k(w, m) : path == kGemm ? cq_gemm_splits_k(w, m) : false;
-        if (splits && clear_in_quantizer_ok(y_dev, m * w->n, x_dev, m * w->k, pre)) {
-            clear = cq_clear{y_dev, m * w->n};
-            y_cleared = true;
-        }
+        cq_clear clear = path == kGemm ? cq_gemm_clears(w, m, turns, y_dev)
+                                       : path == kGemm32 && cq_gemm32_splits_k(w, m) ? cq_clear{y_dev, m * w->n} : cq_no_clear();
+        cleared = clear.p && (clear.p != y_dev || clear_in_quantizer_ok(y_dev, m * w->n, x_dev, m * w->k, pre));
+        if (!cleared) clear = cq_no_clear();
         CQ_HIP_CHECK(cq_launch_quantize_act_ws(act, x_dev, nullptr, m, w->k, pre, v, clear, s));
     }
     switch (path) {
         case kSkinny: CQ_HIP_CHECK(direct ? cq_launch_skinny_direct(w, v, x_dev, m, y_dev, s) : cq_launch_skinny(w, v, act, m, y_dev, s)); break;
-        case kGemm32: CQ_HIP_CHECK(cq_launch_gemm32(w, v, act, m, y_dev, y_cleared, s)); break;
-        case kGemm: CQ_HIP_CHECK(cq_launch_gemm(w, v, act, m, y_dev, y_cleared, s)); break;
+        case kGemm32: CQ_HIP_CHECK(cq_launch_gemm32(w, v, act, m, y_dev, cleared, s)); break;
+        case kGemm: CQ_HIP_CHECK(cq_launch_gemm(w, v, act, m, turns, y_dev, cleared, s)); break;
         case kMatvec: CQ_HIP_CHECK(cq_launch_matvec(w, v, act, m, y_dev, s)); break;
     }
     // (the split-K kernel adds the offset term itself)
@@ -901,17 +900,17 @@ static int grouped_impl(const cq_weight *const *experts, int n_experts, const fl
         };
         if (skinny && !force_gemm && (force_skinny || path == kEach || most <= grouped_skinny_rows(w0) || ahead())) path = kSkinny;
     }
-    // gather + quantize every routed row once (clearing the output on the way if the grouped launch splits K;
-    // with row ids the extent of x is not known here, so nothing is cleared then)
-    cq_clear clear = cq_no_clear();
-    const bool splits = path == kGemm ? cq_gemm_grouped_splits_k(experts, n_experts, offsets)
-                                      : path == kGemm32 && cq_gemm32_grouped_splits_k(experts, n_experts, offsets);
-    if (!reuse && !row_ids_dev && splits && clear_in_quantizer_ok(y_dev, total * w0->n, x_dev, total * w0->k, pre))
-        clear = cq_clear{y_dev, total * w0->n};
+    // gather + quantize every routed row once (clearing on the way what a grouped launch that splits K wants zero; with row ids the
+    // extent of x is not known here, so no output is cleared then)
+    uint32_t *const turns = path == kGemm ? cq_act_turns(v, w0->k) : nullptr;
+    cq_clear clear = path == kGemm ? cq_gemm_grouped_clears(experts, n_experts, offsets, turns, y_dev)
+                                   : path == kGemm32 && cq_gemm32_grouped_splits_k(experts, n_experts, offsets) ? cq_clear{y_dev, total * w0->n}
+                                                                                                                : cq_no_clear();
+    if (reuse || (clear.p == y_dev && (row_ids_dev || !clear_in_quantizer_ok(y_dev, total * w0->n, x_dev, total * w0->k, pre)))) clear = cq_no_clear();
     if (!reuse) CQ_HIP_CHECK(cq_launch_quantize_act_ws(act, x_dev, row_ids_dev, total, w0->k, pre, v, clear, s));
     switch (path) {
     case kSkinny: CQ_HIP_CHECK(cq_launch_skinny_grouped(experts, n_experts, offsets, v, y_dev, s)); return CQ_OK;
-    case kGemm: CQ_HIP_CHECK(cq_launch_gemm_grouped(experts, n_experts, offsets, v, y_dev, clear.p != nullptr, s)); return CQ_OK;
+    case kGemm: CQ_HIP_CHECK(cq_launch_gemm_grouped(experts, n_experts, offsets, v, turns, y_dev, clear.p != nullptr, s)); return CQ_OK;
     case kGemm32: CQ_HIP_CHECK(cq_launch_gemm32_grouped(experts, n_experts, offsets, v, y_dev, clear.p != nullptr, s)); return CQ_OK;
     case kEach: break;
     }
@@ -935,7 +934,7 @@ static int grouped_impl(const cq_weight *const *experts, int n_experts, const fl
         const bool use_gemm = (flags & CQ_FLAG_FORCE_GEMM) ? true
                               : (flags & CQ_FLAG_FORCE_MATVEC) ? false
                                                                : (te > 8 && cq_gemm_takes(experts[e], act));
-        if (use_gemm) CQ_HIP_CHECK(cq_launch_gemm(experts[e], ve, act, te, ye, false, s));
+        if (use_gemm) CQ_HIP_CHECK(cq_launch_gemm(experts[e], ve, act, te, nullptr, ye, false, s));
         else CQ_HIP_CHECK(cq_launch_matvec(experts[e], ve, act, te, ye, s));
     }
     return CQ_OK;

@@ -25,7 +25,7 @@
 // instruction reads eight whole 128-byte lines (8 rows x 128 B) - the texture path pays per line
 // touched - and the 16-byte chunks of a row are XOR-swizzled by the row number on the way in, so
 // that the MFMA operand reads (lanes = rows, one chunk column) spread over all LDS banks.  With few
-// workgroups (small n) K is split over blockIdx.z and the partial results are added atomically.
+// workgroups (small n) K is split over blockIdx.z: two parts take turns at the results, more add theirs atomically.
 #include <type_traits>
 
 #include "qhip_internal.h"
@@ -602,13 +602,58 @@ __device__ __forceinline__ void block_step(const uint8_t *__restrict__ cur, uint
 // earlier, at row n - 32, and stores only its share (every column is contracted by itself, so nothing else changes).
 __device__ __forceinline__ int64_t last_tile(int64_t n_own, int64_t n) { return n_own + 32 <= n ? n_own : n - 32; }
 
+// K split in two over workgroups: the parts of a wave's results take turns (an atomic counter for every tile and wave).  The first one done stores
+// them, the other waits until they are there, reads them, adds its own and stores the sum: the same bits whichever is first.  A part waits only for
+// one that has taken its turn before, is past all its own waits and runs to its end, whatever else runs on the device.  What is passed on goes
+// through the memory that all XCDs see (stores and loads of device scope; a store has arrived there when s_waitcnt says so, and only then the turn
+// is passed on).  `turn`: {turns taken, turns done}, zero before the launch.
+// Adding to a cleared y atomically moves about 1.1 TB/s at the end of all workgroups at once, and y is cleared first.  Whole calls, weights from
+// HBM, us, atomic additions -> turns: Q6K 4096 x 14336 at 1003 rows 164.8 -> 152.5, 7510 x 5376 at 423 80.1 -> 63.0, Q4K 8382 x 14336 at 375
+// 134.2 -> 120.3, Q3K 3102 x 9216 at 1089 110.6 -> 94.4, Q6K 21822 x 5376 at 96 62.9 -> 54.8; 8 experts of 1024 x 3584 with 100 tokens
+// 57.4 -> 51.8.  More parts stay with the additions: a turn of each costs some 5 us, one after the other (Q6K 4096 x 14336 at 512 / 128 rows, four
+// and eight parts, 96.2 -> 93.8 and 39.8 -> 58.7, Q4K 4096 x 14336 at 256 52.7 -> 54.7).
+template <int MT>
+__device__ __forceinline__ void put_in_turn(uint32_t *turn, float *y, float *yc, int64_t pitch, int64_t left, int lane, v16f (&out)[MT]) {
+    uint32_t mine = 0;
+    if (lane == 0) mine = __hip_atomic_fetch_add(turn, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const auto at = [&](int t, int i) { return (int64_t)(t * 32 + (i >> 2) * 8 + (i & 3)); };
+    if (__builtin_amdgcn_readfirstlane((int)mine) > 0) {   // the second
+        // (bounded, a second or so: calls that share a workspace although they overlap spoil each other's turns as well as rows)
+        for (int looks = 1 << 20; looks > 0; looks--) {
+            if (__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(turn + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        asm volatile("" ::: "memory");   // (the results are requested behind this)
+        float held[MT][16];
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) held[t][i] = __hip_atomic_load(at(t, i) < left ? yc + at(t, i) * pitch : y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (at(t, i) < left) yc[at(t, i) * pitch] = out[t][i] + held[t][i];
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            if (at(t, i) < left) __hip_atomic_store(yc + at(t, i) * pitch, out[t][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (lane == 0) __hip_atomic_store(turn + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ------------------------------------------------------------------ kernel ----
 // Requires n >= 32 and an activation workspace with padded rows (cq_act_view::m_stride).
 // One workgroup: activation rows [m0, m0 + 32*MT) (stored up to row m - 1) x the 256 weight rows of
 // blockIdx.x, K blocks of part blockIdx.z.
-template <int DT, int MT, bool DUMP = false, int WBUF = 1, bool ONCE = false>
+// TURN: two parts, whose waves take turns at the results.
+template <int DT, int MT, bool DUMP = false, int WBUF = 1, bool ONCE = false, bool TURN = false>
 __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view &a, int64_t bx, int64_t m0, int64_t m,
-                                          float *__restrict__ y, int ksplit, bool stream, cq_mfma_dump dump = cq_mfma_dump{nullptr, nullptr, 0}) {
+                                          float *__restrict__ y, int ksplit, bool stream, cq_mfma_dump dump = cq_mfma_dump{nullptr, nullptr, 0},
+                                          uint32_t *turns = nullptr) {
     static_assert(WBUF == 1 || DT == CQ_DTYPE_Q4K || DT == CQ_DTYPE_Q5K, "block headers of 20 bytes");
     typedef Tile<DT, MT> T;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -692,6 +737,15 @@ __device__ __forceinline__ void gemm_body(const cq_weight &w, const cq_act_view 
         else run(T_{}, F_{});
     }
 
+    if constexpr (TURN) {
+        if (!n_ok) return;
+        int wv = wave, ln = lane;
+        asm volatile("" : "+s"(wv), "+v"(ln));
+        const int64_t own = (bx * kWaves + wv) * 32, c = last_tile(own, w.n) + (ln & 31);
+        put_in_turn<MT>(turns + ((blockIdx.x + (size_t)gridDim.x * blockIdx.y) * kWaves + wv) * 2, y, y + (m0 + (ln >> 5) * 4) * w.n + c, w.n,
+                        c < own ? 0 : m - m0 - (ln >> 5) * 4, ln, out);
+        return;
+    }
     if (n_ok && !DUMP) {
         // (the lane's column anew: kept from above it would take registers that the 128-row tiles do not have)
         int wv = wave, ln = lane;
@@ -718,6 +772,11 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(cq_weight w, cq_act_view
                                                         int ksplit, int strips, int stream) {
     const cq_tile t = cq_tile_at(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, strips);
     gemm_body<DT, MT>(w, a, t.x, (int64_t)t.y * (MT * 32), m, y, ksplit, stream != 0);
+}
+// (kernels of their own: as a branch in the others' ends, the main loops were allocated otherwise and launches that do not split lost 1.2 %)
+template <int DT, int MT>
+__global__ void __launch_bounds__(kThreads) gemm_turns_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t *turns) {
+    gemm_body<DT, MT, false, 1, false, true>(w, a, blockIdx.x, (int64_t)blockIdx.y * (MT * 32), m, y, 2, false, cq_mfma_dump{nullptr, nullptr, 0}, turns);
 }
 
 // 128-row tiles in whole rounds of workgroups, and what is left of them in tiles of 32 * TAIL rows: the last round of a launch
@@ -750,6 +809,10 @@ template <int DT>
 __global__ void __launch_bounds__(kThreads) gemm_once_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y,
                                                              int ksplit) {
     gemm_body<DT, 1, false, once_wbuf<DT>(), true>(w, a, blockIdx.x, 0, m, y, ksplit, false);
+}
+template <int DT>
+__global__ void __launch_bounds__(kThreads) gemm_once_turns_kernel(cq_weight w, cq_act_view a, int64_t m, float *__restrict__ y, uint32_t *turns) {
+    gemm_body<DT, 1, false, once_wbuf<DT>(), true, true>(w, a, blockIdx.x, 0, m, y, 2, false, cq_mfma_dump{nullptr, nullptr, 0}, turns);
 }
 
 // The same launch with the block integers stored instead of the result (verification).
@@ -911,6 +974,14 @@ __global__ void __launch_bounds__(kThreads) gemm_grouped_kernel(cq_group_args ga
     const cq_weight w = ga.w[ga.expert[tile]];
     if constexpr (MT == 1) gemm_body<DT, 1, false, grouped_wbuf<DT>(), true>(w, a, blockIdx.x, ga.row0[tile], ga.row_end[tile], y, ksplit, false);
     else gemm_body<DT, MT>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, ksplit, false);
+}
+template <int DT, int MT>
+__global__ void __launch_bounds__(kThreads) gemm_grouped_turns_kernel(cq_group_args ga, cq_act_view a, float *__restrict__ y, uint32_t *turns) {
+    const int tile = blockIdx.y;
+    const cq_weight w = ga.w[ga.expert[tile]];
+    const cq_mfma_dump none{nullptr, nullptr, 0};
+    if constexpr (MT == 1) gemm_body<DT, 1, false, grouped_wbuf<DT>(), true, true>(w, a, blockIdx.x, ga.row0[tile], ga.row_end[tile], y, 2, false, none, turns);
+    else gemm_body<DT, MT, false, 1, false, true>(w, a, blockIdx.x, ga.row0[tile], min(ga.row0[tile] + 32 * MT, ga.row_end[tile]), y, 2, false, none, turns);
 }
 
 // ------------------------------------------------ K-quant weights x Q8_1 activations (tile kernel) ----
@@ -1124,7 +1195,9 @@ int64_t n_tiles(const cq_weight *w) { return (w->n + kWaves * 32 - 1) / (kWaves 
 // Tile height (MT x 32 activation rows per workgroup) and K split of a launch, from a cost model fitted to
 // measurements (Q4K, 256 CUs; unit 1/16 us): a workgroup spends 22 units per K block unpacking its weights
 // and 13.5 per 32-row tile on it, 24 on starting and finishing; workgroups run one per CU, in rounds; a split
-// launch adds every part to the output atomically, which moves about 1.1 TB/s.  Tall tiles amortise
+// launch adds every part to the output atomically, which moves about 1.1 TB/s (two parts take turns and are less than that; the plan is as it was:
+// with their own price, 3 us and 2.7 TB/s, 1.1 % of the calls change, on average 4 % slower, as the work's price is above what it costs).  Tall
+// tiles amortise
 // the unpacking, short ones fill the machine without splitting K: 4096 x 4096 at 512 rows takes 54 us as
 // 64 tiles of 128 rows split four ways and 42 us as 256 tiles of 32 rows.
 struct Plan {
@@ -1189,25 +1262,47 @@ Plan pick_plan(const cq_weight *w, int64_t m) {
     return best;
 }
 
+// Words of the turns of a launch over `tiles` tiles, or 0 where they do not fit their place (64 rows of quants).
+int64_t turn_words(int64_t tiles, int64_t k) { return tiles * kWaves * 8 <= 64 * k ? tiles * kWaves * 2 : 0; }
+// What such a launch of `parts` parts wants zero: the turns, or the output of `count` floats that is added to atomically.
+cq_clear clears(int parts, int64_t tiles, int64_t k, uint32_t *turns, float *y, int64_t count) {
+    if (parts <= 1) return cq_no_clear();
+    const int64_t words = turns && parts == 2 ? turn_words(tiles, k) : 0;
+    return words ? cq_clear{(float *)turns, words} : cq_clear{y, count};
+}
+// ... cleared by a launch of its own where it is not yet; `turns` stays only if they are used.
+hipError_t clear_parts(int parts, int64_t tiles, int64_t k, uint32_t *&turns, float *y, int64_t count, bool cleared, hipStream_t s) {
+    const cq_clear c = clears(parts, tiles, k, turns, y, count);
+    if (c.p != (float *)turns) turns = nullptr;
+    return c.p && !cleared ? cq_launch_fill_zero(c.p, c.count, s) : hipSuccess;
+}
+
 template <int DT> constexpr size_t once_lds() { return once_wbuf<DT>() == 2 ? Tile<DT, 1>::kTotal2 : Tile<DT, 1>::kTotal; }
 template <int DT, int MT>
-hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, float *y, int ksplit, bool y_cleared, hipStream_t s) {
-    const size_t lds = Tile<DT, MT>::kTotal;
-    if (hipError_t e = cq_ensure_lds<gemm_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
+hipError_t launch_mt(const cq_weight *w, cq_act_view a, int64_t m, uint32_t *turns, float *y, int ksplit, bool cleared, hipStream_t s) {
     const int64_t gx = n_tiles(w), gy = (m + MT * 32 - 1) / (MT * 32);
-    if (ksplit > 1 && !y_cleared) {
-        hipError_t e = cq_launch_fill_zero(y, m * w->n, s);
-        if (e != hipSuccess) return e;
-    }
-    dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)ksplit);
+    if (hipError_t e = clear_parts(ksplit, gx * gy, w->k, turns, y, m * w->n, cleared, s); e != hipSuccess) return e;
+    const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)ksplit);
     if constexpr (MT == 1) {
         if (gy == 1) {
             const size_t lds1 = once_lds<DT>();
+            if (turns) {
+                if (hipError_t e = cq_ensure_lds<gemm_once_turns_kernel<DT>>(w->dev, lds1); e != hipSuccess) return e;
+                CQ_LAUNCH((gemm_once_turns_kernel<DT>), grid, kThreads, lds1, s, *w, a, m, y, turns);
+                return hipGetLastError();
+            }
             if (hipError_t e = cq_ensure_lds<gemm_once_kernel<DT>>(w->dev, lds1); e != hipSuccess) return e;
             CQ_LAUNCH((gemm_once_kernel<DT>), grid, kThreads, lds1, s, *w, a, m, y, ksplit);
             return hipGetLastError();
         }
     }
+    const size_t lds = Tile<DT, MT>::kTotal;
+    if (turns) {
+        if (hipError_t e = cq_ensure_lds<gemm_turns_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm_turns_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y, turns);
+        return hipGetLastError();
+    }
+    if (hipError_t e = cq_ensure_lds<gemm_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
     CQ_LAUNCH((gemm_kernel<DT, MT>), grid, kThreads, lds, s, *w, a, m, y, ksplit, cq_tiles_in_strips(gx * gy, ksplit), (int)cq_streams_result(w, m));
     return hipGetLastError();
 }
@@ -1243,15 +1338,15 @@ hipError_t launch_tail(const cq_weight *w, cq_act_view a, int64_t m, float *y, c
 }
 
 template <int DT>
-hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, float *y, bool y_cleared, hipStream_t s) {
+hipError_t launch_dt(const cq_weight *w, cq_act_view a, int64_t m, uint32_t *turns, float *y, bool cleared, hipStream_t s) {
     const Plan p = pick_plan(w, m);
     const cq_mfma_dump none{nullptr, nullptr, 0};
     if (p.tail == 2) return launch_tail<DT, 2, false>(w, a, m, y, none, s);
     if (p.tail == 1) return launch_tail<DT, 1, false>(w, a, m, y, none, s);
     if (p.kh == 2) return p.mt == 1 ? launch_kh<DT, 1, false>(w, a, m, y, none, s) : launch_kh<DT, 2, false>(w, a, m, y, none, s);
-    if (p.mt == 1) return launch_mt<DT, 1>(w, a, m, y, p.ksplit, y_cleared, s);
-    if (p.mt == 2) return launch_mt<DT, 2>(w, a, m, y, p.ksplit, y_cleared, s);
-    return launch_mt<DT, 4>(w, a, m, y, p.ksplit, y_cleared, s);
+    if (p.mt == 1) return launch_mt<DT, 1>(w, a, m, turns, y, p.ksplit, cleared, s);
+    if (p.mt == 2) return launch_mt<DT, 2>(w, a, m, turns, y, p.ksplit, cleared, s);
+    return launch_mt<DT, 4>(w, a, m, turns, y, p.ksplit, cleared, s);
 }
 
 // The launch cq_launch_gemm would make, storing the block integers.
@@ -1289,28 +1384,30 @@ cq_grouped_plan pick_grouped(const cq_weight *w, const int32_t *offsets, int n_e
 
 template <int DT, int MT>
 hipError_t launch_grouped_mt(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
-                             float *y, int ksplit, bool y_cleared, hipStream_t s) {
+                             uint32_t *turns, float *y, int ksplit, bool cleared, hipStream_t s) {
     cq_group_args ga;
     const int ntiles = cq_group_table(experts, n_experts, offsets, 32 * MT, &ga);
     if (ntiles <= 0) return ntiles == 0 ? hipSuccess : hipErrorInvalidConfiguration;
     const cq_weight *w = experts[0];
     const size_t lds = MT == 1 && grouped_wbuf<DT>() == 2 ? Tile<DT, MT>::kTotal2 : Tile<DT, MT>::kTotal;
-    if (hipError_t e = cq_ensure_lds<gemm_grouped_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
-    if (ksplit > 1 && !y_cleared) {
-        hipError_t e = cq_launch_fill_zero(y, (int64_t)offsets[n_experts] * w->n, s);
-        if (e != hipSuccess) return e;
+    if (hipError_t e = clear_parts(ksplit, n_tiles(w) * ntiles, w->k, turns, y, (int64_t)offsets[n_experts] * w->n, cleared, s); e != hipSuccess) return e;
+    const dim3 grid((unsigned)n_tiles(w), (unsigned)ntiles, (unsigned)ksplit);
+    if (turns) {
+        if (hipError_t e = cq_ensure_lds<gemm_grouped_turns_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
+        CQ_LAUNCH((gemm_grouped_turns_kernel<DT, MT>), grid, kThreads, lds, s, ga, a, y, turns);
+        return hipGetLastError();
     }
-    dim3 grid((unsigned)n_tiles(w), (unsigned)ntiles, (unsigned)ksplit);
+    if (hipError_t e = cq_ensure_lds<gemm_grouped_kernel<DT, MT>>(w->dev, lds); e != hipSuccess) return e;
     CQ_LAUNCH((gemm_grouped_kernel<DT, MT>), grid, kThreads, lds, s, ga, a, y, ksplit);
     return hipGetLastError();
 }
 template <int DT>
 hipError_t launch_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
-                          float *y, bool y_cleared, hipStream_t s) {
+                          uint32_t *turns, float *y, bool cleared, hipStream_t s) {
     const cq_grouped_plan p = pick_grouped(experts[0], offsets, n_experts);
-    if (p.mt == 1) return launch_grouped_mt<DT, 1>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
-    if (p.mt == 2) return launch_grouped_mt<DT, 2>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
-    return launch_grouped_mt<DT, 4>(experts, n_experts, offsets, a, y, p.ksplit, y_cleared, s);
+    if (p.mt == 1) return launch_grouped_mt<DT, 1>(experts, n_experts, offsets, a, turns, y, p.ksplit, cleared, s);
+    if (p.mt == 2) return launch_grouped_mt<DT, 2>(experts, n_experts, offsets, a, turns, y, p.ksplit, cleared, s);
+    return launch_grouped_mt<DT, 4>(experts, n_experts, offsets, a, turns, y, p.ksplit, cleared, s);
 }
 
 template <int DT, int MT>
@@ -1339,11 +1436,11 @@ bool cq_gemm_grouped_supported(const cq_weight *const *experts, int n_experts, c
 }
 
 hipError_t cq_launch_gemm_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
-                                  float *y, bool y_cleared, hipStream_t s) {
+                                  uint32_t *turns, float *y, bool cleared, hipStream_t s) {
     if (a.m_stride < (int64_t)offsets[n_experts] + 127) return hipErrorInvalidValue;   // tiles of up to 128 rows from any row on
-    if (experts[0]->dtype == CQ_DTYPE_Q4K) return launch_grouped<CQ_DTYPE_Q4K>(experts, n_experts, offsets, a, y, y_cleared, s);
-    if (experts[0]->dtype == CQ_DTYPE_Q5K) return launch_grouped<CQ_DTYPE_Q5K>(experts, n_experts, offsets, a, y, y_cleared, s);
-    return launch_grouped<CQ_DTYPE_Q6K>(experts, n_experts, offsets, a, y, y_cleared, s);
+    if (experts[0]->dtype == CQ_DTYPE_Q4K) return launch_grouped<CQ_DTYPE_Q4K>(experts, n_experts, offsets, a, turns, y, cleared, s);
+    if (experts[0]->dtype == CQ_DTYPE_Q5K) return launch_grouped<CQ_DTYPE_Q5K>(experts, n_experts, offsets, a, turns, y, cleared, s);
+    return launch_grouped<CQ_DTYPE_Q6K>(experts, n_experts, offsets, a, turns, y, cleared, s);
 }
 
 hipError_t cq_launch_gemm_dump(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, cq_mfma_dump d, hipStream_t s) {
@@ -1355,8 +1452,11 @@ hipError_t cq_launch_gemm_dump(const cq_weight *w, cq_act_view a, int act_dtype,
     return launch_dump_dt<CQ_DTYPE_Q6K>(w, a, m, d, s);
 }
 
-bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets) {
-    return cq_group_tiles(offsets, n_experts, 32) > 0 && pick_grouped(experts[0], offsets, n_experts).ksplit > 1;
+cq_clear cq_gemm_grouped_clears(const cq_weight *const *experts, int n_experts, const int32_t *offsets, uint32_t *turns, float *y) {
+    if (cq_group_tiles(offsets, n_experts, 32) == 0) return cq_no_clear();
+    const cq_weight *w = experts[0];
+    const cq_grouped_plan p = pick_grouped(w, offsets, n_experts);
+    return clears(p.ksplit, n_tiles(w) * cq_group_tiles(offsets, n_experts, 32 * p.mt), w->k, turns, y, (int64_t)offsets[n_experts] * w->n);
 }
 
 double cq_gemm_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets) { return pick_grouped(w, offsets, n_experts).us; }
@@ -1376,7 +1476,11 @@ double cq_gemm_few_us(const cq_weight *w, int64_t m) {
     const double(&c)[4] = sum[w->dtype == CQ_DTYPE_Q4K ? 0 : w->dtype == CQ_DTYPE_Q5K ? 1 : 2];
     return c[0] + (c[1] * p.work + c[2] * p.merge) / 16.0 + c[3] * (double)w->n * (double)(w->k / 256) * (double)cq_type_size(w->dtype) / 1e6;
 }
-bool cq_gemm_splits_k(const cq_weight *w, int64_t m) { return m > 0 && pick_plan(w, m).ksplit > 1; }
+cq_clear cq_gemm_clears(const cq_weight *w, int64_t m, uint32_t *turns, float *y) {
+    if (m == 0) return cq_no_clear();
+    const Plan p = pick_plan(w, m);
+    return clears(p.ksplit, n_tiles(w) * ((m + p.mt * 32 - 1) / (p.mt * 32)), w->k, turns, y, m * w->n);
+}
 
 bool cq_gemm_takes(const cq_weight *w, int act_dtype) {
     // the copies address rows with 32-bit offsets: 8 rows of activations, 16 rows of a weight plane
@@ -1388,14 +1492,14 @@ bool cq_gemm_supported(const cq_weight *w, int64_t m, int act_dtype) {
     return cq_gemm_takes(w, act_dtype) && w->n % 32 == 0;
 }
 
-hipError_t cq_launch_gemm(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, bool y_cleared,
+hipError_t cq_launch_gemm(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, uint32_t *turns, float *y, bool cleared,
                           hipStream_t s) {
     if (!cq_gemm_takes(w, act_dtype)) return hipErrorNotSupported;
     if (m == 0 || w->n == 0) return hipSuccess;
     if (a.m_stride < (m + 127) / 128 * 128) return hipErrorInvalidValue;   // rows the last tile may read
-    if (w->dtype == CQ_DTYPE_Q4K) return launch_dt<CQ_DTYPE_Q4K>(w, a, m, y, y_cleared, s);
-    if (w->dtype == CQ_DTYPE_Q5K) return launch_dt<CQ_DTYPE_Q5K>(w, a, m, y, y_cleared, s);
-    return launch_dt<CQ_DTYPE_Q6K>(w, a, m, y, y_cleared, s);
+    if (w->dtype == CQ_DTYPE_Q4K) return launch_dt<CQ_DTYPE_Q4K>(w, a, m, turns, y, cleared, s);
+    if (w->dtype == CQ_DTYPE_Q5K) return launch_dt<CQ_DTYPE_Q5K>(w, a, m, turns, y, cleared, s);
+    return launch_dt<CQ_DTYPE_Q6K>(w, a, m, turns, y, cleared, s);
 }
 
 // K-quant weights x Q8_1 activations on the matrix cores (see gemm_q81_kernel).  The workspace rows are padded to whole

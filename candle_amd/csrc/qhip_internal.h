@@ -151,7 +151,7 @@ struct cq_pre {
 };
 static inline cq_pre cq_no_pre() { return cq_pre{CQ_PRE_NONE, nullptr, 0.0f}; }
 // Floats the activation quantizer sets to zero on its way: the output of a matmul that splits K and adds
-// its partial sums atomically (the launch it saves costs as much as the clearing).  p == nullptr: nothing.
+// its partial sums atomically, or the turns its parts take (the launch it saves costs as much as the clearing).  p == nullptr: nothing.
 struct cq_clear {
     float *p;
     int64_t count;
@@ -209,20 +209,25 @@ hipError_t cq_launch_skinny_dump(const cq_weight *w, cq_act_view a, int act_dtyp
 // gemm.hip
 bool cq_gemm_takes(const cq_weight *w, int act_dtype);
 bool cq_gemm_supported(const cq_weight *w, int64_t m, int act_dtype);
-// `y_cleared`: y is already zero (a launch that splits K otherwise clears it first); *_splits_k tell
-// beforehand whether the launch will add its results atomically
-hipError_t cq_launch_gemm(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, bool y_cleared,
+// `turns`: 64 * k bytes for the parts of a K split (cq_act_turns), or null.  What a launch that splits K wants to find zero (p null: nothing);
+// `cleared`: it does (else a launch in front clears it).
+inline uint32_t *cq_act_turns(const cq_act_view &a, int64_t k) {   // Q8K: in padding rows (tiles read at most 127 rows past the last one)
+    return (uint32_t *)(a.qs + (a.m_stride - 64) * k);
+}
+cq_clear cq_gemm_clears(const cq_weight *w, int64_t m, uint32_t *turns, float *y);
+hipError_t cq_launch_gemm(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, uint32_t *turns, float *y, bool cleared,
                           hipStream_t s);
-bool cq_gemm_splits_k(const cq_weight *w, int64_t m);
 // all experts of a mixture-of-experts projection in one launch; `a` and `y` cover all routed rows
 bool cq_gemm_grouped_supported(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype);
 hipError_t cq_launch_gemm_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,
-                                  float *y, bool y_cleared, hipStream_t s);
-bool cq_gemm_grouped_splits_k(const cq_weight *const *experts, int n_experts, const int32_t *offsets);
+                                  uint32_t *turns, float *y, bool cleared, hipStream_t s);
+cq_clear cq_gemm_grouped_clears(const cq_weight *const *experts, int n_experts, const int32_t *offsets, uint32_t *turns, float *y);
 double cq_gemm_grouped_us(const cq_weight *w, int n_experts, const int32_t *offsets);
 // gemm_blk32.hip: the tile kernel for Q8_0 / Q4_0 weights with Q8_0 activations (K a multiple of 64)
 bool cq_gemm32_takes(const cq_weight *w, int act_dtype);
 bool cq_gemm32_supported(const cq_weight *w, int act_dtype);
+// `y_cleared`: y is already zero (a launch that splits K otherwise clears it first); *_splits_k tell
+// beforehand whether the launch will add its results atomically
 hipError_t cq_launch_gemm32(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, float *y, bool y_cleared,
                             hipStream_t s);
 bool cq_gemm32_splits_k(const cq_weight *w, int64_t m);

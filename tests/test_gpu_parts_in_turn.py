@@ -1,0 +1,65 @@
+"""K split in two over workgroups (K-quant tile launches, plain and grouped): the two parts of a tile take turns at its results.  Rows and weight rows of
+no whole tile, an odd number of blocks, outputs that hold NaN before the call, the turns cleared by the quantizer and, with reused rows, by a launch
+of their own, replays of a captured call.  Against the launch that does not split (the same block integers, f32 sums over a row's blocks in another
+order); from call to call the same bits."""
+import numpy as np
+import pytest
+import torch
+
+from candle_amd.quantized import GgmlDType, QTensor
+from tests.test_gpu_few_rows_long import close
+from tests.test_gpu_fused_neighbours import qh  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [("Q4K", 2304, 3584, 1052), ("Q6K", 3102, 9216, 1089), ("Q3K", 6966, 5632, 280), ("Q5K", 2305, 3840, 1040), ("Q2K", 3102, 9216, 1089),
+          ("Q6K", 21822, 5376, 97)]
+
+
+def inputs(dt, n, k, m):
+    g = torch.Generator(device="cuda").manual_seed(n + k + m)
+    return QTensor.quantize(torch.randn(n, k, generator=g, device="cuda") * 0.02, GgmlDType[dt]).weight, torch.randn(m, k, generator=g, device="cuda")
+
+
+@pytest.mark.parametrize("dt,n,k,m", SHAPES)
+def test_two_parts(qh, dt, n, k, m):  # noqa: F811
+    w, x = inputs(dt, n, k, m)
+    want = qh.qmatmul(w, x, qh.FLAG_DETERMINISTIC)
+    ws, first = qh.Workspace(), None
+    for flags in (0, 0, qh.FLAG_REUSE_ACT, 0):
+        out = torch.full((m + 1, n), float("nan"), device="cuda")
+        qh.qmatmul(w, x, flags, out=out[:m], workspace=ws)
+        assert bool(torch.isnan(out[m]).all())
+        close(out[:m], want, k // 256)
+        first = out[:m] if first is None else first
+        assert torch.equal(first, out[:m])
+
+
+@pytest.mark.parametrize("dt,n,k,m", SHAPES[:3])
+def test_replays(qh, dt, n, k, m):  # noqa: F811
+    w, x = inputs(dt, n, k, m)
+    ws = qh.Workspace()
+    qh.qmatmul(w, x, workspace=ws)
+    y = torch.empty(m, n, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        qh.qmatmul(w, x, out=y, workspace=ws)
+    for i in range(4):
+        x.normal_()
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, qh.qmatmul(w, x))
+
+
+@pytest.mark.parametrize("dt,n,k,counts", [("Q6K", 4096, 14336, (16, 9, 22, 0, 31, 17, 20, 13)), ("Q4K", 1030, 3584, (40, 25, 1, 33, 20, 30, 26, 25)),
+                                           ("Q5K", 2048, 7168, (10, 12, 8, 9, 14, 6, 11, 10))])
+def test_experts(qh, dt, n, k, counts):  # noqa: F811
+    experts = [inputs(dt, n, k, 8 + e)[0] for e in range(len(counts))]
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    x = torch.randn(int(offsets[-1]), k, device="cuda")
+    ids = torch.arange(x.shape[0], device="cuda", dtype=torch.int32).flip(0).contiguous()
+    for rows in (None, ids):
+        want = qh.qmatmul_grouped(experts, x, rows, offsets, flags=qh.FLAG_DETERMINISTIC | qh.FLAG_FORCE_GEMM)
+        for _ in range(3):
+            close(qh.qmatmul_grouped(experts, x, rows, offsets, flags=qh.FLAG_FORCE_GEMM), want, k // 256)
