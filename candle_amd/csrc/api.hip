@@ -672,7 +672,8 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     }
     cq_act_view v;
     act_ws_layout(act, m, w->k, (uint8_t *)ws, &v);
-    uint32_t *const turns = path == kGemm ? cq_act_turns(v, w->k) : nullptr;
+    // (calls that reuse rows only read the workspace, and several streams may do so at once: their parts add atomically)
+    uint32_t *const turns = path == kGemm && !(flags & CQ_FLAG_REUSE_ACT) ? cq_act_turns(v, w->k) : nullptr;
     bool cleared = false;
     // a small weight: the rows quantized by the waves of the split-K kernel, which leaves them in the workspace as well
     const bool direct = flags == 0 && pre.kind == CQ_PRE_NONE && !in_place && path == kSkinny && cq_skinny_direct_takes(w, act, m);
@@ -902,7 +903,7 @@ static int grouped_impl(const cq_weight *const *experts, int n_experts, const fl
     }
     // gather + quantize every routed row once (clearing on the way what a grouped launch that splits K wants zero; with row ids the
     // extent of x is not known here, so no output is cleared then)
-    uint32_t *const turns = path == kGemm ? cq_act_turns(v, w0->k) : nullptr;
+    uint32_t *const turns = path == kGemm && !reuse ? cq_act_turns(v, w0->k) : nullptr;   // (reused rows: as in qmatmul_impl)
     cq_clear clear = path == kGemm ? cq_gemm_grouped_clears(experts, n_experts, offsets, turns, y_dev)
                                    : path == kGemm32 && cq_gemm32_grouped_splits_k(experts, n_experts, offsets) ? cq_clear{y_dev, total * w0->n}
                                                                                                                 : cq_no_clear();

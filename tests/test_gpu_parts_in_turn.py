@@ -1,6 +1,6 @@
 """K split in two over workgroups (K-quant tile launches, plain and grouped): the two parts of a tile take turns at its results.  Rows and weight rows of
-no whole tile, an odd number of blocks, outputs that hold NaN before the call, the turns cleared by the quantizer and, with reused rows, by a launch
-of their own, replays of a captured call.  Against the launch that does not split (the same block integers, f32 sums over a row's blocks in another
+no whole tile, an odd number of blocks, outputs that hold NaN before the call, replays of a captured call, calls that reuse the rows (they only read
+the workspace, which several streams may then do at once).  Against the launch that does not split (the same block integers, f32 sums over a row's blocks in another
 order); from call to call the same bits."""
 import numpy as np
 import pytest
@@ -28,7 +28,9 @@ def test_two_parts(qh, dt, n, k, m):  # noqa: F811
     ws, first = qh.Workspace(), None
     for flags in (0, 0, qh.FLAG_REUSE_ACT, 0):
         out = torch.full((m + 1, n), float("nan"), device="cuda")
+        before = ws.buf.clone() if flags else None
         qh.qmatmul(w, x, flags, out=out[:m], workspace=ws)
+        assert before is None or torch.equal(before, ws.buf)
         assert bool(torch.isnan(out[m]).all())
         close(out[:m], want, k // 256)
         first = out[:m] if first is None else first
@@ -63,3 +65,8 @@ def test_experts(qh, dt, n, k, counts):  # noqa: F811
         want = qh.qmatmul_grouped(experts, x, rows, offsets, flags=qh.FLAG_DETERMINISTIC | qh.FLAG_FORCE_GEMM)
         for _ in range(3):
             close(qh.qmatmul_grouped(experts, x, rows, offsets, flags=qh.FLAG_FORCE_GEMM), want, k // 256)
+    ws = qh.Workspace()
+    want = qh.qmatmul_grouped(experts, x, ids, offsets, flags=qh.FLAG_FORCE_GEMM, workspace=ws)
+    before = ws.buf.clone()
+    close(qh.qmatmul_grouped(experts, x, ids, offsets, flags=qh.FLAG_FORCE_GEMM | qh.FLAG_REUSE_ACT, workspace=ws), want, k // 256)
+    assert torch.equal(before, ws.buf)
