@@ -903,11 +903,19 @@ static int grouped_impl(const cq_weight *const *experts, int n_experts, const fl
     }
     // gather + quantize every routed row once (clearing on the way what a grouped launch that splits K wants zero; with row ids the
     // extent of x is not known here, so no output is cleared then)
-    uint32_t *const turns = path == kGemm && !reuse ? cq_act_turns(v, w0->k) : nullptr;   // (reused rows: as in qmatmul_impl)
+    const int64_t count = total * w0->n;
+    const bool clearable = !reuse && !row_ids_dev && clear_in_quantizer_ok(y_dev, count, x_dev, total * w0->k, pre);
+    // Two parts of K add atomically where the output is cleared on the way and has 0.9 to 3.7 MB: there the wait for the turn costs more than the
+    // additions.  250 calls of 4 to 15 experts in two parts, weights from HBM, time with turns over time with additions, mean (most): up to 0.9 MB
+    // 0.99 (1.02), 1 to 1.5 1.01 (1.12), 1.5 to 2 1.03 (1.11), 2 to 2.5 1.02 (1.085), 2.5 to 3.7 1.02 (1.07), 3.7 to 5 0.99 (1.035), more 0.95 (0.99);
+    // us, additions / turns: Q6K 1216 x 1024 with 206 rows 13.1 / 14.4, Q4K 2176 x 2048 with 201 17.3 / 18.7, Q5K 3360 x 3072 with 468 (6.3 MB) 38.4 / 34.4.
+    // Where a launch of its own would clear the output (row ids), turns at every size (127 calls: 0.86 to 1.02).
+    const bool add = clearable && count >= (7 << 15) && count < (7 << 17);
+    uint32_t *const turns = path == kGemm && !reuse && !add ? cq_act_turns(v, w0->k) : nullptr;   // (reused rows: as in qmatmul_impl)
     cq_clear clear = path == kGemm ? cq_gemm_grouped_clears(experts, n_experts, offsets, turns, y_dev)
-                                   : path == kGemm32 && cq_gemm32_grouped_splits_k(experts, n_experts, offsets) ? cq_clear{y_dev, total * w0->n}
+                                   : path == kGemm32 && cq_gemm32_grouped_splits_k(experts, n_experts, offsets) ? cq_clear{y_dev, count}
                                                                                                                 : cq_no_clear();
-    if (reuse || (clear.p == y_dev && (row_ids_dev || !clear_in_quantizer_ok(y_dev, total * w0->n, x_dev, total * w0->k, pre)))) clear = cq_no_clear();
+    if (reuse || (clear.p == y_dev && !clearable)) clear = cq_no_clear();
     if (!reuse) CQ_HIP_CHECK(cq_launch_quantize_act_ws(act, x_dev, row_ids_dev, total, w0->k, pre, v, clear, s));
     switch (path) {
     case kSkinny: CQ_HIP_CHECK(cq_launch_skinny_grouped(experts, n_experts, offsets, v, y_dev, s)); return CQ_OK;

@@ -70,3 +70,28 @@ def test_experts(qh, dt, n, k, counts):  # noqa: F811
     before = ws.buf.clone()
     close(qh.qmatmul_grouped(experts, x, ids, offsets, flags=qh.FLAG_FORCE_GEMM | qh.FLAG_REUSE_ACT, workspace=ws), want, k // 256)
     assert torch.equal(before, ws.buf)
+
+
+def turns_taken(ws, m, k):
+    """The counters of the parts in the padding rows of a workspace of m quantized rows that held 0xEE before the call: {turns taken, turns done} of every
+    tile and wave that took them."""
+    words = ws.buf[((m + 63) // 64 * 64 + 192) * k:][:64 * k].view(torch.int32).view(-1, 2)
+    return int((words == torch.tensor([2, 1], device="cuda", dtype=torch.int32)).all(1).sum()), int((words == -0x11111112).all(1).sum()), len(words)
+
+
+@pytest.mark.parametrize("dt,n,k,counts,by_turns", [("Q4K", 960, 1280, (10, 11, 9, 14, 8, 12, 10, 10), True), ("Q4K", 2176, 2048, (25, 30, 20, 26, 31, 17, 28, 24), False),
+                                                    ("Q6K", 1216, 1024, (25, 30, 20, 26, 31, 17, 28, 29), False), ("Q6K", 3552, 4096, (64, 50, 60, 33, 47, 56, 60, 60), True)])
+def test_experts_take_turns_where_ahead(qh, dt, n, k, counts, by_turns):  # noqa: F811
+    """Outputs of middle size that the quantizer clears are added to; where a launch would have to clear them (row ids) the parts take turns."""
+    experts = [inputs(dt, n, k, 8 + e)[0] for e in range(len(counts))]
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    m = int(offsets[-1])
+    x = torch.randn(m, k, device="cuda")
+    ids = torch.arange(m, device="cuda", dtype=torch.int32)
+    want = qh.qmatmul_grouped(experts, x, None, offsets, flags=qh.FLAG_DETERMINISTIC | qh.FLAG_FORCE_GEMM)
+    for rows in (None, ids):
+        ws = qh.Workspace()
+        ws.get(64 << 20, x.device).fill_(0xEE)
+        close(qh.qmatmul_grouped(experts, x, rows, offsets, flags=qh.FLAG_FORCE_GEMM, workspace=ws), want, k // 256)
+        taken, untouched, pairs = turns_taken(ws, m, k)
+        assert taken >= (n + 31) // 32 * len(counts) if by_turns or rows is not None else untouched == pairs
