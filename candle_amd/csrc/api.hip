@@ -1046,3 +1046,11 @@ extern "C" int cq_selfcheck_round(int dev, uint64_t *mismatches) {
     *mismatches = host;
     return CQ_OK;
 }
+
+extern "C" int cq_selfcheck_turns(int dev, int32_t *turn, float *y, int looks, void *stream) {
+    if (!turn || !y) return cq_set_error(CQ_ERR_INVALID, "null argument");
+    if (looks < 1) return cq_set_error(CQ_ERR_INVALID, "at least one look is needed, not %d", looks);
+    CQ_HIP_CHECK(hipSetDevice(dev));
+    CQ_HIP_CHECK(cq_launch_turns_check((uint32_t *)turn, y, looks, (hipStream_t)stream));
+    return CQ_OK;
+}

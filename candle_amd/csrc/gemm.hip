@@ -612,16 +612,29 @@ __device__ __forceinline__ int64_t last_tile(int64_t n_own, int64_t n) { return 
 // 134.2 -> 120.3, Q3K 3102 x 9216 at 1089 110.6 -> 94.4, Q6K 21822 x 5376 at 96 62.9 -> 54.8; 8 experts of 1024 x 3584 with 100 tokens
 // 57.4 -> 51.8.  More parts stay with the additions: a turn of each costs some 5 us, one after the other (Q6K 4096 x 14336 at 512 / 128 rows, four
 // and eight parts, 96.2 -> 93.8 and 39.8 -> 58.7, Q4K 4096 x 14336 at 256 52.7 -> 54.7).
+// A turn that cannot come right is shown: where the first part is not there after `looks` looks (a second or so) or the turn is a third one, calls
+// overlap on one workspace, and the wave's share of y is NaN.
+constexpr int kTurnLooks = 1 << 20;
 template <int MT>
-__device__ __forceinline__ void put_in_turn(uint32_t *turn, float *y, float *yc, int64_t pitch, int64_t left, int lane, v16f (&out)[MT]) {
+__device__ __forceinline__ void put_in_turn(uint32_t *turn, float *y, float *yc, int64_t pitch, int64_t left, int lane, v16f (&out)[MT], int looks = kTurnLooks) {
     uint32_t mine = 0;
     if (lane == 0) mine = __hip_atomic_fetch_add(turn, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const auto at = [&](int t, int i) { return (int64_t)(t * 32 + (i >> 2) * 8 + (i & 3)); };
-    if (__builtin_amdgcn_readfirstlane((int)mine) > 0) {   // the second
-        // (bounded, a second or so: calls that share a workspace although they overlap spoil each other's turns as well as rows)
-        for (int looks = 1 << 20; looks > 0; looks--) {
-            if (__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(turn + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) break;
+    const int order = __builtin_amdgcn_readfirstlane((int)mine);
+    if (order > 0) {   // the second
+        bool there = false;
+        for (; looks > 0; looks--) {
+            there = __builtin_amdgcn_readfirstlane((int)__hip_atomic_load(turn + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
+            if (there) break;
             __builtin_amdgcn_s_sleep(1);
+        }
+        if (!there || order > 1) {
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (at(t, i) < left) yc[at(t, i) * pitch] = __builtin_nanf("");
+            return;
         }
         asm volatile("" ::: "memory");   // (the results are requested behind this)
         float held[MT][16];
@@ -772,6 +785,14 @@ __global__ void __launch_bounds__(kThreads) gemm_kernel(cq_weight w, cq_act_view
                                                         int ksplit, int strips, int stream) {
     const cq_tile t = cq_tile_at(blockIdx.x, blockIdx.y, gridDim.x, gridDim.y, strips);
     gemm_body<DT, MT>(w, a, t.x, (int64_t)t.y * (MT * 32), m, y, ksplit, stream != 0);
+}
+// One wave's turn at a tile of 32 x 32 results, 1 + column each.
+__global__ void __launch_bounds__(64) turns_check_kernel(uint32_t *turn, float *y, int looks) {
+    const int lane = threadIdx.x, h = lane >> 5, c = lane & 31;
+    v16f out[1];
+#pragma unroll
+    for (int i = 0; i < 16; i++) out[0][i] = (float)(1 + c);
+    put_in_turn<1>(turn, y, y + h * 4 * 32 + c, 32, 32 - h * 4, lane, out, looks);
 }
 // (kernels of their own: as a branch in the others' ends, the main loops were allocated otherwise and launches that do not split lost 1.2 %)
 template <int DT, int MT>
@@ -1441,6 +1462,11 @@ hipError_t cq_launch_gemm_grouped(const cq_weight *const *experts, int n_experts
     if (experts[0]->dtype == CQ_DTYPE_Q4K) return launch_grouped<CQ_DTYPE_Q4K>(experts, n_experts, offsets, a, turns, y, cleared, s);
     if (experts[0]->dtype == CQ_DTYPE_Q5K) return launch_grouped<CQ_DTYPE_Q5K>(experts, n_experts, offsets, a, turns, y, cleared, s);
     return launch_grouped<CQ_DTYPE_Q6K>(experts, n_experts, offsets, a, turns, y, cleared, s);
+}
+
+hipError_t cq_launch_turns_check(uint32_t *turn, float *y, int looks, hipStream_t s) {
+    turns_check_kernel<<<1, 64, 0, s>>>(turn, y, looks < kTurnLooks ? looks : kTurnLooks);
+    return hipGetLastError();
 }
 
 hipError_t cq_launch_gemm_dump(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, cq_mfma_dump d, hipStream_t s) {

@@ -217,6 +217,7 @@ inline uint32_t *cq_act_turns(const cq_act_view &a, int64_t k) {   // Q8K: in pa
 cq_clear cq_gemm_clears(const cq_weight *w, int64_t m, uint32_t *turns, float *y);
 hipError_t cq_launch_gemm(const cq_weight *w, cq_act_view a, int act_dtype, int64_t m, uint32_t *turns, float *y, bool cleared,
                           hipStream_t s);
+hipError_t cq_launch_turns_check(uint32_t *turn, float *y, int looks, hipStream_t s);   // cq_selfcheck_turns
 // all experts of a mixture-of-experts projection in one launch; `a` and `y` cover all routed rows
 bool cq_gemm_grouped_supported(const cq_weight *const *experts, int n_experts, const int32_t *offsets, int act_dtype);
 hipError_t cq_launch_gemm_grouped(const cq_weight *const *experts, int n_experts, const int32_t *offsets, cq_act_view a,

@@ -27,7 +27,7 @@ EXPORTS = [
     "cq_weight_device", "cq_weight_shape", "cq_weight_destroy", "cq_act_bytes", "cq_quantize_act",
     "cq_workspace_bytes", "cq_qmatmul", "cq_qmatmul_int_dots", "cq_qmatmul_int_dots_mfma", "cq_grouped_workspace_bytes",
     "cq_qmatmul_grouped", "cq_silu_mul", "cq_moe_scatter_add", "cq_moe_scatter", "cq_timing_arm", "cq_timing_elapsed_us",
-    "cq_selfcheck_round", "cq_quantize_act_fused", "cq_qmatmul_fused", "cq_qmatmul_grouped_fused", "cq_qmatmul_multi",
+    "cq_selfcheck_round", "cq_selfcheck_turns", "cq_quantize_act_fused", "cq_qmatmul_fused", "cq_qmatmul_grouped_fused", "cq_qmatmul_multi",
     "cq_weight_zeros_flat", "cq_weight_create_flat", "cq_weight_elem_count", "cq_weight_set_shape",
     "cq_workspace_bytes_shaped", "cq_qmatmul_shaped", "cq_qmatmul_static",
 ]
@@ -81,6 +81,7 @@ def load():
     L.cq_timing_arm.argtypes = []
     L.cq_timing_elapsed_us.argtypes = [C.POINTER(C.c_double)]
     L.cq_selfcheck_round.argtypes = [ci, C.POINTER(C.c_uint64)]
+    L.cq_selfcheck_turns.argtypes = [ci, vp, vp, ci, vp]
     L.cq_quantize_act_fused.argtypes = [ci, ci, ci, vp, vp, C.c_float, i64, i64, vp, vp]
     L.cq_qmatmul_fused.argtypes = [vp, ci, vp, vp, C.c_float, i64, vp, ci, vp, sz, vp]
     L.cq_qmatmul_grouped_fused.argtypes = [C.POINTER(vp), ci, ci, vp, vp, C.c_float, vp, C.POINTER(C.c_int32), vp, ci,

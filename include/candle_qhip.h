@@ -170,7 +170,9 @@ int cq_quantize_act(int dev, int act_dtype, const float *x_dev, int64_t m, int64
 
 /* ---- matmul -------------------------------------------------------------- */
 /* Scratch the caller must provide to cq_qmatmul for m activation rows (the reference allocates
- * its quantized-activation buffer per call, cuda.rs:249-252, 322-325). */
+ * its quantized-activation buffer per call, cuda.rs:249-252, 322-325).  It belongs to one call until the stream has passed
+ * that call: calls that overlap on it in time spoil each other's results, whole tiles of which may be NaN then.  Calls with
+ * CQ_FLAG_REUSE_ACT only read it and may share it. */
 size_t cq_workspace_bytes(const cq_weight *w, int64_t m, int flags);
 /* QCudaStorage::fwd (cuda.rs:478-499) = <QTensor as CustomOp1>::cuda_fwd (mod.rs:514-524):
  * y[m, n] = x[m, k] . W[n, k]^T with x quantized to W's VecDotType first (k_quants.rs:1842-1883).
@@ -310,6 +312,12 @@ int cq_timing_elapsed_us(double *us);
  * every f32 t with |t| <= 130 (both signs, denormals included) and stores the number of
  * mismatches, which must be zero on any device the library is used on. */
 int cq_selfcheck_round(int dev, uint64_t *mismatches);
+/* Two parts of a matmul whose K is split take turns at a tile of results by a pair of counters in the workspace, {turns taken,
+ * turns done}.  This call lets one part take its turn at 32 x 32 results (1 + column each) with the counters turn_dev[2] and
+ * y_dev[32 * 32] as they are: {0, 0} stores the results, {1, 1} adds them to y.  The wait for the other part ends after
+ * `looks` looks (1 and more; at most as many as in a matmul): where it is not done by then, or the turn is a third one - calls
+ * that overlap on one workspace - y is NaN. */
+int cq_selfcheck_turns(int dev, int32_t *turn_dev, float *y_dev, int looks, void *stream);
 
 #ifdef __cplusplus
 }

@@ -95,3 +95,21 @@ def test_experts_take_turns_where_ahead(qh, dt, n, k, counts, by_turns):  # noqa
         close(qh.qmatmul_grouped(experts, x, rows, offsets, flags=qh.FLAG_FORCE_GEMM, workspace=ws), want, k // 256)
         taken, untouched, pairs = turns_taken(ws, m, k)
         assert taken >= (n + 31) // 32 * len(counts) if by_turns or rows is not None else untouched == pairs
+
+
+@pytest.mark.parametrize("taken,done,held,want", [(0, 0, float("nan"), 0.0), (1, 1, 0.5, 0.5), (1, 0, 0.5, None), (2, 1, 0.5, None)])
+def test_a_turn(qh, taken, done, held, want):  # noqa: F811
+    """The first part stores, the second adds; where the first does not come, or there is a third, the results say so."""
+    turn = torch.tensor([taken, done], device="cuda", dtype=torch.int32)
+    y = torch.full((33, 32), held, device="cuda")
+    y[32] = 7.0
+    for looks in (0, -1):
+        assert qh.load().cq_selfcheck_turns(0, turn.data_ptr(), y.data_ptr(), looks, None) == -1
+    torch.cuda.synchronize()
+    qh.check(qh.load().cq_selfcheck_turns(0, turn.data_ptr(), y.data_ptr(), 4, torch.cuda.current_stream().cuda_stream))
+    assert turn.tolist() == [taken + 1, 1 if taken == 0 else done]
+    assert bool((y[32] == 7.0).all())
+    if want is None:
+        assert bool(torch.isnan(y[:32]).all())
+    else:
+        assert torch.equal(y[:32], (torch.arange(32, device="cuda") + (1.0 + want)).expand(32, 32))
