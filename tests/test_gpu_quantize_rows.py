@@ -51,3 +51,15 @@ def test_many_rows_give_the_bytes_of_few(qh, m, k, silu):  # noqa: F811
         ok = np.isfinite(blocks).all(1)
         want = np.stack([orc.quantize(orc.Q8K, b) for b in blocks[ok]])
         assert np.array_equal(got.cpu().numpy().reshape(len(blocks), -1)[ok], want)
+
+
+@pytest.mark.parametrize("dt", [orc.Q4K, orc.Q5K, orc.Q6K])
+@pytest.mark.parametrize("k", [256, 2304, 4096, 16384])
+def test_one_row_gives_the_bits_of_its_quantized_row(qh, dt, k):  # noqa: F811
+    """The one-launch kernels quantize their row in code of their own: on such blocks too the bits of the call that goes through the quantizer."""
+    blocks = orc.quantize(dt, np.random.default_rng(k).standard_normal((24, k)).astype(np.float32) * np.float32(0.02))
+    w = qh.QWeight.from_ggml(dt, blocks, 24, k)
+    for row in rows(11, k):
+        x = dev(row[None])
+        one, staged = qh.qmatmul(w, x), qh.qmatmul(w, x, qh.FLAG_STAGED_ACT)
+        assert torch.equal(one.view(torch.int32), staged.view(torch.int32))
