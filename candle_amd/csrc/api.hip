@@ -464,7 +464,7 @@ extern "C" int cq_quantize_act_fused(int dev, int act_dtype, int pre, const floa
 static size_t act_ws_layout(int act_dtype, int64_t m, int64_t k, uint8_t *base, cq_act_view *v, bool grouped = false) {
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off = cq_align_up(off + bytes, 256); return o; };
-    // Q8K rows are padded (see cq_act_view::m_stride); the others to whole 32-row groups, which the
+    // Q8K rows are padded, for what the tiles read past the last one and for the turns of a K split (see cq_act_view::m_stride); the others to whole 32-row groups, which the
     // split-K MFMA kernel copies without looking at the row count
     // (beyond 32 rows to whole 128-row tiles, which the 32-element-block tile kernel reads)
     const int64_t m_pad = act_dtype == CQ_DTYPE_Q8K ? (m + 63) / 64 * 64 + 256 : (m <= 32 ? (m + 31) / 32 * 32 : (m + 127) / 128 * 128) + (grouped ? 128 : 0);
@@ -672,7 +672,8 @@ static int qmatmul_impl(const cq_weight *w, const float *x_dev, cq_pre pre, int6
     }
     cq_act_view v;
     act_ws_layout(act, m, w->k, (uint8_t *)ws, &v);
-    // (calls that reuse rows only read the workspace, and several streams may do so at once: their parts add atomically)
+    // (calls that reuse rows only read the workspace, and several streams may do so at once: their parts add atomically, as do those of the second and
+    // third weight of cq_qmatmul_multi, which come here with the same flag)
     uint32_t *const turns = path == kGemm && !(flags & CQ_FLAG_REUSE_ACT) ? cq_act_turns(v, w->k) : nullptr;
     bool cleared = false;
     // a small weight: the rows quantized by the waves of the split-K kernel, which leaves them in the workspace as well

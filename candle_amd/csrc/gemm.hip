@@ -608,10 +608,11 @@ __device__ __forceinline__ int64_t last_tile(int64_t n_own, int64_t n) { return 
 // through the memory that all XCDs see (stores and loads of device scope; a store has arrived there when s_waitcnt says so, and only then the turn
 // is passed on).  `turn`: {turns taken, turns done}, zero before the launch.
 // Adding to a cleared y atomically moves about 1.1 TB/s at the end of all workgroups at once, and y is cleared first.  Whole calls, weights from
-// HBM, us, atomic additions -> turns: Q6K 4096 x 14336 at 1003 rows 164.8 -> 152.5, 7510 x 5376 at 423 80.1 -> 63.0, Q4K 8382 x 14336 at 375
-// 134.2 -> 120.3, Q3K 3102 x 9216 at 1089 110.6 -> 94.4, Q6K 21822 x 5376 at 96 62.9 -> 54.8; 8 experts of 1024 x 3584 with 100 tokens
-// 57.4 -> 51.8.  More parts stay with the additions: a turn of each costs some 5 us, one after the other (Q6K 4096 x 14336 at 512 / 128 rows, four
-// and eight parts, 96.2 -> 93.8 and 39.8 -> 58.7, Q4K 4096 x 14336 at 256 52.7 -> 54.7).
+// HBM, us, atomic additions -> turns: Q6K 4096 x 14336 at 1003 rows 164.6 -> 154.8, 7510 x 5376 at 423 79.6 -> 66.8, Q4K 8382 x 14336 at 375
+// 133.8 -> 124.0, Q3K 3102 x 9216 at 1089 110.4 -> 98.3, Q6K 21822 x 5376 at 96 64.4 -> 56.0.  Of 124 random calls in two parts, by the size of y:
+// up to 1 MB 0.98 of the time (15 calls), 4.7 to 8 MB 0.99 (20; tiles with few live rows up to 1.025: Q6K 17824 x 7424 at 68 67.4 -> 69.1), more 0.95 (89);
+// experts: grouped_impl in api.hip.  More parts stay with the additions: a turn of each costs some 5 us, one after the other (Q6K 4096 x 14336
+// at 512 / 128 rows, four and eight parts, 96.2 -> 93.8 and 39.8 -> 58.7, Q4K 4096 x 14336 at 256 52.7 -> 54.7).
 // A turn that cannot come right is shown: where the first part is not there after `looks` looks (a second or so) or the turn is a third one, calls
 // overlap on one workspace, and the wave's share of y is NaN.
 constexpr int kTurnLooks = 1 << 20;
@@ -1216,11 +1217,11 @@ int64_t n_tiles(const cq_weight *w) { return (w->n + kWaves * 32 - 1) / (kWaves 
 // Tile height (MT x 32 activation rows per workgroup) and K split of a launch, from a cost model fitted to
 // measurements (Q4K, 256 CUs; unit 1/16 us): a workgroup spends 22 units per K block unpacking its weights
 // and 13.5 per 32-row tile on it, 24 on starting and finishing; workgroups run one per CU, in rounds; a split
-// launch adds every part to the output atomically, which moves about 1.1 TB/s (two parts take turns and are less than that; the plan is as it was:
-// with their own price, 3 us and 2.7 TB/s, 1.1 % of the calls change, on average 4 % slower, as the work's price is above what it costs).  Tall
-// tiles amortise
-// the unpacking, short ones fill the machine without splitting K: 4096 x 4096 at 512 rows takes 54 us as
-// 64 tiles of 128 rows split four ways and 42 us as 256 tiles of 32 rows.
+// launch adds every part to the output atomically, which moves about 1.1 TB/s.  (Two parts take turns, 3 us and 2.7 TB/s; the plan keeps the price
+// of the additions for them: with their own 1.1 % of the calls change, on average 4 % slower, as the work's price is above what it costs.  So do
+// the estimates that choose the kernel, cq_gemm_us and the two others below: with the turns' price none of 3 million calls in groups of rows
+// and none of 300000 over experts would choose otherwise, and 0.03 % of those of 17 to 32 rows.)  Tall tiles amortise the unpacking, short ones
+// fill the machine without splitting K: 4096 x 4096 at 512 rows takes 54 us as 64 tiles of 128 rows split four ways and 42 us as 256 tiles of 32 rows.
 struct Plan {
     int mt, ksplit;
     int kh = 1;   // 2: gemm_kh_kernel (K halved inside the workgroup, 128 weight rows per workgroup)

@@ -12,9 +12,9 @@
 // work per element is one conversion and one fma.
 // Bound by vector issue.  ns a step of the two waves of a SIMD (a tile and block of each) in a loop of nothing but steps, the scales as two bf16
 // pieces each (v_mfma_f32_32x32x16_bf16: three instructions for the operand, three for the zeros beside it) -> as f16: Q8_0 70.9 -> 62.8, Q4_0
-// 68.5 -> 61.0; without the second MFMA 55.6.  Whole calls, weights from HBM, us: Q8_0 11008 x 4096 at 4096 / 512 / 64 rows 511 -> 474, 93.6 -> 87.4,
-// 23.9 -> 23.3, Q4_0 4096 x 4096 at 512 / 1024 rows 35.6 -> 33.4, 59.0 -> 55.0, 11008 x 4096 at 4096 498 -> 459, Q5_0 4096 x 11008 at 700
-// 150.9 -> 141.2.  (The next step's weight operands read under this step's last tile instead of behind the barrier: level to 2 % slower.)
+// 68.5 -> 61.0; without the second MFMA 55.6.  Whole calls, weights from HBM, us: Q8_0 11008 x 4096 at 4096 / 512 / 64 rows 520 -> 483, 99.3 -> 93.7,
+// 27.7 -> 27.6, Q4_0 4096 x 4096 at 512 / 1024 rows 37.2 -> 35.5, 61.3 -> 57.4, 11008 x 4096 at 4096 499 -> 459, Q5_0 4096 x 11008 at 700
+// 154.6 -> 144.8.  (The next step's weight operands read under this step's last tile instead of behind the barrier: level to 2 % slower.)
 //
 // Work split as in the K-quant tile kernel (gemm.hip): a workgroup of eight waves covers 32*MT
 // activation rows x 256 weight rows, a wave owns 32 weight rows; per 256-element step of K the

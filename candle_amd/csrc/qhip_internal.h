@@ -69,8 +69,8 @@ struct cq_act_view {
     // For the matrix-core kernels (block-major so that a tile of rows is contiguous per block):
     float *dT;         // Q8K [k/256][m_stride], Q8_0 [k/32][m_stride] f32, the same values as d
     uint16_t *bsh;     // Q8K: [k/256][m_stride][16] f16: the block's sixteen bsums as f16 (exact), the min term's operand
-    int64_t m_stride;  // rows allocated: at least 256 more than the rows quantized, so that the GEMM
-                       // may read (and ignore) whole 128-row tiles past the last row
+    int64_t m_stride;  // rows allocated.  Q8K: at least 256 more than the rows quantized; the tile kernels read (and ignore) whole 128-row
+                       // tiles, up to 127 rows past the last one, and the last 64 hold the turns of a K split (cq_act_turns)
     int16_t *bsum32; // Q8_0 / Q8_1: the block's sum of quants (at most 4096 in magnitude)
     uint16_t *s16;   // Q8_1: the block's `s` field (f16 bits)
 };

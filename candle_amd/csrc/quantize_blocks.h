@@ -61,10 +61,11 @@ __device__ __forceinline__ void cq_q8k_of_sixteen(const float4 (&f)[4], int l, u
     bsum = j == 0 ? sum[0] : j == 1 ? sum[1] : j == 2 ? sum[2] : sum[3];
 }
 
-// The same for a block per wave: lane l holds elements 4l .. 4l + 3; all arguments but `f` and `packed` are the wave's.  `sum`: of the lane's four
-// lanes (bsums[l / 4]).  For few blocks: the launch waits for one chain of dependent instructions, which the search for the first largest element,
-// the rounding by itself and the clamp by another made twice as long (24 such launches behind rms_norm and silu, among them the step's other
-// launches: 481.9 -> 479.2 us; eight rows of 4096 with their matmul 10.21 -> 10.18).
+// The same for a block per wave: lane l holds elements 4l .. 4l + 3 in `f` and their quants in `packed`; `sum` is that of its four lanes (bsums[l / 4]),
+// `d` the same in all.  For few blocks: the launch waits for one chain of dependent instructions, which the search for the first largest element,
+// the rounding by itself and the clamp by another made twice as long.  Kernel alone, us: eight rows of 4096 3.00 -> 2.84, four behind rms_norm
+// 4.84 -> 4.44, four of 14336 behind silu * mul 3.96 -> 3.96; in the calls that is 0.3 to 0.4 % (a step's 17 such launches among 41: 476.7 -> 474.6 us,
+// eight rows with their matmul 10.21 -> 10.18).
 __device__ __forceinline__ void cq_q8k_of_wave(const float4 f, int lane, uint32_t &packed, float &d, int &sum) {
     float hi = fmaxf(fmaxf(fmaxf(fmaxf(0.0f, f.x), f.y), f.z), f.w), lo = fminf(fminf(fminf(fminf(0.0f, f.x), f.y), f.z), f.w);
     hi = fmaxf(hi, dpp_f<kQuadSwap1>(hi));

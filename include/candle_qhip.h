@@ -91,8 +91,8 @@ enum {
                                  not: the tile kernels (17 rows and more; grouped experts with more than 16, of large Q8_0 weights 4) split K
                                  over several workgroups when the weight has few row tiles - n = 4096 at 33 .. 1024
                                  rows, the w2 projection of an expert - and add the partial sums atomically in
-                                 arrival order (but for two parts of a K-quant: the sum of two is the same), so the last bits of a result can differ between two runs (far inside
-                                 the 1e-4 bar; the reference's CUDA arm is allowed 1e-4 of drift between batch sizes,
+                                 arrival order, so the last bits of a result can differ between two runs where there are more than two
+                                 parts (a sum of two is the same in either order; far inside the 1e-4 bar; the reference's CUDA arm is allowed 1e-4 of drift between batch sizes,
                                  quantized_tests.rs:203-209).  With the flag those launches never split K: each
                                  result is one sum in a fixed order, at the price of fewer workgroups in flight.
                                  Every other kernel is deterministic as it is.  Accepted by all matmul entry points. */
